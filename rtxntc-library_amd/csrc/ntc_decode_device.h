@@ -60,6 +60,17 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int kWaveTexels  = 64;
 
+// The entries of a launch's table, which is the kernel's FIRST argument.  The arguments are addressed where they lie:
+// indexed as a by-value parameter the table would be copied to scratch first.  Both sources are constant memory for
+// the whole launch, so uniform reads stay scalar loads.
+__device__ __forceinline__ DevMip const* table_entries(DevMip const* entries)
+{
+    typedef __attribute__((address_space(4))) DevMip const* ConstantMips;
+    ConstantMips const inlined = (ConstantMips)__builtin_amdgcn_kernarg_segment_ptr();
+    ConstantMips const stored = (ConstantMips)(uintptr_t)entries;
+    return (DevMip const*)(entries ? stored : inlined);
+}
+
 // ---- small device helpers -----------------------------------------------------------
 
 __device__ __forceinline__ uint32_t spread2(uint32_t byte)     // 4 x 2-bit fields -> 4 bytes

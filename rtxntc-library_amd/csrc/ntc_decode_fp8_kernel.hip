@@ -759,8 +759,9 @@ __device__ __forceinline__ void mlp_forward_fp8(Fp8Lds<V>& lds, int wave, int la
 // of a common sequence drift apart in time, and the latent reads from memory doubled.)
 template <class V>
 __global__ void __launch_bounds__(V::THREADS, 1)
-decode_fp8_kernel(DevMip const* __restrict__ mips, int numMips, int totalTiles, Fp8Handoff handoff)
+decode_fp8_kernel(MipTable table, int numMips, int totalTiles, Fp8Handoff handoff)
 {
+    DevMip const* const mips = table_entries(table.entries);
     if (!V::ONE && *handoff.word != handoff.serial) return;  // the one-plane launch before this one met only its own sets
     __shared__ Fp8Lds<V> lds;
     int const lane = threadIdx.x & 63;
@@ -855,9 +856,10 @@ decode_fp8_kernel(DevMip const* __restrict__ mips, int numMips, int totalTiles, 
 // weight blob, per launch.  A query whose mip is out of range writes zeros.
 template <class V>
 __global__ void __launch_bounds__(V::THREADS, 1)
-query_fp8_kernel(DevMip const* __restrict__ mips, int numMips, DevQuery const* __restrict__ queries, uint64_t numQueries,
+query_fp8_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queries, uint64_t numQueries,
                  uint16_t* __restrict__ out, Fp8Handoff handoff)
 {
+    DevMip const* const mips = table_entries(table.entries);
     if (!V::ONE && *handoff.word != handoff.serial) return;  // the set went to the one-plane launch before this one
     __shared__ Fp8Lds<V> lds;
     __shared__ QueryMip qmips[16];
@@ -950,7 +952,7 @@ using VFp8_16 = Fp8Variant<16>;
 // find that number there (nothing ever clears the word: a stale match only costs the second launch its look at
 // the weights, after which it passes over the sets that are not its own as before).
 template <int FEATURES>
-static hipError_t launch_fp8_variant(DevMip const* mips, int numMips, int totalTiles, int gridSize, Fp8Handoff handoff, hipStream_t stream)
+static hipError_t launch_fp8_variant(MipTable const& mips, int numMips, int totalTiles, int gridSize, Fp8Handoff handoff, hipStream_t stream)
 {
     using One = Fp8Variant<FEATURES, true>;
     using Any = Fp8Variant<FEATURES, false>;
@@ -961,7 +963,7 @@ static hipError_t launch_fp8_variant(DevMip const* mips, int numMips, int totalT
     return hipGetLastError();
 }
 
-hipError_t launch_decode_fp8(int variant, DevMip const* mips, int numMips, int totalTiles, int gridSize, Fp8Handoff handoff, hipStream_t stream)
+hipError_t launch_decode_fp8(int variant, MipTable const& mips, int numMips, int totalTiles, int gridSize, Fp8Handoff handoff, hipStream_t stream)
 {
     switch (variant) {
     case NTC_HIP_VARIANT_REF16_FP8: return launch_fp8_variant<16>(mips, numMips, totalTiles, gridSize, handoff, stream);
@@ -973,7 +975,7 @@ hipError_t launch_decode_fp8(int variant, DevMip const* mips, int numMips, int t
 }
 
 template <int FEATURES>
-static hipError_t launch_fp8_query_variant(DevMip const* mips, int numMips, DevQuery const* queries, uint64_t numQueries, uint16_t* out, int gridSize, Fp8Handoff handoff, hipStream_t stream)
+static hipError_t launch_fp8_query_variant(MipTable const& mips, int numMips, DevQuery const* queries, uint64_t numQueries, uint16_t* out, int gridSize, Fp8Handoff handoff, hipStream_t stream)
 {
     using One = Fp8Variant<FEATURES, true>;
     using Any = Fp8Variant<FEATURES, false>;
@@ -984,7 +986,7 @@ static hipError_t launch_fp8_query_variant(DevMip const* mips, int numMips, DevQ
     return hipGetLastError();
 }
 
-hipError_t launch_queries_fp8(int variant, DevMip const* mips, int numMips, DevQuery const* queries, uint64_t numQueries,
+hipError_t launch_queries_fp8(int variant, MipTable const& mips, int numMips, DevQuery const* queries, uint64_t numQueries,
                               uint16_t* out, int gridSize, Fp8Handoff handoff, hipStream_t stream)
 {
     switch (variant) {

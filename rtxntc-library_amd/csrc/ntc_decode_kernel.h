@@ -55,6 +55,17 @@ struct DevMip {
     uint8_t const* lrBricks;
 };
 
+// The mip table of a launch.  Up to kInlineMips entries travel in the kernel's own arguments, where every wave reads
+// them as scalars: nothing to copy to the device in front of the launch and no device memory that successive calls
+// would have to hand on to each other.  (A table copied from pinned memory took a copy and an event record per call:
+// one 128 x 128 mip, another set each call: 16.3 us, 9.1 us with the table in the arguments.)  Longer tables
+// - batches of sets - lie in device memory at `entries`, which is null otherwise.
+constexpr int kInlineMips = 16;                            // one set with a full mip chain; 1 920 bytes of arguments
+struct MipTable {
+    DevMip inlined[kInlineMips];
+    DevMip const* entries;
+};
+
 // Brick geometry of a grid with `layers` u16 layers: log2 of the brick's side in cells.
 constexpr int brick_side_log2(int layers) { return layers == 1 ? 3 : 2; }
 constexpr int brick_bytes(int layers) { return (1 << (2 * brick_side_log2(layers))) * layers * 2; }
@@ -149,18 +160,18 @@ hipError_t launch_block_compress(BlockCompressArgs const& args, int dstFormat /*
 hipError_t launch_bc6_compress(BlockCompressArgs const& args, hipStream_t stream);
 hipError_t launch_bc7_compress(BlockCompressArgs const& args, hipStream_t stream);
 
-hipError_t launch_decode(int variant, DevMip const* mips, int numMips, int totalTiles, int gridSize, hipStream_t stream);
-hipError_t launch_queries(int variant, DevMip const* mips, int numMips, DevQuery const* queries, uint64_t numQueries,
+hipError_t launch_decode(int variant, MipTable const& mips, int numMips, int totalTiles, int gridSize, hipStream_t stream);
+hipError_t launch_queries(int variant, MipTable const& mips, int numMips, DevQuery const* queries, uint64_t numQueries,
                           uint16_t* out, int gridSize, hipStream_t stream);
 // The FP8 network is launched twice (weights of one plane per layer, then any weights); `word` is a dword of device
 // memory through which the first launch tells the second whether any set is left for it, `serial` a number the
 // caller changes with every pair of launches that shares the word.
 struct Fp8Handoff { uint32_t* word; uint32_t serial; };
-hipError_t launch_decode_fp8(int variant, DevMip const* mips, int numMips, int totalTiles, int gridSize, Fp8Handoff handoff, hipStream_t stream);
+hipError_t launch_decode_fp8(int variant, MipTable const& mips, int numMips, int totalTiles, int gridSize, Fp8Handoff handoff, hipStream_t stream);
 int resident_fp8_workgroups_per_cu();
 int fp8_tiles_per_round();               // tiles a workgroup of decode_fp8_kernel works on at a time
 int fp8_threads_per_workgroup();
-hipError_t launch_queries_fp8(int variant, DevMip const* mips, int numMips, DevQuery const* queries, uint64_t numQueries,
+hipError_t launch_queries_fp8(int variant, MipTable const& mips, int numMips, DevQuery const* queries, uint64_t numQueries,
                               uint16_t* out, int gridSize, Fp8Handoff handoff, hipStream_t stream);
 hipError_t launch_selftest_fp8_activation(uint16_t const* in, uint16_t* out, int n, hipStream_t stream);
 int resident_workgroups_per_cu(int variant);

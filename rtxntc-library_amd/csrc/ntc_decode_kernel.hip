@@ -1204,8 +1204,9 @@ __device__ __forceinline__ void mlp_forward_f16(LdsT<V>& lds, int wave, int lane
 // Two workgroups of eight waves per CU: sixteen waves, 128 VGPRs each, four to a SIMD.
 template <class V>
 __global__ void __launch_bounds__(V::THREADS, V::WAVES_PER_SIMD)
-decode_kernel(DevMip const* __restrict__ mips, int numMips, int totalTiles)
+decode_kernel(MipTable table, int numMips, int totalTiles)
 {
+    DevMip const* const mips = table_entries(table.entries);
     __shared__ LdsT<V> lds;
     constexpr int GROUP = V::WAVES / 4;                      // quartets of a workgroup
     int const lane = threadIdx.x & 63;
@@ -1340,9 +1341,10 @@ decode_kernel(DevMip const* __restrict__ mips, int numMips, int totalTiles)
 // A query whose mip is out of range writes zeros.
 template <class V>
 __global__ void __launch_bounds__(V::THREADS, V::WAVES_PER_SIMD)
-query_kernel(DevMip const* __restrict__ mips, int numMips, DevQuery const* __restrict__ queries, uint64_t numQueries,
+query_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queries, uint64_t numQueries,
              uint16_t* __restrict__ out)
 {
+    DevMip const* const mips = table_entries(table.entries);
     __shared__ LdsT<V> lds;
     __shared__ QueryMip qmips[16];
     if (threadIdx.x < 16) {
@@ -1493,13 +1495,13 @@ using VRef4   = Variant<0, 4, 4, 16, 4, 16, 2, 48, 64, 48, 32>;
 using VCfg3   = Variant<0, 16, 4, 16, 16, 16, 2, 48, 64, 64, 64, true>;   // wide decoder, e4m3 hidden-layer weights
 
 template <class V>
-static hipError_t launch_variant(DevMip const* mips, int numMips, int totalTiles, int gridSize, hipStream_t stream)
+static hipError_t launch_variant(MipTable const& mips, int numMips, int totalTiles, int gridSize, hipStream_t stream)
 {
     hipLaunchKernelGGL(decode_kernel<V>, dim3(gridSize), dim3(V::THREADS), 0, stream, mips, numMips, totalTiles);
     return hipGetLastError();
 }
 
-hipError_t launch_decode(int variant, DevMip const* mips, int numMips, int totalTiles, int gridSize, hipStream_t stream)
+hipError_t launch_decode(int variant, MipTable const& mips, int numMips, int totalTiles, int gridSize, hipStream_t stream)
 {
     switch (variant) {
     case NTC_HIP_VARIANT_CFG01: return launch_variant<VCfg01>(mips, numMips, totalTiles, gridSize, stream);
@@ -1514,7 +1516,7 @@ hipError_t launch_decode(int variant, DevMip const* mips, int numMips, int total
 }
 
 template <class V>
-static hipError_t launch_query_variant(DevMip const* mips, int numMips, DevQuery const* queries, uint64_t numQueries,
+static hipError_t launch_query_variant(MipTable const& mips, int numMips, DevQuery const* queries, uint64_t numQueries,
                                        uint16_t* out, int gridSize, hipStream_t stream)
 {
     hipLaunchKernelGGL(query_kernel<V>, dim3(gridSize), dim3(V::THREADS), 0, stream, mips, numMips, queries, numQueries, out);
@@ -1545,7 +1547,7 @@ hipError_t launch_build_bricks(uint16_t const* src, uint8_t* dst, int width, int
     return hipGetLastError();
 }
 
-hipError_t launch_queries(int variant, DevMip const* mips, int numMips, DevQuery const* queries, uint64_t numQueries,
+hipError_t launch_queries(int variant, MipTable const& mips, int numMips, DevQuery const* queries, uint64_t numQueries,
                           uint16_t* out, int gridSize, hipStream_t stream)
 {
     switch (variant) {

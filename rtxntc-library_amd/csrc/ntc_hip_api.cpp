@@ -88,7 +88,8 @@ struct NtcHipContext {
     struct Slot { DevMip* host = nullptr; size_t capacity = 0; hipEvent_t done = nullptr; bool inFlight = false; };
     Slot slots[kSlots];                // pinned staging for asynchronous table uploads
     int nextSlot = 0;
-    DevMip staticBuild[NTC_HIP_STATIC_TABLE_MIPS];   // where ntc_hip_decode_static assembles its table (it allocates nothing)
+    DevMip build[NTC_HIP_STATIC_TABLE_MIPS];   // where a call assembles its table: nothing is allocated per call
+    std::vector<DevMip> buildLonger;   // the table of a call with more entries than that
 };
 
 
@@ -271,38 +272,31 @@ bool plan_bricks(NtcHipTextureSet const& set, BrickPlan& plan)
     return true;
 }
 
-// Validates the sets, builds the mip table (sorted by tileStart) and picks the kernel.
-// Where build_table puts its entries: a vector, or (ntc_hip_decode_static, which may not allocate) a fixed array.
+// Where build_table puts its entries: the context's own array and, beyond its capacity, a vector (null: entries
+// beyond the capacity are counted, not stored).
 struct TableSink {
-    std::vector<DevMip>* vector = nullptr;
-    DevMip* fixed = nullptr;
-    size_t capacity = 0, count = 0;
-    void clear() { count = 0; if (vector) vector->clear(); }
+    DevMip* fixed;
+    size_t capacity;
+    std::vector<DevMip>* longer;
+    size_t count = 0;
+    TableSink(Library& L, bool unlimited) : fixed(L.build), capacity(NTC_HIP_STATIC_TABLE_MIPS), longer(unlimited ? &L.buildLonger : nullptr) {}
     void push_back(DevMip const& e)
     {
-        if (vector) vector->push_back(e);
-        else if (count < capacity) fixed[count] = e;
-        ++count;                                              // beyond the capacity entries are counted, not stored
+        if (count < capacity) {
+            fixed[count] = e;
+        } else if (longer) {
+            if (count == capacity) longer->assign(fixed, fixed + capacity);
+            longer->push_back(e);
+        }
+        ++count;
     }
+    DevMip const* entries() const { return count <= capacity ? fixed : longer->data(); }
 };
 
-int build_table(NtcHipTextureSet const* sets, int32_t numSets, TableSink table, size_t& entries, int& variant, int& totalTiles,
-                bool forQueries = false);
-int build_table(NtcHipTextureSet const* sets, int32_t numSets, std::vector<DevMip>& table, int& variant, int& totalTiles,
-                bool forQueries = false)
+// Validates the sets, builds the mip table (sorted by tileStart) and picks the kernel.
+int build_table(NtcHipTextureSet const* sets, int32_t numSets, TableSink& table, int& variant, int& totalTiles, bool forQueries = false)
 {
-    TableSink sink;
-    sink.vector = &table;
-    size_t entries = 0;
-    return build_table(sets, numSets, sink, entries, variant, totalTiles, forQueries);
-}
-
-int build_table(NtcHipTextureSet const* sets, int32_t numSets, TableSink table, size_t& entries, int& variant, int& totalTiles,
-                bool forQueries)
-{
-    entries = 0;
     if (!sets || numSets < 1) { set_error("ntc_hip_decode: no texture sets given."); return NTC_HIP_ERR_INVALID_ARG; }
-    table.clear();
     totalTiles = 0;
     for (int s = 0; s < numSets; ++s) {
         NtcHipTextureSet const& set = sets[s];
@@ -409,7 +403,6 @@ int build_table(NtcHipTextureSet const* sets, int32_t numSets, TableSink table, 
             table.push_back(e);
         }
     }
-    entries = table.count;
     variant = pick_variant(sets[0].spec);
     if (variant == NTC_HIP_VARIANT_NONE) {
         set_error("ntc_hip_decode: no compiled kernel covers this decoder spec "
@@ -423,17 +416,16 @@ int build_table(NtcHipTextureSet const* sets, int32_t numSets, TableSink table, 
     return 0;
 }
 
-// Makes the device table hold `table` (re-uploads only when it changed).  The copy is asynchronous
+// Makes the device table hold `count` entries (re-uploads only when they changed).  The copy is asynchronous
 // from one of a few pinned staging slots; a slot is reused only after the copy that last read it
 // has completed (its event), so back-to-back launches with different tables never wait on the GPU.
-int upload_table(Library& L, std::vector<DevMip> const& table)
+int upload_table(Library& L, DevMip const* table, size_t count)
 {
-    bool const same = L.lastTable.size() == table.size()
-        && std::memcmp(L.lastTable.data(), table.data(), table.size() * sizeof(DevMip)) == 0;
+    bool const same = L.lastTable.size() == count && std::memcmp(L.lastTable.data(), table, count * sizeof(DevMip)) == 0;
     if (same) return 0;
-    if (table.size() > L.tableCapacity) {
+    if (count > L.tableCapacity) {
         // The device table is read by kernels already queued on the stream: wait before replacing it.
-        size_t const cap = table.size() * 2 + 16;
+        size_t const cap = count * 2 + 16;
         HIP_TRY(hipStreamSynchronize(L.stream));
         if (L.tableDev) { HIP_TRY(hipFree(L.tableDev)); L.tableDev = nullptr; }
         L.tableCapacity = 0; L.lastTable.clear();
@@ -443,17 +435,30 @@ int upload_table(Library& L, std::vector<DevMip> const& table)
     Library::Slot& slot = L.slots[L.nextSlot];
     L.nextSlot = (L.nextSlot + 1) % Library::kSlots;
     if (slot.inFlight) { HIP_TRY(hipEventSynchronize(slot.done)); slot.inFlight = false; }
-    if (table.size() > slot.capacity) {
+    if (count > slot.capacity) {
         if (slot.host) { HIP_TRY(hipHostFree(slot.host)); slot.host = nullptr; slot.capacity = 0; }
         HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&slot.host), L.tableCapacity * sizeof(DevMip), hipHostMallocDefault));
         slot.capacity = L.tableCapacity;
     }
     if (!slot.done) HIP_TRY(hipEventCreateWithFlags(&slot.done, hipEventDisableTiming));
-    std::memcpy(slot.host, table.data(), table.size() * sizeof(DevMip));
-    HIP_TRY(hipMemcpyAsync(L.tableDev, slot.host, table.size() * sizeof(DevMip), hipMemcpyHostToDevice, L.stream));
+    std::memcpy(slot.host, table, count * sizeof(DevMip));
+    HIP_TRY(hipMemcpyAsync(L.tableDev, slot.host, count * sizeof(DevMip), hipMemcpyHostToDevice, L.stream));
     HIP_TRY(hipEventRecord(slot.done, L.stream));
     slot.inFlight = true;
-    L.lastTable = table;
+    L.lastTable.assign(table, table + count);
+    return 0;
+}
+
+// The table as a launch takes it: in the kernel's arguments while it fits there, else in the context's device table.
+int place_table(Library& L, TableSink const& sink, MipTable& table)
+{
+    table.entries = nullptr;
+    if (sink.count <= size_t(kInlineMips)) {
+        std::memcpy(table.inlined, sink.entries(), sink.count * sizeof(DevMip));
+        return 0;
+    }
+    if (int r = upload_table(L, sink.entries(), sink.count)) return r;
+    table.entries = L.tableDev;
     return 0;
 }
 
@@ -473,19 +478,21 @@ int grid_size_for(Library const& L, int variant, int totalTiles)
     return rounds < resident ? int(rounds) : resident;
 }
 
-// The hand-off word of a launch pair of the FP8 network over table `mips`: the context's own, or the one behind
-// the per-device table when that is the table (then nothing of the context's device memory is used).
-Fp8Handoff next_handoff(Library& L, DevMip const* mips)
+// The hand-off word of a launch pair of the FP8 network: the context's own or, for ntc_hip_decode_static (which uses
+// nothing of the context's device memory), the one behind the per-device table.
+Fp8Handoff next_handoff(Library& L, bool useStatic)
 {
-    uint32_t* const word = mips == L.staticTable
+    uint32_t* const word = useStatic
         ? reinterpret_cast<uint32_t*>(reinterpret_cast<unsigned char*>(L.staticTable) + kStaticTableBytes) : L.handoffDev;
     return Fp8Handoff{ word, ++L.handoffSerial };
 }
 
-hipError_t launch_decode_any(Library& L, int variant, DevMip const* mips, int numMips, int totalTiles, int gridSize)
+hipError_t launch_decode_any(Library& L, int variant, MipTable const& mips, size_t numMips, int totalTiles, bool useStatic = false)
 {
-    return variant_is_fp8_network(variant) ? launch_decode_fp8(variant, mips, numMips, totalTiles, gridSize, next_handoff(L, mips), L.stream)
-                                           : launch_decode(variant, mips, numMips, totalTiles, gridSize, L.stream);
+    int const gridSize = grid_size_for(L, variant, totalTiles);
+    return variant_is_fp8_network(variant)
+        ? launch_decode_fp8(variant, mips, int(numMips), totalTiles, gridSize, next_handoff(L, useStatic), L.stream)
+        : launch_decode(variant, mips, int(numMips), totalTiles, gridSize, L.stream);
 }
 
 } // namespace
@@ -706,11 +713,12 @@ uint64_t ntc_hip_grid_bytes(int32_t width, int32_t height, int32_t features, int
 int ntc_hip_ctx_decode(NtcHipContext* ctx, const NtcHipTextureSet* sets, int32_t numSets)
 {
     CTX_ENTER(ctx);
-    std::vector<DevMip> table;
+    TableSink sink(L, true);
+    MipTable table;
     int variant = NTC_HIP_VARIANT_NONE, totalTiles = 0;
-    if (int r = build_table(sets, numSets, table, variant, totalTiles)) return r;
-    if (int r = upload_table(L, table)) return r;
-    HIP_TRY(launch_decode_any(L, variant, L.tableDev, int(table.size()), totalTiles, grid_size_for(L, variant, totalTiles)));
+    if (int r = build_table(sets, numSets, sink, variant, totalTiles)) return r;
+    if (int r = place_table(L, sink, table)) return r;
+    HIP_TRY(launch_decode_any(L, variant, table, sink.count, totalTiles));
     clear_error();
     return 0;
 }
@@ -720,29 +728,32 @@ int ntc_hip_ctx_decode_static(NtcHipContext* ctx, const NtcHipTextureSet* sets, 
     CTX_ENTER(ctx);
     // No allocation on either side: the table is assembled in the context's own array (not in a vector) and
     // travels to the device as kernel arguments.
-    TableSink sink;
-    sink.fixed = L.staticBuild;
-    sink.capacity = size_t(kStaticTableEntries);
-    size_t entries = 0;
+    TableSink sink(L, false);
+    MipTable table;
     int variant = NTC_HIP_VARIANT_NONE, totalTiles = 0;
-    if (int r = build_table(sets, numSets, sink, entries, variant, totalTiles)) return r;
-    if (entries > size_t(kStaticTableEntries)) {
+    if (int r = build_table(sets, numSets, sink, variant, totalTiles)) return r;
+    if (sink.count > size_t(kStaticTableEntries)) {
         set_error("ntc_hip_decode_static: %zu mips in one call; the built-in table holds %d (use ntc_hip_decode).",
-                  entries, kStaticTableEntries);
+                  sink.count, kStaticTableEntries);
         return NTC_HIP_ERR_INVALID_ARG;
     }
-    // A chunk per launch, into this device's built-in array.  Stream order keeps a decode that still reads the
-    // previous table ahead of these stores.
-    for (size_t first = 0; first < entries; first += kTableChunkEntries) {
-        size_t const count = entries - first < size_t(kTableChunkEntries) ? entries - first : size_t(kTableChunkEntries);
-        TableChunk chunk;
-        std::memset(&chunk, 0, sizeof(chunk));
-        std::memcpy(chunk.entries, L.staticBuild + first, count * sizeof(DevMip));
-        write_table_kernel<<<1, 256, 0, L.stream>>>(reinterpret_cast<uint32_t*>(L.staticTable + first), chunk,
-                                                    int(count * sizeof(DevMip) / 4));
-        HIP_TRY(hipGetLastError());
+    if (sink.count <= size_t(kInlineMips)) {
+        if (int r = place_table(L, sink, table)) return r;
+    } else {
+        // A chunk per launch, into this device's built-in array.  Stream order keeps a decode that still reads the
+        // previous table ahead of these stores.
+        for (size_t first = 0; first < sink.count; first += kTableChunkEntries) {
+            size_t const count = sink.count - first < size_t(kTableChunkEntries) ? sink.count - first : size_t(kTableChunkEntries);
+            TableChunk chunk;
+            std::memset(&chunk, 0, sizeof(chunk));
+            std::memcpy(chunk.entries, L.build + first, count * sizeof(DevMip));
+            write_table_kernel<<<1, 256, 0, L.stream>>>(reinterpret_cast<uint32_t*>(L.staticTable + first), chunk,
+                                                        int(count * sizeof(DevMip) / 4));
+            HIP_TRY(hipGetLastError());
+        }
+        table.entries = L.staticTable;
     }
-    HIP_TRY(launch_decode_any(L, variant, L.staticTable, int(entries), totalTiles, grid_size_for(L, variant, totalTiles)));
+    HIP_TRY(launch_decode_any(L, variant, table, sink.count, totalTiles, true));
     clear_error();
     return 0;
 }
@@ -751,14 +762,14 @@ int ntc_hip_ctx_decode_timed(NtcHipContext* ctx, const NtcHipTextureSet* sets, i
 {
     CTX_ENTER(ctx);
     if (iterations < 1 || !outMs) { set_error("ntc_hip_decode_timed: iterations must be >= 1 and the result pointer non-null."); return NTC_HIP_ERR_INVALID_ARG; }
-    std::vector<DevMip> table;
+    TableSink sink(L, true);
+    MipTable table;
     int variant = NTC_HIP_VARIANT_NONE, totalTiles = 0;
-    if (int r = build_table(sets, numSets, table, variant, totalTiles)) return r;
-    if (int r = upload_table(L, table)) return r;
-    int const grid = grid_size_for(L, variant, totalTiles);
+    if (int r = build_table(sets, numSets, sink, variant, totalTiles)) return r;
+    if (int r = place_table(L, sink, table)) return r;
     HIP_TRY(hipEventRecord(L.evStart, L.stream));
     for (int i = 0; i < iterations; ++i)
-        HIP_TRY(launch_decode_any(L, variant, L.tableDev, int(table.size()), totalTiles, grid));
+        HIP_TRY(launch_decode_any(L, variant, table, sink.count, totalTiles));
     HIP_TRY(hipEventRecord(L.evStop, L.stream));
     HIP_TRY(hipEventSynchronize(L.evStop));
     float ms = 0.f;
@@ -799,20 +810,21 @@ static int run_queries(NtcHipContext* ctx, const NtcHipTextureSet* set, const Nt
     if (numQueries > (uint64_t(1) << 40)) { set_error("ntc_hip_decode_queries: too many queries in one call."); return NTC_HIP_ERR_INVALID_ARG; }
     if (outBytes < numQueries * 32u) { set_error("ntc_hip_decode_queries: the output buffer holds %llu bytes, %llu queries need %llu.", (unsigned long long)outBytes, (unsigned long long)numQueries, (unsigned long long)(numQueries * 32u)); return NTC_HIP_ERR_INVALID_ARG; }
     if ((reinterpret_cast<uintptr_t>(out) & 7u) || (reinterpret_cast<uintptr_t>(queries) & 3u)) { set_error("ntc_hip_decode_queries: output must be 8-byte and queries 4-byte aligned."); return NTC_HIP_ERR_INVALID_ARG; }
-    std::vector<DevMip> table;
+    TableSink sink(L, true);
+    MipTable table;
     int variant = NTC_HIP_VARIANT_NONE, totalTiles = 0;
-    if (int r = build_table(set, 1, table, variant, totalTiles, true)) return r;
+    if (int r = build_table(set, 1, sink, variant, totalTiles, true)) return r;
     bool const fp8 = variant_is_fp8_network(variant);
-    if (int r = upload_table(L, table)) return r;
+    if (int r = place_table(L, sink, table)) return r;
     uint64_t const perBlock = uint64_t(fp8 ? fp8_threads_per_workgroup() : threads_per_workgroup(variant));
     uint64_t const blocks = (numQueries + perBlock - 1) / perBlock;
     uint64_t const resident = uint64_t(L.computeUnits) * uint64_t(grid_size_for(L, variant, 0x7fffffff) / L.computeUnits);
     int const grid = int(blocks < resident ? blocks : resident);
     if (outMs) HIP_TRY(hipEventRecord(L.evStart, L.stream));
     for (int i = 0; i < iterations; ++i)
-        HIP_TRY(fp8 ? launch_queries_fp8(variant, L.tableDev, int(table.size()), reinterpret_cast<DevQuery const*>(queries), numQueries,
-                                         static_cast<uint16_t*>(out), grid, next_handoff(L, L.tableDev), L.stream)
-                    : launch_queries(variant, L.tableDev, int(table.size()), reinterpret_cast<DevQuery const*>(queries), numQueries,
+        HIP_TRY(fp8 ? launch_queries_fp8(variant, table, int(sink.count), reinterpret_cast<DevQuery const*>(queries), numQueries,
+                                         static_cast<uint16_t*>(out), grid, next_handoff(L, false), L.stream)
+                    : launch_queries(variant, table, int(sink.count), reinterpret_cast<DevQuery const*>(queries), numQueries,
                                      static_cast<uint16_t*>(out), grid, L.stream));
     if (outMs) {
         HIP_TRY(hipEventRecord(L.evStop, L.stream));

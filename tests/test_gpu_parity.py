@@ -377,6 +377,22 @@ def test_decode_is_idempotent_and_timed_variant_matches(ntc, device):
     assert np.array_equal(first, case.d_output.download())
 
 
+@pytest.mark.parametrize("sets", [1, 15, 16, 17, 33])
+@pytest.mark.parametrize("entry", ["decode", "decode_static"])
+def test_tables_in_and_beyond_the_kernel_arguments(ntc, device, sets, entry):
+    """One mip per set: tables of up to 16 entries travel in the kernel's arguments, longer ones lie in device memory."""
+    cases = [cfg_case(ntc, ntc.presets.spec_cfg2(), 24, 9, 1, 5, ntc.abi.OUT_UNORM8_PIXELS, seed=300 + s, scale_log2_range=ACTIVE)
+             for s in range(sets)]
+    dsets = [c.device_set(device) for c in cases]
+    for _ in range(2):
+        getattr(device, entry)(dsets)
+    device.synchronize()
+    for s, case in enumerate(cases):
+        host = case.host_set()
+        host.decode(threads=2)
+        assert_equal_bytes(host.output, case.d_output.download(), f"{entry}, set {s} of {sets}")
+
+
 def test_timer_spans_the_calls_between_its_two_ends(ntc, device):
     """ntc_hip_timer_begin / _end: device time of whatever was queued between them.  A span around five decodes is
     at least as long as five decodes timed back to back by ntc_hip_decode_timed (it also holds the table uploads
