@@ -7,6 +7,8 @@
 // HBM-bound: 2 bytes read and 1-4 bytes written per channel.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <atomic>
+#include <type_traits>
 #include "ntc_decode_kernel.h"
 
 namespace ntc_hip_dev {
@@ -44,9 +46,96 @@ __device__ __forceinline__ float encode_color_space(int colorSpace, float v)
     return v;
 }
 
+// ---- the transfer functions of stored values, by table -----------------------------------------------
+//
+// What the copies convert is a half (the internal layout, FLOAT16 images) or a UNORM code: a function of 16 bits, so
+// encode(dst, decode(src, value)) is tabulated for the eight pairs of colour spaces that change a value, by the
+// device functions above (same bits), once per device when its first context is created.  A powf costs some seventy
+// vector instructions, sRGB to sRGB takes two of them and two divisions per channel: 2048 x 2048 sRGB pixels of 8
+// bits, dithered, took 103 us to read that way and 91 us to write.
+//
+// With the tables (and the groups of four pixels below) they take 23 and 16 us.
+//
+// The floats of the halves in [1/64, 1], which is nearly everything a texture holds, are copied into LDS by launches
+// large enough to pay for it; other halves are read from the table in memory (256 KB a pair, cached).
+constexpr int kTransferPairs = 8;                            // src * 3 + dst - 1; linear to linear has no table
+constexpr uint32_t kStageFirst = 0x2400u, kStageCount = 0x1801u;     // halves 1/64 .. 1
+static __device__ float transferOfHalf[kTransferPairs][65536];
+static __device__ uint16_t storedOfUnorm16[kTransferPairs][65536];   // UNORM16 code -> half of the internal layout
+static __device__ uint16_t storedOfUnorm8[kTransferPairs + 1][256];  // UNORM8 code -> half; [8]: linear
+
+__device__ __forceinline__ uint16_t stored_half(float v)     // WriteImageChannel FLOAT16, src/ImageProcessing.cu:154-156
+{
+    v = fmaxf(-65504.f, fminf(65504.f, v));
+    asm volatile("" : "+v"(v));
+    return __builtin_bit_cast(uint16_t, (_Float16)v);
+}
+
+__global__ void __launch_bounds__(256)
+transfer_tables_kernel()
+{
+    int const pair = blockIdx.y, src = pair == kTransferPairs ? 0 : (pair + 1) / 3, dst = pair == kTransferPairs ? 0 : (pair + 1) % 3;
+    uint32_t const i = blockIdx.x * 256u + threadIdx.x;      // 65536 values
+    auto transfer = [&](float v) { return encode_color_space(dst, decode_color_space(src, v)); };
+    if (pair < kTransferPairs) {
+        transferOfHalf[pair][i] = transfer(float(__builtin_bit_cast(_Float16, uint16_t(i))));
+        storedOfUnorm16[pair][i] = stored_half(transfer(float(i) / 65535.f));
+    }
+    if (i < 256u) storedOfUnorm8[pair][i] = stored_half(transfer(float(i) / 255.f));
+}
+
+hipError_t launch_transfer_tables(hipStream_t stream)
+{
+    hipLaunchKernelGGL(transfer_tables_kernel, dim3(256, kTransferPairs + 1), dim3(256), 0, stream);
+    return hipGetLastError();
+}
+
+__host__ __device__ __forceinline__ int transfer_pair(int src, int dst) { return src * 3 + dst - 1; }     // -1: linear to linear
+
+// encode(dst, decode(src, half)) for a channel of the pair of colour spaces `pair` (uniform).
+__device__ __forceinline__ float transfer_half(int pair, uint32_t bits)
+{
+    return pair < 0 ? float(__builtin_bit_cast(_Float16, uint16_t(bits))) : transferOfHalf[pair][bits];
+}
+// The same for four pixels' halves of one channel through the copies in LDS: slot 1 or 2 (uniform) names the copy that
+// holds the pair, 0 none.  (The look-up in LDS happens for every half, out-of-range ones clamped: a choice between the
+// two tables per half would become a choice of address and a flat load.)
+__device__ __forceinline__ void transfer_halves(float const* staged, int slot, int pair, uint32_t const (&bits)[4], float (&value)[4])
+{
+    if (pair < 0) {                                          // uniform
+#pragma unroll
+        for (int k = 0; k < 4; ++k) value[k] = float(__builtin_bit_cast(_Float16, uint16_t(bits[k])));
+    } else if (slot == 0) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) value[k] = transferOfHalf[pair][bits[k]];
+    } else {
+        float const* const copy = staged + (slot - 1) * int(kStageCount);
+        uint32_t at[4];
+        bool beyond = false;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            at[k] = bits[k] - kStageFirst;
+            value[k] = copy[min(at[k], kStageCount - 1u)];
+            beyond |= at[k] >= kStageCount;
+        }
+        if (beyond) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) if (at[k] >= kStageCount) value[k] = transferOfHalf[pair][bits[k]];
+        }
+    }
+}
+// a / b for b = 255 or 65535 and every a that occurs here (codes, dither draws): the product with the reciprocal
+// corrected by its remainder is the correctly rounded quotient for all of them (checked exhaustively).
+__device__ __forceinline__ float divide_by_top(float a, float top, float reciprocal)
+{
+    float const q = a * reciprocal;
+    return __builtin_fmaf(__builtin_fmaf(-q, top, a), reciprocal, q);
+}
+
 // HashBasedRNG, src/CudaUtils.h:117-184: Jenkins hash of the pixel index seeds a Murmur3 round per draw.
 struct DitherRng {
     uint32_t seed, index;
+    __device__ DitherRng() {}
     __device__ explicit DitherRng(uint32_t linearIndex) : index(1)
     {
         uint32_t a = linearIndex;
@@ -93,26 +182,29 @@ inline dim3 copy_grid(int width, int height, int& xShift, bool wide = true)
     return dim3((width + (1 << xShift) - 1) >> xShift, (height + rows - 1) / rows);
 }
 
-// WriteImageChannel (src/ImageProcessing.cu:141-164): the channel's bits in the destination format.
+// WriteImageChannel (src/ImageProcessing.cu:141-164): the bits, in the destination format, of a channel whose
+// value is in the destination's colour space already.
 template <int FORMAT>
-__device__ __forceinline__ uint32_t encode_channel(int colorSpace, float value, bool dithering, float dither)
+__device__ __forceinline__ uint32_t encode_value(float value, bool dithering, float dither)
 {
-    value = encode_color_space(colorSpace, value);
     if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_UNORM8) {
-        if (dithering) value += dither / 255.f;
+        if (dithering) value += divide_by_top(dither, 255.f, 1.f / 255.f);
         return unorm_code(value * 255.f, 255.f);
     } else if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_UNORM16) {
-        if (dithering) value += dither / 65535.f;
+        if (dithering) value += divide_by_top(dither, 65535.f, 1.f / 65535.f);
         return unorm_code(value * 65535.f, 65535.f);
     } else if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_FLOAT16) {
-        float v = fmaxf(-65504.f, fminf(65504.f, value));
-        asm volatile("" : "+v"(v));                          // round the clamped value, not a fused expression
-        return uint32_t(__builtin_bit_cast(uint16_t, (_Float16)v));
+        return stored_half(value);
     } else if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_FLOAT32) {
         return __builtin_bit_cast(uint32_t, value);
     } else {
         return uint32_t(fmaxf(value, 0.f));
     }
+}
+template <int FORMAT>
+__device__ __forceinline__ uint32_t encode_channel(int colorSpace, float value, bool dithering, float dither)
+{
+    return encode_value<FORMAT>(encode_color_space(colorSpace, value), dithering, dither);
 }
 
 // One lane per pixel.  All the half2 pairs the pixel needs are loaded before any arithmetic (the
@@ -157,17 +249,17 @@ read_channels_kernel(ReadChannelsArgs a)
             float value;
             if (ch < a.numChannels) {
                 uint32_t const bits = odd ? half_of(ch + 1) : half_of(ch);
-                value = float(__builtin_bit_cast(_Float16, uint16_t(bits)));
-                if constexpr (!PLAIN) value = decode_color_space(a.srcColorSpaces[ch], value);
+                value = transfer_half(PLAIN ? -1 : transfer_pair(a.srcColorSpaces[ch], a.dstColorSpaces[ch]), bits);
             } else {
                 value = (ch == 3) ? 1.f : 0.f;               // GetDefaultChannelValue, src/ImageProcessing.cu:166-170
+                if constexpr (!PLAIN) value = encode_color_space(a.dstColorSpaces[ch], value);
             }
             uint32_t bits;
             if constexpr (PLAIN) {
-                bits = encode_channel<FORMAT>(0, value, false, 0.f);
+                bits = encode_value<FORMAT>(value, false, 0.f);
             } else {
                 float const dither = a.useDithering ? rng.next_float() - 0.5f : 0.f;  // one draw per destination channel
-                bits = encode_channel<FORMAT>(a.dstColorSpaces[ch], value, a.useDithering != 0, dither);
+                bits = encode_value<FORMAT>(value, a.useDithering != 0, dither);
             }
             words[(k * BPC) >> 2] |= bits << (8 * ((k * BPC) & 3));
         }
@@ -201,6 +293,190 @@ read_channels_kernel(ReadChannelsArgs a)
     }
 }
 
+// ---- small pixels: four at a time ---------------------------------------------------------------------
+//
+// Images of at most eight bytes a pixel: a lane takes four adjacent pixels, so that it reads 16 bytes of each channel
+// pair and writes its pixels as whole dwords.  (One pixel a lane, the kernel above, moved 5 bytes per lane for a
+// single-channel 8-bit image and took 16.5 us for 2048 x 2048 of it, five times what its bytes take.)  The lanes of a
+// wave cover 64, 32, 16 or 8 such groups of a row, whatever is the least that covers the row.  Accesses are whole
+// vectors at whatever alignment the image has; the last group of a row that is no multiple of four goes pixel by pixel.
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t u32_any   __attribute__((aligned(1)));
+typedef uint32_t u32x4_a4  __attribute__((ext_vector_type(4), aligned(4)));
+
+// Which pixels a lane works on: tiles of lanesX groups by threads / lanesX rows, a workgroup takes tiles
+// blockIdx.x, blockIdx.x + gridDim.x, ...
+struct GroupGrid { int32_t log2LanesX, tilesX, tiles; };
+
+static int compute_units_of_current_device()
+{
+    static std::atomic<int> units[64];
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess) return 256;
+    int n = units[device & 63].load(std::memory_order_relaxed);
+    if (n == 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n < 1) n = 256;
+        units[device & 63].store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
+
+static GroupGrid group_grid(int width, int height, int threads)
+{
+    GroupGrid g;
+    int const groups = (width + 3) / 4;
+    g.log2LanesX = groups > 32 ? 6 : groups > 16 ? 5 : groups > 8 ? 4 : 3;
+    int const rows = threads >> g.log2LanesX;
+    g.tilesX = (groups + (1 << g.log2LanesX) - 1) >> g.log2LanesX;
+    g.tiles = g.tilesX * ((height + rows - 1) / rows);
+    return g;
+}
+
+// The tables that a launch copies into LDS: the first two pairs of colour spaces that its channels use.
+struct StagedTransfers {
+    int32_t count;                                           // 0: nothing staged
+    int8_t staged[2];                                        // the pairs
+    int8_t pair[8], slot[8];                                 // per channel: its pair (-1 linear) and the copy that holds it (0 none)
+};
+
+// Launch shape of the group kernels.  Images of two million pixels and more stage: workgroups of 1024 threads, two to
+// a compute unit, that share a copy among two tiles or more each (2048 x 2048 read as dithered sRGB: 22.9 us, 24.4 with
+// 512 threads, 28 with 256, 24.8 straight from the table in memory; HLG to linear halves: 19.6, 23.4, 22.6, 24.5).
+// Smaller images, and those of linear channels, take small workgroups, a tile each.
+struct GroupLaunch {
+    GroupGrid grid;
+    StagedTransfers transfers;
+    unsigned blocks, threads, ldsBytes;
+};
+
+static GroupLaunch plan_groups(int width, int height, uint8_t const* src, uint8_t const* dst, int channels, bool readsHalves)
+{
+    constexpr int kStagingThreads = 1024, kSmallThreads = 256, kTilesPerStaging = 2;
+    GroupLaunch l{};
+    StagedTransfers& s = l.transfers;
+    int const units = compute_units_of_current_device();
+    l.grid = group_grid(width, height, kStagingThreads);
+    bool const stage = readsHalves && l.grid.tiles >= kTilesPerStaging * units;
+    for (int c = 0; c < 8; ++c) {
+        s.pair[c] = c < channels ? int8_t(transfer_pair(src[c], dst[c])) : int8_t(-1);
+        if (s.pair[c] < 0 || !stage) continue;
+        for (int k = 0; k < s.count; ++k) if (s.staged[k] == s.pair[c]) s.slot[c] = int8_t(k + 1);
+        if (s.slot[c] == 0 && s.count < 2) { s.staged[s.count] = s.pair[c]; s.slot[c] = int8_t(++s.count); }
+    }
+    if (s.count) {
+        int const share = (l.grid.tiles + kTilesPerStaging - 1) / kTilesPerStaging;
+        l.threads = kStagingThreads;
+        l.blocks = unsigned(2 * units < share ? 2 * units : share);
+        l.ldsBytes = unsigned(s.count * kStageCount * sizeof(float));
+    } else {
+        l.grid = group_grid(width, height, kSmallThreads);
+        l.threads = kSmallThreads;
+        l.blocks = unsigned(l.grid.tiles);
+    }
+    return l;
+}
+
+__device__ __forceinline__ void copy_staged(StagedTransfers const& s, float* lds)
+{
+    for (int k = 0; k < s.count; ++k) {
+        float const* const from = &transferOfHalf[s.staged[k]][kStageFirst];
+        for (uint32_t i = threadIdx.x; i < kStageCount; i += blockDim.x) lds[k * int(kStageCount) + int(i)] = from[i];
+    }
+    if (s.count) __syncthreads();
+}
+
+struct ReadGroupsArgs { ReadChannelsArgs a; GroupGrid grid; StagedTransfers transfers; };
+
+// CHANNELS = channels of a destination pixel.
+template <int FORMAT, int CHANNELS, bool DITHER>
+__global__ void __launch_bounds__(1024)
+read_groups_kernel(ReadGroupsArgs args)
+{
+    constexpr int BPC = bytes_per_channel(FORMAT), PIXEL = CHANNELS * BPC, PAIRS = CHANNELS / 2 + 1;
+    static_assert(PIXEL <= 8, "the words of four pixels stay in registers");
+    extern __shared__ float staged[];
+    ReadChannelsArgs const& a = args.a;
+    copy_staged(args.transfers, staged);
+    int const lanesX = 1 << args.grid.log2LanesX;
+    int const lx = int(threadIdx.x) & (lanesX - 1), ly = int(threadIdx.x) >> args.grid.log2LanesX;
+    int const firstPair = a.firstChannel >> 1;
+    bool const odd = (a.firstChannel & 1) != 0;
+    int const copied = min(a.numChannels, CHANNELS);
+    int const pairs = ((a.firstChannel + copied + 1) >> 1) - firstPair;      // at most PAIRS
+    for (int tile = blockIdx.x; tile < args.grid.tiles; tile += gridDim.x) {
+        int const tileY = tile / args.grid.tilesX, tileX = tile - tileY * args.grid.tilesX;
+        int const x = (tileX * lanesX + lx) * 4, y = tileY * int(blockDim.x >> args.grid.log2LanesX) + ly;
+        if (x >= a.width || y >= a.height) continue;
+        bool const whole = x + 4 <= a.width;
+        uint16_t const* const src = a.planarPairs + size_t(y) * size_t(a.width) * size_t(a.setChannels) + size_t(x) * 2;
+        uint32_t pr[PAIRS][4];
+#pragma unroll
+        for (int p = 0; p < PAIRS; ++p) {
+            uint32_t const* const from = reinterpret_cast<uint32_t const*>(src + size_t(2 * (firstPair + min(p, pairs - 1))) * size_t(a.width));
+            if (whole) {
+                u32x4_a4 const v = *reinterpret_cast<u32x4_a4 const*>(from);
+                pr[p][0] = v[0]; pr[p][1] = v[1]; pr[p][2] = v[2]; pr[p][3] = v[3];
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) pr[p][k] = from[min(k, a.width - 1 - x)];
+            }
+        }
+        uint32_t words[PIXEL];                               // four pixels
+#pragma unroll
+        for (int w = 0; w < PIXEL; ++w) words[w] = 0u;
+        uint32_t const index = uint32_t(x) + uint32_t(y) * uint32_t(a.width);
+[[maybe_unused]] DitherRng rng[4];                   // one draw per pixel and destination channel, in channel order
+        if constexpr (DITHER) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) rng[k] = DitherRng(index + uint32_t(k));
+        }
+#pragma unroll
+        for (int ch = 0; ch < CHANNELS; ++ch) {
+            float value[4];
+            if (ch < copied) {                               // uniform
+                uint32_t bits[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    uint32_t const even = (ch & 1) ? pr[ch >> 1][k] >> 16 : pr[ch >> 1][k] & 0xffffu;
+                    uint32_t const next = (ch & 1) ? pr[(ch >> 1) + 1][k] & 0xffffu : pr[ch >> 1][k] >> 16;
+                    bits[k] = odd ? next : even;
+                }
+                transfer_halves(staged, args.transfers.slot[ch], args.transfers.pair[ch], bits, value);
+            } else {                                         // GetDefaultChannelValue; 0 is 0 in every colour space
+                float const fill = (ch == 3) ? encode_color_space(a.dstColorSpaces[ch], 1.f) : 0.f;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) value[k] = fill;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                float const dither = DITHER ? rng[k].next_float() - 0.5f : 0.f;
+                uint32_t const bits = encode_value<FORMAT>(value[k], DITHER, dither);
+                int const at = k * PIXEL + ch * BPC;         // byte of the group
+                words[at >> 2] |= BPC == 4 ? bits : bits << (8 * (at & 3));
+            }
+        }
+        uint8_t* const out = a.dst + size_t(y) * a.rowPitch + size_t(x) * PIXEL;
+        if (whole) {
+constexpr int FOURS = PIXEL & ~3, TWOS = FOURS + (PIXEL & 2);
+#pragma unroll
+            for (int w = 0; w < FOURS; w += 4)
+                *reinterpret_cast<u32x4_any*>(out + 4 * w) = u32x4_any{ words[w], words[w + 1], words[w + 2], words[w + 3] };
+            if constexpr ((PIXEL & 2) != 0) *reinterpret_cast<u32x2_any*>(out + 4 * FOURS) = u32x2_any{ words[FOURS], words[FOURS + 1] };
+            if constexpr ((PIXEL & 1) != 0) *reinterpret_cast<u32_any*>(out + 4 * TWOS) = words[TWOS];
+        } else {
+#pragma unroll
+            for (int b = 0; b < 4 * PIXEL; b += BPC) {
+                if (x + b / PIXEL >= a.width) continue;
+                uint32_t const bits = words[b >> 2] >> (8 * (b & 3));
+                if constexpr (BPC == 1)      out[b] = uint8_t(bits);
+                else if constexpr (BPC == 2) *reinterpret_cast<uint16_t*>(out + b) = uint16_t(bits);
+                else                         *reinterpret_cast<uint32_t*>(out + b) = bits;
+            }
+        }
+    }
+}
+
 // ReadImageChannel, src/ImageProcessing.cu:113-139: channel k of a 16-byte piece of the pixel.
 template <int FORMAT>
 __device__ __forceinline__ float decode_channel(uint32_t const (&words)[4], int k, float const* unorm8Table)
@@ -214,6 +490,137 @@ __device__ __forceinline__ float decode_channel(uint32_t const (&words)[4], int 
     else                                                     return float(w);
 }
 
+// The half of the internal layout that a channel of the user image becomes: its bits (upper bits are ignored by the
+// narrow formats) through both colour spaces (uniform).
+template <int FORMAT>
+__device__ __forceinline__ uint32_t stored_half_of(uint32_t bits, int srcSpace, int dstSpace)
+{
+    int const pair = transfer_pair(srcSpace, dstSpace);
+    if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_UNORM8) {
+        return storedOfUnorm8[pair < 0 ? kTransferPairs : pair][bits & 0xffu];
+    } else if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_UNORM16) {
+        return pair < 0 ? stored_half(divide_by_top(float(bits & 0xffffu), 65535.f, 1.f / 65535.f)) : storedOfUnorm16[pair][bits & 0xffffu];
+    } else if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_FLOAT16) {
+        return stored_half(transfer_half(pair, bits & 0xffffu));
+    } else {
+        float const v = FORMAT == NTC_HIP_DEV_FORMAT_FLOAT32 ? __builtin_bit_cast(float, bits) : float(bits);
+        return stored_half(pair < 0 ? v : encode_color_space(dstSpace, decode_color_space(srcSpace, v)));
+    }
+}
+
+struct WriteGroupsArgs { WriteChannelsArgs a; GroupGrid grid; StagedTransfers transfers; };
+
+// Four pixels of at most eight bytes a lane, like read_groups_kernel the other way round: whole dwords of the pixels
+// in, 16 bytes of each complete channel pair out (2048 x 2048 of 8 bits: RGBA 16 us, with sRGB 91 before the tables; one
+// channel 11 us, 15 before, of which the 2-byte stores into half a pair are the larger part; HLG halves 21 us, 29
+// before); where the image has only one channel of a pair, its halves go out
+// one by one between those of the other.  CHANNELS = channels of a source pixel, of which a.numChannels are stored.
+// 8-bit codes become halves through a table in LDS, a row of 256 per channel.
+template <int FORMAT, int CHANNELS>
+__global__ void __launch_bounds__(1024)
+write_groups_kernel(WriteGroupsArgs args)
+{
+    constexpr int BPC = bytes_per_channel(FORMAT), PIXEL = CHANNELS * BPC, PAIRS = CHANNELS / 2 + 1;
+    constexpr bool CODES = FORMAT == NTC_HIP_DEV_FORMAT_UNORM8, HALVES = FORMAT == NTC_HIP_DEV_FORMAT_FLOAT16;
+    static_assert(PIXEL <= 8, "the words of four pixels stay in registers");
+    __shared__ uint16_t codes[CODES ? CHANNELS : 1][256];
+    extern __shared__ float staged[];
+    WriteChannelsArgs const& a = args.a;
+    if constexpr (CODES) {
+        for (int i = threadIdx.x; i < CHANNELS * 256; i += blockDim.x) {
+            int const ch = i >> 8, pair = transfer_pair(a.srcColorSpaces[ch], a.dstColorSpaces[ch]);
+            codes[ch][i & 255] = storedOfUnorm8[pair < 0 ? kTransferPairs : pair][i & 255];
+        }
+        __syncthreads();
+    }
+    if constexpr (HALVES) copy_staged(args.transfers, staged);
+    int const lanesX = 1 << args.grid.log2LanesX;
+    int const lx = int(threadIdx.x) & (lanesX - 1), ly = int(threadIdx.x) >> args.grid.log2LanesX;
+    int const odd = a.firstChannel & 1;
+    for (int tile = blockIdx.x; tile < args.grid.tiles; tile += gridDim.x) {
+        int const tileY = tile / args.grid.tilesX, tileX = tile - tileY * args.grid.tilesX;
+        int const x = (tileX * lanesX + lx) * 4, y = tileY * int(blockDim.x >> args.grid.log2LanesX) + ly;
+        if (x >= a.width || y >= a.height) continue;
+        bool const whole = x + 4 <= a.width;
+        uint8_t const* const in = a.src + size_t(a.verticalFlip ? a.height - 1 - y : y) * a.rowPitch + size_t(x) * PIXEL;
+        uint32_t words[PIXEL];
+        if (whole) {
+            constexpr int FOURS = PIXEL & ~3, TWOS = FOURS + (PIXEL & 2);
+#pragma unroll
+            for (int w = 0; w < FOURS; w += 4) {
+                u32x4_any const v = *reinterpret_cast<u32x4_any const*>(in + 4 * w);
+                words[w] = v[0]; words[w + 1] = v[1]; words[w + 2] = v[2]; words[w + 3] = v[3];
+            }
+            if constexpr ((PIXEL & 2) != 0) {
+                u32x2_any const v = *reinterpret_cast<u32x2_any const*>(in + 4 * FOURS);
+                words[FOURS] = v[0]; words[FOURS + 1] = v[1];
+            }
+            if constexpr ((PIXEL & 1) != 0) words[TWOS] = *reinterpret_cast<u32_any const*>(in + 4 * TWOS);
+        } else {
+#pragma unroll
+            for (int w = 0; w < PIXEL; ++w) words[w] = 0u;
+#pragma unroll
+            for (int b = 0; b < 4 * PIXEL; b += BPC) {
+                if (x + b / PIXEL >= a.width) continue;
+                if constexpr (BPC == 1)      words[b >> 2] |= uint32_t(in[b]) << (8 * (b & 3));
+                else if constexpr (BPC == 2) words[b >> 2] |= uint32_t(*reinterpret_cast<uint16_t const*>(in + b)) << (8 * (b & 3));
+                else                         words[b >> 2] = *reinterpret_cast<uint32_t const*>(in + b);
+            }
+        }
+        uint32_t half[CHANNELS][4];
+#pragma unroll
+        for (int ch = 0; ch < CHANNELS; ++ch) {
+            uint32_t bits[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                int const at = k * PIXEL + ch * BPC;         // byte of the group
+                bits[k] = words[at >> 2] >> (8 * (at & 3));
+                if constexpr (BPC == 1) bits[k] &= 0xffu;
+                if constexpr (BPC == 2) bits[k] &= 0xffffu;
+            }
+            if constexpr (CODES) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) half[ch][k] = codes[ch][bits[k]];
+            } else if constexpr (HALVES) {
+                float value[4];
+                transfer_halves(staged, args.transfers.slot[ch], args.transfers.pair[ch], bits, value);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) half[ch][k] = stored_half(value[k]);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) half[ch][k] = stored_half_of<FORMAT>(bits[k], a.srcColorSpaces[ch], a.dstColorSpaces[ch]);
+            }
+        }
+        uint16_t* const dst = a.planarPairs + size_t(y) * size_t(a.width) * size_t(a.setChannels) + size_t(x) * 2;
+#pragma unroll
+        for (int p = 0; p < PAIRS; ++p) {
+            int const lower = 2 * p - odd;                   // the image's channel in the pair's first half, lower + 1 in its second
+            if (lower >= a.numChannels) continue;            // uniform, and so is everything about p
+            uint16_t* const to = dst + size_t((a.firstChannel & ~1) + 2 * p) * size_t(a.width);
+            bool const hasLower = lower >= 0, hasUpper = lower + 1 < a.numChannels;
+            uint32_t pair[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                uint32_t const even = 2 * p < CHANNELS ? half[2 * p < CHANNELS ? 2 * p : 0][k] : 0u, before = p > 0 ? half[p > 0 ? 2 * p - 1 : 0][k] : 0u;
+                uint32_t const after = 2 * p + 1 < CHANNELS ? half[2 * p + 1 < CHANNELS ? 2 * p + 1 : 0][k] : 0u;
+                pair[k] = odd ? before | (even << 16) : even | (after << 16);
+            }
+            if (hasLower && hasUpper) {
+                if (whole) {
+                    *reinterpret_cast<u32x4_a4*>(to) = u32x4_a4{ pair[0], pair[1], pair[2], pair[3] };
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) if (x + k < a.width) *reinterpret_cast<uint32_t*>(to + 2 * k) = pair[k];
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (whole || x + k < a.width) to[2 * k + (hasLower ? 0 : 1)] = uint16_t(hasLower ? pair[k] : pair[k] >> 16);
+            }
+        }
+    }
+}
+
 // User image -> internal fp16 planar pairs: ITextureSet::WriteChannels through CopyImageKernel's 1:1
 // branch (src/TextureSet.cpp:835-913, src/ImageProcessing.cu:220-265), optional vertical flip.
 // The pixel is read 16 bytes at a time with the widest loads its alignment allows; channel pairs
@@ -224,7 +631,7 @@ write_channels_kernel(WriteChannelsArgs a)
 {
     constexpr int BPC = bytes_per_channel(FORMAT), PER = 16 / BPC;
     __shared__ float unorm8Table[FORMAT == NTC_HIP_DEV_FORMAT_UNORM8 ? 256 : 1];
-    if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_UNORM8) {     // one correctly rounded division per code instead of per channel
+    if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_UNORM8 && PLAIN) {     // one correctly rounded division per code instead of per channel
         unorm8Table[threadIdx.x & 255] = float(threadIdx.x & 255) / 255.f;
         __syncthreads();
     }
@@ -258,11 +665,9 @@ write_channels_kernel(WriteChannelsArgs a)
         for (int k = 0; k < PER; ++k) {
             int const ch = base + k;
             if (ch >= a.numChannels) continue;                       // uniform
-            float v = decode_channel<FORMAT>(words, k, unorm8Table);
-            if constexpr (!PLAIN) v = encode_color_space(a.dstColorSpaces[ch], decode_color_space(a.srcColorSpaces[ch], v));
-            v = fmaxf(-65504.f, fminf(65504.f, v));                  // WriteImageChannel FLOAT16, src/ImageProcessing.cu:154-156
-            asm volatile("" : "+v"(v));
-            uint32_t const half = __builtin_bit_cast(uint16_t, (_Float16)v);
+            uint32_t half;
+            if constexpr (PLAIN) half = stored_half(decode_channel<FORMAT>(words, k, unorm8Table));
+            else                 half = stored_half_of<FORMAT>(words[(k * BPC) >> 2] >> (8 * ((k * BPC) & 3)), a.srcColorSpaces[ch], a.dstColorSpaces[ch]);
             int const c = a.firstChannel + ch;
             uint16_t* const to = dst + size_t(c & ~1) * size_t(a.width);
             if ((c & 1) == 0) {
@@ -323,13 +728,6 @@ __device__ __forceinline__ float user_channel(uint8_t const* px, int format, int
     case NTC_HIP_DEV_FORMAT_FLOAT32: return reinterpret_cast<float const*>(px)[k];
     default:                         return float(reinterpret_cast<uint32_t const*>(px)[k]);
     }
-}
-
-__device__ __forceinline__ uint16_t stored_half(float v)     // WriteImageChannel FLOAT16, src/ImageProcessing.cu:154-156
-{
-    v = fmaxf(-65504.f, fminf(65504.f, v));
-    asm volatile("" : "+v"(v));
-    return __builtin_bit_cast(uint16_t, (_Float16)v);
 }
 
 template <int FORMAT>
@@ -434,6 +832,49 @@ static bool plain_copy(uint8_t const* srcSpaces, uint8_t const* dstSpaces, int u
 }
 
 template <int FORMAT>
+static hipError_t launch_write_groups_of(WriteGroupsArgs const& args, GroupLaunch const& plan, hipStream_t stream)
+{
+    auto launch = [&](auto channels) {
+        constexpr int CHANNELS = decltype(channels)::value;
+        if constexpr (CHANNELS * bytes_per_channel(FORMAT) <= 8)
+            hipLaunchKernelGGL((write_groups_kernel<FORMAT, CHANNELS>), dim3(plan.blocks), dim3(plan.threads), plan.ldsBytes, stream, args);
+    };
+    switch (int(args.a.pixelStride) / bytes_per_channel(FORMAT)) {
+    case 1: launch(std::integral_constant<int, 1>{}); break;
+    case 2: launch(std::integral_constant<int, 2>{}); break;
+    case 3: launch(std::integral_constant<int, 3>{}); break;
+    case 4: launch(std::integral_constant<int, 4>{}); break;
+    case 5: launch(std::integral_constant<int, 5>{}); break;
+    case 6: launch(std::integral_constant<int, 6>{}); break;
+    case 7: launch(std::integral_constant<int, 7>{}); break;
+    case 8: launch(std::integral_constant<int, 8>{}); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+static hipError_t launch_write_groups(WriteChannelsArgs const& a, hipStream_t stream)
+{
+    WriteGroupsArgs args{};
+    args.a = a;
+    GroupLaunch plan = plan_groups(a.width, a.height, a.srcColorSpaces, a.dstColorSpaces, a.numChannels, a.format == NTC_HIP_DEV_FORMAT_FLOAT16);
+    if (a.format == NTC_HIP_DEV_FORMAT_UNORM8) {             // a workgroup fills its table once for all of its tiles
+        unsigned const resident = 8u * unsigned(compute_units_of_current_device());
+        if (plan.blocks > resident) plan.blocks = resident;
+    }
+    args.grid = plan.grid;
+    args.transfers = plan.transfers;
+    switch (a.format) {
+    case NTC_HIP_DEV_FORMAT_UNORM8:  return launch_write_groups_of<NTC_HIP_DEV_FORMAT_UNORM8>(args, plan, stream);
+    case NTC_HIP_DEV_FORMAT_UNORM16: return launch_write_groups_of<NTC_HIP_DEV_FORMAT_UNORM16>(args, plan, stream);
+    case NTC_HIP_DEV_FORMAT_FLOAT16: return launch_write_groups_of<NTC_HIP_DEV_FORMAT_FLOAT16>(args, plan, stream);
+    case NTC_HIP_DEV_FORMAT_FLOAT32: return launch_write_groups_of<NTC_HIP_DEV_FORMAT_FLOAT32>(args, plan, stream);
+    case NTC_HIP_DEV_FORMAT_UINT32:  return launch_write_groups_of<NTC_HIP_DEV_FORMAT_UINT32>(args, plan, stream);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+template <int FORMAT>
 static void launch_write_format(WriteChannelsArgs const& a, dim3 grid, bool plain, hipStream_t stream)
 {
     if (plain) hipLaunchKernelGGL((write_channels_kernel<FORMAT, true>), grid, dim3(256), 0, stream, a);
@@ -447,6 +888,7 @@ hipError_t launch_write_channels(WriteChannelsArgs const& args, hipStream_t stre
         hipLaunchKernelGGL(write_channels_resize_kernel, dim3((a.width + 63) / 64, (a.height + 3) / 4), dim3(256), 0, stream, a);
         return hipGetLastError();
     }
+    if (a.pixelStride <= 8 && a.wholePixels) return launch_write_groups(a, stream);
     dim3 const grid = copy_grid(a.width, a.height, a.xShift, false);
     bool const plain = plain_copy(a.srcColorSpaces, a.dstColorSpaces, 0);
     switch (a.format) {
@@ -679,6 +1121,48 @@ static void launch_read_format(ReadChannelsArgs const& a, dim3 grid, bool plain,
     else       hipLaunchKernelGGL((read_channels_kernel<FORMAT, false>), grid, dim3(256), 0, stream, a);
 }
 
+template <int FORMAT>
+static hipError_t launch_read_groups_of(ReadGroupsArgs const& args, GroupLaunch const& plan, hipStream_t stream)
+{
+    auto launch = [&](auto channels) {
+        constexpr int CHANNELS = decltype(channels)::value;
+        if constexpr (CHANNELS * bytes_per_channel(FORMAT) <= 8) {
+            constexpr bool unorm = FORMAT == NTC_HIP_DEV_FORMAT_UNORM8 || FORMAT == NTC_HIP_DEV_FORMAT_UNORM16;   // (dithering changes only these)
+            if (unorm && args.a.useDithering) hipLaunchKernelGGL((read_groups_kernel<FORMAT, CHANNELS, unorm>), dim3(plan.blocks), dim3(plan.threads), plan.ldsBytes, stream, args);
+            else                              hipLaunchKernelGGL((read_groups_kernel<FORMAT, CHANNELS, false>), dim3(plan.blocks), dim3(plan.threads), plan.ldsBytes, stream, args);
+        }
+    };
+    switch (args.a.dstChannels) {
+    case 1: launch(std::integral_constant<int, 1>{}); break;
+    case 2: launch(std::integral_constant<int, 2>{}); break;
+    case 3: launch(std::integral_constant<int, 3>{}); break;
+    case 4: launch(std::integral_constant<int, 4>{}); break;
+    case 5: launch(std::integral_constant<int, 5>{}); break;
+    case 6: launch(std::integral_constant<int, 6>{}); break;
+    case 7: launch(std::integral_constant<int, 7>{}); break;
+    case 8: launch(std::integral_constant<int, 8>{}); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+static hipError_t launch_read_groups(ReadChannelsArgs const& a, hipStream_t stream)
+{
+    ReadGroupsArgs args{};
+    args.a = a;
+    GroupLaunch const plan = plan_groups(a.width, a.height, a.srcColorSpaces, a.dstColorSpaces, a.numChannels < a.dstChannels ? a.numChannels : a.dstChannels, true);
+    args.grid = plan.grid;
+    args.transfers = plan.transfers;
+    switch (a.format) {
+    case NTC_HIP_DEV_FORMAT_UNORM8:  return launch_read_groups_of<NTC_HIP_DEV_FORMAT_UNORM8>(args, plan, stream);
+    case NTC_HIP_DEV_FORMAT_UNORM16: return launch_read_groups_of<NTC_HIP_DEV_FORMAT_UNORM16>(args, plan, stream);
+    case NTC_HIP_DEV_FORMAT_FLOAT16: return launch_read_groups_of<NTC_HIP_DEV_FORMAT_FLOAT16>(args, plan, stream);
+    case NTC_HIP_DEV_FORMAT_FLOAT32: return launch_read_groups_of<NTC_HIP_DEV_FORMAT_FLOAT32>(args, plan, stream);
+    case NTC_HIP_DEV_FORMAT_UINT32:  return launch_read_groups_of<NTC_HIP_DEV_FORMAT_UINT32>(args, plan, stream);
+    default: return hipErrorInvalidValue;
+    }
+}
+
 hipError_t launch_read_channels(ReadChannelsArgs const& args, hipStream_t stream)
 {
     ReadChannelsArgs a = args;
@@ -694,6 +1178,7 @@ hipError_t launch_read_channels(ReadChannelsArgs const& args, hipStream_t stream
         }
         return hipGetLastError();
     }
+    if (a.dstChannels * bytes_per_channel(a.format) <= 8) return launch_read_groups(a, stream);
     dim3 const grid = copy_grid(a.width, a.height, a.xShift);
     bool const plain = plain_copy(a.srcColorSpaces, a.dstColorSpaces, a.useDithering);
     switch (a.format) {

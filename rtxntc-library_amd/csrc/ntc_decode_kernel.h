@@ -93,6 +93,8 @@ struct ReadChannelsArgs {
     int32_t dstWidth, dstHeight;   // size of the user image when it differs from the mip's (resampling copy), else 0
     uint8_t srcColorSpaces[16], dstColorSpaces[16];   // per copied channel: 0 linear, 1 sRGB, 2 HLG
 };
+// Fills the colour-space tables of the current device that the copies read.
+hipError_t launch_transfer_tables(hipStream_t stream);
 hipError_t launch_read_channels(ReadChannelsArgs const& args, hipStream_t stream);
 
 constexpr int NTC_HIP_DEV_MAX_CHANNELS = 16;
@@ -103,6 +105,7 @@ struct WriteChannelsArgs {
     uint64_t pixelStride, rowPitch;
     int32_t width, height, setChannels, firstChannel, numChannels, format, verticalFlip;
     int32_t vectorBytes;           // widest load every pixel start is aligned to
+    int32_t wholePixels;           // the buffer holds all pixelStride bytes of the last pixel too
     int32_t xShift;                // set by the launcher
     int32_t srcWidth, srcHeight;   // size of the user image when it differs from the mip's (resampling copy), else 0
     uint8_t srcColorSpaces[16], dstColorSpaces[16];

@@ -523,6 +523,9 @@ static int create_context(int device, NtcHipContext** outContext)
     {                                   // once per device, with that device current
         std::lock_guard<std::mutex> lock(g_liveMutex);
         if (!g_staticTable[device]) {
+            // the tables of the channel copies, complete before any context can use them
+            HIP_TRY(launch_transfer_tables(nullptr));
+            HIP_TRY(hipStreamSynchronize(nullptr));
             void* address = nullptr;
             HIP_TRY(hipGetSymbolAddress(&address, HIP_SYMBOL(scratch)));
             g_staticTable[device] = address;
@@ -985,6 +988,7 @@ int ntc_hip_ctx_write_channels(NtcHipContext* ctx, const NtcHipWriteChannels* p)
     a.width = p->width; a.height = p->height; a.setChannels = p->setChannels;
     a.firstChannel = p->firstChannel; a.numChannels = p->numChannels; a.format = p->format; a.verticalFlip = p->verticalFlip ? 1 : 0;
     a.vectorBytes = common_alignment(reinterpret_cast<uintptr_t>(p->src), p->rowPitch, p->pixelStride);
+    a.wholePixels = uint64_t(imageHeight - 1) * p->rowPitch + uint64_t(imageWidth) * p->pixelStride <= p->srcBytes;
     a.srcWidth = resample ? p->srcWidth : 0; a.srcHeight = resample ? p->srcHeight : 0;
     for (int i = 0; i < 16; ++i) {
         if (p->srcColorSpaces[i] > 2 || p->dstColorSpaces[i] > 2) { set_error("ntc_hip_write_channels: unknown colour space for channel %d.", i); return NTC_HIP_ERR_INVALID_ARG; }

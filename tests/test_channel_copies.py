@@ -1,0 +1,88 @@
+"""ReadChannels / WriteChannels of small pixels (four pixels a lane) and their transfer tables on the GPU, at the sizes
+where the split of a row into groups, the alignment of the user image or the tables' bounds matter."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+BPC = {1: 1, 2: 2, 3: 2, 4: 4, 5: 4}
+SMALL_PIXELS = [(fmt, channels) for fmt in BPC for channels in range(1, 9) if channels * BPC[fmt] <= 8]
+
+
+def halves(rng, count):
+    return rng.integers(0, 0x3C01, count, dtype=np.uint16)                # [0, 1]
+
+
+def read(ntc, device, d_planar, w, h, set_channels, first, count, fmt, stride, offset, dither=0, spaces=(0, 0), pitch=None):
+    pitch = pitch or w * stride + BPC[fmt]
+    d_dst = device.alloc(offset + h * pitch)
+    d_dst.fill(0xEE)
+    rc = ntc.abi.ReadChannels()
+    rc.planarPairs, rc.planarBytes = d_planar.ptr, d_planar.nbytes
+    rc.width, rc.height, rc.setChannels, rc.firstChannel, rc.numChannels = w, h, set_channels, first, count
+    rc.dst, rc.dstBytes, rc.format, rc.pixelStride, rc.rowPitch, rc.useDithering = d_dst.ptr + offset, d_dst.nbytes - offset, fmt, stride, pitch, dither
+    for i in range(count):
+        rc.srcColorSpaces[i], rc.dstColorSpaces[i] = spaces
+    device.call("read_channels", rc)
+    device.synchronize()
+    return d_dst.download()[offset:], pitch
+
+
+@pytest.mark.parametrize("fmt,channels", SMALL_PIXELS)
+def test_read_groups_at_their_edges(ntc, device, oracle, fmt, channels):
+    rng = np.random.default_rng(10 * fmt + channels)
+    zeros = np.zeros(16, dtype=np.uint8)
+    for w, h, first, dither in ((1, 3, 0, 0), (3, 1, 1, 1), (4, 2, 1, 0), (5, 9, 0, 1), (31, 3, 2, 0), (33, 35, 1, 1), (130, 5, 3, 0), (257, 18, 0, 1), (259, 4, 4, 0)):
+        count = min(channels, 12 - first) if w != 130 else max(1, channels - 2)          # (130: default-valued channels behind the copied ones)
+        planar = halves(rng, w * h * 12)
+        d_planar = device.upload(planar)
+        got, pitch = read(ntc, device, d_planar, w, h, 12, first, count, fmt, channels * BPC[fmt], (w % 3) * BPC[fmt], dither)
+        want = np.full(got.size, 0xEE, dtype=np.uint8)
+        assert oracle.ntc_oracle_read_channels_ex(planar.ctypes.data, w, h, 12, first, count, want.ctypes.data, fmt, channels * BPC[fmt], pitch, dither,
+                                                  zeros.ctypes.data, zeros.ctypes.data) == 0
+        assert np.array_equal(got, want), (w, h, first)
+
+
+@pytest.mark.parametrize("fmt,channels", SMALL_PIXELS)
+def test_write_groups_at_their_edges(ntc, device, oracle, fmt, channels):
+    rng = np.random.default_rng(100 + 10 * fmt + channels)
+    for w, h, first, flip in ((1, 3, 0, 0), (3, 1, 1, 1), (4, 2, 1, 0), (5, 9, 0, 1), (31, 3, 2, 0), (33, 35, 1, 1), (130, 5, 3, 0), (257, 18, 0, 1), (259, 4, 4, 0)):
+        count = min(channels, 12 - first) if w != 130 else max(1, channels - 2)
+        stride, offset = channels * BPC[fmt], (w % 3) * BPC[fmt]
+        pitch = w * stride + BPC[fmt]
+        if fmt == 3:
+            image = halves(rng, (offset + h * pitch) // 2).view(np.uint8)
+        elif fmt == 4:
+            image = rng.uniform(-2, 70000, (offset + h * pitch) // 4).astype(np.float32).view(np.uint8)
+        else:
+            image = rng.integers(0, 256, offset + h * pitch, dtype=np.uint8)
+        start = np.full(w * h * 12, 0x1234, dtype=np.uint16)
+        d_image, d_planar = device.upload(image), device.upload(start)
+        wc = ntc.abi.WriteChannels()
+        wc.src, wc.srcBytes, wc.format, wc.verticalFlip, wc.pixelStride, wc.rowPitch = d_image.ptr + offset, d_image.nbytes - offset, fmt, flip, stride, pitch
+        wc.planarPairs, wc.planarBytes = d_planar.ptr, d_planar.nbytes
+        wc.width, wc.height, wc.setChannels, wc.firstChannel, wc.numChannels = w, h, 12, first, count
+        device.call("write_channels", wc)
+        device.synchronize()
+        want, user = start.copy(), np.ascontiguousarray(image[offset:])
+        assert oracle.ntc_oracle_write_channels(user.ctypes.data, fmt, flip, stride, pitch, want.ctypes.data, w, h, 12, first, count) == 0
+        assert np.array_equal(d_planar.download().view(np.uint16), want), (w, h, first, flip)
+
+
+@pytest.mark.parametrize("spaces", [(1, 1), (1, 0), (0, 1), (2, 0), (0, 2), (2, 1), (1, 2), (2, 2)])
+def test_tables_in_lds_and_in_memory_give_the_same(ntc, device, spaces):
+    """Every half, through the launch that stages a table (an image of two million pixels) and through one that does
+    not (65536 pixels); one pixel a lane (a stride of 16 bytes) as well."""
+    w, h = 2048, 1028
+    every = np.arange(65536, dtype=np.uint16)
+    planar = np.zeros(w * h * 2, dtype=np.uint16).reshape(h, w, 2)
+    planar[:, :, 0] = np.resize(every, w * h).reshape(h, w)
+    d_big = device.upload(planar.reshape(-1))
+    big, pitch = read(ntc, device, d_big, w, h, 2, 0, 1, 4, 4, 0, spaces=spaces, pitch=4 * w)
+    small_planar = np.zeros(65536 * 2, dtype=np.uint16)
+    small_planar[0::2] = every
+    d_small = device.upload(small_planar)
+    small, _ = read(ntc, device, d_small, 256, 256, 2, 0, 1, 4, 4, 0, spaces=spaces, pitch=4 * 256)
+    wide, _ = read(ntc, device, d_small, 256, 256, 2, 0, 1, 4, 16, 0, spaces=spaces, pitch=16 * 256)
+    assert np.array_equal(big.view(np.uint32), np.resize(small.view(np.uint32), w * h))
+    assert np.array_equal(wide.view(np.uint32).reshape(-1, 4)[:, 0], small.view(np.uint32))
