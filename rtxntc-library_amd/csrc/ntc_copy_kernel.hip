@@ -13,6 +13,9 @@
 
 namespace ntc_hip_dev {
 
+typedef float    v2f __attribute__((ext_vector_type(2)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+
 // u(clamp(roundf(p), 0, top)) of WriteImageChannel (src/ImageProcessing.cu:141-152) for the UNORM formats.
 // roundf rounds halves away from zero; for |p| < 2^23 it equals trunc(p + copysign(c, p)) with c the
 // largest float below 1/2 (the sum rounds up to the next integer exactly when the fraction is at
@@ -69,6 +72,31 @@ __device__ __forceinline__ uint16_t stored_half(float v)     // WriteImageChanne
     v = fmaxf(-65504.f, fminf(65504.f, v));
     asm volatile("" : "+v"(v));
     return __builtin_bit_cast(uint16_t, (_Float16)v);
+}
+
+// stored_half(encode_color_space(space, v)) for a value computed in fp32, most of the time without the math library: the
+// hardware's log2, exp2 and square root are good to 2^-21 of what encode_color_space makes of v (over every v of the
+// ranges below), so where y - e and y + e, e = 2^-20, round to the same half, that is the answer.  The few lanes in
+// doubt (one in five hundred), and values outside the ranges, take the exact function.  `space` is uniform.
+__device__ __forceinline__ uint32_t encoded_half(int space, float v)
+{
+    if (space == 0) return stored_half(v);
+    constexpr float kError = 0x1p-20f;
+    float y, e;
+    bool certain;
+    if (space == 1) {
+        y = 1.055f * __builtin_amdgcn_exp2f(__builtin_amdgcn_logf(v) * (1.0f / 2.4f)) - 0.055f;
+        e = __builtin_fmaf(y, kError, 0.055f * kError);
+        certain = v > 0.0031308f && v <= 1.f;
+    } else {
+        y = 0.5f * __builtin_amdgcn_sqrtf(v);
+        e = y * kError;
+        certain = v >= 0x1p-100f && v < 1.f;
+    }
+    v2h const around = __builtin_convertvector(v2f{ y - e, y + e }, v2h);
+    uint32_t const bits = __builtin_bit_cast(uint32_t, around), half = bits & 0xffffu;
+    if (!certain || half != bits >> 16) return stored_half(encode_color_space(space, v));
+    return half;
 }
 
 __global__ void __launch_bounds__(256)
@@ -303,6 +331,7 @@ read_channels_kernel(ReadChannelsArgs a)
 typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
 typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(1)));
 typedef uint32_t u32_any   __attribute__((aligned(1)));
+typedef uint32_t u32x2_a4  __attribute__((ext_vector_type(2), aligned(4)));
 typedef uint32_t u32x4_a4  __attribute__((ext_vector_type(4), aligned(4)));
 
 // Which pixels a lane works on: tiles of lanesX groups by threads / lanesX rows, a workgroup takes tiles
@@ -390,7 +419,7 @@ struct ReadGroupsArgs { ReadChannelsArgs a; GroupGrid grid; StagedTransfers tran
 
 // CHANNELS = channels of a destination pixel.
 template <int FORMAT, int CHANNELS, bool DITHER>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(1024, 8)
 read_groups_kernel(ReadGroupsArgs args)
 {
     constexpr int BPC = bytes_per_channel(FORMAT), PIXEL = CHANNELS * BPC, PAIRS = CHANNELS / 2 + 1;
@@ -511,13 +540,12 @@ __device__ __forceinline__ uint32_t stored_half_of(uint32_t bits, int srcSpace, 
 struct WriteGroupsArgs { WriteChannelsArgs a; GroupGrid grid; StagedTransfers transfers; };
 
 // Four pixels of at most eight bytes a lane, like read_groups_kernel the other way round: whole dwords of the pixels
-// in, 16 bytes of each complete channel pair out (2048 x 2048 of 8 bits: RGBA 16 us, with sRGB 91 before the tables; one
-// channel 11 us, 15 before, of which the 2-byte stores into half a pair are the larger part; HLG halves 21 us, 29
-// before); where the image has only one channel of a pair, its halves go out
+// in, 16 bytes of each complete channel pair out (2048 x 2048 of 8 bits: RGBA with sRGB 14 us, 91 before the tables; two
+// channels in halves of two pairs 13 us, one 10 us, 15 before; HLG halves 18 us, 29 before); where the image has only one channel of a pair, its halves go out
 // one by one between those of the other.  CHANNELS = channels of a source pixel, of which a.numChannels are stored.
 // 8-bit codes become halves through a table in LDS, a row of 256 per channel.
 template <int FORMAT, int CHANNELS>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(1024, 8)
 write_groups_kernel(WriteGroupsArgs args)
 {
     constexpr int BPC = bytes_per_channel(FORMAT), PIXEL = CHANNELS * BPC, PAIRS = CHANNELS / 2 + 1;
@@ -540,7 +568,7 @@ write_groups_kernel(WriteGroupsArgs args)
     for (int tile = blockIdx.x; tile < args.grid.tiles; tile += gridDim.x) {
         int const tileY = tile / args.grid.tilesX, tileX = tile - tileY * args.grid.tilesX;
         int const x = (tileX * lanesX + lx) * 4, y = tileY * int(blockDim.x >> args.grid.log2LanesX) + ly;
-        if (x >= a.width || y >= a.height) continue;
+        if (y >= a.height) continue;                         // (uniform across a wave that covers one row)
         bool const whole = x + 4 <= a.width;
         uint8_t const* const in = a.src + size_t(a.verticalFlip ? a.height - 1 - y : y) * a.rowPitch + size_t(x) * PIXEL;
         uint32_t words[PIXEL];
@@ -612,10 +640,26 @@ write_groups_kernel(WriteGroupsArgs args)
 #pragma unroll
                     for (int k = 0; k < 4; ++k) if (x + k < a.width) *reinterpret_cast<uint32_t*>(to + 2 * k) = pair[k];
                 }
+            } else if (args.grid.log2LanesX == 6) {
+                // One half of a pair, a wave per row: the wave's 256 halves are dealt out anew, 64 neighbours to a
+                // store, so that a store touches 256 bytes and not 1 KB (one channel 12 -> 10 us, two
+                // 19 -> 13 us).  Lane i's pixel of store s is element i % 4
+                // of lane 16 s + i / 4.
+                uint32_t const low = hasLower ? __builtin_amdgcn_perm(pair[1], pair[0], 0x05040100u) : __builtin_amdgcn_perm(pair[1], pair[0], 0x07060302u);
+                uint32_t const high = hasLower ? __builtin_amdgcn_perm(pair[3], pair[2], 0x05040100u) : __builtin_amdgcn_perm(pair[3], pair[2], 0x07060302u);
+                uint16_t* const from = to - 2 * 4 * lx + 2 * lx + (hasLower ? 0 : 1);      // the wave's first pixel, then the lane's
+                int const left = a.width - tileX * 256 - lx;                                 // pixels of the row from the lane's first on
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    int const source = (16 * s + (lx >> 2)) * 4;
+                    uint32_t const l = uint32_t(__builtin_amdgcn_ds_bpermute(source, int(low))), h = uint32_t(__builtin_amdgcn_ds_bpermute(source, int(high)));
+                    uint32_t const two = (lx & 2) ? h : l;
+                    if (64 * s < left) from[2 * 64 * s] = uint16_t((lx & 1) ? two >> 16 : two);
+                }
             } else {
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
-                    if (whole || x + k < a.width) to[2 * k + (hasLower ? 0 : 1)] = uint16_t(hasLower ? pair[k] : pair[k] >> 16);
+                    if (x + k < a.width) to[2 * k + (hasLower ? 0 : 1)] = uint16_t(hasLower ? pair[k] : pair[k] >> 16);
             }
         }
     }
@@ -706,9 +750,13 @@ __device__ __forceinline__ BilinearTaps setup_bilinear(int srcW, int srcH, int d
     return t;
 }
 
+// ALL_WEIGHTED: the caller knows that no weight is zero.
+template <bool ALL_WEIGHTED = false>
 __device__ __forceinline__ float blend_taps(BilinearTaps const& t, float a, float b, float c, float d)
 {
-    a = t.w[0] > 0.f ? a : 0.f; b = t.w[1] > 0.f ? b : 0.f; c = t.w[2] > 0.f ? c : 0.f; d = t.w[3] > 0.f ? d : 0.f;
+    if constexpr (!ALL_WEIGHTED) {
+        a = t.w[0] > 0.f ? a : 0.f; b = t.w[1] > 0.f ? b : 0.f; c = t.w[2] > 0.f ? c : 0.f; d = t.w[3] > 0.f ? d : 0.f;
+    }
     return __builtin_fmaf(d, t.w[3], __builtin_fmaf(c, t.w[2], __builtin_fmaf(b, t.w[1], a * t.w[0])));
 }
 
@@ -781,36 +829,77 @@ write_channels_resize_kernel(WriteChannelsArgs a)
 
 // ResizeMultichannelImageKernel (src/ImageProcessing.cu:178-207): every channel of one image of the
 // internal layout resampled into another; a channel pair is read as dwords and written as one.
+//
+// A lane makes one pixel of a range of channel pairs.  The two taps of a source row are neighbours: one 8-byte load
+// (shifted left by a pixel at the right edge), and the next pair's are under way while a pair is filtered.  Stored
+// values are decoded by table (from LDS in launches large enough, as in the copies above; a powf per tap and channel
+// kept the kernel at 0.9 TB/s), the filtered value is encoded by the device function.  Images too small to fill the
+// GPU are split by channel pairs: one mip of 64 x 64 and six pairs is 64 waves, not 4, in a chain a sixth as long.
+// 2048 x 2048, 12 channels (three sRGB, three HLG): 39 us for the 1024 x 1024 mip, 68 before (56 with the math library's
+// encoding, which took half of the vector instructions); 13 for the next, 24 before; the nine smaller ones 4 - 6 each,
+// 12 - 24 before.
 struct ResizePlanarArgs {
     uint16_t const* src; uint16_t* dst;
     int32_t srcWidth, srcHeight, dstWidth, dstHeight, setChannels;
+    int32_t tilesX, tiles, pairsPerLane;                     // tiles of 64 x blockDim.x / 64 pixels
+    StagedTransfers transfers;                               // of the decoding pairs; pair / slot: per colour space
     uint8_t colorSpaces[16];
 };
 
-__global__ void __launch_bounds__(256)
+template <bool LINEAR>
+__global__ void __launch_bounds__(1024, 8)
 resize_planar_kernel(ResizePlanarArgs a)
 {
-    int const x = blockIdx.x * 64 + (threadIdx.x & 63), y = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (x >= a.dstWidth || y >= a.dstHeight) return;
-    BilinearTaps const t = setup_bilinear(a.srcWidth, a.srcHeight, a.dstWidth, a.dstHeight, x, y);
+    extern __shared__ float staged[];
+    if constexpr (!LINEAR) copy_staged(a.transfers, staged);
+    int const pairBegin = int(blockIdx.y) * a.pairsPerLane, pairEnd = min(a.setChannels >> 1, pairBegin + a.pairsPerLane);
     size_t const srcRow = size_t(a.srcWidth) * size_t(a.setChannels), pairStride = size_t(a.srcWidth) * 2;
-    uint16_t const* const r0 = a.src + size_t(t.y0) * srcRow;
-    uint16_t const* const r1 = a.src + size_t(t.y1) * srcRow;
-    uint32_t* const out = reinterpret_cast<uint32_t*>(a.dst + size_t(y) * size_t(a.dstWidth) * size_t(a.setChannels) + size_t(x) * 2);
-    for (int p = 0; p < a.setChannels / 2; ++p) {
-        uint32_t const v00 = *reinterpret_cast<uint32_t const*>(r0 + p * pairStride + size_t(t.x0) * 2);
-        uint32_t const v10 = *reinterpret_cast<uint32_t const*>(r0 + p * pairStride + size_t(t.x1) * 2);
-        uint32_t const v01 = *reinterpret_cast<uint32_t const*>(r1 + p * pairStride + size_t(t.x0) * 2);
-        uint32_t const v11 = *reinterpret_cast<uint32_t const*>(r1 + p * pairStride + size_t(t.x1) * 2);
-        uint32_t packed = 0;
+    for (int tile = blockIdx.x; tile < a.tiles; tile += gridDim.x) {
+        int const tileY = tile / a.tilesX, tileX = tile - tileY * a.tilesX;
+        int const x = tileX * 64 + int(threadIdx.x & 63), y = tileY * int(blockDim.x >> 6) + int(threadIdx.x >> 6);
+        if (x >= a.dstWidth || y >= a.dstHeight) continue;
+        BilinearTaps const t = setup_bilinear(a.srcWidth, a.srcHeight, a.dstWidth, a.dstHeight, x, y);
+        int const left = max(0, min(t.x0, a.srcWidth - 2));  // columns left and left + 1 hold both taps
+        bool const shift0 = t.x0 != left, shift1 = t.x1 != left;
+        uint16_t const* const r0 = a.src + size_t(t.y0) * srcRow + size_t(left) * 2;
+        uint16_t const* const r1 = a.src + size_t(t.y1) * srcRow + size_t(left) * 2;
+        uint32_t* const out = reinterpret_cast<uint32_t*>(a.dst + size_t(y) * size_t(a.dstWidth) * size_t(a.setChannels) + size_t(x) * 2);
+        auto load = [&](uint16_t const* row, int p, uint32_t (&taps)[2]) {
+            if (a.srcWidth < 2) {                            // uniform
+                taps[0] = taps[1] = *reinterpret_cast<uint32_t const*>(row + size_t(p) * pairStride);
+            } else {
+                u32x2_a4 const v = *reinterpret_cast<u32x2_a4 const*>(row + size_t(p) * pairStride);
+                taps[0] = v[0]; taps[1] = v[1];
+            }
+        };
+        // (taps of zero weight have to be dropped: the product with an infinity would not be zero.  Away from the
+        // edges of a 2 : 1 reduction no lane has one.)
+        auto pairs = [&](auto allWeighted) __attribute__((always_inline)) {
+            constexpr bool ALL = decltype(allWeighted)::value;
+            uint32_t top[2], bottom[2];
+            load(r0, pairBegin, top);
+            load(r1, pairBegin, bottom);
+            for (int p = pairBegin; p < pairEnd; ++p) {
+                uint32_t const v00 = shift0 ? top[1] : top[0], v10 = shift1 ? top[1] : top[0];
+                uint32_t const v01 = shift0 ? bottom[1] : bottom[0], v11 = shift1 ? bottom[1] : bottom[0];
+                int const next = min(p + 1, pairEnd - 1);
+                load(r0, next, top);
+                load(r1, next, bottom);
+                uint32_t packed = 0;
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            int const space = a.colorSpaces[2 * p + k];
-            auto half_of = [&](uint32_t v) { return decode_color_space(space, float(__builtin_bit_cast(_Float16, uint16_t(v >> (16 * k))))); };
-            float const value = blend_taps(t, half_of(v00), half_of(v10), half_of(v01), half_of(v11));
-            packed |= uint32_t(stored_half(encode_color_space(space, value))) << (16 * k);
-        }
-        out[size_t(p) * size_t(a.dstWidth)] = packed;
+                for (int k = 0; k < 2; ++k) {
+                    int const space = LINEAR ? 0 : a.colorSpaces[2 * p + k];
+                    uint32_t const bits[4] = { (v00 >> (16 * k)) & 0xffffu, (v10 >> (16 * k)) & 0xffffu, (v01 >> (16 * k)) & 0xffffu, (v11 >> (16 * k)) & 0xffffu };
+                    float v[4];
+                    if constexpr (LINEAR) transfer_halves(staged, 0, -1, bits, v);
+                    else                  transfer_halves(staged, a.transfers.slot[space], a.transfers.pair[space], bits, v);
+                    packed |= encoded_half(space, blend_taps<ALL>(t, v[0], v[1], v[2], v[3])) << (16 * k);
+                }
+                out[size_t(p) * size_t(a.dstWidth)] = packed;
+            }
+        };
+        if (__all(t.w[0] > 0.f && t.w[1] > 0.f && t.w[2] > 0.f && t.w[3] > 0.f)) pairs(std::true_type{});
+        else                                                                     pairs(std::false_type{});
     }
 }
 
@@ -819,8 +908,44 @@ hipError_t launch_resize_planar(uint16_t const* src, int srcWidth, int srcHeight
 {
     ResizePlanarArgs a{};
     a.src = src; a.dst = dst; a.srcWidth = srcWidth; a.srcHeight = srcHeight; a.dstWidth = dstWidth; a.dstHeight = dstHeight; a.setChannels = setChannels;
-    for (int i = 0; i < 16; ++i) a.colorSpaces[i] = colorSpaces ? colorSpaces[i] : 0;
-    hipLaunchKernelGGL(resize_planar_kernel, dim3((dstWidth + 63) / 64, (dstHeight + 3) / 4), dim3(256), 0, stream, a);
+    bool linear = true;
+    for (int i = 0; i < 16; ++i) {
+        a.colorSpaces[i] = colorSpaces ? colorSpaces[i] : 0;
+        linear = linear && (a.colorSpaces[i] == 0 || i >= setChannels);
+    }
+    int const units = compute_units_of_current_device(), pairs = setChannels / 2;
+    auto tile = [&](int threads) {
+        a.tilesX = (dstWidth + 63) / 64;
+        a.tiles = a.tilesX * ((dstHeight + threads / 64 - 1) / (threads / 64));
+    };
+    int threads = 1024;
+    tile(threads);
+    bool const stage = !linear && a.tiles >= 2 * units;      // as in plan_groups: each copy serves two tiles or more
+    a.transfers.pair[0] = -1;
+    for (int space = 1; space <= 2; ++space) {
+        a.transfers.pair[space] = int8_t(transfer_pair(space, 0));
+        bool used = false;
+        for (int i = 0; i < setChannels; ++i) used = used || a.colorSpaces[i] == space;
+        if (!stage || !used) continue;
+        a.transfers.staged[a.transfers.count] = a.transfers.pair[space];
+        a.transfers.slot[space] = int8_t(++a.transfers.count);
+    }
+    dim3 grid(1);
+    a.pairsPerLane = pairs;
+    if (stage) {
+        grid.x = unsigned(2 * units < a.tiles ? 2 * units : a.tiles);
+    } else {
+        threads = 256;
+        tile(threads);
+        // as many ranges of pairs as it takes to have eight waves for every SIMD
+        int const waves = a.tiles * (threads / 64), wanted = (32 * units + waves - 1) / waves;
+        int const ranges = wanted < 1 ? 1 : wanted > pairs ? pairs : wanted;
+        a.pairsPerLane = (pairs + ranges - 1) / ranges;
+        grid = dim3(unsigned(a.tiles), unsigned((pairs + a.pairsPerLane - 1) / a.pairsPerLane));
+    }
+    size_t const lds = size_t(a.transfers.count) * kStageCount * sizeof(float);
+    if (linear) hipLaunchKernelGGL(resize_planar_kernel<true>, grid, dim3(threads), lds, stream, a);
+    else        hipLaunchKernelGGL(resize_planar_kernel<false>, grid, dim3(threads), lds, stream, a);
     return hipGetLastError();
 }
 

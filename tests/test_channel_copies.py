@@ -86,3 +86,35 @@ def test_tables_in_lds_and_in_memory_give_the_same(ntc, device, spaces):
     wide, _ = read(ntc, device, d_small, 256, 256, 2, 0, 1, 4, 16, 0, spaces=spaces, pitch=16 * 256)
     assert np.array_equal(big.view(np.uint32), np.resize(small.view(np.uint32), w * h))
     assert np.array_equal(wide.view(np.uint32).reshape(-1, 4)[:, 0], small.view(np.uint32))
+
+
+@pytest.mark.parametrize("space", [1, 2])
+@pytest.mark.parametrize("w,h", [(64, 16), (2048, 1024)])
+def test_resized_colour_channels_equal_their_parts(ntc, device, space, w, h):
+    """A 2 : 1 reduction of a channel stored in sRGB / HLG against decoding (read as FLOAT32), averaging (numpy) and
+    encoding (write from FLOAT32, by the math library): halves of every magnitude, with and without tables in LDS."""
+    rng = np.random.default_rng(w + space)
+    planar = np.zeros((h, 2, w, 2), dtype=np.uint16)                      # four channels: pairs (0, 1) and (2, 3)
+    planar[:, 0] = halves(rng, h * w * 2).reshape(h, w, 2)
+    planar[:, 1] = rng.integers(0x3000, 0x3E00, h * w * 2, dtype=np.uint16).reshape(h, w, 2)      # up to 1.5
+    d_src = device.upload(planar.reshape(-1))
+    spaces = (ntc.abi.C.c_uint8 * 16)(*([space, 0, space, space] + [0] * 12))
+    d_dst = device.alloc(w * h * 2)
+    device.call("resize_planar", d_src.ptr, d_src.nbytes, w, h, d_dst.ptr, d_dst.nbytes, w // 2, h // 2, 4, spaces)
+    device.synchronize()
+    got = d_dst.download().view(np.uint16).reshape(h // 2, 2, w // 2, 2)
+    for channel in range(4):
+        linear, _ = read(ntc, device, d_src, w, h, 4, channel, 1, 4, 4, 0, spaces=(spaces[channel], 0), pitch=4 * w)
+        v = linear.view(np.float32).reshape(h, w)
+        mean = ((v[0::2, 0::2] + v[0::2, 1::2]) + v[1::2, 0::2]) + v[1::2, 1::2]
+        mean = np.ascontiguousarray(mean * np.float32(0.25))
+        d_mean, d_out = device.upload(mean), device.alloc(w * h)
+        wc = ntc.abi.WriteChannels()
+        wc.src, wc.srcBytes, wc.format, wc.pixelStride, wc.rowPitch = d_mean.ptr, d_mean.nbytes, 4, 4, 2 * w
+        wc.planarPairs, wc.planarBytes = d_out.ptr, d_out.nbytes
+        wc.width, wc.height, wc.setChannels, wc.firstChannel, wc.numChannels = w // 2, h // 2, 2, 0, 1
+        wc.dstColorSpaces[0] = spaces[channel]
+        device.call("write_channels", wc)
+        device.synchronize()
+        want = d_out.download().view(np.uint16).reshape(h // 2, w // 2, 2)[:, :, 0]
+        assert np.array_equal(got[:, channel // 2, :, channel % 2], want), channel
