@@ -1177,6 +1177,12 @@ hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int heig
 // by width * height, scaled by 2^16, split into floor and fraction * 2^32 and added to the 64-bit
 // accumulators (ImageDifference.hlsl:103-127; the integer atomics make the total independent of
 // the order in which workgroups finish).
+//
+// Images of four channels in one UNORM or float format, the usual ones, are read as whole pixels, all of a thread's
+// rows (or as many as 32 registers hold) before any arithmetic, and UNORM8 codes are divided by the corrected
+// reciprocal.  A workgroup takes several tiles and adds its 64-bit sums to the accumulators once (four workgroups a compute unit: with eight, the atomics on four addresses add 9 us, with two
+// there are too few waves: 4 us).  4096 x 4096 RGBA8:
+// 33 us (the bytes take 27), 156 with four byte loads a pixel, one row after the other.
 __device__ __forceinline__ float diff_channel(DiffImageArgs const& im, uint8_t const* px, int c)
 {
     if (c >= im.numChannels) return c == 3 ? 1.f : 0.f;
@@ -1189,53 +1195,125 @@ __device__ __forceinline__ float diff_channel(DiffImageArgs const& im, uint8_t c
     }
 }
 
+// A pixel of four channels of FORMAT as dwords, at whatever alignment it has.
+template <int FORMAT>
+__device__ __forceinline__ void load_pixel(uint8_t const* px, uint32_t (&words)[bytes_per_channel(FORMAT)])
+{
+    if constexpr (bytes_per_channel(FORMAT) == 1) {
+        words[0] = *reinterpret_cast<u32_any const*>(px);
+    } else if constexpr (bytes_per_channel(FORMAT) == 2) {
+        u32x2_any const v = *reinterpret_cast<u32x2_any const*>(px);
+        words[0] = v[0]; words[1] = v[1];
+    } else {
+        u32x4_any const v = *reinterpret_cast<u32x4_any const*>(px);
+        words[0] = v[0]; words[1] = v[1]; words[2] = v[2]; words[3] = v[3];
+    }
+}
+template <int FORMAT>
+__device__ __forceinline__ float pixel_channel(uint32_t const (&words)[bytes_per_channel(FORMAT)], int c)
+{
+    constexpr int BPC = bytes_per_channel(FORMAT);
+    uint32_t const w = words[(c * BPC) >> 2] >> (8 * ((c * BPC) & 3));
+    if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_UNORM8)       return divide_by_top(float(w & 0xffu), 255.f, 1.f / 255.f);
+    else if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_UNORM16) return divide_by_top(float(w & 0xffffu), 65535.f, 1.f / 65535.f);
+    else if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_FLOAT16) return float(__builtin_bit_cast(_Float16, uint16_t(w)));
+    else                                                     return __builtin_bit_cast(float, w);
+}
+
+// FORMAT: of both images, four channels each; 0: any two images.
+template <int FORMAT, bool MSLE>
 __global__ void __launch_bounds__(256)
-image_difference_kernel(ImageDifferenceArgs a)
+image_difference_kernel(ImageDifferenceArgs a, int tilesX, int tiles)
 {
     __shared__ float sums[4][4];
     int const lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int const x = blockIdx.x * 64 + lane;
-    float mse[4] = { 0.f, 0.f, 0.f, 0.f };
-    for (int r = 0; r < 16; ++r) {
-        int const y = blockIdx.y * 64 + wave * 16 + r;
-        if (x >= a.width || y >= a.height) continue;
-        uint8_t const* const pa = a.a.data + size_t(y + a.top) * a.a.rowPitch + size_t(x + a.left) * a.a.pixelStride;
-        uint8_t const* const pb = a.b.data + size_t(y + a.top) * a.b.rowPitch + size_t(x + a.left) * a.b.pixelStride;
-        float t1[4], t2[4], diff[4];
+    unsigned long long fixed = 0;                            // threads 0 ... 3: the workgroup's share of a channel's sum
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        int const tileY = tile / tilesX, tileX = tile - tileY * tilesX;
+        int const x = tileX * 64 + lane, yBegin = tileY * 64 + wave * 16;
+        float mse[4] = { 0.f, 0.f, 0.f, 0.f };
+        auto add_pixel = [&](float const (&t1)[4], float const (&t2)[4]) {
+            float diff[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) { t1[c] = diff_channel(a.a, pa, c); t2[c] = diff_channel(a.b, pb, c); }
+            for (int c = 0; c < 4; ++c)
+                diff[c] = MSLE ? __fsub_rn(logf(fabsf(t1[c]) + 1.f), logf(fabsf(t2[c]) + 1.f)) : __fsub_rn(t1[c], t2[c]);
+            if (a.useAlphaThreshold && t1[3] < a.alphaThreshold && t2[3] < a.alphaThreshold) { diff[0] = 0.f; diff[1] = 0.f; diff[2] = 0.f; }
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            diff[c] = a.useMSLE ? __fsub_rn(logf(fabsf(t1[c]) + 1.f), logf(fabsf(t2[c]) + 1.f)) : __fsub_rn(t1[c], t2[c]);
-        if (a.useAlphaThreshold && t1[3] < a.alphaThreshold && t2[3] < a.alphaThreshold) { diff[0] = 0.f; diff[1] = 0.f; diff[2] = 0.f; }
+            for (int c = 0; c < 4; ++c) mse[c] = __fadd_rn(mse[c], __fmul_rn(diff[c], diff[c]));
+        };
+        if constexpr (FORMAT != 0) {
+            constexpr int BPC = bytes_per_channel(FORMAT), ROWS = BPC == 1 ? 16 : BPC == 2 ? 8 : 4;
+            int const xIn = min(x, a.width - 1) + a.left;    // (pixels outside the extent are read inside it and dropped)
+            for (int first = 0; first < 16 && yBegin + first < a.height; first += ROWS) {
+                uint32_t wa[ROWS][BPC], wb[ROWS][BPC];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) mse[c] = __fadd_rn(mse[c], __fmul_rn(diff[c], diff[c]));
+                for (int r = 0; r < ROWS; ++r) {
+                    size_t const y = size_t(min(yBegin + first + r, a.height - 1) + a.top);
+                    load_pixel<FORMAT>(a.a.data + y * a.a.rowPitch + size_t(xIn) * a.a.pixelStride, wa[r]);
+                    load_pixel<FORMAT>(a.b.data + y * a.b.rowPitch + size_t(xIn) * a.b.pixelStride, wb[r]);
+                }
+                __builtin_amdgcn_sched_barrier(0);           // keep the loads ahead of the arithmetic
+#pragma unroll
+                for (int r = 0; r < ROWS; ++r) {
+                    if (x >= a.width || yBegin + first + r >= a.height) continue;
+                    float t1[4], t2[4];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) { t1[c] = pixel_channel<FORMAT>(wa[r], c); t2[c] = pixel_channel<FORMAT>(wb[r], c); }
+                    add_pixel(t1, t2);
+                }
+            }
+        } else {
+            for (int r = 0; r < 16; ++r) {
+                int const y = yBegin + r;
+                if (x >= a.width || y >= a.height) continue;
+                uint8_t const* const pa = a.a.data + size_t(y + a.top) * a.a.rowPitch + size_t(x + a.left) * a.a.pixelStride;
+                uint8_t const* const pb = a.b.data + size_t(y + a.top) * a.b.rowPitch + size_t(x + a.left) * a.b.pixelStride;
+                float t1[4], t2[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) { t1[c] = diff_channel(a.a, pa, c); t2[c] = diff_channel(a.b, pb, c); }
+                add_pixel(t1, t2);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            float v = mse[c];
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) v = __fadd_rn(v, __shfl_xor(v, off, 64));
+            if (lane == 0) sums[wave][c] = v;
+        }
+        __syncthreads();
+        if (threadIdx.x < 4) {
+            int const c = threadIdx.x;
+            float total = __fadd_rn(__fadd_rn(__fadd_rn(sums[0][c], sums[1][c]), sums[2][c]), sums[3][c]);
+            total = __fdiv_rn(total, float(a.width * a.height));
+            total = __fmul_rn(total, 65536.f);
+            float const whole = floorf(total);
+            // float -> uint32 conversions saturate; a NaN (from NaN pixels) adds nothing
+            unsigned long long const high = uint32_t(whole), low = uint32_t(floorf(__fmul_rn(__fsub_rn(total, whole), 4294967296.f)));
+            fixed += (high << 32) | low;
+        }
+        __syncthreads();
     }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        float v = mse[c];
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) v = __fadd_rn(v, __shfl_xor(v, off, 64));
-        if (lane == 0) sums[wave][c] = v;
-    }
-    __syncthreads();
-    if (threadIdx.x < 4) {
-        int const c = threadIdx.x;
-        float total = __fadd_rn(__fadd_rn(__fadd_rn(sums[0][c], sums[1][c]), sums[2][c]), sums[3][c]);
-        total = __fdiv_rn(total, float(a.width * a.height));
-        total = __fmul_rn(total, 65536.f);
-        float const whole = floorf(total);
-        // float -> uint32 conversions saturate; a NaN (from NaN pixels) adds nothing
-        unsigned long long const high = uint32_t(whole), low = uint32_t(floorf(__fmul_rn(__fsub_rn(total, whole), 4294967296.f)));
-        unsigned long long const fixed = (high << 32) | low;
-        if (fixed) atomicAdd(a.output + c, fixed);
-    }
+    if (threadIdx.x < 4 && fixed) atomicAdd(a.output + threadIdx.x, fixed);
 }
 
 hipError_t launch_image_difference(ImageDifferenceArgs const& a, hipStream_t stream)
 {
-    dim3 const grid((a.width + 63) / 64, (a.height + 63) / 64);
-    hipLaunchKernelGGL(image_difference_kernel, grid, dim3(256), 0, stream, a);
+    int const tilesX = (a.width + 63) / 64, tiles = tilesX * ((a.height + 63) / 64);
+    int const resident = 4 * compute_units_of_current_device();
+    dim3 const grid(unsigned(tiles < resident ? tiles : resident));
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, a, tilesX, tiles); };
+    auto of_format = [&](auto format) {
+        constexpr int FORMAT = decltype(format)::value;
+        if (a.useMSLE) launch(image_difference_kernel<FORMAT, true>);
+        else           launch(image_difference_kernel<FORMAT, false>);
+    };
+    bool const alike = a.a.format == a.b.format && a.a.numChannels == 4 && a.b.numChannels == 4;
+    if (alike && a.a.format == NTC_HIP_DEV_FORMAT_UNORM8)       of_format(std::integral_constant<int, NTC_HIP_DEV_FORMAT_UNORM8>{});
+    else if (alike && a.a.format == NTC_HIP_DEV_FORMAT_UNORM16) of_format(std::integral_constant<int, NTC_HIP_DEV_FORMAT_UNORM16>{});
+    else if (alike && a.a.format == NTC_HIP_DEV_FORMAT_FLOAT16) of_format(std::integral_constant<int, NTC_HIP_DEV_FORMAT_FLOAT16>{});
+    else if (alike && a.a.format == NTC_HIP_DEV_FORMAT_FLOAT32) of_format(std::integral_constant<int, NTC_HIP_DEV_FORMAT_FLOAT32>{});
+    else                                                        of_format(std::integral_constant<int, 0>{});
     return hipGetLastError();
 }
 
