@@ -1033,15 +1033,60 @@ hipError_t launch_write_channels(WriteChannelsArgs const& args, hipStream_t stre
 // clamped (Inference.cu:96-97,112; a negative zero becomes +0 as the device max() of the reference
 // returns), and with discardMaskedOut a texel whose REFERENCE mask value is zero counts on the mask
 // channel only (Inference.cu:80-84,107-108).
-// A lane takes PX adjacent texels (2 when the width is even: 8-byte loads) of kLossRowsPerWave rows; all
+// A lane takes PX adjacent texels (2 when the width is even: 8-byte loads) of rowsPerWave rows; all
 // loads of a row are issued before its arithmetic.  Squares are fp32 as in the reference; their sum over the
-// lane's texels of a row goes into a double accumulator, and the workgroup writes 16 double partial sums
-// (channel-major, so that the second stage reads them coalesced); ReduceLoss likewise finishes in
-// double (src/Optimizer.cu:382-387).
+// lane's texels of a row goes into a double accumulator, and the workgroup writes 16 double partial sums;
+// ReduceLoss likewise finishes in double (src/Optimizer.cu:382-387).
+//
+// The same launch finishes the sum and hands it to the host: the last of every kLossGroup workgroups to arrive adds
+// the group's partial sums, the last group to finish adds those of the groups (each in a fixed order, so results are
+// reproducible) and writes the 16 totals and a serial number into pinned host memory, where the caller is looking
+// (a second kernel, a copy and a stream synchronisation made most of the 28 us a call on 64 x 64 texels took; 14 now.
+// 4096 x 4096 texels of 16 channels: 192 us, 5.6 TB/s).
+// The partial sums pass between workgroups of different dies, whose caches do not see each other: they are stored and
+// loaded as device-scope atomics, which go past those caches, and a store is acknowledged before its workgroup counts
+// itself as arrived.  (Fences instead write back and invalidate a die's whole L2, a thousand times in a launch over
+// 2048 x 2048 texels: 154 us against 50.)
+__device__ __forceinline__ void publish(double* to, double v) { __hip_atomic_store(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ double published(double const* from) { return __hip_atomic_load(from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// Sums over the workgroup of the 16 channels' terms entries[i * 16 + channel], i < count, in a fixed order.
+__device__ __forceinline__ double sum_entries(double const* entries, int count, double (&scratch)[16][NTC_HIP_DEV_MAX_CHANNELS])
+{
+    int const c = threadIdx.x & 15, part = threadIdx.x >> 4;                     // 16 threads per channel
+    double v = 0.0;
+    for (int i = part; i < count; i += 16) v += published(entries + size_t(i) * NTC_HIP_DEV_MAX_CHANNELS + c);
+    scratch[part][c] = v;
+    __syncthreads();
+    double total = 0.0;
+    if (threadIdx.x < NTC_HIP_DEV_MAX_CHANNELS)
+#pragma unroll
+        for (int k = 0; k < 16; ++k) total += scratch[k][c];
+    return total;                                            // in threads 0 ... 15
+}
+
+// Whether this workgroup is the last of `count` to come here (uniform), after its first wave has published its sums.
+__device__ __forceinline__ bool arrived_last(uint32_t* counter, uint32_t count, int& scratch)
+{
+    __syncthreads();
+    if (threadIdx.x < 64) {                                  // the wave whose stores have to be in place
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0);
+        asm volatile("" ::: "memory");
+        if (threadIdx.x == 0) {
+            bool const last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == count - 1u;
+            if (last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // as the next launch expects it
+            scratch = last;
+        }
+    }
+    __syncthreads();
+    return scratch != 0;
+}
+
 template <int PX, bool MASKED>
 __global__ void __launch_bounds__(256)
-image_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int width, int height, int setChannels,
-                  uint32_t validChannelMask, int maskChannel, int discardMaskedOut, double* __restrict__ partials)
+image_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int width, int height, int setChannels, int rowsPerWave,
+                  uint32_t validChannelMask, int maskChannel, int discardMaskedOut, LossWorkspace work)
 {
     constexpr int PAIRS = NTC_HIP_DEV_MAX_CHANNELS / 2;
     __shared__ double sums[4][NTC_HIP_DEV_MAX_CHANNELS];
@@ -1051,8 +1096,8 @@ image_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int 
     double acc[NTC_HIP_DEV_MAX_CHANNELS];
 #pragma unroll
     for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) acc[c] = 0.0;
-    for (int r = 0; r < kLossRowsPerWave; ++r) {
-        int const y = (blockIdx.y * 4 + wave) * kLossRowsPerWave + r;
+    for (int r = 0; r < rowsPerWave; ++r) {
+        int const y = (blockIdx.y * 4 + wave) * rowsPerWave + r;
         if (x >= width || y >= height) continue;             // width is a multiple of PX
         size_t const base = size_t(y) * size_t(width) * size_t(setChannels) + size_t(x) * 2;
         uint32_t va[PAIRS][PX], vb[PAIRS][PX];
@@ -1111,59 +1156,63 @@ image_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int 
         }
     }
 #pragma unroll
-    for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) {
-        double v = (c < setChannels && ((validChannelMask >> c) & 1u)) ? acc[c] : 0.0;
+    for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c)
+        if (c >= setChannels || !((validChannelMask >> c) & 1u)) acc[c] = 0.0;
+    // Across the lanes by halving: partners 32, 16, 8 and 4 lanes apart each keep one half of the channels they both
+    // have and hand over the other, after which every lane has one channel; the last two steps add whole values.  17
+    // exchanges of a double instead of the 96 of one butterfly per channel.
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-        if (lane == 0) sums[wave][c] = v;
+    for (int n = 8, off = 32; n >= 1; n >>= 1, off >>= 1) {
+        bool const upper = (lane & off) != 0;
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+            double const keep = upper ? acc[i + n] : acc[i], give = upper ? acc[i] : acc[i + n];
+            acc[i] = keep + __shfl_xor(give, off, 64);
+        }
     }
+    double mine = acc[0] + __shfl_xor(acc[0], 2, 64);
+    mine += __shfl_xor(mine, 1, 64);
+    if ((lane & 3) == 0) sums[wave][lane >> 2] = mine;       // bits 5 ... 2 of the lane number are its channel's, most significant first
     __syncthreads();
+    uint32_t const block = blockIdx.y * gridDim.x + blockIdx.x, blocks = gridDim.x * gridDim.y;
+    uint32_t const group = block / kLossGroup, groups = (blocks + kLossGroup - 1) / kLossGroup, first = group * kLossGroup;
+    double total = 0.0;                                      // threads 0 ... 15
     if (threadIdx.x < NTC_HIP_DEV_MAX_CHANNELS) {
         int const c = threadIdx.x;
-        size_t const block = size_t(blockIdx.y) * gridDim.x + blockIdx.x, blocks = size_t(gridDim.x) * gridDim.y;
-        partials[size_t(c) * blocks + block] = sums[0][c] + sums[1][c] + sums[2][c] + sums[3][c];
+        total = sums[0][c] + sums[1][c] + sums[2][c] + sums[3][c];
+        if (blocks > 1) publish(work.partials + size_t(block) * NTC_HIP_DEV_MAX_CHANNELS + c, total);
     }
-}
-
-// Second stage: workgroup c adds the partial sums of channel c, in double and in a fixed order
-// (thread t takes entries t, t + 256, ... into four interleaved sub-totals; then one thread adds the
-// 256 thread totals), and writes the total behind the partials.
-__global__ void __launch_bounds__(256)
-image_loss_reduce_kernel(double const* __restrict__ partials, size_t blocks, double* __restrict__ totals)
-{
-    __shared__ double sums[256];
-    double const* const mine = partials + size_t(blockIdx.x) * blocks;
-    double acc[4] = { 0.0, 0.0, 0.0, 0.0 };
-    size_t b = threadIdx.x;
-    for (; b + 768 < blocks; b += 1024) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) acc[k] += mine[b + size_t(k) * 256];
+    __shared__ double scratch[16][NTC_HIP_DEV_MAX_CHANNELS];
+    __shared__ int last;
+    if (blocks > 1) {
+        int const members = int(min(uint32_t(kLossGroup), blocks - first));
+        if (!arrived_last(work.counters + 1 + group, uint32_t(members), last)) return;
+        total = sum_entries(work.partials + size_t(first) * NTC_HIP_DEV_MAX_CHANNELS, members, scratch);
     }
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-        if (b + size_t(k) * 256 < blocks) acc[k] += mine[b + size_t(k) * 256];
-    sums[threadIdx.x] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    if (groups > 1) {
+        if (threadIdx.x < NTC_HIP_DEV_MAX_CHANNELS) publish(work.groupSums + size_t(group) * NTC_HIP_DEV_MAX_CHANNELS + threadIdx.x, total);
+        if (!arrived_last(work.counters, groups, last)) return;
+        total = sum_entries(work.groupSums, int(groups), scratch);
+    }
+    if (threadIdx.x < NTC_HIP_DEV_MAX_CHANNELS) work.result->totals[threadIdx.x] = total;
     __syncthreads();
     if (threadIdx.x == 0) {
-        double total = 0.0;
-        for (int t = 0; t < 256; ++t) total += sums[t];
-        totals[blockIdx.x] = total;
+        __threadfence_system();
+        __hip_atomic_store(&work.result->serial, work.serial, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
-hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int height, int setChannels,
-                             uint32_t validChannelMask, int maskChannel, int discardMaskedOut, double* partials, hipStream_t stream)
+hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int height, int setChannels, uint32_t validChannelMask,
+                             int maskChannel, int discardMaskedOut, LossWorkspace const& work, hipStream_t stream)
 {
-    dim3 const grid = image_loss_grid(width, height);
-    size_t const blocks = size_t(grid.x) * size_t(grid.y);
+    LossGrid const grid = image_loss_grid(width, height, compute_units_of_current_device());
     bool const two = (width & 1) == 0, masked = maskChannel >= 0;
     auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, a, b, width, height, setChannels, validChannelMask,
-                           maskChannel, discardMaskedOut, partials);
+        hipLaunchKernelGGL(kernel, dim3(grid.x, grid.y), dim3(256), 0, stream, a, b, width, height, setChannels, grid.rowsPerWave,
+                           validChannelMask, maskChannel, discardMaskedOut, work);
     };
     if (two) { if (masked) launch(image_loss_kernel<2, true>); else launch(image_loss_kernel<2, false>); }
     else     { if (masked) launch(image_loss_kernel<1, true>); else launch(image_loss_kernel<1, false>); }
-    hipLaunchKernelGGL(image_loss_reduce_kernel, dim3(NTC_HIP_DEV_MAX_CHANNELS), dim3(256), 0, stream, partials, blocks, partials + blocks * NTC_HIP_DEV_MAX_CHANNELS);
     return hipGetLastError();
 }
 

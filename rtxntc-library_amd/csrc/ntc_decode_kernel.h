@@ -113,20 +113,29 @@ struct WriteChannelsArgs {
 hipError_t launch_write_channels(WriteChannelsArgs const& args, hipStream_t stream);
 
 // Grid of the loss kernel: a workgroup (= one row of 16 double partial sums) covers 64 lanes x 1 or 2
-// texels (2 when the width is even) by 4 waves x kLossRowsPerWave rows.
-constexpr int kLossRowsPerWave = 8;
-inline dim3 image_loss_grid(int width, int height)
+// texels (2 when the width is even) by 4 waves x rowsPerWave rows.  Four workgroups are resident on a compute unit; as
+// many rows per wave as make the grid about that large (every workgroup ends in 16 reductions across its lanes, and a
+// row is a memory round trip), from one, for images that would not fill the GPU, to 32.
+struct LossGrid { uint32_t x, y; int32_t rowsPerWave; };
+inline LossGrid image_loss_grid(int width, int height, int computeUnits)
 {
-    int const perLane = (width & 1) ? 1 : 2;
-    return dim3((width + 64 * perLane - 1) / (64 * perLane), (height + 4 * kLossRowsPerWave - 1) / (4 * kLossRowsPerWave));
+    uint32_t const perLane = (width & 1) ? 1u : 2u, x = (uint32_t(width) + 64u * perLane - 1u) / (64u * perLane);
+    uint64_t const quads = (uint32_t(height) + 3u) / 4u;
+    uint64_t const wanted = (quads * x + uint64_t(4 * computeUnits) - 1u) / uint64_t(4 * computeUnits);
+    uint32_t const rows = uint32_t(wanted < 1u ? 1u : wanted > 32u ? 32u : wanted);
+    return LossGrid{ x, (uint32_t(height) + 4u * rows - 1u) / (4u * rows), int32_t(rows) };
 }
-inline size_t image_loss_blocks(int width, int height)
-{
-    dim3 const grid = image_loss_grid(width, height);
-    return size_t(grid.x) * size_t(grid.y);
-}
-hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int height, int setChannels,
-                             uint32_t validChannelMask, int maskChannel, int discardMaskedOut, double* partials, hipStream_t stream);
+constexpr uint32_t kLossGroup = 32;                         // workgroups whose partial sums are added first
+struct LossResult { double totals[16]; uint32_t serial; };  // pinned host memory
+struct LossWorkspace {
+    double* partials;              // 16 per workgroup
+    double* groupSums;             // 16 per kLossGroup workgroups
+    uint32_t* counters;            // one, then one per kLossGroup workgroups: zero before and after every launch
+    LossResult* result;            // device address; `serial` is stored last
+    uint32_t serial;
+};
+hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int height, int setChannels, uint32_t validChannelMask,
+                             int maskChannel, int discardMaskedOut, LossWorkspace const& work, hipStream_t stream);
 
 hipError_t launch_resize_planar(uint16_t const* src, int srcWidth, int srcHeight, uint16_t* dst, int dstWidth, int dstHeight,
                                 int setChannels, uint8_t const* colorSpaces, hipStream_t stream);

@@ -11,6 +11,7 @@
 #include <cstring>
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -81,9 +82,11 @@ struct NtcHipContext {
     uint32_t handoffSerial = 0;        // changes with every pair of such launches
     size_t tableCapacity = 0;          // entries
     std::vector<DevMip> lastTable;     // what tableDev currently holds (or will, in stream order)
-    double* lossDev = nullptr;         // per-workgroup partial sums of the loss pass
-    double* lossHost = nullptr;        // pinned copy of them
-    size_t lossBytes = 0;
+    double* lossDev = nullptr;         // partial sums of the loss pass: 16 per workgroup, then 16 per group of workgroups
+    size_t lossBlocks = 0;             // workgroups it has room for
+    uint32_t* lossCounters = nullptr;  // arrivals, zero between calls
+    LossResult* lossHost = nullptr;    // pinned: what the loss pass hands to the host
+    uint32_t lossSerial = 0;
     static constexpr int kSlots = 4;
     struct Slot { DevMip* host = nullptr; size_t capacity = 0; hipEvent_t done = nullptr; bool inFlight = false; };
     Slot slots[kSlots];                // pinned staging for asynchronous table uploads
@@ -576,6 +579,7 @@ static void destroy_context(NtcHipContext* L)
     if (L->tableDev) (void)hipFree(L->tableDev);
     if (L->handoffDev) (void)hipFree(L->handoffDev);
     if (L->lossDev) (void)hipFree(L->lossDev);
+    if (L->lossCounters) (void)hipFree(L->lossCounters);
     if (L->lossHost) (void)hipHostFree(L->lossHost);
     for (Library::Slot& slot : L->slots) {
         if (slot.host) (void)hipHostFree(slot.host);
@@ -1021,24 +1025,45 @@ int ntc_hip_ctx_image_loss(NtcHipContext* ctx, void* decoded, const void* refere
             return NTC_HIP_ERR_INVALID_ARG;
         }
     }
-    size_t const blocks = image_loss_blocks(width, height);
-    size_t const bytes = (blocks + 1) * NTC_HIP_DEV_MAX_CHANNELS * sizeof(double);    // partial sums, then the 16 totals
-    if (bytes > L.lossBytes) {
+    LossGrid const grid = image_loss_grid(width, height, L.computeUnits);
+    size_t const blocks = size_t(grid.x) * grid.y, groups = (blocks + kLossGroup - 1) / kLossGroup;
+    if (blocks > L.lossBlocks) {
         HIP_TRY(hipStreamSynchronize(L.stream));
         if (L.lossDev) { HIP_TRY(hipFree(L.lossDev)); L.lossDev = nullptr; }
-        L.lossBytes = 0;
-        HIP_TRY(hipMalloc(reinterpret_cast<void**>(&L.lossDev), bytes));
-        if (!L.lossHost) HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&L.lossHost), NTC_HIP_DEV_MAX_CHANNELS * sizeof(double), hipHostMallocDefault));
-        L.lossBytes = bytes;
+        if (L.lossCounters) { HIP_TRY(hipFree(L.lossCounters)); L.lossCounters = nullptr; }
+        L.lossBlocks = 0;
+        HIP_TRY(hipMalloc(reinterpret_cast<void**>(&L.lossDev), (blocks + groups) * NTC_HIP_DEV_MAX_CHANNELS * sizeof(double)));
+        HIP_TRY(hipMalloc(reinterpret_cast<void**>(&L.lossCounters), (1 + groups) * sizeof(uint32_t)));
+        HIP_TRY(launch_fill(reinterpret_cast<uint8_t*>(L.lossCounters), 0, (1 + groups) * sizeof(uint32_t), L.stream));
+        if (!L.lossHost) {
+            HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&L.lossHost), sizeof(LossResult), hipHostMallocMapped | hipHostMallocCoherent));
+            L.lossHost->serial = 0;
+        }
+        L.lossBlocks = blocks;
     }
+    LossWorkspace work{};
+    work.partials = L.lossDev;
+    work.groupSums = L.lossDev + blocks * NTC_HIP_DEV_MAX_CHANNELS;
+    work.counters = L.lossCounters;
+    work.serial = ++L.lossSerial;
+    HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void**>(&work.result), L.lossHost, 0));
     HIP_TRY(launch_image_loss(static_cast<uint16_t*>(decoded), static_cast<uint16_t const*>(reference), width, height,
                               setChannels, validChannelMask, maskChannelIndex < 0 ? -1 : maskChannelIndex,
-                              discardMaskedOutPixels ? 1 : 0, L.lossDev, L.stream));
-    HIP_TRY(hipMemcpyAsync(L.lossHost, L.lossDev + blocks * NTC_HIP_DEV_MAX_CHANNELS, NTC_HIP_DEV_MAX_CHANNELS * sizeof(double),
-                           hipMemcpyDeviceToHost, L.stream));
-    HIP_TRY(hipStreamSynchronize(L.stream));
+                              discardMaskedOutPixels ? 1 : 0, work, L.stream));
+    // The kernel's last act is to store the serial number behind the totals.  Most calls are done in microseconds, so
+    // the host looks for it; one that takes longer (work queued in front of it), or an error, is left to the stream.
+    // So is a call with a mask channel, which changes the decoded image: it returns when that is complete.
+    auto const begin = std::chrono::steady_clock::now();
+    if (maskChannelIndex >= 0) HIP_TRY(hipStreamSynchronize(L.stream));
+    while (__atomic_load_n(&L.lossHost->serial, __ATOMIC_ACQUIRE) != work.serial) {
+        __builtin_ia32_pause();
+        if (std::chrono::steady_clock::now() - begin > std::chrono::milliseconds(2)) {
+            HIP_TRY(hipStreamSynchronize(L.stream));
+            break;
+        }
+    }
     double const norm = 1.0 / (double(width) * double(height));
-    for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) outMse[c] = float(L.lossHost[c] * norm);
+    for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) outMse[c] = float(L.lossHost->totals[c] * norm);
     clear_error();
     return 0;
 }

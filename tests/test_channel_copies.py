@@ -118,3 +118,20 @@ def test_resized_colour_channels_equal_their_parts(ntc, device, space, w, h):
         device.synchronize()
         want = d_out.download().view(np.uint16).reshape(h // 2, w // 2, 2)[:, :, 0]
         assert np.array_equal(got[:, channel // 2, :, channel % 2], want), channel
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (128, 4), (128, 8), (129, 5), (256, 127), (1024, 1028), (4100, 33)])
+def test_loss_sums_of_one_group_and_of_many(ntc, device, oracle, w, h):
+    """One workgroup, one group of workgroups, several groups, one row a wave and more: twice, so that the arrival
+    counters are found as they were left."""
+    rng = np.random.default_rng(w + h)
+    a, b = halves(rng, w * h * 6), halves(rng, w * h * 6)
+    d_a, d_b = device.upload(a), device.upload(b)
+    want = np.zeros(16, dtype=np.float64)
+    oracle.ntc_oracle_image_loss(a.ctypes.data, b.ctypes.data, w, h, 6, 0x37, want.ctypes.data)
+    results = []
+    for _ in range(2):
+        got = (ntc.abi.C.c_float * 16)()
+        device.call("image_loss", d_a.ptr, d_b.ptr, d_a.nbytes, w, h, 6, 0x37, -1, 0, got)
+        results.append(np.array(got[:]))
+    assert np.allclose(results[0], want, rtol=2e-7, atol=0) and np.array_equal(results[0], results[1])
