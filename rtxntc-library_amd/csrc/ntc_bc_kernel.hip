@@ -36,94 +36,111 @@ namespace ntc_hip_dev {
 
 namespace {
 
-// The eight values a block's two endpoints stand for (integer interpolation with the reference's
-// rounding bias: +3 before /7, +2 before /5).
-__device__ __forceinline__ void bc4_palette(uint32_t e0, uint32_t e1, uint32_t (&p)[8])
-{
-    p[0] = e0; p[1] = e1;
-    if (e0 > e1) {
-#pragma unroll
-        for (uint32_t k = 1; k < 7; ++k) p[k + 1] = ((7 - k) * e0 + k * e1 + 3) / 7;
-    } else {
-#pragma unroll
-        for (uint32_t k = 1; k < 5; ++k) p[k + 1] = ((5 - k) * e0 + k * e1 + 2) / 5;
-        p[6] = 0; p[7] = 255;
+// A block's endpoints, and its sixteen 3-bit indices in two words of eight.
+struct Bc4 {
+    uint32_t e0, e1, low, high;
+    __device__ __forceinline__ uint64_t bits() const
+    {
+        return uint64_t(e0) | (uint64_t(e1) << 8) | (uint64_t(low) << 16) | (uint64_t(high) << 40);
     }
-}
+};
 
-// Block = endpoint 0 | endpoint 1 << 8 | sixteen 3-bit indices from bit 16 up.
-__device__ __forceinline__ uint64_t bc4_with_endpoints(uint64_t block, uint32_t e0, uint32_t e1)
+// The eight values that two endpoints stand for, times eight.  With e0 > e1 entry k + 1 is ((7 - k) e0 + k e1 + 3) / 7,
+// else ((5 - k) e0 + k e1 + 2) / 5 and the last two are 0 and 255 (the reference's rounding biases); a product and a
+// shift are those quotients for every numerator that occurs.
+__device__ __forceinline__ void bc4_palette8(uint32_t e0, uint32_t e1, uint32_t (&p)[8])
 {
-    return (block & ~uint64_t(0xffff)) | uint64_t(e0 & 0xffu) | (uint64_t(e1 & 0xffu) << 8);
+    bool const eight = e0 > e1;
+    uint32_t const multiplier = eight ? 9363u : 13108u, step = e1 - e0;
+    uint32_t n = eight ? 7u * e0 + 3u : 5u * e0 + 2u;
+    p[0] = e0 << 3; p[1] = e1 << 3;
+#pragma unroll
+    for (int k = 2; k < 8; ++k) {
+        n += step;
+        p[k] = (__umul24(n, multiplier) >> 13) & ~7u;
+    }
+    if (!eight) { p[6] = 0u; p[7] = 255u << 3; }
 }
-__device__ __forceinline__ uint32_t bc4_index(uint64_t block, int texel) { return uint32_t(block >> (16 + 3 * texel)) & 7u; }
 
 // Nearest palette entry for every texel (the first of equally near ones); returns the summed squared error.
-__device__ __forceinline__ float bc4_assign(uint32_t const (&values)[16], uint64_t& block)
+// values8: the texels times eight, so that |value - entry| * 8 + k is one instruction per entry: the smallest of these
+// keys is the nearest entry, the first among equally near ones.  keys: the chosen ones.
+__device__ __forceinline__ uint32_t bc4_assign(uint32_t const (&values8)[16], Bc4& block, uint32_t (&keys)[16])
 {
-    uint32_t palette[8];
-    bc4_palette(uint32_t(block) & 0xffu, (uint32_t(block) >> 8) & 0xffu, palette);
-    block &= 0xffff;
-    float total = 0.f;
+    uint32_t p[8];
+    bc4_palette8(block.e0, block.e1, p);
+    uint32_t total = 0;
+    block.low = block.high = 0;
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-        // key = distance * 8 + entry: the smallest key is the nearest entry, the first among equally near ones
+    for (int t = 15; t >= 0; --t) {
         uint32_t key[8];
 #pragma unroll
-        for (uint32_t k = 0; k < 8; ++k) key[k] = (__sad(int(values[t]), int(palette[k]), 0u) << 3) + k;
-        uint32_t const best = min(min(min(key[0], key[1]), min(key[2], key[3])), min(min(key[4], key[5]), min(key[6], key[7])));
+        for (uint32_t k = 0; k < 8; ++k) key[k] = __usad(values8[t], p[k], k);
+        uint32_t const best = min3_u32(min3_u32(key[0], key[1], key[2]), min3_u32(key[3], key[4], key[5]), min(key[6], key[7]));
         uint32_t const distance = best >> 3;
-        total += float(distance * distance);
-        block |= uint64_t(best & 7u) << (16 + 3 * t);
+        total += __umul24(distance, distance);               // at most 16 * 255^2: exact as the float sum it stands for
+        uint32_t& word = t < 8 ? block.low : block.high;
+        word = (word << 3) | (best & 7u);
+        keys[t] = best;
     }
     return total;
 }
 
 __device__ __forceinline__ uint32_t bc4_endpoint(float v) { return uint32_t(rintf(fminf(fmaxf(v, 0.f), 255.f))); }   // a NaN becomes 0
 
-// Weight of endpoint 0 in palette entry k, for the eight-value and the six-value palette (entries 6 and 7
-// of the latter are the constants 0 and 255 and take no part in a fit): the quotients the fit divides
-// out, (8 - k) / 7 and (6 - k) / 5, evaluated once by the compiler.
-__constant__ float kWeight8[8] = { 1.f, 0.f, 6.f / 7.f, 5.f / 7.f, 4.f / 7.f, 3.f / 7.f, 2.f / 7.f, 1.f / 7.f };
-__constant__ float kWeight6[8] = { 1.f, 0.f, 4.f / 5.f, 3.f / 5.f, 2.f / 5.f, 1.f / 5.f, 0.f, 0.f };
-
-// Least-squares endpoints for the block's current assignment.  With `eightValues` every texel takes
-// part and weights are 1, 0, 6/7 ... 1/7; otherwise indices 6 and 7 (the fixed 0 and 255) are left
-// out and weights are 1, 0, 4/5 ... 1/5, and a singular system leaves the endpoints alone.
-__device__ __forceinline__ uint64_t bc4_refit(uint32_t const (&values)[16], uint64_t block, bool eightValues, bool keep255, bool keep0)
+// Least-squares endpoints for the block's current assignment.  EIGHT: every texel takes part and the weights of
+// endpoint 0 are 1, 0, 6/7 ... 1/7; otherwise indices 6 and 7 (the fixed 0 and 255) are left out and the weights are
+// 1, 0, 4/5 ... 1/5, and a singular system leaves the endpoints alone.  The numerators are bytes of a permute, and
+// w / 7 as w * hi + w * lo with hi + lo = 1/7, w / 5 as w * (1/5), are the correctly rounded quotients for all of them.
+// (Weights from a table in constant memory were a gather per texel and round.)
+template <bool EIGHT>
+__device__ __forceinline__ void bc4_refit(uint32_t const (&values8)[16], uint32_t const (&keys)[16], Bc4& block, bool keep255, bool keep0)
 {
     float aa = 0.f, bb = 0.f, ab = 0.f, ax = 0.f, bx = 0.f;
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
-        uint32_t const k = bc4_index(block, t);
-        if (!eightValues && k >= 6) continue;
-        float const alpha = eightValues ? kWeight8[k] : kWeight6[k];
-        float const beta = 1.f - alpha, x = float(values[t]);
+        uint32_t const select = (keys[t] & 7u) | 0x0c0c0c00u;                    // upper bytes: zero
+        float alpha, beta;
+        if constexpr (EIGHT) {
+            float const w = float(__builtin_amdgcn_perm(0x01020304u, 0x05060007u, select) & 0xffu);
+            alpha = __builtin_fmaf(w, 1.f / 7.f, w * float(1.0 / 7.0 - double(1.f / 7.f)));
+            beta = 1.f - alpha;
+        } else {
+            float const w = float(__builtin_amdgcn_perm(0x00000102u, 0x03040005u, select) & 0xffu);
+            alpha = w * (1.f / 5.f);
+            beta = (keys[t] & 7u) >= 6u ? 0.f : 1.f - alpha;                     // adding zeros is leaving the texel out
+        }
+        float const x = float(values8[t] >> 3);
         aa += alpha * alpha; bb += beta * beta; ab += alpha * beta;
         ax += alpha * x; bx += beta * x;
     }
-    if (eightValues) {
+    if constexpr (EIGHT) {
         float const factor = 1.f / (aa * bb - ab * ab);
-        uint32_t e0 = keep255 ? 255u : bc4_endpoint((ax * bb - bx * ab) * factor);
-        uint32_t e1 = keep0 ? 0u : bc4_endpoint((bx * aa - ax * ab) * factor);
-        if (e0 < e1) { uint32_t const t = e0; e0 = e1; e1 = t; }
-        return bc4_with_endpoints(block, e0, e1);
+        uint32_t const e0 = keep255 ? 255u : bc4_endpoint((ax * bb - bx * ab) * factor);
+        uint32_t const e1 = keep0 ? 0u : bc4_endpoint((bx * aa - ax * ab) * factor);
+        block.e0 = max(e0, e1); block.e1 = min(e0, e1);
+    } else {
+        float const det = aa * bb - ab * ab;
+        if (det == 0.f) return;
+        block.e0 = bc4_endpoint((ax * bb - bx * ab) / det);
+        block.e1 = bc4_endpoint((bx * aa - ax * ab) / det);
     }
-    float const det = aa * bb - ab * ab;
-    if (det == 0.f) return block;
-    return bc4_with_endpoints(block, bc4_endpoint((ax * bb - bx * ab) / det), bc4_endpoint((bx * aa - ax * ab) / det));
 }
 
-// Up to eight rounds of refit + re-assign from a starting block; returns the best block and its error.
-__device__ __forceinline__ uint64_t bc4_refine(uint32_t const (&values)[16], uint64_t block, bool eightValues, bool keep255, bool keep0, float& bestError)
+// Up to eight rounds of refit + re-assign from the endpoints (e0, e1); returns the best block and its error.
+template <bool EIGHT>
+__device__ __forceinline__ Bc4 bc4_refine(uint32_t const (&values8)[16], uint32_t e0, uint32_t e1, bool keep255, bool keep0, uint32_t& bestError)
 {
-    bestError = bc4_assign(values, block);
-    uint64_t best = block;
+    Bc4 block{ e0 & 0xffu, e1 & 0xffu, 0u, 0u };
+    uint32_t keys[16];
+    bestError = bc4_assign(values8, block, keys);
+    Bc4 best = block;
+#pragma unroll 1
     for (int round = 0; round < 8; ++round) {
-        block = bc4_refit(values, block, eightValues, keep255, keep0);
-        float const error = bc4_assign(values, block);
+        bc4_refit<EIGHT>(values8, keys, block, keep255, keep0);
+        uint32_t const error = bc4_assign(values8, block, keys);
         if (error >= bestError) break;
-        bool const repeated = (block >> 16) == (best >> 16);
+        bool const repeated = block.low == best.low && block.high == best.high;
         best = block;
         if (repeated) break;
         bestError = error;
@@ -131,26 +148,72 @@ __device__ __forceinline__ uint64_t bc4_refine(uint32_t const (&values)[16], uin
     return best;
 }
 
+// The candidate of one palette.
+template <bool EIGHT>
+__device__ __forceinline__ Bc4 bc4_candidate(uint32_t const (&values8)[16], uint32_t& error)
+{
+    uint32_t lo = 255u << 3, hi = 0;
+    if constexpr (EIGHT) {
+#pragma unroll
+        for (int t = 0; t < 16; ++t) { lo = min(lo, values8[t]); hi = max(hi, values8[t]); }
+        lo >>= 3; hi >>= 3;
+        bool const keep0 = lo == 0, keep255 = hi == 255u;
+        uint32_t const inset = (hi - lo) / 34u;
+        return bc4_refine<true>(values8, keep255 ? 255u : hi - inset, keep0 ? 0u : lo + inset, keep255, keep0, error);
+    } else {
+        // extremes among the values that are not 0 / not 255
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            if (values8[t] != 0) lo = min(lo, values8[t]);
+            if (values8[t] != (255u << 3)) hi = max(hi, values8[t]);
+        }
+        lo >>= 3; hi >>= 3;
+        // unsigned arithmetic on purpose: with no inner values (all texels 0 or 255) the difference wraps, as in the reference
+        uint32_t const inset = (hi - lo) / 34u;
+        return bc4_refine<false>(values8, lo + inset, hi - inset, false, false, error);
+    }
+}
+
+__device__ __forceinline__ uint32_t bc4_value8(float texel)
+{
+    float const s = fminf(fmaxf(texel, 0.f), 1.f);           // saturate: a NaN becomes 0
+    return uint32_t(rintf(s * 255.f)) << 3;
+}
+
 __device__ uint64_t bc4_encode(float const (&texels)[16])
 {
-    uint32_t values[16];
-    uint32_t lo = 255, hi = 0, loInner = 255, hiInner = 0;      // extremes; extremes among values that are not 0 / not 255
+    uint32_t values8[16], error8, error6;
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-        float const s = fminf(fmaxf(texels[t], 0.f), 1.f);     // saturate: a NaN becomes 0
-        values[t] = uint32_t(rintf(s * 255.f));
-        lo = min(lo, values[t]); hi = max(hi, values[t]);
-        if (values[t] != 0) loInner = min(loInner, values[t]);
-        if (values[t] != 255) hiInner = max(hiInner, values[t]);
+    for (int t = 0; t < 16; ++t) values8[t] = bc4_value8(texels[t]);
+    Bc4 const block8 = bc4_candidate<true>(values8, error8), block6 = bc4_candidate<false>(values8, error6);
+    return error6 < error8 ? block6.bits() : block8.bits();
+}
+
+// Channel `c` of the sixteen texels of block (bx, by), as 8-bit values times eight.
+__device__ __forceinline__ void bc4_load(BlockCompressArgs const& a, int bx, int by, int c, uint32_t (&values8)[16])
+{
+    int const x0 = a.srcLeft + bx * 4, y0 = a.srcTop + by * 4;
+    if (a.packedRows && x0 + 4 <= a.srcWidth && y0 + 4 <= a.srcHeight) {
+        // UNORM8 pixels without padding, the whole block inside the image: a row of four is four dwords at most, and
+        // a code is its own value (rint(code / 255 * 255) = code)
+        uint8_t const* px = a.src + size_t(y0) * a.rowPitch + size_t(x0) * a.pixelStride + size_t(c);
+#pragma unroll
+        for (int y = 0; y < 4; ++y, px += a.rowPitch) {
+            uint32_t words[4];
+            if (a.pixelStride == 1) {                        // uniform; c is 0
+                uint32_t const v = *reinterpret_cast<u32_unaligned const*>(px);
+                words[0] = v; words[1] = v >> 8; words[2] = v >> 16; words[3] = v >> 24;
+            } else {
+#pragma unroll
+                for (int x = 0; x < 4; ++x) words[x] = px[size_t(x) * a.pixelStride];
+            }
+#pragma unroll
+            for (int x = 0; x < 4; ++x) values8[4 * y + x] = (words[x] & 0xffu) << 3;
+        }
+    } else {
+#pragma unroll
+        for (int t = 0; t < 16; ++t) values8[t] = bc4_value8(source_channel(a, x0 + (t & 3), y0 + (t >> 2), c));
     }
-    bool const keep0 = lo == 0, keep255 = hi == 255;
-    float error8, error6;
-    uint64_t const block8 = bc4_refine(values, bc4_with_endpoints(0, keep255 ? 255u : hi - (hi - lo) / 34u, keep0 ? 0u : lo + (hi - lo) / 34u),
-                                       true, keep255, keep0, error8);
-    // unsigned arithmetic on purpose: with no inner values (all texels 0 or 255) the difference wraps, as in the reference
-    uint32_t const inset = (hiInner - loInner) / 34u;
-    uint64_t const block6 = bc4_refine(values, bc4_with_endpoints(0, loInner + inset, hiInner - inset), false, false, false, error6);
-    return error6 < error8 ? block6 : block8;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -455,24 +518,38 @@ __device__ __forceinline__ uint64_t bc2_alpha(float const (&alpha)[16])
 
 } // namespace
 
-// Thread groups of 16 x 8 blocks as in the reference (BLOCK_COMPRESS_CS_GROUP_WIDTH / HEIGHT).
+// A wave encodes one channel of 64 blocks (16 x 4) with one palette, so that the palettes' refinements, each a chain of
+// up to nine passes over the texels, run side by side and not one after the other: a workgroup is the two palettes of
+// both channels of 64 blocks (BC5) or of one channel of 128 (BC4).  The waves of the six-value palette leave their
+// candidates in LDS for those of the eight-value one to choose from.  2048 x 2048: BC5 66 us, BC4 36 (136 and 67 with one
+// lane per block and all of its channels and palettes, two to three instructions per palette entry and the weights from
+// memory);
+// 64 x 64: 10 and 9 us, 54 and 29 before.
 template <int CHANNELS>
-__global__ void __launch_bounds__(128)
+__global__ void __launch_bounds__(256)
 bc4_compress_kernel(BlockCompressArgs a)
 {
-    int const bx = blockIdx.x * 16 + (threadIdx.x & 15), by = blockIdx.y * 8 + (threadIdx.x >> 4);
-    if (bx >= a.widthInBlocks || by >= a.heightInBlocks) return;
-    uint64_t out[CHANNELS];
-#pragma unroll
-    for (int c = 0; c < CHANNELS; ++c) {
-        float texels[16];
-#pragma unroll
-        for (int t = 0; t < 16; ++t) texels[t] = source_channel(a, a.srcLeft + bx * 4 + (t & 3), a.srcTop + by * 4 + (t >> 2), c);
-        out[c] = bc4_encode(texels);
+    __shared__ uint32_t candidates[2][5][64];
+    int const wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63, pair = wave >> 1;
+    int const bx = blockIdx.x * 16 + (lane & 15), by = (CHANNELS == 1 ? blockIdx.y * 8 + pair * 4 : blockIdx.y * 4) + (lane >> 4);
+    bool const inside = bx < a.widthInBlocks && by < a.heightInBlocks;
+    int const channel = CHANNELS == 1 ? 0 : pair;
+    bool const eight = (wave & 1) == 0;
+    uint32_t values8[16], error = 0;
+    Bc4 mine{ 0u, 0u, 0u, 0u };
+    if (inside) {
+        bc4_load(a, bx, by, channel, values8);
+        mine = eight ? bc4_candidate<true>(values8, error) : bc4_candidate<false>(values8, error);
+        if (!eight) {
+            candidates[pair][0][lane] = mine.e0; candidates[pair][1][lane] = mine.e1;
+            candidates[pair][2][lane] = mine.low; candidates[pair][3][lane] = mine.high; candidates[pair][4][lane] = error;
+        }
     }
-    uint64_t* const dst = reinterpret_cast<uint64_t*>(a.dst + size_t(by + a.dstOffsetY) * a.dstRowPitch) + size_t(bx + a.dstOffsetX) * CHANNELS;
-#pragma unroll
-    for (int c = 0; c < CHANNELS; ++c) dst[c] = out[c];
+    __syncthreads();
+    if (!inside || !eight) return;
+    if (candidates[pair][4][lane] < error)
+        mine = Bc4{ candidates[pair][0][lane], candidates[pair][1][lane], candidates[pair][2][lane], candidates[pair][3][lane] };
+    reinterpret_cast<uint64_t*>(a.dst + size_t(by + a.dstOffsetY) * a.dstRowPitch)[size_t(bx + a.dstOffsetX) * CHANNELS + channel] = mine.bits();
 }
 
 // BC1 (8 bytes per block), BC2 and BC3 (alpha block, then colour block).  At least three waves per SIMD: the BC1
@@ -530,8 +607,8 @@ hipError_t launch_block_compress(BlockCompressArgs const& a, int dstFormat, hipS
     case 1: hipLaunchKernelGGL(bc1_compress_kernel<1>, grid, dim3(128), 0, stream, a); break;
     case 2: hipLaunchKernelGGL(bc1_compress_kernel<2>, grid, dim3(128), 0, stream, a); break;
     case 3: hipLaunchKernelGGL(bc1_compress_kernel<3>, grid, dim3(128), 0, stream, a); break;
-    case 4: hipLaunchKernelGGL(bc4_compress_kernel<1>, grid, dim3(128), 0, stream, a); break;
-    case 5: hipLaunchKernelGGL(bc4_compress_kernel<2>, grid, dim3(128), 0, stream, a); break;
+    case 4: hipLaunchKernelGGL(bc4_compress_kernel<1>, grid, dim3(256), 0, stream, a); break;
+    case 5: hipLaunchKernelGGL(bc4_compress_kernel<2>, dim3(grid.x, (a.heightInBlocks + 3) / 4), dim3(256), 0, stream, a); break;
     case 6: return launch_bc6_compress(a, stream);
     case 7: return launch_bc7_compress(a, stream);
     default: return hipErrorInvalidValue;

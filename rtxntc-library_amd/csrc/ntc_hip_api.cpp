@@ -1161,6 +1161,7 @@ int ntc_hip_ctx_block_compress(NtcHipContext* ctx, const NtcHipBlockCompress* p)
     }
     a.src = image.data; a.pixelStride = image.pixelStride; a.rowPitch = image.rowPitch; a.format = image.format; a.numChannels = image.numChannels;
     a.srcWidth = p->src.width; a.srcHeight = p->src.height;
+    a.packedRows = image.format == NTC_HIP_DEV_FORMAT_UNORM8 && image.pixelStride == uint64_t(image.numChannels);
     a.packedRgba8 = image.format == NTC_HIP_DEV_FORMAT_UNORM8 && image.numChannels == 4
         && ((reinterpret_cast<uintptr_t>(image.data) | image.pixelStride | image.rowPitch) & 3u) == 0;
     a.dst = static_cast<uint8_t*>(p->dst); a.dstRowPitch = p->dstRowPitch;

@@ -227,6 +227,31 @@ def test_gpu_block_compress_matches_checker(ntc, device, oracle, fmt, dst_format
     assert device.lib.ntc_hip_block_compress(p) == ntc.abi.ERR_INVALID_ARG
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("channels,dst_format", [(1, 4), (2, 5), (3, 5)])
+@pytest.mark.parametrize("w,h", [(4, 4), (68, 36), (130, 71)])
+def test_gpu_extreme_blocks_of_packed_rows_match_checker(ntc, device, oracle, channels, dst_format, w, h):
+    """UNORM8 pixels without padding; blocks of one, two and few values with 0 and 255 among them, so that either
+    palette's endpoints coincide, wrap or stay pinned; full blocks beside cut-off ones."""
+    rng = np.random.default_rng(w + channels)
+    image = np.zeros((h, w, channels), dtype=np.uint8)
+    for y in range(0, h, 4):
+        for x in range(0, w, 4):
+            pool = rng.choice([0, 255, 1, 254, int(rng.integers(0, 256)), int(rng.integers(0, 256))], size=int(rng.integers(1, 5)))
+            block = image[y:y + 4, x:x + 4]
+            block[...] = rng.choice(pool, size=block.shape)
+    bx, by, per = (w + 3) // 4, (h + 3) // 4, 8 if dst_format == 4 else 16
+    pitch = bx * per
+    want = oracle_bc(ntc, oracle, image, 1, channels, dst_format, bx, by, 0, 0, 0, 0, pitch)
+    d_src, d_dst = device.upload(image.reshape(-1)), device.upload(np.full(by * pitch, 0xEE, dtype=np.uint8))
+    p = ntc.abi.BlockCompress()
+    fill_image(p.src, d_src.ptr, d_src.nbytes, channels, channels * w, w, h, 1, channels)
+    p.widthInBlocks, p.heightInBlocks, p.dstFormat, p.dst, p.dstBytes, p.dstRowPitch = bx, by, dst_format, d_dst.ptr, d_dst.nbytes, pitch
+    device.call("block_compress", p)
+    device.synchronize()
+    assert np.array_equal(d_dst.download().view(np.uint64).reshape(by, pitch // 8), want)
+
+
 def test_unorm_quotient_shortcut_is_exact():
     """The kernels turn UNORM8 / UNORM16 texels into floats with q = k * r, q + fma(-q, d, k) * r (r = 1 / d
     rounded) instead of a division; that is the correctly rounded k / d for every k (exact rationals here)."""
