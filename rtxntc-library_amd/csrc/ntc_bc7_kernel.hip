@@ -385,55 +385,22 @@ template <class M, int C> BC7_INLINE void finish(Color<C> const (&px)[16], int p
     best.error = error; best.lo = b.lo; best.hi = b.hi;
 }
 
-// The partition with the smallest estimated error (the first of equals) over [first, last) and its
-// start endpoints: per subset the bounding box, oriented if asked.  A range of one partition is taken
-// as it is.
-template <int SUBSETS, int C> BC7_INLINE int pick_partition(Color<C> const (&px)[16], bool orientEnds, int searchIndexBits, int first, int last,
-                                                            Color<C> (&bestEnds)[2 * SUBSETS])
+// Start endpoints of every subset of a partition: the subset's bounding box, oriented if asked.
+template <int SUBSETS, int C, bool ORIENT> BC7_INLINE void partition_ends(Color<C> const (&px)[16], int partition, Color<C> (&ends)[2 * SUBSETS])
 {
-    int bestPartition = first;
-    float bestError = FLT_MAX;
-    bool const single = last - first == 1;
-    // a NaN texel makes every estimate NaN and no partition "best": the endpoints are then zero
+    uint32_t const word = partition_word<SUBSETS>(partition);
 #pragma unroll
-    for (int i = 0; i < 2 * SUBSETS; ++i)
-#pragma unroll
-        for (int k = 0; k < C; ++k) bestEnds[i].c[k] = 0.f;
-#pragma unroll 1
-    for (int p = first; p < last; ++p) {
-        uint32_t const word = partition_word<SUBSETS>(p);
-        Color<C> e[2 * SUBSETS];
-        float error = 0.f;
-#pragma unroll
-        for (int s = 0; s < SUBSETS; ++s) {
-            uint32_t const mask = spread_mask(word, s);
-            min_max(px, mask, e[2 * s], e[2 * s + 1]);
-            if (orientEnds) orient(px, mask, e[2 * s], e[2 * s + 1]);
-        }
-        if (!single) {
-#pragma unroll
-            for (int s = 0; s < SUBSETS; ++s) {
-                float const e2 = estimate(px, spread_mask(word, s), e[2 * s], e[2 * s + 1], searchIndexBits);
-                error = s == 0 ? e2 : error + e2;
-            }
-        }
-        if (single || error < bestError) {
-            bestPartition = p; bestError = error;
-#pragma unroll
-            for (int i = 0; i < 2 * SUBSETS; ++i) bestEnds[i] = e[i];
-        }
+    for (int s = 0; s < SUBSETS; ++s) {
+        uint32_t const mask = spread_mask(word, s);
+        min_max(px, mask, ends[2 * s], ends[2 * s + 1]);
+        if constexpr (ORIENT) orient(px, mask, ends[2 * s], ends[2 * s + 1]);
     }
-    return bestPartition;
 }
 
 // Modes 4 and 5: a colour plane of three channels and a scalar plane, each with its own endpoints and
 // indices; the scalar plane takes channel {A, R, G, B}[rotation] and alpha takes its place.
-BC7_INLINE void dual_plane(int mode, bool wideColorIndex, Color<4> const (&rgba)[16], uint32_t rotation, bool fixedMode, Best& best)
+BC7_INLINE void split_planes(Color<4> const (&rgba)[16], uint32_t rotation, Color<3> (&rgb)[16], Color<1> (&a)[16])
 {
-    int const colorIndexBits = mode == 5 ? 2 : (wideColorIndex ? 3 : 2), alphaIndexBits = mode == 5 ? 2 : (wideColorIndex ? 2 : 3);
-    int const colorBits = mode == 5 ? 7 : 5, alphaBits = mode == 5 ? 8 : 6;
-    Color<3> rgb[16];
-    Color<1> a[16];
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
         Color<4> const& p = rgba[t];
@@ -442,18 +409,20 @@ BC7_INLINE void dual_plane(int mode, bool wideColorIndex, Color<4> const (&rgba)
         rgb[t].c[2] = rotation == 3 ? p.c[3] : p.c[2];
         a[t].c[0] = rotation == 0 ? p.c[3] : rotation == 1 ? p.c[0] : rotation == 2 ? p.c[1] : p.c[2];
     }
-    Color<1> a0, a1;
-    min_max(a, kAllTexels, a0, a1);
-    refine(a, kAllTexels, a0, a1, alphaIndexBits);
-    Color<3> e0, e1;
-    min_max(rgb, kAllTexels, e0, e1);
-    orient(rgb, kAllTexels, e0, e1);
-    refine(rgb, kAllTexels, e0, e1, colorIndexBits);
+}
+template <int C> struct Ends { Color<C> e0, e1; };
+
+// One candidate of the two modes from the refined endpoints of both planes.
+BC7_INLINE void finish_dual_plane(int mode, bool wideColorIndex, Color<3> const (&rgb)[16], Color<1> const (&a)[16], Ends<3> const& color, Ends<1> const& alpha,
+                                  uint32_t rotation, bool fixedMode, Best& best)
+{
+    int const colorIndexBits = mode == 5 ? 2 : (wideColorIndex ? 3 : 2), alphaIndexBits = mode == 5 ? 2 : (wideColorIndex ? 2 : 3);
+    int const colorBits = mode == 5 ? 7 : 5, alphaBits = mode == 5 ? 8 : 6;
     Quantized<3> q0, q1;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) { q0.c[k] = quantize(e0.c[k], colorBits); q1.c[k] = quantize(e1.c[k], colorBits); }
+    for (int k = 0; k < 3; ++k) { q0.c[k] = quantize(color.e0.c[k], colorBits); q1.c[k] = quantize(color.e1.c[k], colorBits); }
     Quantized<1> qa0, qa1;
-    qa0.c[0] = quantize(a0.c[0], alphaBits); qa1.c[0] = quantize(a1.c[0], alphaBits);
+    qa0.c[0] = quantize(alpha.e0.c[0], alphaBits); qa1.c[0] = quantize(alpha.e1.c[0], alphaBits);
     int colorIndex[16], alphaIndex[16];
     float error = 0.f;
     if (assign(rgb, kAllTexels, 0, colorIndexBits, colorBits, q0, q1, colorIndex)) { Quantized<3> const t = q0; q0 = q1; q1 = t; }
@@ -478,56 +447,59 @@ BC7_INLINE void dual_plane(int mode, bool wideColorIndex, Color<4> const (&rgba)
     best.error = error; best.lo = b.lo; best.hi = b.hi;
 }
 
-// One block.  FIXED false: every mode is tried; true: only fixedMode with fixedPartition (for modes 4 / 5:
-// rotation in bits 0-1 of the partition, "wide colour index" in bit 2).  Both cases run through the same
-// code, the fixed one with every range narrowed to one candidate.  (Two instantiations because in the
-// full search every lane of a wave walks the same partitions, so the subset masks are uniform and the
-// texel loops branch on scalar bits instead of being predicated per lane.)
-template <bool FIXED>
-BC7_INLINE void bc7_encode(Color<4> const (&px)[16], int fixedMode, int fixedPartition, uint64_t& lo, uint64_t& hi)
+template <int C> BC7_INLINE Ends<C> box_of(Color<C> const (&px)[16])
 {
-    constexpr bool fixed = FIXED;
-    Best best{ FLT_MAX, 0, 0 };
-    bool opaque = true;
-#pragma unroll
-    for (int t = 0; t < 16; ++t) if (px[t].c[3] < 1.f) opaque = false;
-    int const firstPartition = fixed ? fixedPartition : 0, lastPartition = fixed ? fixedPartition + 1 : 64;
+    Ends<C> e;
+    min_max(px, kAllTexels, e.e0, e.e1);
+    if constexpr (C > 1) orient(px, kAllTexels, e.e0, e.e1);
+    return e;
+}
+template <int C> BC7_INLINE Ends<C> refined(Color<C> const (&px)[16], Ends<C> e, int indexBits)
+{
+    refine(px, kAllTexels, e.e0, e.e1, indexBits);
+    return e;
+}
 
-    if (fixed ? (fixedMode <= 3) : opaque) {
+// One candidate, with a given mode.
+BC7_INLINE void fixed_dual_plane(int mode, bool wideColorIndex, Color<4> const (&rgba)[16], uint32_t rotation, Best& best)
+{
+    Color<3> rgb[16];
+    Color<1> a[16];
+    split_planes(rgba, rotation, rgb, a);
+    int const colorIndexBits = mode == 5 ? 2 : (wideColorIndex ? 3 : 2), alphaIndexBits = mode == 5 ? 2 : (wideColorIndex ? 2 : 3);
+    finish_dual_plane(mode, wideColorIndex, rgb, a, refined(rgb, box_of(rgb), colorIndexBits), refined(a, box_of(a), alphaIndexBits), rotation, true, best);
+}
+
+// One block with a given mode and partition (for modes 4 / 5: rotation in bits 0-1 of the partition, "wide colour
+// index" in bit 2).
+BC7_INLINE void bc7_encode_fixed(Color<4> const (&px)[16], int mode, int partition, uint64_t& lo, uint64_t& hi)
+{
+    Best best{ FLT_MAX, 0, 0 };
+    if (mode <= 3) {
         Color<3> rgb[16];
 #pragma unroll
         for (int t = 0; t < 16; ++t) { rgb[t].c[0] = px[t].c[0]; rgb[t].c[1] = px[t].c[1]; rgb[t].c[2] = px[t].c[2]; }
-        if (!fixed || fixedMode == 0 || fixedMode == 2) {
+        if (mode == 0 || mode == 2) {
             Color<3> ends[6];
-            int const p = pick_partition<3>(rgb, true, 3, firstPartition, lastPartition, ends);
-            if (fixed ? fixedMode == 0 : p < 16) finish<Mode0>(rgb, p, ends, fixed, best);
-            if (!fixed || fixedMode == 2) finish<Mode2>(rgb, p, ends, fixed, best);
-        }
-        if (!fixed || fixedMode == 1 || fixedMode == 3) {
+            partition_ends<3, 3, true>(rgb, partition, ends);
+            if (mode == 0) finish<Mode0>(rgb, partition, ends, true, best);
+            else           finish<Mode2>(rgb, partition, ends, true, best);
+        } else {
             Color<3> ends[4];
-            int const p = pick_partition<2>(rgb, true, 3, firstPartition, lastPartition, ends);
-            if (!fixed || fixedMode == 1) finish<Mode1>(rgb, p, ends, fixed, best);
-            if (!fixed || fixedMode == 3) finish<Mode3>(rgb, p, ends, fixed, best);
+            partition_ends<2, 3, true>(rgb, partition, ends);
+            if (mode == 1) finish<Mode1>(rgb, partition, ends, true, best);
+            else           finish<Mode3>(rgb, partition, ends, true, best);
         }
-    }
-    if (!fixed || fixedMode == 4 || fixedMode == 5) {
-        uint32_t const firstRotation = fixed ? uint32_t(fixedPartition) & 3u : 0u, lastRotation = fixed ? firstRotation + 1u : 4u;
-#pragma unroll 1
-        for (uint32_t rotation = firstRotation; rotation < lastRotation; ++rotation) {
-            if (!fixed || (fixedMode == 4 && !(fixedPartition & 4))) dual_plane(4, false, px, rotation, fixed, best);
-            if (!fixed || (fixedMode == 4 && (fixedPartition & 4))) dual_plane(4, true, px, rotation, fixed, best);
-            if (!fixed || fixedMode == 5) dual_plane(5, false, px, rotation, fixed, best);
-        }
-    }
-    if (!fixed || fixedMode == 6) {
+    } else if (mode <= 5) {
+        fixed_dual_plane(mode, mode == 4 && (partition & 4), px, uint32_t(partition) & 3u, best);
+    } else if (mode == 6) {
         Color<4> ends[2];
-        pick_partition<1>(px, true, 4, 0, 1, ends);
-        finish<Mode6>(px, 0, ends, fixed, best);
-    }
-    if (!fixed || fixedMode == 7) {
+        partition_ends<1, 4, true>(px, 0, ends);
+        finish<Mode6>(px, 0, ends, true, best);
+    } else {
         Color<4> ends[4];
-        int const p = pick_partition<2>(px, false, 2, firstPartition, lastPartition, ends);
-        finish<Mode7>(px, p, ends, fixed, best);
+        partition_ends<2, 4, false>(px, partition, ends);
+        finish<Mode7>(px, partition, ends, true, best);
     }
     lo = best.lo; hi = best.hi;
 }
@@ -548,20 +520,595 @@ BC7_INLINE void store_block(BlockCompressArgs const& a, int bx, int by, uint64_t
 
 } // namespace
 
-// Full search.  8 x 8 blocks per 64-thread group, registers capped at 256 so that two waves share a SIMD:
-// the search is a long chain of scalar branches over uniform subset masks, and a second wave fills the
-// issue slots the first one leaves (1.7 times faster than one wave with 263 registers; three waves
-// with 168 registers spill and gain nothing more).
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+// ---- full search --------------------------------------------------------------------------------------
+//
+// A workgroup of WAVES waves encodes GROUPS x 64 blocks; the lanes of a wave are blocks, and the waves divide the search
+// among themselves.  The texels lie in LDS.
+//   1. Every task is some partitions of a search (three subsets and two subsets of opaque blocks, two subsets of blocks
+//      with alpha), whose smallest error per block is found by an atomic minimum in LDS.  All lanes take the same
+//      partition: for each subset its texels are read into registers and go through code for exactly that many.
+//   2. Every task is one candidate, or the three forms of modes 4 and 5 of one channel rotation, from its endpoints to
+//      the encoded block.  Every lane has a partition of its own here and walks its own list of texels.
+//   3. A thread per block goes through the candidates in the order given at the top with "not larger replaces".
+// Blocks with and without alpha are gathered in groups of their own for the tasks that only one kind has.
+//
+// The search is bound by vector instruction issue where it fills the GPU and by the length of one lane's chain where it
+// does not.  One lane per block with the texels in 255 registers and a scalar branch around every texel of every pass
+// took 0.9 ms for any image of up to 1024 x 1024 and 2.0 ms for 2048 x 2048; this takes 0.10 ms for 64 x 64, 0.11 for
+// 512 x 512, 0.29 for 1024 x 1024 and 0.95 for 2048 x 2048 (half of it opaque), where every issue slot of the vector units
+// is taken.
+enum { kSlots = 10, kPickThree = 0, kPickTwo, kPickTwoAlpha, kPicks };
+
+template <int BLOCKS_>
+struct SearchLds {
+    static constexpr int BLOCKS = BLOCKS_;
+    float4 texels[16][BLOCKS];
+    uint64_t picks[kPicks][BLOCKS];                          // error bits << 32 | partition
+    uint4 words[kSlots][BLOCKS];
+    float errors[kSlots][BLOCKS];
+    uint32_t withAlpha[BLOCKS];
+    uint8_t blocks[2][BLOCKS];                               // numbers of the opaque blocks, of those with alpha
+    int counts[2];
+};
+template <class S> using SearchPtr = __attribute__((address_space(3))) S*;
+
+// The tasks are functions of their own (arguments reach them per lane: what is uniform is made so again): in one body
+// the compiler keeps the texels of several of them in registers and spills three thousand.
+#define BC7_TASK __device__ __attribute__((noinline))
+
+template <int C, class S> BC7_INLINE Color<C> texel(SearchPtr<S> lds, int b, int t)
+{
+    Color<C> p;
+    p.c[0] = lds->texels[t][b].x; p.c[1] = lds->texels[t][b].y; p.c[2] = lds->texels[t][b].z;
+    if constexpr (C == 4) p.c[3] = lds->texels[t][b].w;
+    return p;
+}
+BC7_INLINE int first_texel(uint32_t mask) { return (__ffs(int(mask)) - 1) >> 1; }
+
+// Endpoints' swaps of orient() from the finished covariances.
+template <int C> BC7_INLINE void orient_by(float const (&cov)[C][C], Color<C>& e0, Color<C>& e1)
+{
+    bool done = false;
+#pragma unroll
+    for (int a = 0; a + 1 < C; ++a) {
+        if (!done && e0.c[a] != e1.c[a]) {
+#pragma unroll
+            for (int b = a + 1; b < C; ++b)
+                if (cov[a][b] < 0.f) { float const t = e0.c[b]; e0.c[b] = e1.c[b]; e1.c[b] = t; }
+            done = true;
+        }
+    }
+}
+template <int C> BC7_INLINE void add_covariance(float (&cov)[C][C], Color<C> const& d)
+{
+#pragma unroll
+    for (int a = 0; a < C; ++a)
+#pragma unroll
+        for (int b = a + 1; b < C; ++b) cov[a][b] += d.c[a] * d.c[b];
+}
+template <int C> BC7_INLINE float inverse_square(Color<C> const& axis) { float const l = dot(axis, axis); return l > 0.f ? 1.f / l : l; }
+
+// Squared error of N texels if each took the nearest of the 2^BITS points between e0 and e1.
+template <int BITS, int C, int N> BC7_INLINE float estimate_of(Color<C> const (&px)[N], Color<C> const& e0, Color<C> const& e1)
+{
+    Color<C> const axis = sub(e1, e0);
+    float const mul = inverse_square(axis);
+    constexpr float maxIndex = float((1u << BITS) - 1u), indexScale = 1.f / maxIndex;
+    float error = 0.f;
+#pragma unroll
+    for (int t = 0; t < N; ++t) {
+        Color<C> const p = sub(px[t], e0);
+        float const f = rintf(dot(p, axis) * mul * maxIndex) * indexScale;
+        Color<C> diff;
+#pragma unroll
+        for (int k = 0; k < C; ++k) diff.c[k] = f * axis.c[k] - p.c[k];
+        error += dot(diff, diff);
+    }
+    return error;
+}
+
+// Estimated errors of the subset `mask` (uniform, of N texels): with oriented ends and eight points (three-channel modes 0
+// to 3) if ORIENTED, with the box's own corners and four points (mode 7) if PLAIN.
+struct SubsetErrors { float oriented, plain; };
+template <int C, int N, bool ORIENTED, bool PLAIN, class S> BC7_INLINE SubsetErrors subset_errors(SearchPtr<S> lds, int b, uint32_t mask)
+{
+    Color<C> px[N];
+#pragma unroll
+    for (int t = 0; t < N; ++t) { px[t] = texel<C, S>(lds, b, first_texel(mask)); mask &= mask - 1; }
+    Color<C> lo, hi;
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+        lo.c[k] = FLT_MAX; hi.c[k] = -FLT_MAX;
+#pragma unroll
+        for (int t = 0; t + 1 < N; t += 2) { lo.c[k] = min3_f32(lo.c[k], px[t].c[k], px[t + 1].c[k]); hi.c[k] = max3_f32(hi.c[k], px[t].c[k], px[t + 1].c[k]); }
+        if constexpr (N & 1) { lo.c[k] = min_f32(lo.c[k], px[N - 1].c[k]); hi.c[k] = max_f32(hi.c[k], px[N - 1].c[k]); }
+    }
+    SubsetErrors e{ 0.f, 0.f };
+    if constexpr (PLAIN) e.plain = estimate_of<2>(px, lo, hi);
+    if constexpr (ORIENTED) {
+        Color<C> center;
+#pragma unroll
+        for (int k = 0; k < C; ++k) {
+            center.c[k] = 0.f;
+#pragma unroll
+            for (int t = 0; t < N; ++t) center.c[k] += px[t].c[k];
+            center.c[k] /= float(N);
+        }
+        float cov[C][C] = {};
+#pragma unroll
+        for (int t = 0; t < N; ++t) add_covariance(cov, sub(px[t], center));
+        orient_by(cov, lo, hi);
+        e.oriented = estimate_of<3>(px, lo, hi);
+    }
+    return e;
+}
+
+// Of the partitions [first, last) of `pick` the one with the smallest estimated error (the first of equals), as error bits
+// << 32 | partition: errors are not negative, so the smallest such number over several ranges is the same over all of them.
+template <class S, int SUBSETS, int C, bool ORIENTED, bool PLAIN>
+BC7_TASK void pick_task(SearchPtr<S> lds, int b, int first, int last)
+{
+    first = __builtin_amdgcn_readfirstlane(first);
+    last = __builtin_amdgcn_readfirstlane(last);
+    uint64_t bestOriented = ~uint64_t(0), bestPlain = ~uint64_t(0);
+#pragma unroll 1
+    for (int p = first; p < last; ++p) {
+        uint32_t const word = partition_word<SUBSETS>(p);
+        SubsetErrors error{ 0.f, 0.f };
+#pragma unroll 1
+        for (int s = 0; s < SUBSETS; ++s) {
+            uint32_t const mask = spread_mask(word, uint32_t(s));
+            SubsetErrors e{ 0.f, 0.f };
+            switch (__popc(mask)) {                          // the sizes that the partitions' subsets have
+            case 2:  if constexpr (SUBSETS == 3) e = subset_errors<C, 2, ORIENTED, PLAIN, S>(lds, b, mask); break;
+            case 3:  e = subset_errors<C, 3, ORIENTED, PLAIN, S>(lds, b, mask); break;
+            case 4:  e = subset_errors<C, 4, ORIENTED, PLAIN, S>(lds, b, mask); break;
+            case 5:  e = subset_errors<C, 5, ORIENTED, PLAIN, S>(lds, b, mask); break;
+            case 6:  e = subset_errors<C, 6, ORIENTED, PLAIN, S>(lds, b, mask); break;
+            case 7:  if constexpr (SUBSETS == 3) e = subset_errors<C, 7, ORIENTED, PLAIN, S>(lds, b, mask); break;
+            case 8:  e = subset_errors<C, 8, ORIENTED, PLAIN, S>(lds, b, mask); break;
+            case 10: if constexpr (SUBSETS == 2) e = subset_errors<C, 10, ORIENTED, PLAIN, S>(lds, b, mask); break;
+            case 11: if constexpr (SUBSETS == 2) e = subset_errors<C, 11, ORIENTED, PLAIN, S>(lds, b, mask); break;
+            case 12: e = subset_errors<C, 12, ORIENTED, PLAIN, S>(lds, b, mask); break;
+            case 13: if constexpr (SUBSETS == 2) e = subset_errors<C, 13, ORIENTED, PLAIN, S>(lds, b, mask); break;
+            default: break;
+            }
+            error.oriented = s == 0 ? e.oriented : error.oriented + e.oriented;
+            error.plain = s == 0 ? e.plain : error.plain + e.plain;
+        }
+        auto const consider = [&](uint64_t& best, float e) {
+            uint64_t const key = uint64_t(__float_as_uint(e)) << 32 | uint32_t(p);
+            best = key < best ? key : best;
+        };
+        if constexpr (ORIENTED) consider(bestOriented, error.oriented);
+        if constexpr (PLAIN) consider(bestPlain, error.plain);
+    }
+    if constexpr (ORIENTED) __hip_atomic_fetch_min(&lds->picks[SUBSETS == 3 ? kPickThree : kPickTwo][b], bestOriented, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if constexpr (PLAIN) __hip_atomic_fetch_min(&lds->picks[kPickTwoAlpha][b], bestPlain, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Sums of one refinement round (refine() above) and its solution; false when the system is singular.
+template <int C> struct Refinement {
+    float a2 = 0.f, b2 = 0.f, ab = 0.f;
+    Color<C> ax, bx;
+    BC7_INLINE Refinement()
+    {
+#pragma unroll
+        for (int k = 0; k < C; ++k) ax.c[k] = bx.c[k] = 0.f;
+    }
+    // f: the texel's saturated place between the ends
+    BC7_INLINE void add(float f, Color<C> const& p, int indexBits)
+    {
+        float const scale = float((1u << indexBits) - 1u), iscale = 1.f / scale;
+        float const beta = rintf(f * scale) * iscale, alpha = 1.f - beta;
+        a2 += alpha * alpha; b2 += beta * beta; ab += alpha * beta;
+#pragma unroll
+        for (int k = 0; k < C; ++k) { ax.c[k] += alpha * p.c[k]; bx.c[k] += beta * p.c[k]; }
+    }
+    BC7_INLINE bool solve(Color<C>& e0, Color<C>& e1) const
+    {
+        float const denom = a2 * b2 - ab * ab;
+        if (!(fabsf(denom) > 0.0001f)) return false;
+        float const factor = 1.f / denom;
+#pragma unroll
+        for (int k = 0; k < C; ++k) {
+            float const a = saturate((ax.c[k] * b2 - bx.c[k] * ab) * factor), b = saturate((bx.c[k] * a2 - ax.c[k] * ab) * factor);
+            if (!(e0.c[k] == 0.f || e0.c[k] == 1.f)) e0.c[k] = a;
+            if (!(e1.c[k] == 0.f || e1.c[k] == 1.f)) e1.c[k] = b;
+        }
+        return true;
+    }
+};
+
+// Start ends of the lane's own subset: its box, oriented if asked.
+template <int C, bool ORIENT, class S> BC7_INLINE void listed_ends(SearchPtr<S> lds, int b, uint32_t mask, Color<C>& e0, Color<C>& e1)
+{
+    Color<C> center;
+#pragma unroll
+    for (int k = 0; k < C; ++k) { e0.c[k] = FLT_MAX; e1.c[k] = -FLT_MAX; center.c[k] = 0.f; }
+    for (uint32_t m = mask; m; m &= m - 1) {
+        Color<C> const p = texel<C, S>(lds, b, first_texel(m));
+#pragma unroll
+        for (int k = 0; k < C; ++k) { e0.c[k] = min_f32(e0.c[k], p.c[k]); e1.c[k] = max_f32(e1.c[k], p.c[k]); center.c[k] += p.c[k]; }
+    }
+    if constexpr (ORIENT) {
+        float const count = float(__popc(mask));
+#pragma unroll
+        for (int k = 0; k < C; ++k) center.c[k] /= count;
+        float cov[C][C] = {};
+        for (uint32_t m = mask; m; m &= m - 1) add_covariance(cov, sub(texel<C, S>(lds, b, first_texel(m)), center));
+        orient_by(cov, e0, e1);
+    }
+}
+template <int C, int INDEX_BITS, class S> BC7_INLINE void listed_refine(SearchPtr<S> lds, int b, uint32_t mask, Color<C>& e0, Color<C>& e1)
+{
+#pragma unroll 1
+    for (int iter = 0; iter < 2; ++iter) {
+        Color<C> const axis = sub(e1, e0);
+        float const mul = inverse_square(axis);
+        Refinement<C> sums;
+        for (uint32_t m = mask; m; m &= m - 1) {
+            Color<C> const p = texel<C, S>(lds, b, first_texel(m));
+            sums.add(saturate(dot(sub(p, e0), axis) * mul), p, INDEX_BITS);
+        }
+        if (!sums.solve(e0, e1)) break;
+    }
+}
+
+// Dequantised endpoints: where texels fall between them and what a decoder shows there.
+template <int C, int INDEX_BITS> struct Decoded {
+    Color<C> e0, axis;
+    float mul;
+    int base[C], step[C];
+    BC7_INLINE Decoded(Quantized<C> const& q0, Quantized<C> const& q1, int endpointBits)
+    {
+        Color<C> e1;
+#pragma unroll
+        for (int k = 0; k < C; ++k) {
+            int const x0 = expand8(q0.c[k], endpointBits), x1 = expand8(q1.c[k], endpointBits);
+            base[k] = 64 * x0 + 32; step[k] = x1 - x0;
+            e0.c[k] = unorm_quotient(float(x0), 255.f, 1.f / 255.f); e1.c[k] = unorm_quotient(float(x1), 255.f, 1.f / 255.f);
+        }
+        axis = sub(e1, e0);
+        mul = inverse_square(axis);
+    }
+    // The texel's index, and its error added.  Weights of complemented indices on swapped endpoints are complements
+    // themselves, so the error is that of the final form whichever way the anchor turns out.
+    BC7_INLINE uint32_t index(Color<C> const& p, float& error) const
+    {
+        constexpr float top = float((1u << INDEX_BITS) - 1u);
+        float const place = rintf(saturate(dot(sub(p, e0), axis) * mul) * top);
+        int const w = int(rintf(place * (64.f / top)));
+        Color<C> diff;
+#pragma unroll
+        for (int k = 0; k < C; ++k) diff.c[k] = unorm_quotient(float((base[k] + __mul24(step[k], w)) >> 6), 255.f, 1.f / 255.f) - p.c[k];
+        error += dot(diff, diff);
+        return uint32_t(place);
+    }
+};
+
+// A field of a block from bit `at` on, and the removal of the anchors' top index bits, which are zero.
+BC7_INLINE void put_indices(uint64_t& lo, uint64_t& hi, int at, uint64_t v)
+{
+    if (at < 64) { lo |= v << at; hi |= at ? v >> (64 - at) : 0; }
+    else hi |= v << (at - 64);
+}
+BC7_INLINE uint64_t without_bit(uint64_t v, int at)
+{
+    uint64_t const below = (uint64_t(1) << at) - 1u;
+    return (v & below) | ((v >> 1) & ~below);
+}
+
+template <class S, class M, int C, bool ORIENT>
+BC7_TASK void finish_task(SearchPtr<S> lds, int b, int pick, int slot)
+{
+    pick = __builtin_amdgcn_readfirstlane(pick);
+    slot = __builtin_amdgcn_readfirstlane(slot);
+    constexpr int N = 2 * M::subsets;
+    int partition = 0;
+    bool none = false;
+    if constexpr (M::subsets > 1) {
+        // A NaN or infinite texel can leave every partition without a finite estimate: then none is "best", and
+        // partition 0 is tried with endpoints of zero.
+        uint64_t const key = lds->picks[pick][b];
+        none = uint32_t(key >> 32) >= __float_as_uint(FLT_MAX);
+        partition = none ? 0 : int(uint32_t(key));
+    }
+    if (partition >= (1 << M::partitionBits)) {              // mode 0 has sixteen partitions only
+        lds->errors[slot][b] = __uint_as_float(0x7f800000u); // never taken
+        return;
+    }
+    uint32_t const word = partition_word<M::subsets>(partition);
+    Color<C> e[N];
+    Quantized<C> q[N];
+#pragma unroll
+    for (int s = 0; s < M::subsets; ++s) {
+        uint32_t const mask = spread_mask(word, uint32_t(s));
+        listed_ends<C, ORIENT, S>(lds, b, mask, e[2 * s], e[2 * s + 1]);
+        if (none) {
+#pragma unroll
+            for (int k = 0; k < C; ++k) e[2 * s].c[k] = e[2 * s + 1].c[k] = 0.f;
+        }
+        listed_refine<C, M::indexBits, S>(lds, b, mask, e[2 * s], e[2 * s + 1]);
+    }
+    quantize_endpoints<M, C>(e, q);
+    uint64_t indices = 0;
+    float error = 0.f;
+    int anchors[M::subsets];
+#pragma unroll
+    for (int s = 0; s < M::subsets; ++s) {
+        Decoded<C, M::indexBits> const ends(q[2 * s], q[2 * s + 1], M::endpointBits);
+        float e2 = 0.f;
+        uint64_t ones = 0;
+        for (uint32_t m = spread_mask(word, uint32_t(s)); m; m &= m - 1) {
+            int const t = first_texel(m);
+            uint64_t const one = uint64_t(1) << (t * M::indexBits);
+            indices |= uint64_t(ends.index(texel<C, S>(lds, b, t), e2)) << (t * M::indexBits);
+            ones |= one;
+        }
+        error = s == 0 ? e2 : error + e2;
+        // a decoder assumes the anchor's top index bit to be 0: if it is 1 the endpoints trade places
+        anchors[s] = subset_anchor<M::subsets>(partition, s);
+        if ((indices >> (anchors[s] * M::indexBits + M::indexBits - 1)) & 1u) {
+            indices ^= ones * ((1u << M::indexBits) - 1u);
+            Quantized<C> const x = q[2 * s]; q[2 * s] = q[2 * s + 1]; q[2 * s + 1] = x;
+        }
+    }
+    Bits bits;
+    bits.put(M::id + 1, 1u << M::id);
+    bits.put(M::partitionBits, uint32_t(partition));
+    constexpr int drop = M::pbit == kNoPBit ? 0 : 1;
+#pragma unroll
+    for (int k = 0; k < C; ++k)
+#pragma unroll
+        for (int i = 0; i < N; ++i) bits.put(M::endpointBits - drop, uint32_t(q[i].c[k]) >> drop);
+    if constexpr (M::pbit == kPBitPerEndpoint) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) bits.put(1, uint32_t(q[i].c[0]));
+    }
+    if constexpr (M::pbit == kPBitPerSubset) {
+#pragma unroll
+        for (int s = 0; s < M::subsets; ++s) bits.put(1, uint32_t(q[2 * s].c[0]));
+    }
+    constexpr int top = M::indexBits - 1;
+    if constexpr (M::subsets == 3) {
+        indices = without_bit(indices, max(anchors[1], anchors[2]) * M::indexBits + top);
+        indices = without_bit(indices, min(anchors[1], anchors[2]) * M::indexBits + top);
+    } else if constexpr (M::subsets == 2) {
+        indices = without_bit(indices, anchors[1] * M::indexBits + top);
+    }
+    indices = without_bit(indices, top);
+    put_indices(bits.lo, bits.hi, bits.at, indices);
+    lds->errors[slot][b] = error;
+    lds->words[slot][b].x = uint32_t(bits.lo); lds->words[slot][b].y = uint32_t(bits.lo >> 32);
+    lds->words[slot][b].z = uint32_t(bits.hi); lds->words[slot][b].w = uint32_t(bits.hi >> 32);
+}
+
+// The colour plane and the scalar plane of a texel under a channel rotation (uniform).
+template <class S> BC7_INLINE void planes_of(SearchPtr<S> lds, int b, int t, int rotation, Color<3>& rgb, Color<1>& a)
+{
+    Color<4> const p = texel<4, S>(lds, b, t);
+    rgb.c[0] = rotation == 1 ? p.c[3] : p.c[0];
+    rgb.c[1] = rotation == 2 ? p.c[3] : p.c[1];
+    rgb.c[2] = rotation == 3 ? p.c[3] : p.c[2];
+    a.c[0] = rotation == 0 ? p.c[3] : rotation == 1 ? p.c[0] : rotation == 2 ? p.c[1] : p.c[2];
+}
+
+template <int FORM> struct DualForm {                        // mode 4 with 2-bit colour indices, with 3-bit ones, mode 5
+    static constexpr int mode = FORM == 2 ? 5 : 4, colorIndexBits = FORM == 1 ? 3 : 2, alphaIndexBits = FORM == 0 ? 3 : 2;
+    static constexpr int colorBits = FORM == 2 ? 7 : 5, alphaBits = FORM == 2 ? 8 : 6;
+};
+
+template <class S, int FORM>
+BC7_TASK void dual_plane_form(SearchPtr<S> lds, int b, int rotation, Ends<3> color, Ends<1> alpha, Best& best)
+{
+    using F = DualForm<FORM>;
+    rotation = __builtin_amdgcn_readfirstlane(rotation);
+    Quantized<3> q0, q1;
+    Quantized<1> qa0, qa1;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) { q0.c[k] = quantize(color.e0.c[k], F::colorBits); q1.c[k] = quantize(color.e1.c[k], F::colorBits); }
+    qa0.c[0] = quantize(alpha.e0.c[0], F::alphaBits); qa1.c[0] = quantize(alpha.e1.c[0], F::alphaBits);
+    Decoded<3, F::colorIndexBits> const colorEnds(q0, q1, F::colorBits);
+    Decoded<1, F::alphaIndexBits> const alphaEnds(qa0, qa1, F::alphaBits);
+    uint64_t colorIndices = 0, alphaIndices = 0;
+    float colorError = 0.f, alphaError = 0.f;
+#pragma unroll 4
+    for (int t = 0; t < 16; ++t) {
+        Color<3> rgb;
+        Color<1> a;
+        planes_of<S>(lds, b, t, rotation, rgb, a);
+        colorIndices |= uint64_t(colorEnds.index(rgb, colorError)) << (t * F::colorIndexBits);
+        alphaIndices |= uint64_t(alphaEnds.index(a, alphaError)) << (t * F::alphaIndexBits);
+    }
+    float const error = colorError + alphaError;
+    if (error > best.error) return;
+    auto const complemented = [](uint64_t v, int bits) { return bits == 2 ? v ^ 0xffffffffull : v ^ 0xffffffffffffull; };
+    if (colorIndices & (1u << (F::colorIndexBits - 1))) { colorIndices = complemented(colorIndices, F::colorIndexBits); Quantized<3> const x = q0; q0 = q1; q1 = x; }
+    if (alphaIndices & (1u << (F::alphaIndexBits - 1))) { alphaIndices = complemented(alphaIndices, F::alphaIndexBits); Quantized<1> const x = qa0; qa0 = qa1; qa1 = x; }
+    Bits bits;
+    bits.put(F::mode + 1, 1u << F::mode);
+    bits.put(2, uint32_t(rotation));
+    if constexpr (F::mode == 4) bits.put(1, FORM == 1 ? 1u : 0u);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) { bits.put(F::colorBits, uint32_t(q0.c[k])); bits.put(F::colorBits, uint32_t(q1.c[k])); }
+    bits.put(F::alphaBits, uint32_t(qa0.c[0])); bits.put(F::alphaBits, uint32_t(qa1.c[0]));
+    colorIndices = without_bit(colorIndices, F::colorIndexBits - 1);
+    alphaIndices = without_bit(alphaIndices, F::alphaIndexBits - 1);
+    // mode 4 stores its 2-bit indices first, then the 3-bit ones; mode 5 colour first, then the scalar
+    constexpr int firstBits = 16 * (FORM == 1 ? F::alphaIndexBits : F::colorIndexBits) - 1;
+    put_indices(bits.lo, bits.hi, bits.at, FORM == 1 ? alphaIndices : colorIndices);
+    put_indices(bits.lo, bits.hi, bits.at + firstBits, FORM == 1 ? colorIndices : alphaIndices);
+    best.error = error; best.lo = bits.lo; best.hi = bits.hi;
+}
+
+// The refined ends of one rotation's planes, for 2-bit and for 3-bit indices: mode 5 shares its colour ends with mode
+// 4's narrow form and its scalar ends with the wide form.
+template <class S>
+BC7_TASK void dual_plane_ends(SearchPtr<S> lds, int b, int rotation, Ends<3> (&color)[2], Ends<1> (&alpha)[2])
+{
+    rotation = __builtin_amdgcn_readfirstlane(rotation);
+    Ends<3> c;
+    Ends<1> s;
+    {
+        Color<3> center;
+        for (int k = 0; k < 3; ++k) { c.e0.c[k] = FLT_MAX; c.e1.c[k] = -FLT_MAX; center.c[k] = 0.f; }
+        s.e0.c[0] = FLT_MAX; s.e1.c[0] = -FLT_MAX;
+#pragma unroll 4
+        for (int t = 0; t < 16; ++t) {
+            Color<3> rgb;
+            Color<1> a;
+            planes_of<S>(lds, b, t, rotation, rgb, a);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) { c.e0.c[k] = min_f32(c.e0.c[k], rgb.c[k]); c.e1.c[k] = max_f32(c.e1.c[k], rgb.c[k]); center.c[k] += rgb.c[k]; }
+            s.e0.c[0] = min_f32(s.e0.c[0], a.c[0]); s.e1.c[0] = max_f32(s.e1.c[0], a.c[0]);
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) center.c[k] /= 16.f;
+        float cov[3][3] = {};
+#pragma unroll 4
+        for (int t = 0; t < 16; ++t) {
+            Color<3> rgb;
+            Color<1> a;
+            planes_of<S>(lds, b, t, rotation, rgb, a);
+            add_covariance(cov, sub(rgb, center));
+        }
+        orient_by(cov, c.e0, c.e1);
+    }
+    color[0] = color[1] = c;
+    alpha[0] = alpha[1] = s;
+    bool colorGoesOn[2] = { true, true }, alphaGoesOn[2] = { true, true };
+#pragma unroll 1
+    for (int iter = 0; iter < 2; ++iter) {
+        Refinement<3> colorSums[2];
+        Refinement<1> alphaSums[2];
+        Color<3> axis[2];
+        Color<1> range[2];
+        float mul[2], scale[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            axis[i] = sub(color[i].e1, color[i].e0); mul[i] = inverse_square(axis[i]);
+            range[i] = sub(alpha[i].e1, alpha[i].e0); scale[i] = inverse_square(range[i]);
+        }
+#pragma unroll 2
+        for (int t = 0; t < 16; ++t) {
+            Color<3> rgb;
+            Color<1> a;
+            planes_of<S>(lds, b, t, rotation, rgb, a);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                colorSums[i].add(saturate(dot(sub(rgb, color[i].e0), axis[i]) * mul[i]), rgb, 2 + i);
+                alphaSums[i].add(saturate(dot(sub(a, alpha[i].e0), range[i]) * scale[i]), a, 2 + i);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            if (colorGoesOn[i]) colorGoesOn[i] = colorSums[i].solve(color[i].e0, color[i].e1);
+            if (alphaGoesOn[i]) alphaGoesOn[i] = alphaSums[i].solve(alpha[i].e0, alpha[i].e1);
+        }
+    }
+}
+
+template <int GROUPS, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES, 4)
 bc7_compress_kernel(BlockCompressArgs a)
 {
-    int const bx = blockIdx.x * 8 + (threadIdx.x & 7), by = blockIdx.y * 8 + (threadIdx.x >> 3);
-    if (bx >= a.widthInBlocks || by >= a.heightInBlocks) return;
-    Color<4> px[16];
-    load_block(a, bx, by, px);
-    uint64_t lo, hi;
-    bc7_encode<false>(px, -1, 0, lo, hi);
-    store_block(a, bx, by, lo, hi);
+    constexpr int BLOCKS = 64 * GROUPS, THREADS = 64 * WAVES, CHUNK = 64 * GROUPS / WAVES >= 8 ? 8 : 4, CHUNKS = 64 / CHUNK;
+    static_assert(THREADS >= 4 * BLOCKS, "a thread per row of a block at least");
+    using S = SearchLds<BLOCKS>;
+    __shared__ S shared;
+    SearchPtr<S> const lds = (SearchPtr<S>)&shared;
+    int const tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // blocks: 8 x 8 per group, the groups side by side
+    auto const block_x = [&](int b) { return int(blockIdx.x) * 8 * GROUPS + (b >> 6) * 8 + (b & 7); };
+    auto const block_y = [&](int b) { return int(blockIdx.y) * 8 + ((b >> 3) & 7); };
+
+    for (int i = tid; i < BLOCKS; i += THREADS) {
+        shared.withAlpha[i] = 0u;
+        for (int k = 0; k < kPicks; ++k) shared.picks[k][i] = ~uint64_t(0);
+    }
+    __syncthreads();
+    if (int const b = tid % BLOCKS, row = tid / BLOCKS; row < 4) {
+        int const bx = block_x(b), by = block_y(b);
+        bool const inside = bx < a.widthInBlocks && by < a.heightInBlocks;
+        bool alpha = false;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float c[4] = { 0.f, 0.f, 0.f, 0.f };
+            if (inside) source_pixel(a, a.srcLeft + bx * 4 + i, a.srcTop + by * 4 + row, c);
+            alpha = alpha || c[3] < 1.f;
+            shared.texels[4 * row + i][b] = make_float4(c[0], c[1], c[2], c[3]);
+        }
+        if (alpha && inside) shared.withAlpha[b] = 1u;
+    }
+    __syncthreads();
+    if (wave < 2) {                                          // wave 0 lists the opaque blocks, wave 1 those with alpha
+        int count = 0;
+        for (int g = 0; g < GROUPS; ++g) {
+            int const b = 64 * g + lane;
+            bool const mine = block_x(b) < a.widthInBlocks && block_y(b) < a.heightInBlocks && int(shared.withAlpha[b]) == wave;
+            uint64_t const ballot = __ballot(mine);
+            if (mine) shared.blocks[wave][count + int(__builtin_amdgcn_mbcnt_hi(uint32_t(ballot >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(ballot), 0u)))] = uint8_t(b);
+            count += __popcll(ballot);
+        }
+        if (lane == 0) shared.counts[wave] = count;
+    }
+    __syncthreads();
+    int const opaque = __builtin_amdgcn_readfirstlane(shared.counts[0]), withAlpha = __builtin_amdgcn_readfirstlane(shared.counts[1]);
+    int const opaqueGroups = (opaque + 63) / 64, alphaGroups = (withAlpha + 63) / 64, groups = opaqueGroups + alphaGroups;
+    // the lane's block of a group of one kind (lanes beyond the last block repeat it)
+    auto const block_of = [&](int kind, int group) { return int(shared.blocks[kind][min(64 * group + lane, (kind ? withAlpha : opaque) - 1)]); };
+
+    // ---- 1. partitions
+    for (int task = wave; task < (2 * opaqueGroups + alphaGroups) * CHUNKS; task += WAVES) {
+        int const first = (task % CHUNKS) * CHUNK, what = task / CHUNKS;
+        if (what >= 2 * opaqueGroups) pick_task<S, 2, 4, false, true>(lds, block_of(1, what - 2 * opaqueGroups), first, first + CHUNK);
+        else if (what & 1)            pick_task<S, 2, 3, true, true>(lds, block_of(0, what >> 1), first, first + CHUNK);     // mode 7's too: alpha is 1, its terms are zeros
+        else                          pick_task<S, 3, 3, true, false>(lds, block_of(0, what >> 1), first, first + CHUNK);
+    }
+    __syncthreads();
+
+    // ---- 2. candidates
+    for (int task = wave; task < 4 * opaqueGroups + 6 * groups; task += WAVES) {
+        if (task < 4 * opaqueGroups) {
+            int const which = task & 3, b = block_of(0, task >> 2);
+            if (which == 0)      finish_task<S, Mode0, 3, true>(lds, b, kPickThree, 0);
+            else if (which == 1) finish_task<S, Mode2, 3, true>(lds, b, kPickThree, 1);
+            else if (which == 2) finish_task<S, Mode1, 3, true>(lds, b, kPickTwo, 2);
+            else                 finish_task<S, Mode3, 3, true>(lds, b, kPickTwo, 3);
+        } else {
+            int const which = (task - 4 * opaqueGroups) % 6, group = (task - 4 * opaqueGroups) / 6;
+            int const b = group < opaqueGroups ? block_of(0, group) : block_of(1, group - opaqueGroups);
+            if (which < 4) {
+                Ends<3> color[2];                            // refined for 2-bit and 3-bit indices
+                Ends<1> alpha[2];
+                dual_plane_ends<S>(lds, b, which, color, alpha);
+                Best best{ FLT_MAX, 0, 0 };
+                dual_plane_form<S, 0>(lds, b, which, color[0], alpha[1], best);
+                dual_plane_form<S, 1>(lds, b, which, color[1], alpha[0], best);
+                dual_plane_form<S, 2>(lds, b, which, color[0], alpha[0], best);
+                shared.errors[4 + which][b] = best.error;
+                shared.words[4 + which][b] = make_uint4(uint32_t(best.lo), uint32_t(best.lo >> 32), uint32_t(best.hi), uint32_t(best.hi >> 32));
+            } else if (which == 4) {
+                finish_task<S, Mode6, 4, true>(lds, b, 0, 8);
+            } else {
+                finish_task<S, Mode7, 4, false>(lds, b, kPickTwoAlpha, 9);
+            }
+        }
+    }
+    __syncthreads();
+
+    // ---- 3. the best candidate
+    if (tid < BLOCKS) {
+        int const b = tid, bx = block_x(b), by = block_y(b);
+        if (bx < a.widthInBlocks && by < a.heightInBlocks) {
+            float bestError = FLT_MAX;
+            uint4 best = make_uint4(0u, 0u, 0u, 0u);
+            for (int slot = shared.withAlpha[b] ? 4 : 0; slot < kSlots; ++slot)
+                if (!(shared.errors[slot][b] > bestError)) { bestError = shared.errors[slot][b]; best = shared.words[slot][b]; }
+            store_block(a, bx, by, uint64_t(best.x) | uint64_t(best.y) << 32, uint64_t(best.z) | uint64_t(best.w) << 32);
+        }
+    }
 }
 
 // With a mode buffer.  A workgroup covers 16 x 16 blocks; its threads first read their blocks' entries,
@@ -617,7 +1164,7 @@ bc7_compress_modes_kernel(BlockCompressArgs a)
     Color<4> px[16];
     load_block(a, bx, by, px);
     uint64_t lo, hi;
-    bc7_encode<true>(px, mode, int(task >> 8), lo, hi);
+    bc7_encode_fixed(px, mode, int(task >> 8), lo, hi);
     store_block(a, bx, by, lo, hi);
 }
 
@@ -627,8 +1174,16 @@ hipError_t launch_bc7_compress(BlockCompressArgs const& a, hipStream_t stream)
         dim3 const grid((a.widthInBlocks + 15) / 16, (a.heightInBlocks + 15) / 16);
         hipLaunchKernelGGL(bc7_compress_modes_kernel, grid, dim3(256), 0, stream, a);
     } else {
-        dim3 const grid((a.widthInBlocks + 7) / 8, (a.heightInBlocks + 7) / 8);
-        hipLaunchKernelGGL(bc7_compress_kernel, grid, dim3(64), 0, stream, a);
+        // One group of 64 blocks per workgroup while there are no more groups than compute units (sixteen waves then
+        // have a unit to themselves), else two and half the waves, two workgroups to a unit: the groups' blocks with
+        // and without alpha fill their tasks' lanes better, and one workgroup works while the other waits for its
+        // last task.  512 x 512: 111 us (174 with two groups); 700 x 700: 222 (293 with four); 1024 x 1024: 290 (427
+        // with one).
+        int const groupsX = (a.widthInBlocks + 7) / 8, groupsY = (a.heightInBlocks + 7) / 8;
+        if (int64_t(groupsX) * groupsY <= compute_units_of_current_device())
+            hipLaunchKernelGGL((bc7_compress_kernel<1, 16>), dim3(groupsX, groupsY), dim3(1024), 0, stream, a);
+        else
+            hipLaunchKernelGGL((bc7_compress_kernel<2, 8>), dim3((groupsX + 1) / 2, groupsY), dim3(512), 0, stream, a);
     }
     return hipGetLastError();
 }

@@ -338,7 +338,7 @@ typedef uint32_t u32x4_a4  __attribute__((ext_vector_type(4), aligned(4)));
 // blockIdx.x, blockIdx.x + gridDim.x, ...
 struct GroupGrid { int32_t log2LanesX, tilesX, tiles; };
 
-static int compute_units_of_current_device()
+int compute_units_of_current_device()
 {
     static std::atomic<int> units[64];
     int device = 0;

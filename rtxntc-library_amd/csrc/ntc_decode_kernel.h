@@ -93,6 +93,8 @@ struct ReadChannelsArgs {
     int32_t dstWidth, dstHeight;   // size of the user image when it differs from the mip's (resampling copy), else 0
     uint8_t srcColorSpaces[16], dstColorSpaces[16];   // per copied channel: 0 linear, 1 sRGB, 2 HLG
 };
+// Compute units of the device that is current (kept per device after the first call).
+int compute_units_of_current_device();
 // Fills the colour-space tables of the current device that the copies read.
 hipError_t launch_transfer_tables(hipStream_t stream);
 hipError_t launch_read_channels(ReadChannelsArgs const& args, hipStream_t stream);

@@ -356,6 +356,30 @@ def test_gpu_bc7_matches_checker(ntc, device, oracle, tables, fmt):
 
 
 @pytest.mark.gpu
+def test_gpu_bc7_workgroups_of_one_and_of_two_groups_agree(ntc, device):
+    """An image with more groups of 8 x 8 blocks than the GPU has compute units against its two halves, which have
+    fewer; the last groups and pairs of groups are incomplete, opaque and other blocks come in every proportion."""
+    w, h = 4 * 131, 4 * 141                                                   # 17 x 18 groups
+    image = np.clip(np.rint(gpu_image(np.random.default_rng(77), w, h) * 255), 0, 255).astype(np.uint8)
+    image[: h // 3, :, 3] = 255
+    whole = compress_bc7(ntc, None, device, image, 1, 4, 131, 141)
+    upper = compress_bc7(ntc, None, device, image, 1, 4, 131, 72)
+    lower = compress_bc7(ntc, None, device, image, 1, 4, 131, 69, top=4 * 72)
+    assert np.array_equal(whole, np.concatenate([upper, lower]))
+
+
+@pytest.mark.gpu
+def test_gpu_bc7_infinite_and_huge_texels_match_checker(ntc, device, oracle):
+    rng = np.random.default_rng(78)
+    image = gpu_image(rng, 40, 24).astype(np.float32)
+    for value in (np.inf, -np.inf, np.nan, 1e30, -1e30, 3e38):
+        for _ in range(4):
+            image[rng.integers(0, 24), rng.integers(0, 40), rng.integers(0, 4)] = value
+    args = (image, 4, 4, 10, 6)
+    assert np.array_equal(compress_bc7(ntc, None, device, *args), compress_bc7(ntc, oracle, None, *args))
+
+
+@pytest.mark.gpu
 def test_gpu_bc7_arguments(ntc, device, oracle):
     from test_image_difference import fill_image
     rng = np.random.default_rng(9)
