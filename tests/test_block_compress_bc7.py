@@ -369,6 +369,23 @@ def test_gpu_bc7_workgroups_of_one_and_of_two_groups_agree(ntc, device):
 
 
 @pytest.mark.gpu
+def test_gpu_bc7_mode_lists_of_256_and_of_1024_blocks_agree(ntc, device):
+    """Given modes, an image beyond 256 blocks per compute unit (lists of 1024 blocks) against bands of it that are
+    not; every mode, blocks without an entry, incomplete workgroups."""
+    bx, by = 281, 259                                                         # 18 x 17 workgroups of 16 x 16 blocks
+    rng = np.random.default_rng(79)
+    image = np.clip(np.rint(gpu_image(rng, 4 * bx, 4 * by) * 255), 0, 255).astype(np.uint8)
+    mode = rng.choice(8, size=bx * by, p=[0.02, 0.1, 0.03, 0.1, 0.35, 0.25, 0.05, 0.1])
+    entries = np.where(rng.random(bx * by) < 0.01, 0, [entry_of(int(m), int(q) % (16 if m == 0 else 64)) for m, q in zip(mode, rng.integers(0, 64, bx * by))])
+    bits = ((entries[:, None] >> np.arange(9)) & 1).astype(np.uint8).reshape(-1)
+    buffer = np.packbits(np.concatenate([bits, np.zeros(-len(bits) % 32 + 32, dtype=np.uint8)]), bitorder="little")
+    args = dict(mode_buffer=buffer, map_size=(bx, by))
+    whole = compress_bc7(ntc, None, device, image, 1, 4, bx, by, **args)
+    bands = [compress_bc7(ntc, None, device, image, 1, 4, bx, rows, top=4 * top, map_offset=(0, top), **args) for top, rows in ((0, 100), (100, 100), (200, by - 200))]
+    assert np.array_equal(whole, np.concatenate(bands))
+
+
+@pytest.mark.gpu
 def test_gpu_bc7_infinite_and_huge_texels_match_checker(ntc, device, oracle):
     rng = np.random.default_rng(78)
     image = gpu_image(rng, 40, 24).astype(np.float32)
