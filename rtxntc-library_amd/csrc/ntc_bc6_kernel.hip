@@ -1,8 +1,8 @@
 // ntc_bc6_kernel.hip - BC6H (unsigned half float) block compression of a decoded image (gfx950).
 //
 // The reference's BC6 pass (IContext::MakeBlockCompressionComputePass with BlockCompressedFormat::BC6,
-// src/shaders/CompressBC6.hlsl) as a compute kernel: one lane encodes one 4 x 4 block.  Two candidates,
-// the smaller luminance-weighted mean squared log2 error wins:
+// src/shaders/CompressBC6.hlsl) as a compute kernel.  Two candidates, the
+// smaller luminance-weighted mean squared log2 error wins:
 //   * one subset, 10-bit endpoints, 4-bit indices (mode 11 of the format): bounding box, pulled inwards in
 //     log2 space by at most 1/32 of its extent, one least-squares refit in half-code space;
 //   * two subsets with 3-bit indices on the partition (of the format's first 32) whose texels lie closest
@@ -31,8 +31,47 @@ __constant__ uint16_t kSecondSubset[32] = {
 };
 __constant__ uint8_t kSecondAnchor[32] = { 15, 15, 15, 15, 15, 15, 15, 15, 15, 15, 15, 15, 15, 15, 15, 15, 15, 2, 8, 2, 2, 8, 8, 15, 2, 8, 2, 2, 8, 8, 2, 2 };
 
+// a / b in fewer instructions than the compiler's division, which scales its operands against overflow and always
+// refines the hardware's reciprocal and the quotient as far as the worst operands need.  REFINED: how often the
+// reciprocal is; then the quotient is corrected once by its remainder, which leaves it within 2^-44 of itself before the
+// last rounding.  Where it is used the result is the correctly rounded one.  <0>: integers below 2^17, whose quotients
+// are no nearer than 2^-42 to the middle between two numbers; (m - 1) / (m + 1), m in [0.70, 1.42], compared with the
+// division for every m.  <1>: (y + 1) / (x + 1) with y a half and x a half, a UNORM code over its maximum or an integer
+// up to 65504, compared for every pair.  quotient_by() is the compiler's own sequence without the scaling, which none of
+// the operands needs where texels are no FLOAT32.
+BC6_INLINE float corrected(float a, float b, float r)
+{
+    float const q = a * r;
+    return __builtin_fmaf(__builtin_fmaf(-q, b, a), r, q);
+}
+template <int REFINED> BC6_INLINE float reciprocal(float b)
+{
+    float r = __builtin_amdgcn_rcpf(b);
+    if constexpr (REFINED == 1) r = __builtin_fmaf(__builtin_fmaf(-b, r, 1.f), r, r);
+    return r;
+}
+template <int REFINED> BC6_INLINE float quotient(float a, float b) { return corrected(a, b, reciprocal<REFINED>(b)); }
+BC6_INLINE float quotient_by(float a, float b, float r)      // r = reciprocal<1>(b)
+{
+    float const q = corrected(a, b, r);
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-q, b, a), r, q), b, a);
+}
+
 // log2 for x >= 0 (0 -> -inf); NaN for a negative or NaN argument.  Argument reduction to [sqrt(1/2), sqrt 2),
 // then the series of atanh; a few units in the last place.
+// (normal_log2: of a normal number's bits, the exponent raised by `e`.)
+BC6_INLINE float normal_log2(uint32_t bits, int e)
+{
+    int const above = int(bits - 0x3f3504f4u);               // of the number that follows 1.41421354 / 2
+    e += above >> 23;
+    float const m = __uint_as_float(bits - (uint32_t(above) & 0xff800000u));
+    float const t = quotient<0>(m - 1.f, m + 1.f), t2 = t * t;
+    float p = t2 * (1.f / 9.f) + (1.f / 7.f);
+    p = p * t2 + 0.2f;
+    p = p * t2 + (1.f / 3.f);
+    p = p * t2 + 1.f;
+    return float(e) + p * t * 2.88539004f;
+}
 BC6_INLINE float det_log2(float x)
 {
     if (!(x >= 0.f)) return __uint_as_float(0x7fc00000u);
@@ -41,23 +80,12 @@ BC6_INLINE float det_log2(float x)
     if (b >= 0x7f800000u) return x;
     int e = 0;
     if (b < 0x00800000u) { x *= 8388608.f; b = __float_as_uint(x); e = -23; }
-    e += int(b >> 23) - 127;
-    float m = __uint_as_float((b & 0x007fffffu) | 0x3f800000u);
-    if (m > 1.41421354f) { m *= 0.5f; e += 1; }
-    float const t = (m - 1.f) / (m + 1.f), t2 = t * t;
-    float p = t2 * (1.f / 9.f) + (1.f / 7.f);
-    p = p * t2 + 0.2f;
-    p = p * t2 + (1.f / 3.f);
-    p = p * t2 + 1.f;
-    return float(e) + p * t * 2.88539004f;
+    return normal_log2(b, e);
 }
 
-// 2^x: +inf from 128, 0 below -150.
-BC6_INLINE float det_exp2(float x)
+// 2^x for the x that occur here: logarithms of numbers between 1 and 65505.
+BC6_INLINE float exp2_of_log(float x)
 {
-    if (x != x) return x;
-    if (x >= 128.f) return __uint_as_float(0x7f800000u);
-    if (x < -150.f) return 0.f;
     float const n = rintf(x), g = (x - n) * 0.693147182f;
     float p = g * (1.f / 5040.f) + (1.f / 720.f);
     p = p * g + (1.f / 120.f);
@@ -66,10 +94,7 @@ BC6_INLINE float det_exp2(float x)
     p = p * g + 0.5f;
     p = p * g + 1.f;
     p = p * g + 1.f;
-    int k = int(n);
-    if (k > 127) { p *= 2.f; k -= 1; }
-    if (k < -126) { p *= 5.96046448e-08f; k += 24; }
-    return p * __uint_as_float(uint32_t(k + 127) << 23);
+    return p * __uint_as_float(uint32_t(int(n) + 127) << 23);
 }
 
 struct V3 { float x, y, z; };
@@ -83,24 +108,42 @@ BC6_INLINE V3 vmax(V3 a, V3 b) { return { max_f32(a.x, b.x), max_f32(a.y, b.y), 
 BC6_INLINE float clampf(float v, float lo, float hi) { return fminf(fmaxf(v, lo), hi); }
 // A float as the number of its half-precision bit pattern, and back (the latter truncates to an integer first).
 // (a NaN always gives the code 0x7e00, whatever its sign and payload)
-BC6_INLINE float to_half_bits(float v) { return v != v ? 32256.f : float(__builtin_bit_cast(uint16_t, _Float16(v))); }
+BC6_INLINE float number_to_half_bits(float v) { return float(__builtin_bit_cast(uint16_t, _Float16(v))); }
+BC6_INLINE float to_half_bits(float v) { return v != v ? 32256.f : number_to_half_bits(v); }
 BC6_INLINE float from_half_bits(float v) { return float(__builtin_bit_cast(_Float16, uint16_t(uint32_t(v)))); }
 BC6_INLINE V3 to_half_bits(V3 v) { return { to_half_bits(v.x), to_half_bits(v.y), to_half_bits(v.z) }; }
 
 constexpr float kHalfMax = 65504.f;
 constexpr float kHalfMaxCode = 31743.f;         // 0x7bff, the code of 65504
 
-BC6_INLINE float msle(V3 a, V3 b)
-{
-    V3 const d{ det_log2((b.x + 1.f) / (a.x + 1.f)), det_log2((b.y + 1.f) / (a.y + 1.f)), det_log2((b.z + 1.f) / (a.z + 1.f)) };
-    V3 const sq = d * d * V3{ 0.299f, 0.587f, 0.114f };
-    return sq.x + sq.y + sq.z;
-}
+// One texel against what a decoder shows: WIDE texels come from a FLOAT32 image and can be any number up to 65504,
+// others are halves, UNORM quotients or integers.
+template <bool WIDE> struct Msle {
+    V3 a, r;                                                 // the texel plus 1, its reciprocals
+    BC6_INLINE explicit Msle(V3 texel) : a(texel + V3{ 1.f, 1.f, 1.f })
+    {
+        if constexpr (!WIDE) r = V3{ reciprocal<1>(a.x), reciprocal<1>(a.y), reciprocal<1>(a.z) };
+    }
+    BC6_INLINE float operator()(V3 b) const
+    {
+        V3 d;
+        uint32_t const largest = max(max(__float_as_uint(b.x), __float_as_uint(b.y)), __float_as_uint(b.z));
+        if (WIDE || largest >= 0x7f800000u) {                // (endpoints near the top decode to infinity or NaN)
+            d = V3{ det_log2((b.x + 1.f) / a.x), det_log2((b.y + 1.f) / a.y), det_log2((b.z + 1.f) / a.z) };
+        } else {
+            d = V3{ normal_log2(__float_as_uint(corrected(b.x + 1.f, a.x, r.x)), 0), normal_log2(__float_as_uint(corrected(b.y + 1.f, a.y, r.y)), 0),
+                    normal_log2(__float_as_uint(corrected(b.z + 1.f, a.z, r.z)), 0) };
+        }
+        V3 const sq = d * d * V3{ 0.299f, 0.587f, 0.114f };
+        return sq.x + sq.y + sq.z;
+    }
+};
 
+// (the quotients by constants here and below are those of integers, times a power of two)
 BC6_INLINE V3 quantize(V3 v, float levels)
 {
     V3 const h = to_half_bits(v);
-    return { (h.x * levels) / 31744.f, (h.y * levels) / 31744.f, (h.z * levels) / 31744.f };
+    return { corrected(h.x * levels, 31744.f, 1.f / 31744.f), corrected(h.y * levels, 31744.f, 1.f / 31744.f), corrected(h.z * levels, 31744.f, 1.f / 31744.f) };
 }
 BC6_INLINE V3 unquantize(V3 v, float levels)
 {
@@ -113,24 +156,69 @@ BC6_INLINE V3 interpolate(V3 e0, V3 e1, float weight)
 }
 BC6_INLINE uint32_t index_of(float pos, float e0, float e1, float scale, float bias, float top)
 {
-    float const r = (pos - e0) / (e1 - e0);
+    float const a = pos - e0, b = e1 - e0;                   // half codes: integers
+    float const r = __builtin_amdgcn_div_fixupf(quotient<0>(a, b), b, a);
     return uint32_t(clampf(r * scale + bias + 0.5f, 0.f, top));      // a NaN (coinciding ends) gives 0
 }
 BC6_INLINE uint32_t index3(float pos, float e0, float e1) { return index_of(pos, e0, e1, 6.98182f, 0.00909f, 7.f); }
 BC6_INLINE uint32_t index4(float pos, float e0, float e1) { return index_of(pos, e0, e1, 14.93333f, 0.03333f, 15.f); }
-BC6_INLINE V3 direction(V3 lo, V3 hi) { V3 const d = hi - lo; float const s = d.x + d.y + d.z; return { d.x / s, d.y / s, d.z / s }; }
+template <bool WIDE> BC6_INLINE V3 divided(V3 v, float s)
+{
+    if constexpr (WIDE) return { v.x / s, v.y / s, v.z / s };
+    float const r = reciprocal<1>(s);
+    return { quotient_by(v.x, s, r), quotient_by(v.y, s, r), quotient_by(v.z, s, r) };
+}
+template <bool WIDE> BC6_INLINE V3 direction(V3 lo, V3 hi) { V3 const d = hi - lo; return divided<WIDE>(d, d.x + d.y + d.z); }
 
-BC6_INLINE float log1(float c) { return det_log2(c + 1.f); }
-BC6_INLINE float exp1(float c) { return det_exp2(c) - 1.f; }
+BC6_INLINE float log1(float c) { return normal_log2(__float_as_uint(c + 1.f), 0); }
+BC6_INLINE float exp1(float c) { return exp2_of_log(c) - 1.f; }
+
+// ---- the workgroup ------------------------------------------------------------------------------------
+//
+// Four waves encode 64 blocks, whose texels lie in LDS; the lanes of a wave are blocks.
+//   1. one wave: the one-subset endpoints; then all: patterns' scores, taken in turn, their minimum by an atomic in LDS;
+//   2. a wave per subset of each block's pattern: its endpoints;
+//   3. each wave four of the sixteen texels: indices and errors of all three candidates;
+//   4. one wave: the errors added up in texel order, the choice, the block.
+// Bound by the issue of vector instructions: about 34000 for the 64 blocks, 20000 of them for the 32 scores (a score's
+// boxes are straight-line code per subset size, read with uniform masks).  Each part is a function with registers of its
+// own, so that four waves fit a SIMD and nothing is spilled in a loop; the search is one call because a call saves
+// registers to scratch (a call per two patterns: 257 us at 2048 x 2048).  One lane per block, all parts in one body with
+// 168 registers, took 121 us at 64 x 64, 151 at 1024 x 1024 and 287 at 2048 x 2048; this takes 30, 61 and 204: the
+// chain of one lane's scores is what small images waited for, and large ones for its spills and longer divisions.
+struct Bc6Lds {
+    float4 texels[16][64];
+    float one[11][64];                                       // one subset: lo, hi, direction, codes of the ends along it
+    float two[2][11][64];                                    // each of two subsets
+    float errors[3][16][64];                                 // per texel: one subset, 7 + 6 bits, 9 + 5 bits
+    uint32_t indices[2][4][64];                              // of four texels: 4 bits each, 3 bits each
+    uint64_t pick[64];                                       // score bits << 32 | pattern
+    uint32_t unscored[64];                                   // pattern 0's score is a NaN: the search stays there
+    int next;
+};
+using Bc6Ptr = __attribute__((address_space(3))) Bc6Lds*;
+#define BC6_TASK __device__ __attribute__((noinline))        // (separate register allocation; uniform arguments are made so again)
+
+BC6_INLINE V3 texel(Bc6Ptr lds, int b, int t) { return { lds->texels[t][b].x, lds->texels[t][b].y, lds->texels[t][b].z }; }
+struct SubsetEnds { V3 lo, hi, dir; float e0, e1; };
+template <class P> BC6_INLINE void store_ends(P to, int b, SubsetEnds const& s)
+{
+    to[0][b] = s.lo.x; to[1][b] = s.lo.y; to[2][b] = s.lo.z; to[3][b] = s.hi.x; to[4][b] = s.hi.y; to[5][b] = s.hi.z;
+    to[6][b] = s.dir.x; to[7][b] = s.dir.y; to[8][b] = s.dir.z; to[9][b] = s.e0; to[10][b] = s.e1;
+}
+template <class P> BC6_INLINE SubsetEnds load_ends(P from, int b)
+{
+    return { { from[0][b], from[1][b], from[2][b] }, { from[3][b], from[4][b], from[5][b] }, { from[6][b], from[7][b], from[8][b] }, from[9][b], from[10][b] };
+}
 
 // Pulls the box inwards in log2(1 + x) space: towards the smallest / largest values that are not the
 // extremes themselves, by at most 1/32 of the extent.
-BC6_INLINE void inset_box(V3 const (&px)[16], V3& lo, V3& hi)
+BC6_INLINE void inset_box(Bc6Ptr lds, int b, V3& lo, V3& hi)
 {
     V3 innerLo = hi, innerHi = lo;
-#pragma unroll
+#pragma unroll 4
     for (int t = 0; t < 16; ++t) {
-        V3 const p = px[t];
+        V3 const p = texel(lds, b, t);
         innerLo = vmin(innerLo, V3{ p.x == lo.x ? innerLo.x : p.x, p.y == lo.y ? innerLo.y : p.y, p.z == lo.z ? innerLo.z : p.z });
         innerHi = vmax(innerHi, V3{ p.x == hi.x ? innerHi.x : p.x, p.y == hi.y ? innerHi.y : p.y, p.z == hi.z ? innerHi.z : p.z });
     }
@@ -145,34 +233,32 @@ BC6_INLINE void inset_box(V3 const (&px)[16], V3& lo, V3& hi)
 
 // Least-squares endpoints, in half-code space, for the indices the current endpoints give to the texels
 // of `members` (bit t = texel t takes part).  False when the system is singular.
-template <bool FOUR_BIT>
-BC6_INLINE bool refit(V3 const (&px)[16], uint32_t members, V3 lo, V3 hi, V3& outLo, V3& outHi)
+template <bool WIDE, bool FOUR_BIT>
+BC6_INLINE bool refit(Bc6Ptr lds, int b, uint32_t members, V3 lo, V3 hi, V3& outLo, V3& outHi)
 {
-    V3 const dir = direction(lo, hi);
+    V3 const dir = direction<WIDE>(lo, hi);
     float const e0 = to_half_bits(dot(lo, dir)), e1 = to_half_bits(dot(hi, dir));
     V3 alphaSum{ 0.f, 0.f, 0.f }, betaSum{ 0.f, 0.f, 0.f };
     float ab = 0.f, aa = 0.f, bb = 0.f;
-#pragma unroll
-    for (int t = 0; t < 16; ++t)
-        if ((members >> t) & 1u) {
-            float const pos = to_half_bits(dot(px[t], dir));
-            uint32_t const index = FOUR_BIT ? index4(pos, e0, e1) : index3(pos, e0, e1);
-            float const beta = clampf(float(index) / (FOUR_BIT ? 15.f : 7.f), 0.f, 1.f), alpha = 1.f - beta;
-            V3 const h = to_half_bits(px[t]);
-            alphaSum = alphaSum + h * alpha; betaSum = betaSum + h * beta;
-            ab += alpha * beta; aa += alpha * alpha; bb += beta * beta;
-        }
+    for (uint32_t m = members; m; m &= m - 1) {
+        V3 const p = texel(lds, b, __ffs(int(m)) - 1);
+        float const pos = to_half_bits(dot(p, dir));
+        uint32_t const index = FOUR_BIT ? index4(pos, e0, e1) : index3(pos, e0, e1);
+        constexpr float top = FOUR_BIT ? 15.f : 7.f;
+        float const beta = clampf(corrected(float(index), top, 1.f / top), 0.f, 1.f), alpha = 1.f - beta;
+        V3 const h{ number_to_half_bits(p.x), number_to_half_bits(p.y), number_to_half_bits(p.z) };
+        alphaSum = alphaSum + h * alpha; betaSum = betaSum + h * beta;
+        ab += alpha * beta; aa += alpha * alpha; bb += beta * beta;
+    }
     float const det = aa * bb - ab * ab;
     if (!(fabsf(det) > 0.00001f)) return false;
     float const rcp = 1.f / det;
-    V3 const a = (alphaSum * bb - betaSum * ab) * rcp, b = (betaSum * aa - alphaSum * ab) * rcp;
+    V3 const u = (alphaSum * bb - betaSum * ab) * rcp, v = (betaSum * aa - alphaSum * ab) * rcp;
     // (the shader clamps these codes to 65504, which lets the codes of infinities and NaNs through)
-    outLo = V3{ from_half_bits(clampf(a.x, 0.f, kHalfMaxCode)), from_half_bits(clampf(a.y, 0.f, kHalfMaxCode)), from_half_bits(clampf(a.z, 0.f, kHalfMaxCode)) };
-    outHi = V3{ from_half_bits(clampf(b.x, 0.f, kHalfMaxCode)), from_half_bits(clampf(b.y, 0.f, kHalfMaxCode)), from_half_bits(clampf(b.z, 0.f, kHalfMaxCode)) };
+    outLo = V3{ from_half_bits(clampf(u.x, 0.f, kHalfMaxCode)), from_half_bits(clampf(u.y, 0.f, kHalfMaxCode)), from_half_bits(clampf(u.z, 0.f, kHalfMaxCode)) };
+    outHi = V3{ from_half_bits(clampf(v.x, 0.f, kHalfMaxCode)), from_half_bits(clampf(v.y, 0.f, kHalfMaxCode)), from_half_bits(clampf(v.z, 0.f, kHalfMaxCode)) };
     return true;
 }
-
-struct Block { uint64_t lo, hi; float error; };
 
 // 128-bit field writer for constant positions.
 struct Bits {
@@ -185,186 +271,270 @@ struct Bits {
     }
 };
 
-BC6_INLINE Block encode_one_subset(V3 const (&px)[16])
+// Endpoints of the one-subset candidate, in the order that gives texel 0 an index below 8 (`lo` and the first code are
+// the first endpoint's).
+template <bool WIDE>
+BC6_TASK void one_subset_ends(Bc6Ptr lds, int b)
 {
-    V3 lo = px[0], hi = px[0];
-#pragma unroll
-    for (int t = 1; t < 16; ++t) { lo = vmin(lo, px[t]); hi = vmax(hi, px[t]); }
+    V3 lo = texel(lds, b, 0), hi = lo;
+#pragma unroll 5
+    for (int t = 1; t < 16; ++t) { V3 const p = texel(lds, b, t); lo = vmin(lo, p); hi = vmax(hi, p); }
     V3 const boxLo = lo, boxHi = hi;
-    inset_box(px, lo, hi);
+    inset_box(lds, b, lo, hi);
     V3 fitLo, fitHi;
-    if (refit<true>(px, 0xffffu, lo, hi, fitLo, fitHi)) {
+    if (refit<WIDE, true>(lds, b, 0xffffu, lo, hi, fitLo, fitHi)) {
         lo = vmin(vmax(fitLo, boxLo), boxHi);
         hi = vmin(vmax(fitHi, boxLo), boxHi);
     }
-    V3 const dir = direction(lo, hi);
-    V3 q0 = quantize(lo, 1024.f), q1 = quantize(hi, 1024.f);
-    float e0 = to_half_bits(dot(lo, dir)), e1 = to_half_bits(dot(hi, dir));
-    if (index4(to_half_bits(dot(px[0], dir)), e0, e1) > 7) {
-        float const t = e0; e0 = e1; e1 = t;
-        V3 const q = q0; q0 = q1; q1 = q;
+    SubsetEnds s{ lo, hi, direction<WIDE>(lo, hi), 0.f, 0.f };
+    s.e0 = to_half_bits(dot(lo, s.dir)); s.e1 = to_half_bits(dot(hi, s.dir));
+    if (index4(to_half_bits(dot(texel(lds, b, 0), s.dir)), s.e0, s.e1) > 7) {
+        float const e = s.e0; s.e0 = s.e1; s.e1 = e;
+        V3 const v = s.lo; s.lo = s.hi; s.hi = v;
     }
-    V3 const u0 = unquantize(q0, 1024.f), u1 = unquantize(q1, 1024.f);
-    Bits b;
-    b.put(0, 0x03, 5);
-    b.put(5, uint32_t(q0.x), 10); b.put(15, uint32_t(q0.y), 10); b.put(25, uint32_t(q0.z), 10);
-    b.put(35, uint32_t(q1.x), 10); b.put(45, uint32_t(q1.y), 10); b.put(55, uint32_t(q1.z), 10);
-    float error = 0.f;
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-        uint32_t const index = index4(to_half_bits(dot(px[t], dir)), e0, e1);
-        error += msle(px[t], interpolate(u0, u1, floorf((float(index) * 64.f) / 15.f + 0.5f)));
-        b.put(t == 0 ? 65 : 64 + 4 * t, index, t == 0 ? 3 : 4);
-    }
-    return Block{ b.lo, b.hi, error };
+    store_ends(lds->one, b, s);
 }
 
-BC6_INLINE void subset_boxes(V3 const (&px)[16], uint32_t second, V3 (&lo)[2], V3 (&hi)[2])
-{
-#pragma unroll
-    for (int s = 0; s < 2; ++s) { lo[s] = V3{ kHalfMax, kHalfMax, kHalfMax }; hi[s] = V3{ 0.f, 0.f, 0.f }; }
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-        if ((second >> t) & 1u) { lo[1] = vmin(lo[1], px[t]); hi[1] = vmax(hi[1], px[t]); }
-        else                    { lo[0] = vmin(lo[0], px[t]); hi[0] = vmax(hi[0], px[t]); }
-    }
-}
-
-BC6_INLINE V3 normalized(V3 v) { float const len = sqrtf(dot(v, v)); return { v.x / len, v.y / len, v.z / len }; }
+template <bool WIDE> BC6_INLINE V3 normalized(V3 v) { return divided<WIDE>(v, sqrtf(dot(v, v))); }
 BC6_INLINE float distance_to_line2(V3 origin, V3 dir, V3 p)
 {
     V3 const w = p - origin, x = w - dir * dot(w, dir);
     return dot(x, x);
 }
 
-// Sum of the texels' squared distances from the diagonal of their subset's bounding box.
-BC6_INLINE float pattern_score(V3 const (&px)[16], uint32_t second)
+// Bounding box of the N texels of a subset (uniform), the box of no texel being [65504, 0] as in the start values.
+template <int N> BC6_INLINE void box_of(Bc6Ptr lds, int b, uint32_t members, V3& lo, V3& hi)
 {
-    V3 lo[2], hi[2];
-    subset_boxes(px, second, lo, hi);
-    V3 const dir0 = normalized(hi[0] - lo[0]), dir1 = normalized(hi[1] - lo[1]);
-    float total = 0.f;
+    V3 p[N];
 #pragma unroll
-    for (int t = 0; t < 16; ++t)
-        total += ((second >> t) & 1u) ? distance_to_line2(lo[1], dir1, px[t]) : distance_to_line2(lo[0], dir0, px[t]);
-    return total;
+    for (int i = 0; i < N; ++i) { p[i] = texel(lds, b, __ffs(int(members)) - 1); members &= members - 1; }
+    lo = V3{ kHalfMax, kHalfMax, kHalfMax }; hi = V3{ 0.f, 0.f, 0.f };
+#pragma unroll
+    for (int i = 0; i + 1 < N; i += 2) {
+        lo = V3{ min3_f32(lo.x, p[i].x, p[i + 1].x), min3_f32(lo.y, p[i].y, p[i + 1].y), min3_f32(lo.z, p[i].z, p[i + 1].z) };
+        hi = V3{ max3_f32(hi.x, p[i].x, p[i + 1].x), max3_f32(hi.y, p[i].y, p[i + 1].y), max3_f32(hi.z, p[i].z, p[i + 1].z) };
+    }
+    if constexpr (N & 1) { lo = vmin(lo, p[N - 1]); hi = vmax(hi, p[N - 1]); }
+}
+BC6_INLINE void box_of_members(Bc6Ptr lds, int b, uint32_t members, V3& lo, V3& hi)
+{
+    switch (__popc(members)) {                               // the sizes that the patterns' subsets have
+    case 3:  box_of<3>(lds, b, members, lo, hi); break;
+    case 4:  box_of<4>(lds, b, members, lo, hi); break;
+    case 6:  box_of<6>(lds, b, members, lo, hi); break;
+    case 8:  box_of<8>(lds, b, members, lo, hi); break;
+    case 10: box_of<10>(lds, b, members, lo, hi); break;
+    case 12: box_of<12>(lds, b, members, lo, hi); break;
+    default: box_of<13>(lds, b, members, lo, hi); break;
+    }
+}
+
+// Scores of the patterns that this wave takes: the sum of the texels' squared distances from the diagonal of their
+// subset's bounding box.
+template <bool WIDE>
+BC6_TASK void score_patterns(Bc6Ptr lds, int b)
+{
+    V3 px[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) px[t] = texel(lds, b, t);
+    uint64_t best = ~uint64_t(0);
+#pragma unroll 1
+    for (;;) {
+        int p = 0;
+        if (b == 0) p = __hip_atomic_fetch_add(&lds->next, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        p = __builtin_amdgcn_readfirstlane(p);
+        if (p >= 32) break;                                  // uniform: every wave gets here
+        uint32_t const second = kSecondSubset[p];
+        V3 lo[2], hi[2];
+        box_of_members(lds, b, ~second & 0xffffu, lo[0], hi[0]);
+        box_of_members(lds, b, second, lo[1], hi[1]);
+        V3 const dir0 = normalized<WIDE>(hi[0] - lo[0]), dir1 = normalized<WIDE>(hi[1] - lo[1]);
+        float score = 0.f;
+#pragma unroll
+        for (int t = 0; t < 16; ++t)
+            score += ((second >> t) & 1u) ? distance_to_line2(lo[1], dir1, px[t]) : distance_to_line2(lo[0], dir0, px[t]);
+        // scores are not negative, a NaN's bits are above all numbers': the smallest key is the first smallest score
+        uint64_t const key = uint64_t(__float_as_uint(score) & 0x7fffffffu) << 32 | uint32_t(p);
+        best = key < best ? key : best;
+        if (p == 0) lds->unscored[b] = score != score;
+    }
+    __hip_atomic_fetch_min(&lds->pick[b], best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+BC6_INLINE int picked_pattern(Bc6Ptr lds, int b) { return lds->unscored[b] ? 0 : int(uint32_t(lds->pick[b])); }
+
+// Endpoints of subset s of the picked pattern, in the order that gives its anchor an index below 4.
+template <bool WIDE>
+BC6_TASK void subset_ends(Bc6Ptr lds, int b, int s)
+{
+    s = __builtin_amdgcn_readfirstlane(s);
+    int const pattern = picked_pattern(lds, b);
+    uint32_t const members = s ? uint32_t(kSecondSubset[pattern]) : ~uint32_t(kSecondSubset[pattern]) & 0xffffu;
+    V3 lo{ kHalfMax, kHalfMax, kHalfMax }, hi{ 0.f, 0.f, 0.f };
+    for (uint32_t m = members; m; m &= m - 1) { V3 const p = texel(lds, b, __ffs(int(m)) - 1); lo = vmin(lo, p); hi = vmax(hi, p); }
+    V3 fitLo, fitHi;
+    if (refit<WIDE, false>(lds, b, members, lo, hi, fitLo, fitHi)) { lo = fitLo; hi = fitHi; }
+    SubsetEnds e{ lo, hi, direction<WIDE>(lo, hi), 0.f, 0.f };
+    e.e0 = to_half_bits(dot(lo, e.dir)); e.e1 = to_half_bits(dot(hi, e.dir));
+    if (index3(to_half_bits(dot(texel(lds, b, s ? int(kSecondAnchor[pattern]) : 0), e.dir)), e.e0, e.e1) > 3) {
+        float const x = e.e0; e.e0 = e.e1; e.e1 = x;
+        V3 const v = e.lo; e.lo = e.hi; e.hi = v;
+    }
+    store_ends(lds->two[s], b, e);
 }
 
 BC6_INLINE uint32_t field(float v, int bits) { return uint32_t(int(v)) & ((1u << bits) - 1u); }      // two's complement of a small integer
 BC6_INLINE V3 floor3(V3 v) { return { floorf(v.x), floorf(v.y), floorf(v.z) }; }
 BC6_INLINE V3 clamp3(V3 v, float limit) { return { clampf(v.x, -limit, limit), clampf(v.y, -limit, limit), clampf(v.z, -limit, limit) }; }
 
-BC6_INLINE void encode_two_subsets(V3 const (&px)[16], int pattern, Block& best)
+// The two-subset endpoints as a base and three signed deltas.
+BC6_INLINE void base_and_deltas(Bc6Ptr lds, int b, float levels, float limit, V3 (&q)[4])
 {
-    uint32_t const second = kSecondSubset[pattern];
-    int const anchor1 = kSecondAnchor[pattern];
-    V3 lo[2], hi[2];
-    subset_boxes(px, second, lo, hi);
-    {
-        V3 fitLo, fitHi;
-        if (refit<false>(px, ~second & 0xffffu, lo[0], hi[0], fitLo, fitHi)) { lo[0] = fitLo; hi[0] = fitHi; }
-        if (refit<false>(px, second, lo[1], hi[1], fitLo, fitHi)) { lo[1] = fitLo; hi[1] = fitHi; }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        auto const& from = lds->two[i >> 1];
+        int const at = 3 * (i & 1);
+        q[i] = floor3(quantize(V3{ from[at][b], from[at + 1][b], from[at + 2][b] }, levels));
     }
-    V3 const dir0 = direction(lo[0], hi[0]), dir1 = direction(lo[1], hi[1]);
-    float e00 = to_half_bits(dot(lo[0], dir0)), e01 = to_half_bits(dot(hi[0], dir0));
-    float e10 = to_half_bits(dot(lo[1], dir1)), e11 = to_half_bits(dot(hi[1], dir1));
-    V3 anchorTexel = px[0];
 #pragma unroll
-    for (int t = 1; t < 16; ++t) if (t == anchor1) anchorTexel = px[t];
-    if (index3(to_half_bits(dot(px[0], dir0)), e00, e01) > 3) { float const t = e00; e00 = e01; e01 = t; V3 const v = lo[0]; lo[0] = hi[0]; hi[0] = v; }
-    if (index3(to_half_bits(dot(anchorTexel, dir1)), e10, e11) > 3) { float const t = e10; e10 = e11; e11 = t; V3 const v = lo[1]; lo[1] = hi[1]; hi[1] = v; }
+    for (int i = 1; i < 4; ++i) q[i] = clamp3(q[i] - q[0], limit);
+}
 
-    // endpoints: base + three signed deltas, as 7 + 6 bits and as 9 + 5 bits
-    V3 const ends[4] = { lo[0], hi[0], lo[1], hi[1] };
-    V3 q7[4], q9[4], u7[4], u9[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { q7[i] = floor3(quantize(ends[i], 128.f)); q9[i] = floor3(quantize(ends[i], 512.f)); }
-#pragma unroll
-    for (int i = 1; i < 4; ++i) { q7[i] = clamp3(q7[i] - q7[0], 31.f); q9[i] = clamp3(q9[i] - q9[0], 15.f); }
+// Indices and errors of four texels under the three candidates.
+template <bool WIDE>
+BC6_TASK void texel_errors(Bc6Ptr lds, int b, int quarter)
+{
+    quarter = __builtin_amdgcn_readfirstlane(quarter);
+    uint32_t indices = 0;
+    {
+        SubsetEnds const s = load_ends(lds->one, b);
+        V3 const u0 = unquantize(quantize(s.lo, 1024.f), 1024.f), u1 = unquantize(quantize(s.hi, 1024.f), 1024.f);
+#pragma unroll 2
+        for (int i = 0; i < 4; ++i) {
+            V3 const p = texel(lds, b, 4 * quarter + i);
+            uint32_t const index = index4(to_half_bits(dot(p, s.dir)), s.e0, s.e1);
+            lds->errors[0][4 * quarter + i][b] = Msle<WIDE>(p)(interpolate(u0, u1, floorf(corrected(float(index) * 64.f, 15.f, 1.f / 15.f) + 0.5f)));
+            indices |= index << (4 * i);
+        }
+        lds->indices[0][quarter][b] = indices;
+    }
+    V3 q7[4], q9[4];
+    base_and_deltas(lds, b, 128.f, 31.f, q7);
+    base_and_deltas(lds, b, 512.f, 15.f, q9);
+    V3 u7[4], u9[4];
     u7[0] = unquantize(q7[0], 128.f); u9[0] = unquantize(q9[0], 512.f);
 #pragma unroll
     for (int i = 1; i < 4; ++i) { u7[i] = unquantize(q7[0] + q7[i], 128.f); u9[i] = unquantize(q9[0] + q9[i], 512.f); }
-    float error7 = 0.f, error9 = 0.f;
-    uint32_t index[16];
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
+    uint32_t const second = kSecondSubset[picked_pattern(lds, b)];
+    indices = 0;
+#pragma unroll 1
+    for (int i = 0; i < 4; ++i) {
+        int const t = 4 * quarter + i;
+        V3 const p = texel(lds, b, t);
         bool const s = (second >> t) & 1u;
-        index[t] = s ? index3(to_half_bits(dot(px[t], dir1)), e10, e11) : index3(to_half_bits(dot(px[t], dir0)), e00, e01);
-        float const weight = floorf((float(index[t]) * 64.f) / 7.f + 0.5f);
-        error7 += msle(px[t], interpolate(s ? u7[2] : u7[0], s ? u7[3] : u7[1], weight));
-        error9 += msle(px[t], interpolate(s ? u9[2] : u9[0], s ? u9[3] : u9[1], weight));
+        V3 const dir{ lds->two[s][6][b], lds->two[s][7][b], lds->two[s][8][b] };
+        uint32_t const index = index3(to_half_bits(dot(p, dir)), lds->two[s][9][b], lds->two[s][10][b]);
+        float const weight = floorf(corrected(float(index) * 64.f, 7.f, 1.f / 7.f) + 0.5f);
+        Msle<WIDE> const error(p);
+        lds->errors[1][t][b] = error(interpolate(s ? u7[2] : u7[0], s ? u7[3] : u7[1], weight));
+        lds->errors[2][t][b] = error(interpolate(s ? u9[2] : u9[0], s ? u9[3] : u9[1], weight));
+        indices |= index << (3 * i);
     }
+    lds->indices[1][quarter][b] = indices;
+}
+
+// The choice between the candidates and the block.
+BC6_INLINE void final_block(Bc6Ptr lds, int b, uint64_t& outLo, uint64_t& outHi)
+{
+    float error1 = 0.f, error7 = 0.f, error9 = 0.f;
+#pragma unroll
+    for (int t = 0; t < 16; ++t) { error1 += lds->errors[0][t][b]; error7 += lds->errors[1][t][b]; error9 += lds->errors[2][t][b]; }
     float const error = fminf(error7, error9);
-    if (!(error < best.error)) return;
+    Bits bits;
+    if (!(error < error1)) {
+        V3 const q0 = quantize(V3{ lds->one[0][b], lds->one[1][b], lds->one[2][b] }, 1024.f), q1 = quantize(V3{ lds->one[3][b], lds->one[4][b], lds->one[5][b] }, 1024.f);
+        bits.put(0, 0x03, 5);
+        bits.put(5, uint32_t(q0.x), 10); bits.put(15, uint32_t(q0.y), 10); bits.put(25, uint32_t(q0.z), 10);
+        bits.put(35, uint32_t(q1.x), 10); bits.put(45, uint32_t(q1.y), 10); bits.put(55, uint32_t(q1.z), 10);
+        uint64_t const indices = uint64_t(lds->indices[0][0][b]) | uint64_t(lds->indices[0][1][b]) << 16 | uint64_t(lds->indices[0][2][b]) << 32 | uint64_t(lds->indices[0][3][b]) << 48;
+        // texel 0 has three bits from bit 65 on, the others four each
+        outLo = bits.lo;
+        outHi = bits.hi | (indices & 7u) << 1 | (indices & ~uint64_t(15));
+        return;
+    }
+    int const pattern = picked_pattern(lds, b), anchor1 = kSecondAnchor[pattern];
     bool const sevenSix = error == error7;
+    V3 q[4];
+    base_and_deltas(lds, b, sevenSix ? 128.f : 512.f, sevenSix ? 31.f : 15.f, q);
     int const baseBits = sevenSix ? 7 : 9, deltaBits = sevenSix ? 6 : 5;
-    V3 const w = sevenSix ? q7[0] : q9[0], x = sevenSix ? q7[1] : q9[1], y = sevenSix ? q7[2] : q9[2], z = sevenSix ? q7[3] : q9[3];
+    V3 const w = q[0], x = q[1], y = q[2], z = q[3];
     uint32_t const rw = field(w.x, baseBits), gw = field(w.y, baseBits), bw = field(w.z, baseBits);
     uint32_t const rx = field(x.x, deltaBits), gx = field(x.y, deltaBits), bx = field(x.z, deltaBits);
     uint32_t const ry = field(y.x, deltaBits), gy = field(y.y, deltaBits), by = field(y.z, deltaBits);
     uint32_t const rz = field(z.x, deltaBits), gz = field(z.y, deltaBits), bz = field(z.z, deltaBits);
-    Bits b;
     if (sevenSix) {         // mode 2 of the format: 7.666
-        b.put(0, 0x01, 2);
-        b.put(2, gy >> 5, 1); b.put(3, gz >> 4, 1); b.put(4, gz >> 5, 1);
-        b.put(5, rw, 7); b.put(12, bz, 1); b.put(13, bz >> 1, 1); b.put(14, by >> 4, 1);
-        b.put(15, gw, 7); b.put(22, by >> 5, 1); b.put(23, bz >> 2, 1); b.put(24, gy >> 4, 1);
-        b.put(25, bw, 7); b.put(32, bz >> 3, 1); b.put(33, bz >> 5, 1); b.put(34, bz >> 4, 1);
-        b.put(35, rx, 6); b.put(41, gy, 4); b.put(45, gx, 6); b.put(51, gz, 4); b.put(55, bx, 6); b.put(61, by, 4);
-        b.put(65, ry, 6); b.put(71, rz, 6);
+        bits.put(0, 0x01, 2);
+        bits.put(2, gy >> 5, 1); bits.put(3, gz >> 4, 1); bits.put(4, gz >> 5, 1);
+        bits.put(5, rw, 7); bits.put(12, bz, 1); bits.put(13, bz >> 1, 1); bits.put(14, by >> 4, 1);
+        bits.put(15, gw, 7); bits.put(22, by >> 5, 1); bits.put(23, bz >> 2, 1); bits.put(24, gy >> 4, 1);
+        bits.put(25, bw, 7); bits.put(32, bz >> 3, 1); bits.put(33, bz >> 5, 1); bits.put(34, bz >> 4, 1);
+        bits.put(35, rx, 6); bits.put(41, gy, 4); bits.put(45, gx, 6); bits.put(51, gz, 4); bits.put(55, bx, 6); bits.put(61, by, 4);
+        bits.put(65, ry, 6); bits.put(71, rz, 6);
     } else {                // mode 6 of the format: 9.555
-        b.put(0, 0x0E, 5);
-        b.put(5, rw, 9); b.put(14, by >> 4, 1); b.put(15, gw, 9); b.put(24, gy >> 4, 1); b.put(25, bw, 9); b.put(34, bz >> 4, 1);
-        b.put(35, rx, 5); b.put(40, gz >> 4, 1); b.put(41, gy, 4); b.put(45, gx, 5); b.put(50, bz, 1); b.put(51, gz, 4);
-        b.put(55, bx, 5); b.put(60, bz >> 1, 1); b.put(61, by, 4); b.put(65, ry, 5); b.put(70, bz >> 2, 1); b.put(71, rz, 5); b.put(76, bz >> 3, 1);
+        bits.put(0, 0x0E, 5);
+        bits.put(5, rw, 9); bits.put(14, by >> 4, 1); bits.put(15, gw, 9); bits.put(24, gy >> 4, 1); bits.put(25, bw, 9); bits.put(34, bz >> 4, 1);
+        bits.put(35, rx, 5); bits.put(40, gz >> 4, 1); bits.put(41, gy, 4); bits.put(45, gx, 5); bits.put(50, bz, 1); bits.put(51, gz, 4);
+        bits.put(55, bx, 5); bits.put(60, bz >> 1, 1); bits.put(61, by, 4); bits.put(65, ry, 5); bits.put(70, bz >> 2, 1); bits.put(71, rz, 5); bits.put(76, bz >> 3, 1);
     }
-    b.put(77, uint32_t(pattern), 5);
-    int at = 82;
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-        int const n = (t == 0 || t == anchor1) ? 2 : 3;
-        uint64_t const v = index[t] & ((1u << n) - 1u);
-        b.hi |= v << (at - 64);
-        at += n;
-    }
-    best = Block{ b.lo, b.hi, error };
+    bits.put(77, uint32_t(pattern), 5);
+    // three bits per texel from bit 82 on, the anchors' (texel 0 and anchor1) without the top one, which is zero
+    uint64_t indices = uint64_t(lds->indices[1][0][b]) | uint64_t(lds->indices[1][1][b]) << 12 | uint64_t(lds->indices[1][2][b]) << 24 | uint64_t(lds->indices[1][3][b]) << 36;
+    uint64_t const below = (uint64_t(1) << (3 * anchor1 + 2)) - 1u;
+    indices = (indices & below) | ((indices >> 1) & ~below);
+    indices = (indices & 3u) | ((indices >> 1) & ~uint64_t(3));
+    outLo = bits.lo;
+    outHi = bits.hi | indices << 18;
 }
 
 } // namespace
 
-// Registers capped at 168 so that three waves share a SIMD: the encoder is long chains of dependent divisions
-// and logarithms, and the other waves fill the issue slots one leaves (4096^2: 1.77 ms with one wave and 256
-// registers, 1.05 ms with two, 0.98 ms with three in spite of 175 spilled registers, 1.02 ms with four).
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(3)))
+template <bool WIDE>
+__global__ void __launch_bounds__(256, 4)
 bc6_compress_kernel(BlockCompressArgs a)
 {
-    int const bx = blockIdx.x * 16 + (threadIdx.x & 15), by = blockIdx.y * 8 + (threadIdx.x >> 4);
-    if (bx >= a.widthInBlocks || by >= a.heightInBlocks) return;
-    V3 px[16];
+    __shared__ Bc6Lds shared;
+    Bc6Ptr const lds = (Bc6Ptr)&shared;
+    int const tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int const bx = blockIdx.x * 8 + (lane & 7), by = blockIdx.y * 8 + (lane >> 3);
+    bool const inside = bx < a.widthInBlocks && by < a.heightInBlocks;
+    // a row of the block per wave; lanes outside encode black
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-        int const x = a.srcLeft + bx * 4 + (t & 3), y = a.srcTop + by * 4 + (t >> 2);
-        float c[4];
-        source_pixel(a, x, y, c);
-        px[t] = V3{ clampf(c[0], 0.f, kHalfMax), clampf(c[1], 0.f, kHalfMax), clampf(c[2], 0.f, kHalfMax) };
+    for (int i = 0; i < 4; ++i) {
+        float c[4] = { 0.f, 0.f, 0.f, 0.f };
+        if (inside) source_pixel(a, a.srcLeft + bx * 4 + i, a.srcTop + by * 4 + wave, c);
+        shared.texels[4 * wave + i][lane] = make_float4(clampf(c[0], 0.f, kHalfMax), clampf(c[1], 0.f, kHalfMax), clampf(c[2], 0.f, kHalfMax), 0.f);
     }
-    Block best = encode_one_subset(px);
-    float bestScore = pattern_score(px, kSecondSubset[0]);
-    int bestPattern = 0;
-#pragma unroll 1
-    for (int p = 1; p < 32; ++p) {
-        float const score = pattern_score(px, kSecondSubset[p]);
-        if (score < bestScore) { bestPattern = p; bestScore = score; }
-    }
-    encode_two_subsets(px, bestPattern, best);
+    if (wave == 0) { shared.pick[lane] = ~uint64_t(0); if (lane == 0) shared.next = 0; }
+    __syncthreads();
+    if (wave == 0) one_subset_ends<WIDE>(lds, lane);
+    score_patterns<WIDE>(lds, lane);
+    __syncthreads();
+    if (wave < 2) subset_ends<WIDE>(lds, lane, wave);
+    __syncthreads();
+    texel_errors<WIDE>(lds, lane, wave);
+    __syncthreads();
+    if (wave != 0 || !inside) return;
+    uint64_t lo, hi;
+    final_block(lds, lane, lo, hi);
     uint64_t* const dst = reinterpret_cast<uint64_t*>(a.dst + size_t(by + a.dstOffsetY) * a.dstRowPitch) + size_t(bx + a.dstOffsetX) * 2;
-    dst[0] = best.lo; dst[1] = best.hi;
+    dst[0] = lo; dst[1] = hi;
 }
 
 hipError_t launch_bc6_compress(BlockCompressArgs const& a, hipStream_t stream)
 {
-    dim3 const grid((a.widthInBlocks + 15) / 16, (a.heightInBlocks + 7) / 8);
-    hipLaunchKernelGGL(bc6_compress_kernel, grid, dim3(128), 0, stream, a);
+    dim3 const grid((a.widthInBlocks + 7) / 8, (a.heightInBlocks + 7) / 8);
+    if (a.format == NTC_HIP_DEV_FORMAT_FLOAT32) hipLaunchKernelGGL(bc6_compress_kernel<true>, grid, dim3(256), 0, stream, a);
+    else                                        hipLaunchKernelGGL(bc6_compress_kernel<false>, grid, dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 

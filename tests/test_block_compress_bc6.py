@@ -212,3 +212,29 @@ def test_gpu_bc6_matches_checker(ntc, device, oracle, fmt):
         got = compress(ntc, None, device, image, fmt, 3, 6, bx, by, left, top, off_x, off_y, pitch)
         bad = np.argwhere(got != want)
         assert bad.size == 0, (fmt, len(bad), bad[:3], [hex(int(got[tuple(b)])) for b in bad[:3]], [hex(int(want[tuple(b)])) for b in bad[:3]])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("blocks_x,blocks_y", [(1, 1), (8, 8), (9, 17)])
+def test_gpu_bc6_over_each_formats_range(ntc, device, oracle, fmt, blocks_x, blocks_y):
+    """One block, a full workgroup of blocks and remainders in both directions; texels over all magnitudes, up to those
+    whose endpoints decode to infinity, with few different values per block (ties, flat subsets) in half of the blocks."""
+    rng = np.random.default_rng(660 + fmt)
+    h, w = 4 * blocks_y, 4 * blocks_x
+    if fmt in (3, 4):
+        image = rng.integers(0, 0x7C00, (h, w, 3)).astype(np.uint16).view(np.float16)
+        near_top = rng.random((blocks_y, blocks_x)).repeat(4, 0).repeat(4, 1) < 0.3
+        image[near_top] = rng.integers(0x7B80, 0x7C00, (int(near_top.sum()), 3)).astype(np.uint16).view(np.float16)
+        if fmt == 4:
+            image = image.astype(np.float32) * rng.uniform(0.9, 1.1, image.shape).astype(np.float32)
+    else:
+        dtype, top = {1: (np.uint8, 8), 2: (np.uint16, 16), 5: (np.uint32, 17)}[fmt]
+        image = np.minimum(np.exp2(rng.uniform(0, top, (h, w, 3))), 2.0 ** min(top, 16) - 1).astype(dtype)
+    few = (rng.random((blocks_y, blocks_x)) < 0.5).repeat(4, 0).repeat(4, 1)
+    image[few] = image[::4, ::4].repeat(4, 0).repeat(4, 1)[few]
+    image[1::4, 2::4] = image[0, 0]
+    want = compress(ntc, oracle, None, image, fmt, 3, 6, blocks_x, blocks_y)
+    got = compress(ntc, None, device, image, fmt, 3, 6, blocks_x, blocks_y)
+    bad = np.argwhere(got != want)
+    assert bad.size == 0, (fmt, len(bad), bad[:3], [hex(int(got[tuple(b)])) for b in bad[:3]], [hex(int(want[tuple(b)])) for b in bad[:3]])
