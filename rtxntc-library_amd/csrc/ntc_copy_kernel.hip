@@ -10,6 +10,7 @@
 #include <atomic>
 #include <type_traits>
 #include "ntc_decode_kernel.h"
+#include "ntc_launch.h"
 
 namespace ntc_hip_dev {
 
@@ -335,8 +336,8 @@ typedef uint32_t u32x2_a4  __attribute__((ext_vector_type(2), aligned(4)));
 typedef uint32_t u32x4_a4  __attribute__((ext_vector_type(4), aligned(4)));
 
 // Which pixels a lane works on: tiles of lanesX groups by threads / lanesX rows, a workgroup takes tiles
-// blockIdx.x, blockIdx.x + gridDim.x, ...
-struct GroupGrid { int32_t log2LanesX, tilesX, tiles; };
+// blockIdx.x, blockIdx.x + step, ...
+struct GroupGrid { int32_t tilesX, tiles, step; uint8_t log2LanesX, log2Rows; };
 
 int compute_units_of_current_device()
 {
@@ -355,16 +356,18 @@ static GroupGrid group_grid(int width, int height, int threads)
 {
     GroupGrid g;
     int const groups = (width + 3) / 4;
-    g.log2LanesX = groups > 32 ? 6 : groups > 16 ? 5 : groups > 8 ? 4 : 3;
+    g.log2LanesX = uint8_t(groups > 32 ? 6 : groups > 16 ? 5 : groups > 8 ? 4 : 3);
     int const rows = threads >> g.log2LanesX;
+    g.log2Rows = uint8_t(__builtin_ctz(unsigned(rows)));
     g.tilesX = (groups + (1 << g.log2LanesX) - 1) >> g.log2LanesX;
     g.tiles = g.tilesX * ((height + rows - 1) / rows);
+    g.step = g.tiles;
     return g;
 }
 
 // The tables that a launch copies into LDS: the first two pairs of colour spaces that its channels use.
 struct StagedTransfers {
-    int32_t count;                                           // 0: nothing staged
+    int8_t count;                                            // 0: nothing staged
     int8_t staged[2];                                        // the pairs
     int8_t pair[8], slot[8];                                 // per channel: its pair (-1 linear) and the copy that holds it (0 none)
 };
@@ -376,7 +379,7 @@ struct StagedTransfers {
 struct GroupLaunch {
     GroupGrid grid;
     StagedTransfers transfers;
-    unsigned blocks, threads, ldsBytes;
+    unsigned threads, ldsBytes;
 };
 
 static GroupLaunch plan_groups(int width, int height, uint8_t const* src, uint8_t const* dst, int channels, bool readsHalves)
@@ -396,49 +399,60 @@ static GroupLaunch plan_groups(int width, int height, uint8_t const* src, uint8_
     if (s.count) {
         int const share = (l.grid.tiles + kTilesPerStaging - 1) / kTilesPerStaging;
         l.threads = kStagingThreads;
-        l.blocks = unsigned(2 * units < share ? 2 * units : share);
+        l.grid.step = 2 * units < share ? 2 * units : share;
         l.ldsBytes = unsigned(s.count * kStageCount * sizeof(float));
     } else {
         l.grid = group_grid(width, height, kSmallThreads);
         l.threads = kSmallThreads;
-        l.blocks = unsigned(l.grid.tiles);
     }
     return l;
 }
 
-__device__ __forceinline__ void copy_staged(StagedTransfers const& s, float* lds)
+__device__ __forceinline__ void copy_staged(StagedTransfers const& s, float* lds, uint32_t threads)
 {
     for (int k = 0; k < s.count; ++k) {
         float const* const from = &transferOfHalf[s.staged[k]][kStageFirst];
-        for (uint32_t i = threadIdx.x; i < kStageCount; i += blockDim.x) lds[k * int(kStageCount) + int(i)] = from[i];
+        for (uint32_t i = threadIdx.x; i < kStageCount; i += threads) lds[k * int(kStageCount) + int(i)] = from[i];
     }
     if (s.count) __syncthreads();
 }
 
-struct ReadGroupsArgs { ReadChannelsArgs a; GroupGrid grid; StagedTransfers transfers; };
+// What the kernels need of a ReadChannelsArgs or WriteChannelsArgs, in as few bytes as launches are quick with.
+struct GroupsArgs {
+    uint16_t* planar;
+    uint8_t* image;
+    uint64_t rowPitch;
+    int32_t width, height;
+    GroupGrid grid;
+    StagedTransfers transfers;
+    uint8_t setChannels, firstChannel, channels;             // channels: copied ones
+    uint8_t fillSpace;                                       // read: the destination's colour space of a fourth channel the set does not have
+    uint8_t verticalFlip;                                    // write
+};
+static_assert(sizeof(GroupsArgs) <= 128, "");
 
 // CHANNELS = channels of a destination pixel.
 template <int FORMAT, int CHANNELS, bool DITHER>
 __global__ void __launch_bounds__(1024, 8)
-read_groups_kernel(ReadGroupsArgs args)
+read_groups_kernel(GroupsArgs a)
 {
     constexpr int BPC = bytes_per_channel(FORMAT), PIXEL = CHANNELS * BPC, PAIRS = CHANNELS / 2 + 1;
     static_assert(PIXEL <= 8, "the words of four pixels stay in registers");
     extern __shared__ float staged[];
-    ReadChannelsArgs const& a = args.a;
-    copy_staged(args.transfers, staged);
-    int const lanesX = 1 << args.grid.log2LanesX;
-    int const lx = int(threadIdx.x) & (lanesX - 1), ly = int(threadIdx.x) >> args.grid.log2LanesX;
+    uint32_t const threads = 1u << (a.grid.log2LanesX + a.grid.log2Rows);
+    copy_staged(a.transfers, staged, threads);
+    int const lanesX = 1 << a.grid.log2LanesX;
+    int const lx = int(threadIdx.x) & (lanesX - 1), ly = int(threadIdx.x) >> a.grid.log2LanesX;
     int const firstPair = a.firstChannel >> 1;
     bool const odd = (a.firstChannel & 1) != 0;
-    int const copied = min(a.numChannels, CHANNELS);
+    int const copied = min(int(a.channels), CHANNELS);
     int const pairs = ((a.firstChannel + copied + 1) >> 1) - firstPair;      // at most PAIRS
-    for (int tile = blockIdx.x; tile < args.grid.tiles; tile += gridDim.x) {
-        int const tileY = tile / args.grid.tilesX, tileX = tile - tileY * args.grid.tilesX;
-        int const x = (tileX * lanesX + lx) * 4, y = tileY * int(blockDim.x >> args.grid.log2LanesX) + ly;
+    for (int tile = blockIdx.x; tile < a.grid.tiles; tile += a.grid.step) {
+        int const tileY = tile / a.grid.tilesX, tileX = tile - tileY * a.grid.tilesX;
+        int const x = (tileX * lanesX + lx) * 4, y = (tileY << a.grid.log2Rows) + ly;
         if (x >= a.width || y >= a.height) continue;
         bool const whole = x + 4 <= a.width;
-        uint16_t const* const src = a.planarPairs + size_t(y) * size_t(a.width) * size_t(a.setChannels) + size_t(x) * 2;
+        uint16_t const* const src = a.planar + size_t(y) * size_t(a.width) * size_t(a.setChannels) + size_t(x) * 2;
         uint32_t pr[PAIRS][4];
 #pragma unroll
         for (int p = 0; p < PAIRS; ++p) {
@@ -455,14 +469,16 @@ read_groups_kernel(ReadGroupsArgs args)
 #pragma unroll
         for (int w = 0; w < PIXEL; ++w) words[w] = 0u;
         uint32_t const index = uint32_t(x) + uint32_t(y) * uint32_t(a.width);
-[[maybe_unused]] DitherRng rng[4];                   // one draw per pixel and destination channel, in channel order
+        [[maybe_unused]] DitherRng rng[4];                   // one draw per pixel and destination channel, in channel order
         if constexpr (DITHER) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) rng[k] = DitherRng(index + uint32_t(k));
         }
+        // (all look-ups before the first use of one: small images wait for their latency)
+        float values[CHANNELS][4];
 #pragma unroll
         for (int ch = 0; ch < CHANNELS; ++ch) {
-            float value[4];
+            float (&value)[4] = values[ch];
             if (ch < copied) {                               // uniform
                 uint32_t bits[4];
 #pragma unroll
@@ -471,23 +487,26 @@ read_groups_kernel(ReadGroupsArgs args)
                     uint32_t const next = (ch & 1) ? pr[(ch >> 1) + 1][k] & 0xffffu : pr[ch >> 1][k] >> 16;
                     bits[k] = odd ? next : even;
                 }
-                transfer_halves(staged, args.transfers.slot[ch], args.transfers.pair[ch], bits, value);
+                transfer_halves(staged, a.transfers.slot[ch], a.transfers.pair[ch], bits, value);
             } else {                                         // GetDefaultChannelValue; 0 is 0 in every colour space
-                float const fill = (ch == 3) ? encode_color_space(a.dstColorSpaces[ch], 1.f) : 0.f;
+                float const fill = (ch == 3) ? encode_color_space(a.fillSpace, 1.f) : 0.f;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) value[k] = fill;
             }
+        }
+#pragma unroll
+        for (int ch = 0; ch < CHANNELS; ++ch) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 float const dither = DITHER ? rng[k].next_float() - 0.5f : 0.f;
-                uint32_t const bits = encode_value<FORMAT>(value[k], DITHER, dither);
+                uint32_t const bits = encode_value<FORMAT>(values[ch][k], DITHER, dither);
                 int const at = k * PIXEL + ch * BPC;         // byte of the group
                 words[at >> 2] |= BPC == 4 ? bits : bits << (8 * (at & 3));
             }
         }
-        uint8_t* const out = a.dst + size_t(y) * a.rowPitch + size_t(x) * PIXEL;
+        uint8_t* const out = a.image + size_t(y) * a.rowPitch + size_t(x) * PIXEL;
         if (whole) {
-constexpr int FOURS = PIXEL & ~3, TWOS = FOURS + (PIXEL & 2);
+            constexpr int FOURS = PIXEL & ~3, TWOS = FOURS + (PIXEL & 2);
 #pragma unroll
             for (int w = 0; w < FOURS; w += 4)
                 *reinterpret_cast<u32x4_any*>(out + 4 * w) = u32x4_any{ words[w], words[w + 1], words[w + 2], words[w + 3] };
@@ -520,11 +539,10 @@ __device__ __forceinline__ float decode_channel(uint32_t const (&words)[4], int 
 }
 
 // The half of the internal layout that a channel of the user image becomes: its bits (upper bits are ignored by the
-// narrow formats) through both colour spaces (uniform).
+// narrow formats) through the pair of colour spaces (uniform).
 template <int FORMAT>
-__device__ __forceinline__ uint32_t stored_half_of(uint32_t bits, int srcSpace, int dstSpace)
+__device__ __forceinline__ uint32_t stored_half_of(uint32_t bits, int pair)
 {
-    int const pair = transfer_pair(srcSpace, dstSpace);
     if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_UNORM8) {
         return storedOfUnorm8[pair < 0 ? kTransferPairs : pair][bits & 0xffu];
     } else if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_UNORM16) {
@@ -533,11 +551,9 @@ __device__ __forceinline__ uint32_t stored_half_of(uint32_t bits, int srcSpace, 
         return stored_half(transfer_half(pair, bits & 0xffffu));
     } else {
         float const v = FORMAT == NTC_HIP_DEV_FORMAT_FLOAT32 ? __builtin_bit_cast(float, bits) : float(bits);
-        return stored_half(pair < 0 ? v : encode_color_space(dstSpace, decode_color_space(srcSpace, v)));
+        return stored_half(pair < 0 ? v : encode_color_space((pair + 1) % 3, decode_color_space((pair + 1) / 3, v)));
     }
 }
-
-struct WriteGroupsArgs { WriteChannelsArgs a; GroupGrid grid; StagedTransfers transfers; };
 
 // Four pixels of at most eight bytes a lane, like read_groups_kernel the other way round: whole dwords of the pixels
 // in, 16 bytes of each complete channel pair out (2048 x 2048 of 8 bits: RGBA with sRGB 14 us, 91 before the tables; two
@@ -546,31 +562,31 @@ struct WriteGroupsArgs { WriteChannelsArgs a; GroupGrid grid; StagedTransfers tr
 // 8-bit codes become halves through a table in LDS, a row of 256 per channel.
 template <int FORMAT, int CHANNELS>
 __global__ void __launch_bounds__(1024, 8)
-write_groups_kernel(WriteGroupsArgs args)
+write_groups_kernel(GroupsArgs a)
 {
     constexpr int BPC = bytes_per_channel(FORMAT), PIXEL = CHANNELS * BPC, PAIRS = CHANNELS / 2 + 1;
     constexpr bool CODES = FORMAT == NTC_HIP_DEV_FORMAT_UNORM8, HALVES = FORMAT == NTC_HIP_DEV_FORMAT_FLOAT16;
     static_assert(PIXEL <= 8, "the words of four pixels stay in registers");
     __shared__ uint16_t codes[CODES ? CHANNELS : 1][256];
     extern __shared__ float staged[];
-    WriteChannelsArgs const& a = args.a;
+    uint32_t const threads = 1u << (a.grid.log2LanesX + a.grid.log2Rows);
     if constexpr (CODES) {
-        for (int i = threadIdx.x; i < CHANNELS * 256; i += blockDim.x) {
-            int const ch = i >> 8, pair = transfer_pair(a.srcColorSpaces[ch], a.dstColorSpaces[ch]);
+        for (uint32_t i = threadIdx.x; i < CHANNELS * 256u; i += threads) {
+            int const ch = int(i >> 8), pair = a.transfers.pair[ch];
             codes[ch][i & 255] = storedOfUnorm8[pair < 0 ? kTransferPairs : pair][i & 255];
         }
         __syncthreads();
     }
-    if constexpr (HALVES) copy_staged(args.transfers, staged);
-    int const lanesX = 1 << args.grid.log2LanesX;
-    int const lx = int(threadIdx.x) & (lanesX - 1), ly = int(threadIdx.x) >> args.grid.log2LanesX;
+    if constexpr (HALVES) copy_staged(a.transfers, staged, threads);
+    int const lanesX = 1 << a.grid.log2LanesX;
+    int const lx = int(threadIdx.x) & (lanesX - 1), ly = int(threadIdx.x) >> a.grid.log2LanesX;
     int const odd = a.firstChannel & 1;
-    for (int tile = blockIdx.x; tile < args.grid.tiles; tile += gridDim.x) {
-        int const tileY = tile / args.grid.tilesX, tileX = tile - tileY * args.grid.tilesX;
-        int const x = (tileX * lanesX + lx) * 4, y = tileY * int(blockDim.x >> args.grid.log2LanesX) + ly;
+    for (int tile = blockIdx.x; tile < a.grid.tiles; tile += a.grid.step) {
+        int const tileY = tile / a.grid.tilesX, tileX = tile - tileY * a.grid.tilesX;
+        int const x = (tileX * lanesX + lx) * 4, y = (tileY << a.grid.log2Rows) + ly;
         if (y >= a.height) continue;                         // (uniform across a wave that covers one row)
         bool const whole = x + 4 <= a.width;
-        uint8_t const* const in = a.src + size_t(a.verticalFlip ? a.height - 1 - y : y) * a.rowPitch + size_t(x) * PIXEL;
+        uint8_t const* const in = a.image + size_t(a.verticalFlip ? a.height - 1 - y : y) * a.rowPitch + size_t(x) * PIXEL;
         uint32_t words[PIXEL];
         if (whole) {
             constexpr int FOURS = PIXEL & ~3, TWOS = FOURS + (PIXEL & 2);
@@ -611,21 +627,21 @@ write_groups_kernel(WriteGroupsArgs args)
                 for (int k = 0; k < 4; ++k) half[ch][k] = codes[ch][bits[k]];
             } else if constexpr (HALVES) {
                 float value[4];
-                transfer_halves(staged, args.transfers.slot[ch], args.transfers.pair[ch], bits, value);
+                transfer_halves(staged, a.transfers.slot[ch], a.transfers.pair[ch], bits, value);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) half[ch][k] = stored_half(value[k]);
             } else {
 #pragma unroll
-                for (int k = 0; k < 4; ++k) half[ch][k] = stored_half_of<FORMAT>(bits[k], a.srcColorSpaces[ch], a.dstColorSpaces[ch]);
+                for (int k = 0; k < 4; ++k) half[ch][k] = stored_half_of<FORMAT>(bits[k], a.transfers.pair[ch]);
             }
         }
-        uint16_t* const dst = a.planarPairs + size_t(y) * size_t(a.width) * size_t(a.setChannels) + size_t(x) * 2;
+        uint16_t* const dst = a.planar + size_t(y) * size_t(a.width) * size_t(a.setChannels) + size_t(x) * 2;
 #pragma unroll
         for (int p = 0; p < PAIRS; ++p) {
             int const lower = 2 * p - odd;                   // the image's channel in the pair's first half, lower + 1 in its second
-            if (lower >= a.numChannels) continue;            // uniform, and so is everything about p
+            if (lower >= int(a.channels)) continue;          // uniform, and so is everything about p
             uint16_t* const to = dst + size_t((a.firstChannel & ~1) + 2 * p) * size_t(a.width);
-            bool const hasLower = lower >= 0, hasUpper = lower + 1 < a.numChannels;
+            bool const hasLower = lower >= 0, hasUpper = lower + 1 < int(a.channels);
             uint32_t pair[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
@@ -640,7 +656,7 @@ write_groups_kernel(WriteGroupsArgs args)
 #pragma unroll
                     for (int k = 0; k < 4; ++k) if (x + k < a.width) *reinterpret_cast<uint32_t*>(to + 2 * k) = pair[k];
                 }
-            } else if (args.grid.log2LanesX == 6) {
+            } else if (a.grid.log2LanesX == 6) {
                 // One half of a pair, a wave per row: the wave's 256 halves are dealt out anew, 64 neighbours to a
                 // store, so that a store touches 256 bytes and not 1 KB (one channel 12 -> 10 us, two
                 // 19 -> 13 us).  Lane i's pixel of store s is element i % 4
@@ -711,7 +727,7 @@ write_channels_kernel(WriteChannelsArgs a)
             if (ch >= a.numChannels) continue;                       // uniform
             uint32_t half;
             if constexpr (PLAIN) half = stored_half(decode_channel<FORMAT>(words, k, unorm8Table));
-            else                 half = stored_half_of<FORMAT>(words[(k * BPC) >> 2] >> (8 * ((k * BPC) & 3)), a.srcColorSpaces[ch], a.dstColorSpaces[ch]);
+            else                 half = stored_half_of<FORMAT>(words[(k * BPC) >> 2] >> (8 * ((k * BPC) & 3)), transfer_pair(a.srcColorSpaces[ch], a.dstColorSpaces[ch]));
             int const c = a.firstChannel + ch;
             uint16_t* const to = dst + size_t(c & ~1) * size_t(a.width);
             if ((c & 1) == 0) {
@@ -841,7 +857,8 @@ write_channels_resize_kernel(WriteChannelsArgs a)
 struct ResizePlanarArgs {
     uint16_t const* src; uint16_t* dst;
     int32_t srcWidth, srcHeight, dstWidth, dstHeight, setChannels;
-    int32_t tilesX, tiles, pairsPerLane;                     // tiles of 64 x blockDim.x / 64 pixels
+    int32_t tilesX, tiles, pairsPerLane;                     // tiles of 64 pixels x a row per wave
+    int32_t step, threads;                                   // workgroups in x, threads of each
     StagedTransfers transfers;                               // of the decoding pairs; pair / slot: per colour space
     uint8_t colorSpaces[16];
 };
@@ -851,12 +868,12 @@ __global__ void __launch_bounds__(1024, 8)
 resize_planar_kernel(ResizePlanarArgs a)
 {
     extern __shared__ float staged[];
-    if constexpr (!LINEAR) copy_staged(a.transfers, staged);
+    if constexpr (!LINEAR) copy_staged(a.transfers, staged, uint32_t(a.threads));
     int const pairBegin = int(blockIdx.y) * a.pairsPerLane, pairEnd = min(a.setChannels >> 1, pairBegin + a.pairsPerLane);
     size_t const srcRow = size_t(a.srcWidth) * size_t(a.setChannels), pairStride = size_t(a.srcWidth) * 2;
-    for (int tile = blockIdx.x; tile < a.tiles; tile += gridDim.x) {
+    for (int tile = blockIdx.x; tile < a.tiles; tile += a.step) {
         int const tileY = tile / a.tilesX, tileX = tile - tileY * a.tilesX;
-        int const x = tileX * 64 + int(threadIdx.x & 63), y = tileY * int(blockDim.x >> 6) + int(threadIdx.x >> 6);
+        int const x = tileX * 64 + int(threadIdx.x & 63), y = tileY * (a.threads >> 6) + int(threadIdx.x >> 6);
         if (x >= a.dstWidth || y >= a.dstHeight) continue;
         BilinearTaps const t = setup_bilinear(a.srcWidth, a.srcHeight, a.dstWidth, a.dstHeight, x, y);
         int const left = max(0, min(t.x0, a.srcWidth - 2));  // columns left and left + 1 hold both taps
@@ -944,9 +961,10 @@ hipError_t launch_resize_planar(uint16_t const* src, int srcWidth, int srcHeight
         grid = dim3(unsigned(a.tiles), unsigned((pairs + a.pairsPerLane - 1) / a.pairsPerLane));
     }
     size_t const lds = size_t(a.transfers.count) * kStageCount * sizeof(float);
-    if (linear) hipLaunchKernelGGL(resize_planar_kernel<true>, grid, dim3(threads), lds, stream, a);
-    else        hipLaunchKernelGGL(resize_planar_kernel<false>, grid, dim3(threads), lds, stream, a);
-    return hipGetLastError();
+    a.step = int(grid.x);
+    a.threads = threads;
+    return linear ? launch_kernel<resize_planar_kernel<true>>(grid, dim3(threads), lds, stream, a)
+                  : launch_kernel<resize_planar_kernel<false>>(grid, dim3(threads), lds, stream, a);
 }
 
 static bool plain_copy(uint8_t const* srcSpaces, uint8_t const* dstSpaces, int useDithering)
@@ -957,74 +975,72 @@ static bool plain_copy(uint8_t const* srcSpaces, uint8_t const* dstSpaces, int u
 }
 
 template <int FORMAT>
-static hipError_t launch_write_groups_of(WriteGroupsArgs const& args, GroupLaunch const& plan, hipStream_t stream)
+static hipError_t launch_write_groups_of(GroupsArgs const& args, int srcChannels, GroupLaunch const& plan, hipStream_t stream)
 {
-    auto launch = [&](auto channels) {
+    auto launch = [&](auto channels) -> hipError_t {
         constexpr int CHANNELS = decltype(channels)::value;
         if constexpr (CHANNELS * bytes_per_channel(FORMAT) <= 8)
-            hipLaunchKernelGGL((write_groups_kernel<FORMAT, CHANNELS>), dim3(plan.blocks), dim3(plan.threads), plan.ldsBytes, stream, args);
+            return launch_kernel<write_groups_kernel<FORMAT, CHANNELS>>(dim3(plan.grid.step), dim3(plan.threads), plan.ldsBytes, stream, args);
+        else
+            return hipErrorInvalidValue;
     };
-    switch (int(args.a.pixelStride) / bytes_per_channel(FORMAT)) {
-    case 1: launch(std::integral_constant<int, 1>{}); break;
-    case 2: launch(std::integral_constant<int, 2>{}); break;
-    case 3: launch(std::integral_constant<int, 3>{}); break;
-    case 4: launch(std::integral_constant<int, 4>{}); break;
-    case 5: launch(std::integral_constant<int, 5>{}); break;
-    case 6: launch(std::integral_constant<int, 6>{}); break;
-    case 7: launch(std::integral_constant<int, 7>{}); break;
-    case 8: launch(std::integral_constant<int, 8>{}); break;
+    switch (srcChannels) {
+    case 1: return launch(std::integral_constant<int, 1>{});
+    case 2: return launch(std::integral_constant<int, 2>{});
+    case 3: return launch(std::integral_constant<int, 3>{});
+    case 4: return launch(std::integral_constant<int, 4>{});
+    case 5: return launch(std::integral_constant<int, 5>{});
+    case 6: return launch(std::integral_constant<int, 6>{});
+    case 7: return launch(std::integral_constant<int, 7>{});
+    case 8: return launch(std::integral_constant<int, 8>{});
     default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 static hipError_t launch_write_groups(WriteChannelsArgs const& a, hipStream_t stream)
 {
-    WriteGroupsArgs args{};
-    args.a = a;
     GroupLaunch plan = plan_groups(a.width, a.height, a.srcColorSpaces, a.dstColorSpaces, a.numChannels, a.format == NTC_HIP_DEV_FORMAT_FLOAT16);
     if (a.format == NTC_HIP_DEV_FORMAT_UNORM8) {             // a workgroup fills its table once for all of its tiles
-        unsigned const resident = 8u * unsigned(compute_units_of_current_device());
-        if (plan.blocks > resident) plan.blocks = resident;
+        int const resident = 8 * compute_units_of_current_device();
+        if (plan.grid.step > resident) plan.grid.step = resident;
     }
-    args.grid = plan.grid;
-    args.transfers = plan.transfers;
+    GroupsArgs const args{ a.planarPairs, const_cast<uint8_t*>(a.src), a.rowPitch, a.width, a.height, plan.grid, plan.transfers,
+                           uint8_t(a.setChannels), uint8_t(a.firstChannel), uint8_t(a.numChannels), 0, uint8_t(a.verticalFlip != 0) };
+    int const channels = int(a.pixelStride) / bytes_per_channel(a.format);
     switch (a.format) {
-    case NTC_HIP_DEV_FORMAT_UNORM8:  return launch_write_groups_of<NTC_HIP_DEV_FORMAT_UNORM8>(args, plan, stream);
-    case NTC_HIP_DEV_FORMAT_UNORM16: return launch_write_groups_of<NTC_HIP_DEV_FORMAT_UNORM16>(args, plan, stream);
-    case NTC_HIP_DEV_FORMAT_FLOAT16: return launch_write_groups_of<NTC_HIP_DEV_FORMAT_FLOAT16>(args, plan, stream);
-    case NTC_HIP_DEV_FORMAT_FLOAT32: return launch_write_groups_of<NTC_HIP_DEV_FORMAT_FLOAT32>(args, plan, stream);
-    case NTC_HIP_DEV_FORMAT_UINT32:  return launch_write_groups_of<NTC_HIP_DEV_FORMAT_UINT32>(args, plan, stream);
+    case NTC_HIP_DEV_FORMAT_UNORM8:  return launch_write_groups_of<NTC_HIP_DEV_FORMAT_UNORM8>(args, channels, plan, stream);
+    case NTC_HIP_DEV_FORMAT_UNORM16: return launch_write_groups_of<NTC_HIP_DEV_FORMAT_UNORM16>(args, channels, plan, stream);
+    case NTC_HIP_DEV_FORMAT_FLOAT16: return launch_write_groups_of<NTC_HIP_DEV_FORMAT_FLOAT16>(args, channels, plan, stream);
+    case NTC_HIP_DEV_FORMAT_FLOAT32: return launch_write_groups_of<NTC_HIP_DEV_FORMAT_FLOAT32>(args, channels, plan, stream);
+    case NTC_HIP_DEV_FORMAT_UINT32:  return launch_write_groups_of<NTC_HIP_DEV_FORMAT_UINT32>(args, channels, plan, stream);
     default: return hipErrorInvalidValue;
     }
 }
 
 template <int FORMAT>
-static void launch_write_format(WriteChannelsArgs const& a, dim3 grid, bool plain, hipStream_t stream)
+static hipError_t launch_write_format(WriteChannelsArgs const& a, dim3 grid, bool plain, hipStream_t stream)
 {
-    if (plain) hipLaunchKernelGGL((write_channels_kernel<FORMAT, true>), grid, dim3(256), 0, stream, a);
-    else       hipLaunchKernelGGL((write_channels_kernel<FORMAT, false>), grid, dim3(256), 0, stream, a);
+    return plain ? launch_kernel<write_channels_kernel<FORMAT, true>>(grid, dim3(256), 0, stream, a)
+                 : launch_kernel<write_channels_kernel<FORMAT, false>>(grid, dim3(256), 0, stream, a);
 }
 
 hipError_t launch_write_channels(WriteChannelsArgs const& args, hipStream_t stream)
 {
     WriteChannelsArgs a = args;
     if (a.srcWidth > 0) {                                    // resampling copy
-        hipLaunchKernelGGL(write_channels_resize_kernel, dim3((a.width + 63) / 64, (a.height + 3) / 4), dim3(256), 0, stream, a);
-        return hipGetLastError();
+        return launch_kernel<write_channels_resize_kernel>(dim3((a.width + 63) / 64, (a.height + 3) / 4), dim3(256), 0, stream, a);
     }
     if (a.pixelStride <= 8 && a.wholePixels) return launch_write_groups(a, stream);
     dim3 const grid = copy_grid(a.width, a.height, a.xShift, false);
     bool const plain = plain_copy(a.srcColorSpaces, a.dstColorSpaces, 0);
     switch (a.format) {
-    case NTC_HIP_DEV_FORMAT_UNORM8:  launch_write_format<NTC_HIP_DEV_FORMAT_UNORM8>(a, grid, plain, stream); break;
-    case NTC_HIP_DEV_FORMAT_UNORM16: launch_write_format<NTC_HIP_DEV_FORMAT_UNORM16>(a, grid, plain, stream); break;
-    case NTC_HIP_DEV_FORMAT_FLOAT16: launch_write_format<NTC_HIP_DEV_FORMAT_FLOAT16>(a, grid, plain, stream); break;
-    case NTC_HIP_DEV_FORMAT_FLOAT32: launch_write_format<NTC_HIP_DEV_FORMAT_FLOAT32>(a, grid, plain, stream); break;
-    case NTC_HIP_DEV_FORMAT_UINT32:  launch_write_format<NTC_HIP_DEV_FORMAT_UINT32>(a, grid, plain, stream); break;
+    case NTC_HIP_DEV_FORMAT_UNORM8:  return launch_write_format<NTC_HIP_DEV_FORMAT_UNORM8>(a, grid, plain, stream);
+    case NTC_HIP_DEV_FORMAT_UNORM16: return launch_write_format<NTC_HIP_DEV_FORMAT_UNORM16>(a, grid, plain, stream);
+    case NTC_HIP_DEV_FORMAT_FLOAT16: return launch_write_format<NTC_HIP_DEV_FORMAT_FLOAT16>(a, grid, plain, stream);
+    case NTC_HIP_DEV_FORMAT_FLOAT32: return launch_write_format<NTC_HIP_DEV_FORMAT_FLOAT32>(a, grid, plain, stream);
+    case NTC_HIP_DEV_FORMAT_UINT32:  return launch_write_format<NTC_HIP_DEV_FORMAT_UINT32>(a, grid, plain, stream);
     default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 // Per-channel sum of squared differences between a decoded mip and its reference image, both in the
@@ -1086,7 +1102,7 @@ __device__ __forceinline__ bool arrived_last(uint32_t* counter, uint32_t count, 
 template <int PX, bool MASKED>
 __global__ void __launch_bounds__(256)
 image_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int width, int height, int setChannels, int rowsPerWave,
-                  uint32_t validChannelMask, int maskChannel, int discardMaskedOut, LossWorkspace work)
+                  uint32_t validChannelMask, int maskChannel, int discardMaskedOut, uint32_t gridX, uint32_t blocks, LossWorkspace work)
 {
     constexpr int PAIRS = NTC_HIP_DEV_MAX_CHANNELS / 2;
     __shared__ double sums[4][NTC_HIP_DEV_MAX_CHANNELS];
@@ -1174,7 +1190,7 @@ image_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int 
     mine += __shfl_xor(mine, 1, 64);
     if ((lane & 3) == 0) sums[wave][lane >> 2] = mine;       // bits 5 ... 2 of the lane number are its channel's, most significant first
     __syncthreads();
-    uint32_t const block = blockIdx.y * gridDim.x + blockIdx.x, blocks = gridDim.x * gridDim.y;
+    uint32_t const block = blockIdx.y * gridX + blockIdx.x;
     uint32_t const group = block / kLossGroup, groups = (blocks + kLossGroup - 1) / kLossGroup, first = group * kLossGroup;
     double total = 0.0;                                      // threads 0 ... 15
     if (threadIdx.x < NTC_HIP_DEV_MAX_CHANNELS) {
@@ -1207,13 +1223,13 @@ hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int heig
 {
     LossGrid const grid = image_loss_grid(width, height, compute_units_of_current_device());
     bool const two = (width & 1) == 0, masked = maskChannel >= 0;
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(grid.x, grid.y), dim3(256), 0, stream, a, b, width, height, setChannels, grid.rowsPerWave,
-                           validChannelMask, maskChannel, discardMaskedOut, work);
+    auto launch = [&](auto perLane, auto masks) {
+        constexpr auto kernel = image_loss_kernel<decltype(perLane)::value, decltype(masks)::value>;
+        return launch_kernel<kernel>(dim3(grid.x, grid.y), dim3(256), 0, stream, a, b, width, height, setChannels, grid.rowsPerWave,
+                                     validChannelMask, maskChannel, discardMaskedOut, grid.x, grid.x * grid.y, work);
     };
-    if (two) { if (masked) launch(image_loss_kernel<2, true>); else launch(image_loss_kernel<2, false>); }
-    else     { if (masked) launch(image_loss_kernel<1, true>); else launch(image_loss_kernel<1, false>); }
-    return hipGetLastError();
+    auto of_width = [&](auto perLane) { return masked ? launch(perLane, std::true_type{}) : launch(perLane, std::false_type{}); };
+    return two ? of_width(std::integral_constant<int, 2>{}) : of_width(std::integral_constant<int, 1>{});
 }
 
 // ---- image difference (src/shaders/ImageDifference.hlsl) -------------------------------------------
@@ -1272,12 +1288,12 @@ __device__ __forceinline__ float pixel_channel(uint32_t const (&words)[bytes_per
 // FORMAT: of both images, four channels each; 0: any two images.
 template <int FORMAT, bool MSLE>
 __global__ void __launch_bounds__(256)
-image_difference_kernel(ImageDifferenceArgs a, int tilesX, int tiles)
+image_difference_kernel(ImageDifferenceArgs a, int tilesX, int tiles, int step)
 {
     __shared__ float sums[4][4];
     int const lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     unsigned long long fixed = 0;                            // threads 0 ... 3: the workgroup's share of a channel's sum
-    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    for (int tile = blockIdx.x; tile < tiles; tile += step) {
         int const tileY = tile / tilesX, tileX = tile - tileY * tilesX;
         int const x = tileX * 64 + lane, yBegin = tileY * 64 + wave * 16;
         float mse[4] = { 0.f, 0.f, 0.f, 0.f };
@@ -1350,67 +1366,67 @@ hipError_t launch_image_difference(ImageDifferenceArgs const& a, hipStream_t str
 {
     int const tilesX = (a.width + 63) / 64, tiles = tilesX * ((a.height + 63) / 64);
     int const resident = 4 * compute_units_of_current_device();
-    dim3 const grid(unsigned(tiles < resident ? tiles : resident));
-    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, a, tilesX, tiles); };
+    int const workgroups = tiles < resident ? tiles : resident;
     auto of_format = [&](auto format) {
         constexpr int FORMAT = decltype(format)::value;
-        if (a.useMSLE) launch(image_difference_kernel<FORMAT, true>);
-        else           launch(image_difference_kernel<FORMAT, false>);
+        return a.useMSLE ? launch_kernel<image_difference_kernel<FORMAT, true>>(dim3(workgroups), dim3(256), 0, stream, a, tilesX, tiles, workgroups)
+                         : launch_kernel<image_difference_kernel<FORMAT, false>>(dim3(workgroups), dim3(256), 0, stream, a, tilesX, tiles, workgroups);
     };
     bool const alike = a.a.format == a.b.format && a.a.numChannels == 4 && a.b.numChannels == 4;
-    if (alike && a.a.format == NTC_HIP_DEV_FORMAT_UNORM8)       of_format(std::integral_constant<int, NTC_HIP_DEV_FORMAT_UNORM8>{});
-    else if (alike && a.a.format == NTC_HIP_DEV_FORMAT_UNORM16) of_format(std::integral_constant<int, NTC_HIP_DEV_FORMAT_UNORM16>{});
-    else if (alike && a.a.format == NTC_HIP_DEV_FORMAT_FLOAT16) of_format(std::integral_constant<int, NTC_HIP_DEV_FORMAT_FLOAT16>{});
-    else if (alike && a.a.format == NTC_HIP_DEV_FORMAT_FLOAT32) of_format(std::integral_constant<int, NTC_HIP_DEV_FORMAT_FLOAT32>{});
-    else                                                        of_format(std::integral_constant<int, 0>{});
-    return hipGetLastError();
+    switch (alike ? a.a.format : 0) {
+    case NTC_HIP_DEV_FORMAT_UNORM8:  return of_format(std::integral_constant<int, NTC_HIP_DEV_FORMAT_UNORM8>{});
+    case NTC_HIP_DEV_FORMAT_UNORM16: return of_format(std::integral_constant<int, NTC_HIP_DEV_FORMAT_UNORM16>{});
+    case NTC_HIP_DEV_FORMAT_FLOAT16: return of_format(std::integral_constant<int, NTC_HIP_DEV_FORMAT_FLOAT16>{});
+    case NTC_HIP_DEV_FORMAT_FLOAT32: return of_format(std::integral_constant<int, NTC_HIP_DEV_FORMAT_FLOAT32>{});
+    default:                         return of_format(std::integral_constant<int, 0>{});
+    }
 }
 
 template <int FORMAT>
-static void launch_read_format(ReadChannelsArgs const& a, dim3 grid, bool plain, hipStream_t stream)
+static hipError_t launch_read_format(ReadChannelsArgs const& a, dim3 grid, bool plain, hipStream_t stream)
 {
-    if (plain) hipLaunchKernelGGL((read_channels_kernel<FORMAT, true>), grid, dim3(256), 0, stream, a);
-    else       hipLaunchKernelGGL((read_channels_kernel<FORMAT, false>), grid, dim3(256), 0, stream, a);
+    return plain ? launch_kernel<read_channels_kernel<FORMAT, true>>(grid, dim3(256), 0, stream, a)
+                 : launch_kernel<read_channels_kernel<FORMAT, false>>(grid, dim3(256), 0, stream, a);
 }
 
 template <int FORMAT>
-static hipError_t launch_read_groups_of(ReadGroupsArgs const& args, GroupLaunch const& plan, hipStream_t stream)
+static hipError_t launch_read_groups_of(GroupsArgs const& args, int dstChannels, bool dithering, GroupLaunch const& plan, hipStream_t stream)
 {
-    auto launch = [&](auto channels) {
+    auto launch = [&](auto channels) -> hipError_t {
         constexpr int CHANNELS = decltype(channels)::value;
         if constexpr (CHANNELS * bytes_per_channel(FORMAT) <= 8) {
             constexpr bool unorm = FORMAT == NTC_HIP_DEV_FORMAT_UNORM8 || FORMAT == NTC_HIP_DEV_FORMAT_UNORM16;   // (dithering changes only these)
-            if (unorm && args.a.useDithering) hipLaunchKernelGGL((read_groups_kernel<FORMAT, CHANNELS, unorm>), dim3(plan.blocks), dim3(plan.threads), plan.ldsBytes, stream, args);
-            else                              hipLaunchKernelGGL((read_groups_kernel<FORMAT, CHANNELS, false>), dim3(plan.blocks), dim3(plan.threads), plan.ldsBytes, stream, args);
+            if (unorm && dithering) return launch_kernel<read_groups_kernel<FORMAT, CHANNELS, unorm>>(dim3(plan.grid.step), dim3(plan.threads), plan.ldsBytes, stream, args);
+            return launch_kernel<read_groups_kernel<FORMAT, CHANNELS, false>>(dim3(plan.grid.step), dim3(plan.threads), plan.ldsBytes, stream, args);
+        } else {
+            return hipErrorInvalidValue;
         }
     };
-    switch (args.a.dstChannels) {
-    case 1: launch(std::integral_constant<int, 1>{}); break;
-    case 2: launch(std::integral_constant<int, 2>{}); break;
-    case 3: launch(std::integral_constant<int, 3>{}); break;
-    case 4: launch(std::integral_constant<int, 4>{}); break;
-    case 5: launch(std::integral_constant<int, 5>{}); break;
-    case 6: launch(std::integral_constant<int, 6>{}); break;
-    case 7: launch(std::integral_constant<int, 7>{}); break;
-    case 8: launch(std::integral_constant<int, 8>{}); break;
+    switch (dstChannels) {
+    case 1: return launch(std::integral_constant<int, 1>{});
+    case 2: return launch(std::integral_constant<int, 2>{});
+    case 3: return launch(std::integral_constant<int, 3>{});
+    case 4: return launch(std::integral_constant<int, 4>{});
+    case 5: return launch(std::integral_constant<int, 5>{});
+    case 6: return launch(std::integral_constant<int, 6>{});
+    case 7: return launch(std::integral_constant<int, 7>{});
+    case 8: return launch(std::integral_constant<int, 8>{});
     default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 static hipError_t launch_read_groups(ReadChannelsArgs const& a, hipStream_t stream)
 {
-    ReadGroupsArgs args{};
-    args.a = a;
     GroupLaunch const plan = plan_groups(a.width, a.height, a.srcColorSpaces, a.dstColorSpaces, a.numChannels < a.dstChannels ? a.numChannels : a.dstChannels, true);
-    args.grid = plan.grid;
-    args.transfers = plan.transfers;
+    GroupsArgs const args{ const_cast<uint16_t*>(a.planarPairs), a.dst, a.rowPitch, a.width, a.height, plan.grid, plan.transfers,
+                           uint8_t(a.setChannels), uint8_t(a.firstChannel), uint8_t(a.numChannels), a.dstColorSpaces[3], 0 };
+    bool const dithering = a.useDithering != 0;
     switch (a.format) {
-    case NTC_HIP_DEV_FORMAT_UNORM8:  return launch_read_groups_of<NTC_HIP_DEV_FORMAT_UNORM8>(args, plan, stream);
-    case NTC_HIP_DEV_FORMAT_UNORM16: return launch_read_groups_of<NTC_HIP_DEV_FORMAT_UNORM16>(args, plan, stream);
-    case NTC_HIP_DEV_FORMAT_FLOAT16: return launch_read_groups_of<NTC_HIP_DEV_FORMAT_FLOAT16>(args, plan, stream);
-    case NTC_HIP_DEV_FORMAT_FLOAT32: return launch_read_groups_of<NTC_HIP_DEV_FORMAT_FLOAT32>(args, plan, stream);
-    case NTC_HIP_DEV_FORMAT_UINT32:  return launch_read_groups_of<NTC_HIP_DEV_FORMAT_UINT32>(args, plan, stream);
+    case NTC_HIP_DEV_FORMAT_UNORM8:  return launch_read_groups_of<NTC_HIP_DEV_FORMAT_UNORM8>(args, a.dstChannels, dithering, plan, stream);
+    case NTC_HIP_DEV_FORMAT_UNORM16: return launch_read_groups_of<NTC_HIP_DEV_FORMAT_UNORM16>(args, a.dstChannels, dithering, plan, stream);
+    case NTC_HIP_DEV_FORMAT_FLOAT16: return launch_read_groups_of<NTC_HIP_DEV_FORMAT_FLOAT16>(args, a.dstChannels, dithering, plan, stream);
+    case NTC_HIP_DEV_FORMAT_FLOAT32: return launch_read_groups_of<NTC_HIP_DEV_FORMAT_FLOAT32>(args, a.dstChannels, dithering, plan, stream);
+    case NTC_HIP_DEV_FORMAT_UINT32:  return launch_read_groups_of<NTC_HIP_DEV_FORMAT_UINT32>(args, a.dstChannels, dithering, plan, stream);
     default: return hipErrorInvalidValue;
     }
 }
@@ -1421,27 +1437,25 @@ hipError_t launch_read_channels(ReadChannelsArgs const& args, hipStream_t stream
     if (a.dstWidth > 0) {                                    // resampling copy
         dim3 const grid((a.dstWidth + 63) / 64, (a.dstHeight + 3) / 4);
         switch (a.format) {
-        case NTC_HIP_DEV_FORMAT_UNORM8:  hipLaunchKernelGGL(read_channels_resize_kernel<NTC_HIP_DEV_FORMAT_UNORM8>, grid, dim3(256), 0, stream, a); break;
-        case NTC_HIP_DEV_FORMAT_UNORM16: hipLaunchKernelGGL(read_channels_resize_kernel<NTC_HIP_DEV_FORMAT_UNORM16>, grid, dim3(256), 0, stream, a); break;
-        case NTC_HIP_DEV_FORMAT_FLOAT16: hipLaunchKernelGGL(read_channels_resize_kernel<NTC_HIP_DEV_FORMAT_FLOAT16>, grid, dim3(256), 0, stream, a); break;
-        case NTC_HIP_DEV_FORMAT_FLOAT32: hipLaunchKernelGGL(read_channels_resize_kernel<NTC_HIP_DEV_FORMAT_FLOAT32>, grid, dim3(256), 0, stream, a); break;
-        case NTC_HIP_DEV_FORMAT_UINT32:  hipLaunchKernelGGL(read_channels_resize_kernel<NTC_HIP_DEV_FORMAT_UINT32>, grid, dim3(256), 0, stream, a); break;
+        case NTC_HIP_DEV_FORMAT_UNORM8:  return launch_kernel<read_channels_resize_kernel<NTC_HIP_DEV_FORMAT_UNORM8>>(grid, dim3(256), 0, stream, a);
+        case NTC_HIP_DEV_FORMAT_UNORM16: return launch_kernel<read_channels_resize_kernel<NTC_HIP_DEV_FORMAT_UNORM16>>(grid, dim3(256), 0, stream, a);
+        case NTC_HIP_DEV_FORMAT_FLOAT16: return launch_kernel<read_channels_resize_kernel<NTC_HIP_DEV_FORMAT_FLOAT16>>(grid, dim3(256), 0, stream, a);
+        case NTC_HIP_DEV_FORMAT_FLOAT32: return launch_kernel<read_channels_resize_kernel<NTC_HIP_DEV_FORMAT_FLOAT32>>(grid, dim3(256), 0, stream, a);
+        case NTC_HIP_DEV_FORMAT_UINT32:  return launch_kernel<read_channels_resize_kernel<NTC_HIP_DEV_FORMAT_UINT32>>(grid, dim3(256), 0, stream, a);
         default: return hipErrorInvalidValue;
         }
-        return hipGetLastError();
     }
     if (a.dstChannels * bytes_per_channel(a.format) <= 8) return launch_read_groups(a, stream);
     dim3 const grid = copy_grid(a.width, a.height, a.xShift);
     bool const plain = plain_copy(a.srcColorSpaces, a.dstColorSpaces, a.useDithering);
     switch (a.format) {
-    case NTC_HIP_DEV_FORMAT_UNORM8:  launch_read_format<NTC_HIP_DEV_FORMAT_UNORM8>(a, grid, plain, stream); break;
-    case NTC_HIP_DEV_FORMAT_UNORM16: launch_read_format<NTC_HIP_DEV_FORMAT_UNORM16>(a, grid, plain, stream); break;
-    case NTC_HIP_DEV_FORMAT_FLOAT16: launch_read_format<NTC_HIP_DEV_FORMAT_FLOAT16>(a, grid, plain, stream); break;
-    case NTC_HIP_DEV_FORMAT_FLOAT32: launch_read_format<NTC_HIP_DEV_FORMAT_FLOAT32>(a, grid, plain, stream); break;
-    case NTC_HIP_DEV_FORMAT_UINT32:  launch_read_format<NTC_HIP_DEV_FORMAT_UINT32>(a, grid, plain, stream); break;
+    case NTC_HIP_DEV_FORMAT_UNORM8:  return launch_read_format<NTC_HIP_DEV_FORMAT_UNORM8>(a, grid, plain, stream);
+    case NTC_HIP_DEV_FORMAT_UNORM16: return launch_read_format<NTC_HIP_DEV_FORMAT_UNORM16>(a, grid, plain, stream);
+    case NTC_HIP_DEV_FORMAT_FLOAT16: return launch_read_format<NTC_HIP_DEV_FORMAT_FLOAT16>(a, grid, plain, stream);
+    case NTC_HIP_DEV_FORMAT_FLOAT32: return launch_read_format<NTC_HIP_DEV_FORMAT_FLOAT32>(a, grid, plain, stream);
+    case NTC_HIP_DEV_FORMAT_UINT32:  return launch_read_format<NTC_HIP_DEV_FORMAT_UINT32>(a, grid, plain, stream);
     default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -24,6 +24,7 @@
 // launch, a workgroup tile of 64 x 4 texels = four wave tiles of 32 x 2 (see decode_kernel); lane = texel in the input stage,
 // lane (j = lane%16, g = lane/16) = channels 16t+4g..+3 of texel j in the matrix stages.
 #include "ntc_decode_device.h"
+#include "ntc_launch.h"
 #include <type_traits>
 
 namespace ntc_hip_dev {
@@ -502,10 +503,10 @@ __device__ void build_fp8_posenc_table(Lds& lds)
 }
 
 // Fills the feature table with the same operations the arithmetic path applies per lane.
-template <class Lds>
+template <int THREADS, class Lds>
 __device__ void build_fp8_feature_lut(Lds& lds)
 {
-    for (int e = threadIdx.x; e < 1279; e += blockDim.x) {
+    for (int e = threadIdx.x; e < 1279; e += THREADS) {
         int const n = e < 16 ? 0 : (e < 77 ? 2 : (e < 318 ? 4 : 6));
         int const T = e - kFeatureLutBase(n);
         float const v = __builtin_fmaf(float(T), __builtin_ldexpf(0.13333334f, -n), -1.f);
@@ -759,7 +760,7 @@ __device__ __forceinline__ void mlp_forward_fp8(Fp8Lds<V>& lds, int wave, int la
 // of a common sequence drift apart in time, and the latent reads from memory doubled.)
 template <class V>
 __global__ void __launch_bounds__(V::THREADS, 1)
-decode_fp8_kernel(MipTable table, int numMips, int totalTiles, Fp8Handoff handoff)
+decode_fp8_kernel(MipTable table, int numMips, int totalTiles, int workgroups, Fp8Handoff handoff)
 {
     DevMip const* const mips = table_entries(table.entries);
     if (!V::ONE && *handoff.word != handoff.serial) return;  // the one-plane launch before this one met only its own sets
@@ -769,13 +770,13 @@ decode_fp8_kernel(MipTable table, int numMips, int totalTiles, Fp8Handoff handof
     int const member = wave >> 2;                            // which quartet of the workgroup
     int const j = lane & 15, g = lane >> 4;
 
-    int const per = (totalTiles + gridDim.x - 1) / gridDim.x;
+    int const per = (totalTiles + workgroups - 1) / workgroups;
     int const tileBegin = blockIdx.x * per;
     int const tileEnd = min(totalTiles, tileBegin + per);
     if (tileBegin >= tileEnd) return;                        // uniform across the workgroup
 
     build_fp8_posenc_table(lds);
-    build_fp8_feature_lut(lds);
+    build_fp8_feature_lut<V::THREADS>(lds);
 
     int modes = 7;                                           // uniform: the hidden layers' modes (stage_fp8_weights)
 
@@ -857,7 +858,7 @@ decode_fp8_kernel(MipTable table, int numMips, int totalTiles, Fp8Handoff handof
 template <class V>
 __global__ void __launch_bounds__(V::THREADS, 1)
 query_fp8_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queries, uint64_t numQueries,
-                 uint16_t* __restrict__ out, Fp8Handoff handoff)
+                 uint16_t* __restrict__ out, int workgroups, Fp8Handoff handoff)
 {
     DevMip const* const mips = table_entries(table.entries);
     if (!V::ONE && *handoff.word != handoff.serial) return;  // the set went to the one-plane launch before this one
@@ -884,12 +885,12 @@ query_fp8_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queri
         return;
     }
     build_fp8_posenc_table(lds);
-    build_fp8_feature_lut(lds);
+    build_fp8_feature_lut<V::THREADS>(lds);
     stage_fp8_weights<V>(lds, mips[0].weights, modes);
     __syncthreads();
 
     uint64_t const numBlocks = (numQueries + V::THREADS - 1) / V::THREADS;
-    for (uint64_t block = blockIdx.x; block < numBlocks; block += gridDim.x) {
+    for (uint64_t block = blockIdx.x; block < numBlocks; block += uint32_t(workgroups)) {
         uint64_t const q0 = block * V::THREADS + uint64_t(wave) * 64;
         if (q0 >= numQueries) continue;
         uint64_t const qi = min(q0 + uint64_t(lane), numQueries - 1);
@@ -956,11 +957,9 @@ static hipError_t launch_fp8_variant(MipTable const& mips, int numMips, int tota
 {
     using One = Fp8Variant<FEATURES, true>;
     using Any = Fp8Variant<FEATURES, false>;
-    hipLaunchKernelGGL(decode_fp8_kernel<One>, dim3(gridSize), dim3(One::THREADS), 0, stream, mips, numMips, totalTiles, handoff);
-    hipError_t const e = hipGetLastError();
+    hipError_t const e = launch_kernel<decode_fp8_kernel<One>>(dim3(gridSize), dim3(One::THREADS), 0, stream, mips, numMips, totalTiles, gridSize, handoff);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(decode_fp8_kernel<Any>, dim3(gridSize), dim3(Any::THREADS), 0, stream, mips, numMips, totalTiles, handoff);
-    return hipGetLastError();
+    return launch_kernel<decode_fp8_kernel<Any>>(dim3(gridSize), dim3(Any::THREADS), 0, stream, mips, numMips, totalTiles, gridSize, handoff);
 }
 
 hipError_t launch_decode_fp8(int variant, MipTable const& mips, int numMips, int totalTiles, int gridSize, Fp8Handoff handoff, hipStream_t stream)
@@ -979,11 +978,9 @@ static hipError_t launch_fp8_query_variant(MipTable const& mips, int numMips, De
 {
     using One = Fp8Variant<FEATURES, true>;
     using Any = Fp8Variant<FEATURES, false>;
-    hipLaunchKernelGGL(query_fp8_kernel<One>, dim3(gridSize), dim3(One::THREADS), 0, stream, mips, numMips, queries, numQueries, out, handoff);
-    hipError_t const e = hipGetLastError();
+    hipError_t const e = launch_kernel<query_fp8_kernel<One>>(dim3(gridSize), dim3(One::THREADS), 0, stream, mips, numMips, queries, numQueries, out, gridSize, handoff);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(query_fp8_kernel<Any>, dim3(gridSize), dim3(Any::THREADS), 0, stream, mips, numMips, queries, numQueries, out, handoff);
-    return hipGetLastError();
+    return launch_kernel<query_fp8_kernel<Any>>(dim3(gridSize), dim3(Any::THREADS), 0, stream, mips, numMips, queries, numQueries, out, gridSize, handoff);
 }
 
 hipError_t launch_queries_fp8(int variant, MipTable const& mips, int numMips, DevQuery const* queries, uint64_t numQueries,

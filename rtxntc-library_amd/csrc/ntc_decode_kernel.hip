@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "ntc_decode_kernel.h"
+#include "ntc_launch.h"
 #include "ntc_decode_device.h"
 #include <type_traits>
 
@@ -1204,7 +1205,7 @@ __device__ __forceinline__ void mlp_forward_f16(LdsT<V>& lds, int wave, int lane
 // Two workgroups of eight waves per CU: sixteen waves, 128 VGPRs each, four to a SIMD.
 template <class V>
 __global__ void __launch_bounds__(V::THREADS, V::WAVES_PER_SIMD)
-decode_kernel(MipTable table, int numMips, int totalTiles)
+decode_kernel(MipTable table, int numMips, int totalTiles, int workgroups)
 {
     DevMip const* const mips = table_entries(table.entries);
     __shared__ LdsT<V> lds;
@@ -1218,9 +1219,9 @@ decode_kernel(MipTable table, int numMips, int totalTiles)
     // device in turn, and each die has a cache of its own: the shares are numbered so that a die's workgroups hold
     // neighbouring shares - one eighth of the list per die - and the grid rows that vertically adjacent shares both
     // read come from memory once per die, not once per share.
-    int const per = (totalTiles + gridDim.x - 1) / gridDim.x;
+    int const per = (totalTiles + workgroups - 1) / workgroups;
     constexpr int kDies = 8;
-    int const share = (gridDim.x % kDies == 0) ? int(blockIdx.x % kDies) * int(gridDim.x / kDies) + int(blockIdx.x / kDies) : int(blockIdx.x);
+    int const share = (workgroups % kDies == 0) ? int(blockIdx.x % kDies) * (workgroups / kDies) + int(blockIdx.x / kDies) : int(blockIdx.x);
     int const tileBegin = share * per;
     int const tileEnd = min(totalTiles, tileBegin + per);
 
@@ -1342,7 +1343,7 @@ decode_kernel(MipTable table, int numMips, int totalTiles)
 template <class V>
 __global__ void __launch_bounds__(V::THREADS, V::WAVES_PER_SIMD)
 query_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queries, uint64_t numQueries,
-             uint16_t* __restrict__ out)
+             uint16_t* __restrict__ out, int workgroups)
 {
     DevMip const* const mips = table_entries(table.entries);
     __shared__ LdsT<V> lds;
@@ -1375,7 +1376,7 @@ query_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queries, 
     __syncthreads();
 
     uint64_t const numBlocks = (numQueries + V::THREADS - 1) / V::THREADS;
-    for (uint64_t block = blockIdx.x; block < numBlocks; block += gridDim.x) {
+    for (uint64_t block = blockIdx.x; block < numBlocks; block += uint32_t(workgroups)) {
         uint64_t const q0 = block * V::THREADS + uint64_t(wave) * 64;
         if (q0 >= numQueries) continue;
         uint64_t const qi = min(q0 + uint64_t(lane), numQueries - 1);
@@ -1497,8 +1498,7 @@ using VCfg3   = Variant<0, 16, 4, 16, 16, 16, 2, 48, 64, 64, 64, true>;   // wid
 template <class V>
 static hipError_t launch_variant(MipTable const& mips, int numMips, int totalTiles, int gridSize, hipStream_t stream)
 {
-    hipLaunchKernelGGL(decode_kernel<V>, dim3(gridSize), dim3(V::THREADS), 0, stream, mips, numMips, totalTiles);
-    return hipGetLastError();
+    return launch_kernel<decode_kernel<V>>(dim3(gridSize), dim3(V::THREADS), 0, stream, mips, numMips, totalTiles, gridSize);
 }
 
 hipError_t launch_decode(int variant, MipTable const& mips, int numMips, int totalTiles, int gridSize, hipStream_t stream)
@@ -1519,8 +1519,7 @@ template <class V>
 static hipError_t launch_query_variant(MipTable const& mips, int numMips, DevQuery const* queries, uint64_t numQueries,
                                        uint16_t* out, int gridSize, hipStream_t stream)
 {
-    hipLaunchKernelGGL(query_kernel<V>, dim3(gridSize), dim3(V::THREADS), 0, stream, mips, numMips, queries, numQueries, out);
-    return hipGetLastError();
+    return launch_kernel<query_kernel<V>>(dim3(gridSize), dim3(V::THREADS), 0, stream, mips, numMips, queries, numQueries, out, gridSize);
 }
 
 // Plain grid ([layer][row][column] u16) -> bricks; one thread per stored u16, reads coalesced.
