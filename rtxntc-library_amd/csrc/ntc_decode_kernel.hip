@@ -157,20 +157,14 @@ struct alignas(16) LdsT : BiasLoT<V::FP8_WEIGHTS, V::NTILES> {
     uint32_t ytab[64][4];             // same for y, one byte up
 };
 
-// OCP e4m3 (1-4-3, bias 7, no infinities) byte -> the integer 512*value: subnormals m * 2^-9,
-// normals (8+m) * 2^(e-10).  The two NaN encodings decode as 0.
-__device__ __forceinline__ int32_t e4m3_times_512(uint32_t byte)
+// Four OCP e4m3 (1-4-3, bias 7, no infinities) bytes -> the integers 512*value (the conversion is exact and so is the
+// product: at most 448 * 512).  The two NaN encodings decode as 0.
+__device__ __forceinline__ void e4m3_times_512(uint32_t bytes, int32_t (&w)[4])
 {
-    uint32_t const e = (byte >> 3) & 15u, m = byte & 7u;
-    int32_t mag = (e == 0) ? int32_t(m) : int32_t((8u + m) << (e - 1u));
-    if ((byte & 0x7fu) == 0x7fu) mag = 0;
-    return (byte & 0x80u) ? -mag : mag;
-}
-
-// A operand dword of an int8 layer: four consecutive weights of one row (0 beyond the layer's inputs).
-__device__ __forceinline__ uint32_t weight_dword(uint32_t const* blob32, int woff, int row, int in, int k)
-{
-    return (k < in) ? blob32[(woff + row * in + k) >> 2] : 0u;
+    v2f const lo = __builtin_amdgcn_cvt_pk_f32_fp8(int(bytes), false), hi = __builtin_amdgcn_cvt_pk_f32_fp8(int(bytes), true);
+    float const f[4] = { lo[0], lo[1], hi[0], hi[1] };
+#pragma unroll
+    for (int r = 0; r < 4; ++r) w[r] = f[r] == f[r] ? int32_t(f[r] * 512.f) : 0;
 }
 
 __device__ __forceinline__ uint32_t halves_of_ints(int a, int b)                   // two integers of at most 11 bits -> two fp16 (exact)
@@ -183,12 +177,13 @@ __device__ __forceinline__ uint32_t halves_of_ints(int a, int b)                
 __device__ __forceinline__ void int8_planes(uint32_t v, uint32_t (&planes)[3])
 {
     planes[0] = planes[1] = planes[2] = 0;
+    int32_t W[4];
+    e4m3_times_512(v, W);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        int32_t const W = e4m3_times_512((v >> (8 * r)) & 0xffu);
-        planes[0] |= uint32_t(W & 63) << (8 * r);
-        planes[1] |= uint32_t((W >> 6) & 63) << (8 * r);
-        planes[2] |= (uint32_t(W >> 12) & 0xffu) << (8 * r);
+        planes[0] |= uint32_t(W[r] & 63) << (8 * r);
+        planes[1] |= uint32_t((W[r] >> 6) & 63) << (8 * r);
+        planes[2] |= (uint32_t(W[r] >> 12) & 0xffu) << (8 * r);
     }
 }
 
@@ -204,6 +199,46 @@ __device__ __forceinline__ int lane_id()
     return int(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
 }
 
+// One byte of the positional encoding (Inference.hlsli:89-113): int(enc * 127.5), truncating.
+__device__ __forceinline__ uint32_t posenc_byte(float p)
+{
+    float const e = (p - floorf(p)) * 2.f - 1.f;
+    return uint32_t(int(e * 127.5f)) & 0xffu;
+}
+
+// Fills the phase tables.  For positionScale = 2^-k the encoding of texel x depends only on
+// x mod 2^k, and all arithmetic involved is exact, so table and per-lane evaluation agree; scales of
+// 1 and above have period 1 (k = 0).  One entry per thread, threads 0..62 fill both tables.
+template <class V>
+__device__ __forceinline__ void build_posenc_tables(LdsT<V>& lds, int t)
+{
+    if (t < 63) {
+        int const k = 31 - __builtin_clz(uint32_t(t + 1));   // floor(log2(t + 1))
+        int const phase = t + 1 - (1 << k);
+        float p = float(phase) * __builtin_ldexpf(1.f, -k);
+        uint32_t e[3];
+#pragma unroll
+        for (int w = 0; w < 3; ++w) {
+            e[w] = posenc_byte(p) | (posenc_byte(p + 0.25f) << 16);
+            p *= 2.f;
+        }
+        lds.xtab[t][0] = e[0];      lds.xtab[t][1] = e[1];      lds.xtab[t][2] = e[2];      lds.xtab[t][3] = 0;
+        lds.ytab[t][0] = e[0] << 8; lds.ytab[t][1] = e[1] << 8; lds.ytab[t][2] = e[2] << 8; lds.ytab[t][3] = 0;
+    }
+}
+
+// The tables of a workgroup: positional encoding, and 2-bit code bytes -> input bytes (code q maps to 85*q - 128,
+// 255/3 = 85).
+template <class V>
+__device__ __forceinline__ void build_tables(LdsT<V>& lds, int tid)
+{
+    uint32_t x = uint32_t(tid) & 0xffu;
+    x = (x | (x << 12)) & 0x000f000fu;
+    x = (x | (x << 6))  & 0x03030303u;
+    lds.lut2[tid & 0xff] = (x * 85u) ^ 0x80808080u;
+    build_posenc_tables<V>(lds, tid);
+}
+
 // Copies the int8 blob (src/WeightLayout.cpp:42-49: matrices, then fp32 scales, then int32
 // biases; W[c*IN + k]) into LDS in MFMA operand order.  Returns kStagedF16 when layers 1..3 were
 // staged for the fp16 matrix instruction (see mlp_forward_f16): that needs, for every channel of
@@ -216,219 +251,214 @@ __device__ __forceinline__ int lane_id()
 // (needs |acc| < 2^22: |bias| <= 3 100 000 for every channel, the inputs add at most 64 * 128 * 127).
 constexpr int kStagedF16 = 1, kOutputsBounded = 2, kL0Magic = 4;
 constexpr int32_t kMagicBits = 0x4B400000;                   // 12582912.0f = 1.5 * 2^23
+//
+// A wave takes whole output tiles (16 rows of a layer).  Its lane (i, kg) holds, for every layer, exactly the dwords of
+// row i that it will write - the int8 and the fp16 operand order differ in where a dword goes, not in which lane holds
+// it - so the weights come from memory straight into registers, all of a wave's loads in flight together, a row's sums
+// are sums over the lane's dwords and two exchanges, and one barrier (the conditions of all waves) lies between.  The
+// tables of the workgroup (`tables`: the first call) are built while the loads are under way.  A workgroup waits for
+// this before its first tile: 7900 cycles, tables included, when the blob went through LDS, was read from there again by
+// every step, and the rows were summed by four threads each; 5300 this way (a 128 x 128 decode: 9.1 us, 8.5 now; with
+// e4m3 weights, whose conversion also got shorter, 15.6 and 14.4).
 template <class V>
-__device__ __attribute__((noinline)) int stage_weights(LdsT<V>& lds, uint8_t const* __restrict__ blob, int const tid)
+__device__ __attribute__((noinline)) int stage_weights(LdsT<V>& lds, uint8_t const* blobOfLanes, int const tid, int tables)
 {
-    constexpr int ins[4]   = { V::IN, V::H0, V::H1, V::H2 };
-    constexpr int tiles[4] = { V::T0, V::T1, V::T2, V::T3 };
-    constexpr int woff[4]  = { 0, V::W1_OFF, V::W2_OFF, V::W3_OFF };
-    // The blob first goes into LDS as it is (the transposition buffers are idle now), in one pass of coalesced loads:
-    // everything below - the row sums above all, one thread per channel walking its row - then reads LDS instead of
-    // following a chain of loads from memory.
-    constexpr int kBlobDwords = (V::BIAS_OFF + 4 * V::TOTAL_OUT) / 4;
-    static_assert(sizeof(lds.in) >= size_t(kBlobDwords + 4) * 4, "the blob fits the transposition buffers");
-    uint32_t* const flags = &lds.in[0][0][0];                  // one word for the workgroup's flags, then the blob
-    uint32_t* const raw32 = flags + 4;
-    {
-        uint32_t const* const src = reinterpret_cast<uint32_t const*>(blob);
-        for (int e = tid; e < kBlobDwords; e += V::THREADS) raw32[e] = src[e];
-        if (tid == 0) *flags = 7u;
-    }
-    __syncthreads();
-    uint32_t const* const blob32 = raw32;
-    uint8_t const* const blobBytes = reinterpret_cast<uint8_t const*>(raw32);
+    constexpr int ROUNDS = (V::NTILES + V::WAVES - 1) / V::WAVES;
+    static_assert(V::H0 % 16 == 0 && V::H1 % 16 == 0 && V::H2 % 16 == 0 && V::IN % 16 == 0, "whole tiles of 16 x 16");
+    typedef __attribute__((address_space(1))) uint32_t const* GlobalU32Ptr;
+    GlobalU8Ptr const blob = (GlobalU8Ptr)uniform_pointer(reinterpret_cast<uint64_t>(blobOfLanes));
+    int const lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int const i = lane & 15, kg = lane >> 4;
 
-    // scales and biases of every layer, in D-register order
-    {
-        int tileBase = 0, chanBase = 0;
+    struct Tile { int index, layer, first, in, woff, base; };                // uniform; `first`: of the layer's tiles
+    auto const tile_of = [&](int round) -> Tile {
+        int const k = wave + round * V::WAVES;
+        if (k < V::T0)                 return { k, 0, 0,                     V::IN, 0,         0 };
+        if (k < V::T0 + V::T1)         return { k, 1, V::T0,                 V::H0, V::W1_OFF, V::F16_L1 };
+        if (k < V::T0 + V::T1 + V::T2) return { k, 2, V::T0 + V::T1,         V::H1, V::W2_OFF, V::F16_L2 };
+        return                                { k, 3, V::T0 + V::T1 + V::T2, V::H2, V::W3_OFF, V::F16_L3 };
+    };
+    // dword d of the lane: inputs 16kg+4d.. of layer 0, 16d+4kg.. of the others
+    auto const has_dword = [&](Tile const& t, int d) { return t.layer == 0 ? 16 * kg + 4 * d < V::IN : 16 * d < t.in; };
+
+    uint32_t v[ROUNDS][4];
+    float scale[ROUNDS];
+    int32_t bias[ROUNDS];
 #pragma unroll
-        for (int l = 0; l < 4; ++l) {
-            for (int e = tid; e < tiles[l] * 16; e += V::THREADS) {
-                int const r = e & 3, g = (e >> 2) & 3, t = e >> 4;
-                int const c = chanBase + 16 * t + 4 * g + r;
-                lds.scale[tileBase + t][g][r] = reinterpret_cast<float const*>(blobBytes + V::SCALE_OFF)[c];
-                lds.bias[tileBase + t][g][r]  = reinterpret_cast<int32_t const*>(blobBytes + V::BIAS_OFF)[c];
-            }
-            tileBase += tiles[l];
-            chanBase += tiles[l] * 16;
-        }
-    }
-
-    // int8 tiles of layer 0 (three planes for e4m3 weights)
-    for (int e = tid; e < V::T0 * 64 * 4; e += V::THREADS) {
-        int const d = e & 3, lane = (e >> 2) & 63, t = e >> 8;
-        int const i = lane & 15, g = lane >> 4;
-        // k-slot (g, 4d+r) = input 16g+4d+r
-        uint32_t const v = weight_dword(blob32, 0, 16 * t + i, V::IN, 16 * g + 4 * d);
-        if constexpr (V::FP8_WEIGHTS) {
-            uint32_t planes[3];
-            int8_planes(v, planes);
+    for (int round = 0; round < ROUNDS; ++round) {
+        Tile const t = tile_of(round);
+        if (t.index >= V::NTILES) continue;                  // uniform
+        uint32_t const row = uint32_t(t.woff + (16 * (t.index - t.first) + i) * t.in);
 #pragma unroll
-            for (int q = 0; q < V::PLANES; ++q) lds.w[q][t][lane][d] = planes[q];
-        } else {
-            lds.w[0][t][lane][d] = v;
+        for (int d = 0; d < 4; ++d) {
+            uint32_t const at = row + uint32_t(t.layer == 0 ? 16 * kg + 4 * d : 16 * d + 4 * kg);
+            v[round][d] = *reinterpret_cast<GlobalU32Ptr>(blob + (has_dword(t, d) ? at : 0u));
         }
+        uint32_t const channel = uint32_t(16 * t.index + i);
+        scale[round] = __builtin_bit_cast(float, *reinterpret_cast<GlobalU32Ptr>(blob + (V::SCALE_OFF + 4u * channel)));
+        bias[round] = int32_t(*reinterpret_cast<GlobalU32Ptr>(blob + (V::BIAS_OFF + 4u * channel)));
     }
+    if (tables) build_tables<V>(lds, tid);                   // uniform
 
-    // Four threads per channel of layers 1..3 (two or one where the workgroup has not that many), a part of the row
-    // each: row sums decide whether the fp16 path is exact.  (The sums fit 32 bits: at most 64 weights of at most
-    // 448 * 512 in magnitude.)  After the exchange all of them hold the totals; the first writes the channel's
-    // constants further down.
-    bool fits = true, bounded = true;
-    int64_t shifted = 0;
-    bool twoPlanes = false;
-    int slotTile = 0, slotG = 0, slotR = 0;
-    constexpr int kSplit = 4 * V::LATE_CHANNELS <= V::THREADS ? 4 : (2 * V::LATE_CHANNELS <= V::THREADS ? 2 : 1);
-    static_assert(V::LATE_CHANNELS <= V::THREADS, "a thread per channel at least");
-    bool const rowThread = tid < kSplit * V::LATE_CHANNELS;
-    bool const rowWriter = rowThread && tid % kSplit == 0;
-    int const c = tid / kSplit;                              // the thread's channel among those of layers 1..3
-    if (rowThread) {
-        int const part = tid % kSplit;
-        int const l = c < V::H1 ? 1 : (c < V::H1 + V::H2 ? 2 : 3);
-        int const row = c - (l == 1 ? 0 : (l == 2 ? V::H1 : V::H1 + V::H2));
-        int const in = l == 1 ? V::H0 : (l == 2 ? V::H1 : V::H2);
-        int const off = l == 1 ? V::W1_OFF : (l == 2 ? V::W2_OFF : V::W3_OFF);
-        twoPlanes = V::FP8_WEIGHTS && l < 3;
-        static_assert(V::H0 % 16 == 0 && V::H1 % 16 == 0 && V::H2 % 16 == 0, "a part of a row is whole dwords");
+    // Row sums of layers 1..3 decide whether the fp16 path is exact.  (They fit 32 bits: at most 64 weights of at most
+    // 448 * 512 in magnitude.)
+    bool fits = true, bounded = true, small = true;
+    int64_t shifted[ROUNDS];
+#pragma unroll
+    for (int round = 0; round < ROUNDS; ++round) {
+        Tile const t = tile_of(round);
+        shifted[round] = 0;
+        if (t.index >= V::NTILES) continue;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) v[round][d] = has_dword(t, d) ? v[round][d] : 0u;
+        if (t.layer == 0) {
+            if constexpr (!V::FP8_WEIGHTS) small = small && bias[round] >= -3100000 && bias[round] <= 3100000;
+            continue;
+        }
+        bool const twoPlanes = V::FP8_WEIGHTS && t.layer < 3;
         int32_t sum = 0, sumAbs = 0, sumAbsHi = 0, sumLo = 0;
-        for (int k = part * (in / kSplit); k < (part + 1) * (in / kSplit); k += 4) {
-            uint32_t const v = blob32[(off + row * in + k) >> 2];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                uint32_t const byte = (v >> (8 * r)) & 0xffu;
-                int const w = twoPlanes ? e4m3_times_512(byte) : int(int8_t(byte));
-                int const hi = w >> 10;
-                sum += w;
-                sumAbs += w < 0 ? -w : w;
-                sumAbsHi += hi < 0 ? -hi : hi;
-                sumLo += w & 1023;
+        for (int d = 0; d < 4; ++d) {
+            if (twoPlanes) {
+                int32_t w[4];
+                e4m3_times_512(v[round][d], w);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    int32_t const hi = w[r] >> 10;
+                    sum += w[r];
+                    sumAbs += w[r] < 0 ? -w[r] : w[r];
+                    sumAbsHi += hi < 0 ? -hi : hi;
+                    sumLo += w[r] & 1023;
+                }
+            } else {
+                sum = __builtin_amdgcn_sdot4(int(v[round][d]), 0x01010101, sum, false);
+                sumAbs = int32_t(__builtin_amdgcn_sad_u8(v[round][d] ^ 0x80808080u, 0x80808080u, uint32_t(sumAbs)));
             }
         }
 #pragma unroll
-        for (int step = 1; step < kSplit; step *= 2) {        // the parts sit in neighbouring lanes of one wave
+        for (int step = 16; step <= 32; step *= 2) {
             sum += __shfl_xor(sum, step, 64);
             sumAbs += __shfl_xor(sumAbs, step, 64);
-            if constexpr (V::FP8_WEIGHTS) {
+            if (twoPlanes) {
                 sumAbsHi += __shfl_xor(sumAbsHi, step, 64);
                 sumLo += __shfl_xor(sumLo, step, 64);
             }
         }
-        int32_t const bias = reinterpret_cast<int32_t const*>(blobBytes + V::BIAS_OFF)[V::H0 + c];
-        shifted = int64_t(bias) - 113 * int64_t(sum);     // activations enter as q + 113 in [-15, 240]
-        int64_t const absBias = bias < 0 ? -int64_t(bias) : int64_t(bias);
-        int64_t const absShifted = shifted < 0 ? -shifted : shifted;
+        int64_t const start = int64_t(bias[round]) - 113 * int64_t(sum);     // activations enter as q + 113 in [-15, 240]
+        int64_t const absBias = bias[round] < 0 ? -int64_t(bias[round]) : int64_t(bias[round]);
+        int64_t const absStart = start < 0 ? -start : start;
+        shifted[round] = start;
         if (twoPlanes) {
             // Exact when the int32 accumulator the result is defined by cannot wrap (inputs in [-128, 127])
-            // and both fp32 partial sums, started at floor(shifted / 1024) and shifted mod 1024, stay integers.
-            int64_t const startHi = shifted >> 10;
-            fits = absBias + 128 * int64_t(sumAbs) < (int64_t(1) << 31)
+            // and both fp32 partial sums, started at floor(start / 1024) and start mod 1024, stay integers.
+            int64_t const startHi = start >> 10;
+            fits = fits && absBias + 128 * int64_t(sumAbs) < (int64_t(1) << 31)
                 && (startHi < 0 ? -startHi : startHi) + 240 * int64_t(sumAbsHi) < (int64_t(1) << 24)
                 && 1023 + 240 * int64_t(sumLo) < (int64_t(1) << 24);
         } else {
-            int64_t const bound = absShifted + 240 * int64_t(sumAbs);
-            fits = bound < (int64_t(1) << 24);
-            if (l == 3) bounded = float(bound) * fabsf(reinterpret_cast<float const*>(blobBytes + V::SCALE_OFF)[V::H0 + c]) < 60000.f;
+            int64_t const bound = absStart + 240 * int64_t(sumAbs);
+            fits = fits && bound < (int64_t(1) << 24);
+            if (t.layer == 3) bounded = bounded && float(bound) * fabsf(scale[round]) < 60000.f;
         }
         // the channel's scale gets multiplied by 2^24 (activations enter as (q + 113) * 2^-24): must stay finite
-        fits = fits && fabsf(reinterpret_cast<float const*>(blobBytes + V::SCALE_OFF)[V::H0 + c]) < 0x1p100f;
-        slotTile = V::T0 + (l == 1 ? 0 : (l == 2 ? V::T1 : V::T1 + V::T2)) + row / 16;
-        slotG = (row >> 2) & 3;
-        slotR = row & 3;
+        fits = fits && fabsf(scale[round]) < 0x1p100f;
     }
-    bool small = true;
-    if constexpr (!V::FP8_WEIGHTS) {
-        if (tid < V::H0) {
-            int32_t const b = reinterpret_cast<int32_t const*>(blobBytes + V::BIAS_OFF)[tid];
-            small = b >= -3100000 && b <= 3100000;
-        }
-    }
-    // The three conditions, each over every thread of the workgroup: a ballot per wave, one LDS atomic per wave on a
-    // word of the (idle) transposition buffer.  The barriers also order the bias writes above.  (The runtime's
-    // workgroup reduction would do, but as a library call it needs the caller's thread ids kept in a vector register
-    // for the whole kernel.)
+
+    // The three conditions, each over every thread of the workgroup: a word per wave in the (idle) transposition buffer.
+    // (Written before the barrier and read after it; what the buffer is used for next follows another barrier.)
+    uint32_t* const flags = &lds.in[0][0][0];
     {
         uint32_t const mine = (__all(fits ? 1 : 0) ? 1u : 0u) | (__all(bounded ? 1 : 0) ? 2u : 0u) | (__all(small ? 1 : 0) ? 4u : 0u);
-        if ((tid & 63) == 0) atomicAnd(flags, mine);
+        if (lane == 0) flags[wave] = mine;
     }
     __syncthreads();
-    uint32_t const all = __builtin_amdgcn_readfirstlane(*flags);
-    __syncthreads();                                         // every wave has read the word before the buffer is used again
+    uint32_t all = 7u;
+#pragma unroll
+    for (int w = 0; w < V::WAVES; ++w) all &= flags[w];
+    all = __builtin_amdgcn_readfirstlane(all);
     bool const useF16 = (all & 1u) != 0, outputsBounded = (all & 2u) != 0;
-    bool l0Magic = false;
-    if constexpr (!V::FP8_WEIGHTS) {
-        l0Magic = (all & 4u) != 0 && useF16;
-        if (l0Magic && tid < V::H0) {
-            int const c = tid;
-            lds.bias[c >> 4][(c >> 2) & 3][c & 3] += kMagicBits;
-        }
-    }
-    constexpr int base[4] = { 0, V::F16_L1, V::F16_L2, V::F16_L3 };
+    bool const l0Magic = !V::FP8_WEIGHTS && useF16 && (all & 4u) != 0;
+
     uint32_t* const late32 = reinterpret_cast<uint32_t*>(lds.late);
-    if (useF16) {
-        if (rowWriter) {
+    float* const scales = &lds.scale[0][0][0];               // in channel order, as it happens
+    int32_t* const biases = &lds.bias[0][0][0];
+#pragma unroll
+    for (int round = 0; round < ROUNDS; ++round) {
+        Tile const t = tile_of(round);
+        if (t.index >= V::NTILES) continue;
+        uint32_t const (&w)[4] = v[round];
+        int const channel = 16 * t.index + i, at = t.index - t.first;
+        bool const twoPlanes = V::FP8_WEIGHTS && (t.layer == 1 || t.layer == 2);
+        float channelScale = scale[round];
+        int32_t channelBias = bias[round];
+        if (t.layer == 0) {
+            // int8 tiles (three planes for e4m3 weights)
+            if (l0Magic) channelBias += kMagicBits;
             if constexpr (V::FP8_WEIGHTS) {
-                if (twoPlanes) lds.biasLo[slotTile][slotG][slotR] = float(shifted & 1023) * 0x1p-24f;
+                uint32_t planes[4][3];
+#pragma unroll
+                for (int d = 0; d < 4; ++d) int8_planes(w[d], planes[d]);
+#pragma unroll
+                for (int q = 0; q < V::PLANES; ++q)
+                    *reinterpret_cast<uint4*>(&lds.w[q][at][lane][0]) = make_uint4(planes[0][q], planes[1][q], planes[2][q], planes[3][q]);
+            } else {
+                *reinterpret_cast<uint4*>(&lds.w[0][at][lane][0]) = make_uint4(w[0], w[1], w[2], w[3]);
             }
+        } else if (useF16) {
             // sums run over (q + 113) * 2^-24 (see activate_scale4): every term, this start value included, is an
             // integer below 2^24 times 2^-24, exact in fp32; the scale takes the 2^24 back
-            lds.bias[slotTile][slotG][slotR] = __builtin_bit_cast(int32_t, float(twoPlanes ? (shifted >> 10) : shifted) * 0x1p-24f);
-            lds.scale[slotTile][slotG][slotR] = reinterpret_cast<float const*>(blobBytes + V::SCALE_OFF)[V::H0 + c] * 0x1p24f;
-        }
-        // fp16 blocks.  Lane (i, kg) of the block of output tile t and input-tile pair p holds
-        // W[16t + i][16*(2p + e/4) + 4*kg + e%4], e = 0..7: the channels lane (j, kg) of the
-        // previous layer's D registers owns, in register order.
+            if constexpr (V::FP8_WEIGHTS) {
+                if (twoPlanes && kg == 0) (&lds.biasLo[0][0][0])[channel] = float(shifted[round] & 1023) * 0x1p-24f;
+            }
+            channelBias = __builtin_bit_cast(int32_t, float(twoPlanes ? (shifted[round] >> 10) : shifted[round]) * 0x1p-24f);
+            channelScale *= 0x1p24f;
+            // fp16 blocks.  Lane (i, kg) of the block of output tile t and input-tile pair p holds
+            // W[16t + i][16*(2p + e/4) + 4*kg + e%4], e = 0..7: the channels lane (j, kg) of the
+            // previous layer's D registers owns, in register order.  A last block of one input tile has half of that.
+            int const inTiles = t.in / 16, per = V::f16_units(inTiles);
+            auto const write_blocks = [&](int dword, uint32_t const (&h)[4][2]) {        // dword: where the tile's blocks begin
 #pragma unroll
-        for (int l = 1; l < 4; ++l) {
-            int const in = ins[l];
-            int const inTiles = tiles[l - 1], pairs = inTiles / 2, per = V::f16_units(inTiles);
-            int const planeDwords = tiles[l] * per * 4;
-            // one work item = one (output tile, input tile, lane): 4 weights -> 2 dwords (per plane)
-            for (int e = tid; e < tiles[l] * inTiles * 64; e += V::THREADS) {
-                int const lane = e & 63, rest = e >> 6;
-                int const ti = rest % inTiles, t = rest / inTiles;
-                int const i = lane & 15, kg = lane >> 4;
-                uint32_t const v = blob32[(woff[l] + (16 * t + i) * in + 16 * ti + 4 * kg) >> 2];
-                int const p = ti >> 1;
-                // dword index inside `late`: paired blocks hold 4 dwords per lane, the tail block 2
-                int const at = (p < pairs) ? ((base[l] + t * per + p * 64 + lane) * 4 + (ti & 1) * 2)
-                                           : ((base[l] + t * per + pairs * 64) * 4 + lane * 2);
-                if (V::FP8_WEIGHTS && l < 3) {
+                for (int p = 0; p < 2; ++p) {
+                    if (2 * p + 1 < inTiles)  *reinterpret_cast<uint4*>(late32 + dword + (p * 64 + lane) * 4) = make_uint4(h[2 * p][0], h[2 * p][1], h[2 * p + 1][0], h[2 * p + 1][1]);
+                    else if (2 * p < inTiles) *reinterpret_cast<uint2*>(late32 + dword + p * 256 + lane * 2) = make_uint2(h[2 * p][0], h[2 * p][1]);
+                }
+            };
+            int const begin = (t.base + at * per) * 4;
+            if (twoPlanes) {
+                int const planeDwords = (t.layer == 1 ? V::T1 : V::T2) * per * 4;
+                uint32_t upper[4][2], lower[4][2];
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
                     int32_t W[4];
+                    e4m3_times_512(w[d], W);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) W[r] = e4m3_times_512((v >> (8 * r)) & 0xffu);
-                    late32[at]     = halves_of_ints(W[0] >> 10, W[1] >> 10);
-                    late32[at + 1] = halves_of_ints(W[2] >> 10, W[3] >> 10);
-                    late32[at + planeDwords]     = halves_of_ints(W[0] & 1023, W[1] & 1023);
-                    late32[at + planeDwords + 1] = halves_of_ints(W[2] & 1023, W[3] & 1023);
-                } else {
-                    late32[at]     = halves_of_bytes(v, 0);
-                    late32[at + 1] = halves_of_bytes(v, 2);
+                    for (int h = 0; h < 2; ++h) {
+                        upper[d][h] = halves_of_ints(W[2 * h] >> 10, W[2 * h + 1] >> 10);
+                        lower[d][h] = halves_of_ints(W[2 * h] & 1023, W[2 * h + 1] & 1023);
+                    }
                 }
+                write_blocks(begin, upper);
+                write_blocks(begin + planeDwords, lower);
+            } else {
+                uint32_t halves[4][2];
+#pragma unroll
+                for (int d = 0; d < 4; ++d) { halves[d][0] = halves_of_bytes(w[d], 0); halves[d][1] = halves_of_bytes(w[d], 2); }
+                write_blocks(begin, halves);
+            }
+        } else {
+            // int8 tiles: k-slot (g, 4d+r) = channel 16d+4g+r of the previous layer
+            uint4* const to = &lds.late[(t.index - V::T0) * 64 + lane];
+            if (twoPlanes) {
+                uint32_t planes[4][3];
+#pragma unroll
+                for (int d = 0; d < 4; ++d) int8_planes(w[d], planes[d]);
+#pragma unroll
+                for (int q = 0; q < V::PLANES; ++q) to[q * V::LATE_TILES * 64] = make_uint4(planes[0][q], planes[1][q], planes[2][q], planes[3][q]);
+            } else {
+                *to = make_uint4(w[0], w[1], w[2], w[3]);
             }
         }
-    } else {
-        int tileBase = 0;
-#pragma unroll
-        for (int l = 1; l < 4; ++l) {
-            int const in = ins[l];
-            for (int e = tid; e < tiles[l] * 64 * 4; e += V::THREADS) {
-                int const d = e & 3, lane = (e >> 2) & 63, t = e >> 8;
-                int const i = lane & 15, g = lane >> 4;
-                // k-slot (g, 4d+r) = channel 16d+4g+r of the previous layer
-                uint32_t const v = weight_dword(blob32, woff[l], 16 * t + i, in, 16 * d + 4 * g);
-                int const at = ((tileBase + t) * 64 + lane) * 4 + d;
-                if (V::FP8_WEIGHTS && l < 3) {
-                    uint32_t planes[3];
-                    int8_planes(v, planes);
-#pragma unroll
-                    for (int q = 0; q < V::PLANES; ++q) late32[q * V::LATE_TILES * 256 + at] = planes[q];
-                } else {
-                    late32[at] = v;
-                }
-            }
-            tileBase += tiles[l];
-        }
+        if (kg == 0) { scales[channel] = channelScale; biases[channel] = channelBias; }
     }
     return useF16 ? (kStagedF16 | (outputsBounded ? kOutputsBounded : 0) | (l0Magic ? kL0Magic : 0)) : 0;
 }
@@ -787,35 +817,6 @@ __device__ __forceinline__ void prepare_inputs_bricked(Mip const& m, LdsT<V> con
             uint32_t const l = uint32_t(int(m.positionLod * 127.5f)) & 0xffu;
             in[V::POS_BASE / 4 + 3] = l | (l << 8);
         }
-    }
-}
-
-// One byte of the positional encoding (Inference.hlsli:89-113): int(enc * 127.5), truncating.
-__device__ __forceinline__ uint32_t posenc_byte(float p)
-{
-    float const e = (p - floorf(p)) * 2.f - 1.f;
-    return uint32_t(int(e * 127.5f)) & 0xffu;
-}
-
-// Fills the phase tables.  For positionScale = 2^-k the encoding of texel x depends only on
-// x mod 2^k, and all arithmetic involved is exact, so table and per-lane evaluation agree; scales of
-// 1 and above have period 1 (k = 0).  One entry per thread, threads 0..62 fill both tables.
-template <class V>
-__device__ void build_posenc_tables(LdsT<V>& lds)
-{
-    int const t = threadIdx.x;
-    if (t < 63) {
-        int const k = 31 - __builtin_clz(uint32_t(t + 1));   // floor(log2(t + 1))
-        int const phase = t + 1 - (1 << k);
-        float p = float(phase) * __builtin_ldexpf(1.f, -k);
-        uint32_t e[3];
-#pragma unroll
-        for (int w = 0; w < 3; ++w) {
-            e[w] = posenc_byte(p) | (posenc_byte(p + 0.25f) << 16);
-            p *= 2.f;
-        }
-        lds.xtab[t][0] = e[0];      lds.xtab[t][1] = e[1];      lds.xtab[t][2] = e[2];      lds.xtab[t][3] = 0;
-        lds.ytab[t][0] = e[0] << 8; lds.ytab[t][1] = e[1] << 8; lds.ytab[t][2] = e[2] << 8; lds.ytab[t][3] = 0;
     }
 }
 
@@ -1225,15 +1226,6 @@ decode_kernel(MipTable table, int numMips, int totalTiles, int workgroups)
     int const tileBegin = share * per;
     int const tileEnd = min(totalTiles, tileBegin + per);
 
-    {   // 2-bit code bytes -> input bytes: code q maps to 85*q - 128 (255/3 = 85)
-        uint32_t x = threadIdx.x & 0xffu;
-        x = (x | (x << 12)) & 0x000f000fu;
-        x = (x | (x << 6))  & 0x03030303u;
-        lds.lut2[threadIdx.x & 0xffu] = (x * 85u) ^ 0x80808080u;
-    }
-
-    build_posenc_tables<V>(lds);
-
     uint8_t const* stagedBlob = nullptr;
     int staged = 0;                                          // uniform: how layers 1..3 of the staged set run (kStagedF16, ...)
     int entry = 0;
@@ -1306,9 +1298,9 @@ decode_kernel(MipTable table, int numMips, int totalTiles, int workgroups)
             if (mips[k].weights != blob) { segEnd = mips[k].tileStart; break; }
         if (blob != stagedBlob) {                            // uniform across the workgroup
             __syncthreads();                                 // every wave has left the previous segment's weights
-            staged = __builtin_amdgcn_readfirstlane(stage_weights<V>(lds, blob, wave * 64 + lane_id()));
+            staged = __builtin_amdgcn_readfirstlane(stage_weights<V>(lds, blob, wave * 64 + lane_id(), stagedBlob == nullptr));
             stagedBlob = blob;
-            __syncthreads();                                 // also publishes the tables built above
+            __syncthreads();
         }
         int const part = (segEnd - segBegin + GROUP - 1) / GROUP;
         int const myBegin = segBegin + member * part, myEnd = min(segEnd, myBegin + part);
@@ -1364,14 +1356,7 @@ query_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queries, 
     int const j = lane & 15, g = lane >> 4;
 
 
-    {   // 2-bit code bytes -> input bytes (see decode_kernel)
-        uint32_t x = threadIdx.x & 0xffu;
-        x = (x | (x << 12)) & 0x000f000fu;
-        x = (x | (x << 6))  & 0x03030303u;
-        lds.lut2[threadIdx.x & 0xffu] = (x * 85u) ^ 0x80808080u;
-    }
-    build_posenc_tables<V>(lds);
-    int const staged = __builtin_amdgcn_readfirstlane(stage_weights<V>(lds, mips[0].weights, wave * 64 + lane_id()));
+    int const staged = __builtin_amdgcn_readfirstlane(stage_weights<V>(lds, mips[0].weights, wave * 64 + lane_id(), 1));
     bool const useF16 = (staged & kStagedF16) != 0;
     __syncthreads();
 
