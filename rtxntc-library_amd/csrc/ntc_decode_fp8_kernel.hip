@@ -299,53 +299,62 @@ __device__ void stage_fp8_weights(Fp8Lds<V>& lds, uint8_t const* __restrict__ bl
     }
 }
 
+// The positional encoding from the phase table.
+template <class V>
+__device__ __forceinline__ void position_from_table(uint32_t posMask, Fp8Lds<V> const& lds, int x, int y, uint32_t (&in)[24])
+{
+    uint32_t const* const ex = lds.postab[posMask + (uint32_t(x) & posMask)];
+    uint32_t const* const ey = lds.postab[posMask + (uint32_t(y) & posMask)];
+    uint4 const x0 = *reinterpret_cast<uint4 const*>(ex), y0 = *reinterpret_cast<uint4 const*>(ey);
+    uint2 const x1 = *reinterpret_cast<uint2 const*>(ex + 4), y1 = *reinterpret_cast<uint2 const*>(ey + 4);
+    in[16] = x0.x | (y0.x << 16);  in[17] = x0.w | (y0.w << 16);     // (e0, e1), (e2, e3) of wave 0
+    in[18] = x0.y | (y0.y << 16);  in[19] = x1.x | (y1.x << 16);
+    in[20] = x0.z | (y0.z << 16);  in[21] = x1.y | (y1.y << 16);
+}
+
 // The 48 inputs of one texel as 24 dwords of e4m3-rounded halves (NtcPrepareNetworkInputsInternal_FP16,
 // InferenceCoopVec.hlsli:22-107): [high-res features 0..15 | low-res features 0..15 | 12 x positional encoding |
 // lod, lod | 0, 0].  Features a grid does not store stay zero (hlsli:36-40).
 template <class V>
-__device__ __forceinline__ void prepare_inputs_fp8(DevMip const& m, int x, int y, uint32_t (&in)[24])
+__device__ __forceinline__ void prepare_inputs_fp8(DevMip const& m, Fp8Lds<V> const& lds, int x, int y, uint32_t (&in)[24])
 {
 #pragma unroll
     for (int i = 0; i < 24; ++i) in[i] = 0;
-    float const u = (float(x) + 0.5f) / float(m.width);      // hlsli:117-118
-    float const v = (float(y) + 0.5f) / float(m.height);
     constexpr int layers = (V::F + 3) / 4;
+    float const u = texel_centre(x, m.width), v = texel_centre(y, m.height);     // hlsli:117-118
+    FloatAxis const ax[2] = { axis_general(u, m.hrWidth), axis_general(u, m.lrWidth) }, ay[2] = { axis_general(v, m.hrHeight), axis_general(v, m.lrHeight) };
+    uint32_t cells[2][layers][4];
+    load_cells<layers>(m.hr, m.hrWidth, m.hrHeight, ax[0], ay[0], cells[0]);
+    load_cells<layers>(m.lr, m.lrWidth, m.lrHeight, ax[1], ay[1], cells[1]);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int grid = 0; grid < 2; ++grid) {
-        int const gw = grid == 0 ? m.hrWidth : m.lrWidth, gh = grid == 0 ? m.hrHeight : m.lrHeight;
-        uint16_t const* __restrict__ g = grid == 0 ? m.hr : m.lr;
-        Taps const tp = footprint(u, v, gw, gh);
-        size_t const layerStride = size_t(gw) * size_t(gh);
-        size_t const a00 = size_t(tp.y0) * gw + tp.x0, a10 = size_t(tp.y0) * gw + tp.x1;
-        size_t const a01 = size_t(tp.y1) * gw + tp.x0, a11 = size_t(tp.y1) * gw + tp.x1;
+        FloatTaps const tp(ax[grid], ay[grid]);
 #pragma unroll
         for (int L = 0; L < layers; ++L) {
-            uint32_t const s00 = spread4(g[a00 + L * layerStride]), s10 = spread4(g[a10 + L * layerStride]);
-            uint32_t const s01 = spread4(g[a01 + L * layerStride]), s11 = spread4(g[a11 + L * layerStride]);
-            float value[4];
+            float t[4], value[4];
+            filter4(tp, cells[grid][L], t);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float t = tp.w00 * float((s00 >> (8 * i)) & 0xffu);
-                t = __builtin_fmaf(tp.w10, float((s10 >> (8 * i)) & 0xffu), t);
-                t = __builtin_fmaf(tp.w01, float((s01 >> (8 * i)) & 0xffu), t);
-                t = __builtin_fmaf(tp.w11, float((s11 >> (8 * i)) & 0xffu), t);
-                value[i] = (4 * L + i < V::F) ? __builtin_fmaf(t, 0.13333334f, -1.f) : 0.f;
-            }
+            for (int i = 0; i < 4; ++i) value[i] = (4 * L + i < V::F) ? __builtin_fmaf(t[i], (i & 1) ? 0.13333334f / 16.f : 0.13333334f, -1.f) : 0.f;
             in[8 * grid + 2 * L]     = round_e4m3_pk(halves_rne(value[0], value[1]));
             in[8 * grid + 2 * L + 1] = round_e4m3_pk(halves_rne(value[2], value[3]));
         }
     }
-    float px = float(x) * m.positionScale, py = float(y) * m.positionScale;   // hlsli:51-75, Inference.hlsli:89-113
+    if (m.posMask <= kMaxPosMask) {
+        position_from_table<V>(m.posMask, lds, x, y, in);
+    } else {
+        float px = float(x) * m.positionScale, py = float(y) * m.positionScale;   // hlsli:51-75, Inference.hlsli:89-113
 #pragma unroll
-    for (int w = 0; w < 3; ++w) {
-        float const e0 = (px - floorf(px)) * 2.f - 1.f;
-        float const e1 = (py - floorf(py)) * 2.f - 1.f;
-        float const qx = px + 0.25f, qy = py + 0.25f;
-        float const e2 = (qx - floorf(qx)) * 2.f - 1.f;
-        float const e3 = (qy - floorf(qy)) * 2.f - 1.f;
-        in[16 + 2 * w]     = round_e4m3_pk(halves_rne(e0, e1));
-        in[16 + 2 * w + 1] = round_e4m3_pk(halves_rne(e2, e3));
-        px *= 2.f; py *= 2.f;
+        for (int w = 0; w < 3; ++w) {
+            float const e0 = (px - floorf(px)) * 2.f - 1.f;
+            float const e1 = (py - floorf(py)) * 2.f - 1.f;
+            float const qx = px + 0.25f, qy = py + 0.25f;
+            float const e2 = (qx - floorf(qx)) * 2.f - 1.f;
+            float const e3 = (qy - floorf(qy)) * 2.f - 1.f;
+            in[16 + 2 * w]     = round_e4m3_pk(halves_rne(e0, e1));
+            in[16 + 2 * w + 1] = round_e4m3_pk(halves_rne(e2, e3));
+            px *= 2.f; py *= 2.f;
+        }
     }
     in[22] = round_e4m3_pk(halves_rne(m.positionLod, m.positionLod));
 }
@@ -468,15 +477,7 @@ __device__ __forceinline__ void finish_inputs_fast(Mip const& m, Fp8Lds<V> const
             in[8 * grid + 2 * L + 1] = round_e4m3_pk(halves_rne(value[2], value[3]));
         }
     }
-    {
-        uint32_t const* const ex = lds.postab[m.posMask + (uint32_t(x) & m.posMask)];
-        uint32_t const* const ey = lds.postab[m.posMask + (uint32_t(y) & m.posMask)];
-        uint4 const x0 = *reinterpret_cast<uint4 const*>(ex), y0 = *reinterpret_cast<uint4 const*>(ey);
-        uint2 const x1 = *reinterpret_cast<uint2 const*>(ex + 4), y1 = *reinterpret_cast<uint2 const*>(ey + 4);
-        in[16] = x0.x | (y0.x << 16);  in[17] = x0.w | (y0.w << 16);     // (e0, e1), (e2, e3) of wave 0
-        in[18] = x0.y | (y0.y << 16);  in[19] = x1.x | (y1.x << 16);
-        in[20] = x0.z | (y0.z << 16);  in[21] = x1.y | (y1.y << 16);
-    }
+    position_from_table<V>(m.posMask, lds, x, y, in);
     in[22] = round_e4m3_pk(halves_rne(m.positionLod, m.positionLod));
 }
 
@@ -793,7 +794,7 @@ decode_fp8_kernel(MipTable table, int numMips, int totalTiles, int workgroups, F
                 fetch_latents_fast<V>(m.full, x, y, fetch);
                 finish_inputs_fast<V>(m.full, lds, x, y, fetch, in);
             } else {
-                prepare_inputs_fp8<V>(m.full, x, y, in);
+                prepare_inputs_fp8<V>(m.full, lds, x, y, in);
             }
         }
         v4i D[4];
@@ -908,7 +909,7 @@ query_fp8_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queri
             else         fetch_latents_fast<V>(m, x, y, fetch);
             finish_inputs_fast<V>(m, lds, x, y, fetch, in);
         } else {
-            prepare_inputs_fp8<V>(mips[validMip ? query.mip : 0], x, y, in);
+            prepare_inputs_fp8<V>(mips[validMip ? query.mip : 0], lds, x, y, in);
         }
         v4i D[4];
         v4f S;

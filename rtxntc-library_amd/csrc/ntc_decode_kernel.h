@@ -30,6 +30,8 @@ enum {
 };
 inline bool variant_is_fp8_network(int variant) { return variant >= NTC_HIP_VARIANT_REF16_FP8 && variant <= NTC_HIP_VARIANT_REF4_FP8; }
 
+constexpr uint32_t kMaxPosMask = 31;                       // the kernels' phase tables
+
 // One colour mip of one texture set, as the kernel sees it.  Entries are sorted by
 // tileStart; a workgroup tile covers 64 x 4 texels.
 struct DevMip {
@@ -48,7 +50,8 @@ struct DevMip {
     // N = ((2x+1) << shl) - (1 << sublog):  shl | n << 8 | sublog << 16 | log2(grid size) << 24.
     uint32_t fast;
     uint32_t hrAxisX, hrAxisY, lrAxisX, lrAxisY;
-    uint32_t posMask;          // (texels per period of the positional encoding) - 1
+    uint32_t posMask;          // (texels per period of the positional encoding) - 1, or beyond kMaxPosMask: the period is
+                               // not a power of two up to 32
     // The two grids once more in query order (bricks of 4 x 4 or 8 x 8 cells, all layers of a cell
     // together), or null; read by the query kernel only.
     uint8_t const* hrBricks;

@@ -463,100 +463,76 @@ __device__ __attribute__((noinline)) int stage_weights(LdsT<V>& lds, uint8_t con
     return useF16 ? (kStagedF16 | (outputsBounded ? kOutputsBounded : 0) | (l0Magic ? kL0Magic : 0)) : 0;
 }
 
+// The positional encoding from the phase tables.
 template <class V>
-__device__ __forceinline__ void prepare_inputs_general(DevMip const& m, int x, int y, uint32_t (&in)[16])
+__device__ __forceinline__ void position_from_tables(uint32_t posMask, LdsT<V> const& lds, int x, int y, uint32_t (&in)[16])
 {
+    uint4 const ex = *reinterpret_cast<uint4 const*>(&lds.xtab[posMask + (uint32_t(x) & posMask)][0]);
+    uint4 const ey = *reinterpret_cast<uint4 const*>(&lds.ytab[posMask + (uint32_t(y) & posMask)][0]);
+    in[V::POS_BASE / 4 + 0] = ex.x | ey.x;
+    in[V::POS_BASE / 4 + 1] = ex.y | ey.y;
+    in[V::POS_BASE / 4 + 2] = ex.z | ey.z;
+}
+
+// Input vector of one texel of any sizes (src/Inference.cu:52-53, FeatureGridDevice.h).
+template <class V>
+__device__ __forceinline__ void prepare_inputs_general(DevMip const& m, LdsT<V> const& lds, int x, int y, uint32_t (&in)[16])
+{
+    constexpr int HL = V::HR_MODE == 1 ? 1 : (V::HR_F + 3) / 4, LL = (V::LR_F + 3) / 4;
 #pragma unroll
     for (int i = 0; i < 16; ++i) in[i] = 0;
 
-    float const u = (float(x) + 0.5f) / float(m.width);      // src/Inference.cu:52-53
-    float const v = (float(y) + 0.5f) / float(m.height);
+    float const u = texel_centre(x, m.width), v = texel_centre(y, m.height);
+    FloatAxis const hx = axis_general(u, m.hrWidth), hy = axis_general(v, m.hrHeight);
+    FloatAxis const lx = axis_general(u, m.lrWidth), ly = axis_general(v, m.lrHeight);
+    uint32_t hv[HL][4], lv[LL][4];                           // [layer][tap 00, 10, 01, 11]
+    load_cells<HL>(m.hr, m.hrWidth, m.hrHeight, hx, hy, hv);
+    load_cells<LL>(m.lr, m.lrWidth, m.lrHeight, lx, ly, lv);
+    __builtin_amdgcn_sched_barrier(0);
 
     // ---- high-res grid
-    {
-        Taps const tp = footprint(u, v, m.hrWidth, m.hrHeight);
-        uint16_t const* __restrict__ g = m.hr;
-        size_t const layerStride = size_t(m.hrWidth) * size_t(m.hrHeight);
-        size_t const a00 = size_t(tp.y0) * m.hrWidth + tp.x0, a10 = size_t(tp.y0) * m.hrWidth + tp.x1;
-        size_t const a01 = size_t(tp.y1) * m.hrWidth + tp.x0, a11 = size_t(tp.y1) * m.hrWidth + tp.x1;
-        constexpr int perWord = 16 / V::HR_BITS;
-        constexpr int layers = (V::HR_F + perWord - 1) / perWord;
-        if constexpr (V::HR_MODE == 1) {
-            // 2x2 concat: taps a00,a01,a10,a11 of FeatureGridDevice.h:67-70 = (x0,y0),(x1,y0),(x0,y1),(x1,y1)
-            size_t const addr[4] = { a00, a10, a01, a11 };
+    if constexpr (V::HR_MODE == 1) {
+        // 2x2 concat: taps a00,a01,a10,a11 of FeatureGridDevice.h:67-70 = (x0,y0),(x1,y0),(x0,y1),(x1,y1)
+        static_assert(V::HR_MODE != 1 || (V::HR_BITS == 2 && V::HR_F == 8 && V::HR_SLOTS == 8), "concat grids: 8 x 2-bit");
 #pragma unroll
-            for (int tap = 0; tap < 4; ++tap) {
+        for (int tap = 0; tap < 4; ++tap) {
+            in[2 * tap]     = lds.lut2[hv[0][tap] & 0xffu];
+            in[2 * tap + 1] = lds.lut2[hv[0][tap] >> 8];
+        }
+    } else {
+        static_assert(V::HR_MODE == 1 || V::HR_BITS == 4, "bilinear grids are 4-bit");
+        FloatTaps const tp(hx, hy);
 #pragma unroll
-                for (int L = 0; L < layers; ++L) {
-                    uint32_t const w = g[addr[tap] + L * layerStride];
-#pragma unroll
-                    for (int q = 0; q < perWord / 4; ++q) {
-                        int const f0 = L * perWord + 4 * q;          // first feature of this dword
-                        if (f0 < V::HR_F) {
-                            uint32_t s, b;
-                            if constexpr (V::HR_BITS == 2) { s = spread2(w >> (8 * q));  b = s * 85u; }
-                            else                           { s = spread4(w >> (16 * q)); b = s * 17u; }
-                            b ^= 0x80808080u;
-                            if (f0 + 4 > V::HR_F) b &= (1u << (8 * (V::HR_F - f0))) - 1u;   // masked features stay 0
-                            in[(tap * V::HR_SLOTS + f0) / 4] = b;
-                        }
-                    }
-                }
-            }
-        } else {
-            static_assert(V::HR_MODE == 1 || V::HR_BITS == 4, "bilinear grids are 4-bit");
-#pragma unroll
-            for (int L = 0; L < layers; ++L) {
-                uint32_t const s00 = spread4(g[a00 + L * layerStride]);
-                uint32_t const s10 = spread4(g[a10 + L * layerStride]);
-                uint32_t const s01 = spread4(g[a01 + L * layerStride]);
-                uint32_t const s11 = spread4(g[a11 + L * layerStride]);
-                uint32_t b = bilinear4(tp, s00, s10, s01, s11, 17.f);
-                if (4 * L + 4 > V::HR_F) b &= (1u << (8 * (V::HR_F - 4 * L))) - 1u;
-                in[L] = b;
-            }
+        for (int L = 0; L < HL; ++L) {
+            uint32_t b = bilinear4(tp, hv[L]);
+            if (4 * L + 4 > V::HR_F) b &= (1u << (8 * (V::HR_F - 4 * L))) - 1u;      // masked features stay 0
+            in[L] = b;
         }
     }
     // ---- low-res grid: bilinear, 4-bit
     {
-        Taps const tp = footprint(u, v, m.lrWidth, m.lrHeight);
-        uint16_t const* __restrict__ g = m.lr;
-        size_t const layerStride = size_t(m.lrWidth) * size_t(m.lrHeight);
-        size_t const a00 = size_t(tp.y0) * m.lrWidth + tp.x0, a10 = size_t(tp.y0) * m.lrWidth + tp.x1;
-        size_t const a01 = size_t(tp.y1) * m.lrWidth + tp.x0, a11 = size_t(tp.y1) * m.lrWidth + tp.x1;
-        constexpr int layers = (V::LR_F + 3) / 4;
+        FloatTaps const tp(lx, ly);
 #pragma unroll
-        for (int L = 0; L < layers; ++L) {
-            uint32_t const s00 = spread4(g[a00 + L * layerStride]);
-            uint32_t const s10 = spread4(g[a10 + L * layerStride]);
-            uint32_t const s01 = spread4(g[a01 + L * layerStride]);
-            uint32_t const s11 = spread4(g[a11 + L * layerStride]);
-            uint32_t b = bilinear4(tp, s00, s10, s01, s11, 17.f);
+        for (int L = 0; L < LL; ++L) {
+            uint32_t b = bilinear4(tp, lv[L]);
             if (4 * L + 4 > V::LR_F) b &= (1u << (8 * (V::LR_F - 4 * L))) - 1u;
             in[V::HR_INPUTS / 4 + L] = b;
         }
     }
-    // ---- positional encoding (Inference.hlsli:89-120); int() truncates
-    {
+    // ---- positional encoding (Inference.hlsli:89-120)
+    if (m.posMask <= kMaxPosMask) {
+        position_from_tables<V>(m.posMask, lds, x, y, in);
+    } else {
         float px = float(x) * m.positionScale, py = float(y) * m.positionScale;
 #pragma unroll
         for (int w = 0; w < 3; ++w) {
-            float const e0 = (px - floorf(px)) * 2.f - 1.f;
-            float const e1 = (py - floorf(py)) * 2.f - 1.f;
-            float const qx = px + 0.25f, qy = py + 0.25f;
-            float const e2 = (qx - floorf(qx)) * 2.f - 1.f;
-            float const e3 = (qy - floorf(qy)) * 2.f - 1.f;
-            uint32_t const p = (uint32_t(int(e0 * 127.5f)) & 0xffu)
-                             | ((uint32_t(int(e1 * 127.5f)) & 0xffu) << 8)
-                             | ((uint32_t(int(e2 * 127.5f)) & 0xffu) << 16)
-                             | ((uint32_t(int(e3 * 127.5f)) & 0xffu) << 24);
-            in[V::POS_BASE / 4 + w] = p;
+            in[V::POS_BASE / 4 + w] = posenc_byte(px) | (posenc_byte(py) << 8) | (posenc_byte(px + 0.25f) << 16) | (posenc_byte(py + 0.25f) << 24);
             px *= 2.f; py *= 2.f;
         }
-        if constexpr (V::LOD == 2) {
-            uint32_t const l = uint32_t(int(m.positionLod * 127.5f)) & 0xffu;
-            in[V::POS_BASE / 4 + 3] = l | (l << 8);
-        }
+    }
+    if constexpr (V::LOD == 2) {
+        uint32_t const l = uint32_t(int(m.positionLod * 127.5f)) & 0xffu;
+        in[V::POS_BASE / 4 + 3] = l | (l << 8);
     }
 }
 
@@ -632,11 +608,7 @@ __device__ __forceinline__ void prepare_inputs_fast(Mip const& m, LdsT<V> const&
     }
     // ---- positional encoding from the per-mip phase tables
     {
-        uint4 const ex = *reinterpret_cast<uint4 const*>(&lds.xtab[m.posMask + (uint32_t(x) & m.posMask)][0]);
-        uint4 const ey = *reinterpret_cast<uint4 const*>(&lds.ytab[m.posMask + (uint32_t(y) & m.posMask)][0]);
-        in[V::POS_BASE / 4 + 0] = ex.x | ey.x;
-        in[V::POS_BASE / 4 + 1] = ex.y | ey.y;
-        in[V::POS_BASE / 4 + 2] = ex.z | ey.z;
+        position_from_tables<V>(m.posMask, lds, x, y, in);
         if constexpr (V::LOD == 2) {
             uint32_t const l = uint32_t(int(m.positionLod * 127.5f)) & 0xffu;
             in[V::POS_BASE / 4 + 3] = l | (l << 8);
@@ -736,11 +708,7 @@ __device__ __forceinline__ void prepare_inputs_scattered(Mip const& m, LdsT<V> c
         }
     }
     {
-        uint4 const ex = *reinterpret_cast<uint4 const*>(&lds.xtab[m.posMask + (uint32_t(x) & m.posMask)][0]);
-        uint4 const ey = *reinterpret_cast<uint4 const*>(&lds.ytab[m.posMask + (uint32_t(y) & m.posMask)][0]);
-        in[V::POS_BASE / 4 + 0] = ex.x | ey.x;
-        in[V::POS_BASE / 4 + 1] = ex.y | ey.y;
-        in[V::POS_BASE / 4 + 2] = ex.z | ey.z;
+        position_from_tables<V>(m.posMask, lds, x, y, in);
         if constexpr (V::LOD == 2) {
             uint32_t const l = uint32_t(int(m.positionLod * 127.5f)) & 0xffu;
             in[V::POS_BASE / 4 + 3] = l | (l << 8);
@@ -808,11 +776,7 @@ __device__ __forceinline__ void prepare_inputs_bricked(Mip const& m, LdsT<V> con
         }
     }
     {
-        uint4 const ex = *reinterpret_cast<uint4 const*>(&lds.xtab[m.posMask + (uint32_t(x) & m.posMask)][0]);
-        uint4 const ey = *reinterpret_cast<uint4 const*>(&lds.ytab[m.posMask + (uint32_t(y) & m.posMask)][0]);
-        in[V::POS_BASE / 4 + 0] = ex.x | ey.x;
-        in[V::POS_BASE / 4 + 1] = ex.y | ey.y;
-        in[V::POS_BASE / 4 + 2] = ex.z | ey.z;
+        position_from_tables<V>(m.posMask, lds, x, y, in);
         if constexpr (V::LOD == 2) {
             uint32_t const l = uint32_t(int(m.positionLod * 127.5f)) & 0xffu;
             in[V::POS_BASE / 4 + 3] = l | (l << 8);
@@ -1245,7 +1209,7 @@ decode_kernel(MipTable table, int numMips, int totalTiles, int workgroups)
         {
             int const x = min(x0 + j + 16 * (g & 1), m.width - 1), y = min(y0 + (g >> 1), m.height - 1);
             if (m.fast) prepare_inputs_fast<V>(m.full, lds, x, y, in);
-            else        prepare_inputs_general<V>(m.full, x, y, in);
+            else        prepare_inputs_general<V>(m.full, lds, x, y, in);
         }
         // ---- 2.-4. transpose, hidden layers, output layer
         if (V::F16_LAYERS && (staged & kStagedF16)) {
@@ -1377,7 +1341,7 @@ query_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queries, 
             if (bricked) prepare_inputs_bricked<V>(m, lds, x, y, in);
             else         prepare_inputs_scattered<V>(m, lds, x, y, (GlobalU8Ptr)mips, in);
         }
-        else                    prepare_inputs_general<V>(mips[validMip ? query.mip : 0], x, y, in);
+        else                    prepare_inputs_general<V>(mips[validMip ? query.mip : 0], lds, x, y, in);
 
         // lane (j, g) holds channels 4g..4g+3 of query q0 + 16b + j; validity travels by shuffle
         auto store_outputs = [&](auto checked, int b, v4f Fb, v4f S) __attribute__((always_inline)) {

@@ -202,7 +202,8 @@ bool axis_params(int32_t size, int32_t grid, uint32_t& packed, int& n)
     return true;
 }
 
-// Decides whether a mip may take the kernel's all-integer input stage and fills its parameters.
+// Decides whether a mip may take the kernel's all-integer input stage and fills its parameters, and whether its
+// positional encoding comes from the kernel's tables (which mips of other sizes can use too).
 // Conditions: every size a power of two (then every float operation of the general stage is
 // exact and the integer form gives the same bytes); bilinear weights of at most 8 fractional
 // bits in total (16-bit lanes of the packed filter cannot overflow); positionScale a power of
@@ -210,6 +211,13 @@ bool axis_params(int32_t size, int32_t grid, uint32_t& packed, int& n)
 void fill_fast_path(NtcHipDecoderSpec const& spec, DevMip& e)
 {
     e.fast = 0;
+    e.posMask = ~0u;
+    int exp2 = 0;
+    float const mant = std::frexp(e.positionScale, &exp2);      // scale = mant * 2^exp2, mant in [0.5, 1)
+    if (mant == 0.5f && exp2 - 1 >= -5 && exp2 - 1 <= 20) {
+        int const k = -(exp2 - 1);                              // scale = 2^-k
+        e.posMask = k > 0 ? (1u << k) - 1u : 0u;
+    }
     int hx, hy, lx, ly;
     if (!axis_params(e.width, e.hrWidth, e.hrAxisX, hx) || !axis_params(e.height, e.hrHeight, e.hrAxisY, hy)) return;
     if (!axis_params(e.width, e.lrWidth, e.lrAxisX, lx) || !axis_params(e.height, e.lrHeight, e.lrAxisY, ly)) return;
@@ -217,12 +225,7 @@ void fill_fast_path(NtcHipDecoderSpec const& spec, DevMip& e)
     if (spec.hrMode == NTC_HIP_GRID_BILINEAR && hx + hy > 8) return;
     if (grid_bytes(e.hrWidth, e.hrHeight, spec.hrFeatures, spec.hrBits) >= (1ull << 31)) return;
     if (grid_bytes(e.lrWidth, e.lrHeight, spec.lrFeatures, spec.lrBits) >= (1ull << 31)) return;
-    int exp2 = 0;
-    float const mant = std::frexp(e.positionScale, &exp2);      // scale = mant * 2^exp2, mant in [0.5, 1)
-    if (!(mant == 0.5f) || exp2 - 1 < -5 || exp2 - 1 > 20) return;
-    int const k = -(exp2 - 1);                                  // scale = 2^-k
-    e.posMask = k > 0 ? (1u << k) - 1u : 0u;
-    e.fast = 1;
+    e.fast = e.posMask <= kMaxPosMask;
 }
 
 uint64_t grid_bytes(int32_t w, int32_t h, int32_t features, int32_t bits)

@@ -5,7 +5,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from cases import cfg_case, ref_case, first_mismatch
+from cases import Case, cfg_case, ref_case, first_mismatch
 
 pytestmark = pytest.mark.gpu
 
@@ -364,6 +364,26 @@ def test_pixel_layouts_with_and_without_vector_stores(ntc, device, fmt_name, shi
     case.output_bytes = cursor + 16
     expected, got = run_both(device, case)
     assert_equal_bytes(expected, got, f"{fmt_name} start {shift} pad {row_pad} stride {stride}")
+
+
+@pytest.mark.parametrize("network", ["cfg01", "ref16", "ref12", "fp8_16", "fp8_8"])
+@pytest.mark.parametrize("width,height,hr,lr,scale", [
+    (70, 6, (35, 3), (17, 1), 0.25), (33, 5, (33, 5), (1, 1), 1 / 64), (33, 5, (64, 2), (7, 9), 0.3), (65535, 1, (32767, 1), (3, 1), 1 / 32),
+    (65536, 3, (21845, 2), (65536, 3), 2.0), (1, 37, (1, 12), (1, 1000), 1 / 32)])
+def test_sampling_of_sizes_that_are_no_powers_of_two(ntc, device, network, width, height, hr, lr, scale):
+    """Texel centres, wraps and weights in floats up to the largest mips, grids coarser and finer than the image, and
+    positional encodings in and beyond the tables' range."""
+    spec = {"cfg01": ntc.presets.spec_cfg01, "ref16": lambda: ntc.presets.spec_ref092(16), "ref12": lambda: ntc.presets.spec_ref092(12),
+            "fp8_16": lambda: ntc.presets.spec_ref092_fp8(16), "fp8_8": lambda: ntc.presets.spec_ref092_fp8(8)}[network]()
+    d = ntc.abi.MipDesc()
+    d.width, d.height, d.positionScale, d.positionLod = width, height, scale, 0.25
+    (d.hrWidth, d.hrHeight), (d.lrWidth, d.lrHeight) = hr, lr
+    d.lrOffset = ntc.presets.grid_bytes(hr[0], hr[1], spec.hrFeatures, spec.hrBits)
+    latent_bytes = d.lrOffset + ntc.presets.grid_bytes(lr[0], lr[1], spec.lrFeatures, spec.lrBits)
+    kw = {"weights": ntc.synth.make_fp8_weights(spec, 5)} if network.startswith("fp8") else {"scale_log2_range": ACTIVE}
+    case = Case(ntc, spec, [d], latent_bytes, 16, ntc.abi.OUT_FP16_PLANAR_PAIRS, width + height, **kw)
+    expected, got = run_both(device, case)
+    assert_equal_bytes(expected, got, f"{network} {width}x{height} hr {hr} lr {lr} scale {scale}")
 
 
 def test_decode_is_idempotent_and_timed_variant_matches(ntc, device):
