@@ -229,12 +229,39 @@ __device__ __forceinline__ GlobalOutPtr uniform_pointer(uint64_t address)
 
 // Stores of one 16-texel block row.  `row` is uniform (start of image row y in the output), `laneOff` the
 // lane's byte offset inside the row (`laneOff2` that of the second channel pair of planar output), h01/h23 the
-// lane's four channels as halves.  `vectorStores` (uniform; RunMip) says that every lane's four channels of a
-// pixel format start at a multiple of their size and can go out as one store; otherwise channels go out one by
-// one (a per-lane look at the address as second chance cost every instantiation registers: 8 to 110 spilled).
+// lane's four channels as halves.  Four channels of a pixel go out as one store at whatever alignment the pixels have,
+// fewer as up to two.
+typedef __attribute__((address_space(1))) uint16_t* GlobalHalfOutPtr;
+typedef uint32_t __attribute__((aligned(1))) u32_any;
+typedef uint16_t __attribute__((aligned(1))) u16_any;
+typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t __attribute__((aligned(2))) u32_a2;
+typedef __attribute__((address_space(1))) u32_any*  GlobalU32AnyPtr;
+typedef __attribute__((address_space(1))) u16_any*  GlobalU16AnyPtr;
+typedef __attribute__((address_space(1))) u32x2_a2* GlobalU32x2A2Ptr;
+typedef __attribute__((address_space(1))) u32_a2*   GlobalU32A2OutPtr;
+
+// One to three channels of a pixel format (`count` uniform in the lanes that are active): u8 as packed bytes.
+__device__ __forceinline__ void store_few_bytes(GlobalOutPtr dst, uint32_t u8, int count)
+{
+    if (count & 2) { *reinterpret_cast<GlobalU16AnyPtr>(dst) = uint16_t(u8); u8 >>= 16; dst += 2; }
+    if (count & 1) *dst = uint8_t(u8);
+}
+__device__ __forceinline__ void store_few_halves(GlobalOutPtr dst, uint32_t h01, uint32_t h23, int count)
+{
+    if (count & 2) { *reinterpret_cast<GlobalU32A2OutPtr>(dst) = h01; h01 = h23; dst += 4; }
+    if (count & 1) *reinterpret_cast<GlobalHalfOutPtr>(dst) = uint16_t(h01);
+}
+
+__device__ __forceinline__ uint32_t unorm8_of_halves(uint32_t h01, uint32_t h23)
+{
+    v2h const a = __builtin_bit_cast(v2h, h01), b = __builtin_bit_cast(v2h, h23);
+    return pack_unorm8(b[1], 3, pack_unorm8(b[0], 2, pack_unorm8(a[1], 1, pack_unorm8(a[0], 0, 0u))));
+}
+
 template <int FORMAT>
 __device__ __forceinline__ void store_channels(GlobalOutPtr row, uint32_t laneOff, uint32_t laneOff2,
-                                               uint32_t h01, uint32_t h23, int nch, bool vectorStores)
+                                               uint32_t h01, uint32_t h23, int nch)
 {
     GlobalOutPtr const dst = row + laneOff;
     if constexpr (FORMAT == NTC_HIP_DEV_OUT_FP16_PLANAR_PAIRS) {
@@ -242,20 +269,12 @@ __device__ __forceinline__ void store_channels(GlobalOutPtr row, uint32_t laneOf
         *reinterpret_cast<__attribute__((address_space(1))) uint32_t*>(dst) = h01;
         if (nch > 2) *reinterpret_cast<__attribute__((address_space(1))) uint32_t*>(row + laneOff2) = h23;
     } else if constexpr (FORMAT == NTC_HIP_DEV_OUT_FP16_PIXELS) {
-        if (nch == 4 && vectorStores) {
-            *reinterpret_cast<__attribute__((address_space(1))) u32x2*>(dst) = u32x2{ h01, h23 };
-        } else {
-            uint32_t const h[4] = { h01 & 0xffffu, h01 >> 16, h23 & 0xffffu, h23 >> 16 };
-            for (int r = 0; r < nch; ++r) reinterpret_cast<__attribute__((address_space(1))) uint16_t*>(dst)[r] = uint16_t(h[r]);
-        }
+        if (nch == 4) *reinterpret_cast<GlobalU32x2A2Ptr>(dst) = u32x2_a2{ h01, h23 };
+        else          store_few_halves(dst, h01, h23, nch);
     } else {
-        v2h const a = __builtin_bit_cast(v2h, h01), b = __builtin_bit_cast(v2h, h23);
-        uint32_t const u8 = pack_unorm8(b[1], 3, pack_unorm8(b[0], 2, pack_unorm8(a[1], 1, pack_unorm8(a[0], 0, 0u))));
-        if (nch == 4 && vectorStores) {
-            *reinterpret_cast<__attribute__((address_space(1))) uint32_t*>(dst) = u8;
-        } else {
-            for (int r = 0; r < nch; ++r) dst[r] = uint8_t(u8 >> (8 * r));
-        }
+        uint32_t const u8 = unorm8_of_halves(h01, h23);
+        if (nch == 4) *reinterpret_cast<GlobalU32AnyPtr>(dst) = u8;
+        else          store_few_bytes(dst, u8, nch);
     }
 }
 
@@ -267,15 +286,9 @@ struct RunMip {
     uint64_t outRowPitch;
     int32_t width, height, numChannels, outPixelStride, outFormat;
     uint32_t fast;
-    // Pixel formats: every lane's group of four channels (8 bytes of fp16, 4 of unorm8; the groups of a pixel
-    // follow each other) starts at a multiple of its size - decided once here from the mip's start, row pitch and
-    // pixel stride, not per lane and store from a 64-bit address (headline -0.4 %, batch of sets -0.9 %).
-    bool vectorStores;
     __device__ __forceinline__ explicit RunMip(DevMip const& m)
         : full(m), out(m.out), outRowPitch(m.outRowPitch), width(m.width), height(m.height), numChannels(m.numChannels),
-          outPixelStride(m.outPixelStride), outFormat(m.outFormat), fast(m.fast),
-          vectorStores(((reinterpret_cast<uint64_t>(m.out) | m.outRowPitch | uint64_t(uint32_t(m.outPixelStride)))
-                        & (m.outFormat == NTC_HIP_DEV_OUT_FP16_PIXELS ? 7u : 3u)) == 0) {}
+          outPixelStride(m.outPixelStride), outFormat(m.outFormat), fast(m.fast) {}
 };
 
 // Look-ups in the table of a decode call (one entry per mip of every set, sorted by tileStart).  Both go through
@@ -341,7 +354,7 @@ __device__ __forceinline__ void store_row(Mip const& m, StorePlace<FORMAT, Mip> 
     uint32_t const h01 = to_half2_bits<CHECKED>(float(D[0]) * S[0], float(D[1]) * S[1]);
     uint32_t const h23 = to_half2_bits<CHECKED>(float(D[2]) * S[2], float(D[3]) * S[3]);
     GlobalOutPtr const row = uniform_pointer(reinterpret_cast<uint64_t>(m.out) + size_t(y) * at.rowBytes);
-    store_channels<FORMAT>(row, at.laneOff, at.laneOff2, h01, h23, at.nch, m.vectorStores);
+    store_channels<FORMAT>(row, at.laneOff, at.laneOff2, h01, h23, at.nch);
 }
 
 // The stores of one wave tile: D[b] holds the lane's four channels of the texel in column `x` of block b, where block
@@ -358,9 +371,8 @@ __device__ __forceinline__ void store_tile(Mip const& m, Acc const (&D)[4], v4f 
     }
 }
 
-// The stores of a wave tile at an image edge, of a mip with fewer than sixteen channels or of a pixel format that
-// needs channel-by-channel stores: the general form above, in the mip's format, with the checked conversion (it
-// equals the unchecked one wherever that is allowed).  Not inlined: tiles like these are few, and inlined next to
+// The stores of a wave tile at an image edge: the general form above, in the mip's format, with the checked conversion
+// (it equals the unchecked one wherever that is allowed).  Not inlined: tiles like these are few, and inlined next to
 // the fast form the six instantiations cost the kernels registers.
 template <class Acc>
 __device__ __attribute__((noinline)) void store_tile_general(DevMip const* mip, Acc D0, Acc D1, Acc D2, Acc D3, v4f S, int x, int y0, int chBase)
@@ -372,21 +384,27 @@ __device__ __attribute__((noinline)) void store_tile_general(DevMip const* mip, 
     else                                                   store_tile<NTC_HIP_DEV_OUT_UNORM8_PIXELS, true>(m, D, S, x, y0, chBase);
 }
 
-// The stores of a wave tile that lies inside the image of a mip whose channel count is a multiple of four (the common
-// case): no bounds to test, every lane stores its four channels of all four blocks (block b: 16 texels from
-// x0 + 16 * (b & 1) in row y0 + (b >> 1)), and the row addresses are one uniform
+// The stores of a wave tile that lies inside the image: no bounds to test, every lane stores its channels of all four
+// blocks (block b: 16 texels from x0 + 16 * (b & 1) in row y0 + (b >> 1)), and the row addresses are one uniform
 // base plus multiples of the row size - a handful of scalar additions instead of a 64-bit product, a test and a
 // branch per row.  x0, y0: first texel of the wave tile; lane = (j, g) holds channels 4g..4g+3 of texel column j.
+//
+// A channel count that is no multiple of four leaves the lanes of one group with one to three channels: a second,
+// uniform part stores those (planar pairs: the group's first pair only, or both).  1920 x 1080 texels of nine unorm8
+// channels took 13 us more than of sixteen planar ones when such mips took the general form, 5 now.
 template <int FORMAT, bool CHECKED, class Acc, class Mip>
 __device__ __forceinline__ void store_tile_inside(Mip const& m, Acc const (&D)[4], v4f S, int x0, int y0, int j, int g)
 {
     typedef __attribute__((address_space(1))) uint32_t* DwordPtr;
+    constexpr bool PLANAR = FORMAT == NTC_HIP_DEV_OUT_FP16_PLANAR_PAIRS;
+    int const rest = m.numChannels & 3;                                          // uniform
+    int const mine = m.numChannels - 4 * g;                                      // channels from the lane's first on
     size_t rowBytes;
     uint32_t laneOff;
     GlobalOutPtr tile;
-    if (4 * g >= m.numChannels) return;                                          // lanes of channel groups the mip does not have
-    if constexpr (FORMAT == NTC_HIP_DEV_OUT_FP16_PLANAR_PAIRS) {
-        rowBytes = size_t(m.width) * size_t(m.numChannels) * 2;                  // fp16, a multiple of four channels
+    if (mine <= 0) return;                                                       // lanes of channel groups the mip does not have
+    if constexpr (PLANAR) {
+        rowBytes = size_t(m.width) * size_t((m.numChannels + 1) & ~1) * 2;       // fp16, whole pairs
         laneOff = uint32_t(g) * (uint32_t(m.width) * 8u) + uint32_t(j) * 4u;     // (4g * width + 2j) halves
         tile = (GlobalOutPtr)m.out + (size_t(y0) * rowBytes + size_t(x0) * 4);
     } else {
@@ -398,20 +416,41 @@ __device__ __forceinline__ void store_tile_inside(Mip const& m, Acc const (&D)[4
     // The offsets stay 32-bit values of this tile (hoisted out of the tile loop they become 64-bit lane addresses, and
     // the stores lose their "scalar base + 32-bit lane offset" form).
     asm volatile("" : "+v"(laneOff), "+v"(laneOff2));
+    auto const row_of = [&](int b) -> GlobalOutPtr {
+        return tile + size_t(b >> 1) * rowBytes + ((b & 1) ? size_t(16) * (PLANAR ? size_t(4) : size_t(m.outPixelStride)) : size_t(0));
+    };
+    auto const halves = [&](int b, uint32_t& h01, uint32_t& h23) {
+        h01 = to_half2_bits<CHECKED>(float(D[b][0]) * S[0], float(D[b][1]) * S[1]);
+        h23 = to_half2_bits<CHECKED>(float(D[b][2]) * S[2], float(D[b][3]) * S[3]);
+    };
+    if (mine >= 4) {
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        uint32_t const h01 = to_half2_bits<CHECKED>(float(D[b][0]) * S[0], float(D[b][1]) * S[1]);
-        uint32_t const h23 = to_half2_bits<CHECKED>(float(D[b][2]) * S[2], float(D[b][3]) * S[3]);
-        GlobalOutPtr const row = tile + size_t(b >> 1) * rowBytes
-                               + ((b & 1) ? size_t(16) * (FORMAT == NTC_HIP_DEV_OUT_FP16_PLANAR_PAIRS ? size_t(4) : size_t(m.outPixelStride)) : size_t(0));
-        if constexpr (FORMAT == NTC_HIP_DEV_OUT_FP16_PLANAR_PAIRS) {
-            *reinterpret_cast<DwordPtr>(row + laneOff) = h01;
-            *reinterpret_cast<DwordPtr>(row + laneOff2) = h23;
-        } else if constexpr (FORMAT == NTC_HIP_DEV_OUT_FP16_PIXELS) {
-            *reinterpret_cast<__attribute__((address_space(1))) u32x2*>(row + laneOff) = u32x2{ h01, h23 };
-        } else {
-            v2h const a = __builtin_bit_cast(v2h, h01), c = __builtin_bit_cast(v2h, h23);
-            *reinterpret_cast<DwordPtr>(row + laneOff) = pack_unorm8(c[1], 3, pack_unorm8(c[0], 2, pack_unorm8(a[1], 1, pack_unorm8(a[0], 0, 0u))));
+        for (int b = 0; b < 4; ++b) {
+            uint32_t h01, h23;
+            halves(b, h01, h23);
+            if constexpr (PLANAR) {
+                *reinterpret_cast<DwordPtr>(row_of(b) + laneOff) = h01;
+                *reinterpret_cast<DwordPtr>(row_of(b) + laneOff2) = h23;
+            } else if constexpr (FORMAT == NTC_HIP_DEV_OUT_FP16_PIXELS) {
+                *reinterpret_cast<GlobalU32x2A2Ptr>(row_of(b) + laneOff) = u32x2_a2{ h01, h23 };
+            } else {
+                *reinterpret_cast<GlobalU32AnyPtr>(row_of(b) + laneOff) = unorm8_of_halves(h01, h23);
+            }
+        }
+    }
+    if (rest != 0 && mine < 4) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            uint32_t h01, h23;
+            halves(b, h01, h23);
+            if constexpr (PLANAR) {
+                *reinterpret_cast<DwordPtr>(row_of(b) + laneOff) = h01;
+                if (rest == 3) *reinterpret_cast<DwordPtr>(row_of(b) + laneOff2) = h23;
+            } else if constexpr (FORMAT == NTC_HIP_DEV_OUT_FP16_PIXELS) {
+                store_few_halves(row_of(b) + laneOff, h01, h23, rest);
+            } else {
+                store_few_bytes(row_of(b) + laneOff, unorm8_of_halves(h01, h23), rest);
+            }
         }
     }
 }

@@ -800,11 +800,9 @@ decode_fp8_kernel(MipTable table, int numMips, int totalTiles, int workgroups, F
         v4i D[4];
         v4f S;
         mlp_forward_fp8<V>(lds, wave, lane, modes, in, D, S);
-        // a wave tile inside the image, channels in whole groups of four (pixel formats: vector stores possible), takes
-        // the stores without tests; the one-plane instantiation also without the fp16-overflow check where no output
-        // can come near it (the general instantiation keeps to the checked conversion)
-        bool const inside = x0 + 32 <= m.width && y0 + 2 <= m.height && (m.numChannels & 3) == 0
-                         && (m.outFormat == NTC_HIP_DEV_OUT_FP16_PLANAR_PAIRS || m.vectorStores);
+        // a wave tile inside the image takes the stores without tests; the one-plane instantiation also without the
+        // fp16-overflow check where no output can come near it (the general instantiation keeps to the checked conversion)
+        bool const inside = x0 + 32 <= m.width && y0 + 2 <= m.height;
         if (!inside) {
             store_tile_general(&m.full, D[0], D[1], D[2], D[3], S, x0 + j, y0, 4 * g);
         } else if (V::ONE && (modes & kFp8OutputsBounded)) {

@@ -1216,10 +1216,8 @@ decode_kernel(MipTable table, int numMips, int totalTiles, int workgroups)
             v4f D[4];
             v4f S;
             mlp_forward_f16<V>(lds, wave, lane, (staged & kL0Magic) != 0, in, D, S);
-            // a wave tile inside the image, channels in whole groups of four (pixel formats: vector stores possible),
-            // takes the stores without tests
-            bool const inside = x0 + 32 <= m.width && y0 + 2 <= m.height && (m.numChannels & 3) == 0
-                             && (m.outFormat == NTC_HIP_DEV_OUT_FP16_PLANAR_PAIRS || m.vectorStores);
+            // a wave tile inside the image takes the stores without tests
+            bool const inside = x0 + 32 <= m.width && y0 + 2 <= m.height;
             if (!inside) {
                 store_tile_general(&m.full, D[0], D[1], D[2], D[3], S, x0 + j, y0, 4 * g);
             } else if (staged & kOutputsBounded) {

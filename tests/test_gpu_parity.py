@@ -386,6 +386,17 @@ def test_sampling_of_sizes_that_are_no_powers_of_two(ntc, device, network, width
     assert_equal_bytes(expected, got, f"{network} {width}x{height} hr {hr} lr {lr} scale {scale}")
 
 
+@pytest.mark.parametrize("channels", [1, 2, 3, 5, 6, 7, 9, 11, 14, 15])
+def test_channel_counts_that_leave_part_of_a_group(ntc, device, channels):
+    """Tiles inside the image and at its edges, with one to three channels in the last group of four, pixels packed as
+    tightly as the format allows."""
+    for fmt, size in ((ntc.abi.OUT_FP16_PLANAR_PAIRS, None), (ntc.abi.OUT_FP16_PIXELS, 2), (ntc.abi.OUT_UNORM8_PIXELS, 1)):
+        case = cfg_case(ntc, ntc.presets.spec_cfg01(), 128, 8, 2, channels, fmt, seed=channels, scale_log2_range=ACTIVE,
+                        **({"pixel_stride": size * channels} if size else {}))
+        expected, got = run_both(device, case)
+        assert_equal_bytes(expected, got, f"{channels} channels, fmt {fmt}")
+
+
 def test_decode_is_idempotent_and_timed_variant_matches(ntc, device):
     case = cfg_case(ntc, ntc.presets.spec_cfg01(), 320, 200, 4, 16, ntc.abi.OUT_UNORM8_PIXELS, seed=21, scale_log2_range=ACTIVE)
     dset = case.device_set(device)
