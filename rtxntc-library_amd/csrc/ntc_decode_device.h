@@ -186,6 +186,30 @@ typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef float    v2f __attribute__((ext_vector_type(2)));
 
+// ---- weights ------------------------------------------------------------------------------------
+
+// Four OCP e4m3 (1-4-3, bias 7, no infinities) bytes -> the integers 512*value (the conversion is exact and so is the
+// product: at most 448 * 512).  The two NaN encodings decode as 0.
+__device__ __forceinline__ void e4m3_times_512(uint32_t bytes, int32_t (&w)[4])
+{
+    v2f const lo = __builtin_amdgcn_cvt_pk_f32_fp8(int(bytes), false), hi = __builtin_amdgcn_cvt_pk_f32_fp8(int(bytes), true);
+    float const f[4] = { lo[0], lo[1], hi[0], hi[1] };
+#pragma unroll
+    for (int r = 0; r < 4; ++r) w[r] = f[r] == f[r] ? int32_t(f[r] * 512.f) : 0;
+}
+
+__device__ __forceinline__ uint32_t halves_of_bytes(uint32_t v, int firstByte)     // two int8 -> two fp16 (exact)
+{
+    v2h const h = { _Float16(int(int8_t(v >> (8 * firstByte)))), _Float16(int(int8_t(v >> (8 * firstByte + 8)))) };
+    return __builtin_bit_cast(uint32_t, h);
+}
+
+// The lane's number in its wave from the execution mask: no register has to keep the thread id alive for it.
+__device__ __forceinline__ int lane_id()
+{
+    return int(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
+}
+
 // Two network outputs -> two fp16 in one dword.  The output is an fp32 product that is THEN
 // rounded to half (round-nearest-even); a half that would be Inf/NaN is stored as zero
 // (IsHalfSpecial, Inference.cu:125-126).  |o| >= 65520 is exactly the set that rounds to

@@ -83,7 +83,7 @@ __device__ __forceinline__ uint32_t quantize_int8_pk(uint32_t yBits)
 }
 
 // ONE_: the instantiation for texture sets all of whose hidden layers run on one weight plane (see
-// classify_fp8_weights): it holds one plane in LDS instead of three, which leaves room for the transposition
+// stage_fp8_weights): it holds one plane in LDS instead of three, which leaves room for the transposition
 // buffers of sixteen waves, and its network has one form per layer, which fits the 128 registers four waves per
 // SIMD leave a lane (108 used; the general form needs 150).  The two instantiations are launched one after the
 // other; each decodes the sets that are its own.
@@ -125,52 +125,33 @@ struct alignas(16) Fp8LdsT {
     // e4m3-rounded half of fma(float(T), (2/15) * 2^-n, -1) for T = 0 .. 15 * 2^n, n = 0, 2, 4, 6 (what square
     // power-of-two geometry produces; other n take the arithmetic).
     uint16_t featureLut[1280];
-    // classify_fp8_weights: sum |512 w| of every output channel of the three hidden layers, and the flags it gathers
-    int32_t channelSum[3][64];
-    uint32_t classFlags;
+    uint32_t classFlags[WAVES];   // stage_fp8_weights: what each wave found in the weights
 };
 template <class V> using Fp8Lds = Fp8LdsT<V::HELD, V::WAVES>;
 __host__ __device__ constexpr int kFeatureLutBase(int n) { return n == 0 ? 0 : (n == 2 ? 16 : (n == 4 ? 77 : 318)); }   // 16 + 61 + 241 + 961 = 1279 entries
 
-// OCP e4m3 byte -> the integer 512 * value (NaN encodings decode as 0).
-__device__ __forceinline__ int32_t fp8_times_512(uint32_t byte)
+// Two e4m3 weights, given as 512 w, as the halves of plane p: bits [7p, 7p+7) (the top plane: the rest) of |512 w|, with
+// w's sign, in units of 2^(7p - 9); `whole`: the weights themselves (every e4m3 value is a half).
+__device__ __forceinline__ uint32_t plane_halves(int32_t w0, int32_t w1, int plane, bool whole)
 {
-    uint32_t const e = (byte >> 3) & 15u, m = byte & 7u;
-    int32_t mag = (e == 0) ? int32_t(m) : int32_t((8u + m) << (e - 1u));
-    if ((byte & 0x7fu) == 0x7fu) mag = 0;
-    return (byte & 0x80u) ? -mag : mag;
-}
-
-// Plane p of an e4m3 weight as an fp16 value: bits [7p, 7p+7) (the top plane: the rest) of |512 w|, with w's
-// sign, in units of 2^(7p - 9).
-__device__ __forceinline__ _Float16 plane_value(int32_t w512, int plane, bool whole = false)
-{
-    if (whole) return _Float16(float(w512) * 0x1p-9f);       // the weight itself: every e4m3 value is a half
-    int32_t const mag = w512 < 0 ? -w512 : w512;
-    int32_t const bits = plane == 2 ? mag >> 14 : (mag >> (7 * plane)) & 127;
-    float const unit = plane == 0 ? 0x1p-9f : (plane == 1 ? 0x1p-2f : 0x1p5f);
-    float const v = float(bits) * unit;
-    return _Float16(w512 < 0 ? -v : v);
-}
-
-// Stores the 8 (or 4) halves of one lane of an A block: weights W[row][k[e]] of one plane.
-template <class V>
-__device__ __forceinline__ void stage_plane_halves(uint32_t* dst, uint8_t const* __restrict__ matrix, int in, int row, int const* k, int count, int plane,
-                                                   bool whole)
-{
-    for (int e = 0; e < count; e += 2) {
-        _Float16 const a = plane_value(fp8_times_512(matrix[row * in + k[e]]), plane, whole);
-        _Float16 const b = plane_value(fp8_times_512(matrix[row * in + k[e + 1]]), plane, whole);
-        v2h const h = { a, b };
-        dst[e >> 1] = __builtin_bit_cast(uint32_t, h);
+    int32_t const w[2] = { w0, w1 };
+    v2h h;
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        int32_t const mag = w[r] < 0 ? -w[r] : w[r];
+        int32_t const bits = plane == 2 ? mag >> 14 : (mag >> (7 * plane)) & 127;
+        float const unit = plane == 0 ? 0x1p-9f : (plane == 1 ? 0x1p-2f : 0x1p5f);
+        float const v = float(bits) * unit;
+        h[r] = _Float16(whole ? float(w[r]) * 0x1p-9f : (w[r] < 0 ? -v : v));
     }
+    return __builtin_bit_cast(uint32_t, h);
 }
 
 // Copies the FP8 blob into LDS in matrix-instruction operand order.  Layer 0 takes its inputs in their
 // natural order (lane (i, kg) of a block of 32 holds inputs 8kg..8kg+7, of a block of 16 inputs 32+4kg..+3);
 // layers 1..3 take theirs in the order the previous layer's result registers hold them: lane (i, kg) of the
 // block for input tiles (2p, 2p+1) holds inputs 16*(2p + e/4) + 4kg + e%4, e = 0..7.
-// stage_fp8_weights takes the layers' modes from classify_fp8_weights, which reads the blob only.  Bit l is set when hidden layer l needs the general evaluation (three planes, both
+// The layers' modes that it returns: bit l is set when hidden layer l needs the general evaluation (three planes, both
 // clamps of the activation), i.e. when some weight of it has a non-zero top plane (|w| >= 32) or some bias is not
 // a finite half of magnitude <= 57344.  The other layers (every layer of a trained network) are "tame": two
 // planes, and since |sum| <= 64 * 31.75 * 3 = 6096 their outputs stay below 63440 + rounding < 65520, finite as
@@ -191,112 +172,134 @@ constexpr int kAllOnePlane = 7 << kOnePlaneShift;         // every hidden layer 
 // unless the scale is tiny, and then |bias| itself must be checked).
 constexpr int kFp8OutputsBounded = 1 << 8;
 
-// Reads the blob a dword per thread (the api requires 4-byte alignment; rows of 48 or 64 bytes: a dword never
-// straddles two channels) and gathers sums and flags in LDS: every workgroup of both instantiations does this for
-// every set it meets, and the workgroups of the one that passes over the set do nothing else.
-template <class V>
-__device__ int classify_fp8_weights(Fp8Lds<V>& lds, uint8_t const* __restrict__ blob)
+// Fills the positional table: one entry per thread, threads 0..62.
+template <class Lds>
+__device__ __forceinline__ void build_fp8_posenc_table(Lds& lds, int t)
 {
-    int const tid = threadIdx.x;
-    constexpr int rows[3] = { V::H0, V::H1, V::H2 }, ins[3] = { V::IN, V::H0, V::H1 };
-    constexpr int dwords[3] = { V::W1_OFF / 4, (V::W2_OFF - V::W1_OFF) / 4, (V::W3_OFF - V::W2_OFF) / 4 };
-    static_assert(V::IN % 4 == 0 && V::H0 % 4 == 0 && V::H1 % 4 == 0 && V::H0 <= 64, "a dword of weights belongs to one channel");
-    if (tid == 0) lds.classFlags = 0;
-    if (tid < 192) (&lds.channelSum[0][0])[tid] = 0;
-    __syncthreads();                                         // also: every wave has left the previous set's tiles
-    for (int e = tid; e < dwords[0] + dwords[1] + dwords[2]; e += V::THREADS) {
-        int const l = e < dwords[0] ? 0 : (e < dwords[0] + dwords[1] ? 1 : 2);
-        int const d = e - (l == 0 ? 0 : (l == 1 ? dwords[0] : dwords[0] + dwords[1]));
-        uint32_t const four = reinterpret_cast<uint32_t const*>(blob)[e];      // the three matrices follow each other
-        int32_t sum = 0, top = 0;
+    if (t < 63) {
+        int const k = 31 - __builtin_clz(uint32_t(t + 1));   // floor(log2(t + 1))
+        int const phase = t + 1 - (1 << k);
+        float p = float(phase) * __builtin_ldexpf(1.f, -k);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            int32_t const w = fp8_times_512((four >> (8 * q)) & 0xffu);
-            int32_t const mag = w < 0 ? -w : w;
-            sum += mag;
-            top |= mag >> 14;
+        for (int w = 0; w < 3; ++w) {
+            float const q = p + 0.25f;
+            float const e0 = (p - floorf(p)) * 2.f - 1.f, e2 = (q - floorf(q)) * 2.f - 1.f;
+            uint32_t const pair = round_e4m3_pk(halves_rne(e0, e2));
+            lds.postab[t][w] = pair & 0xffffu;
+            lds.postab[t][3 + w] = pair >> 16;
+            p *= 2.f;
         }
-        atomicAdd(&lds.channelSum[l][(4 * d) / ins[l]], sum);
-        if (top) atomicOr(&lds.classFlags, 1u << l);
+        lds.postab[t][6] = lds.postab[t][7] = 0;
     }
-    if (tid < V::OUT) {
-        float const bias = fabsf(float(reinterpret_cast<int32_t const*>(blob + V::BIAS3_OFF)[tid]));
-        float const scale = fabsf(reinterpret_cast<float const*>(blob + V::SCALE3_OFF)[tid]);
-        if (!((bias + 520192.f) * scale < 60000.f) || !(bias < 2.0e9f)) atomicOr(&lds.classFlags, 1u << 8);
-    }
-    if (tid < V::H0 + V::H1 + V::H2) {                       // a bias that is not a finite half of at most 57344
-        int const l = tid < V::H0 ? 0 : (tid < V::H0 + V::H1 ? 1 : 2);
-        if ((reinterpret_cast<uint16_t const*>(blob + V::BIAS_OFF)[tid] & 0x7fffu) > 0x7b00u) atomicOr(&lds.classFlags, 1u << l);
-    }
-    __syncthreads();
-    if (tid < 192) {
-        int const l = tid >> 6, r = tid & 63;
-        if (r < rows[l] && lds.channelSum[l][r] > kOnePlaneLimit) atomicOr(&lds.classFlags, 16u << l);
-    }
-    __syncthreads();
-    uint32_t const flags = lds.classFlags;
-    __syncthreads();                                         // read by all before the next call clears it
-    int const topMask = int(flags & 7u);
-    int const oneMask = int(~(flags >> 4) & ~flags & 7u);
-    return topMask | (oneMask << kOnePlaneShift) | ((flags & (1u << 8)) ? 0 : kFp8OutputsBounded);
 }
 
-template <class V>
-__device__ void stage_fp8_weights(Fp8Lds<V>& lds, uint8_t const* __restrict__ blob, int modes)
+// Fills the feature table with the same operations the arithmetic path applies per lane.
+template <int THREADS, class Lds>
+__device__ __forceinline__ void build_fp8_feature_lut(Lds& lds, int tid)
 {
-    int const tid = threadIdx.x;
-    int const oneMask = modes >> kOnePlaneShift;
-    // biases of the hidden layers (fp16 in the blob), scale and bias of the output layer
-    for (int e = tid; e < 9 * 16; e += V::THREADS) {
-        int const r = e & 3, g = (e >> 2) & 3, t = e >> 4;
-        int const c = 16 * t + 4 * g + r;                    // layers 0..2 back to back: 64 + 48 + 32 channels
-        lds.bias[t][g][r] = float(reinterpret_cast<_Float16 const*>(blob + V::BIAS_OFF)[c]);
+    for (int e = tid; e < 1279; e += THREADS) {
+        int const n = e < 16 ? 0 : (e < 77 ? 2 : (e < 318 ? 4 : 6));
+        int const T = e - kFeatureLutBase(n);
+        float const v = __builtin_fmaf(float(T), __builtin_ldexpf(0.13333334f, -n), -1.f);
+        lds.featureLut[e] = uint16_t(round_e4m3_pk(halves_rne(v, v)));
     }
-    if (tid < 16) {
-        lds.outScale[tid >> 2][tid & 3] = reinterpret_cast<float const*>(blob + V::SCALE3_OFF)[tid];
-        lds.outBias[tid >> 2][tid & 3] = reinterpret_cast<int32_t const*>(blob + V::BIAS3_OFF)[tid];
-    }
-    // layer 0: (plane, tile, lane) -> one K32 unit and half a K16 unit
-    for (int e = tid; e < V::HELD * V::T0 * 64; e += V::THREADS) {
-        int const lane = e & 63, t = (e >> 6) % V::T0, p = e / (64 * V::T0);
-        int const i = lane & 15, kg = lane >> 4;
-        int k32[8], k16[4];
-        for (int q = 0; q < 8; ++q) k32[q] = 8 * kg + q;
-        for (int q = 0; q < 4; ++q) k16[q] = 32 + 4 * kg + q;
-        bool const whole = p == 0 && (oneMask & 1);
-        stage_plane_halves<V>(reinterpret_cast<uint32_t*>(&lds.w0[p][t][lane]), blob, V::IN, 16 * t + i, k32, 8, p, whole);
-        stage_plane_halves<V>(reinterpret_cast<uint32_t*>(&lds.w0[p][t][64]) + 2 * lane, blob, V::IN, 16 * t + i, k16, 4, p, whole);
-    }
-    // layer 1: 64 inputs = two blocks of 32
-    for (int e = tid; e < V::HELD * V::T1 * 2 * 64; e += V::THREADS) {
-        int const lane = e & 63, pair = (e >> 6) & 1, t = (e >> 7) % V::T1, p = e / (128 * V::T1);
-        int const i = lane & 15, kg = lane >> 4;
-        int k[8];
-        for (int q = 0; q < 8; ++q) k[q] = 16 * (2 * pair + q / 4) + 4 * kg + q % 4;
-        stage_plane_halves<V>(reinterpret_cast<uint32_t*>(&lds.w1[p][t][pair * 64 + lane]), blob + V::W1_OFF, V::H0, 16 * t + i, k, 8, p, p == 0 && (oneMask & 2));
-    }
-    // layer 2: 48 inputs = one block of 32 and one of 16
-    for (int e = tid; e < V::HELD * V::T2 * 64; e += V::THREADS) {
-        int const lane = e & 63, t = (e >> 6) % V::T2, p = e / (64 * V::T2);
-        int const i = lane & 15, kg = lane >> 4;
-        int k32[8], k16[4];
-        for (int q = 0; q < 8; ++q) k32[q] = 16 * (q / 4) + 4 * kg + q % 4;
-        for (int q = 0; q < 4; ++q) k16[q] = 32 + 4 * kg + q;
-        bool const whole = p == 0 && (oneMask & 4);
-        stage_plane_halves<V>(reinterpret_cast<uint32_t*>(&lds.w2[p][t][lane]), blob + V::W2_OFF, V::H1, 16 * t + i, k32, 8, p, whole);
-        stage_plane_halves<V>(reinterpret_cast<uint32_t*>(&lds.w2[p][t][64]) + 2 * lane, blob + V::W2_OFF, V::H1, 16 * t + i, k16, 4, p, whole);
-    }
-    // output layer: int8 weights as halves, 32 inputs = one block
-    if (tid < 64) {
-        int const lane = tid, i = lane & 15, kg = lane >> 4;
-        uint32_t* dst = reinterpret_cast<uint32_t*>(&lds.w3[lane]);
-        int8_t const* W = reinterpret_cast<int8_t const*>(blob + V::W3_OFF);
-        for (int q = 0; q < 8; q += 2) {
-            int const ka = 16 * (q / 4) + 4 * kg + q % 4;
-            v2h const h = { _Float16(int(W[i * V::H2 + ka])), _Float16(int(W[i * V::H2 + ka + 1])) };
-            dst[q >> 1] = __builtin_bit_cast(uint32_t, h);
+}
+
+// A wave takes one output tile (16 rows of a layer; ten tiles) and its lane (i, kg) holds the dwords of row i that it will
+// write: they come from memory straight into registers, all loads in flight together, a row's sum is the lane's and two
+// exchanges, and one barrier - the waves' flags - lies between.  Every workgroup of both instantiations does this much
+// for every set it meets; operands are written only for sets that are the instantiation's own.  The tables of the
+// workgroup (`tables`: the first call) are built while the loads are under way.  Every wave has left the previous set's
+// weights behind the first barrier; the caller adds one behind the call.  (With the blob read twice, once per thread and
+// dword into atomic sums and once byte by byte into operands: 18.0 us for a 128 x 128 decode, 13.8 now.)
+template <class V>
+__device__ __attribute__((noinline)) int stage_fp8_weights(Fp8Lds<V>& lds, uint8_t const* blobOfLanes, int const tid, int tables)
+{
+    constexpr int TILES = V::T0 + V::T1 + V::T2 + 1;
+    static_assert(TILES <= V::WAVES, "a tile per wave at most");
+    typedef __attribute__((address_space(1))) uint32_t const* GlobalU32Ptr;
+    GlobalU8Ptr const blob = (GlobalU8Ptr)uniform_pointer(reinterpret_cast<uint64_t>(blobOfLanes));
+    int const lane = tid & 63, tile = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int const i = lane & 15, kg = lane >> 4;
+    int const layer = tile < V::T0 ? 0 : (tile < V::T0 + V::T1 ? 1 : (tile < V::T0 + V::T1 + V::T2 ? 2 : 3));
+    int const t = tile - (layer == 0 ? 0 : (layer == 1 ? V::T0 : (layer == 2 ? V::T0 + V::T1 : V::T0 + V::T1 + V::T2)));
+    int const in = layer == 0 ? V::IN : (layer == 1 ? V::H0 : (layer == 2 ? V::H1 : V::H2));
+    int const woff = layer == 0 ? 0 : (layer == 1 ? V::W1_OFF : (layer == 2 ? V::W2_OFF : V::W3_OFF));
+    bool const mine = tile < TILES;                          // uniform
+    uint32_t v[4] = { 0u, 0u, 0u, 0u }, bias = 0u, scale = 0u;
+    if (mine) {
+        uint32_t const row = uint32_t(woff + (16 * t + i) * in);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            if (16 * d >= in) continue;                      // uniform
+            v[d] = *reinterpret_cast<GlobalU32Ptr>(blob + (row + uint32_t(layer == 0 && d < 2 ? 8 * kg + 4 * d : 16 * d + 4 * kg)));
+        }
+        if (layer < 3) {
+            bias = load_u16(blob, uint32_t(V::BIAS_OFF + 2 * (16 * tile + i)));
+        } else {
+            bias = *reinterpret_cast<GlobalU32Ptr>(blob + uint32_t(V::BIAS3_OFF + 4 * i));
+            scale = *reinterpret_cast<GlobalU32Ptr>(blob + uint32_t(V::SCALE3_OFF + 4 * i));
         }
     }
+    if (tables) {                                            // uniform
+        build_fp8_posenc_table(lds, tid);
+        build_fp8_feature_lut<V::THREADS>(lds, tid);
+    }
+
+    uint32_t found = 0;                                      // bit l: not tame; bit 4 + l: not one plane; bit 8: outputs not bounded
+    if (mine && layer < 3) {
+        int32_t sum = 0, top = 0;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            int32_t w[4];
+            e4m3_times_512(v[d], w);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                int32_t const mag = w[r] < 0 ? -w[r] : w[r];
+                sum += mag;
+                top |= mag >> 14;
+            }
+        }
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+        bool const wild = top != 0 || (bias & 0x7fffu) > 0x7b00u;       // or a bias that is not a finite half of at most 57344
+        found = (__any(wild) ? 1u << layer : 0u) | (__any(sum > kOnePlaneLimit) ? 16u << layer : 0u);
+    } else if (mine) {
+        float const b = fabsf(float(int32_t(bias))), s = fabsf(__builtin_bit_cast(float, scale));
+        found = __any(!((b + 520192.f) * s < 60000.f) || !(b < 2.0e9f)) ? 1u << 8 : 0u;
+    }
+    __syncthreads();
+    if (lane == 0) lds.classFlags[tile] = found;
+    __syncthreads();
+    uint32_t flags = 0;
+#pragma unroll
+    for (int w = 0; w < V::WAVES; ++w) flags |= lds.classFlags[w];
+    flags = __builtin_amdgcn_readfirstlane(flags);
+    int const oneMask = int(~(flags >> 4) & ~flags & 7u);
+    int const modes = int(flags & 7u) | (oneMask << kOnePlaneShift) | ((flags & (1u << 8)) ? 0 : kFp8OutputsBounded);
+    if (((modes & kAllOnePlane) == kAllOnePlane) != V::ONE || !mine) return modes;
+
+    if (layer == 3) {                                        // int8 weights as halves, 32 inputs = one block
+        lds.w3[lane] = make_uint4(halves_of_bytes(v[0], 0), halves_of_bytes(v[0], 2), halves_of_bytes(v[1], 0), halves_of_bytes(v[1], 2));
+        if (kg == 0) { (&lds.outScale[0][0])[i] = __builtin_bit_cast(float, scale); (&lds.outBias[0][0])[i] = int32_t(bias); }
+        return modes;
+    }
+    if (kg == 0) (&lds.bias[0][0][0])[16 * tile + i] = float(__builtin_bit_cast(_Float16, uint16_t(bias)));
+    int32_t w[4][4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) e4m3_times_512(v[d], w[d]);
+#pragma unroll
+    for (int p = 0; p < V::HELD; ++p) {
+        bool const whole = V::ONE || (p == 0 && ((oneMask >> layer) & 1));
+        uint32_t h[4][2];
+#pragma unroll
+        for (int d = 0; d < 4; ++d) { h[d][0] = plane_halves(w[d][0], w[d][1], p, whole); h[d][1] = plane_halves(w[d][2], w[d][3], p, whole); }
+        uint4* const block = layer == 0 ? &lds.w0[p][t][0] : (layer == 1 ? &lds.w1[p][t][0] : &lds.w2[p][t][0]);
+        block[lane] = make_uint4(h[0][0], h[0][1], h[1][0], h[1][1]);
+        if (layer == 1) block[64 + lane] = make_uint4(h[2][0], h[2][1], h[3][0], h[3][1]);
+        else            reinterpret_cast<uint2*>(block + 64)[lane] = make_uint2(h[2][0], h[2][1]);
+    }
+    return modes;
 }
 
 // The positional encoding from the phase table.
@@ -479,40 +482,6 @@ __device__ __forceinline__ void finish_inputs_fast(Mip const& m, Fp8Lds<V> const
     }
     position_from_table<V>(m.posMask, lds, x, y, in);
     in[22] = round_e4m3_pk(halves_rne(m.positionLod, m.positionLod));
-}
-
-// Fills the positional table: one entry per thread, threads 0..62.
-template <class Lds>
-__device__ void build_fp8_posenc_table(Lds& lds)
-{
-    int const t = threadIdx.x;
-    if (t < 63) {
-        int const k = 31 - __builtin_clz(uint32_t(t + 1));   // floor(log2(t + 1))
-        int const phase = t + 1 - (1 << k);
-        float p = float(phase) * __builtin_ldexpf(1.f, -k);
-#pragma unroll
-        for (int w = 0; w < 3; ++w) {
-            float const q = p + 0.25f;
-            float const e0 = (p - floorf(p)) * 2.f - 1.f, e2 = (q - floorf(q)) * 2.f - 1.f;
-            uint32_t const pair = round_e4m3_pk(halves_rne(e0, e2));
-            lds.postab[t][w] = pair & 0xffffu;
-            lds.postab[t][3 + w] = pair >> 16;
-            p *= 2.f;
-        }
-        lds.postab[t][6] = lds.postab[t][7] = 0;
-    }
-}
-
-// Fills the feature table with the same operations the arithmetic path applies per lane.
-template <int THREADS, class Lds>
-__device__ void build_fp8_feature_lut(Lds& lds)
-{
-    for (int e = threadIdx.x; e < 1279; e += THREADS) {
-        int const n = e < 16 ? 0 : (e < 77 ? 2 : (e < 318 ? 4 : 6));
-        int const T = e - kFeatureLutBase(n);
-        float const v = __builtin_fmaf(float(T), __builtin_ldexpf(0.13333334f, -n), -1.f);
-        lds.featureLut[e] = uint16_t(round_e4m3_pk(halves_rne(v, v)));
-    }
 }
 
 // One hidden layer's epilogue for the four channels a lane holds of one texel: sums of the three planes ->
@@ -776,9 +745,6 @@ decode_fp8_kernel(MipTable table, int numMips, int totalTiles, int workgroups, F
     int const tileEnd = min(totalTiles, tileBegin + per);
     if (tileBegin >= tileEnd) return;                        // uniform across the workgroup
 
-    build_fp8_posenc_table(lds);
-    build_fp8_feature_lut<V::THREADS>(lds);
-
     int modes = 7;                                           // uniform: the hidden layers' modes (stage_fp8_weights)
 
     // One wave tile: the 32 x 2 texels of this wave in tile (tileX, tileY) of mip m; block b of 16 texels begins at
@@ -821,15 +787,13 @@ decode_fp8_kernel(MipTable table, int numMips, int totalTiles, int workgroups, F
         entry = table_entry_of(mips, numMips, entry, segBegin);
         uint8_t const* const blob = mips[entry].weights;
         int const segEnd = segment_end(mips, numMips, entry, tileEnd, blob);
-        modes = classify_fp8_weights<V>(lds, blob);
+        modes = __builtin_amdgcn_readfirstlane(stage_fp8_weights<V>(lds, blob, wave * 64 + lane_id(), segBegin == tileBegin));
         if (((modes & kAllOnePlane) == kAllOnePlane) != V::ONE) { // the other instantiation's segment
             if (V::ONE && threadIdx.x == 0) *handoff.word = handoff.serial;
             segBegin = segEnd;
             continue;
         }
-        __syncthreads();                                     // every wave has left the previous segment's weights
-        stage_fp8_weights<V>(lds, blob, modes);
-        __syncthreads();                                     // also publishes the tables built above
+        __syncthreads();
 
         int const part = (segEnd - segBegin + V::GROUP - 1) / V::GROUP;
         int const myBegin = segBegin + member * part, myEnd = min(segEnd, myBegin + part);
@@ -878,14 +842,11 @@ query_fp8_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queri
     int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int const j = lane & 15, g = lane >> 4;
 
-    int const modes = classify_fp8_weights<V>(lds, mips[0].weights);
+    int const modes = __builtin_amdgcn_readfirstlane(stage_fp8_weights<V>(lds, mips[0].weights, wave * 64 + lane_id(), 1));
     if (((modes & kAllOnePlane) == kAllOnePlane) != V::ONE) {            // the other instantiation's set (uniform over the grid)
         if (V::ONE && threadIdx.x == 0) *handoff.word = handoff.serial;
         return;
     }
-    build_fp8_posenc_table(lds);
-    build_fp8_feature_lut<V::THREADS>(lds);
-    stage_fp8_weights<V>(lds, mips[0].weights, modes);
     __syncthreads();
 
     uint64_t const numBlocks = (numQueries + V::THREADS - 1) / V::THREADS;

@@ -157,16 +157,6 @@ struct alignas(16) LdsT : BiasLoT<V::FP8_WEIGHTS, V::NTILES> {
     uint32_t ytab[64][4];             // same for y, one byte up
 };
 
-// Four OCP e4m3 (1-4-3, bias 7, no infinities) bytes -> the integers 512*value (the conversion is exact and so is the
-// product: at most 448 * 512).  The two NaN encodings decode as 0.
-__device__ __forceinline__ void e4m3_times_512(uint32_t bytes, int32_t (&w)[4])
-{
-    v2f const lo = __builtin_amdgcn_cvt_pk_f32_fp8(int(bytes), false), hi = __builtin_amdgcn_cvt_pk_f32_fp8(int(bytes), true);
-    float const f[4] = { lo[0], lo[1], hi[0], hi[1] };
-#pragma unroll
-    for (int r = 0; r < 4; ++r) w[r] = f[r] == f[r] ? int32_t(f[r] * 512.f) : 0;
-}
-
 __device__ __forceinline__ uint32_t halves_of_ints(int a, int b)                   // two integers of at most 11 bits -> two fp16 (exact)
 {
     v2h const h = { _Float16(a), _Float16(b) };
@@ -185,18 +175,6 @@ __device__ __forceinline__ void int8_planes(uint32_t v, uint32_t (&planes)[3])
         planes[1] |= uint32_t((W[r] >> 6) & 63) << (8 * r);
         planes[2] |= (uint32_t(W[r] >> 12) & 0xffu) << (8 * r);
     }
-}
-
-__device__ __forceinline__ uint32_t halves_of_bytes(uint32_t v, int firstByte)     // two int8 -> two fp16 (exact)
-{
-    v2h const h = { _Float16(int(int8_t(v >> (8 * firstByte)))), _Float16(int(int8_t(v >> (8 * firstByte + 8)))) };
-    return __builtin_bit_cast(uint32_t, h);
-}
-
-// The lane's number in its wave from the execution mask: no register has to keep the thread id alive for it.
-__device__ __forceinline__ int lane_id()
-{
-    return int(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
 }
 
 // One byte of the positional encoding (Inference.hlsli:89-113): int(enc * 127.5), truncating.
