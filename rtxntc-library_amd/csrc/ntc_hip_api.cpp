@@ -480,6 +480,8 @@ int grid_size_for(Library const& L, int variant, int totalTiles)
     int const resident = L.computeUnits * workgroups;
     // a workgroup takes tiles_per_round(variant) tiles at a time: fewer workgroups than that leaves waves idle
     int const group = variant_is_fp8_network(variant) ? fp8_tiles_per_round() : tiles_per_round(variant);
+    // - unless there are no more tiles than compute units: then half of the waves idle, but no two share a SIMD
+    if (totalTiles <= L.computeUnits) return totalTiles;
     int64_t const rounds = (int64_t(totalTiles) + group - 1) / group;
     return rounds < resident ? int(rounds) : resident;
 }
