@@ -1267,6 +1267,114 @@ decode_kernel(MipTable table, int numMips, int totalTiles, int workgroups)
     }
 }
 
+// ---- few tiles ----------------------------------------------------------------------------------------
+//
+// Where every wave of the device would get one wave tile at most, the launch takes as long as one wave takes for its 64
+// texels.  These kernels give a wave 16: the same network for one block of texels, without the sections above (they order
+// the work of waves that share a SIMD; here nobody does), the weights staged as above.
+template <class V, int IN_TILES, int OUT_TILES, bool TWO_PLANES>
+__device__ __forceinline__ void f16_layer_of_block(LdsT<V> const& lds, int base, int tileBase, int lane,
+                                                   uint32_t const (&Hin)[4][4][2], uint32_t (&Hout)[4][4][2])
+{
+    constexpr int PLANE = OUT_TILES * V::f16_units(IN_TILES);
+    int const g = lane >> 4;
+#pragma unroll
+    for (int t = 0; t < OUT_TILES; ++t) {
+        v4f const Sc = *reinterpret_cast<v4f const*>(&lds.scale[tileBase + t][g][0]);
+        v4f acc[1] = { *reinterpret_cast<v4f const*>(&lds.bias[tileBase + t][g][0]) };
+        f16_tile<V, IN_TILES, 0, 1>(lds, base, t, lane, Hin, acc);
+        if constexpr (TWO_PLANES) {
+            v4f lo[1] = { *reinterpret_cast<v4f const*>(&lds.biasLo[tileBase + t][g][0]) };
+            f16_tile<V, IN_TILES, 0, 1>(lds, base + PLANE, t, lane, Hin, lo);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[0][r] = __builtin_fmaf(acc[0][r], 1024.f, lo[0][r]);
+        }
+        float z[4];
+        activate_scale4(acc[0], Sc, z);
+        activate_pack4(z, Hout[0][t]);
+    }
+}
+
+template <class V>
+__device__ __forceinline__ void mlp_forward_f16_of_block(LdsT<V> const& lds, int lane, bool l0Magic, v4i X, v4f& D, v4f& S)
+{
+    int const g = lane >> 4;
+    uint32_t Ha[4][4][2], Hb[4][4][2];                       // (the first block of each)
+    float const magic = l0Magic ? 12582912.f : 0.f;          // see first_layer
+#pragma unroll
+    for (int t = 0; t < V::T0; ++t) {
+        auto const operand = [&](int q) {
+            uint4 const w = *reinterpret_cast<uint4 const*>(&lds.w[q][t][lane][0]);
+            return v4i{ int(w.x), int(w.y), int(w.z), int(w.w) };
+        };
+        v4i const C = *reinterpret_cast<v4i const*>(&lds.bias[t][g][0]);
+        v4f const Sc = *reinterpret_cast<v4f const*>(&lds.scale[t][g][0]);
+        v4i Dh = __builtin_amdgcn_mfma_i32_16x16x64_i8(operand(0), X, C, 0, 0, 0);
+        if constexpr (V::FP8_WEIGHTS) {
+            v4i const Z = v4i{ 0, 0, 0, 0 };
+            v4i const D1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(operand(1), X, Z, 0, 0, 0);
+            v4i const D2 = __builtin_amdgcn_mfma_i32_16x16x64_i8(operand(2), X, Z, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)                        // 4096*D2 + 64*D1 + D0, wrapping like int32
+                Dh[r] = int((((uint32_t(D2[r]) << 6) + uint32_t(D1[r])) << 6) + uint32_t(Dh[r]));
+        }
+        v4f acc;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            int32_t const bits = Dh[r];
+            acc[r] = l0Magic ? __builtin_bit_cast(float, bits) - magic : float(bits);
+        }
+        float z[4];
+        activate_scale4(acc, Sc, z);
+        activate_pack4(z, Ha[0][t]);
+    }
+    f16_layer_of_block<V, V::T0, V::T1, V::FP8_WEIGHTS>(lds, V::F16_L1, V::T0, lane, Ha, Hb);
+    f16_layer_of_block<V, V::T1, V::T2, V::FP8_WEIGHTS>(lds, V::F16_L2, V::T0 + V::T1, lane, Hb, Ha);
+    constexpr int outTile = V::T0 + V::T1 + V::T2;
+    S = *reinterpret_cast<v4f const*>(&lds.scale[outTile][g][0]);
+    v4f acc[1] = { *reinterpret_cast<v4f const*>(&lds.bias[outTile][g][0]) };
+    f16_tile<V, V::T2, 0, 1>(lds, V::F16_L3, 0, lane, Ha, acc);
+    D = acc[0];
+}
+
+// A tile in 2^log2Parts workgroups, 16 / 2^log2Parts of the first waves of each take a block of 16 x 1 texels.
+template <class V>
+__global__ void __launch_bounds__(V::THREADS, V::WAVES_PER_SIMD)
+decode_few_kernel(MipTable table, int numMips, int log2Parts)
+{
+    DevMip const* const mips = table_entries(table.entries);
+    __shared__ LdsT<V> lds;
+    int const lane = threadIdx.x & 63;
+    int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int const j = lane & 15, g = lane >> 4;
+    int const tile = int(blockIdx.x >> log2Parts), part = int(blockIdx.x) - (tile << log2Parts);
+    int entry = 0;
+    while (entry + 1 < numMips && mips[entry + 1].tileStart <= tile) ++entry;
+    RunMip const m(mips[entry]);
+    int const staged = __builtin_amdgcn_readfirstlane(stage_weights<V>(lds, m.full.weights, wave * 64 + lane_id(), 1));
+    __syncthreads();
+    if (wave >= 16 >> log2Parts) return;
+    int const block = (part << (4 - log2Parts)) + wave;
+    int const local = tile - m.full.tileStart, tileY = local / m.full.tilesX, tileX = local - tileY * m.full.tilesX;
+    int const x = tileX * 64 + (block & 3) * 16 + j, y = tileY * 4 + (block >> 2);
+    if (x - j >= m.width || y >= m.height) return;           // uniform
+    uint32_t in[16];                                         // four lanes alike per texel
+    if (m.fast) prepare_inputs_fast<V>(m.full, lds, min(x, m.width - 1), y, in);
+    else        prepare_inputs_general<V>(m.full, lds, min(x, m.width - 1), y, in);
+    write_inputs<V>(lds, wave, lane, in);
+    v4i const X = read_input_block<V>(lds, wave, lane, 0);
+    v4f S;
+    if (staged & kStagedF16) {
+        v4f D;
+        mlp_forward_f16_of_block<V>(lds, lane, (staged & kL0Magic) != 0, X, D, S);
+        store_row_any_format(m, D, S, x, y, 4 * g);
+    } else {
+        v4i D;
+        mlp_forward_block<V>(lds, lane, X, D, S);
+        store_row_any_format(m, D, S, x, y, 4 * g);
+    }
+}
+
 // Random-access decode ("inference on sample", NtcSampleTextureSet of Inference.hlsli:282-357):
 // one query = (u, v, mip) -> the 16 outputs of texel (floor(u*W), floor(v*H)) of that mip, clamped to
 // the image, as 16 fp16.  Lane = query in the input stage (each lane carries its own mip, so the
@@ -1423,6 +1531,12 @@ using VCfg3   = Variant<0, 16, 4, 16, 16, 16, 2, 48, 64, 64, 64, true>;   // wid
 template <class V>
 static hipError_t launch_variant(MipTable const& mips, int numMips, int totalTiles, int gridSize, hipStream_t stream)
 {
+    // Up to half as many tiles as compute units: quarter or half tiles, so that hardly two waves share a SIMD (128 x 128:
+    // 7.7 -> 6.3 us, e4m3 weights 12.8 -> 9.2; 256 x 128: 7.8 -> 6.8).  With as many tiles as compute units, two to four
+    // waves would share one, and each would read every weight from LDS for a quarter of the texels: 256 x 256 8.5 us
+    // against 7.9 with whole tiles.
+    int const units = compute_units_of_current_device(), log2Parts = 4 * totalTiles <= units ? 2 : (2 * totalTiles <= units ? 1 : 0);
+    if (log2Parts) return launch_kernel<decode_few_kernel<V>>(dim3(unsigned(totalTiles) << log2Parts), dim3(V::THREADS), 0, stream, mips, numMips, log2Parts);
     return launch_kernel<decode_kernel<V>>(dim3(gridSize), dim3(V::THREADS), 0, stream, mips, numMips, totalTiles, gridSize);
 }
 

@@ -386,6 +386,27 @@ def test_sampling_of_sizes_that_are_no_powers_of_two(ntc, device, network, width
     assert_equal_bytes(expected, got, f"{network} {width}x{height} hr {hr} lr {lr} scale {scale}")
 
 
+@pytest.mark.parametrize("weights", ["fp16 layers", "int8 layers", "converted layer 0"])
+@pytest.mark.parametrize("spec_name", ["spec_cfg01", "spec_cfg3"])
+def test_tile_counts_around_the_compute_units(ntc, device, spec_name, weights):
+    """Quarter, half and whole tiles per workgroup, one and several tiles per workgroup: the counts where the launch
+    changes, with every form of the network, ragged images among them."""
+    spec = getattr(ntc.presets, spec_name)()
+    layout = ntc.synth.weight_layout(spec)
+    blob = ntc.synth.make_weights(spec, 7, scale_log2_range=ACTIVE)
+    bias = blob[layout.biasOffset[0]:layout.bufferSize].view(np.int32)
+    if weights == "int8 layers":
+        bias[70] = 2 ** 31 - 1
+    elif weights == "converted layer 0":
+        bias[5] = 3100001
+    units = device.compute_units
+    for tiles in sorted({1, units // 4, units // 4 + 1, units // 2, units // 2 + 1, units, units + 1, 3 * units + 5}):
+        for width, height in ((64, 4 * tiles), (61, 4 * tiles - 1)):
+            case = cfg_case(ntc, spec, width, height, 1, 5 if tiles & 1 else 16, ntc.abi.OUT_FP16_PLANAR_PAIRS, seed=tiles, weights=blob)
+            expected, got = run_both(device, case)
+            assert_equal_bytes(expected, got, f"{spec_name}, {weights}, {tiles} tiles, {width} x {height}")
+
+
 @pytest.mark.parametrize("channels", [1, 2, 3, 5, 6, 7, 9, 11, 14, 15])
 def test_channel_counts_that_leave_part_of_a_group(ntc, device, channels):
     """Tiles inside the image and at its edges, with one to three channels in the last group of four, pixels packed as
