@@ -3,7 +3,7 @@
 // The step after decode in a load path that hands block-compressed textures to a renderer:
 // the reference runs it as a graphics compute pass (IContext::MakeBlockCompressionComputePass,
 // src/shaders/CompressBC1.hlsl .. CompressBC5.hlsl, src/shaders/BlockCompressCommon.hlsli).
-// One lane encodes one 4 x 4 block, as one thread does there.
+// (One thread encodes a 4 x 4 block there; here waves share the candidates of 64 blocks.)
 //
 // BC4 (one channel; BC5 = two of them, BC3 = one for alpha).  The encoder tries both BC4 palettes.
 // Eight-value palette (endpoint 0 > endpoint 1): start from the
@@ -29,6 +29,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <atomic>
+#include <type_traits>
 #include "ntc_decode_kernel.h"
 #include "ntc_bc_source.h"
 
@@ -180,15 +181,6 @@ __device__ __forceinline__ uint32_t bc4_value8(float texel)
     return uint32_t(rintf(s * 255.f)) << 3;
 }
 
-__device__ uint64_t bc4_encode(float const (&texels)[16])
-{
-    uint32_t values8[16], error8, error6;
-#pragma unroll
-    for (int t = 0; t < 16; ++t) values8[t] = bc4_value8(texels[t]);
-    Bc4 const block8 = bc4_candidate<true>(values8, error8), block6 = bc4_candidate<false>(values8, error6);
-    return error6 < error8 ? block6.bits() : block8.bits();
-}
-
 // Channel `c` of the sixteen texels of block (bx, by), as 8-bit values times eight.
 __device__ __forceinline__ void bc4_load(BlockCompressArgs const& a, int bx, int by, int c, uint32_t (&values8)[16])
 {
@@ -245,7 +237,7 @@ __device__ __forceinline__ uint32_t nearest_pair(int value, int bits)
 struct Rgb { float r, g, b; };
 struct Rgba { float r, g, b, a; };
 
-__device__ __forceinline__ float saturate(float v) { return fminf(fmaxf(v, 0.f), 1.f); }      // a NaN becomes 0
+__device__ __forceinline__ float saturate(float v) { return __builtin_amdgcn_fmed3f(v, 0.f, 1.f); }      // a NaN becomes 0
 __device__ __forceinline__ Rgb rgb_of(Rgba const& p) { return Rgb{ p.r, p.g, p.b }; }
 __device__ __forceinline__ float distance2(Rgb const& a, Rgb const& b)
 {
@@ -256,33 +248,43 @@ __device__ __forceinline__ Rgb mix(Rgb const& a, Rgb const& b, float t)
 {
     return Rgb{ a.r + (b.r - a.r) * t, a.g + (b.g - a.g) * t, a.b + (b.b - a.b) * t };
 }
-__device__ __forceinline__ Rgb expand565(uint32_t w)
+// k / 31 and k / 63: the product with the reciprocal, corrected by its remainder, is the correctly rounded quotient for
+// every k below 64.
+__device__ __forceinline__ float code_quotient(float k, float d, float r)
 {
-    return Rgb{ float((w >> 11) & 31u) / 31.f, float((w >> 5) & 63u) / 63.f, float(w & 31u) / 31.f };
+    float const q = k * r;
+    return __builtin_fmaf(__builtin_fmaf(-q, d, k), r, q);
 }
+__device__ __forceinline__ Rgb of_codes(uint32_t r, uint32_t g, uint32_t b)
+{
+    return Rgb{ code_quotient(float(r), 31.f, 1.f / 31.f), code_quotient(float(g), 63.f, 1.f / 63.f), code_quotient(float(b), 31.f, 1.f / 31.f) };
+}
+__device__ __forceinline__ Rgb expand565(uint32_t w) { return of_codes((w >> 11) & 31u, (w >> 5) & 63u, w & 31u); }
 __device__ __forceinline__ Rgb round565(Rgb const& v, uint32_t& w)
 {
     uint32_t const r = uint32_t(rintf(saturate(v.r) * 31.f)), g = uint32_t(rintf(saturate(v.g) * 63.f)), b = uint32_t(rintf(saturate(v.b) * 31.f));
     w = (r << 11) | (g << 5) | b;
-    return Rgb{ float(r) / 31.f, float(g) / 63.f, float(b) / 31.f };
+    return of_codes(r, g, b);
 }
 
 // Of four distances the smallest; pairs (0, 1) and (2, 3) are compared first, ties go to the later
 // pair and, inside a pair, to its second member (hlsli:116-144).
 __device__ __forceinline__ uint32_t nearest_of_four(float d0, float d1, float d2, float d3, float& error)
 {
-    if (fminf(d0, d1) < fminf(d2, d3)) {
-        if (d0 < d1) { error = d0; return 0; }
-        error = d1; return 1;
-    }
-    if (d2 < d3) { error = d2; return 2; }
-    error = d3; return 3;
+    bool const first = d0 < d1, third = d2 < d3, earlier = min_f32(d0, d1) < min_f32(d2, d3);
+    float const e01 = first ? d0 : d1, e23 = third ? d2 : d3;
+    uint32_t const k01 = first ? 0u : 1u, k23 = third ? 2u : 3u;
+    error = earlier ? e01 : e23;
+    return earlier ? k01 : k23;
 }
 
-// Palette index of a texel in four-colour mode: entries hi, lo, 1/3 and 2/3 of the way from hi to lo.
+// Palette index of a texel in four-colour mode: entries hi, lo, 1/3 and 2/3 of the way from hi to lo.  OPAQUE: the texel's
+// alpha is 1, and 0 need not be added to its distances.
+template <bool OPAQUE>
 __device__ __forceinline__ uint32_t index_of_four(Rgba const& p, Rgb const& hi, Rgb const& lo, float& error)
 {
     Rgb const c = rgb_of(p), third = mix(hi, lo, 1.f / 3.f), twoThirds = mix(hi, lo, 2.f / 3.f);
+    if constexpr (OPAQUE) return nearest_of_four(distance2(hi, c), distance2(lo, c), distance2(third, c), distance2(twoThirds, c), error);
     float const alphaTerm = (1.f - p.a) * (1.f - p.a);
     return nearest_of_four(distance2(hi, c) + alphaTerm, distance2(lo, c) + alphaTerm,
                            distance2(third, c) + alphaTerm, distance2(twoThirds, c) + alphaTerm, error);
@@ -306,7 +308,7 @@ __device__ __forceinline__ uint32_t table_index(float mean)     // values outsid
     return uint32_t(fminf(fmaxf(rintf(mean * 255.f), 0.f), 255.f));
 }
 
-__device__ ColorBlock bc1_single_color(Rgba const (&px)[16])
+__device__ __forceinline__ ColorBlock bc1_single_color(Rgba const (&px)[16])
 {
     Rgb sum{ 0.f, 0.f, 0.f };
 #pragma unroll
@@ -374,15 +376,16 @@ __device__ __forceinline__ Rgb unless_pinned(Rgb const& current, Rgb const& fitt
     return Rgb{ unless_pinned(current.r, fitted.r), unless_pinned(current.g, fitted.g), unless_pinned(current.b, fitted.b) };
 }
 
-__device__ ColorBlock bc1_four_colors(Rgba const (&px)[16])
+template <bool OPAQUE>
+__device__ __forceinline__ ColorBlock bc1_four_colors(Rgba const (&px)[16])
 {
     Rgb sum{ 0.f, 0.f, 0.f };
     Box box{ Rgb{ 1.f, 1.f, 1.f }, Rgb{ 0.f, 0.f, 0.f } };
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
         sum.r += px[t].r; sum.g += px[t].g; sum.b += px[t].b;
-        box.lo = Rgb{ fminf(box.lo.r, px[t].r), fminf(box.lo.g, px[t].g), fminf(box.lo.b, px[t].b) };
-        box.hi = Rgb{ fmaxf(box.hi.r, px[t].r), fmaxf(box.hi.g, px[t].g), fmaxf(box.hi.b, px[t].b) };
+        box.lo = Rgb{ min_f32(box.lo.r, px[t].r), min_f32(box.lo.g, px[t].g), min_f32(box.lo.b, px[t].b) };
+        box.hi = Rgb{ max_f32(box.hi.r, px[t].r), max_f32(box.hi.g, px[t].g), max_f32(box.hi.b, px[t].b) };
     }
     Rgb const center{ sum.r / 16.f, sum.g / 16.f, sum.b / 16.f };
     float covRG = 0.f, covRB = 0.f, covGB = 0.f;
@@ -394,15 +397,15 @@ __device__ ColorBlock bc1_four_colors(Rgba const (&px)[16])
     orient_and_inset(box, covRG, covRB, covGB, 16.f);
 
     uint32_t c0 = 0, c1 = 0;
+#pragma unroll 1
     for (int round = 0; round < 4; ++round) {
         Fit fit;
 #pragma unroll
         for (int t = 0; t < 16; ++t) {
             float unused;
-            uint32_t const k = index_of_four(px[t], box.hi, box.lo, unused);
-            float beta = float(k & 1u);
-            if (k & 2u) beta = (1.f + beta) / 3.f;
-            fit.add(beta, px[t]);
+            uint32_t const k = index_of_four<OPAQUE>(px[t], box.hi, box.lo, unused);
+            // (selected, not divided: 1/3 and 2/3 rounded)
+            fit.add((k & 2u) ? ((k & 1u) ? 2.f / 3.f : 1.f / 3.f) : float(k & 1u), px[t]);
         }
         Rgb A, B;
         if (fit.solve(A, B)) {
@@ -427,13 +430,13 @@ __device__ ColorBlock bc1_four_colors(Rgba const (&px)[16])
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
         float e;
-        out.indices |= index_of_four(px[t], box.hi, box.lo, e) << (2 * t);
+        out.indices |= index_of_four<OPAQUE>(px[t], box.hi, box.lo, e) << (2 * t);
         out.error += e;
     }
     return out;
 }
 
-__device__ ColorBlock bc1_three_colors(Rgba const (&px)[16], float alphaThreshold)
+__device__ __forceinline__ ColorBlock bc1_three_colors(Rgba const (&px)[16], float alphaThreshold)
 {
     Rgb sum{ 0.f, 0.f, 0.f };
     Box box{ Rgb{ 1.f, 1.f, 1.f }, Rgb{ 0.f, 0.f, 0.f } };
@@ -442,8 +445,8 @@ __device__ ColorBlock bc1_three_colors(Rgba const (&px)[16], float alphaThreshol
     for (int t = 0; t < 16; ++t)
         if (!(px[t].a <= alphaThreshold)) {
             sum.r += px[t].r; sum.g += px[t].g; sum.b += px[t].b;
-            box.lo = Rgb{ fminf(box.lo.r, px[t].r), fminf(box.lo.g, px[t].g), fminf(box.lo.b, px[t].b) };
-            box.hi = Rgb{ fmaxf(box.hi.r, px[t].r), fmaxf(box.hi.g, px[t].g), fmaxf(box.hi.b, px[t].b) };
+            box.lo = Rgb{ min_f32(box.lo.r, px[t].r), min_f32(box.lo.g, px[t].g), min_f32(box.lo.b, px[t].b) };
+            box.hi = Rgb{ max_f32(box.hi.r, px[t].r), max_f32(box.hi.g, px[t].g), max_f32(box.hi.b, px[t].b) };
             ++opaque;
         }
     float const count = float(opaque);
@@ -487,24 +490,19 @@ __device__ ColorBlock bc1_three_colors(Rgba const (&px)[16], float alphaThreshol
     return out;
 }
 
-// Colour block of BC1 (withAlpha: the transparent and three-colour candidates take part) or of BC2 / BC3.
-__device__ __forceinline__ uint64_t bc1_encode(Rgba const (&px)[16], bool withAlpha, float alphaThreshold)
+// The candidates without rounds of refinement: one colour and (BC1) all transparent.
+template <bool TRANSPARENT>
+__device__ __forceinline__ ColorBlock bc1_simple_candidates(Rgba const (&px)[16], float alphaThreshold)
 {
     ColorBlock best = bc1_single_color(px);
-    if (withAlpha) {
+    if constexpr (TRANSPARENT) {
         float transparentError = 0.f;
 #pragma unroll
         for (int t = 0; t < 16; ++t)
             if (!(px[t].a <= alphaThreshold)) transparentError += px[t].r * px[t].r + px[t].g * px[t].g + px[t].b * px[t].b + px[t].a * px[t].a;
         if (!(best.error < transparentError)) best = ColorBlock{ 0u, 0xffffffffu, transparentError };
     }
-    ColorBlock const four = bc1_four_colors(px);
-    if (four.error < best.error) best = four;
-    if (withAlpha) {
-        ColorBlock const three = bc1_three_colors(px, alphaThreshold);
-        if (three.error < best.error) best = three;
-    }
-    return uint64_t(best.endpoints) | (uint64_t(best.indices) << 32);
+    return best;
 }
 
 // BC2 alpha: 4 bits per texel, texel 0 in the lowest bits.
@@ -552,10 +550,130 @@ bc4_compress_kernel(BlockCompressArgs a)
     reinterpret_cast<uint64_t*>(a.dst + size_t(by + a.dstOffsetY) * a.dstRowPitch)[size_t(bx + a.dstOffsetX) * CHANNELS + channel] = mine.bits();
 }
 
-// BC1 (8 bytes per block), BC2 and BC3 (alpha block, then colour block).  At least three waves per SIMD: the BC1
-// instance would otherwise take 203 registers and run two (4096^2: 0.22 ms with two, 0.19 ms with three, 0.26 ms with four).
+// BC1 (8 bytes per block), BC2 and BC3 (alpha block, then colour block), bound by vector instructions: a block's
+// candidates are chains of passes over its texels.
+//
+// bc1_compress_split_kernel: the waves of a workgroup encode the same 64 blocks (16 x 4), a candidate each, and leave what
+// they found in LDS for the first to choose from: that one refines the four-colour endpoints, up to five passes and the
+// longest by far; the second takes the simple candidates and, BC1, the three-colour one, BC2, the alpha, BC3, the
+// six-value alpha palette; BC3's third wave the eight-value one.  A wave waits for the first one's end, so this is for
+// images that do not fill the device anyway.
+// bc1_compress_kernel: a lane per block, all candidates one after the other.
+//
+// 64 x 64 and 1024 x 1024: BC1 27 and 29 us in one lane before, 15 and 16 split; BC2 19 and 20, 15 and 15; BC3 25 and 33,
+// 15 and 19.  2048 x 2048: BC1 58 before, 51 (two waves per SIMD with everything in registers; 82 with three that spill; 55
+// split); BC2 38, 34 (47 split); BC3 61, 52 (72 split).  Thirds are selected and not divided, and k / 31 is a product.
+struct Bc1Exchange { float4 texels[16][64]; uint32_t words[6][64]; uint64_t alpha[64]; uint32_t sixError[64]; };
+template <int FORMAT> constexpr int kBc1Waves = FORMAT == 3 ? 3 : 2;
+
 template <int FORMAT>
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(3)))
+__device__ __forceinline__ ColorBlock bc1_refined_candidate(Rgba const (&px)[16])
+{
+    if constexpr (FORMAT != 1) return bc1_four_colors<true>(px);
+    bool opaque = true;
+#pragma unroll
+    for (int t = 0; t < 16; ++t) opaque = opaque && px[t].a == 1.f;
+    return __all(opaque) ? bc1_four_colors<true>(px) : bc1_four_colors<false>(px);     // (of the active lanes)
+}
+
+// The colour word, and in front of it the alpha word of BC2 and BC3.
+template <int FORMAT>
+__device__ __forceinline__ uint64_t* bc1_place(BlockCompressArgs const& a, int bx, int by)
+{
+    constexpr int WORDS = FORMAT == 1 ? 1 : 2;
+    return reinterpret_cast<uint64_t*>(a.dst + size_t(by + a.dstOffsetY) * a.dstRowPitch) + size_t(bx + a.dstOffsetX) * WORDS;
+}
+
+template <int FORMAT>
+__global__ void __launch_bounds__(64 * kBc1Waves<FORMAT>) __attribute__((amdgpu_waves_per_eu(4)))
+bc1_compress_split_kernel(BlockCompressArgs a)
+{
+    __shared__ Bc1Exchange exchange;
+    int const wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63;
+    int const bx = blockIdx.x * 16 + (lane & 15), by = blockIdx.y * 4 + (lane >> 4);
+    bool const inside = bx < a.widthInBlocks && by < a.heightInBlocks;
+    int const x0 = a.srcLeft + bx * 4, y0 = a.srcTop + by * 4;
+    if (inside) {
+        auto const store = [&](int t, auto packed) {
+            float c[4];
+            if constexpr (decltype(packed)::value) source_packed_pixel(a, x0 + (t & 3), y0 + (t >> 2), c);
+            else                                   source_pixel(a, x0 + (t & 3), y0 + (t >> 2), c);
+            exchange.texels[t][lane] = make_float4(c[0], c[1], c[2], c[3]);
+        };
+        if (a.packedRgba8) {                                 // uniform: one load a texel, all in flight
+#pragma unroll
+            for (int k = 0; k < (16 + kBc1Waves<FORMAT> - 1) / kBc1Waves<FORMAT>; ++k)
+                if (wave + k * kBc1Waves<FORMAT> < 16) store(wave + k * kBc1Waves<FORMAT>, std::true_type{});
+        } else {
+#pragma unroll 2
+            for (int t = wave; t < 16; t += kBc1Waves<FORMAT>) store(t, std::false_type{});
+        }
+    }
+    __syncthreads();
+    auto const alpha_candidate = [&](auto eight, uint32_t& error) {
+        uint32_t values8[16];
+#pragma unroll
+        for (int t = 0; t < 16; ++t) values8[t] = bc4_value8(exchange.texels[t][lane].w);
+        return bc4_candidate<decltype(eight)::value>(values8, error);
+    };
+    ColorBlock best{ 0u, 0u, 0.f };
+    Bc4 alphaBlock{ 0u, 0u, 0u, 0u };
+    uint32_t alphaError = 0;
+    if (inside) {
+        if (wave == 2) {
+            alphaBlock = alpha_candidate(std::true_type{}, alphaError);
+        } else {
+            Rgba px[16];
+#pragma unroll
+            for (int t = 0; t < 16; ++t) {
+                float4 const v = exchange.texels[t][lane];
+                px[t] = Rgba{ v.x, v.y, v.z, FORMAT == 1 ? v.w : 1.f };
+            }
+            if (wave == 0) {
+                best = bc1_refined_candidate<FORMAT>(px);
+            } else {
+                ColorBlock const simple = bc1_simple_candidates<FORMAT == 1>(px, a.alphaThreshold);
+                exchange.words[0][lane] = simple.endpoints; exchange.words[1][lane] = simple.indices; exchange.words[2][lane] = __float_as_uint(simple.error);
+                if constexpr (FORMAT == 1) {
+                    ColorBlock const three = bc1_three_colors(px, a.alphaThreshold);
+                    exchange.words[3][lane] = three.endpoints; exchange.words[4][lane] = three.indices; exchange.words[5][lane] = __float_as_uint(three.error);
+                } else if constexpr (FORMAT == 2) {
+                    float alpha[16];
+#pragma unroll
+                    for (int t = 0; t < 16; ++t) alpha[t] = exchange.texels[t][lane].w;
+                    exchange.alpha[lane] = bc2_alpha(alpha);
+                } else {
+                    alphaBlock = alpha_candidate(std::false_type{}, alphaError);
+                    exchange.alpha[lane] = alphaBlock.bits();
+                    exchange.sixError[lane] = alphaError;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    if (!inside || wave == 1) return;
+    uint64_t* const dst = bc1_place<FORMAT>(a, bx, by);
+    if (wave == 2) {
+        dst[0] = exchange.sixError[lane] < alphaError ? exchange.alpha[lane] : alphaBlock.bits();
+        return;
+    }
+    ColorBlock chosen{ exchange.words[0][lane], exchange.words[1][lane], __uint_as_float(exchange.words[2][lane]) };
+    if (best.error < chosen.error) chosen = best;
+    if constexpr (FORMAT == 1) {
+        float const error = __uint_as_float(exchange.words[5][lane]);
+        if (error < chosen.error) chosen = ColorBlock{ exchange.words[3][lane], exchange.words[4][lane], error };
+    }
+    uint64_t const color = uint64_t(chosen.endpoints) | (uint64_t(chosen.indices) << 32);
+    if constexpr (FORMAT == 1) {
+        dst[0] = color;
+    } else {
+        if constexpr (FORMAT == 2) dst[0] = exchange.alpha[lane];
+        dst[1] = color;
+    }
+}
+
+template <int FORMAT>
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(FORMAT == 1 ? 2 : 4)))
 bc1_compress_kernel(BlockCompressArgs a)
 {
     int const bx = blockIdx.x * 16 + (threadIdx.x & 15), by = blockIdx.y * 8 + (threadIdx.x >> 4);
@@ -564,20 +682,39 @@ bc1_compress_kernel(BlockCompressArgs a)
     float alpha[16];
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
-        int const x = a.srcLeft + bx * 4 + (t & 3), y = a.srcTop + by * 4 + (t >> 2);
         float c[4];
-        source_pixel(a, x, y, c);
-        px[t] = Rgba{ c[0], c[1], c[2], c[3] };
-        if constexpr (FORMAT != 1) { alpha[t] = px[t].a; px[t].a = 1.f; }
+        source_pixel(a, a.srcLeft + bx * 4 + (t & 3), a.srcTop + by * 4 + (t >> 2), c);
+        px[t] = Rgba{ c[0], c[1], c[2], FORMAT == 1 ? c[3] : 1.f };
+        alpha[t] = c[3];
     }
-    uint64_t const color = bc1_encode(px, FORMAT == 1, a.alphaThreshold);
-    constexpr int WORDS = FORMAT == 1 ? 1 : 2;
-    uint64_t* const dst = reinterpret_cast<uint64_t*>(a.dst + size_t(by + a.dstOffsetY) * a.dstRowPitch) + size_t(bx + a.dstOffsetX) * WORDS;
-    if constexpr (FORMAT == 1) dst[0] = color;
-    else {
-        dst[0] = FORMAT == 2 ? bc2_alpha(alpha) : bc4_encode(alpha);
-        dst[1] = color;
+    uint64_t* const dst = bc1_place<FORMAT>(a, bx, by);
+    if constexpr (FORMAT == 2) dst[0] = bc2_alpha(alpha);
+    if constexpr (FORMAT == 3) {
+        uint32_t values8[16], error8, error6;
+#pragma unroll
+        for (int t = 0; t < 16; ++t) values8[t] = bc4_value8(alpha[t]);
+        Bc4 const block8 = bc4_candidate<true>(values8, error8), block6 = bc4_candidate<false>(values8, error6);
+        dst[0] = error6 < error8 ? block6.bits() : block8.bits();
     }
+    ColorBlock best = bc1_simple_candidates<FORMAT == 1>(px, a.alphaThreshold);
+    ColorBlock const four = bc1_four_colors<FORMAT != 1>(px);
+    if (four.error < best.error) best = four;
+    if constexpr (FORMAT == 1) {
+        ColorBlock const three = bc1_three_colors(px, a.alphaThreshold);
+        if (three.error < best.error) best = three;
+    }
+    dst[FORMAT == 1 ? 0 : 1] = uint64_t(best.endpoints) | (uint64_t(best.indices) << 32);
+}
+
+template <int FORMAT>
+static void launch_bc1(BlockCompressArgs const& a, hipStream_t stream)
+{
+    unsigned const x = unsigned(a.widthInBlocks + 15) / 16, y = unsigned(a.heightInBlocks + 3) / 4;
+    // (BC3: split 19 us with four workgroups per compute unit, 42 with eight; unsplit 29 with either)
+    if (uint64_t(x) * y <= 5u * uint64_t(compute_units_of_current_device()))
+        hipLaunchKernelGGL(bc1_compress_split_kernel<FORMAT>, dim3(x, y), dim3(64 * kBc1Waves<FORMAT>), 0, stream, a);
+    else
+        hipLaunchKernelGGL(bc1_compress_kernel<FORMAT>, dim3(x, unsigned(a.heightInBlocks + 7) / 8), dim3(128), 0, stream, a);
 }
 
 __global__ void __launch_bounds__(256)
@@ -589,7 +726,7 @@ bc1_tables_kernel()
 
 hipError_t launch_block_compress(BlockCompressArgs const& a, int dstFormat, hipStream_t stream)
 {
-    dim3 const grid((a.widthInBlocks + 15) / 16, (a.heightInBlocks + 7) / 8);
+    dim3 const grid((a.widthInBlocks + 15) / 16, (a.heightInBlocks + 3) / 4);
     if (dstFormat <= 3) {
         // the single-colour tables are computed on the device the first time each device needs them
         // (every launch of the library is on one stream per device, so the order is given)
@@ -604,11 +741,11 @@ hipError_t launch_block_compress(BlockCompressArgs const& a, int dstFormat, hipS
         }
     }
     switch (dstFormat) {
-    case 1: hipLaunchKernelGGL(bc1_compress_kernel<1>, grid, dim3(128), 0, stream, a); break;
-    case 2: hipLaunchKernelGGL(bc1_compress_kernel<2>, grid, dim3(128), 0, stream, a); break;
-    case 3: hipLaunchKernelGGL(bc1_compress_kernel<3>, grid, dim3(128), 0, stream, a); break;
-    case 4: hipLaunchKernelGGL(bc4_compress_kernel<1>, grid, dim3(256), 0, stream, a); break;
-    case 5: hipLaunchKernelGGL(bc4_compress_kernel<2>, dim3(grid.x, (a.heightInBlocks + 3) / 4), dim3(256), 0, stream, a); break;
+    case 1: launch_bc1<1>(a, stream); break;
+    case 2: launch_bc1<2>(a, stream); break;
+    case 3: launch_bc1<3>(a, stream); break;
+    case 4: hipLaunchKernelGGL(bc4_compress_kernel<1>, dim3(grid.x, (a.heightInBlocks + 7) / 8), dim3(256), 0, stream, a); break;
+    case 5: hipLaunchKernelGGL(bc4_compress_kernel<2>, grid, dim3(256), 0, stream, a); break;
     case 6: return launch_bc6_compress(a, stream);
     case 7: return launch_bc7_compress(a, stream);
     default: return hipErrorInvalidValue;

@@ -48,14 +48,18 @@ __device__ __forceinline__ float source_channel(BlockCompressArgs const& a, int 
 
 // All four channels of a pixel.  The common source, four UNORM8 channels with every pixel on a 4-byte
 // boundary (args.packedRgba8, set by the host), takes one 32-bit load per pixel.
+__device__ __forceinline__ void source_packed_pixel(BlockCompressArgs const& a, int x, int y, float (&rgba)[4])
+{
+    uint32_t v = 0;
+    if (x >= 0 && y >= 0 && x < a.srcWidth && y < a.srcHeight)
+        v = *reinterpret_cast<uint32_t const*>(a.src + size_t(y) * a.rowPitch + size_t(x) * a.pixelStride);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) rgba[c] = unorm_quotient(float((v >> (8 * c)) & 0xffu), 255.f, 1.f / 255.f);
+}
 __device__ __forceinline__ void source_pixel(BlockCompressArgs const& a, int x, int y, float (&rgba)[4])
 {
     if (a.packedRgba8) {
-        uint32_t v = 0;
-        if (x >= 0 && y >= 0 && x < a.srcWidth && y < a.srcHeight)
-            v = *reinterpret_cast<uint32_t const*>(a.src + size_t(y) * a.rowPitch + size_t(x) * a.pixelStride);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) rgba[c] = unorm_quotient(float((v >> (8 * c)) & 0xffu), 255.f, 1.f / 255.f);
+        source_packed_pixel(a, x, y, rgba);
     } else {
 #pragma unroll
         for (int c = 0; c < 4; ++c) rgba[c] = source_channel(a, x, y, c);

@@ -312,3 +312,26 @@ def test_gpu_colour_block_compress_three_channel_source_and_arguments(ntc, devic
     p.dstFormat, p.dstBytes, p.dstRowPitch = 1, 12 * 8 * 8, 12 * 8
     ntc.abi.check(device.lib.ntc_hip_block_compress(p))
     device.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", [1, 4])
+@pytest.mark.parametrize("dst_format", [1, 2, 3])
+def test_gpu_colour_blocks_either_side_of_the_split(ntc, device, oracle, fmt, dst_format):
+    """As many blocks as waves still share, a row more, and one block; opaque and transparent regions."""
+    rng = np.random.default_rng(30 * fmt + dst_format)
+    bx, by = 320, device.compute_units                       # 5 * compute units groups of 16 x 4 blocks
+    h, w = 4 * by + 4, 4 * bx
+    image = rng.random((h // 8 + 1, w // 8, 4)).repeat(8, 0).repeat(8, 1)[:h] + rng.normal(0, 0.08, (h, w, 4))
+    image[:, : w // 2, 3] = 1.0
+    image[:, w // 2:, 3] = np.where(rng.random((h, w - w // 2)) < 0.3, 0.0, image[:, w // 2:, 3])
+    if fmt == 1:
+        image = np.clip(np.rint(image * 255), 0, 255).astype(np.uint8)
+    else:
+        image = image.astype(np.float32)
+        image[9, 9, 1], image[17, w - 5, 3], image[33, 40, 0] = np.nan, np.nan, np.inf
+    want = compress(ntc, oracle, None, image, fmt, 4, dst_format, bx, by + 1)
+    for rows in (by, by + 1):
+        got = compress(ntc, None, device, image, fmt, 4, dst_format, bx, rows)
+        assert np.array_equal(got, want[:rows]), (rows, np.argwhere(got != want[:rows])[:3])
+    assert np.array_equal(compress(ntc, None, device, image, fmt, 4, dst_format, 1, 1), want[:1, : 1 if dst_format == 1 else 2])
