@@ -1375,6 +1375,49 @@ decode_few_kernel(MipTable table, int numMips, int log2Parts)
     }
 }
 
+// The fields of the mips that queries need, into LDS (threads 0 ... 15).
+__device__ __forceinline__ void load_query_mips(QueryMip (&qmips)[16], DevMip const* mips, int numMips)
+{
+    if (threadIdx.x >= 16) return;
+    DevMip const& d = mips[min(int(threadIdx.x), numMips - 1)];
+    QueryMip& q = qmips[threadIdx.x];
+    q.hr = d.hr; q.lr = d.lr;
+    q.hrAxisX = d.hrAxisX; q.hrAxisY = d.hrAxisY; q.lrAxisX = d.lrAxisX; q.lrAxisY = d.lrAxisY;
+    q.hrWidth = d.hrWidth; q.hrHeight = d.hrHeight; q.lrWidth = d.lrWidth; q.lrHeight = d.lrHeight;
+    q.width = d.width; q.height = d.height;
+    q.posMask = d.posMask; q.fast = d.fast; q.positionLod = d.positionLod;
+    q.hrBricks = d.hrBricks; q.lrBricks = d.lrBricks;
+}
+
+// The input vector of a lane's query.  Returns whether its mip exists (mip 0's inputs otherwise).
+template <class V>
+__device__ __forceinline__ bool prepare_query_inputs(DevMip const* mips, QueryMip const (&qmips)[16], int numMips, bool bricked, LdsT<V> const& lds,
+                                                     DevQuery const& query, uint32_t (&in)[16])
+{
+    bool const validMip = query.mip >= 0 && query.mip < numMips;
+    QueryMip const& m = qmips[validMip ? query.mip : 0];
+    int x = int(floorf(query.u * float(m.width)));
+    int y = int(floorf(query.v * float(m.height)));
+    x = max(0, min(x, m.width - 1));
+    y = max(0, min(y, m.height - 1));
+    if (__all(m.fast != 0)) {                                // every lane's mip is power-of-two sized
+        if (bricked) prepare_inputs_bricked<V>(m, lds, x, y, in);
+        else         prepare_inputs_scattered<V>(m, lds, x, y, (GlobalU8Ptr)mips, in);
+    } else {
+        prepare_inputs_general<V>(mips[validMip ? query.mip : 0], lds, x, y, in);
+    }
+    return validMip;
+}
+
+template <bool CHECKED>
+__device__ __forceinline__ void store_query_outputs(uint16_t* out, v4f F, v4f S, bool valid)
+{
+    uint32_t h01 = to_half2_bits<CHECKED>(F[0] * S[0], F[1] * S[1]);
+    uint32_t h23 = to_half2_bits<CHECKED>(F[2] * S[2], F[3] * S[3]);
+    if (!valid) { h01 = 0; h23 = 0; }
+    *reinterpret_cast<u32x2*>(out) = u32x2{ h01, h23 };
+}
+
 // Random-access decode ("inference on sample", NtcSampleTextureSet of Inference.hlsli:282-357):
 // one query = (u, v, mip) -> the 16 outputs of texel (floor(u*W), floor(v*H)) of that mip, clamped to
 // the image, as 16 fp16.  Lane = query in the input stage (each lane carries its own mip, so the
@@ -1383,60 +1426,35 @@ decode_few_kernel(MipTable table, int numMips, int log2Parts)
 template <class V>
 __global__ void __launch_bounds__(V::THREADS, V::WAVES_PER_SIMD)
 query_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queries, uint64_t numQueries,
-             uint16_t* __restrict__ out, int workgroups)
+             uint16_t* __restrict__ out, int workgroups, int waves)
 {
     DevMip const* const mips = table_entries(table.entries);
     __shared__ LdsT<V> lds;
     __shared__ QueryMip qmips[16];
-    if (threadIdx.x < 16) {
-        DevMip const& d = mips[min(int(threadIdx.x), numMips - 1)];
-        QueryMip& q = qmips[threadIdx.x];
-        q.hr = d.hr; q.lr = d.lr;
-        q.hrAxisX = d.hrAxisX; q.hrAxisY = d.hrAxisY; q.lrAxisX = d.lrAxisX; q.lrAxisY = d.lrAxisY;
-        q.hrWidth = d.hrWidth; q.hrHeight = d.hrHeight; q.lrWidth = d.lrWidth; q.lrHeight = d.lrHeight;
-        q.width = d.width; q.height = d.height;
-        q.posMask = d.posMask; q.fast = d.fast; q.positionLod = d.positionLod;
-        q.hrBricks = d.hrBricks; q.lrBricks = d.lrBricks;
-    }
+    load_query_mips(qmips, mips, numMips);
     bool const bricked = mips[0].hrBricks != nullptr;          // a set has the query-ordered copy for all of its mips or for none
     int const lane = threadIdx.x & 63;
     int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int const j = lane & 15, g = lane >> 4;
 
-
     int const staged = __builtin_amdgcn_readfirstlane(stage_weights<V>(lds, mips[0].weights, wave * 64 + lane_id(), 1));
     bool const useF16 = (staged & kStagedF16) != 0;
     __syncthreads();
 
-    uint64_t const numBlocks = (numQueries + V::THREADS - 1) / V::THREADS;
+    uint32_t const perBlock = uint32_t(waves) * 64u;
+    uint64_t const numBlocks = (numQueries + perBlock - 1) / perBlock;
     for (uint64_t block = blockIdx.x; block < numBlocks; block += uint32_t(workgroups)) {
-        uint64_t const q0 = block * V::THREADS + uint64_t(wave) * 64;
-        if (q0 >= numQueries) continue;
-        uint64_t const qi = min(q0 + uint64_t(lane), numQueries - 1);
-        DevQuery const query = queries[qi];
-        bool const validMip = query.mip >= 0 && query.mip < numMips;
-        QueryMip const& m = qmips[validMip ? query.mip : 0];
-        int x = int(floorf(query.u * float(m.width)));
-        int y = int(floorf(query.v * float(m.height)));
-        x = max(0, min(x, m.width - 1));
-        y = max(0, min(y, m.height - 1));
+        uint64_t const q0 = block * perBlock + uint64_t(wave) * 64;
+        if (q0 >= numQueries || wave >= waves) continue;
         uint32_t in[16];
-        if (__all(m.fast != 0)) {                                // every lane's mip is power-of-two sized
-            if (bricked) prepare_inputs_bricked<V>(m, lds, x, y, in);
-            else         prepare_inputs_scattered<V>(m, lds, x, y, (GlobalU8Ptr)mips, in);
-        }
-        else                    prepare_inputs_general<V>(mips[validMip ? query.mip : 0], lds, x, y, in);
+        bool const validMip = prepare_query_inputs<V>(mips, qmips, numMips, bricked, lds, queries[min(q0 + uint64_t(lane), numQueries - 1)], in);
 
         // lane (j, g) holds channels 4g..4g+3 of query q0 + 16b + j; validity travels by shuffle
         auto store_outputs = [&](auto checked, int b, v4f Fb, v4f S) __attribute__((always_inline)) {
             constexpr bool CHECKED = decltype(checked)::value;
             uint64_t const q = q0 + uint64_t(16 * b + j);
             int const ok = __shfl(validMip ? 1 : 0, 16 * b + j, 64);
-            if (q >= numQueries) return;
-            uint32_t h01 = to_half2_bits<CHECKED>(Fb[0] * S[0], Fb[1] * S[1]);
-            uint32_t h23 = to_half2_bits<CHECKED>(Fb[2] * S[2], Fb[3] * S[3]);
-            if (!ok) { h01 = 0; h23 = 0; }
-            *reinterpret_cast<u32x2*>(out + q * 16 + 4 * g) = u32x2{ h01, h23 };
+            if (q < numQueries) store_query_outputs<CHECKED>(out + q * 16 + 4 * g, Fb, S, ok != 0);
         };
         if (V::F16_LAYERS && useF16) {
             // output-layer accumulators as floats: exact integers below 2^24
@@ -1467,6 +1485,37 @@ query_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queries, 
             __builtin_amdgcn_wave_barrier();
         }
     }
+}
+
+// Few queries: sixteen per wave, as decode_few_kernel does with texels.
+template <class V>
+__global__ void __launch_bounds__(V::THREADS, V::WAVES_PER_SIMD)
+query_few_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queries, uint64_t numQueries, uint16_t* __restrict__ out)
+{
+    DevMip const* const mips = table_entries(table.entries);
+    __shared__ LdsT<V> lds;
+    __shared__ QueryMip qmips[16];
+    load_query_mips(qmips, mips, numMips);
+    int const lane = threadIdx.x & 63;
+    int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int const j = lane & 15, g = lane >> 4;
+    int const staged = __builtin_amdgcn_readfirstlane(stage_weights<V>(lds, mips[0].weights, wave * 64 + lane_id(), 1));
+    __syncthreads();
+    uint64_t const q0 = (uint64_t(blockIdx.x) * V::WAVES + uint64_t(wave)) * 16, q = q0 + uint64_t(j);
+    if (q0 >= numQueries) return;                            // uniform
+    uint32_t in[16];                                         // four lanes alike per query
+    bool const valid = prepare_query_inputs<V>(mips, qmips, numMips, mips[0].hrBricks != nullptr, lds, queries[min(q, numQueries - 1)], in);
+    write_inputs<V>(lds, wave, lane, in);
+    v4i const X = read_input_block<V>(lds, wave, lane, 0);
+    v4f F, S;
+    if (staged & kStagedF16) {
+        mlp_forward_f16_of_block<V>(lds, lane, (staged & kL0Magic) != 0, X, F, S);
+    } else {
+        v4i D;
+        mlp_forward_block<V>(lds, lane, X, D, S);
+        F = v4f{ float(D[0]), float(D[1]), float(D[2]), float(D[3]) };
+    }
+    if (q < numQueries) store_query_outputs<true>(out + q * 16 + 4 * g, F, S, valid);
 }
 
 // 16x64 by 64x16 int8 product with the operand layout the decode kernel assumes.
@@ -1558,7 +1607,14 @@ template <class V>
 static hipError_t launch_query_variant(MipTable const& mips, int numMips, DevQuery const* queries, uint64_t numQueries,
                                        uint16_t* out, int gridSize, hipStream_t stream)
 {
-    return launch_kernel<query_kernel<V>>(dim3(gridSize), dim3(V::THREADS), 0, stream, mips, numMips, queries, numQueries, out, gridSize);
+    // Up to as many workgroups of 16 queries per wave as compute units; up to half as many of 64, four of the eight waves
+    // do the work, so that no two share a SIMD (16000 queries: 15.5 us, 7.4 now, the staging of the weights included;
+    // 65536: 15.6, 8.4).
+    int const units = compute_units_of_current_device();
+    uint64_t const few = (numQueries + 16 * V::WAVES - 1) / (16 * V::WAVES);
+    if (few <= uint64_t(units)) return launch_kernel<query_few_kernel<V>>(dim3(unsigned(few)), dim3(V::THREADS), 0, stream, mips, numMips, queries, numQueries, out);
+    if (2 * gridSize <= units) return launch_kernel<query_kernel<V>>(dim3(2 * gridSize), dim3(V::THREADS), 0, stream, mips, numMips, queries, numQueries, out, 2 * gridSize, V::WAVES / 2);
+    return launch_kernel<query_kernel<V>>(dim3(gridSize), dim3(V::THREADS), 0, stream, mips, numMips, queries, numQueries, out, gridSize, V::WAVES);
 }
 
 // Plain grid ([layer][row][column] u16) -> bricks; one thread per stored u16, reads coalesced.

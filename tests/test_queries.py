@@ -127,3 +127,41 @@ def test_gpu_queries_from_query_ordered_latents(ntc, device, oracle, kind):
     assert device.lib.ntc_hip_decode_queries(dset, d_q.ptr, n, d_out.ptr, d_out.nbytes) == A.ERR_INVALID_ARG
     assert device.lib.ntc_hip_build_query_latents(dset, d_bricks.ptr, need - 1) == A.ERR_INVALID_ARG
     device.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["cfg01", "ref8-odd", "cfg3 int8 layers", "fp8_8"])
+def test_gpu_query_counts_around_the_compute_units(ntc, device, oracle, kind):
+    """The counts where the launch gives a wave more queries, a workgroup more waves, or a second round, with and without
+    the query-ordered copy and in the int8 form of the layers."""
+    A, P = ntc.abi, ntc.presets
+    if kind == "cfg01":
+        case = cfg_case(ntc, P.spec_cfg01(), 512, 256, 10, 16, A.OUT_FP16_PLANAR_PAIRS, 61, scale_log2_range=ACTIVE)
+    elif kind == "ref8-odd":
+        case = ref_case(ntc, P.spec_ref092(8), 320, 320, 9, 3, 16, A.OUT_FP16_PLANAR_PAIRS, 62, scale_log2_range=ACTIVE)
+    elif kind == "fp8_8":
+        spec = P.spec_ref092_fp8(8)
+        case = ref_case(ntc, spec, 256, 256, 9, 2, 16, A.OUT_FP16_PLANAR_PAIRS, 63, weights=ntc.synth.make_fp8_weights(spec, 64))
+    else:
+        spec = P.spec_cfg3()
+        blob = ntc.synth.make_weights(spec, 65, scale_log2_range=ACTIVE)
+        layout = ntc.synth.weight_layout(spec)
+        blob[layout.biasOffset[0]:layout.bufferSize].view(np.int32)[70] = 2 ** 31 - 1
+        case = cfg_case(ntc, spec, 128, 128, 8, 16, A.OUT_FP16_PLANAR_PAIRS, 66, weights=blob)
+    units = device.compute_units
+    host = case.host_set()
+    most = 1100 * units
+    q = make_queries(np.random.default_rng(67), most, len(case.mips))
+    want = oracle_queries(oracle, host, q)
+    dset = case.device_set(device)
+    d_bricks = device.alloc(device.lib.ntc_hip_query_latents_bytes(dset))
+    A.check(device.lib.ntc_hip_build_query_latents(dset, d_bricks.ptr, d_bricks.nbytes))
+    d_q, d_out = device.upload(q.view(np.uint8)), device.alloc(most * 32)
+    for n in (15, 17, 128 * units, 128 * units + 1, 256 * units, 256 * units + 1, 512 * units + 1, most):
+        for use_bricks in (False, True):
+            dset.queryLatents, dset.queryLatentsBytes = (d_bricks.ptr, d_bricks.nbytes) if use_bricks else (None, 0)
+            d_out.fill(0xCD)
+            A.check(device.lib.ntc_hip_decode_queries(dset, d_q.ptr, n, d_out.ptr, d_out.nbytes))
+            device.synchronize()
+            got = d_out.download(np.uint16).reshape(most, 16)
+            assert np.array_equal(got[:n], want[:n]) and (got[n:] == 0xCDCD).all(), (kind, n, use_bricks)
