@@ -205,6 +205,15 @@ __device__ __forceinline__ void build_fp8_feature_lut(Lds& lds, int tid)
     }
 }
 
+// Whether a set is decoded by this instantiation.  every: the launch has no other (see launch_decode_fp8), and the general
+// instantiation takes sets of one plane too.
+template <class V>
+__device__ __forceinline__ bool own_fp8_set(int modes, bool every)
+{
+    bool const onePlane = (modes & kAllOnePlane) == kAllOnePlane;
+    return V::ONE ? onePlane : (every || !onePlane);
+}
+
 // A wave takes one output tile (16 rows of a layer; ten tiles) and its lane (i, kg) holds the dwords of row i that it will
 // write: they come from memory straight into registers, all loads in flight together, a row's sum is the lane's and two
 // exchanges, and one barrier - the waves' flags - lies between.  Every workgroup of both instantiations does this much
@@ -213,7 +222,7 @@ __device__ __forceinline__ void build_fp8_feature_lut(Lds& lds, int tid)
 // weights behind the first barrier; the caller adds one behind the call.  (With the blob read twice, once per thread and
 // dword into atomic sums and once byte by byte into operands: 18.0 us for a 128 x 128 decode, 13.8 now.)
 template <class V>
-__device__ __attribute__((noinline)) int stage_fp8_weights(Fp8Lds<V>& lds, uint8_t const* blobOfLanes, int const tid, int tables)
+__device__ __attribute__((noinline)) int stage_fp8_weights(Fp8Lds<V>& lds, uint8_t const* blobOfLanes, int const tid, int tables, int every)
 {
     constexpr int TILES = V::T0 + V::T1 + V::T2 + 1;
     static_assert(TILES <= V::WAVES, "a tile per wave at most");
@@ -277,7 +286,7 @@ __device__ __attribute__((noinline)) int stage_fp8_weights(Fp8Lds<V>& lds, uint8
     flags = __builtin_amdgcn_readfirstlane(flags);
     int const oneMask = int(~(flags >> 4) & ~flags & 7u);
     int const modes = int(flags & 7u) | (oneMask << kOnePlaneShift) | ((flags & (1u << 8)) ? 0 : kFp8OutputsBounded);
-    if (((modes & kAllOnePlane) == kAllOnePlane) != V::ONE || !mine) return modes;
+    if (!own_fp8_set<V>(modes, every != 0) || !mine) return modes;
 
     if (layer == 3) {                                        // int8 weights as halves, 32 inputs = one block
         lds.w3[lane] = make_uint4(halves_of_bytes(v[0], 0), halves_of_bytes(v[0], 2), halves_of_bytes(v[1], 0), halves_of_bytes(v[1], 2));
@@ -290,7 +299,8 @@ __device__ __attribute__((noinline)) int stage_fp8_weights(Fp8Lds<V>& lds, uint8
     for (int d = 0; d < 4; ++d) e4m3_times_512(v[d], w[d]);
 #pragma unroll
     for (int p = 0; p < V::HELD; ++p) {
-        bool const whole = V::ONE || (p == 0 && ((oneMask >> layer) & 1));
+        bool const whole = V::ONE || ((oneMask >> layer) & 1);
+        if (p > 0 && (whole || (p == 2 && !((modes >> layer) & 1)))) break;      // planes that the layer's form does not read
         uint32_t h[4][2];
 #pragma unroll
         for (int d = 0; d < 4; ++d) { h[d][0] = plane_halves(w[d][0], w[d][1], p, whole); h[d][1] = plane_halves(w[d][2], w[d][3], p, whole); }
@@ -733,7 +743,8 @@ __global__ void __launch_bounds__(V::THREADS, 1)
 decode_fp8_kernel(MipTable table, int numMips, int totalTiles, int workgroups, Fp8Handoff handoff)
 {
     DevMip const* const mips = table_entries(table.entries);
-    if (!V::ONE && *handoff.word != handoff.serial) return;  // the one-plane launch before this one met only its own sets
+    bool const every = !V::ONE && !handoff.word;
+    if (!V::ONE && !every && *handoff.word != handoff.serial) return;        // the one-plane launch before this one met only its own sets
     __shared__ Fp8Lds<V> lds;
     int const lane = threadIdx.x & 63;
     int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -787,8 +798,8 @@ decode_fp8_kernel(MipTable table, int numMips, int totalTiles, int workgroups, F
         entry = table_entry_of(mips, numMips, entry, segBegin);
         uint8_t const* const blob = mips[entry].weights;
         int const segEnd = segment_end(mips, numMips, entry, tileEnd, blob);
-        modes = __builtin_amdgcn_readfirstlane(stage_fp8_weights<V>(lds, blob, wave * 64 + lane_id(), segBegin == tileBegin));
-        if (((modes & kAllOnePlane) == kAllOnePlane) != V::ONE) { // the other instantiation's segment
+        modes = __builtin_amdgcn_readfirstlane(stage_fp8_weights<V>(lds, blob, wave * 64 + lane_id(), segBegin == tileBegin, every));
+        if (!own_fp8_set<V>(modes, every)) {                 // the other instantiation's segment
             if (V::ONE && threadIdx.x == 0) *handoff.word = handoff.serial;
             segBegin = segEnd;
             continue;
@@ -824,7 +835,8 @@ query_fp8_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queri
                  uint16_t* __restrict__ out, int workgroups, int waves, Fp8Handoff handoff)
 {
     DevMip const* const mips = table_entries(table.entries);
-    if (!V::ONE && *handoff.word != handoff.serial) return;  // the set went to the one-plane launch before this one
+    bool const every = !V::ONE && !handoff.word;
+    if (!V::ONE && !every && *handoff.word != handoff.serial) return;        // the set went to the one-plane launch before this one
     __shared__ Fp8Lds<V> lds;
     __shared__ QueryMip qmips[16];
     if (threadIdx.x < 16) {
@@ -842,8 +854,8 @@ query_fp8_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queri
     int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int const j = lane & 15, g = lane >> 4;
 
-    int const modes = __builtin_amdgcn_readfirstlane(stage_fp8_weights<V>(lds, mips[0].weights, wave * 64 + lane_id(), 1));
-    if (((modes & kAllOnePlane) == kAllOnePlane) != V::ONE) {            // the other instantiation's set (uniform over the grid)
+    int const modes = __builtin_amdgcn_readfirstlane(stage_fp8_weights<V>(lds, mips[0].weights, wave * 64 + lane_id(), 1, every));
+    if (!own_fp8_set<V>(modes, every)) {                     // the other instantiation's set (uniform over the grid)
         if (V::ONE && threadIdx.x == 0) *handoff.word = handoff.serial;
         return;
     }
@@ -908,7 +920,7 @@ __global__ void selftest_fp8_activation_kernel(uint16_t const* __restrict__ in, 
 
 using VFp8_16 = Fp8Variant<16>;
 
-// Both instantiations, the one-plane one first; a set is decoded by the one it belongs to (decided on the device
+// Large launches: both instantiations, the one-plane one first; a set is decoded by the one it belongs to (decided on the device
 // from its weights).  A workgroup of the first launch that meets a set of the other kind writes the launch pair's
 // serial number into the caller's hand-off word; the workgroups of the second launch leave at once unless they
 // find that number there (nothing ever clears the word: a stale match only costs the second launch its look at
@@ -918,6 +930,12 @@ static hipError_t launch_fp8_variant(MipTable const& mips, int numMips, int tota
 {
     using One = Fp8Variant<FEATURES, true>;
     using Any = Fp8Variant<FEATURES, false>;
+    // Up to eight tiles per compute unit one launch of the general instantiation decodes every set: the second launch and
+    // a pass over weights cost more than three waves per SIMD instead of four.  (64 x 64 ... 1024 x 512 with one plane:
+    // 11.0 and 25.1 us in two launches, 9.6 and 24.6 in one; 2048 x 1024: 74.7 and 76.7.  With two planes: 15.3 and 34.0,
+    // 11.2 and 29.8.)
+    if (totalTiles <= 8 * compute_units_of_current_device())
+        return launch_kernel<decode_fp8_kernel<Any>>(dim3(gridSize), dim3(Any::THREADS), 0, stream, mips, numMips, totalTiles, gridSize, Fp8Handoff{ nullptr, 0u });
     hipError_t const e = launch_kernel<decode_fp8_kernel<One>>(dim3(gridSize), dim3(One::THREADS), 0, stream, mips, numMips, totalTiles, gridSize, handoff);
     if (e != hipSuccess) return e;
     return launch_kernel<decode_fp8_kernel<Any>>(dim3(gridSize), dim3(Any::THREADS), 0, stream, mips, numMips, totalTiles, gridSize, handoff);
@@ -947,6 +965,10 @@ static hipError_t launch_fp8_query_variant(MipTable const& mips, int numMips, De
         waves /= 2;
         grid = (numQueries + 64 * waves - 1) / (64 * waves);
     }
+    // one launch, as in launch_fp8_variant (131072 queries: 14.0 us in two launches, 13.1 in one; 262144: 18.9 and 23.2)
+    if (numQueries <= 512 * uint64_t(compute_units_of_current_device()))
+        return launch_kernel<query_fp8_kernel<Any>>(dim3(unsigned(grid)), dim3(Any::THREADS), 0, stream, mips, numMips, queries, numQueries, out, int(grid),
+                                                    waves < Any::WAVES ? waves : Any::WAVES, Fp8Handoff{ nullptr, 0u });
     hipError_t const e = launch_kernel<query_fp8_kernel<One>>(dim3(unsigned(grid)), dim3(One::THREADS), 0, stream, mips, numMips, queries, numQueries, out, int(grid), waves, handoff);
     if (e != hipSuccess) return e;
     return launch_kernel<query_fp8_kernel<Any>>(dim3(unsigned(grid)), dim3(Any::THREADS), 0, stream, mips, numMips, queries, numQueries, out, int(grid),

@@ -577,3 +577,23 @@ def test_gpu_fp8_launch_pairs_of_one_context_do_not_inherit_each_others_hand_off
             (device.decode_static if static else device.decode)([dsets[i]])
             device.synchronize()
             assert first_mismatch(hset.output, c.d_output.download()) is None, (static, i)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("features", [16, 4])
+def test_gpu_fp8_sets_of_either_kind_in_one_and_two_launches(ntc, device, orc, features):
+    """One-plane and two-plane sets, alone and together, at the tile counts where the launch changes: a tile per
+    workgroup, one launch for all sets, a launch for either kind."""
+    units = device.compute_units
+    for tiles in (units, units + 1, 8 * units, 8 * units + 1):
+        cases = [fp8_case(ntc, features, 64, 4 * tiles - (1 if tiles & 1 else 0), 1, 2, 13, ntc.abi.OUT_FP16_PLANAR_PAIRS, 90 + k, weight_sigma=sigma)
+                 for k, sigma in enumerate((0.35, 1.5))]
+        hosts = [c.host_set() for c in cases]
+        for h in hosts:
+            h.decode(threads=8)
+        for chosen in ([0], [1], [0, 1]) if tiles > units + 1 else ([0, 1],):
+            sets = [cases[k].device_set(device) for k in chosen]
+            device.decode(sets)
+            device.synchronize()
+            for k in chosen:
+                assert first_mismatch(hosts[k].output, cases[k].d_output.download()) is None, (tiles, chosen, k)
