@@ -1210,12 +1210,14 @@ image_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int 
         if (!arrived_last(work.counters, groups, last)) return;
         total = sum_entries(work.groupSums, int(groups), scratch);
     }
-    if (threadIdx.x < NTC_HIP_DEV_MAX_CHANNELS) work.result->totals[threadIdx.x] = total;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        __threadfence_system();
-        __hip_atomic_store(&work.result->serial, work.serial, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    // One wave tells the host: stores of system scope go past the caches, and the totals' are acknowledged before the
+    // serial number's is made.  (Plain stores and a release between them write back the die's whole L2.)
+    if (threadIdx.x >= 64) return;
+    if (threadIdx.x < NTC_HIP_DEV_MAX_CHANNELS) __hip_atomic_store(&work.result->totals[threadIdx.x], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0);
+    asm volatile("" ::: "memory");
+    if (threadIdx.x == 0) __hip_atomic_store(&work.result->serial, work.serial, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int height, int setChannels, uint32_t validChannelMask,

@@ -86,6 +86,7 @@ struct NtcHipContext {
     size_t lossBlocks = 0;             // workgroups it has room for
     uint32_t* lossCounters = nullptr;  // arrivals, zero between calls
     LossResult* lossHost = nullptr;    // pinned: what the loss pass hands to the host
+    LossResult*   lossHostOnDevice = nullptr;  // its device address
     uint32_t lossSerial = 0;
     static constexpr int kSlots = 4;
     struct Slot { DevMip* host = nullptr; size_t capacity = 0; hipEvent_t done = nullptr; bool inFlight = false; };
@@ -1043,6 +1044,7 @@ int ntc_hip_ctx_image_loss(NtcHipContext* ctx, void* decoded, const void* refere
         if (!L.lossHost) {
             HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&L.lossHost), sizeof(LossResult), hipHostMallocMapped | hipHostMallocCoherent));
             L.lossHost->serial = 0;
+            HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void**>(&L.lossHostOnDevice), L.lossHost, 0));
         }
         L.lossBlocks = blocks;
     }
@@ -1051,7 +1053,7 @@ int ntc_hip_ctx_image_loss(NtcHipContext* ctx, void* decoded, const void* refere
     work.groupSums = L.lossDev + blocks * NTC_HIP_DEV_MAX_CHANNELS;
     work.counters = L.lossCounters;
     work.serial = ++L.lossSerial;
-    HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void**>(&work.result), L.lossHost, 0));
+    work.result = L.lossHostOnDevice;
     HIP_TRY(launch_image_loss(static_cast<uint16_t*>(decoded), static_cast<uint16_t const*>(reference), width, height,
                               setChannels, validChannelMask, maskChannelIndex < 0 ? -1 : maskChannelIndex,
                               discardMaskedOutPixels ? 1 : 0, work, L.stream));
