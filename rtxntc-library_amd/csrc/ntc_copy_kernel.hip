@@ -165,7 +165,7 @@ __device__ __forceinline__ float divide_by_top(float a, float top, float recipro
 struct DitherRng {
     uint32_t seed, index;
     __device__ DitherRng() {}
-    __device__ explicit DitherRng(uint32_t linearIndex) : index(1)
+    __device__ explicit DitherRng(uint32_t linearIndex) : index(0)
     {
         uint32_t a = linearIndex;
         a = (a + 0x7ed55d16u) + (a << 12);
@@ -176,9 +176,13 @@ struct DitherRng {
         a = (a ^ 0xb55a4f09u) ^ (a >> 16);
         seed = a;
     }
-    __device__ float next_float()                            // [0, 1)
+    __device__ float next_offset()                           // a draw of [0, 1) less one half (both differences are exact)
     {
-        uint32_t k = index++ * 0xcc9e2d51u;
+        return offset(index++);
+    }
+    __device__ float offset(uint32_t draw) const             // that of one draw, counted from 0
+    {
+        uint32_t k = (draw + 1u) * 0xcc9e2d51u;
         k = (k << 15) | (k >> 17);
         k *= 0x1b873593u;
         uint32_t h = seed ^ k;
@@ -187,7 +191,7 @@ struct DitherRng {
         h ^= h >> 16; h *= 0x85ebca6bu;
         h ^= h >> 13; h *= 0xc2b2ae35u;
         h ^= h >> 16;
-        return __builtin_bit_cast(float, (h & 0x7fffffu) | 0x3f800000u) - 1.f;
+        return __builtin_bit_cast(float, (h & 0x7fffffu) | 0x3f800000u) - 1.5f;
     }
 };
 
@@ -287,7 +291,7 @@ read_channels_kernel(ReadChannelsArgs a)
             if constexpr (PLAIN) {
                 bits = encode_value<FORMAT>(value, false, 0.f);
             } else {
-                float const dither = a.useDithering ? rng.next_float() - 0.5f : 0.f;  // one draw per destination channel
+                float const dither = a.useDithering ? rng.next_offset() : 0.f;  // one draw per destination channel
                 bits = encode_value<FORMAT>(value, a.useDithering != 0, dither);
             }
             words[(k * BPC) >> 2] |= bits << (8 * ((k * BPC) & 3));
@@ -489,19 +493,34 @@ read_groups_kernel(GroupsArgs a)
                 }
                 transfer_halves(staged, a.transfers.slot[ch], a.transfers.pair[ch], bits, value);
             } else {                                         // GetDefaultChannelValue; 0 is 0 in every colour space
-                float const fill = (ch == 3) ? encode_color_space(a.fillSpace, 1.f) : 0.f;
+                float const fill = (ch == 3) ? transfer_half(transfer_pair(0, a.fillSpace), 0x3C00u) : 0.f;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) value[k] = fill;
             }
         }
 #pragma unroll
         for (int ch = 0; ch < CHANNELS; ++ch) {
+            uint32_t bits[4];
+            // A filled channel whose code is the same for the least and the greatest draw has it for all between them, and
+            // its draws, of which each is a seventh of a pixel's work, need not be made.
+            bool drawn = DITHER;                             // uniform
+            if (DITHER && ch >= copied) {
+                bits[0] = encode_value<FORMAT>(values[ch][0], true, -0.5f);
+                bits[1] = encode_value<FORMAT>(values[ch][0], true, 0.5f - 0x1p-23f);
+                drawn = __builtin_amdgcn_readfirstlane(bits[0] ^ bits[1]) != 0u;
+                bits[1] = bits[2] = bits[3] = bits[0];
+            }
+            if (drawn) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) bits[k] = encode_value<FORMAT>(values[ch][k], true, rng[k].offset(ch));
+            } else if (!DITHER) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) bits[k] = encode_value<FORMAT>(values[ch][k], false, 0.f);
+            }
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                float const dither = DITHER ? rng[k].next_float() - 0.5f : 0.f;
-                uint32_t const bits = encode_value<FORMAT>(values[ch][k], DITHER, dither);
                 int const at = k * PIXEL + ch * BPC;         // byte of the group
-                words[at >> 2] |= BPC == 4 ? bits : bits << (8 * (at & 3));
+                words[at >> 2] |= BPC == 4 ? bits[k] : bits[k] << (8 * (at & 3));
             }
         }
         uint8_t* const out = a.image + size_t(y) * a.rowPitch + size_t(x) * PIXEL;
@@ -815,7 +834,7 @@ read_channels_resize_kernel(ReadChannelsArgs a)
         } else {
             value = (ch == 3) ? 1.f : 0.f;
         }
-        float const dither = a.useDithering ? rng.next_float() - 0.5f : 0.f;
+        float const dither = a.useDithering ? rng.next_offset() : 0.f;
         uint32_t const bits = encode_channel<FORMAT>(ch < 16 ? a.dstColorSpaces[ch] : 0, value, a.useDithering != 0, dither);
         if constexpr (BPC == 1) px[ch] = uint8_t(bits);
         else if constexpr (BPC == 2) reinterpret_cast<uint16_t*>(px)[ch] = uint16_t(bits);
