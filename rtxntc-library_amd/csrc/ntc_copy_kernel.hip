@@ -1073,11 +1073,12 @@ hipError_t launch_write_channels(WriteChannelsArgs const& args, hipStream_t stre
 // lane's texels of a row goes into a double accumulator, and the workgroup writes 16 double partial sums;
 // ReduceLoss likewise finishes in double (src/Optimizer.cu:382-387).
 //
-// The same launch finishes the sum and hands it to the host: the last of every kLossGroup workgroups to arrive adds
-// the group's partial sums, the last group to finish adds those of the groups (each in a fixed order, so results are
-// reproducible) and writes the 16 totals and a serial number into pinned host memory, where the caller is looking
-// (a second kernel, a copy and a stream synchronisation made most of the 28 us a call on 64 x 64 texels took; 14 now.
-// 4096 x 4096 texels of 16 channels: 192 us, 5.6 TB/s).
+// The same launch finishes the sum and hands it to the host (a second kernel, a copy and a stream synchronisation made
+// most of the 28 us a call on 64 x 64 texels took).  Workgroups form at most kLossRows groups; the last one of a group
+// to arrive adds the group's partial sums, in a fixed order, so results are reproducible, and stores them into pinned
+// host memory, where the caller is looking and adds the rows, of which an image of up to 128 x 128 texels has one per
+// workgroup.  What such a call waits for is a chain of trips to memory: a second level of groups on the device, and a
+// serial number stored once the totals were acknowledged, made it 2 us longer.
 // The partial sums pass between workgroups of different dies, whose caches do not see each other: they are stored and
 // loaded as device-scope atomics, which go past those caches, and a store is acknowledged before its workgroup counts
 // itself as arrived.  (Fences instead write back and invalidate a die's whole L2, a thousand times in a launch over
@@ -1090,7 +1091,12 @@ __device__ __forceinline__ double sum_entries(double const* entries, int count, 
 {
     int const c = threadIdx.x & 15, part = threadIdx.x >> 4;                     // 16 threads per channel
     double v = 0.0;
-    for (int i = part; i < count; i += 16) v += published(entries + size_t(i) * NTC_HIP_DEV_MAX_CHANNELS + c);
+    for (int i = part; i < count; i += 32) {                 // (two loads in flight: groups have at most 32 members up to 4096 x 4096)
+        double const one = published(entries + size_t(i) * NTC_HIP_DEV_MAX_CHANNELS + c);
+        double const two = published(entries + size_t(min(i + 16, count - 1)) * NTC_HIP_DEV_MAX_CHANNELS + c);
+        v += one;
+        if (i + 16 < count) v += two;
+    }
     scratch[part][c] = v;
     __syncthreads();
     double total = 0.0;
@@ -1100,31 +1106,41 @@ __device__ __forceinline__ double sum_entries(double const* entries, int count, 
     return total;                                            // in threads 0 ... 15
 }
 
-// Whether this workgroup is the last of `count` to come here (uniform), after its first wave has published its sums.
+// Whether this workgroup is the last of `count` to come here (uniform).  Each wave has its own stores in place first.
 __device__ __forceinline__ bool arrived_last(uint32_t* counter, uint32_t count, int& scratch)
 {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0);
+    asm volatile("" ::: "memory");
     __syncthreads();
-    if (threadIdx.x < 64) {                                  // the wave whose stores have to be in place
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(0);
-        asm volatile("" ::: "memory");
-        if (threadIdx.x == 0) {
-            bool const last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == count - 1u;
-            if (last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // as the next launch expects it
-            scratch = last;
-        }
+    if (threadIdx.x == 0) {
+        bool const last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == count - 1u;
+        if (last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // as the next launch expects it
+        scratch = last;
     }
     __syncthreads();
     return scratch != 0;
 }
 
+// v plus the v of another lane of the row of 16: CONTROL is a DPP control.
+template <int CONTROL>
+__device__ __forceinline__ double add_from_row(double v)
+{
+    uint64_t const bits = __builtin_bit_cast(uint64_t, v);
+    uint32_t const low = uint32_t(__builtin_amdgcn_mov_dpp(int(uint32_t(bits)), CONTROL, 0xF, 0xF, true));
+    uint32_t const high = uint32_t(__builtin_amdgcn_mov_dpp(int(uint32_t(bits >> 32)), CONTROL, 0xF, 0xF, true));
+    return v + __builtin_bit_cast(double, uint64_t(high) << 32 | low);
+}
+
 template <int PX, bool MASKED>
 __global__ void __launch_bounds__(256)
 image_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int width, int height, int setChannels, int rowsPerWave,
-                  uint32_t validChannelMask, int maskChannel, int discardMaskedOut, uint32_t gridX, uint32_t blocks, LossWorkspace work)
+                  uint32_t validChannelMask, int maskChannel, int discardMaskedOut, uint32_t gridX, uint32_t blocks, uint32_t groupSize, LossWorkspace work)
 {
     constexpr int PAIRS = NTC_HIP_DEV_MAX_CHANNELS / 2;
-    __shared__ double sums[4][NTC_HIP_DEV_MAX_CHANNELS];
+    constexpr int STRIDE = 256 + 16;                         // (channels half the banks apart)
+    __shared__ double lanes[NTC_HIP_DEV_MAX_CHANNELS * STRIDE];
+    __shared__ double sums[NTC_HIP_DEV_MAX_CHANNELS];
     int const lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int const x = (blockIdx.x * 64 + lane) * PX;
     int const pairs = setChannels >> 1;
@@ -1190,53 +1206,43 @@ image_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int 
             acc[2 * p + 1] += double(s1);
         }
     }
+    // Across the workgroup: 16 threads per channel add 16 of its 256 values each, then each other's.  (With exchanges
+    // between lanes, 17 of a double and 1500 instructions when every lane hands over half of what it holds at a step,
+    // this took 1 us longer.)
 #pragma unroll
-    for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c)
-        if (c >= setChannels || !((validChannelMask >> c) & 1u)) acc[c] = 0.0;
-    // Across the lanes by halving: partners 32, 16, 8 and 4 lanes apart each keep one half of the channels they both
-    // have and hand over the other, after which every lane has one channel; the last two steps add whole values.  17
-    // exchanges of a double instead of the 96 of one butterfly per channel.
-#pragma unroll
-    for (int n = 8, off = 32; n >= 1; n >>= 1, off >>= 1) {
-        bool const upper = (lane & off) != 0;
-#pragma unroll
-        for (int i = 0; i < n; ++i) {
-            double const keep = upper ? acc[i + n] : acc[i], give = upper ? acc[i] : acc[i + n];
-            acc[i] = keep + __shfl_xor(give, off, 64);
-        }
-    }
-    double mine = acc[0] + __shfl_xor(acc[0], 2, 64);
-    mine += __shfl_xor(mine, 1, 64);
-    if ((lane & 3) == 0) sums[wave][lane >> 2] = mine;       // bits 5 ... 2 of the lane number are its channel's, most significant first
+    for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) lanes[c * STRIDE + int(threadIdx.x)] = acc[c];
     __syncthreads();
+    int const channel = int(threadIdx.x) >> 4, part = int(threadIdx.x) & 15;
+    double mine = 0.0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) mine += lanes[channel * STRIDE + part + 16 * k];
+    mine = add_from_row<0xB1>(mine);                         // quad_perm: the neighbour,
+    mine = add_from_row<0x4E>(mine);                         // the other pair,
+    mine = add_from_row<0x141>(mine);                        // row_half_mirror: the other quad,
+    mine = add_from_row<0x140>(mine);                        // row_mirror: the other eight
+    if (channel >= setChannels || !((validChannelMask >> channel) & 1u)) mine = 0.0;
     uint32_t const block = blockIdx.y * gridX + blockIdx.x;
-    uint32_t const group = block / kLossGroup, groups = (blocks + kLossGroup - 1) / kLossGroup, first = group * kLossGroup;
-    double total = 0.0;                                      // threads 0 ... 15
-    if (threadIdx.x < NTC_HIP_DEV_MAX_CHANNELS) {
-        int const c = threadIdx.x;
-        total = sums[0][c] + sums[1][c] + sums[2][c] + sums[3][c];
-        if (blocks > 1) publish(work.partials + size_t(block) * NTC_HIP_DEV_MAX_CHANNELS + c, total);
+    uint32_t const group = block / groupSize, first = group * groupSize, members = min(groupSize, blocks - first);
+    double total;                                            // threads 0 ... 15: a channel's each
+    if (members > 1) {
+        __shared__ double scratch[16][NTC_HIP_DEV_MAX_CHANNELS];
+        __shared__ int last;
+        if (part == 0) publish(work.partials + size_t(block) * NTC_HIP_DEV_MAX_CHANNELS + channel, mine);
+        if (!arrived_last(work.counters + group, members, last)) return;
+        total = sum_entries(work.partials + size_t(first) * NTC_HIP_DEV_MAX_CHANNELS, int(members), scratch);
+    } else {
+        if (part == 0) sums[channel] = mine;
+        __syncthreads();
+        total = sums[threadIdx.x & (NTC_HIP_DEV_MAX_CHANNELS - 1)];
     }
-    __shared__ double scratch[16][NTC_HIP_DEV_MAX_CHANNELS];
-    __shared__ int last;
-    if (blocks > 1) {
-        int const members = int(min(uint32_t(kLossGroup), blocks - first));
-        if (!arrived_last(work.counters + 1 + group, uint32_t(members), last)) return;
-        total = sum_entries(work.partials + size_t(first) * NTC_HIP_DEV_MAX_CHANNELS, members, scratch);
-    }
-    if (groups > 1) {
-        if (threadIdx.x < NTC_HIP_DEV_MAX_CHANNELS) publish(work.groupSums + size_t(group) * NTC_HIP_DEV_MAX_CHANNELS + threadIdx.x, total);
-        if (!arrived_last(work.counters, groups, last)) return;
-        total = sum_entries(work.groupSums, int(groups), scratch);
-    }
-    // One wave tells the host: stores of system scope go past the caches, and the totals' are acknowledged before the
-    // serial number's is made.  (Plain stores and a release between them write back the die's whole L2.)
+    // To the host in one trip: each half of a double is stored together with the serial number, so that every word
+    // says for itself whether it has arrived.  Stores of system scope go past the caches.  (Plain stores and a release
+    // behind them write back the die's whole L2.)
     if (threadIdx.x >= 64) return;
-    if (threadIdx.x < NTC_HIP_DEV_MAX_CHANNELS) __hip_atomic_store(&work.result->totals[threadIdx.x], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0);
-    asm volatile("" ::: "memory");
-    if (threadIdx.x == 0) __hip_atomic_store(&work.result->serial, work.serial, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    uint64_t const sum = __builtin_bit_cast(uint64_t, __shfl(total, lane >> 1, 64));
+    uint64_t const word = uint64_t(work.serial) << 32 | ((lane & 1) ? sum >> 32 : sum & 0xffffffffu);
+    if (lane < 2 * NTC_HIP_DEV_MAX_CHANNELS)
+        __hip_atomic_store(&work.rows[group].words[lane], word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int height, int setChannels, uint32_t validChannelMask,
@@ -1247,7 +1253,7 @@ hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int heig
     auto launch = [&](auto perLane, auto masks) {
         constexpr auto kernel = image_loss_kernel<decltype(perLane)::value, decltype(masks)::value>;
         return launch_kernel<kernel>(dim3(grid.x, grid.y), dim3(256), 0, stream, a, b, width, height, setChannels, grid.rowsPerWave,
-                                     validChannelMask, maskChannel, discardMaskedOut, grid.x, grid.x * grid.y, work);
+                                     validChannelMask, maskChannel, discardMaskedOut, grid.x, grid.x * grid.y, grid.groupSize, work);
     };
     auto of_width = [&](auto perLane) { return masked ? launch(perLane, std::true_type{}) : launch(perLane, std::false_type{}); };
     return two ? of_width(std::integral_constant<int, 2>{}) : of_width(std::integral_constant<int, 1>{});

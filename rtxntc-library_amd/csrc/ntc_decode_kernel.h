@@ -121,22 +121,23 @@ hipError_t launch_write_channels(WriteChannelsArgs const& args, hipStream_t stre
 // texels (2 when the width is even) by 4 waves x rowsPerWave rows.  Four workgroups are resident on a compute unit; as
 // many rows per wave as make the grid about that large (every workgroup ends in 16 reductions across its lanes, and a
 // row is a memory round trip), from one, for images that would not fill the GPU, to 32.
-struct LossGrid { uint32_t x, y; int32_t rowsPerWave; };
+constexpr uint32_t kLossRows = 32;                          // groups of workgroups, each of which hands its sums to the host
+struct LossGrid { uint32_t x, y, groupSize; int32_t rowsPerWave; };
 inline LossGrid image_loss_grid(int width, int height, int computeUnits)
 {
     uint32_t const perLane = (width & 1) ? 1u : 2u, x = (uint32_t(width) + 64u * perLane - 1u) / (64u * perLane);
     uint64_t const quads = (uint32_t(height) + 3u) / 4u;
     uint64_t const wanted = (quads * x + uint64_t(4 * computeUnits) - 1u) / uint64_t(4 * computeUnits);
     uint32_t const rows = uint32_t(wanted < 1u ? 1u : wanted > 32u ? 32u : wanted);
-    return LossGrid{ x, (uint32_t(height) + 4u * rows - 1u) / (4u * rows), int32_t(rows) };
+    uint32_t const y = (uint32_t(height) + 4u * rows - 1u) / (4u * rows);
+    return LossGrid{ x, y, (x * y + kLossRows - 1u) / kLossRows, int32_t(rows) };
 }
-constexpr uint32_t kLossGroup = 32;                         // workgroups whose partial sums are added first
-struct LossResult { double totals[16]; uint32_t serial; };  // pinned host memory
+// Pinned host memory: word 2 c + h holds half h (low, high) of channel c's sum below the serial number of its call.
+struct LossRow { uint64_t words[32]; };
 struct LossWorkspace {
     double* partials;              // 16 per workgroup
-    double* groupSums;             // 16 per kLossGroup workgroups
-    uint32_t* counters;            // one, then one per kLossGroup workgroups: zero before and after every launch
-    LossResult* result;            // device address; `serial` is stored last
+    uint32_t* counters;            // kLossRows: zero before and after every launch
+    LossRow* rows;                 // kLossRows, device address
     uint32_t serial;
 };
 hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int height, int setChannels, uint32_t validChannelMask,

@@ -82,11 +82,11 @@ struct NtcHipContext {
     uint32_t handoffSerial = 0;        // changes with every pair of such launches
     size_t tableCapacity = 0;          // entries
     std::vector<DevMip> lastTable;     // what tableDev currently holds (or will, in stream order)
-    double* lossDev = nullptr;         // partial sums of the loss pass: 16 per workgroup, then 16 per group of workgroups
+    double* lossDev = nullptr;         // partial sums of the loss pass: 16 per workgroup
     size_t lossBlocks = 0;             // workgroups it has room for
     uint32_t* lossCounters = nullptr;  // arrivals, zero between calls
-    LossResult* lossHost = nullptr;    // pinned: what the loss pass hands to the host
-    LossResult*   lossHostOnDevice = nullptr;  // its device address
+    LossRow* lossHost = nullptr;       // pinned: what the loss pass hands to the host
+    LossRow* lossHostOnDevice = nullptr;  // its device address
     uint32_t lossSerial = 0;
     static constexpr int kSlots = 4;
     struct Slot { DevMip* host = nullptr; size_t capacity = 0; hipEvent_t done = nullptr; bool inFlight = false; };
@@ -1032,45 +1032,59 @@ int ntc_hip_ctx_image_loss(NtcHipContext* ctx, void* decoded, const void* refere
         }
     }
     LossGrid const grid = image_loss_grid(width, height, L.computeUnits);
-    size_t const blocks = size_t(grid.x) * grid.y, groups = (blocks + kLossGroup - 1) / kLossGroup;
+    size_t const blocks = size_t(grid.x) * grid.y, rows = (blocks + grid.groupSize - 1) / grid.groupSize;
     if (blocks > L.lossBlocks) {
         HIP_TRY(hipStreamSynchronize(L.stream));
         if (L.lossDev) { HIP_TRY(hipFree(L.lossDev)); L.lossDev = nullptr; }
-        if (L.lossCounters) { HIP_TRY(hipFree(L.lossCounters)); L.lossCounters = nullptr; }
         L.lossBlocks = 0;
-        HIP_TRY(hipMalloc(reinterpret_cast<void**>(&L.lossDev), (blocks + groups) * NTC_HIP_DEV_MAX_CHANNELS * sizeof(double)));
-        HIP_TRY(hipMalloc(reinterpret_cast<void**>(&L.lossCounters), (1 + groups) * sizeof(uint32_t)));
-        HIP_TRY(launch_fill(reinterpret_cast<uint8_t*>(L.lossCounters), 0, (1 + groups) * sizeof(uint32_t), L.stream));
+        HIP_TRY(hipMalloc(reinterpret_cast<void**>(&L.lossDev), blocks * NTC_HIP_DEV_MAX_CHANNELS * sizeof(double)));
+        if (!L.lossCounters) {
+            HIP_TRY(hipMalloc(reinterpret_cast<void**>(&L.lossCounters), kLossRows * sizeof(uint32_t)));
+            HIP_TRY(launch_fill(reinterpret_cast<uint8_t*>(L.lossCounters), 0, kLossRows * sizeof(uint32_t), L.stream));
+        }
         if (!L.lossHost) {
-            HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&L.lossHost), sizeof(LossResult), hipHostMallocMapped | hipHostMallocCoherent));
-            L.lossHost->serial = 0;
+            HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&L.lossHost), kLossRows * sizeof(LossRow), hipHostMallocMapped | hipHostMallocCoherent));
+            std::memset(L.lossHost, 0, kLossRows * sizeof(LossRow));
             HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void**>(&L.lossHostOnDevice), L.lossHost, 0));
         }
         L.lossBlocks = blocks;
     }
     LossWorkspace work{};
     work.partials = L.lossDev;
-    work.groupSums = L.lossDev + blocks * NTC_HIP_DEV_MAX_CHANNELS;
     work.counters = L.lossCounters;
     work.serial = ++L.lossSerial;
-    work.result = L.lossHostOnDevice;
+    work.rows = L.lossHostOnDevice;
     HIP_TRY(launch_image_loss(static_cast<uint16_t*>(decoded), static_cast<uint16_t const*>(reference), width, height,
                               setChannels, validChannelMask, maskChannelIndex < 0 ? -1 : maskChannelIndex,
                               discardMaskedOutPixels ? 1 : 0, work, L.stream));
-    // The kernel's last act is to store the serial number behind the totals.  Most calls are done in microseconds, so
-    // the host looks for it; one that takes longer (work queued in front of it), or an error, is left to the stream.
-    // So is a call with a mask channel, which changes the decoded image: it returns when that is complete.
+    // Every word of the rows that the kernel stores carries the call's serial number.  Most calls are done in
+    // microseconds, so the host looks for it; one that takes longer (work queued in front of it), or an error, is left
+    // to the stream.  So is a call with a mask channel, which changes the decoded image: it returns when that is complete.
     auto const begin = std::chrono::steady_clock::now();
-    if (maskChannelIndex >= 0) HIP_TRY(hipStreamSynchronize(L.stream));
-    while (__atomic_load_n(&L.lossHost->serial, __ATOMIC_ACQUIRE) != work.serial) {
-        __builtin_ia32_pause();
-        if (std::chrono::steady_clock::now() - begin > std::chrono::milliseconds(2)) {
-            HIP_TRY(hipStreamSynchronize(L.stream));
-            break;
+    bool const synchronized = maskChannelIndex >= 0;
+    if (synchronized) HIP_TRY(hipStreamSynchronize(L.stream));
+    bool done = synchronized;
+    double totals[NTC_HIP_DEV_MAX_CHANNELS] = {};
+    for (size_t r = 0; r < rows; ++r) {
+        uint64_t words[32];
+        for (int w = 31; w >= 0; --w) {
+            while (words[w] = __atomic_load_n(&L.lossHost[r].words[w], __ATOMIC_ACQUIRE), uint32_t(words[w] >> 32) != work.serial && !done) {
+                __builtin_ia32_pause();
+                if (std::chrono::steady_clock::now() - begin > std::chrono::milliseconds(2)) {
+                    HIP_TRY(hipStreamSynchronize(L.stream));
+                    done = true;                             // read this word once more
+                }
+            }
+        }
+        for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) {
+            uint64_t const bits = (words[2 * c] & 0xffffffffu) | words[2 * c + 1] << 32;
+            double sum;
+            std::memcpy(&sum, &bits, sizeof(sum));
+            totals[c] += sum;
         }
     }
     double const norm = 1.0 / (double(width) * double(height));
-    for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) outMse[c] = float(L.lossHost->totals[c] * norm);
+    for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) outMse[c] = float(totals[c] * norm);
     clear_error();
     return 0;
 }
