@@ -176,25 +176,31 @@ BC6_INLINE float exp1(float c) { return exp2_of_log(c) - 1.f; }
 // ---- the workgroup ------------------------------------------------------------------------------------
 //
 // Four waves encode 64 blocks, whose texels lie in LDS; the lanes of a wave are blocks.
-//   1. one wave: the one-subset endpoints; then all: patterns' scores, taken in turn, their minimum by an atomic in LDS;
+//   1. one wave: the one-subset endpoints; then all: bounds of the patterns' scores, patterns taken in turn, and the
+//      scores of those that the bounds leave;
 //   2. a wave per subset of each block's pattern: its endpoints;
 //   3. each wave four of the sixteen texels: indices and errors of all three candidates;
 //   4. one wave: the errors added up in texel order, the choice, the block.
-// Bound by the issue of vector instructions: about 34000 for the 64 blocks, 20000 of them for the 32 scores (a score's
-// boxes are straight-line code per subset size, read with uniform masks).  Each part is a function with registers of its
-// own, so that four waves fit a SIMD and nothing is spilled in a loop; the search is one call because a call saves
-// registers to scratch (a call per two patterns: 257 us at 2048 x 2048).  One lane per block, all parts in one body with
-// 168 registers, took 121 us at 64 x 64, 151 at 1024 x 1024 and 287 at 2048 x 2048; this takes 30, 61 and 204: the
-// chain of one lane's scores is what small images waited for, and large ones for its spills and longer divisions.
+// Bound by the issue of vector instructions.  Each part is a function with registers of its own, so that four waves fit
+// a SIMD and nothing is spilled in a loop; the search is one call because a call saves registers to scratch (a call per
+// two patterns: 257 us at 2048 x 2048 instead of 204).  One lane per block, all parts in one body with 168 registers,
+// took 121 us at 64 x 64, 151 at 1024 x 1024 and 287 at 2048 x 2048: small images waited for the chain of one lane's
+// scores, large ones for its spills and longer divisions.  Shared by the waves: 30, 61 and 204 (195 beside other
+// kernels), of which the 32 scores, 625 instructions each, were more than half; with their bounds first: 165 at 2048 x
+// 2048.
 struct Bc6Lds {
     float4 texels[16][64];
     float one[11][64];                                       // one subset: lo, hi, direction, codes of the ends along it
     float two[2][11][64];                                    // each of two subsets
-    float errors[3][16][64];                                 // per texel: one subset, 7 + 6 bits, 9 + 5 bits
+    union {
+        float errors[3][16][64];                             // per texel: one subset, 7 + 6 bits, 9 + 5 bits
+        float least[32][64];                                 // until the pattern is picked: lower bounds of the scores
+    };
     uint32_t indices[2][4][64];                              // of four texels: 4 bits each, 3 bits each
-    uint64_t pick[64];                                       // score bits << 32 | pattern
-    uint32_t unscored[64];                                   // pattern 0's score is a NaN: the search stays there
     int next;
+    uint64_t pick[64];                                       // score bits << 32 | pattern
+    uint32_t bound[64], candidates[64], unbounded[64];       // smallest upper bound of a score; patterns that it leaves; some have no bounds
+    uint32_t unscored[64];                                   // pattern 0's score is a NaN: the search stays there
 };
 using Bc6Ptr = __attribute__((address_space(3))) Bc6Lds*;
 #define BC6_TASK __device__ __attribute__((noinline))        // (separate register allocation; uniform arguments are made so again)
@@ -302,57 +308,125 @@ BC6_INLINE float distance_to_line2(V3 origin, V3 dir, V3 p)
     return dot(x, x);
 }
 
-// Bounding box of the N texels of a subset (uniform), the box of no texel being [65504, 0] as in the start values.
-template <int N> BC6_INLINE void box_of(Bc6Ptr lds, int b, uint32_t members, V3& lo, V3& hi)
+// A pattern's score is the sum of the texels' squared distances from the diagonal of their subset's bounding box; the
+// pattern of the first smallest score is wanted, not the score.  It is bounded first, by the difference of the sums of
+// |w|^2 and (w . d)^2 over the offsets w from the box's corner: half the operations, in any order.  Both that sum and
+// the score as it is defined lie within a hundred units of roundoff of the sum of |w|^2 from the true value, so kScoreError
+// of 512 units separates all patterns but the nearly equal ones, which alone are evaluated as defined.
+constexpr float kScoreError = 0x1p-15f;
+// Squared diagonals below this (texels of a FLOAT32 image can be that close) leave the bounds to underflow.
+constexpr float kShortDiagonal = 1e-30f;
+
+// Adds the two sums over the N texels of a subset (uniform) and takes the minimum of the diagonals' squares, -1 for a
+// subset of equal texels: it has no direction, which makes the pattern's score a NaN.
+template <int N> BC6_INLINE void bound_subset(Bc6Ptr lds, int b, uint32_t members, float& lengths, float& along, float& shortest)
 {
     V3 p[N];
 #pragma unroll
     for (int i = 0; i < N; ++i) { p[i] = texel(lds, b, __ffs(int(members)) - 1); members &= members - 1; }
-    lo = V3{ kHalfMax, kHalfMax, kHalfMax }; hi = V3{ 0.f, 0.f, 0.f };
+    V3 lo = p[0], hi = p[0];
 #pragma unroll
-    for (int i = 0; i + 1 < N; i += 2) {
+    for (int i = 1; i + 1 < N; i += 2) {
         lo = V3{ min3_f32(lo.x, p[i].x, p[i + 1].x), min3_f32(lo.y, p[i].y, p[i + 1].y), min3_f32(lo.z, p[i].z, p[i + 1].z) };
         hi = V3{ max3_f32(hi.x, p[i].x, p[i + 1].x), max3_f32(hi.y, p[i].y, p[i + 1].y), max3_f32(hi.z, p[i].z, p[i + 1].z) };
     }
-    if constexpr (N & 1) { lo = vmin(lo, p[N - 1]); hi = vmax(hi, p[N - 1]); }
+    if constexpr (!(N & 1)) { lo = vmin(lo, p[N - 1]); hi = vmax(hi, p[N - 1]); }
+    V3 const v = hi - lo;
+    float const square = dot(v, v);
+    V3 const d = v * __builtin_amdgcn_rsqf(square);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        V3 const w = p[i] - lo;
+        lengths = __builtin_fmaf(w.x, w.x, lengths);
+        lengths = __builtin_fmaf(w.y, w.y, lengths);
+        lengths = __builtin_fmaf(w.z, w.z, lengths);
+        float const c = __builtin_fmaf(w.z, d.z, __builtin_fmaf(w.y, d.y, w.x * d.x));
+        along = __builtin_fmaf(c, c, along);
+    }
+    // (equal texels: -1)
+    shortest = fminf(shortest, v.x == 0.f && v.y == 0.f && v.z == 0.f ? -1.f : square);
 }
-BC6_INLINE void box_of_members(Bc6Ptr lds, int b, uint32_t members, V3& lo, V3& hi)
+BC6_INLINE void bound_members(Bc6Ptr lds, int b, uint32_t members, float& lengths, float& along, float& shortest)
 {
     switch (__popc(members)) {                               // the sizes that the patterns' subsets have
-    case 3:  box_of<3>(lds, b, members, lo, hi); break;
-    case 4:  box_of<4>(lds, b, members, lo, hi); break;
-    case 6:  box_of<6>(lds, b, members, lo, hi); break;
-    case 8:  box_of<8>(lds, b, members, lo, hi); break;
-    case 10: box_of<10>(lds, b, members, lo, hi); break;
-    case 12: box_of<12>(lds, b, members, lo, hi); break;
-    default: box_of<13>(lds, b, members, lo, hi); break;
+    case 3:  bound_subset<3>(lds, b, members, lengths, along, shortest); break;
+    case 4:  bound_subset<4>(lds, b, members, lengths, along, shortest); break;
+    case 6:  bound_subset<6>(lds, b, members, lengths, along, shortest); break;
+    case 8:  bound_subset<8>(lds, b, members, lengths, along, shortest); break;
+    case 10: bound_subset<10>(lds, b, members, lengths, along, shortest); break;
+    case 12: bound_subset<12>(lds, b, members, lengths, along, shortest); break;
+    default: bound_subset<13>(lds, b, members, lengths, along, shortest); break;
     }
 }
 
-// Scores of the patterns that this wave takes: the sum of the texels' squared distances from the diagonal of their
-// subset's bounding box.
-template <bool WIDE>
-BC6_TASK void score_patterns(Bc6Ptr lds, int b)
+// The least value of each score of the patterns that this wave takes (infinity for a NaN, -1 if there are no bounds), and
+// in `pick` the smallest greatest value.
+BC6_TASK void bound_scores(Bc6Ptr lds, int b)
 {
-    V3 px[16];
-#pragma unroll
-    for (int t = 0; t < 16; ++t) px[t] = texel(lds, b, t);
-    uint64_t best = ~uint64_t(0);
+    float best = __builtin_inff();
 #pragma unroll 1
     for (;;) {
         int p = 0;
         if (b == 0) p = __hip_atomic_fetch_add(&lds->next, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         p = __builtin_amdgcn_readfirstlane(p);
         if (p >= 32) break;                                  // uniform: every wave gets here
-        uint32_t const second = kSecondSubset[p];
-        V3 lo[2], hi[2];
-        box_of_members(lds, b, ~second & 0xffffu, lo[0], hi[0]);
-        box_of_members(lds, b, second, lo[1], hi[1]);
-        V3 const dir0 = normalized<WIDE>(hi[0] - lo[0]), dir1 = normalized<WIDE>(hi[1] - lo[1]);
-        float score = 0.f;
+        uint32_t members = kSecondSubset[p];
+        float lengths = 0.f, along = 0.f, shortest = 1.f;
+#pragma unroll 1
+        for (int s = 0; s < 2; ++s, members ^= 0xffffu) bound_members(lds, b, members, lengths, along, shortest);
+        float const score = lengths - along, error = lengths * kScoreError;
+        float least = fmaxf(score - error, 0.f);
+        if (shortest < kShortDiagonal) least = shortest < 0.f ? __builtin_inff() : -1.f;
+        else best = fminf(best, score + error);
+        lds->least[p][b] = least;
+        if (p == 0) lds->unscored[b] = shortest < 0.f;
+    }
+    __hip_atomic_fetch_min(&lds->bound[b], __float_as_uint(fmaxf(best, 0.f)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Which of the eight patterns 8 * wave ... could have the smallest score.
+BC6_INLINE uint32_t candidate_patterns(Bc6Ptr lds, int b, int wave)
+{
+    float const bound = __uint_as_float(lds->bound[b]);
+    uint32_t mask = 0;
+    bool unbounded = false;
 #pragma unroll
-        for (int t = 0; t < 16; ++t)
-            score += ((second >> t) & 1u) ? distance_to_line2(lo[1], dir1, px[t]) : distance_to_line2(lo[0], dir0, px[t]);
+    for (int i = 0; i < 8; ++i) {
+        float const least = lds->least[8 * wave + i][b];
+        if (least <= bound && least < __builtin_inff()) mask |= 1u << i;
+        unbounded |= least < 0.f;
+    }
+    __hip_atomic_fetch_or(&lds->candidates[b], mask << (8 * wave), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (unbounded) lds->unbounded[b] = 1u;
+    return mask;
+}
+
+// Scores, as they are defined, of the candidates among the eight patterns 8 * wave ... of blocks with more than one, each
+// lane with a pattern of its own.
+template <bool WIDE>
+BC6_TASK void score_candidates(Bc6Ptr lds, int b, int wave, uint32_t mask)
+{
+    wave = __builtin_amdgcn_readfirstlane(wave);
+    uint64_t best = ~uint64_t(0);
+#pragma unroll 1
+    for (; mask; mask &= mask - 1u) {
+        int const p = 8 * wave + __ffs(int(mask)) - 1;
+        uint32_t const second = kSecondSubset[p];
+        V3 lo0{ kHalfMax, kHalfMax, kHalfMax }, hi0{ 0.f, 0.f, 0.f }, lo1 = lo0, hi1 = hi0;
+#pragma unroll 4
+        for (int t = 0; t < 16; ++t) {
+            V3 const q = texel(lds, b, t);
+            if ((second >> t) & 1u) { lo1 = vmin(lo1, q); hi1 = vmax(hi1, q); }
+            else                    { lo0 = vmin(lo0, q); hi0 = vmax(hi0, q); }
+        }
+        V3 const dir0 = normalized<WIDE>(hi0 - lo0), dir1 = normalized<WIDE>(hi1 - lo1);
+        float score = 0.f;
+#pragma unroll 4
+        for (int t = 0; t < 16; ++t) {
+            bool const s = (second >> t) & 1u;
+            V3 const lo{ s ? lo1.x : lo0.x, s ? lo1.y : lo0.y, s ? lo1.z : lo0.z }, dir{ s ? dir1.x : dir0.x, s ? dir1.y : dir0.y, s ? dir1.z : dir0.z };
+            score += distance_to_line2(lo, dir, texel(lds, b, t));
+        }
         // scores are not negative, a NaN's bits are above all numbers': the smallest key is the first smallest score
         uint64_t const key = uint64_t(__float_as_uint(score) & 0x7fffffffu) << 32 | uint32_t(p);
         best = key < best ? key : best;
@@ -514,10 +588,23 @@ bc6_compress_kernel(BlockCompressArgs a)
         if (inside) source_pixel(a, a.srcLeft + bx * 4 + i, a.srcTop + by * 4 + wave, c);
         shared.texels[4 * wave + i][lane] = make_float4(clampf(c[0], 0.f, kHalfMax), clampf(c[1], 0.f, kHalfMax), clampf(c[2], 0.f, kHalfMax), 0.f);
     }
-    if (wave == 0) { shared.pick[lane] = ~uint64_t(0); if (lane == 0) shared.next = 0; }
+    if (wave == 0) {
+        shared.pick[lane] = ~uint64_t(0);
+        shared.bound[lane] = 0x7f800000u; shared.candidates[lane] = shared.unbounded[lane] = 0u;
+        if (lane == 0) shared.next = 0;
+    }
     __syncthreads();
     if (wave == 0) one_subset_ends<WIDE>(lds, lane);
-    score_patterns<WIDE>(lds, lane);
+    bound_scores(lds, lane);
+    __syncthreads();
+    uint32_t mask = candidate_patterns(lds, lane, wave);
+    __syncthreads();
+    uint32_t const candidates = shared.candidates[lane];
+    if ((candidates & (candidates - 1u)) == 0u && !shared.unbounded[lane]) {
+        if (mask) shared.pick[lane] = uint32_t(8 * wave + __ffs(int(mask)) - 1);
+        mask = 0u;
+    }
+    if (__any(mask != 0u)) score_candidates<WIDE>(lds, lane, wave, mask);
     __syncthreads();
     if (wave < 2) subset_ends<WIDE>(lds, lane, wave);
     __syncthreads();

@@ -238,3 +238,30 @@ def test_gpu_bc6_over_each_formats_range(ntc, device, oracle, fmt, blocks_x, blo
     got = compress(ntc, None, device, image, fmt, 3, 6, blocks_x, blocks_y)
     bad = np.argwhere(got != want)
     assert bad.size == 0, (fmt, len(bad), bad[:3], [hex(int(got[tuple(b)])) for b in bad[:3]], [hex(int(want[tuple(b)])) for b in bad[:3]])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt,diagonal", [(1, 3.0), (3, 0.5), (4, 0.5), (4, 3e-14), (4, 1e-15), (4, 1e-22)])
+def test_gpu_bc6_equal_and_short_patterns(ntc, device, oracle, fmt, diagonal):
+    """Blocks whose patterns score alike (symmetric ones, two colours that a pattern separates, one texel of its own) and
+    whose boxes' diagonals reach from ordinary lengths to ones whose squares underflow: the first of the smallest scores
+    decides."""
+    rng = np.random.default_rng(661)
+    blocks_x, blocks_y = 16, 6
+    h, w = 4 * blocks_y, 4 * blocks_x
+    dtype = {1: np.uint8, 3: np.float16, 4: np.float32}[fmt]
+    image = np.zeros((h, w, 3), dtype=np.float64)
+    for by in range(blocks_y):
+        for bx in range(blocks_x):
+            t = rng.random((4, 4, 3)) * diagonal
+            if by == 0: t = t + t.transpose(1, 0, 2)
+            elif by == 1: t = t + t[::-1] + t[:, ::-1] + t[::-1, ::-1]
+            elif by == 2: t = np.where((rng.random((4, 4, 1)) < 0.5) if bx & 1 else (np.arange(4) < 2)[:, None, None], t[0, 0], t[3, 3])
+            elif by == 3: t = np.broadcast_to(t[0, 0], t.shape).copy(); t[bx // 4, bx % 4] += diagonal
+            elif by == 4: t[...] = t[..., :1]
+            image[4 * by: 4 * by + 4, 4 * bx: 4 * bx + 4] = t
+    image = np.ascontiguousarray(image.astype(dtype))
+    want = compress(ntc, oracle, None, image, fmt, 3, 6, blocks_x, blocks_y)
+    got = compress(ntc, None, device, image, fmt, 3, 6, blocks_x, blocks_y)
+    bad = np.argwhere(got != want)
+    assert bad.size == 0, (fmt, diagonal, len(bad), bad[:3])
