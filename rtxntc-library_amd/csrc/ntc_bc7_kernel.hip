@@ -538,6 +538,7 @@ BC7_INLINE void store_block(BlockCompressArgs const& a, int bx, int by, uint64_t
 // 512 x 512, 0.29 for 1024 x 1024 and 0.95 for 2048 x 2048 (half of it opaque), where every issue slot of the vector units
 // is taken.
 enum { kSlots = 10, kPickThree = 0, kPickTwo, kPickTwoAlpha, kPicks };
+enum : uint32_t { kBelowOne = 1, kNotOne = 2 };              // what some alpha of a block is (one above 1 or a NaN is only the second)
 
 template <int BLOCKS_>
 struct SearchLds {
@@ -546,7 +547,7 @@ struct SearchLds {
     uint64_t picks[kPicks][BLOCKS];                          // error bits << 32 | partition
     uint4 words[kSlots][BLOCKS];
     float errors[kSlots][BLOCKS];
-    uint32_t withAlpha[BLOCKS];
+    uint32_t alphas[BLOCKS];                                 // kBelowOne | kNotOne
     uint8_t blocks[2][BLOCKS];                               // numbers of the opaque blocks, of those with alpha
     int counts[2];
 };
@@ -1024,29 +1025,29 @@ bc7_compress_kernel(BlockCompressArgs a)
     auto const block_y = [&](int b) { return int(blockIdx.y) * 8 + ((b >> 3) & 7); };
 
     for (int i = tid; i < BLOCKS; i += THREADS) {
-        shared.withAlpha[i] = 0u;
+        shared.alphas[i] = 0u;
         for (int k = 0; k < kPicks; ++k) shared.picks[k][i] = ~uint64_t(0);
     }
     __syncthreads();
     if (int const b = tid % BLOCKS, row = tid / BLOCKS; row < 4) {
         int const bx = block_x(b), by = block_y(b);
         bool const inside = bx < a.widthInBlocks && by < a.heightInBlocks;
-        bool alpha = false;
+        uint32_t alphas = 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             float c[4] = { 0.f, 0.f, 0.f, 0.f };
             if (inside) source_pixel(a, a.srcLeft + bx * 4 + i, a.srcTop + by * 4 + row, c);
-            alpha = alpha || c[3] < 1.f;
+            alphas |= (c[3] < 1.f ? kBelowOne : 0u) | (c[3] != 1.f ? kNotOne : 0u);
             shared.texels[4 * row + i][b] = make_float4(c[0], c[1], c[2], c[3]);
         }
-        if (alpha && inside) shared.withAlpha[b] = 1u;
+        if (alphas && inside) atomicOr(&shared.alphas[b], alphas);
     }
     __syncthreads();
     if (wave < 2) {                                          // wave 0 lists the opaque blocks, wave 1 those with alpha
         int count = 0;
         for (int g = 0; g < GROUPS; ++g) {
             int const b = 64 * g + lane;
-            bool const mine = block_x(b) < a.widthInBlocks && block_y(b) < a.heightInBlocks && int(shared.withAlpha[b]) == wave;
+            bool const mine = block_x(b) < a.widthInBlocks && block_y(b) < a.heightInBlocks && int(shared.alphas[b] & kBelowOne) == wave;
             uint64_t const ballot = __ballot(mine);
             if (mine) shared.blocks[wave][count + int(__builtin_amdgcn_mbcnt_hi(uint32_t(ballot >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(ballot), 0u)))] = uint8_t(b);
             count += __popcll(ballot);
@@ -1062,9 +1063,21 @@ bc7_compress_kernel(BlockCompressArgs a)
     // ---- 1. partitions
     for (int task = wave; task < (2 * opaqueGroups + alphaGroups) * CHUNKS; task += WAVES) {
         int const first = (task % CHUNKS) * CHUNK, what = task / CHUNKS;
-        if (what >= 2 * opaqueGroups) pick_task<S, 2, 4, false, true>(lds, block_of(1, what - 2 * opaqueGroups), first, first + CHUNK);
-        else if (what & 1)            pick_task<S, 2, 3, true, true>(lds, block_of(0, what >> 1), first, first + CHUNK);     // mode 7's too: alpha is 1, its terms are zeros
-        else                          pick_task<S, 3, 3, true, false>(lds, block_of(0, what >> 1), first, first + CHUNK);
+        if (what >= 2 * opaqueGroups) {
+            pick_task<S, 2, 4, false, true>(lds, block_of(1, what - 2 * opaqueGroups), first, first + CHUNK);
+        } else if (what & 1) {
+            // Mode 7's partition comes with it where every alpha is 1, whose terms are zeros.  Opaque blocks of float
+            // images can hold alphas above 1 and NaNs: their groups estimate it over four channels, as blocks with alpha.
+            int const b = block_of(0, what >> 1);
+            if (__ballot(shared.alphas[b] & kNotOne) == 0) {
+                pick_task<S, 2, 3, true, true>(lds, b, first, first + CHUNK);
+            } else {
+                pick_task<S, 2, 3, true, false>(lds, b, first, first + CHUNK);
+                pick_task<S, 2, 4, false, true>(lds, b, first, first + CHUNK);
+            }
+        } else {
+            pick_task<S, 3, 3, true, false>(lds, block_of(0, what >> 1), first, first + CHUNK);
+        }
     }
     __syncthreads();
 
@@ -1104,7 +1117,7 @@ bc7_compress_kernel(BlockCompressArgs a)
         if (bx < a.widthInBlocks && by < a.heightInBlocks) {
             float bestError = FLT_MAX;
             uint4 best = make_uint4(0u, 0u, 0u, 0u);
-            for (int slot = shared.withAlpha[b] ? 4 : 0; slot < kSlots; ++slot)
+            for (int slot = (shared.alphas[b] & kBelowOne) ? 4 : 0; slot < kSlots; ++slot)
                 if (!(shared.errors[slot][b] > bestError)) { bestError = shared.errors[slot][b]; best = shared.words[slot][b]; }
             store_block(a, bx, by, uint64_t(best.x) | uint64_t(best.y) << 32, uint64_t(best.z) | uint64_t(best.w) << 32);
         }

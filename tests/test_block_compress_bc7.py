@@ -396,6 +396,33 @@ def test_gpu_bc7_infinite_and_huge_texels_match_checker(ntc, device, oracle):
     assert np.array_equal(compress_bc7(ntc, None, device, *args), compress_bc7(ntc, oracle, None, *args))
 
 
+def opaque_blocks_for_mode_7(rng, w, h, dtype, alpha):
+    """Blocks of one colour that mode 7 alone holds exactly (odd 6-bit codes with different bits 4 and 5: their 8-bit forms
+    have no common lowest bit, as modes 3 and 6 want it, and are no 7-bit codes either), opaque by the search's rule (no
+    alpha below 1).  Their colours estimate every partition alike, so that alphas other than 1 alone decide mode 7's."""
+    n = w * h // 16
+    code = rng.integers(0, 8, (n, 3)) * 2 + 1 + np.array([0x10, 0x20, 0x10])
+    blocks = np.ones((n, 16, 4), dtype=np.float32)
+    blocks[:, :, :3] = ((code << 2) | (code >> 4))[:, None, :] / np.float32(255)
+    if alpha == "above":                                     # up to 1.003, on none, some or all texels of a block
+        blocks[:, :, 3] += np.where(rng.random((n, 16)) < rng.choice([0.0, 0.1, 0.5, 1.0], (n, 1)), rng.integers(1, 4, (n, 16)), 0) / 1024
+    else:                                                    # a NaN in one block of ten
+        bad = np.flatnonzero(rng.random(n) < 0.1)
+        blocks[bad, rng.integers(0, 16, bad.size), 3] = np.nan
+    return np.ascontiguousarray(blocks.reshape(h // 4, w // 4, 4, 4, 4).transpose(0, 2, 1, 3, 4).reshape(h, w, 4).astype(dtype))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("alpha", ["above", "nan"])
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("size", [(64, 64), (520, 520)])   # workgroups of one group of 64 blocks, and of two
+def test_gpu_bc7_opaque_blocks_whose_alpha_is_not_one_match_checker(ntc, device, oracle, size, dtype, alpha):
+    """Mode 7 estimates its partition over all four channels, also where no alpha is below 1."""
+    image = opaque_blocks_for_mode_7(np.random.default_rng(79), *size, dtype, alpha)
+    args = (image, 3 if dtype == np.float16 else 4, 4, size[0] // 4, size[1] // 4)
+    assert np.array_equal(compress_bc7(ntc, None, device, *args), compress_bc7(ntc, oracle, None, *args))
+
+
 @pytest.mark.gpu
 def test_gpu_bc7_arguments(ntc, device, oracle):
     from test_image_difference import fill_image
