@@ -487,6 +487,16 @@ int grid_size_for(Library const& L, int variant, int totalTiles)
     return rounds < resident ? int(rounds) : resident;
 }
 
+// Nothing of the loss pass is left; the stream is idle.  The next call makes it anew.
+void release_loss_workspace(Library& L)
+{
+    if (L.lossDev) (void)hipFree(L.lossDev);
+    if (L.lossCounters) (void)hipFree(L.lossCounters);
+    if (L.lossHost) (void)hipHostFree(L.lossHost);
+    L.lossDev = nullptr; L.lossCounters = nullptr; L.lossHost = L.lossHostOnDevice = nullptr;
+    L.lossBlocks = 0;
+}
+
 // The hand-off word of a launch pair of the FP8 network: the context's own or, for ntc_hip_decode_static (which uses
 // nothing of the context's device memory), the one behind the per-device table.
 Fp8Handoff next_handoff(Library& L, bool useStatic)
@@ -584,9 +594,7 @@ static void destroy_context(NtcHipContext* L)
     (void)hipStreamSynchronize(L->stream);
     if (L->tableDev) (void)hipFree(L->tableDev);
     if (L->handoffDev) (void)hipFree(L->handoffDev);
-    if (L->lossDev) (void)hipFree(L->lossDev);
-    if (L->lossCounters) (void)hipFree(L->lossCounters);
-    if (L->lossHost) (void)hipHostFree(L->lossHost);
+    release_loss_workspace(*L);
     for (Library::Slot& slot : L->slots) {
         if (slot.host) (void)hipHostFree(slot.host);
         if (slot.done) (void)hipEventDestroy(slot.done);
@@ -1074,6 +1082,10 @@ int ntc_hip_ctx_image_loss(NtcHipContext* ctx, void* decoded, const void* refere
                     HIP_TRY(hipStreamSynchronize(L.stream));
                     done = true;                             // read this word once more
                 }
+            }
+            if (uint32_t(words[w] >> 32) != work.serial) {   // the launch is complete and did not store it
+                release_loss_workspace(L);                   // (its counters are in no known state either)
+                return hip_fail("image_loss_kernel", hipErrorUnknown);
             }
         }
         for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) {

@@ -1,0 +1,67 @@
+"""Host code of the C ABI (csrc/ntc_hip_api.cpp) where the runtime fails or is late, on the CPU: the file's object linked
+with a runtime on host memory (fake_hip_runtime.cpp) whose calls can be made to fail and whose launches stay outstanding
+until they are waited for."""
+import ctypes as C
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "rtxntc-library_amd", "csrc")
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+
+@pytest.fixture(scope="module")
+def library(tmp_path_factory):
+    if not shutil.which(HIPCC):
+        pytest.skip("hipcc not found")
+    out = tmp_path_factory.mktemp("fake")
+    flags = ["-O1", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-x", "hip"]
+    sources = [os.path.join(CSRC, "ntc_hip_api.cpp"), os.path.join(HERE, "fake_hip_runtime.cpp")]
+    objects = [str(out / f"{i}.o") for i in range(2)]
+    builds = [subprocess.Popen([HIPCC, *flags, "-c", s, "-o", o], stderr=subprocess.PIPE) for s, o in zip(sources, objects)]
+    for b in builds:
+        text = b.communicate(timeout=300)[1]
+        assert b.returncode == 0, text.decode()
+    path = str(out / "libntc_fake.so")
+    subprocess.run(["g++", "-shared", "-Wl,-z,defs", "-Wl,-Bsymbolic", "-o", path, *objects], check=True, timeout=300)
+    return path
+
+
+@pytest.fixture
+def fake(ntc, library):
+    """The library with its exports typed and a context made, both gone after the test."""
+    lib = C.CDLL(library)
+    for name, restype, argtypes in ntc.abi.EXPORTS:
+        getattr(lib, name).restype, getattr(lib, name).argtypes = restype, argtypes
+    handle = C.c_void_p()
+    assert lib.ntc_hip_create(0, C.byref(handle)) == 0, lib.ntc_hip_last_error()
+    lib.context = handle
+    yield lib
+    lib.ntc_hip_destroy(handle)
+    assert lib.fake_allocations() == 0
+
+
+def loss(lib, width=64, height=64, mask=-1):
+    """-> (return code, the 16 values)"""
+    a, b = np.zeros(width * height * 16, dtype=np.float16), np.zeros(width * height * 16, dtype=np.float16)
+    out = (C.c_float * 16)()
+    code = lib.ntc_hip_ctx_image_loss(lib.context, a.ctypes.data, b.ctypes.data, a.nbytes, width, height, 16, 0xFFFF, mask, 0, out)
+    return code, list(out)
+
+
+EXPECTED = [float(c + 1) for c in range(16)]
+
+
+@pytest.mark.parametrize("mask", [-1, 3])
+@pytest.mark.parametrize("size", [1, 64, 512, 1024])
+def test_image_loss_whose_sums_do_not_arrive_is_an_error(fake, size, mask):
+    assert loss(fake, size, size, mask) == (0, EXPECTED)
+    fake.fake_drop_rows(1)
+    code, _ = loss(fake, size, size, mask)
+    assert code != 0 and b"image_loss" in fake.ntc_hip_last_error()
+    assert loss(fake, size, size, mask) == (0, EXPECTED)                # and the next call is whole again
+    assert fake.fake_dirty_counters() == 0
