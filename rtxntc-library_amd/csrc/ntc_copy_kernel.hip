@@ -1246,13 +1246,13 @@ image_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int 
 }
 
 hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int height, int setChannels, uint32_t validChannelMask,
-                             int maskChannel, int discardMaskedOut, LossWorkspace const& work, hipStream_t stream)
+                             int maskChannel, int discardMaskedOut, LossWorkspace const& work, hipStream_t stream, hipEvent_t done)
 {
     LossGrid const grid = image_loss_grid(width, height, compute_units_of_current_device());
     bool const two = (width & 1) == 0, masked = maskChannel >= 0;
     auto launch = [&](auto perLane, auto masks) {
         constexpr auto kernel = image_loss_kernel<decltype(perLane)::value, decltype(masks)::value>;
-        return launch_kernel<kernel>(dim3(grid.x, grid.y), dim3(256), 0, stream, a, b, width, height, setChannels, grid.rowsPerWave,
+        return launch_kernel_with_event<kernel>(dim3(grid.x, grid.y), dim3(256), 0, stream, done, a, b, width, height, setChannels, grid.rowsPerWave,
                                      validChannelMask, maskChannel, discardMaskedOut, grid.x, grid.x * grid.y, grid.groupSize, work);
     };
     auto of_width = [&](auto perLane) { return masked ? launch(perLane, std::true_type{}) : launch(perLane, std::false_type{}); };

@@ -140,8 +140,9 @@ struct LossWorkspace {
     LossRow* rows;                 // kLossRows, device address
     uint32_t serial;
 };
+// `done` completes with the launch.
 hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int height, int setChannels, uint32_t validChannelMask,
-                             int maskChannel, int discardMaskedOut, LossWorkspace const& work, hipStream_t stream);
+                             int maskChannel, int discardMaskedOut, LossWorkspace const& work, hipStream_t stream, hipEvent_t done);
 
 hipError_t launch_resize_planar(uint16_t const* src, int srcWidth, int srcHeight, uint16_t* dst, int dstWidth, int dstHeight,
                                 int setChannels, uint8_t const* colorSpaces, hipStream_t stream);

@@ -88,6 +88,7 @@ struct NtcHipContext {
     LossRow* lossHost = nullptr;       // pinned: what the loss pass hands to the host
     LossRow* lossHostOnDevice = nullptr;  // its device address
     uint32_t lossSerial = 0;
+    hipEvent_t lossDone = nullptr;     // completes with the last loss pass
     static constexpr int kSlots = 4;
     struct Slot { DevMip* host = nullptr; size_t capacity = 0; hipEvent_t done = nullptr; bool inFlight = false; };
     Slot slots[kSlots];                // pinned staging for asynchronous table uploads
@@ -493,7 +494,8 @@ void release_loss_workspace(Library& L)
     if (L.lossDev) (void)hipFree(L.lossDev);
     if (L.lossCounters) (void)hipFree(L.lossCounters);
     if (L.lossHost) (void)hipHostFree(L.lossHost);
-    L.lossDev = nullptr; L.lossCounters = nullptr; L.lossHost = L.lossHostOnDevice = nullptr;
+    if (L.lossDone) (void)hipEventDestroy(L.lossDone);
+    L.lossDev = nullptr; L.lossCounters = nullptr; L.lossHost = L.lossHostOnDevice = nullptr; L.lossDone = nullptr;
     L.lossBlocks = 0;
 }
 
@@ -1018,6 +1020,48 @@ int ntc_hip_ctx_write_channels(NtcHipContext* ctx, const NtcHipWriteChannels* p)
     return 0;
 }
 
+// Adds up the rows that the loss launch `serial` stores; every word of them carries that number.  `wait`: for words that
+// are not there yet, up to a point in time.  False if one is missing.
+static bool add_loss_rows(Library const& L, size_t rows, uint32_t serial, std::chrono::steady_clock::time_point wait, double (&totals)[NTC_HIP_DEV_MAX_CHANNELS])
+{
+    for (double& t : totals) t = 0.0;
+    for (size_t r = 0; r < rows; ++r) {
+        uint64_t words[32];
+        for (int w = 31; w >= 0; --w)
+            while (words[w] = __atomic_load_n(&L.lossHost[r].words[w], __ATOMIC_ACQUIRE), uint32_t(words[w] >> 32) != serial) {
+                if (std::chrono::steady_clock::now() >= wait) return false;
+                __builtin_ia32_pause();
+            }
+        for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) {
+            uint64_t const bits = (words[2 * c] & 0xffffffffu) | words[2 * c + 1] << 32;
+            double sum;
+            std::memcpy(&sum, &bits, sizeof(sum));
+            totals[c] += sum;
+        }
+    }
+    return true;
+}
+
+// Waits for the loss launch `serial` and takes its sums.  They arrive 1 to 2 us before the launch's event completes, and
+// with that everything the stream held before: the host looks for the sums first, reads them meanwhile (after the event
+// that takes 2 us by itself) and then asks for the event (a stream synchronisation puts a packet of its own behind the
+// launch).  A launch that takes longer than most, or work queued in front of it, is slept on.
+static int finish_loss(Library& L, size_t rows, uint32_t serial, double (&totals)[NTC_HIP_DEV_MAX_CHANNELS])
+{
+    auto const patience = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+    bool whole = add_loss_rows(L, rows, serial, patience, totals);
+    hipError_t e;
+    while ((e = hipEventQuery(L.lossDone)) == hipErrorNotReady) {
+        (void)hipGetLastError();                             // not an error that a later call should find
+        if (std::chrono::steady_clock::now() >= patience) e = hipEventSynchronize(L.lossDone);
+        if (e != hipErrorNotReady) break;
+        __builtin_ia32_pause();
+    }
+    HIP_TRY(e);
+    if (!whole) whole = add_loss_rows(L, rows, serial, {}, totals);
+    return whole ? 0 : hip_fail("image_loss_kernel", hipErrorUnknown);      // complete, and a sum missing
+}
+
 int ntc_hip_ctx_image_loss(NtcHipContext* ctx, void* decoded, const void* reference, uint64_t planarBytes, int32_t width, int32_t height, int32_t setChannels, uint32_t validChannelMask, int32_t maskChannelIndex, int32_t discardMaskedOutPixels, float* outMse)
 {
     CTX_ENTER(ctx);
@@ -1050,6 +1094,7 @@ int ntc_hip_ctx_image_loss(NtcHipContext* ctx, void* decoded, const void* refere
             HIP_TRY(hipMalloc(reinterpret_cast<void**>(&L.lossCounters), kLossRows * sizeof(uint32_t)));
             HIP_TRY(launch_fill(reinterpret_cast<uint8_t*>(L.lossCounters), 0, kLossRows * sizeof(uint32_t), L.stream));
         }
+        if (!L.lossDone) HIP_TRY(hipEventCreateWithFlags(&L.lossDone, hipEventDisableTiming));
         if (!L.lossHost) {
             HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&L.lossHost), kLossRows * sizeof(LossRow), hipHostMallocMapped | hipHostMallocCoherent));
             std::memset(L.lossHost, 0, kLossRows * sizeof(LossRow));
@@ -1064,36 +1109,11 @@ int ntc_hip_ctx_image_loss(NtcHipContext* ctx, void* decoded, const void* refere
     work.rows = L.lossHostOnDevice;
     HIP_TRY(launch_image_loss(static_cast<uint16_t*>(decoded), static_cast<uint16_t const*>(reference), width, height,
                               setChannels, validChannelMask, maskChannelIndex < 0 ? -1 : maskChannelIndex,
-                              discardMaskedOutPixels ? 1 : 0, work, L.stream));
-    // Every word of the rows that the kernel stores carries the call's serial number.  Most calls are done in
-    // microseconds, so the host looks for it; one that takes longer (work queued in front of it), or an error, is left
-    // to the stream.  So is a call with a mask channel, which changes the decoded image: it returns when that is complete.
-    auto const begin = std::chrono::steady_clock::now();
-    bool const synchronized = maskChannelIndex >= 0;
-    if (synchronized) HIP_TRY(hipStreamSynchronize(L.stream));
-    bool done = synchronized;
-    double totals[NTC_HIP_DEV_MAX_CHANNELS] = {};
-    for (size_t r = 0; r < rows; ++r) {
-        uint64_t words[32];
-        for (int w = 31; w >= 0; --w) {
-            while (words[w] = __atomic_load_n(&L.lossHost[r].words[w], __ATOMIC_ACQUIRE), uint32_t(words[w] >> 32) != work.serial && !done) {
-                __builtin_ia32_pause();
-                if (std::chrono::steady_clock::now() - begin > std::chrono::milliseconds(2)) {
-                    HIP_TRY(hipStreamSynchronize(L.stream));
-                    done = true;                             // read this word once more
-                }
-            }
-            if (uint32_t(words[w] >> 32) != work.serial) {   // the launch is complete and did not store it
-                release_loss_workspace(L);                   // (its counters are in no known state either)
-                return hip_fail("image_loss_kernel", hipErrorUnknown);
-            }
-        }
-        for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) {
-            uint64_t const bits = (words[2 * c] & 0xffffffffu) | words[2 * c + 1] << 32;
-            double sum;
-            std::memcpy(&sum, &bits, sizeof(sum));
-            totals[c] += sum;
-        }
+                              discardMaskedOutPixels ? 1 : 0, work, L.stream, L.lossDone));
+    double totals[NTC_HIP_DEV_MAX_CHANNELS];
+    if (int r = finish_loss(L, rows, work.serial, totals)) {
+        release_loss_workspace(L);                           // (its counters are in no known state)
+        return r;
     }
     double const norm = 1.0 / (double(width) * double(height));
     for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) outMse[c] = float(totals[c] * norm);

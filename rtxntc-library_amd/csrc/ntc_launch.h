@@ -2,7 +2,9 @@
 #ifndef NTC_LAUNCH_H
 #define NTC_LAUNCH_H
 #include <hip/hip_runtime.h>
+#include <hip/hip_ext.h>
 #include <atomic>
+#include <stdint.h>
 
 namespace ntc_hip_dev {
 
@@ -13,7 +15,7 @@ namespace ntc_hip_dev {
 template <class> struct KernelParameters;
 template <class... T> struct KernelParameters<void (*)(T...)> {
     template <auto KERNEL>
-    static hipError_t launch(dim3 grid, dim3 block, size_t ldsBytes, hipStream_t stream, T... args)
+    static hipError_t launch(dim3 grid, dim3 block, size_t ldsBytes, hipStream_t stream, hipEvent_t done, T... args)
     {
         constexpr int kDevices = 64;
         static std::atomic<hipFunction_t> functions[kDevices];
@@ -26,13 +28,23 @@ template <class... T> struct KernelParameters<void (*)(T...)> {
             if (kept) functions[device].store(function, std::memory_order_release);
         }
         void* pointers[] = { const_cast<void*>(static_cast<void const*>(&args))... };
+        if (done) {                                          // (takes threads, not workgroups)
+            if (uint64_t(grid.x) * block.x > 0xffffffffu || uint64_t(grid.y) * block.y > 0xffffffffu) return hipErrorInvalidConfiguration;
+            return hipExtModuleLaunchKernel(function, grid.x * block.x, grid.y * block.y, grid.z * block.z, block.x, block.y, block.z, ldsBytes, stream, pointers, nullptr, nullptr, done);
+        }
         return hipModuleLaunchKernel(function, grid.x, grid.y, grid.z, block.x, block.y, block.z, unsigned(ldsBytes), stream, pointers, nullptr);
     }
 };
 template <auto KERNEL, class... ARGS>
 inline hipError_t launch_kernel(dim3 grid, dim3 block, size_t ldsBytes, hipStream_t stream, ARGS const&... args)
 {
-    return KernelParameters<decltype(KERNEL)>::template launch<KERNEL>(grid, block, ldsBytes, stream, args...);
+    return KernelParameters<decltype(KERNEL)>::template launch<KERNEL>(grid, block, ldsBytes, stream, nullptr, args...);
+}
+// The same with an event that completes with the launch itself: no packet of its own, as a recorded event is.
+template <auto KERNEL, class... ARGS>
+inline hipError_t launch_kernel_with_event(dim3 grid, dim3 block, size_t ldsBytes, hipStream_t stream, hipEvent_t done, ARGS const&... args)
+{
+    return KernelParameters<decltype(KERNEL)>::template launch<KERNEL>(grid, block, ldsBytes, stream, done, args...);
 }
 
 } // namespace ntc_hip_dev

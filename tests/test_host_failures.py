@@ -65,3 +65,14 @@ def test_image_loss_whose_sums_do_not_arrive_is_an_error(fake, size, mask):
     assert code != 0 and b"image_loss" in fake.ntc_hip_last_error()
     assert loss(fake, size, size, mask) == (0, EXPECTED)                # and the next call is whole again
     assert fake.fake_dirty_counters() == 0
+
+
+@pytest.mark.parametrize("mask", [-1, 3])
+def test_image_loss_is_synchronous(fake, mask):
+    """What the stream held, the launch included, is complete when the call returns, and an error of it is the call's."""
+    for _ in range(2):
+        assert loss(fake, mask=mask) == (0, EXPECTED)
+        assert fake.fake_outstanding() == 0
+    fake.fake_fail(b"hipEventSynchronize", 1)
+    assert loss(fake, mask=mask)[0] != 0
+    assert loss(fake, mask=mask) == (0, EXPECTED) and fake.fake_dirty_counters() == 0
