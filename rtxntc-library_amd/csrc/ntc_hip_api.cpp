@@ -499,6 +499,25 @@ void release_loss_workspace(Library& L)
     L.lossBlocks = 0;
 }
 
+// Room for the partial sums of `blocks` workgroups, and whatever else of the loss pass is not there yet.  All of it or an
+// error, after which the caller releases it.
+int prepare_loss_workspace(Library& L, size_t blocks)
+{
+    if (L.lossBlocks != 0) HIP_TRY(hipStreamSynchronize(L.stream));
+    if (L.lossDev) { HIP_TRY(hipFree(L.lossDev)); L.lossDev = nullptr; }
+    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&L.lossDev), blocks * NTC_HIP_DEV_MAX_CHANNELS * sizeof(double)));
+    if (L.lossBlocks == 0) {
+        HIP_TRY(hipMalloc(reinterpret_cast<void**>(&L.lossCounters), kLossRows * sizeof(uint32_t)));
+        HIP_TRY(launch_fill(reinterpret_cast<uint8_t*>(L.lossCounters), 0, kLossRows * sizeof(uint32_t), L.stream));
+        HIP_TRY(hipEventCreateWithFlags(&L.lossDone, hipEventDisableTiming));
+        HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&L.lossHost), kLossRows * sizeof(LossRow), hipHostMallocMapped | hipHostMallocCoherent));
+        std::memset(L.lossHost, 0, kLossRows * sizeof(LossRow));
+        HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void**>(&L.lossHostOnDevice), L.lossHost, 0));
+    }
+    L.lossBlocks = blocks;
+    return 0;
+}
+
 // The hand-off word of a launch pair of the FP8 network: the context's own or, for ntc_hip_decode_static (which uses
 // nothing of the context's device memory), the one behind the per-device table.
 Fp8Handoff next_handoff(Library& L, bool useStatic)
@@ -1085,23 +1104,11 @@ int ntc_hip_ctx_image_loss(NtcHipContext* ctx, void* decoded, const void* refere
     }
     LossGrid const grid = image_loss_grid(width, height, L.computeUnits);
     size_t const blocks = size_t(grid.x) * grid.y, rows = (blocks + grid.groupSize - 1) / grid.groupSize;
-    if (blocks > L.lossBlocks) {
-        HIP_TRY(hipStreamSynchronize(L.stream));
-        if (L.lossDev) { HIP_TRY(hipFree(L.lossDev)); L.lossDev = nullptr; }
-        L.lossBlocks = 0;
-        HIP_TRY(hipMalloc(reinterpret_cast<void**>(&L.lossDev), blocks * NTC_HIP_DEV_MAX_CHANNELS * sizeof(double)));
-        if (!L.lossCounters) {
-            HIP_TRY(hipMalloc(reinterpret_cast<void**>(&L.lossCounters), kLossRows * sizeof(uint32_t)));
-            HIP_TRY(launch_fill(reinterpret_cast<uint8_t*>(L.lossCounters), 0, kLossRows * sizeof(uint32_t), L.stream));
+    if (blocks > L.lossBlocks)
+        if (int r = prepare_loss_workspace(L, blocks)) {
+            release_loss_workspace(L);
+            return r;
         }
-        if (!L.lossDone) HIP_TRY(hipEventCreateWithFlags(&L.lossDone, hipEventDisableTiming));
-        if (!L.lossHost) {
-            HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&L.lossHost), kLossRows * sizeof(LossRow), hipHostMallocMapped | hipHostMallocCoherent));
-            std::memset(L.lossHost, 0, kLossRows * sizeof(LossRow));
-            HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void**>(&L.lossHostOnDevice), L.lossHost, 0));
-        }
-        L.lossBlocks = blocks;
-    }
     LossWorkspace work{};
     work.partials = L.lossDev;
     work.counters = L.lossCounters;

@@ -57,6 +57,7 @@ hipError_t release(void* p)
 extern "C" {
 
 // ---- the test's side
+void fake_reset() { g_failIn.clear(); g_last = hipSuccess; g_dropRows = g_dirtyCounters = g_nullStreamUses = 0; }
 void fake_fail(char const* name, int call) { g_failIn[name] = call; }
 void fake_drop_rows(int count) { g_dropRows = count; }             // so many of the next loss launches store nothing
 int fake_dirty_counters() { return g_dirtyCounters; }              // loss launches that found a counter other than zero

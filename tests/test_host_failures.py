@@ -37,6 +37,7 @@ def fake(ntc, library):
     lib = C.CDLL(library)
     for name, restype, argtypes in ntc.abi.EXPORTS:
         getattr(lib, name).restype, getattr(lib, name).argtypes = restype, argtypes
+    lib.fake_reset()
     handle = C.c_void_p()
     assert lib.ntc_hip_create(0, C.byref(handle)) == 0, lib.ntc_hip_last_error()
     lib.context = handle
@@ -76,3 +77,21 @@ def test_image_loss_is_synchronous(fake, mask):
     fake.fake_fail(b"hipEventSynchronize", 1)
     assert loss(fake, mask=mask)[0] != 0
     assert loss(fake, mask=mask) == (0, EXPECTED) and fake.fake_dirty_counters() == 0
+
+
+@pytest.mark.parametrize("call", [1, 2, 3])
+@pytest.mark.parametrize("name", ["hipMalloc", "launch_fill", "hipEventCreate", "hipHostMalloc", "hipHostGetDevicePointer", "launch_image_loss"])
+def test_image_loss_after_a_set_up_that_failed(fake, name, call):
+    """The first calls meet a failing allocation or launch (the n-th of its kind; a larger image grows the partial sums):
+    each such call returns an error, and the first one without it finds the working memory whole."""
+    fake.fake_fail(name.encode(), call)
+    codes = []
+    for size in (32, 1024, 4096, 64):
+        code, values = loss(fake, size, size)
+        codes.append(code)
+        if code != 0:
+            code, values = loss(fake, size, size)
+        assert code == 0 and values == EXPECTED, (name, size)
+    assert sum(c != 0 for c in codes) <= 1
+    fake.fake_fail(name.encode(), 1 << 30)
+    assert fake.fake_dirty_counters() == 0
