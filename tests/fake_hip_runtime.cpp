@@ -57,7 +57,7 @@ hipError_t release(void* p)
 extern "C" {
 
 // ---- the test's side
-void fake_reset() { g_failIn.clear(); g_last = hipSuccess; g_dropRows = g_dirtyCounters = g_nullStreamUses = 0; }
+void fake_reset() { g_failIn.clear(); g_last = hipSuccess; g_dropRows = g_dirtyCounters = 0; }
 void fake_fail(char const* name, int call) { g_failIn[name] = call; }
 void fake_drop_rows(int count) { g_dropRows = count; }             // so many of the next loss launches store nothing
 int fake_dirty_counters() { return g_dirtyCounters; }              // loss launches that found a counter other than zero
@@ -93,6 +93,11 @@ hipError_t hipGetSymbolAddress(void** p, void const*) { static char table[1 << 1
 hipError_t hipMemcpy(void* d, void const* s, size_t n, hipMemcpyKind) { std::memcpy(d, s, n); return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, void const* s, size_t n, hipMemcpyKind, hipStream_t) { std::memcpy(d, s, n); return hipSuccess; }
 hipError_t hipStreamCreate(hipStream_t* s) { *s = reinterpret_cast<hipStream_t>(new Stream); return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned)
+{
+    if (hipError_t const e = outcome("hipStreamCreateWithFlags")) return e;
+    return hipStreamCreate(s);
+}
 hipError_t hipStreamDestroy(hipStream_t s) { delete reinterpret_cast<Stream*>(s); return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t s)
 {

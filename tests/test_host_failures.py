@@ -46,6 +46,14 @@ def fake(ntc, library):
     assert lib.fake_allocations() == 0
 
 
+def test_contexts_leave_the_null_stream_alone(fake):
+    """Work on the null stream waits for every blocking stream of the device, and they for it."""
+    handle = C.c_void_p()
+    assert fake.ntc_hip_create(0, C.byref(handle)) == 0
+    fake.ntc_hip_destroy(handle)
+    assert fake.fake_null_stream_uses() == 0                            # since the library was loaded
+
+
 def loss(lib, width=64, height=64, mask=-1):
     """-> (return code, the 16 values)"""
     a, b = np.zeros(width * height * 16, dtype=np.float16), np.zeros(width * height * 16, dtype=np.float16)
