@@ -10,15 +10,14 @@ import pytest
 
 import oracle_lib
 from cases import cfg_case, ref_case
+from host_programs import built
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 EXE = os.path.join(HERE, "host_api_test")
 
 
 def run_exe(*args):
-    if not os.path.exists(EXE):
-        pytest.fail(f"{EXE} is not built; run __graft_entry__.build() (make -C tests)")
-    out = subprocess.run([EXE, *map(str, args)], capture_output=True, text=True, timeout=300)
+    out = subprocess.run([built(EXE), *map(str, args)], capture_output=True, text=True, timeout=300)
     assert out.returncode == 0, f"host_api_test {args[0]} failed:\n{out.stdout}\n{out.stderr}"
     return out.stdout
 

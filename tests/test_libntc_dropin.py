@@ -16,18 +16,17 @@ import numpy as np
 import pytest
 
 from cases import Case
+from host_programs import HEADER as REFERENCE_HEADER, built
 from test_ntc_file import TEXTURES, file_of, make_case, pixels_from_planar
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 EXE = os.path.join(HERE, "libntc_dropin_test")
 LIB = os.path.join(ROOT, "rtxntc-library_amd", "host", "libntc.so")
-REFERENCE_HEADER = "/root/reference/include/libntc/ntc.h"
 
 
 def run_dropin(*args, env=None):
-    if not os.path.exists(EXE):
-        pytest.fail(f"{EXE} is not built; run __graft_entry__.build() (make -C tests)")
+    built(EXE)
     full_env = dict(os.environ)
     full_env.pop("LIBNTC_ALLOW_TEXTURE_SETS_WITHOUT_DEVICE", None)
     full_env.update(env or {})
@@ -54,7 +53,7 @@ def test_every_virtual_of_the_reference_interfaces_answers(ntc, tmp_path, sets_w
 
 def test_library_exports_the_free_functions_of_the_reference_header():
     """Every NTC_API function of include/libntc/ntc.h:1307-1391, by its unmangled name."""
-    exported = subprocess.run(["nm", "-D", "--defined-only", LIB], capture_output=True, text=True, check=True).stdout
+    exported = subprocess.run(["nm", "-D", "--defined-only", built(LIB)], capture_output=True, text=True, check=True).stdout
     names = {line.split()[-1] for line in exported.splitlines() if line.strip()}
     if os.path.exists(REFERENCE_HEADER):
         text = open(REFERENCE_HEADER).read()

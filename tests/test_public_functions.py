@@ -13,6 +13,8 @@ import os
 import numpy as np
 import pytest
 
+from host_programs import built
+
 HOST_LIB = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "rtxntc-library_amd", "host", "libntc.so")
 
 
@@ -30,7 +32,7 @@ class VersionInfo(C.Structure):
 
 @pytest.fixture(scope="module")
 def host():
-    lib = C.CDLL(HOST_LIB)
+    lib = C.CDLL(built(HOST_LIB))
     for name in ("StatusToString", "ChannelFormatToString", "BlockCompressedFormatToString", "ColorSpaceToString",
                  "InferenceWeightTypeToString", "CompressionTypeToString", "GetLastErrorMessage"):
         getattr(lib, name).restype = C.c_char_p

@@ -74,6 +74,7 @@ def test_integer_layer_equals_dequantised_float_layer(oracle, n_in, n_out, input
 
 import ctypes as C
 import os
+from host_programs import built
 
 HOST_LIB = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "rtxntc-library_amd", "host", "libntc.so")
 
@@ -87,7 +88,7 @@ class OutputChannelTransform(C.Structure):
 
 
 def host_lib():
-    lib = C.CDLL(HOST_LIB)
+    lib = C.CDLL(built(HOST_LIB))
     lib.QuantizeNetworkInt8.restype = C.c_int
     lib.QuantizeNetworkInt8.argtypes = [C.POINTER(FloatLayerDesc), C.c_int, C.POINTER(OutputChannelTransform), C.c_void_p, C.c_size_t, C.POINTER(C.c_size_t)]
     lib.GetLastErrorMessage.restype = C.c_char_p
