@@ -1,0 +1,204 @@
+// exact_functions.hip - the kernels' shortcuts for divisions and for storing colours, against what they stand for, over
+// every operand they are used on (tests/test_exact_functions.py).  Compiled together with one kernel file at a time, whose
+// functions it calls: SUBJECT_COPY, SUBJECT_BC, SUBJECT_BC6 or SUBJECT_DECODE.
+#if defined(SUBJECT_COPY)
+#include "../rtxntc-library_amd/csrc/ntc_copy_kernel.hip"
+#elif defined(SUBJECT_BC)
+#include "../rtxntc-library_amd/csrc/ntc_bc_kernel.hip"
+#elif defined(SUBJECT_BC6)
+#include "../rtxntc-library_amd/csrc/ntc_bc6_kernel.hip"
+#else
+#include "../rtxntc-library_amd/csrc/ntc_decode_device.h"
+#endif
+
+using namespace ntc_hip_dev;
+
+namespace {
+
+struct Report { unsigned long long tried, wrong, example; };
+
+// CHECK: number of a case -> 0 not one, 1 right, 2 wrong.  Every wave ends after its share of the cases.
+template <class CHECK>
+__global__ void __launch_bounds__(256) sweep_kernel(uint64_t cases, Report* report)
+{
+    unsigned long long tried = 0, wrong = 0, example = 0;
+    for (uint64_t i = uint64_t(blockIdx.x) * 256u + threadIdx.x; i < cases; i += uint64_t(gridDim.x) * 256u) {
+        int const r = CHECK::check(i);
+        tried += r != 0;
+        if (r == 2) { ++wrong; example = i; }
+    }
+    atomicAdd(&report->tried, tried);
+    if (wrong) { atomicAdd(&report->wrong, wrong); report->example = example; }
+}
+template <class CHECK> int sweep(Report* out)
+{
+    Report* device = nullptr;
+    hipError_t e = hipMalloc(reinterpret_cast<void**>(&device), sizeof(Report));
+    if (e != hipSuccess) return int(e);
+    *out = Report{};
+    e = hipMemcpy(device, out, sizeof(Report), hipMemcpyHostToDevice);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(sweep_kernel<CHECK>, dim3(4096), dim3(256), 0, nullptr, CHECK::cases, device);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpy(out, device, sizeof(Report), hipMemcpyDeviceToHost);
+    (void)hipFree(device);
+    return int(e);
+}
+
+__device__ bool same(float a, float b) { return __float_as_uint(a) == __float_as_uint(b) || (a != a && b != b); }
+__device__ int verdict(bool right) { return right ? 1 : 2; }
+[[maybe_unused]] __device__ float half_of(uint32_t bits) { return float(__builtin_bit_cast(_Float16, uint16_t(bits))); }
+
+#if defined(SUBJECT_COPY)
+
+// encoded_half(): every float.
+template <int SPACE> struct EncodedHalf {
+    static constexpr uint64_t cases = uint64_t(1) << 32;
+    static __device__ int check(uint64_t i)
+    {
+        float const v = __uint_as_float(uint32_t(i));
+        uint32_t const got = encoded_half(SPACE, v), want = stored_half(encode_color_space(SPACE, v));
+        return verdict(got == want);
+    }
+};
+// divide_by_top(): every code and every offset that a draw can have.
+template <int TOP> struct DivideByTop {
+    static constexpr uint64_t cases = (uint64_t(1) << 23) + TOP + 1;
+    static __device__ int check(uint64_t i)
+    {
+        float const a = i <= TOP ? float(uint32_t(i)) : __uint_as_float(uint32_t(i - TOP - 1) | 0x3f800000u) - 1.5f;
+        return verdict(same(divide_by_top(a, float(TOP), 1.f / float(TOP)), a / float(TOP)));
+    }
+};
+
+#elif defined(SUBJECT_BC)
+
+// code_quotient(): five and six bits.
+struct CodeQuotient {
+    static constexpr uint64_t cases = 32 + 64;
+    static __device__ int check(uint64_t i)
+    {
+        float const k = float(uint32_t(i < 32 ? i : i - 32)), d = i < 32 ? 31.f : 63.f;
+        return verdict(same(code_quotient(k, d, 1.f / d), k / d));
+    }
+};
+// bc4_palette8(): every pair of endpoints.
+struct Bc4Palette {
+    static constexpr uint64_t cases = 65536;
+    static __device__ int check(uint64_t i)
+    {
+        uint32_t const e0 = uint32_t(i) >> 8, e1 = uint32_t(i) & 255u;
+        uint32_t p[8];
+        bc4_palette8(e0, e1, p);
+        bool right = p[0] == 8u * e0 && p[1] == 8u * e1;
+        for (uint32_t k = 1; k < 7; ++k) {
+            uint32_t want;
+            if (e0 > e1)    want = ((7 - k) * e0 + k * e1 + 3) / 7;
+            else if (k < 5) want = ((5 - k) * e0 + k * e1 + 2) / 5;
+            else            want = k == 5 ? 0 : 255;
+            right = right && p[k + 1] == 8u * want;
+        }
+        return verdict(right);
+    }
+};
+
+#elif defined(SUBJECT_BC6)
+
+// quotient<0>(): integers below 2^17.
+struct QuotientOfIntegers {
+    static constexpr uint64_t cases = uint64_t(1) << 34;
+    static __device__ int check(uint64_t i)
+    {
+        float const a = float(uint32_t(i) & 0x1ffffu), b = float(uint32_t(i >> 17));
+        return b == 0.f ? 0 : verdict(same(quotient<0>(a, b), a / b));
+    }
+};
+// quotient<0>(): the mantissas that normal_log2() reduces to.
+struct QuotientOfLog2 {
+    static constexpr uint64_t cases = uint64_t(1) << 25;
+    static __device__ int check(uint64_t i)
+    {
+        float const m = __uint_as_float(0x3f000000u + uint32_t(i));
+        return m < 0.70f || m > 1.42f ? 0 : verdict(same(quotient<0>(m - 1.f, m + 1.f), (m - 1.f) / (m + 1.f)));
+    }
+};
+// corrected() by reciprocal<1>(), as Msle does it: 1 + a half over 1 + a texel of any format but FLOAT32.
+struct QuotientOfMsle {
+    static constexpr uint64_t kHalves = 0x7c00, kTexels = kHalves + 256 + 65536 + 65505;
+    static constexpr uint64_t cases = kHalves * kTexels;
+    static __device__ int check(uint64_t i)
+    {
+        uint32_t const texel = uint32_t(i / kHalves);
+        float x;
+        if (texel < kHalves)                    x = half_of(texel);
+        else if (texel < kHalves + 256)         x = float(texel - uint32_t(kHalves)) / 255.f;
+        else if (texel < kHalves + 256 + 65536) x = float(texel - uint32_t(kHalves + 256)) / 65535.f;
+        else                                    x = float(texel - uint32_t(kHalves + 256 + 65536));
+        float const a = half_of(uint32_t(i % kHalves)) + 1.f, b = x + 1.f;
+        return verdict(same(corrected(a, b, reciprocal<1>(b)), a / b));
+    }
+};
+// quantize() and the indices' places.
+struct QuotientOfCodes {
+    static constexpr uint64_t cases = 3 * 65536 + 64;
+    static __device__ int check(uint64_t i)
+    {
+        if (i < 3 * 65536) {
+            float const levels = i < 65536 ? 128.f : i < 2 * 65536 ? 512.f : 1024.f, a = float(uint32_t(i & 65535u)) * levels;
+            return verdict(same(corrected(a, 31744.f, 1.f / 31744.f), a / 31744.f));
+        }
+        uint32_t const k = uint32_t(i) & 15u, kind = (uint32_t(i) >> 4) & 3u;
+        float const top = (kind & 1u) ? 15.f : 7.f, a = float(k) * ((kind & 2u) ? 64.f : 1.f);
+        return verdict(same(corrected(a, top, 1.f / top), a / top));
+    }
+};
+// quotient_by(): a component over the sum or the length of three, halves of all magnitudes.  (There are 2^45 such triples;
+// these are 2^30 of them.)
+struct QuotientOfDiagonals {
+    static constexpr uint64_t cases = uint64_t(1) << 30;
+    static __device__ int check(uint64_t i)
+    {
+        uint64_t h = (i + 1) * 0x9e3779b97f4a7c15ull;
+        h ^= h >> 29; h *= 0xbf58476d1ce4e5b9ull; h ^= h >> 32;
+        float const x = half_of(uint32_t(h) % 0x7c00u), y = half_of(uint32_t(h >> 16) % 0x7c00u), z = half_of(uint32_t(h >> 32) % 0x7c00u);
+        float const s = (i & 1) ? x + y + z : sqrtf(x * x + y * y + z * z);
+        return verdict(same(quotient_by(x, s, reciprocal<1>(s)), x / s));
+    }
+};
+
+#else
+
+// texel_centre(): every texel of every size that a mip can have.
+struct TexelCentre {
+    static constexpr uint64_t cases = uint64_t(1) << 32;
+    static __device__ int check(uint64_t i)
+    {
+        int const x = int(uint32_t(i) & 0xffffu), size = int(i >> 16) + 1;
+        return x >= size ? 0 : verdict(same(texel_centre(x, size), (float(x) + 0.5f) / float(size)));
+    }
+};
+
+#endif
+
+} // namespace
+
+extern "C" {
+#if defined(SUBJECT_COPY)
+int exact_encoded_half_srgb(Report* r) { return sweep<EncodedHalf<1>>(r); }
+int exact_encoded_half_hlg(Report* r) { return sweep<EncodedHalf<2>>(r); }
+int exact_divide_by_255(Report* r) { return sweep<DivideByTop<255>>(r); }
+int exact_divide_by_65535(Report* r) { return sweep<DivideByTop<65535>>(r); }
+#elif defined(SUBJECT_BC)
+int exact_code_quotient(Report* r) { return sweep<CodeQuotient>(r); }
+int exact_bc4_palette(Report* r) { return sweep<Bc4Palette>(r); }
+#elif defined(SUBJECT_BC6)
+int exact_quotient_of_integers(Report* r) { return sweep<QuotientOfIntegers>(r); }
+int exact_quotient_of_log2(Report* r) { return sweep<QuotientOfLog2>(r); }
+int exact_quotient_of_msle(Report* r) { return sweep<QuotientOfMsle>(r); }
+int exact_quotient_of_codes(Report* r) { return sweep<QuotientOfCodes>(r); }
+int exact_quotient_of_diagonals(Report* r) { return sweep<QuotientOfDiagonals>(r); }
+#else
+int exact_texel_centre(Report* r) { return sweep<TexelCentre>(r); }
+#endif
+}
