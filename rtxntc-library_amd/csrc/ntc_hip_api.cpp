@@ -1068,20 +1068,13 @@ static bool add_loss_rows(Library const& L, size_t rows, uint32_t serial, std::c
 
 // Waits for the loss launch `serial` and takes its sums.  They arrive 1 to 2 us before the launch's event completes, and
 // with that everything the stream held before: the host looks for the sums first, reads them meanwhile (after the event
-// that takes 2 us by itself) and then asks for the event (a stream synchronisation puts a packet of its own behind the
-// launch).  A launch that takes longer than most, or work queued in front of it, is slept on.
+// that takes 2 us by itself) and then waits for the event.  4 x 4 texels: 12.2 us a call, of which the event is 0.6 for
+// the launch and 2.4 for its end; with a stream synchronisation, which puts a packet of its own behind the launch, 14.8.
+// Launches that take longer than most, or have work queued in front of them, are slept on.
 static int finish_loss(Library& L, size_t rows, uint32_t serial, double (&totals)[NTC_HIP_DEV_MAX_CHANNELS])
 {
-    auto const patience = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
-    bool whole = add_loss_rows(L, rows, serial, patience, totals);
-    hipError_t e;
-    while ((e = hipEventQuery(L.lossDone)) == hipErrorNotReady) {
-        (void)hipGetLastError();                             // not an error that a later call should find
-        if (std::chrono::steady_clock::now() >= patience) e = hipEventSynchronize(L.lossDone);
-        if (e != hipErrorNotReady) break;
-        __builtin_ia32_pause();
-    }
-    HIP_TRY(e);
+    bool whole = add_loss_rows(L, rows, serial, std::chrono::steady_clock::now() + std::chrono::milliseconds(2), totals);
+    HIP_TRY(hipEventSynchronize(L.lossDone));
     if (!whole) whole = add_loss_rows(L, rows, serial, {}, totals);
     return whole ? 0 : hip_fail("image_loss_kernel", hipErrorUnknown);      // complete, and a sum missing
 }

@@ -135,3 +135,18 @@ def test_loss_sums_of_one_group_and_of_many(ntc, device, oracle, w, h):
         device.call("image_loss", d_a.ptr, d_b.ptr, d_a.nbytes, w, h, 6, 0x37, -1, 0, got)
         results.append(np.array(got[:]))
     assert np.allclose(results[0], want, rtol=2e-7, atol=0) and np.array_equal(results[0], results[1])
+
+
+@pytest.mark.parametrize("mask_channel", [-1, 5])
+def test_loss_behind_queued_work(ntc, device, mask_channel):
+    """Work of several milliseconds in front of the call, the last of which writes the image: the host's look for early sums
+    gives up, and the sums are those of the written image."""
+    big, w, h = device.alloc(1 << 30), 64, 64
+    d_a, d_b = device.upload(np.zeros(w * h * 6, dtype=np.uint16)), device.upload(np.zeros(w * h * 6, dtype=np.uint16))
+    got = (ntc.abi.C.c_float * 16)()
+    for _ in range(30):                                                   # 30 GB written: 4 ms at least
+        device.call("memset", big.ptr, 0, big.nbytes)
+    device.call("memset", d_a.ptr, 0x38, d_a.nbytes)                      # every half 0x3838
+    device.call("image_loss", d_a.ptr, d_b.ptr, d_a.nbytes, w, h, 6, 0x3F, mask_channel, 0, got)
+    value = float(np.array([0x3838], dtype=np.uint16).view(np.float16)[0])
+    assert np.allclose(got[:6], value * value, rtol=2e-7, atol=0) and not any(got[6:])
