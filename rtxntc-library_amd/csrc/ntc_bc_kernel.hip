@@ -28,7 +28,6 @@
 // All float arithmetic is IEEE binary32, unfused, in the order written here.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-#include <atomic>
 #include <type_traits>
 #include "ntc_decode_kernel.h"
 #include "ntc_bc_source.h"
@@ -724,22 +723,15 @@ bc1_tables_kernel()
     g_match6[threadIdx.x] = uint16_t(nearest_pair(int(threadIdx.x), 6));
 }
 
+hipError_t launch_color_tables(hipStream_t stream)
+{
+    hipLaunchKernelGGL(bc1_tables_kernel, dim3(1), dim3(256), 0, stream);
+    return hipGetLastError();
+}
+
 hipError_t launch_block_compress(BlockCompressArgs const& a, int dstFormat, hipStream_t stream)
 {
     dim3 const grid((a.widthInBlocks + 15) / 16, (a.heightInBlocks + 3) / 4);
-    if (dstFormat <= 3) {
-        // the single-colour tables are computed on the device the first time each device needs them
-        // (every launch of the library is on one stream per device, so the order is given)
-        static std::atomic<uint64_t> tablesBuilt{0};
-        int device = 0;
-        if (hipError_t const e = hipGetDevice(&device); e != hipSuccess) return e;
-        uint64_t const bit = uint64_t(1) << (device & 63);
-        if (!(tablesBuilt.load(std::memory_order_acquire) & bit)) {
-            hipLaunchKernelGGL(bc1_tables_kernel, dim3(1), dim3(256), 0, stream);
-            if (hipError_t const e = hipGetLastError(); e != hipSuccess) return e;
-            tablesBuilt.fetch_or(bit, std::memory_order_release);
-        }
-    }
     switch (dstFormat) {
     case 1: launch_bc1<1>(a, stream); break;
     case 2: launch_bc1<2>(a, stream); break;

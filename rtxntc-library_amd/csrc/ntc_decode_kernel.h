@@ -176,6 +176,8 @@ struct BlockCompressArgs {
 };
 // Sets `bytes` bytes at dst to `value` (any alignment).
 hipError_t launch_fill(uint8_t* dst, uint8_t value, uint64_t bytes, hipStream_t stream);
+// Fills the single-colour tables of the current device that BC1, BC2 and BC3 read.
+hipError_t launch_color_tables(hipStream_t stream);
 hipError_t launch_block_compress(BlockCompressArgs const& args, int dstFormat /* 1..7 */, hipStream_t stream);
 hipError_t launch_bc6_compress(BlockCompressArgs const& args, hipStream_t stream);
 hipError_t launch_bc7_compress(BlockCompressArgs const& args, hipStream_t stream);

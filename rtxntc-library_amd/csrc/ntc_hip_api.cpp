@@ -563,14 +563,15 @@ static int create_context(int device, NtcHipContext** outContext)
     {                                   // once per device, with that device current
         std::lock_guard<std::mutex> lock(g_liveMutex);
         if (!g_staticTable[device]) {
-            // the tables of the channel copies, complete before any context can use them; on a stream of their own,
-            // which waits for no other
+            // the tables of the channel copies and of BC1 to BC3, complete before any context can use them; on a stream
+            // of their own, which waits for no other
             hipStream_t tables = nullptr;
             HIP_TRY(hipStreamCreateWithFlags(&tables, hipStreamNonBlocking));
             hipError_t made = launch_transfer_tables(tables);
+            if (made == hipSuccess) made = launch_color_tables(tables);
             if (made == hipSuccess) made = hipStreamSynchronize(tables);
             (void)hipStreamDestroy(tables);
-            if (made != hipSuccess) return hip_fail("transfer_tables_kernel", made);
+            if (made != hipSuccess) return hip_fail("transfer_tables_kernel / bc1_tables_kernel", made);
             void* address = nullptr;
             HIP_TRY(hipGetSymbolAddress(&address, HIP_SYMBOL(scratch)));
             g_staticTable[device] = address;

@@ -18,6 +18,7 @@ Stream g_null;
 std::set<void*> g_memory;
 std::map<std::string, int> g_failIn;       // calls until the one that fails
 hipError_t g_last = hipSuccess;
+std::string g_launches;                    // names of the launches and of the stream waits, a line each
 int g_dropRows = 0, g_dirtyCounters = 0, g_nullStreamUses = 0;
 
 Stream* of(hipStream_t s)
@@ -36,6 +37,7 @@ hipError_t launched(char const* name, hipStream_t stream)
 {
     if (hipError_t const e = outcome(name, hipErrorLaunchFailure)) return e;
     ++of(stream)->outstanding;
+    g_launches += std::string(name) + '\n';
     return hipSuccess;
 }
 hipError_t allocate(char const* name, void** p, size_t bytes)
@@ -62,6 +64,7 @@ void fake_fail(char const* name, int call) { g_failIn[name] = call; }
 void fake_drop_rows(int count) { g_dropRows = count; }             // so many of the next loss launches store nothing
 int fake_dirty_counters() { return g_dirtyCounters; }              // loss launches that found a counter other than zero
 int fake_null_stream_uses() { return g_nullStreamUses; }
+char const* fake_launches() { return g_launches.c_str(); }        // since the library was loaded
 int fake_allocations() { return int(g_memory.size()); }
 hipStream_t fake_last_loss_stream = nullptr;
 int fake_outstanding() { return reinterpret_cast<Stream*>(fake_last_loss_stream)->outstanding; }
@@ -102,6 +105,7 @@ hipError_t hipStreamDestroy(hipStream_t s) { delete reinterpret_cast<Stream*>(s)
 hipError_t hipStreamSynchronize(hipStream_t s)
 {
     of(s)->outstanding = 0;
+    g_launches += "complete\n";
     return outcome("hipStreamSynchronize", hipErrorLaunchFailure);
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned)
@@ -159,6 +163,7 @@ hipError_t launch_image_loss(uint16_t*, uint16_t const*, int width, int height, 
         }
     return hipSuccess;
 }
+hipError_t launch_color_tables(hipStream_t s) { return launched("launch_color_tables", s); }
 hipError_t launch_transfer_tables(hipStream_t s) { return launched("launch_transfer_tables", s); }
 hipError_t launch_read_channels(ReadChannelsArgs const&, hipStream_t s) { return launched("launch_read_channels", s); }
 hipError_t launch_write_channels(WriteChannelsArgs const&, hipStream_t s) { return launched("launch_write_channels", s); }

@@ -46,6 +46,13 @@ def fake(ntc, library):
     assert lib.fake_allocations() == 0
 
 
+def test_tables_of_a_device_are_complete_before_its_first_context(fake):
+    """Contexts have streams of their own: nothing orders one's first launch behind tables that another's call fills."""
+    fake.fake_launches.restype = C.c_char_p
+    first = fake.fake_launches().decode().split()[:3]
+    assert sorted(first[:2]) == ["launch_color_tables", "launch_transfer_tables"] and first[2] == "complete"
+
+
 def test_contexts_leave_the_null_stream_alone(fake):
     """Work on the null stream waits for every blocking stream of the device, and they for it."""
     handle = C.c_void_p()
