@@ -181,7 +181,8 @@ BC6_INLINE float exp1(float c) { return exp2_of_log(c) - 1.f; }
 //   2. a wave per subset of each block's pattern: its endpoints;
 //   3. each wave four of the sixteen texels: indices and errors of all three candidates;
 //   4. one wave: the errors added up in texel order, the choice, the block.
-// Bound by the issue of vector instructions.  Each part is a function with registers of its own, so that four waves fit
+// Bound by the issue of vector instructions: 72 % of the slots at 2048 x 2048, the rest goes where one wave works and the
+// others wait for it, or for texels from LDS.  Each part is a function with registers of its own, so that four waves fit
 // a SIMD and nothing is spilled in a loop; the search is one call because a call saves registers to scratch (a call per
 // two patterns: 257 us at 2048 x 2048 instead of 204).  One lane per block, all parts in one body with 168 registers,
 // took 121 us at 64 x 64, 151 at 1024 x 1024 and 287 at 2048 x 2048: small images waited for the chain of one lane's

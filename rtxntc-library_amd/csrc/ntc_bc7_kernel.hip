@@ -1,7 +1,8 @@
 // ntc_bc7_kernel.hip - BC7 block compression of a decoded image (gfx950).
 //
 // The reference's BC7 pass (IContext::MakeBlockCompressionComputePass with BlockCompressedFormat::BC7,
-// src/shaders/CompressBC7.hlsl) as a compute kernel: one lane encodes one 4 x 4 block.
+// src/shaders/CompressBC7.hlsl) as compute kernels: the full search, which the waves of a workgroup share, and one that
+// encodes given modes, a block per lane.
 //
 // Full search, per block: opaque blocks try the three-subset modes 0 and 2 and the two-subset modes
 // 1 and 3, each on the partition whose bounding-box endpoints give the smallest estimated error over
@@ -535,8 +536,9 @@ BC7_INLINE void store_block(BlockCompressArgs const& a, int bx, int by, uint64_t
 // The search is bound by vector instruction issue where it fills the GPU and by the length of one lane's chain where it
 // does not.  One lane per block with the texels in 255 registers and a scalar branch around every texel of every pass
 // took 0.9 ms for any image of up to 1024 x 1024 and 2.0 ms for 2048 x 2048; this takes 0.10 ms for 64 x 64, 0.11 for
-// 512 x 512, 0.29 for 1024 x 1024 and 0.95 for 2048 x 2048 (half of it opaque), where every issue slot of the vector units
-// is taken.
+// 512 x 512, 0.28 for 1024 x 1024 and 0.95 for 2048 x 2048 (half of it opaque).  Vector issue slots taken: 76 % at
+// 1024 x 1024, which is one residency of workgroups and as long as the longest of them, 79 % at 2048 x 2048; the waves'
+// tasks differ in length and their ends wait at the barriers.
 enum { kSlots = 10, kPickThree = 0, kPickTwo, kPickTwoAlpha, kPicks };
 enum : uint32_t { kBelowOne = 1, kNotOne = 2 };              // what some alpha of a block is (one above 1 or a NaN is only the second)
 

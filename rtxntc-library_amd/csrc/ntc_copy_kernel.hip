@@ -2,9 +2,11 @@
 //
 // The 1:1 branch of the reference's CopyImageKernel as ITextureSet::ReadChannels / WriteChannels
 // use it (src/ImageProcessing.cu:86-164,220-265, src/TextureSet.cpp:835-985): no resize; colour
-// space decode/encode and dithering as the reference defines them.  One lane per pixel; source reads are the half2 pairs of
-// the planar-pair layout (coalesced across x), destination writes are the pixel's bytes.
-// HBM-bound: 2 bytes read and 1-4 bytes written per channel.
+// space decode/encode and dithering as the reference defines them.  Pixels of at most eight bytes go four to a lane
+// (read_groups_kernel, write_groups_kernel), larger ones one to a lane; the planar layout is read and written as half2
+// pairs, coalesced across x.  2 bytes read and 1-4 bytes written per channel: bound by memory where colours are linear,
+// by the draws and the rounding where 8-bit codes are dithered.  Then the copies between images of different sizes, the
+// image loss and the image difference.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <atomic>
