@@ -175,7 +175,8 @@ typedef struct NtcHipTextureSet {
 
 /* A context: one device, one stream (opaque). */
 typedef struct NtcHipContext NtcHipContext;
-/* Creates a context on HIP device `device` (which must be a gfx950 device) with a stream of its own.
+/* Creates a context on HIP device `device` (which must be a gfx950 device) with a stream of its own.  A device's first
+ * context also fills the tables that the library keeps there, and waits for them but for no other work.
  * Replaces the reference's cudaSetDevice + cudaInitDevice in CreateContext (src/PublicFunctions.cpp:84-112). */
 int ntc_hip_create(int device, NtcHipContext** outContext);
 /* Waits for the context's work, then releases its stream and working memory.  Memory from
@@ -335,7 +336,8 @@ int ntc_hip_resize_planar(const void* srcPlanarPairs, uint64_t srcBytes, int32_t
  * channel is clamped to [0, 1] in place before it is compared (Inference.cu:96-97), and with the
  * discard flag texels whose reference mask value is zero count on the mask channel only
  * (Inference.cu:80-84,107-108).  A negative index means no mask channel; the decoded image is then only
- * read.  outMse receives 16 floats.  Synchronous. */
+ * read.  outMse receives 16 floats.  Synchronous: everything that was queued on the context's stream,
+ * the pass included, is complete on return, and an error of it is the call's. */
 int ntc_hip_image_loss(void* decodedPlanarPairs, const void* referencePlanarPairs, uint64_t planarBytes,
                        int32_t width, int32_t height, int32_t setChannels, uint32_t validChannelMask,
                        int32_t maskChannelIndex, int32_t discardMaskedOutPixels, float* outMse);
