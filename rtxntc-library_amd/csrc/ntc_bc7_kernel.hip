@@ -525,33 +525,55 @@ BC7_INLINE void store_block(BlockCompressArgs const& a, int bx, int by, uint64_t
 //
 // A workgroup of WAVES waves encodes GROUPS x 64 blocks; the lanes of a wave are blocks, and the waves divide the search
 // among themselves.  The texels lie in LDS.
-//   1. Every task is some partitions of a search (three subsets and two subsets of opaque blocks, two subsets of blocks
-//      with alpha), whose smallest error per block is found by an atomic minimum in LDS.  All lanes take the same
-//      partition: for each subset its texels are read into registers and go through code for exactly that many.
-//   2. Every task is one candidate, or the three forms of modes 4 and 5 of one channel rotation, from its endpoints to
-//      the encoded block.  Every lane has a partition of its own here and walks its own list of texels.
+//   1. A search is for the partition with the smallest estimated error of 64 blocks: of two and of three subsets for
+//      opaque blocks, of two subsets for mode 7.  Tasks of a range of its partitions bound the errors from below, all
+//      lanes with the same partition; when a search's are done, one more task estimates the error of the partition with
+//      the smallest bound and queues those whose bounds do not exceed it: one to seven of 64 on textures with detail.
+//   2. Tasks of 64 queued estimates, from any blocks of a search; tasks of one candidate, or of the three forms of modes 4
+//      and 5 of one channel rotation, from its endpoints to the encoded block, where every lane has a partition of its
+//      own and walks its own list of texels.
 //   3. A thread per block goes through the candidates in the order given at the top with "not larger replaces".
-// Blocks with and without alpha are gathered in groups of their own for the tasks that only one kind has.
+// Blocks with and without alpha are gathered in groups of their own for the tasks that only one kind has.  Waves take the
+// tasks of a phase in turn; one that builds upon others waits for their count.
 //
 // The search is bound by vector instruction issue where it fills the GPU and by the length of one lane's chain where it
-// does not.  One lane per block with the texels in 255 registers and a scalar branch around every texel of every pass
-// took 0.9 ms for any image of up to 1024 x 1024 and 2.0 ms for 2048 x 2048; this takes 0.10 ms for 64 x 64, 0.11 for
-// 512 x 512, 0.28 for 1024 x 1024 and 0.95 for 2048 x 2048 (half of it opaque).  Vector issue slots taken: 76 % at
-// 1024 x 1024, which is one residency of workgroups and as long as the longest of them, 79 % at 2048 x 2048; the waves'
-// tasks differ in length and their ends wait at the barriers.
+// does not.  One lane per block with the texels in 255 registers took 0.9 ms for any image of up to 1024 x 1024; with the
+// search divided and every partition estimated, 64 x 64 took 98 us, 512 x 512 102, 1024 x 1024 274 and 2048 x 2048 927 (half
+// of it opaque; 183 M vector instructions at 1024 x 1024, seven of ten of them estimates); with bounds first 79, 88, 191
+// and 721 (140 M).  Bounds cost a third of an estimate and leave few to make where texels have noise or detail in three
+// channels; where channels are proportional, every partition's bound is nothing, and searches whose blocks are mostly like
+// that are estimated as a whole without bounds (kNearLine: 1024 x 1024 grey 277 -> 254 us, 700 with queues for them).
+// Hard edges in every block leave a fifth and more of the partitions, more than a queue takes: there the bounds are
+// in vain (284 -> 311 us).
+//
+// Wave priorities fall from phase to phase.  With equal ones the older of the two workgroups of a compute unit runs ahead
+// through the first phase and leaves the younger one alone with half the waves at the end (347 and 485 thousand cycles at
+// 1024 x 1024); a workgroup that is behind now comes first (365 and 422 thousand; 209 -> 188 us).
 enum { kSlots = 10, kPickThree = 0, kPickTwo, kPickTwoAlpha, kPicks };
 enum : uint32_t { kBelowOne = 1, kNotOne = 2 };              // what some alpha of a block is (one above 1 or a NaN is only the second)
 
+// The searches of a workgroup: its opaque groups' partitions of two subsets, then of three, then the partitions for mode 7
+// of all groups, the opaque ones first.  (128 blocks are two groups of one kind, or three of both.)
+enum { kSearches = 7, kQueued = 14 * 64, kWholeChunk = 8 };
 template <int BLOCKS_>
 struct SearchLds {
     static constexpr int BLOCKS = BLOCKS_;
     float4 texels[16][BLOCKS];
     uint64_t picks[kPicks][BLOCKS];                          // error bits << 32 | partition
-    uint4 words[kSlots][BLOCKS];
-    float errors[kSlots][BLOCKS];
+    float scale[kPicks][BLOCKS];                             // of errors before they become codes; 0: the block has no bounds
+    uint32_t lowest[kPicks][BLOCKS];                         // the smallest bound's bits, the low six replaced by its partition
+    union {
+        uint32_t bounds[kPicks][16][BLOCKS];                 // codes of four partitions each; until the picks are made
+        struct { uint4 words[kSlots - 1][BLOCKS]; float errors[kSlots - 1][BLOCKS]; } late;
+    };
+    struct { uint4 words[BLOCKS]; float errors[BLOCKS]; } early;                   // mode 6
+    uint16_t queues[kSearches][kQueued];                     // partition << 7 | block
+    int queued[kSearches];
+    uint8_t whole[kSearches];                                // searches that estimate every partition
     uint32_t alphas[BLOCKS];                                 // kBelowOne | kNotOne
     uint8_t blocks[2][BLOCKS];                               // numbers of the opaque blocks, of those with alpha
-    int counts[2];
+    int counts[2], next[2], wholes;
+    int bounded[kSearches], estimated;                       // tasks done: those of a search's bounds, those of estimates
 };
 template <class S> using SearchPtr = __attribute__((address_space(3))) S*;
 
@@ -566,7 +588,7 @@ template <int C, class S> BC7_INLINE Color<C> texel(SearchPtr<S> lds, int b, int
     if constexpr (C == 4) p.c[3] = lds->texels[t][b].w;
     return p;
 }
-BC7_INLINE int first_texel(uint32_t mask) { return (__ffs(int(mask)) - 1) >> 1; }
+BC7_INLINE int first_texel(uint32_t mask) { return __builtin_ctz(mask) >> 1; }           // (of a mask that has one)
 
 // Endpoints' swaps of orient() from the finished covariances.
 template <int C> BC7_INLINE void orient_by(float const (&cov)[C][C], Color<C>& e0, Color<C>& e1)
@@ -590,6 +612,425 @@ template <int C> BC7_INLINE void add_covariance(float (&cov)[C][C], Color<C> con
         for (int b = a + 1; b < C; ++b) cov[a][b] += d.c[a] * d.c[b];
 }
 template <int C> BC7_INLINE float inverse_square(Color<C> const& axis) { float const l = dot(axis, axis); return l > 0.f ? 1.f / l : l; }
+
+// ---- bounds of the partitions' errors
+//
+// The estimated error of a subset is the texels' squared distance from points of its box's diagonal, at least that from
+// the diagonal itself, D.  With h the middle of the box, a its diagonal, M the second moments about h,
+//     D = trace M - (a M a) / |a|^2,
+// which takes sums over the texels instead of a pass over them for each of centre, covariance, and error, and of the
+// largest subset not even those: its sums are what the others leave of the block's.  All sums are of offsets from texel 0.
+// How far D as computed can be from its true value, and the estimate as computed below its true value: the terms' sizes
+// add up to less than 42 T, T the sum of the block's squared offsets (|h|^2 and the squared mean are at most the subset's
+// share of T, and a subset has at most 13 texels), and none passes through more than 34 roundings: together less than
+// 1100 units of roundoff of T.  kBoundError, of 2048 units, is taken off each bound.
+constexpr float kBoundError = 0x1p-13f;
+// Which components' ends trade places depends on the covariances' signs as orient_by() finds them.  Where one could be
+// 0 within the errors of either evaluation (texel by texel about a rounded mean, which is off by 16 units of roundoff of
+// the texels' size; by sums here, off by 100 units of T), the nearest of the four diagonals counts.
+constexpr float kUnsureOfOffsets = 0x1p-16f, kUnsureOfTexels = 0x1p-35f;
+// Bounds are kept as codes of eight bits: errors over T, four bits of the exponent (2^-16 ... 1) and four of the mantissa,
+// rounded down.  Blocks whose T is no number between these have no bounds, and all of their partitions are estimated.
+constexpr float kNearLine = 1.f / 64.f;                      // squared distances over the squared diagonal; eight points leave 16 / 588 of it
+constexpr float kLeastOffsets = 0x1p-60f, kMostOffsets = 0x1p60f;
+BC7_INLINE uint32_t error_code(float error, float scale)
+{
+    constexpr uint32_t first = (127u - 16u) << 4;
+    uint32_t const bits = __float_as_uint(error * scale) >> 19;                  // (a NaN: the last code)
+    return min(max(bits, first) - first, 255u);
+}
+
+template <int C> struct Sums {
+    float s[C], q[C][C];                                     // of q the upper triangle
+    BC7_INLINE Sums()
+    {
+#pragma unroll
+        for (int i = 0; i < C; ++i) {
+            s[i] = 0.f;
+#pragma unroll
+            for (int j = i; j < C; ++j) q[i][j] = 0.f;
+        }
+    }
+    BC7_INLINE void add(Color<C> const& x)
+    {
+#pragma unroll
+        for (int i = 0; i < C; ++i) {
+            s[i] += x.c[i];
+#pragma unroll
+            for (int j = i; j < C; ++j) q[i][j] = __builtin_fmaf(x.c[i], x.c[j], q[i][j]);
+        }
+    }
+    BC7_INLINE void remove(Sums const& o)
+    {
+#pragma unroll
+        for (int i = 0; i < C; ++i) {
+            s[i] -= o.s[i];
+#pragma unroll
+            for (int j = i; j < C; ++j) q[i][j] -= o.q[i][j];
+        }
+    }
+    BC7_INLINE float trace() const
+    {
+        float t = q[0][0];
+#pragma unroll
+        for (int i = 1; i < C; ++i) t += q[i][i];
+        return t;
+    }
+};
+
+// The box of a subset (uniform, of N texels), and its sums if SUMS.
+template <int C, int N, bool SUMS, class S>
+BC7_INLINE void subset_box(SearchPtr<S> lds, int b, uint32_t mask, Color<C> const& origin, Color<C>& lo, Color<C>& hi, Sums<C>& sums)
+{
+    Color<C> px[N];
+#pragma unroll
+    for (int t = 0; t < N; ++t) {
+        px[t] = texel<C, S>(lds, b, first_texel(mask));
+        if constexpr (SUMS) px[t] = sub(px[t], origin);
+        mask &= mask - 1;
+    }
+    lo = hi = px[0];
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+#pragma unroll
+        for (int t = 1; t + 1 < N; t += 2) { lo.c[k] = min3_f32(lo.c[k], px[t].c[k], px[t + 1].c[k]); hi.c[k] = max3_f32(hi.c[k], px[t].c[k], px[t + 1].c[k]); }
+        if constexpr (!(N & 1)) { lo.c[k] = min_f32(lo.c[k], px[N - 1].c[k]); hi.c[k] = max_f32(hi.c[k], px[N - 1].c[k]); }
+    }
+    if constexpr (SUMS) {
+#pragma unroll
+        for (int t = 0; t < N; ++t) sums.add(px[t]);
+    } else {
+        lo = sub(lo, origin); hi = sub(hi, origin);          // (rounding is monotone: the box of the offsets)
+    }
+}
+
+// The squared distances of a subset's n texels from the diagonal `a` of its box, whose middle is `middle2` / 2.  w: twice
+// the texels' sum less n times the middle.
+template <int C>
+BC7_INLINE float distances(Sums<C> const& sums, Color<C> const& middle2, Color<C> const& w, Color<C> const& a, float inverse)
+{
+    float along = 0.f;                                       // sum of (a . offset from the middle)^2
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+        float row = a.c[i] * sums.q[i][i];
+#pragma unroll
+        for (int j = i + 1; j < C; ++j) row = __builtin_fmaf(a.c[j] + a.c[j], sums.q[i][j], row);
+        along = i == 0 ? a.c[i] * row : __builtin_fmaf(a.c[i], row, along);
+    }
+    float am = a.c[0] * middle2.c[0], aw = a.c[0] * w.c[0], mw = middle2.c[0] * w.c[0];
+#pragma unroll
+    for (int k = 1; k < C; ++k) { am = __builtin_fmaf(a.c[k], middle2.c[k], am); aw = __builtin_fmaf(a.c[k], w.c[k], aw); mw = __builtin_fmaf(middle2.c[k], w.c[k], mw); }
+    along = __builtin_fmaf(-0.5f * am, aw, along);
+    return __builtin_fmaf(-along, inverse, __builtin_fmaf(-0.5f, mw, sums.trace()));
+}
+
+// Adds a subset's squared distances from its box's diagonal: from the one that orient_by() chooses if ORIENTED, from lo to hi
+// if PLAIN.  n: its number of texels.
+template <int C, bool ORIENTED, bool PLAIN>
+BC7_INLINE void add_distances(float n, Sums<C> const& sums, Color<C> const& lo, Color<C> const& hi, float unsure, float& oriented, float& plain)
+{
+    Color<C> const a = sub(hi, lo);
+    Color<C> middle2, w;
+    float length = 0x1p-100f;
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+        middle2.c[k] = lo.c[k] + hi.c[k];
+        w.c[k] = __builtin_fmaf(-0.5f * n, middle2.c[k], sums.s[k] + sums.s[k]);
+        length = __builtin_fmaf(a.c[k], a.c[k], length);
+    }
+    float const inverse = __builtin_amdgcn_rcpf(length);
+    if constexpr (PLAIN) plain += distances(sums, middle2, w, a, inverse);
+    if constexpr (ORIENTED) {
+        static_assert(C == 3, "");
+        float const mean = sums.s[0] * __builtin_amdgcn_rcpf(n);
+        float const c1 = __builtin_fmaf(-mean, sums.s[1], sums.q[0][1]), c2 = __builtin_fmaf(-mean, sums.s[2], sums.q[0][2]);
+        float least = distances(sums, middle2, w, Color<C>{ a.c[0], copysignf(a.c[1], c1), copysignf(a.c[2], c2) }, inverse);
+        bool const sure = min_f32(fabsf(c1), fabsf(c2)) > unsure;                // (a[0] = 0 is not)
+        if (__any(!sure)) {
+            float all = distances(sums, middle2, w, a, inverse);
+            all = fminf(all, distances(sums, middle2, w, Color<C>{ a.c[0], -a.c[1], a.c[2] }, inverse));
+            all = fminf(all, distances(sums, middle2, w, Color<C>{ a.c[0], a.c[1], -a.c[2] }, inverse));
+            all = fminf(all, distances(sums, middle2, w, Color<C>{ a.c[0], -a.c[1], -a.c[2] }, inverse));
+            if (!sure) least = all;
+        }
+        oriented += least;
+    }
+}
+
+// Bounds of the partitions [first, last), multiples of four, of one or both picks.
+template <class S, int SUBSETS, int C, bool ORIENTED, bool PLAIN>
+BC7_TASK void bound_task(SearchPtr<S> lds, int b, int first, int last)
+{
+    first = __builtin_amdgcn_readfirstlane(first);
+    last = __builtin_amdgcn_readfirstlane(last);
+    constexpr int kind = SUBSETS == 3 ? kPickThree : kPickTwo;
+    Color<C> const origin = texel<C, S>(lds, b, 0);
+    Sums<C> total;
+#pragma unroll 5
+    for (int t = 1; t < 16; ++t) total.add(sub(texel<C, S>(lds, b, t), origin));
+    float const offsets = total.trace();
+    bool const bounded = offsets >= kLeastOffsets && offsets <= kMostOffsets;
+    float const scale = bounded ? __builtin_amdgcn_rcpf(offsets) : 0.f, error = offsets * kBoundError;
+    float const unsure = __builtin_fmaf(offsets, kUnsureOfOffsets, dot(origin, origin) * kUnsureOfTexels);
+    if constexpr (ORIENTED) lds->scale[kind][b] = scale;
+    if constexpr (PLAIN) lds->scale[kPickTwoAlpha][b] = scale;
+    // Blocks near a line: what the partitions leave of their distances is less than the steps along the diagonals, and the
+    // bounds tell nothing.  Where three of four blocks are such, every partition is estimated (lowest stays as it is).
+    {
+        Color<C> lo, hi;
+        subset_box<C, 16, false, S>(lds, b, kAllTexels, origin, lo, hi, total);
+        float oriented = 0.f, plain = 0.f;
+        add_distances<C, ORIENTED, !ORIENTED>(16.f, total, lo, hi, unsure, oriented, plain);
+        Color<C> const a = sub(hi, lo);
+        if (__popcll(__ballot(bounded && (ORIENTED ? oriented : plain) < dot(a, a) * kNearLine)) >= 48) return;
+    }
+    uint32_t lowestOriented = ~0u, lowestPlain = ~0u, codesOriented = 0, codesPlain = 0;
+#pragma unroll 1
+    for (int p = first; p < last; ++p) {
+        uint32_t const word = partition_word<SUBSETS>(p);
+        uint32_t masks[SUBSETS];                             // the largest subset last
+#pragma unroll
+        for (int s = 0; s < SUBSETS; ++s) masks[s] = spread_mask(word, uint32_t(s));
+#pragma unroll
+        for (int s = 0; s + 1 < SUBSETS; ++s)
+            if (__popc(masks[s]) > __popc(masks[SUBSETS - 1])) { uint32_t const m = masks[s]; masks[s] = masks[SUBSETS - 1]; masks[SUBSETS - 1] = m; }
+        Sums<C> rest = total;
+        float oriented = 0.f, plain = 0.f;
+        uint32_t mask = masks[0];
+#pragma unroll 1
+        for (int s = 0; s + 1 < SUBSETS; ++s) {
+            Sums<C> sums;
+            Color<C> lo, hi;
+            mask = __builtin_amdgcn_readfirstlane(mask);
+            switch (__popc(mask)) {                          // the sizes that the partitions' smaller subsets have
+            case 2:  if constexpr (SUBSETS == 3) subset_box<C, 2, true, S>(lds, b, mask, origin, lo, hi, sums); break;
+            case 3:  subset_box<C, 3, true, S>(lds, b, mask, origin, lo, hi, sums); break;
+            case 4:  subset_box<C, 4, true, S>(lds, b, mask, origin, lo, hi, sums); break;
+            case 5:  subset_box<C, 5, true, S>(lds, b, mask, origin, lo, hi, sums); break;
+            case 6:  subset_box<C, 6, true, S>(lds, b, mask, origin, lo, hi, sums); break;
+            default: if constexpr (SUBSETS == 2) subset_box<C, 8, true, S>(lds, b, mask, origin, lo, hi, sums); break;
+            }
+            add_distances<C, ORIENTED, PLAIN>(float(__popc(mask)), sums, lo, hi, unsure, oriented, plain);
+            rest.remove(sums);
+            mask = masks[SUBSETS - 2];
+        }
+        Sums<C> none;
+        Color<C> lo, hi;
+        mask = __builtin_amdgcn_readfirstlane(masks[SUBSETS - 1]);
+        switch (__popc(mask)) {                              // and their largest
+        case 6:  if constexpr (SUBSETS == 3) subset_box<C, 6, false, S>(lds, b, mask, origin, lo, hi, none); break;
+        case 7:  if constexpr (SUBSETS == 3) subset_box<C, 7, false, S>(lds, b, mask, origin, lo, hi, none); break;
+        case 8:  subset_box<C, 8, false, S>(lds, b, mask, origin, lo, hi, none); break;
+        case 10: if constexpr (SUBSETS == 2) subset_box<C, 10, false, S>(lds, b, mask, origin, lo, hi, none); break;
+        case 11: if constexpr (SUBSETS == 2) subset_box<C, 11, false, S>(lds, b, mask, origin, lo, hi, none); break;
+        case 12: subset_box<C, 12, false, S>(lds, b, mask, origin, lo, hi, none); break;
+        default: if constexpr (SUBSETS == 2) subset_box<C, 13, false, S>(lds, b, mask, origin, lo, hi, none); break;
+        }
+        add_distances<C, ORIENTED, PLAIN>(float(__popc(mask)), rest, lo, hi, unsure, oriented, plain);
+        auto const consider = [&](float distances, uint32_t& lowest, uint32_t& codes) {
+            float const bound = bounded ? fmaxf(distances - error, 0.f) : 0.f;
+            lowest = min(lowest, (__float_as_uint(bound) & ~63u) | uint32_t(p));
+            codes = codes >> 8 | error_code(bound, scale) << 24;
+        };
+        if constexpr (ORIENTED) consider(oriented, lowestOriented, codesOriented);
+        if constexpr (PLAIN) consider(plain, lowestPlain, codesPlain);
+        if ((p & 3) == 3) {
+            if constexpr (ORIENTED) lds->bounds[kind][p >> 2][b] = codesOriented;
+            if constexpr (PLAIN) lds->bounds[kPickTwoAlpha][p >> 2][b] = codesPlain;
+        }
+    }
+    if constexpr (ORIENTED) __hip_atomic_fetch_min(&lds->lowest[kind][b], lowestOriented, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if constexpr (PLAIN) __hip_atomic_fetch_min(&lds->lowest[kPickTwoAlpha][b], lowestPlain, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Sums of one refinement round (refine() above) and its solution; false when the system is singular.
+template <int C> struct Refinement {
+    float a2 = 0.f, b2 = 0.f, ab = 0.f;
+    Color<C> ax, bx;
+    BC7_INLINE Refinement()
+    {
+#pragma unroll
+        for (int k = 0; k < C; ++k) ax.c[k] = bx.c[k] = 0.f;
+    }
+    // f: the texel's saturated place between the ends
+    BC7_INLINE void add(float f, Color<C> const& p, int indexBits)
+    {
+        float const scale = float((1u << indexBits) - 1u), iscale = 1.f / scale;
+        float const beta = rintf(f * scale) * iscale, alpha = 1.f - beta;
+        a2 += alpha * alpha; b2 += beta * beta; ab += alpha * beta;
+#pragma unroll
+        for (int k = 0; k < C; ++k) { ax.c[k] += alpha * p.c[k]; bx.c[k] += beta * p.c[k]; }
+    }
+    BC7_INLINE bool solve(Color<C>& e0, Color<C>& e1) const
+    {
+        float const denom = a2 * b2 - ab * ab;
+        if (!(fabsf(denom) > 0.0001f)) return false;
+        float const factor = 1.f / denom;
+#pragma unroll
+        for (int k = 0; k < C; ++k) {
+            float const a = saturate((ax.c[k] * b2 - bx.c[k] * ab) * factor), b = saturate((bx.c[k] * a2 - ax.c[k] * ab) * factor);
+            if (!(e0.c[k] == 0.f || e0.c[k] == 1.f)) e0.c[k] = a;
+            if (!(e1.c[k] == 0.f || e1.c[k] == 1.f)) e1.c[k] = b;
+        }
+        return true;
+    }
+};
+
+// Start ends of the lane's own subset: its box, oriented if asked.
+template <int C, bool ORIENT, class S> BC7_INLINE void listed_ends(SearchPtr<S> lds, int b, uint32_t mask, Color<C>& e0, Color<C>& e1)
+{
+    Color<C> center;
+#pragma unroll
+    for (int k = 0; k < C; ++k) { e0.c[k] = FLT_MAX; e1.c[k] = -FLT_MAX; center.c[k] = 0.f; }
+    for (uint32_t m = mask; m; m &= m - 1) {
+        Color<C> const p = texel<C, S>(lds, b, first_texel(m));
+#pragma unroll
+        for (int k = 0; k < C; ++k) { e0.c[k] = min_f32(e0.c[k], p.c[k]); e1.c[k] = max_f32(e1.c[k], p.c[k]); center.c[k] += p.c[k]; }
+    }
+    if constexpr (ORIENT) {
+        float const count = float(__popc(mask));
+#pragma unroll
+        for (int k = 0; k < C; ++k) center.c[k] /= count;
+        float cov[C][C] = {};
+        for (uint32_t m = mask; m; m &= m - 1) add_covariance(cov, sub(texel<C, S>(lds, b, first_texel(m)), center));
+        orient_by(cov, e0, e1);
+    }
+}
+// The estimated error of the lane's own partition, into the pick of its kind: the smallest of these numbers is the smallest
+// error (errors are not negative) and the first partition that has it.
+template <class S> BC7_INLINE void put_estimate(SearchPtr<S> lds, int kind, int b, int partition, float error)
+{
+    uint64_t const key = uint64_t(__float_as_uint(error)) << 32 | uint32_t(partition);
+    __hip_atomic_fetch_min(&lds->picks[kind][b], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// For the modes 0 to 3: squared error if every texel took the nearest of eight points between its subset's oriented ends.
+template <class S, int SUBSETS>
+BC7_TASK void estimate_task(SearchPtr<S> lds, int b, int partition)
+{
+    constexpr float maxIndex = 7.f, indexScale = 1.f / maxIndex;
+    uint32_t const word = partition_word<SUBSETS>(partition);
+    float error = 0.f;
+#pragma unroll 1
+    for (int s = 0; s < SUBSETS; ++s) {
+        uint32_t const mask = spread_mask(word, uint32_t(s));
+        Color<3> e0, e1;
+        listed_ends<3, true, S>(lds, b, mask, e0, e1);
+        Color<3> const axis = sub(e1, e0);
+        float const mul = inverse_square(axis);
+        float e = 0.f;
+        for (uint32_t m = mask; m; m &= m - 1) {
+            Color<3> const p = sub(texel<3, S>(lds, b, first_texel(m)), e0);
+            float const f = rintf(dot(p, axis) * mul * maxIndex) * indexScale;
+            Color<3> diff;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) diff.c[k] = f * axis.c[k] - p.c[k];
+            e += dot(diff, diff);
+        }
+        error = s == 0 ? e : error + e;
+    }
+    put_estimate<S>(lds, SUBSETS == 3 ? kPickThree : kPickTwo, b, partition, error);
+}
+
+// For mode 7: of four points between the corners of its subset's box.  The bounds leave the most partitions of this kind,
+// so that lists of texels, whose addresses are a chain, would be the longest part of the search: here all texels are
+// loaded at once and go through the code of both subsets, as NaNs (which minima and maxima leave out) or zeros where they
+// belong to the other.
+template <class S, int C>
+BC7_TASK void estimate_corners_task(SearchPtr<S> lds, int b, int partition)
+{
+    constexpr float maxIndex = 3.f, indexScale = 1.f / maxIndex;
+    uint32_t const word = partition_word<2>(partition);
+    Color<C> px[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) px[t] = texel<C, S>(lds, b, t);
+    auto const second = [&](int t) { return uint32_t(int32_t(word << (31 - 2 * t)) >> 31); };        // all ones if the texel is in subset 1
+    auto const ored = [](float v, uint32_t m) { return __uint_as_float(__float_as_uint(v) | m); };
+    Color<C> lo[2], axis[2];
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+        float l0 = FLT_MAX, h0 = -FLT_MAX, l1 = FLT_MAX, h1 = -FLT_MAX;
+#pragma unroll
+        for (int t = 0; t < 16; t += 2) {
+            float const a0 = ored(px[t].c[k], second(t)), b0 = ored(px[t + 1].c[k], second(t + 1));
+            float const a1 = ored(px[t].c[k], ~second(t)), b1 = ored(px[t + 1].c[k], ~second(t + 1));
+            l0 = min3_f32(l0, a0, b0); h0 = max3_f32(h0, a0, b0);
+            l1 = min3_f32(l1, a1, b1); h1 = max3_f32(h1, a1, b1);
+        }
+        lo[0].c[k] = l0; axis[0].c[k] = h0 - l0;
+        lo[1].c[k] = l1; axis[1].c[k] = h1 - l1;
+    }
+    float const mul0 = inverse_square(axis[0]), mul1 = inverse_square(axis[1]);
+    float error0 = 0.f, error1 = 0.f;
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+        uint32_t const m = second(t);
+        Color<C> p, ax, diff;
+#pragma unroll
+        for (int k = 0; k < C; ++k) { p.c[k] = px[t].c[k] - (m ? lo[1].c[k] : lo[0].c[k]); ax.c[k] = m ? axis[1].c[k] : axis[0].c[k]; }
+        float const f = rintf(dot(p, ax) * (m ? mul1 : mul0) * maxIndex) * indexScale;
+#pragma unroll
+        for (int k = 0; k < C; ++k) diff.c[k] = f * ax.c[k] - p.c[k];
+        float const d = dot(diff, diff);
+        error0 += m ? 0.f : d;
+        error1 += m ? d : 0.f;
+    }
+    put_estimate<S>(lds, kPickTwoAlpha, b, partition, error0 + error1);
+}
+
+enum { kThree = 0, kTwo, kCorners3, kCorners4 };            // what a search estimates: pick kinds, the last by channels
+template <class S> BC7_INLINE void estimate_one(SearchPtr<S> lds, int what, int b, int partition)      // what: uniform
+{
+    if (what == kThree)         estimate_task<S, 3>(lds, b, partition);
+    else if (what == kTwo)      estimate_task<S, 2>(lds, b, partition);
+    else if (what == kCorners3) estimate_corners_task<S, 3>(lds, b, partition);
+    else                        estimate_corners_task<S, 4>(lds, b, partition);
+}
+
+// With all bounds of a search there: the error of the partition with the smallest one, and the partitions whose bounds do
+// not exceed it into the search's queue.  `mine`: the lane is its block's only one.  Where that leaves more of them than
+// one in five all are estimated, with code for their subsets' sizes, which is then the quicker way.
+template <class S>
+BC7_TASK void select_task(SearchPtr<S> lds, int b, int what, int search, int mine)
+{
+    what = __builtin_amdgcn_readfirstlane(what);
+    search = __builtin_amdgcn_readfirstlane(search);
+    int const kind = what == kCorners4 ? int(kPickTwoAlpha) : what;
+    uint32_t const lowest = lds->lowest[kind][b];
+    uint64_t mask = 0;
+    if (__any(lowest != ~0u)) {                              // (else there are no bounds)
+        estimate_one<S>(lds, what, b, int(lowest & 63u));
+        uint64_t const pick = lds->picks[kind][b];
+        uint32_t const bits = uint32_t(pick >> 32), code = error_code(__uint_as_float(bits), lds->scale[kind][b]);
+#pragma unroll 4
+        for (int j = 0; j < 16; ++j) {
+            uint32_t const codes = lds->bounds[kind][j][b];
+            uint32_t four = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) four |= ((codes >> (8 * i)) & 0xffu) <= code ? 1u << i : 0u;
+            mask |= uint64_t(four) << (4 * j);
+        }
+        // not the picked one again; where it leaves no error only those before it can take its place
+        uint64_t const picked = uint64_t(1) << (uint32_t(pick) & 63u);
+        mask &= bits == 0u ? picked - 1u : ~picked;
+        if (!mine) mask = 0;
+        int const n = __popcll(mask);
+        int place = n ? atomicAdd((int*)&lds->queued[search], n) : 0;
+        if (!__any(place + n > kQueued)) {
+            for (; mask; mask &= mask - 1u, ++place) lds->queues[search][place] = uint16_t(__builtin_ctzll(mask) << 7 | b);
+            return;
+        }
+    }
+    if ((threadIdx.x & 63) == 0) {
+        lds->queued[search] = 0;
+        lds->whole[atomicAdd((int*)&lds->wholes, 1)] = uint8_t(search);
+    }
+}
+
+// ---- estimates of whole ranges of partitions
+//
+// All lanes take the same partition: for each subset its texels are read into registers and go through code for exactly
+// that many.
 
 // Squared error of N texels if each took the nearest of the 2^BITS points between e0 and e1.
 template <int BITS, int C, int N> BC7_INLINE float estimate_of(Color<C> const (&px)[N], Color<C> const& e0, Color<C> const& e1)
@@ -690,59 +1131,6 @@ BC7_TASK void pick_task(SearchPtr<S> lds, int b, int first, int last)
     if constexpr (PLAIN) __hip_atomic_fetch_min(&lds->picks[kPickTwoAlpha][b], bestPlain, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// Sums of one refinement round (refine() above) and its solution; false when the system is singular.
-template <int C> struct Refinement {
-    float a2 = 0.f, b2 = 0.f, ab = 0.f;
-    Color<C> ax, bx;
-    BC7_INLINE Refinement()
-    {
-#pragma unroll
-        for (int k = 0; k < C; ++k) ax.c[k] = bx.c[k] = 0.f;
-    }
-    // f: the texel's saturated place between the ends
-    BC7_INLINE void add(float f, Color<C> const& p, int indexBits)
-    {
-        float const scale = float((1u << indexBits) - 1u), iscale = 1.f / scale;
-        float const beta = rintf(f * scale) * iscale, alpha = 1.f - beta;
-        a2 += alpha * alpha; b2 += beta * beta; ab += alpha * beta;
-#pragma unroll
-        for (int k = 0; k < C; ++k) { ax.c[k] += alpha * p.c[k]; bx.c[k] += beta * p.c[k]; }
-    }
-    BC7_INLINE bool solve(Color<C>& e0, Color<C>& e1) const
-    {
-        float const denom = a2 * b2 - ab * ab;
-        if (!(fabsf(denom) > 0.0001f)) return false;
-        float const factor = 1.f / denom;
-#pragma unroll
-        for (int k = 0; k < C; ++k) {
-            float const a = saturate((ax.c[k] * b2 - bx.c[k] * ab) * factor), b = saturate((bx.c[k] * a2 - ax.c[k] * ab) * factor);
-            if (!(e0.c[k] == 0.f || e0.c[k] == 1.f)) e0.c[k] = a;
-            if (!(e1.c[k] == 0.f || e1.c[k] == 1.f)) e1.c[k] = b;
-        }
-        return true;
-    }
-};
-
-// Start ends of the lane's own subset: its box, oriented if asked.
-template <int C, bool ORIENT, class S> BC7_INLINE void listed_ends(SearchPtr<S> lds, int b, uint32_t mask, Color<C>& e0, Color<C>& e1)
-{
-    Color<C> center;
-#pragma unroll
-    for (int k = 0; k < C; ++k) { e0.c[k] = FLT_MAX; e1.c[k] = -FLT_MAX; center.c[k] = 0.f; }
-    for (uint32_t m = mask; m; m &= m - 1) {
-        Color<C> const p = texel<C, S>(lds, b, first_texel(m));
-#pragma unroll
-        for (int k = 0; k < C; ++k) { e0.c[k] = min_f32(e0.c[k], p.c[k]); e1.c[k] = max_f32(e1.c[k], p.c[k]); center.c[k] += p.c[k]; }
-    }
-    if constexpr (ORIENT) {
-        float const count = float(__popc(mask));
-#pragma unroll
-        for (int k = 0; k < C; ++k) center.c[k] /= count;
-        float cov[C][C] = {};
-        for (uint32_t m = mask; m; m &= m - 1) add_covariance(cov, sub(texel<C, S>(lds, b, first_texel(m)), center));
-        orient_by(cov, e0, e1);
-    }
-}
 template <int C, int INDEX_BITS, class S> BC7_INLINE void listed_refine(SearchPtr<S> lds, int b, uint32_t mask, Color<C>& e0, Color<C>& e1)
 {
 #pragma unroll 1
@@ -802,6 +1190,17 @@ BC7_INLINE uint64_t without_bit(uint64_t v, int at)
     return (v & below) | ((v >> 1) & ~below);
 }
 
+// Slot 8, mode 6, has a place of its own: it is there before the picks are made.
+template <class S> BC7_INLINE void put_candidate(SearchPtr<S> lds, int slot, int b, float error, uint64_t lo, uint64_t hi)
+{
+    auto const put = [&](auto words, auto errors) {
+        *errors = error;
+        words->x = uint32_t(lo); words->y = uint32_t(lo >> 32); words->z = uint32_t(hi); words->w = uint32_t(hi >> 32);
+    };
+    if (slot == 8) put(&lds->early.words[b], &lds->early.errors[b]);             // uniform
+    else           put(&lds->late.words[min(slot, 8)][b], &lds->late.errors[min(slot, 8)][b]);
+}
+
 template <class S, class M, int C, bool ORIENT>
 BC7_TASK void finish_task(SearchPtr<S> lds, int b, int pick, int slot)
 {
@@ -818,7 +1217,7 @@ BC7_TASK void finish_task(SearchPtr<S> lds, int b, int pick, int slot)
         partition = none ? 0 : int(uint32_t(key));
     }
     if (partition >= (1 << M::partitionBits)) {              // mode 0 has sixteen partitions only
-        lds->errors[slot][b] = __uint_as_float(0x7f800000u); // never taken
+        lds->late.errors[slot][b] = __uint_as_float(0x7f800000u);    // never taken
         return;
     }
     uint32_t const word = partition_word<M::subsets>(partition);
@@ -882,9 +1281,7 @@ BC7_TASK void finish_task(SearchPtr<S> lds, int b, int pick, int slot)
     }
     indices = without_bit(indices, top);
     put_indices(bits.lo, bits.hi, bits.at, indices);
-    lds->errors[slot][b] = error;
-    lds->words[slot][b].x = uint32_t(bits.lo); lds->words[slot][b].y = uint32_t(bits.lo >> 32);
-    lds->words[slot][b].z = uint32_t(bits.hi); lds->words[slot][b].w = uint32_t(bits.hi >> 32);
+    put_candidate<S>(lds, slot, b, error, bits.lo, bits.hi);
 }
 
 // The colour plane and the scalar plane of a texel under a channel rotation (uniform).
@@ -1016,8 +1413,9 @@ template <int GROUPS, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES, 4)
 bc7_compress_kernel(BlockCompressArgs a)
 {
-    constexpr int BLOCKS = 64 * GROUPS, THREADS = 64 * WAVES, CHUNK = 64 * GROUPS / WAVES >= 8 ? 8 : 4, CHUNKS = 64 / CHUNK;
-    static_assert(THREADS >= 4 * BLOCKS, "a thread per row of a block at least");
+    // (a task of bounds sums the block first: as many partitions in one as leave a task for each wave)
+    constexpr int BLOCKS = 64 * GROUPS, THREADS = 64 * WAVES, CHUNK = GROUPS == 1 ? 8 : 16, CHUNKS = 64 / CHUNK;
+    static_assert(THREADS >= 4 * BLOCKS && BLOCKS <= 128, "a thread per row of a block at least; seven bits number a block");
     using S = SearchLds<BLOCKS>;
     __shared__ S shared;
     SearchPtr<S> const lds = (SearchPtr<S>)&shared;
@@ -1025,11 +1423,20 @@ bc7_compress_kernel(BlockCompressArgs a)
     // blocks: 8 x 8 per group, the groups side by side
     auto const block_x = [&](int b) { return int(blockIdx.x) * 8 * GROUPS + (b >> 6) * 8 + (b & 7); };
     auto const block_y = [&](int b) { return int(blockIdx.y) * 8 + ((b >> 3) & 7); };
+    // the next of the tasks that the waves take in turn
+    auto const next_task = [&](int counter) {
+        int task = 0;
+        if (lane == 0) task = atomicAdd(&shared.next[counter], 1);
+        return __builtin_amdgcn_readfirstlane(task);
+    };
 
     for (int i = tid; i < BLOCKS; i += THREADS) {
         shared.alphas[i] = 0u;
-        for (int k = 0; k < kPicks; ++k) shared.picks[k][i] = ~uint64_t(0);
+        for (int k = 0; k < kPicks; ++k) { shared.picks[k][i] = ~uint64_t(0); shared.lowest[k][i] = ~0u; }
     }
+    if (tid < kSearches) shared.queued[tid] = shared.bounded[tid] = 0;
+    if (tid < 2) shared.next[tid] = 0;
+    if (tid == 0) shared.wholes = shared.estimated = 0;
     __syncthreads();
     if (int const b = tid % BLOCKS, row = tid / BLOCKS; row < 4) {
         int const bx = block_x(b), by = block_y(b);
@@ -1061,54 +1468,105 @@ bc7_compress_kernel(BlockCompressArgs a)
     int const opaqueGroups = (opaque + 63) / 64, alphaGroups = (withAlpha + 63) / 64, groups = opaqueGroups + alphaGroups;
     // the lane's block of a group of one kind (lanes beyond the last block repeat it)
     auto const block_of = [&](int kind, int group) { return int(shared.blocks[kind][min(64 * group + lane, (kind ? withAlpha : opaque) - 1)]); };
+    auto const block_of_group = [&](int group) { return group < opaqueGroups ? block_of(0, group) : block_of(1, group - opaqueGroups); };
 
-    // ---- 1. partitions
-    for (int task = wave; task < (2 * opaqueGroups + alphaGroups) * CHUNKS; task += WAVES) {
-        int const first = (task % CHUNKS) * CHUNK, what = task / CHUNKS;
-        if (what >= 2 * opaqueGroups) {
-            pick_task<S, 2, 4, false, true>(lds, block_of(1, what - 2 * opaqueGroups), first, first + CHUNK);
-        } else if (what & 1) {
-            // Mode 7's partition comes with it where every alpha is 1, whose terms are zeros.  Opaque blocks of float
-            // images can hold alphas above 1 and NaNs: their groups estimate it over four channels, as blocks with alpha.
-            int const b = block_of(0, what >> 1);
-            if (__ballot(shared.alphas[b] & kNotOne) == 0) {
-                pick_task<S, 2, 3, true, true>(lds, b, first, first + CHUNK);
+    // Waits for the earlier tasks that a task builds upon: each was taken before it, by a wave that comes to its end.
+    auto const wait_for = [&](int& counter, int count) {
+        while (__hip_atomic_load(&counter, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < count) __builtin_amdgcn_s_sleep(1);
+    };
+    auto const add_one = [&](int& counter) { if (lane == 0) __hip_atomic_fetch_add(&counter, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP); };
+    // Mode 7's partition comes with the two subsets where every alpha is 1, whose terms are zeros.  Opaque blocks of float
+    // images can hold alphas above 1 and NaNs: their groups bound it over four channels, as blocks with alpha.
+    auto const all_ones = [&](int b) { return __ballot(shared.alphas[b] & kNotOne) == 0; };
+
+    // what a search is about, the lanes' blocks, and the search whose tasks give its bounds
+    auto const kind_of = [&](int search) { return search < opaqueGroups ? int(kPickTwo) : search < 2 * opaqueGroups ? int(kPickThree) : int(kPickTwoAlpha); };
+    auto const group_of = [&](int search) { return search < opaqueGroups ? search : search < 2 * opaqueGroups ? search - opaqueGroups : search - 2 * opaqueGroups; };
+    auto const what_of = [&](int search, int b) { return kind_of(search) != kPickTwoAlpha ? kind_of(search) : group_of(search) < opaqueGroups && all_ones(b) ? int(kCorners3) : int(kCorners4); };
+    auto const bounds_of = [&](int search) { return kind_of(search) == kPickTwoAlpha && group_of(search) < opaqueGroups ? group_of(search) : search; };
+
+    // ---- 1. bounds of the partitions' errors; mode 6, which has no partitions; the errors of the first partitions
+    __builtin_amdgcn_s_setprio(3);
+    int const searches = 2 * opaqueGroups + groups, boundTasks = (2 * opaqueGroups + alphaGroups) * CHUNKS;
+    for (int task = next_task(0); task < boundTasks + groups + searches; task = next_task(0)) {
+        if (task < boundTasks) {
+            int const first = (task % CHUNKS) * CHUNK, nth = task / CHUNKS, search = nth < 2 * opaqueGroups ? nth : nth + opaqueGroups;
+            int const b = block_of_group(group_of(search));
+            if (kind_of(search) == kPickThree) {
+                bound_task<S, 3, 3, true, false>(lds, b, first, first + CHUNK);
+            } else if (kind_of(search) == kPickTwo && all_ones(b)) {
+                bound_task<S, 2, 3, true, true>(lds, b, first, first + CHUNK);
             } else {
-                pick_task<S, 2, 3, true, false>(lds, b, first, first + CHUNK);
-                pick_task<S, 2, 4, false, true>(lds, b, first, first + CHUNK);
+                if (kind_of(search) == kPickTwo) bound_task<S, 2, 3, true, false>(lds, b, first, first + CHUNK);
+                bound_task<S, 2, 4, false, true>(lds, b, first, first + CHUNK);
             }
+            add_one(shared.bounded[search]);
+        } else if (task < boundTasks + groups) {
+            finish_task<S, Mode6, 4, true>(lds, block_of_group(task - boundTasks), 0, 8);
         } else {
-            pick_task<S, 3, 3, true, false>(lds, block_of(0, what >> 1), first, first + CHUNK);
+            int const search = task - boundTasks - groups, group = group_of(search);
+            int const b = block_of_group(group), mine = 64 * (group < opaqueGroups ? group : group - opaqueGroups) + lane < (group < opaqueGroups ? opaque : withAlpha);
+            wait_for(shared.bounded[bounds_of(search)], CHUNKS);
+            select_task<S>(lds, b, what_of(search, b), search, mine);
         }
     }
+    __builtin_amdgcn_s_setprio(1);
     __syncthreads();
 
-    // ---- 2. candidates
-    for (int task = wave; task < 4 * opaqueGroups + 6 * groups; task += WAVES) {
-        if (task < 4 * opaqueGroups) {
-            int const which = task & 3, b = block_of(0, task >> 2);
+    // ---- 2. the errors of the partitions that are left, then candidates: first those that need no partition
+    int const wholeTasks = __builtin_amdgcn_readfirstlane(shared.wholes) * (64 / kWholeChunk);
+    int estimates = wholeTasks;
+    for (int search = 0; search < searches; ++search) estimates += (__builtin_amdgcn_readfirstlane(shared.queued[search]) + 63) / 64;
+    for (int task = next_task(1); task < estimates + 4 * opaqueGroups + 5 * groups; task = next_task(1)) {
+        if (task < wholeTasks) {
+            int const search = __builtin_amdgcn_readfirstlane(int(shared.whole[task / (64 / kWholeChunk)])), first = task % (64 / kWholeChunk) * kWholeChunk;
+            int const b = block_of_group(group_of(search)), what = what_of(search, b);
+            if (what == kThree)         pick_task<S, 3, 3, true, false>(lds, b, first, first + kWholeChunk);
+            else if (what == kTwo)      pick_task<S, 2, 3, true, false>(lds, b, first, first + kWholeChunk);
+            else if (what == kCorners3) pick_task<S, 2, 3, false, true>(lds, b, first, first + kWholeChunk);
+            else                        pick_task<S, 2, 4, false, true>(lds, b, first, first + kWholeChunk);
+            add_one(shared.estimated);
+            continue;
+        }
+        if (task < estimates) {
+            int search = 0, piece = task - wholeTasks, count = 0;
+            for (;; ++search) {                              // (ends: the task is a piece of one of the queues)
+                count = __builtin_amdgcn_readfirstlane(shared.queued[search]);
+                if (piece < (count + 63) / 64) break;
+                piece -= (count + 63) / 64;
+            }
+            int const what = what_of(search, block_of_group(group_of(search)));
+            if (piece * 64 + lane < count) {
+                int const item = shared.queues[search][piece * 64 + lane];
+                estimate_one<S>(lds, what, item & 127, item >> 7);
+            }
+            add_one(shared.estimated);
+            continue;
+        }
+        __builtin_amdgcn_s_setprio(0);
+        int const candidate = task - estimates;
+        if (candidate < 4 * groups) {
+            int const which = candidate & 3, b = block_of_group(candidate >> 2);
+            Ends<3> color[2];                                // refined for 2-bit and 3-bit indices
+            Ends<1> alpha[2];
+            dual_plane_ends<S>(lds, b, which, color, alpha);
+            Best best{ FLT_MAX, 0, 0 };
+            dual_plane_form<S, 0>(lds, b, which, color[0], alpha[1], best);
+            dual_plane_form<S, 1>(lds, b, which, color[1], alpha[0], best);
+            dual_plane_form<S, 2>(lds, b, which, color[0], alpha[0], best);
+            put_candidate<S>(lds, 4 + which, b, best.error, best.lo, best.hi);
+            continue;
+        }
+        wait_for(shared.estimated, estimates);
+        int const picked = candidate - 4 * groups;
+        if (picked < 4 * opaqueGroups) {
+            int const which = picked & 3, b = block_of(0, picked >> 2);
             if (which == 0)      finish_task<S, Mode0, 3, true>(lds, b, kPickThree, 0);
             else if (which == 1) finish_task<S, Mode2, 3, true>(lds, b, kPickThree, 1);
             else if (which == 2) finish_task<S, Mode1, 3, true>(lds, b, kPickTwo, 2);
             else                 finish_task<S, Mode3, 3, true>(lds, b, kPickTwo, 3);
         } else {
-            int const which = (task - 4 * opaqueGroups) % 6, group = (task - 4 * opaqueGroups) / 6;
-            int const b = group < opaqueGroups ? block_of(0, group) : block_of(1, group - opaqueGroups);
-            if (which < 4) {
-                Ends<3> color[2];                            // refined for 2-bit and 3-bit indices
-                Ends<1> alpha[2];
-                dual_plane_ends<S>(lds, b, which, color, alpha);
-                Best best{ FLT_MAX, 0, 0 };
-                dual_plane_form<S, 0>(lds, b, which, color[0], alpha[1], best);
-                dual_plane_form<S, 1>(lds, b, which, color[1], alpha[0], best);
-                dual_plane_form<S, 2>(lds, b, which, color[0], alpha[0], best);
-                shared.errors[4 + which][b] = best.error;
-                shared.words[4 + which][b] = make_uint4(uint32_t(best.lo), uint32_t(best.lo >> 32), uint32_t(best.hi), uint32_t(best.hi >> 32));
-            } else if (which == 4) {
-                finish_task<S, Mode6, 4, true>(lds, b, 0, 8);
-            } else {
-                finish_task<S, Mode7, 4, false>(lds, b, kPickTwoAlpha, 9);
-            }
+            finish_task<S, Mode7, 4, false>(lds, block_of_group(picked - 4 * opaqueGroups), kPickTwoAlpha, 9);
         }
     }
     __syncthreads();
@@ -1119,8 +1577,10 @@ bc7_compress_kernel(BlockCompressArgs a)
         if (bx < a.widthInBlocks && by < a.heightInBlocks) {
             float bestError = FLT_MAX;
             uint4 best = make_uint4(0u, 0u, 0u, 0u);
-            for (int slot = (shared.alphas[b] & kBelowOne) ? 4 : 0; slot < kSlots; ++slot)
-                if (!(shared.errors[slot][b] > bestError)) { bestError = shared.errors[slot][b]; best = shared.words[slot][b]; }
+            for (int slot = (shared.alphas[b] & kBelowOne) ? 4 : 0; slot < kSlots; ++slot) {
+                float const error = slot == 8 ? shared.early.errors[b] : shared.late.errors[min(slot, 8)][b];
+                if (!(error > bestError)) { bestError = error; best = slot == 8 ? shared.early.words[b] : shared.late.words[min(slot, 8)][b]; }
+            }
             store_block(a, bx, by, uint64_t(best.x) | uint64_t(best.y) << 32, uint64_t(best.z) | uint64_t(best.w) << 32);
         }
     }
@@ -1213,8 +1673,7 @@ hipError_t launch_bc7_compress(BlockCompressArgs const& a, hipStream_t stream)
         // One group of 64 blocks per workgroup while there are no more groups than compute units (sixteen waves then
         // have a unit to themselves), else two and half the waves, two workgroups to a unit: the groups' blocks with
         // and without alpha fill their tasks' lanes better, and one workgroup works while the other waits for its
-        // last task.  512 x 512: 111 us (174 with two groups); 700 x 700: 222 (293 with four); 1024 x 1024: 290 (427
-        // with one).
+        // last task.  (With every partition estimated: 512 x 512 111 us, 174 with two groups; 1024 x 1024 290, 427 with one.)
         int const groupsX = (a.widthInBlocks + 7) / 8, groupsY = (a.heightInBlocks + 7) / 8;
         if (int64_t(groupsX) * groupsY <= compute_units_of_current_device())
             hipLaunchKernelGGL((bc7_compress_kernel<1, 16>), dim3(groupsX, groupsY), dim3(1024), 0, stream, a);

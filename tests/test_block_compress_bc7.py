@@ -423,6 +423,46 @@ def test_gpu_bc7_opaque_blocks_whose_alpha_is_not_one_match_checker(ntc, device,
     assert np.array_equal(compress_bc7(ntc, None, device, *args), compress_bc7(ntc, oracle, None, *args))
 
 
+def image_for_bounds(rng, content, w, h):
+    """RGBA float32, a quarter of the blocks with alpha.  Which of the search's ways the partitions' errors take: "noise" a
+    few estimates beyond the first; "edges" more than the queues hold; "grey" no bounds, because channels are proportional;
+    "level" subsets that are level in channels; "faint" covariances whose signs are within their errors; "tiny" and "huge"
+    texels' offsets outside the range that has bounds."""
+    ys, xs = np.mgrid[0:h, 0:w].astype(np.float32)
+    ramps = 0.3 + 0.4 * np.stack([xs / w, ys / h, (xs + 2 * ys) / (w + 2 * h)], axis=-1)
+    noise = rng.normal(0, 0.02, (h, w, 3))
+    if content == "noise":
+        rgb = ramps + noise
+    elif content == "edges":
+        rgb = np.where(rng.random((h, w, 1)) < 0.5, ramps, ramps[::-1, ::-1] + 0.2)
+    elif content == "grey":
+        rgb = (ramps[..., :1] + noise[..., :1]) * [1.0, 1.0, 0.5]
+    elif content == "level":
+        rgb = np.round((ramps + noise) * 16) / 16
+        rgb[..., 0] = np.where(rng.random((h, w)) < 0.03, 0.75, 0.5)
+    elif content == "faint":
+        rgb = 0.5 + noise * np.float32(2.0 ** -14)
+    else:
+        rgb = noise * (1e-12 if content == "tiny" else 1e12) * np.where(rng.random((h, w, 1)) < 0.5, 1, 30)
+    alpha = np.ones((h, w, 1))
+    alpha[: h // 2, : w // 2] = np.where(rng.random((h // 2, w // 2, 1)) < 0.2, rng.random((h // 2, w // 2, 1)), 1)
+    return np.concatenate([rgb, alpha], axis=-1).astype(np.float32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("content", ["noise", "edges", "grey", "level", "faint", "tiny", "huge"])
+@pytest.mark.parametrize("size", [(68, 60), (520, 524)])    # workgroups of one group of 64 blocks, and of two
+def test_gpu_bc7_search_with_bounds_matches_checker(ntc, device, oracle, size, content):
+    image = image_for_bounds(np.random.default_rng(80), content, *size)
+    formats = [(4, image)]
+    if content in ("noise", "edges", "grey", "level"):
+        formats.append((1, np.clip(np.rint(image * 255), 0, 255).astype(np.uint8)))
+    for fmt, texels in formats:
+        args = (np.ascontiguousarray(texels), fmt, 4, size[0] // 4, size[1] // 4)
+        got, want = compress_bc7(ntc, None, device, *args), compress_bc7(ntc, oracle, None, *args)
+        assert np.array_equal(got, want), (fmt, np.argwhere(got != want)[:4])
+
+
 @pytest.mark.gpu
 def test_gpu_bc7_arguments(ntc, device, oracle):
     from test_image_difference import fill_image
