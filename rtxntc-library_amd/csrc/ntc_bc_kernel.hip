@@ -191,8 +191,8 @@ __device__ __forceinline__ void bc4_load(BlockCompressArgs const& a, int bx, int
 #pragma unroll
         for (int y = 0; y < 4; ++y, px += a.rowPitch) {
             uint32_t words[4];
-            if (a.pixelStride == 1) {                        // uniform; c is 0
-                uint32_t const v = *reinterpret_cast<u32_unaligned const*>(px);
+            if (a.pixelStride == 1) {                        // uniform; the image has no channel 1
+                uint32_t const v = c == 0 ? *reinterpret_cast<u32_unaligned const*>(px) : 0u;
                 words[0] = v; words[1] = v >> 8; words[2] = v >> 16; words[3] = v >> 24;
             } else {
 #pragma unroll

@@ -228,11 +228,11 @@ def test_gpu_block_compress_matches_checker(ntc, device, oracle, fmt, dst_format
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("channels,dst_format", [(1, 4), (2, 5), (3, 5)])
+@pytest.mark.parametrize("channels,dst_format", [(1, 4), (2, 5), (3, 5), (1, 5)])
 @pytest.mark.parametrize("w,h", [(4, 4), (68, 36), (130, 71)])
 def test_gpu_extreme_blocks_of_packed_rows_match_checker(ntc, device, oracle, channels, dst_format, w, h):
     """UNORM8 pixels without padding; blocks of one, two and few values with 0 and 255 among them, so that either
-    palette's endpoints coincide, wrap or stay pinned; full blocks beside cut-off ones."""
+    palette's endpoints coincide, wrap or stay pinned; full blocks beside cut-off ones; a channel that the image lacks."""
     rng = np.random.default_rng(w + channels)
     image = np.zeros((h, w, channels), dtype=np.uint8)
     for y in range(0, h, 4):
