@@ -66,6 +66,8 @@ __device__ __forceinline__ float encode_color_space(int colorSpace, float v)
 // large enough to pay for it; other halves are read from the table in memory (256 KB a pair, cached).
 constexpr int kTransferPairs = 8;                            // src * 3 + dst - 1; linear to linear has no table
 constexpr uint32_t kStageFirst = 0x2400u, kStageCount = 0x1801u;     // halves 1/64 .. 1
+constexpr uint32_t kStageStride = kStageCount + 3u;          // of the copies in LDS, whole vectors
+constexpr uint32_t kStagingThreads = 1024;
 static __device__ float transferOfHalf[kTransferPairs][65536];
 static __device__ uint16_t storedOfUnorm16[kTransferPairs][65536];   // UNORM16 code -> half of the internal layout
 static __device__ uint16_t storedOfUnorm8[kTransferPairs + 1][256];  // UNORM8 code -> half; [8]: linear
@@ -130,7 +132,8 @@ __device__ __forceinline__ float transfer_half(int pair, uint32_t bits)
 }
 // The same for four pixels' halves of one channel through the copies in LDS: slot 1 or 2 (uniform) names the copy that
 // holds the pair, 0 none.  (The look-up in LDS happens for every half, out-of-range ones clamped: a choice between the
-// two tables per half would become a choice of address and a flat load.)
+// two tables per half would become a choice of address and a flat load.  Look-ups in memory are waited for where they
+// are made, or every path would wait there for all loads in flight, the next pixels' among them.)
 __device__ __forceinline__ void transfer_halves(float const* staged, int slot, int pair, uint32_t const (&bits)[4], float (&value)[4])
 {
     if (pair < 0) {                                          // uniform
@@ -139,8 +142,10 @@ __device__ __forceinline__ void transfer_halves(float const* staged, int slot, i
     } else if (slot == 0) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) value[k] = transferOfHalf[pair][bits[k]];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) asm volatile("" : "+v"(value[k]));
     } else {
-        float const* const copy = staged + (slot - 1) * int(kStageCount);
+        float const* const copy = staged + (slot - 1) * int(kStageStride);
         uint32_t at[4];
         bool beyond = false;
 #pragma unroll
@@ -152,6 +157,8 @@ __device__ __forceinline__ void transfer_halves(float const* staged, int slot, i
         if (beyond) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) if (at[k] >= kStageCount) value[k] = transferOfHalf[pair][bits[k]];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) asm volatile("" : "+v"(value[k]));
         }
     }
 }
@@ -372,7 +379,7 @@ static GroupGrid group_grid(int width, int height, int threads)
 }
 
 // The tables that a launch copies into LDS: the first two pairs of colour spaces that its channels use.
-struct StagedTransfers {
+struct alignas(4) StagedTransfers {                         // (at an odd address its bytes would be read by vector loads)
     int8_t count;                                            // 0: nothing staged
     int8_t staged[2];                                        // the pairs
     int8_t pair[8], slot[8];                                 // per channel: its pair (-1 linear) and the copy that holds it (0 none)
@@ -390,11 +397,11 @@ struct GroupLaunch {
 
 static GroupLaunch plan_groups(int width, int height, uint8_t const* src, uint8_t const* dst, int channels, bool readsHalves)
 {
-    constexpr int kStagingThreads = 1024, kSmallThreads = 256, kTilesPerStaging = 2;
+    constexpr int kSmallThreads = 256, kTilesPerStaging = 2;
     GroupLaunch l{};
     StagedTransfers& s = l.transfers;
     int const units = compute_units_of_current_device();
-    l.grid = group_grid(width, height, kStagingThreads);
+    l.grid = group_grid(width, height, int(kStagingThreads));
     bool const stage = readsHalves && l.grid.tiles >= kTilesPerStaging * units;
     for (int c = 0; c < 8; ++c) {
         s.pair[c] = c < channels ? int8_t(transfer_pair(src[c], dst[c])) : int8_t(-1);
@@ -406,7 +413,7 @@ static GroupLaunch plan_groups(int width, int height, uint8_t const* src, uint8_
         int const share = (l.grid.tiles + kTilesPerStaging - 1) / kTilesPerStaging;
         l.threads = kStagingThreads;
         l.grid.step = 2 * units < share ? 2 * units : share;
-        l.ldsBytes = unsigned(s.count * kStageCount * sizeof(float));
+        l.ldsBytes = unsigned(s.count * kStageStride * sizeof(float));
     } else {
         l.grid = group_grid(width, height, kSmallThreads);
         l.threads = kSmallThreads;
@@ -414,13 +421,40 @@ static GroupLaunch plan_groups(int width, int height, uint8_t const* src, uint8_
     return l;
 }
 
-__device__ __forceinline__ void copy_staged(StagedTransfers const& s, float* lds, uint32_t threads)
+// Copies them: workgroups of kStagingThreads, 16 bytes a load and all loads in flight before the first is stored.  (A loop of
+// dword loads, each waited for before the next, was a chain of six or twelve trips to the L2 in front of every launch's
+// pixels: 2048 x 2048, sRGB dithered 19.6 us, HLG halves written 15.5, the 2 : 1 reduction 34.)
+__device__ __forceinline__ void copy_staged(StagedTransfers const& s, float* lds)
 {
-    for (int k = 0; k < s.count; ++k) {
-        float const* const from = &transferOfHalf[s.staged[k]][kStageFirst];
-        for (uint32_t i = threadIdx.x; i < kStageCount; i += threads) lds[k * int(kStageCount) + int(i)] = from[i];
+    if (s.count == 0) return;
+    constexpr uint32_t VECTORS = kStageCount / 4, STEPS = (VECTORS + kStagingThreads - 1) / kStagingThreads;
+    static_assert(kStageCount == 4 * VECTORS + 1, "the table's end is 1");
+    float4 v[2][STEPS];
+    float last[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {                            // (one table twice if there is one)
+        float const* const from = &transferOfHalf[k < s.count ? s.staged[k] : s.staged[0]][kStageFirst];
+#pragma unroll
+        for (uint32_t i = 0; i < STEPS; ++i) v[k][i] = reinterpret_cast<float4 const*>(from)[min(threadIdx.x + i * kStagingThreads, VECTORS - 1u)];
+        last[k] = from[kStageCount - 1u];
     }
-    if (s.count) __syncthreads();
+    // (here, or each is loaded where it is stored)
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        asm volatile("" : "+v"(last[k]));
+#pragma unroll
+        for (uint32_t i = 0; i < STEPS; ++i) asm volatile("" : "+v"(v[k][i].x), "+v"(v[k][i].y), "+v"(v[k][i].z), "+v"(v[k][i].w));
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        if (k >= s.count) continue;
+        float* const to = lds + k * int(kStageStride);
+#pragma unroll
+        for (uint32_t i = 0; i < STEPS; ++i)
+            if (uint32_t const at = threadIdx.x + i * kStagingThreads; at < VECTORS) reinterpret_cast<float4*>(to)[at] = v[k][i];
+        if (threadIdx.x == 0) to[kStageCount - 1u] = last[k];
+    }
+    __syncthreads();
 }
 
 // What the kernels need of a ReadChannelsArgs or WriteChannelsArgs, in as few bytes as launches are quick with.
@@ -446,7 +480,7 @@ read_groups_kernel(GroupsArgs a)
     static_assert(PIXEL <= 8, "the words of four pixels stay in registers");
     extern __shared__ float staged[];
     uint32_t const threads = 1u << (a.grid.log2LanesX + a.grid.log2Rows);
-    copy_staged(a.transfers, staged, threads);
+    copy_staged(a.transfers, staged);
     int const lanesX = 1 << a.grid.log2LanesX;
     int const lx = int(threadIdx.x) & (lanesX - 1), ly = int(threadIdx.x) >> a.grid.log2LanesX;
     int const firstPair = a.firstChannel >> 1;
@@ -598,7 +632,7 @@ write_groups_kernel(GroupsArgs a)
         }
         __syncthreads();
     }
-    if constexpr (HALVES) copy_staged(a.transfers, staged, threads);
+    if constexpr (HALVES) copy_staged(a.transfers, staged);
     int const lanesX = 1 << a.grid.log2LanesX;
     int const lx = int(threadIdx.x) & (lanesX - 1), ly = int(threadIdx.x) >> a.grid.log2LanesX;
     int const odd = a.firstChannel & 1;
@@ -872,16 +906,17 @@ write_channels_resize_kernel(WriteChannelsArgs a)
 // values are decoded by table (from LDS in launches large enough, as in the copies above; a powf per tap and channel
 // kept the kernel at 0.9 TB/s), the filtered value is encoded by the device function.  Images too small to fill the
 // GPU are split by channel pairs: one mip of 64 x 64 and six pairs is 64 waves, not 4, in a chain a sixth as long.
-// 2048 x 2048, 12 channels (three sRGB, three HLG): 39 us for the 1024 x 1024 mip, 68 before (56 with the math library's
-// encoding, which took half of the vector instructions); 13 for the next, 24 before; the nine smaller ones 4 - 6 each,
-// 12 - 24 before.
+// This kernel is for sizes that are no exact halves (a mip of an odd one); the others are halve_planar_kernel's.
 struct ResizePlanarArgs {
     uint16_t const* src; uint16_t* dst;
     int32_t srcWidth, srcHeight, dstWidth, dstHeight, setChannels;
     int32_t tilesX, tiles, pairsPerLane;                     // tiles of 64 pixels x a row per wave
     int32_t step, threads;                                   // workgroups in x, threads of each
-    StagedTransfers transfers;                               // of the decoding pairs; pair / slot: per colour space
-    uint8_t colorSpaces[16];
+    StagedTransfers transfers;                               // of the decoding pairs
+    uint32_t spaces;                                         // two bits a channel; (an array indexed by a loop's variable would be
+    uint32_t slots;                                          // a load from memory each time); per space: the copy that holds its pair
+    __device__ __forceinline__ int space(int channel) const { return int(spaces >> (2 * channel)) & 3; }
+    __device__ __forceinline__ int slot(int space) const { return int(slots >> (2 * space)) & 3; }
 };
 
 template <bool LINEAR>
@@ -889,7 +924,7 @@ __global__ void __launch_bounds__(1024, 8)
 resize_planar_kernel(ResizePlanarArgs a)
 {
     extern __shared__ float staged[];
-    if constexpr (!LINEAR) copy_staged(a.transfers, staged, uint32_t(a.threads));
+    if constexpr (!LINEAR) copy_staged(a.transfers, staged);
     int const pairBegin = int(blockIdx.y) * a.pairsPerLane, pairEnd = min(a.setChannels >> 1, pairBegin + a.pairsPerLane);
     size_t const srcRow = size_t(a.srcWidth) * size_t(a.setChannels), pairStride = size_t(a.srcWidth) * 2;
     for (int tile = blockIdx.x; tile < a.tiles; tile += a.step) {
@@ -926,11 +961,11 @@ resize_planar_kernel(ResizePlanarArgs a)
                 uint32_t packed = 0;
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
-                    int const space = LINEAR ? 0 : a.colorSpaces[2 * p + k];
+                    int const space = LINEAR ? 0 : a.space(2 * p + k);
                     uint32_t const bits[4] = { (v00 >> (16 * k)) & 0xffffu, (v10 >> (16 * k)) & 0xffffu, (v01 >> (16 * k)) & 0xffffu, (v11 >> (16 * k)) & 0xffffu };
                     float v[4];
                     if constexpr (LINEAR) transfer_halves(staged, 0, -1, bits, v);
-                    else                  transfer_halves(staged, a.transfers.slot[space], a.transfers.pair[space], bits, v);
+                    else                  transfer_halves(staged, a.slot(space), transfer_pair(space, 0), bits, v);
                     packed |= encoded_half(space, blend_taps<ALL>(t, v[0], v[1], v[2], v[3])) << (16 * k);
                 }
                 out[size_t(p) * size_t(a.dstWidth)] = packed;
@@ -941,6 +976,71 @@ resize_planar_kernel(ResizePlanarArgs a)
     }
 }
 
+// The same for an image of exactly half the width and height, what each mip is of an even one above it: the taps of pixel x
+// are pixels 2 x and 2 x + 1 whatever the roundings of its position (which is off by less than 0.01 up to 65536 pixels),
+// none of them without weight.  A lane makes two pixels from 16 bytes of each row, and a pair's are under way while the one
+// before is filtered.  Bound by memory where the image is large, by the tables' gathers in the middle, by the launch below
+// 128 x 128.  4096 x 4096, 2048 x 2048 and 1024 x 1024 of 12 channels, three sRGB and three HLG: 162, 35 and 12.2 us with 8
+// bytes a load, colour spaces read from memory at each pair (a wait for everything in flight, the next pair's taps too) and
+// tables copied dword by dword; 106, 24 and 10.5 now, 5.0 of 5.7 TB/s that linear channels reach.  Tables in LDS for the
+// 1024 x 1024 image as well take longer to copy than they save (13.4).
+template <bool LINEAR>
+__global__ void __launch_bounds__(1024, 8)
+halve_planar_kernel(ResizePlanarArgs a)
+{
+    extern __shared__ float staged[];
+    int const pairBegin = int(blockIdx.y) * a.pairsPerLane, pairEnd = min(a.setChannels >> 1, pairBegin + a.pairsPerLane);
+    size_t const srcRow = size_t(a.srcWidth) * size_t(a.setChannels), pairStride = size_t(a.srcWidth) * 2;
+    int const lane = int(threadIdx.x & 63), row = int(threadIdx.x >> 6);
+    // (the last lane of an odd row makes the pixel before the last one too, like the lane that it is another's)
+    auto const row_of = [&](int tile, int& x, int& y) -> uint16_t const* {
+        int const tileY = tile / a.tilesX, tileX = tile - tileY * a.tilesX;
+        x = min((tileX * 64 + lane) * 2, a.dstWidth - 2); y = min(tileY * (a.threads >> 6) + row, a.dstHeight - 1);
+        return a.src + size_t(2 * y) * srcRow + size_t(x) * 4;
+    };
+    u32x4_a4 top, bottom;
+    auto const load = [&](uint16_t const* from) {
+        top = *reinterpret_cast<u32x4_a4 const*>(from);
+        bottom = *reinterpret_cast<u32x4_a4 const*>(from + srcRow);
+    };
+    int x, y;
+    uint16_t const* from = row_of(blockIdx.x, x, y);
+    load(from + size_t(pairBegin) * pairStride);
+    if constexpr (!LINEAR) copy_staged(a.transfers, staged);
+    for (int tile = blockIdx.x; tile < a.tiles; tile += a.step) {
+        int const tileY = tile / a.tilesX, tileX = tile - tileY * a.tilesX;
+        bool const inside = (tileX * 64 + lane) * 2 < a.dstWidth && tileY * (a.threads >> 6) + row < a.dstHeight;
+        BilinearTaps const t0 = setup_bilinear(a.srcWidth, a.srcHeight, a.dstWidth, a.dstHeight, x, y);
+        BilinearTaps const t1 = setup_bilinear(a.srcWidth, a.srcHeight, a.dstWidth, a.dstHeight, x + 1, y);
+        uint16_t* const to = a.dst + size_t(y) * size_t(a.dstWidth) * size_t(a.setChannels) + size_t(x) * 2;
+        for (int p = pairBegin; p < pairEnd; ++p) {
+            u32x4_a4 const upper = top, lower = bottom;
+            if (p + 1 < pairEnd) {
+                load(from + size_t(p + 1) * pairStride);
+            } else if (tile + a.step < a.tiles) {            // (uniform, both)
+                int nextX, nextY;
+                load(row_of(tile + a.step, nextX, nextY) + size_t(pairBegin) * pairStride);
+            }
+            uint32_t packed[2] = { 0u, 0u };
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                int const space = LINEAR ? 0 : a.space(2 * p + k);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    uint32_t const bits[4] = { (upper[2 * i] >> (16 * k)) & 0xffffu, (upper[2 * i + 1] >> (16 * k)) & 0xffffu,
+                                               (lower[2 * i] >> (16 * k)) & 0xffffu, (lower[2 * i + 1] >> (16 * k)) & 0xffffu };
+                    float v[4];
+                    if constexpr (LINEAR) transfer_halves(staged, 0, -1, bits, v);
+                    else                  transfer_halves(staged, a.slot(space), transfer_pair(space, 0), bits, v);
+                    packed[i] |= encoded_half(space, blend_taps<true>(i ? t1 : t0, v[0], v[1], v[2], v[3])) << (16 * k);
+                }
+            }
+            if (inside) *reinterpret_cast<u32x2_a4*>(to + size_t(p) * size_t(a.dstWidth) * 2) = u32x2_a4{ packed[0], packed[1] };
+        }
+        if (tile + a.step < a.tiles) from = row_of(tile + a.step, x, y);
+    }
+}
+
 hipError_t launch_resize_planar(uint16_t const* src, int srcWidth, int srcHeight, uint16_t* dst, int dstWidth, int dstHeight,
                                 int setChannels, uint8_t const* colorSpaces, hipStream_t stream)
 {
@@ -948,25 +1048,26 @@ hipError_t launch_resize_planar(uint16_t const* src, int srcWidth, int srcHeight
     a.src = src; a.dst = dst; a.srcWidth = srcWidth; a.srcHeight = srcHeight; a.dstWidth = dstWidth; a.dstHeight = dstHeight; a.setChannels = setChannels;
     bool linear = true;
     for (int i = 0; i < 16; ++i) {
-        a.colorSpaces[i] = colorSpaces ? colorSpaces[i] : 0;
-        linear = linear && (a.colorSpaces[i] == 0 || i >= setChannels);
+        uint32_t const space = colorSpaces && i < setChannels ? colorSpaces[i] : 0u;
+        a.spaces |= space << (2 * i);
+        linear = linear && space == 0u;
     }
     int const units = compute_units_of_current_device(), pairs = setChannels / 2;
+    bool const half = dstWidth >= 2 && srcWidth == 2 * dstWidth && srcHeight == 2 * dstHeight && srcWidth <= 65536 && srcHeight <= 65536;
+    int const tileWidth = half ? 128 : 64;
     auto tile = [&](int threads) {
-        a.tilesX = (dstWidth + 63) / 64;
+        a.tilesX = (dstWidth + tileWidth - 1) / tileWidth;
         a.tiles = a.tilesX * ((dstHeight + threads / 64 - 1) / (threads / 64));
     };
-    int threads = 1024;
+    int threads = int(kStagingThreads);
     tile(threads);
-    bool const stage = !linear && a.tiles >= 2 * units;      // as in plan_groups: each copy serves two tiles or more
-    a.transfers.pair[0] = -1;
+    bool const stage = !linear && a.tiles * tileWidth >= 128 * units;            // as in plan_groups: each copy serves two pixels a thread or more
     for (int space = 1; space <= 2; ++space) {
-        a.transfers.pair[space] = int8_t(transfer_pair(space, 0));
         bool used = false;
-        for (int i = 0; i < setChannels; ++i) used = used || a.colorSpaces[i] == space;
+        for (int i = 0; i < setChannels; ++i) used = used || ((a.spaces >> (2 * i)) & 3u) == uint32_t(space);
         if (!stage || !used) continue;
-        a.transfers.staged[a.transfers.count] = a.transfers.pair[space];
-        a.transfers.slot[space] = int8_t(++a.transfers.count);
+        a.transfers.staged[a.transfers.count] = int8_t(transfer_pair(space, 0));
+        a.slots |= uint32_t(++a.transfers.count) << (2 * space);
     }
     dim3 grid(1);
     a.pairsPerLane = pairs;
@@ -981,9 +1082,11 @@ hipError_t launch_resize_planar(uint16_t const* src, int srcWidth, int srcHeight
         a.pairsPerLane = (pairs + ranges - 1) / ranges;
         grid = dim3(unsigned(a.tiles), unsigned((pairs + a.pairsPerLane - 1) / a.pairsPerLane));
     }
-    size_t const lds = size_t(a.transfers.count) * kStageCount * sizeof(float);
+    size_t const lds = size_t(a.transfers.count) * kStageStride * sizeof(float);
     a.step = int(grid.x);
     a.threads = threads;
+    if (half) return linear ? launch_kernel<halve_planar_kernel<true>>(grid, dim3(threads), lds, stream, a)
+                            : launch_kernel<halve_planar_kernel<false>>(grid, dim3(threads), lds, stream, a);
     return linear ? launch_kernel<resize_planar_kernel<true>>(grid, dim3(threads), lds, stream, a)
                   : launch_kernel<resize_planar_kernel<false>>(grid, dim3(threads), lds, stream, a);
 }

@@ -185,6 +185,24 @@ def test_gpu_resize_planar_matches_checker(ntc, device, oracle):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("channels", [2, 6, 16])
+@pytest.mark.parametrize("dw,dh", [(1, 3), (2, 1), (3, 3), (129, 5), (1023, 12), (1024, 520)])     # the last: tables in LDS
+def test_gpu_halved_planar_matches_checker(ntc, device, oracle, dw, dh, channels):
+    """Exactly half of both sizes: two pixels a lane, the last ones of odd rows among them."""
+    rng = np.random.default_rng(47 + dw + channels)
+    for spaces in (None, np.array([1, 0, 2, 1] * 4, dtype=np.uint8)):
+        src = random_planar(rng, 2 * dw, 2 * dh, channels, wild=spaces is None)
+        d_src, d_dst = device.upload(src), device.upload(np.full(dw * dh * channels + 8, 0xEEEE, dtype=np.uint16))
+        ntc.abi.check(device.lib.ntc_hip_resize_planar(d_src.ptr, d_src.nbytes, 2 * dw, 2 * dh, d_dst.ptr, d_dst.nbytes - 16, dw, dh, channels,
+                                                       spaces.ctypes.data if spaces is not None else None))
+        device.synchronize()
+        got, want = d_dst.download().view(np.uint16), oracle_resize(oracle, src, 2 * dw, 2 * dh, dw, dh, channels, spaces)
+        assert np.all(got[-8:] == 0xEEEE)
+        # (transfer functions come from each side's math library: one half ulp of slack)
+        assert np.abs(got[:-8].astype(np.int32) - want.astype(np.int32)).max() <= (0 if spaces is None else 1)
+
+
+@pytest.mark.gpu
 def test_host_layer_generate_mips(ntc, oracle, tmp_path):
     """WriteChannels from an image of twice the size of mip 0, GenerateMips, and the reference page of
     every mip against the checker's chain of resamplings (channel 1 stored as sRGB)."""
