@@ -28,6 +28,13 @@ __device__ __forceinline__ uint32_t unorm_code(float p, float top)
     return uint32_t(fminf(fmaxf(p, 0.f) + 0.49999997f, top));
 }
 
+// unorm_code(p, 255) as byte `at` of a word: the conversion that packs it saturates at both ends, in three instructions for
+// five (equal for every float: tests).
+__device__ __forceinline__ uint32_t put_unorm8(float p, uint32_t at, uint32_t word)
+{
+    return __builtin_amdgcn_cvt_pk_u8_f32(__builtin_floorf(p + 0.49999997f), at, word);
+}
+
 // Transfer functions, src/CudaUtils.h:61-114 (sRGB, Hybrid Log-Gamma) and src/ImageProcessing.cu:86-111.
 // The transcendental parts are the device math library's, so results agree with a CPU
 // evaluation to a few units in the last place, not bit for bit.
@@ -60,7 +67,7 @@ __device__ __forceinline__ float encode_color_space(int colorSpace, float v)
 // vector instructions, sRGB to sRGB takes two of them and two divisions per channel: 2048 x 2048 sRGB pixels of 8
 // bits, dithered, took 103 us to read that way and 91 us to write.
 //
-// With the tables (and the groups of four pixels below) they take 23 and 16 us.
+// With the tables (and the groups of four pixels below) they take 19 and 11 us.
 //
 // The floats of the halves in [1/64, 1], which is nearly everything a texture holds, are copied into LDS by launches
 // large enough to pay for it; other halves are read from the table in memory (256 KB a pair, cached).
@@ -76,6 +83,12 @@ __device__ __forceinline__ uint16_t stored_half(float v)     // WriteImageChanne
 {
     v = fmaxf(-65504.f, fminf(65504.f, v));
     asm volatile("" : "+v"(v));
+    return __builtin_bit_cast(uint16_t, (_Float16)v);
+}
+
+__device__ __forceinline__ uint16_t unit_half(float v)       // of a v in [0, 1]
+{
+    asm volatile("" : "+v"(v));                              // (a multiply-add that rounds to a half rounds once)
     return __builtin_bit_cast(uint16_t, (_Float16)v);
 }
 
@@ -162,12 +175,11 @@ __device__ __forceinline__ void transfer_halves(float const* staged, int slot, i
         }
     }
 }
-// a / b for b = 255 or 65535 and every a that occurs here (codes, dither draws): the product with the reciprocal
-// corrected by its remainder is the correctly rounded quotient for all of them (checked exhaustively).
+// a / b for b = 255 or 65535 and every a that occurs here (codes, dither draws): the product with the reciprocal as the sum
+// of two floats, rounded once, is the correctly rounded quotient for all of them (checked exhaustively).
 __device__ __forceinline__ float divide_by_top(float a, float top, float reciprocal)
 {
-    float const q = a * reciprocal;
-    return __builtin_fmaf(__builtin_fmaf(-q, top, a), reciprocal, q);
+    return __builtin_fmaf(a, reciprocal, a * float(1.0 / double(top) - double(reciprocal)));
 }
 
 // HashBasedRNG, src/CudaUtils.h:117-184: Jenkins hash of the pixel index seeds a Murmur3 round per draw.
@@ -350,7 +362,13 @@ typedef uint32_t u32x4_a4  __attribute__((ext_vector_type(4), aligned(4)));
 
 // Which pixels a lane works on: tiles of lanesX groups by threads / lanesX rows, a workgroup takes tiles
 // blockIdx.x, blockIdx.x + step, ...
-struct GroupGrid { int32_t tilesX, tiles, step; uint8_t log2LanesX, log2Rows; };
+// (perRow: 2^40 / tilesX rounded up, 0 where a product with a tile's number could be inexact or too large.)
+struct GroupGrid {
+    int32_t tilesX, tiles, step;
+    uint16_t log2LanesX, log2Rows;
+    uint64_t perRow;
+    __device__ __forceinline__ int row_of(int tile) const { return perRow ? int((uint32_t(tile) * perRow) >> 40) : tile / tilesX; }
+};
 
 int compute_units_of_current_device()
 {
@@ -369,29 +387,51 @@ static GroupGrid group_grid(int width, int height, int threads)
 {
     GroupGrid g;
     int const groups = (width + 3) / 4;
-    g.log2LanesX = uint8_t(groups > 32 ? 6 : groups > 16 ? 5 : groups > 8 ? 4 : 3);
+    g.log2LanesX = uint16_t(groups > 32 ? 6 : groups > 16 ? 5 : groups > 8 ? 4 : 3);
     int const rows = threads >> g.log2LanesX;
-    g.log2Rows = uint8_t(__builtin_ctz(unsigned(rows)));
+    g.log2Rows = uint16_t(__builtin_ctz(unsigned(rows)));
     g.tilesX = (groups + (1 << g.log2LanesX) - 1) >> g.log2LanesX;
     g.tiles = g.tilesX * ((height + rows - 1) / rows);
     g.step = g.tiles;
+    g.perRow = g.tiles < 1 << 23 && g.tilesX < 1 << 16 ? ((uint64_t(1) << 40) + unsigned(g.tilesX) - 1u) / unsigned(g.tilesX) : 0u;
     return g;
 }
 
-// The tables that a launch copies into LDS: the first two pairs of colour spaces that its channels use.
-struct alignas(4) StagedTransfers {                         // (at an odd address its bytes would be read by vector loads)
-    int8_t count;                                            // 0: nothing staged
-    int8_t staged[2];                                        // the pairs
-    int8_t pair[8], slot[8];                                 // per channel: its pair (-1 linear) and the copy that holds it (0 none)
+// The pairs of colour spaces of a launch's channels, and the tables that it copies into LDS: the first two that they use.
+// (In words: bytes of a kernel's arguments can be vector loads, and those indexed by a loop's variable always are.)
+struct Transfers {
+    uint32_t pairs = 0;                                      // four bits a channel: its pair + 1 (0: linear)
+    uint32_t rest = 0;                                       // two bits a channel: the copy that holds it (0 none); from bit 16 on the number of copies and their pairs
+    void set(int channel, int pair, int copy) { pairs |= uint32_t(pair + 1) << (4 * channel); rest |= uint32_t(copy) << (2 * channel); }
+    int copy_of(int pair) const
+    {
+        for (int k = 0; k < count(); ++k) if (staged(k) == pair) return k + 1;
+        return 0;
+    }
+    int stage(int pair)                                      // the copy that holds it, a new one while there are less than two
+    {
+        int const n = count();
+        if (int const k = copy_of(pair)) return k;
+        if (n == 2) return 0;
+        rest += 1u << 16;
+        rest |= uint32_t(pair) << (20 + 4 * n);
+        return n + 1;
+    }
+    __host__ __device__ __forceinline__ int pair(int channel) const { return int((pairs >> (4 * channel)) & 15u) - 1; }
+    __host__ __device__ __forceinline__ int slot(int channel) const { return int((rest >> (2 * channel)) & 3u); }
+    __host__ __device__ __forceinline__ int count() const { return int((rest >> 16) & 3u); }
+    __host__ __device__ __forceinline__ int staged(int k) const { return int((rest >> (20 + 4 * k)) & 15u); }
 };
 
 // Launch shape of the group kernels.  Images of two million pixels and more stage: workgroups of 1024 threads, two to
 // a compute unit, that share a copy among two tiles or more each (2048 x 2048 read as dithered sRGB: 22.9 us, 24.4 with
-// 512 threads, 28 with 256, 24.8 straight from the table in memory; HLG to linear halves: 19.6, 23.4, 22.6, 24.5).
-// Smaller images, and those of linear channels, take small workgroups, a tile each.
+// 512 threads, 28 with 256, 24.8 straight from the table in memory; HLG to linear halves: 19.6, 23.4, 22.6, 24.5; before
+// the copies' loads were made at once and the next tile's pixels loaded ahead: 18.6 and 14.3 now).
+// Smaller images, and those of linear channels, take small workgroups.  Either way no more than are resident: a workgroup
+// loads its next tile's pixels before it works on one's, and its first tile's before it fills its tables.
 struct GroupLaunch {
     GroupGrid grid;
-    StagedTransfers transfers;
+    Transfers transfers;
     unsigned threads, ldsBytes;
 };
 
@@ -399,24 +439,24 @@ static GroupLaunch plan_groups(int width, int height, uint8_t const* src, uint8_
 {
     constexpr int kSmallThreads = 256, kTilesPerStaging = 2;
     GroupLaunch l{};
-    StagedTransfers& s = l.transfers;
+    Transfers& s = l.transfers;
     int const units = compute_units_of_current_device();
     l.grid = group_grid(width, height, int(kStagingThreads));
     bool const stage = readsHalves && l.grid.tiles >= kTilesPerStaging * units;
-    for (int c = 0; c < 8; ++c) {
-        s.pair[c] = c < channels ? int8_t(transfer_pair(src[c], dst[c])) : int8_t(-1);
-        if (s.pair[c] < 0 || !stage) continue;
-        for (int k = 0; k < s.count; ++k) if (s.staged[k] == s.pair[c]) s.slot[c] = int8_t(k + 1);
-        if (s.slot[c] == 0 && s.count < 2) { s.staged[s.count] = s.pair[c]; s.slot[c] = int8_t(++s.count); }
+    for (int c = 0; c < channels; ++c) {
+        int const pair = transfer_pair(src[c], dst[c]);
+        s.set(c, pair, pair >= 0 && stage ? s.stage(pair) : 0);
     }
-    if (s.count) {
+    if (s.count()) {
         int const share = (l.grid.tiles + kTilesPerStaging - 1) / kTilesPerStaging;
         l.threads = kStagingThreads;
         l.grid.step = 2 * units < share ? 2 * units : share;
-        l.ldsBytes = unsigned(s.count * kStageStride * sizeof(float));
+        l.ldsBytes = unsigned(s.count() * kStageStride * sizeof(float));
     } else {
         l.grid = group_grid(width, height, kSmallThreads);
         l.threads = kSmallThreads;
+        int const resident = 8 * units;                      // then a workgroup's next pixels are under way while it works
+        if (l.grid.step > resident) l.grid.step = resident;
     }
     return l;
 }
@@ -424,16 +464,16 @@ static GroupLaunch plan_groups(int width, int height, uint8_t const* src, uint8_
 // Copies them: workgroups of kStagingThreads, 16 bytes a load and all loads in flight before the first is stored.  (A loop of
 // dword loads, each waited for before the next, was a chain of six or twelve trips to the L2 in front of every launch's
 // pixels: 2048 x 2048, sRGB dithered 19.6 us, HLG halves written 15.5, the 2 : 1 reduction 34.)
-__device__ __forceinline__ void copy_staged(StagedTransfers const& s, float* lds)
+__device__ __forceinline__ void copy_staged(Transfers const& s, float* lds)
 {
-    if (s.count == 0) return;
+    if (s.count() == 0) return;
     constexpr uint32_t VECTORS = kStageCount / 4, STEPS = (VECTORS + kStagingThreads - 1) / kStagingThreads;
     static_assert(kStageCount == 4 * VECTORS + 1, "the table's end is 1");
     float4 v[2][STEPS];
     float last[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {                            // (one table twice if there is one)
-        float const* const from = &transferOfHalf[k < s.count ? s.staged[k] : s.staged[0]][kStageFirst];
+        float const* const from = &transferOfHalf[k < s.count() ? s.staged(k) : s.staged(0)][kStageFirst];
 #pragma unroll
         for (uint32_t i = 0; i < STEPS; ++i) v[k][i] = reinterpret_cast<float4 const*>(from)[min(threadIdx.x + i * kStagingThreads, VECTORS - 1u)];
         last[k] = from[kStageCount - 1u];
@@ -447,7 +487,7 @@ __device__ __forceinline__ void copy_staged(StagedTransfers const& s, float* lds
     }
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-        if (k >= s.count) continue;
+        if (k >= s.count()) continue;
         float* const to = lds + k * int(kStageStride);
 #pragma unroll
         for (uint32_t i = 0; i < STEPS; ++i)
@@ -464,12 +504,25 @@ struct GroupsArgs {
     uint64_t rowPitch;
     int32_t width, height;
     GroupGrid grid;
-    StagedTransfers transfers;
+    Transfers transfers;
     uint8_t setChannels, firstChannel, channels;             // channels: copied ones
     uint8_t fillSpace;                                       // read: the destination's colour space of a fourth channel the set does not have
-    uint8_t verticalFlip;                                    // write
+    uint32_t verticalFlip;                                   // write
 };
 static_assert(sizeof(GroupsArgs) <= 128, "");
+
+// Where a lane works in a tile: the first of its four pixels.
+struct GroupPlace {
+    GroupGrid const& grid;
+    int lx, ly;
+    __device__ __forceinline__ explicit GroupPlace(GroupsArgs const& a)
+        : grid(a.grid), lx(int(threadIdx.x) & ((1 << a.grid.log2LanesX) - 1)), ly(int(threadIdx.x) >> a.grid.log2LanesX) {}
+    __device__ __forceinline__ void of_tile(int tile, int& x, int& y) const
+    {
+        int const tileY = grid.row_of(tile), tileX = tile - tileY * grid.tilesX;
+        x = ((tileX << grid.log2LanesX) + lx) * 4; y = (tileY << grid.log2Rows) + ly;
+    }
+};
 
 // CHANNELS = channels of a destination pixel.
 template <int FORMAT, int CHANNELS, bool DITHER>
@@ -479,31 +532,48 @@ read_groups_kernel(GroupsArgs a)
     constexpr int BPC = bytes_per_channel(FORMAT), PIXEL = CHANNELS * BPC, PAIRS = CHANNELS / 2 + 1;
     static_assert(PIXEL <= 8, "the words of four pixels stay in registers");
     extern __shared__ float staged[];
-    uint32_t const threads = 1u << (a.grid.log2LanesX + a.grid.log2Rows);
-    copy_staged(a.transfers, staged);
-    int const lanesX = 1 << a.grid.log2LanesX;
-    int const lx = int(threadIdx.x) & (lanesX - 1), ly = int(threadIdx.x) >> a.grid.log2LanesX;
+    GroupPlace const place(a);
     int const firstPair = a.firstChannel >> 1;
     bool const odd = (a.firstChannel & 1) != 0;
     int const copied = min(int(a.channels), CHANNELS);
     int const pairs = ((a.firstChannel + copied + 1) >> 1) - firstPair;      // at most PAIRS
+    auto const pair_at = [&](int x, int y, int p) {
+        return reinterpret_cast<uint32_t const*>(a.planar + size_t(y) * size_t(a.width) * size_t(a.setChannels) + size_t(2 * (firstPair + min(p, pairs - 1))) * size_t(a.width) + size_t(x) * 2);
+    };
+    // (four pixels of the row wherever the lane's group lies; a group that the row cuts off is read again)
+    u32x4_a4 ahead[PAIRS];
+    auto const load = [&](int tile) {
+        int x, y;
+        place.of_tile(tile, x, y);
+        if (a.width < 4) return;                             // uniform
+#pragma unroll
+        for (int p = 0; p < PAIRS; ++p) ahead[p] = *reinterpret_cast<u32x4_a4 const*>(pair_at(min(x, a.width - 4), min(y, a.height - 1), p));
+    };
+    load(blockIdx.x);
+    copy_staged(a.transfers, staged);
     for (int tile = blockIdx.x; tile < a.grid.tiles; tile += a.grid.step) {
-        int const tileY = tile / a.grid.tilesX, tileX = tile - tileY * a.grid.tilesX;
-        int const x = (tileX * lanesX + lx) * 4, y = (tileY << a.grid.log2Rows) + ly;
-        if (x >= a.width || y >= a.height) continue;
-        bool const whole = x + 4 <= a.width;
-        uint16_t const* const src = a.planar + size_t(y) * size_t(a.width) * size_t(a.setChannels) + size_t(x) * 2;
         uint32_t pr[PAIRS][4];
 #pragma unroll
-        for (int p = 0; p < PAIRS; ++p) {
-            uint32_t const* const from = reinterpret_cast<uint32_t const*>(src + size_t(2 * (firstPair + min(p, pairs - 1))) * size_t(a.width));
-            if (whole) {
-                u32x4_a4 const v = *reinterpret_cast<u32x4_a4 const*>(from);
-                pr[p][0] = v[0]; pr[p][1] = v[1]; pr[p][2] = v[2]; pr[p][3] = v[3];
-            } else {
+        for (int p = 0; p < PAIRS; ++p)
 #pragma unroll
-                for (int k = 0; k < 4; ++k) pr[p][k] = from[min(k, a.width - 1 - x)];
-            }
+            for (int k = 0; k < 4; ++k) pr[p][k] = ahead[p][k];
+        if (tile + a.grid.step < a.grid.tiles) load(tile + a.grid.step);     // uniform
+        int x, y;
+        place.of_tile(tile, x, y);
+        if (x >= a.width || y >= a.height) continue;
+        // (what the channels' bits say is found out here again: kept from before the loop it is thirty spilled registers)
+        Transfers transfers = a.transfers;
+        asm volatile("" : "+s"(transfers.pairs), "+s"(transfers.rest));
+        bool const whole = x + 4 <= a.width;
+        if (!whole) {
+#pragma unroll
+            for (int p = 0; p < PAIRS; ++p)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) pr[p][k] = pair_at(x, y, p)[min(k, a.width - 1 - x)];
+#pragma unroll
+            for (int p = 0; p < PAIRS; ++p)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) asm volatile("" : "+v"(pr[p][k]));           // (waited for here)
         }
         uint32_t words[PIXEL];                               // four pixels
 #pragma unroll
@@ -527,7 +597,7 @@ read_groups_kernel(GroupsArgs a)
                     uint32_t const next = (ch & 1) ? pr[(ch >> 1) + 1][k] & 0xffffu : pr[ch >> 1][k] >> 16;
                     bits[k] = odd ? next : even;
                 }
-                transfer_halves(staged, a.transfers.slot[ch], a.transfers.pair[ch], bits, value);
+                transfer_halves(staged, transfers.slot(ch), transfers.pair(ch), bits, value);
             } else {                                         // GetDefaultChannelValue; 0 is 0 in every colour space
                 float const fill = (ch == 3) ? transfer_half(transfer_pair(0, a.fillSpace), 0x3C00u) : 0.f;
 #pragma unroll
@@ -536,27 +606,30 @@ read_groups_kernel(GroupsArgs a)
         }
 #pragma unroll
         for (int ch = 0; ch < CHANNELS; ++ch) {
-            uint32_t bits[4];
             // A filled channel whose code is the same for the least and the greatest draw has it for all between them, and
             // its draws, of which each is a seventh of a pixel's work, need not be made.
-            bool drawn = DITHER;                             // uniform
             if (DITHER && ch >= copied) {
-                bits[0] = encode_value<FORMAT>(values[ch][0], true, -0.5f);
-                bits[1] = encode_value<FORMAT>(values[ch][0], true, 0.5f - 0x1p-23f);
-                drawn = __builtin_amdgcn_readfirstlane(bits[0] ^ bits[1]) != 0u;
-                bits[1] = bits[2] = bits[3] = bits[0];
-            }
-            if (drawn) {
+                uint32_t const least = encode_value<FORMAT>(values[ch][0], true, -0.5f), greatest = encode_value<FORMAT>(values[ch][0], true, 0.5f - 0x1p-23f);
+                if (__builtin_amdgcn_readfirstlane(least ^ greatest) == 0u) {    // uniform
 #pragma unroll
-                for (int k = 0; k < 4; ++k) bits[k] = encode_value<FORMAT>(values[ch][k], true, rng[k].offset(ch));
-            } else if (!DITHER) {
-#pragma unroll
-                for (int k = 0; k < 4; ++k) bits[k] = encode_value<FORMAT>(values[ch][k], false, 0.f);
+                    for (int k = 0; k < 4; ++k) {
+                        int const at = k * PIXEL + ch * BPC; // byte of the group
+                        words[at >> 2] |= least << (8 * (at & 3));
+                    }
+                    continue;
+                }
             }
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                int const at = k * PIXEL + ch * BPC;         // byte of the group
-                words[at >> 2] |= BPC == 4 ? bits[k] : bits[k] << (8 * (at & 3));
+                int const at = k * PIXEL + ch * BPC;
+                float value = values[ch][k];
+                if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_UNORM8) {
+                    if constexpr (DITHER) value += divide_by_top(rng[k].offset(ch), 255.f, 1.f / 255.f);
+                    words[at >> 2] = put_unorm8(value * 255.f, at & 3, words[at >> 2]);
+                } else {
+                    uint32_t const bits = encode_value<FORMAT>(value, DITHER, DITHER ? rng[k].offset(ch) : 0.f);
+                    words[at >> 2] |= BPC == 4 ? bits : bits << (8 * (at & 3));
+                }
             }
         }
         uint8_t* const out = a.image + size_t(y) * a.rowPitch + size_t(x) * PIXEL;
@@ -601,7 +674,7 @@ __device__ __forceinline__ uint32_t stored_half_of(uint32_t bits, int pair)
     if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_UNORM8) {
         return storedOfUnorm8[pair < 0 ? kTransferPairs : pair][bits & 0xffu];
     } else if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_UNORM16) {
-        return pair < 0 ? stored_half(divide_by_top(float(bits & 0xffffu), 65535.f, 1.f / 65535.f)) : storedOfUnorm16[pair][bits & 0xffffu];
+        return pair < 0 ? unit_half(divide_by_top(float(bits & 0xffffu), 65535.f, 1.f / 65535.f)) : storedOfUnorm16[pair][bits & 0xffffu];
     } else if constexpr (FORMAT == NTC_HIP_DEV_FORMAT_FLOAT16) {
         return stored_half(transfer_half(pair, bits & 0xffffu));
     } else {
@@ -611,10 +684,12 @@ __device__ __forceinline__ uint32_t stored_half_of(uint32_t bits, int pair)
 }
 
 // Four pixels of at most eight bytes a lane, like read_groups_kernel the other way round: whole dwords of the pixels
-// in, 16 bytes of each complete channel pair out (2048 x 2048 of 8 bits: RGBA with sRGB 14 us, 91 before the tables; two
-// channels in halves of two pairs 13 us, one 10 us, 15 before; HLG halves 18 us, 29 before); where the image has only one channel of a pair, its halves go out
+// in, 16 bytes of each complete channel pair out; where the image has only one channel of a pair, its halves go out
 // one by one between those of the other.  CHANNELS = channels of a source pixel, of which a.numChannels are stored.
-// 8-bit codes become halves through a table in LDS, a row of 256 per channel.
+// 8-bit codes of linear channels become halves by a product, others through a table in LDS, a row of 256 per channel.
+// Bound by memory, and by the start and end of a launch where there is little of it: 2048 x 2048 of 8 bits, RGBA with sRGB
+// 11.0 us (its bytes take 7), two channels in halves of two pairs 10.5 (4), one 7.8 (2), HLG halves 14.9 (10); one pixel a
+// lane took 91, 15 (one channel) and 29, tables filled before the first pixels were asked for 11.9, 11.5, 7.9 and 15.5.
 template <int FORMAT, int CHANNELS>
 __global__ void __launch_bounds__(1024, 8)
 write_groups_kernel(GroupsArgs a)
@@ -624,38 +699,53 @@ write_groups_kernel(GroupsArgs a)
     static_assert(PIXEL <= 8, "the words of four pixels stay in registers");
     __shared__ uint16_t codes[CODES ? CHANNELS : 1][256];
     extern __shared__ float staged[];
-    uint32_t const threads = 1u << (a.grid.log2LanesX + a.grid.log2Rows);
-    if constexpr (CODES) {
-        for (uint32_t i = threadIdx.x; i < CHANNELS * 256u; i += threads) {
-            int const ch = int(i >> 8), pair = a.transfers.pair[ch];
-            codes[ch][i & 255] = storedOfUnorm8[pair < 0 ? kTransferPairs : pair][i & 255];
+    GroupPlace const place(a);
+    int const lx = place.lx, odd = a.firstChannel & 1;
+    auto const pixel_at = [&](int x, int y) { return a.image + size_t(a.verticalFlip ? a.height - 1 - y : y) * a.rowPitch + size_t(x) * PIXEL; };
+    constexpr int FOURS = PIXEL & ~3, TWOS = FOURS + (PIXEL & 2);
+    // (four pixels of the row wherever the lane's group lies; a group that the row cuts off is read again)
+    uint32_t ahead[PIXEL];
+    auto const load = [&](int tile) {
+        int x, y;
+        place.of_tile(tile, x, y);
+        if (a.width < 4) return;                             // uniform
+        uint8_t const* const in = pixel_at(min(x, a.width - 4), min(y, a.height - 1));
+#pragma unroll
+        for (int w = 0; w < FOURS; w += 4) {
+            u32x4_any const v = *reinterpret_cast<u32x4_any const*>(in + 4 * w);
+            ahead[w] = v[0]; ahead[w + 1] = v[1]; ahead[w + 2] = v[2]; ahead[w + 3] = v[3];
         }
-        __syncthreads();
+        if constexpr ((PIXEL & 2) != 0) {
+            u32x2_any const v = *reinterpret_cast<u32x2_any const*>(in + 4 * FOURS);
+            ahead[FOURS] = v[0]; ahead[FOURS + 1] = v[1];
+        }
+        if constexpr ((PIXEL & 1) != 0) ahead[TWOS] = *reinterpret_cast<u32_any const*>(in + 4 * TWOS);
+    };
+    load(blockIdx.x);
+    if constexpr (CODES) {
+        // (256 threads; the tables' loads are all in flight before the first is stored)
+        if (a.transfers.pairs != 0u) {                       // uniform
+            uint32_t code[CHANNELS];
+#pragma unroll
+            for (int ch = 0; ch < CHANNELS; ++ch) code[ch] = storedOfUnorm8[max(a.transfers.pair(ch), 0)][threadIdx.x & 255u];
+#pragma unroll
+            for (int ch = 0; ch < CHANNELS; ++ch) codes[ch][threadIdx.x & 255u] = uint16_t(code[ch]);
+            __syncthreads();
+        }
     }
     if constexpr (HALVES) copy_staged(a.transfers, staged);
-    int const lanesX = 1 << a.grid.log2LanesX;
-    int const lx = int(threadIdx.x) & (lanesX - 1), ly = int(threadIdx.x) >> a.grid.log2LanesX;
-    int const odd = a.firstChannel & 1;
     for (int tile = blockIdx.x; tile < a.grid.tiles; tile += a.grid.step) {
-        int const tileY = tile / a.grid.tilesX, tileX = tile - tileY * a.grid.tilesX;
-        int const x = (tileX * lanesX + lx) * 4, y = (tileY << a.grid.log2Rows) + ly;
-        if (y >= a.height) continue;                         // (uniform across a wave that covers one row)
-        bool const whole = x + 4 <= a.width;
-        uint8_t const* const in = a.image + size_t(a.verticalFlip ? a.height - 1 - y : y) * a.rowPitch + size_t(x) * PIXEL;
         uint32_t words[PIXEL];
-        if (whole) {
-            constexpr int FOURS = PIXEL & ~3, TWOS = FOURS + (PIXEL & 2);
 #pragma unroll
-            for (int w = 0; w < FOURS; w += 4) {
-                u32x4_any const v = *reinterpret_cast<u32x4_any const*>(in + 4 * w);
-                words[w] = v[0]; words[w + 1] = v[1]; words[w + 2] = v[2]; words[w + 3] = v[3];
-            }
-            if constexpr ((PIXEL & 2) != 0) {
-                u32x2_any const v = *reinterpret_cast<u32x2_any const*>(in + 4 * FOURS);
-                words[FOURS] = v[0]; words[FOURS + 1] = v[1];
-            }
-            if constexpr ((PIXEL & 1) != 0) words[TWOS] = *reinterpret_cast<u32_any const*>(in + 4 * TWOS);
-        } else {
+        for (int w = 0; w < PIXEL; ++w) words[w] = ahead[w];
+        if (tile + a.grid.step < a.grid.tiles) load(tile + a.grid.step);     // uniform
+        int x, y;
+        place.of_tile(tile, x, y);
+        if (y >= a.height) continue;                         // (uniform across a wave that covers one row)
+        int const tileX = (x >> 2) >> a.grid.log2LanesX;
+        bool const whole = x + 4 <= a.width;
+        if (!whole) {
+            uint8_t const* const in = pixel_at(x, y);
 #pragma unroll
             for (int w = 0; w < PIXEL; ++w) words[w] = 0u;
 #pragma unroll
@@ -665,6 +755,8 @@ write_groups_kernel(GroupsArgs a)
                 else if constexpr (BPC == 2) words[b >> 2] |= uint32_t(*reinterpret_cast<uint16_t const*>(in + b)) << (8 * (b & 3));
                 else                         words[b >> 2] = *reinterpret_cast<uint32_t const*>(in + b);
             }
+#pragma unroll
+            for (int w = 0; w < PIXEL; ++w) asm volatile("" : "+v"(words[w]));           // (waited for here)
         }
         uint32_t half[CHANNELS][4];
 #pragma unroll
@@ -678,16 +770,21 @@ write_groups_kernel(GroupsArgs a)
                 if constexpr (BPC == 2) bits[k] &= 0xffffu;
             }
             if constexpr (CODES) {
+                if (a.transfers.pair(ch) < 0) {              // uniform
 #pragma unroll
-                for (int k = 0; k < 4; ++k) half[ch][k] = codes[ch][bits[k]];
+                    for (int k = 0; k < 4; ++k) half[ch][k] = unit_half(divide_by_top(float(bits[k]), 255.f, 1.f / 255.f));
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) half[ch][k] = codes[ch][bits[k]];
+                }
             } else if constexpr (HALVES) {
                 float value[4];
-                transfer_halves(staged, a.transfers.slot[ch], a.transfers.pair[ch], bits, value);
+                transfer_halves(staged, a.transfers.slot(ch), a.transfers.pair(ch), bits, value);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) half[ch][k] = stored_half(value[k]);
             } else {
 #pragma unroll
-                for (int k = 0; k < 4; ++k) half[ch][k] = stored_half_of<FORMAT>(bits[k], a.transfers.pair[ch]);
+                for (int k = 0; k < 4; ++k) half[ch][k] = stored_half_of<FORMAT>(bits[k], a.transfers.pair(ch));
             }
         }
         uint16_t* const dst = a.planar + size_t(y) * size_t(a.width) * size_t(a.setChannels) + size_t(x) * 2;
@@ -912,11 +1009,9 @@ struct ResizePlanarArgs {
     int32_t srcWidth, srcHeight, dstWidth, dstHeight, setChannels;
     int32_t tilesX, tiles, pairsPerLane;                     // tiles of 64 pixels x a row per wave
     int32_t step, threads;                                   // workgroups in x, threads of each
-    StagedTransfers transfers;                               // of the decoding pairs
-    uint32_t spaces;                                         // two bits a channel; (an array indexed by a loop's variable would be
-    uint32_t slots;                                          // a load from memory each time); per space: the copy that holds its pair
-    __device__ __forceinline__ int space(int channel) const { return int(spaces >> (2 * channel)) & 3; }
-    __device__ __forceinline__ int slot(int space) const { return int(slots >> (2 * space)) & 3; }
+    Transfers transfers;                                     // of the decoding pairs; those of the colour spaces in the place of channels
+    uint32_t spaces;                                         // two bits a channel
+    __host__ __device__ __forceinline__ int space(int channel) const { return int(spaces >> (2 * channel)) & 3; }
 };
 
 template <bool LINEAR>
@@ -965,7 +1060,7 @@ resize_planar_kernel(ResizePlanarArgs a)
                     uint32_t const bits[4] = { (v00 >> (16 * k)) & 0xffffu, (v10 >> (16 * k)) & 0xffffu, (v01 >> (16 * k)) & 0xffffu, (v11 >> (16 * k)) & 0xffffu };
                     float v[4];
                     if constexpr (LINEAR) transfer_halves(staged, 0, -1, bits, v);
-                    else                  transfer_halves(staged, a.slot(space), transfer_pair(space, 0), bits, v);
+                    else                  transfer_halves(staged, a.transfers.slot(space), a.transfers.pair(space), bits, v);
                     packed |= encoded_half(space, blend_taps<ALL>(t, v[0], v[1], v[2], v[3])) << (16 * k);
                 }
                 out[size_t(p) * size_t(a.dstWidth)] = packed;
@@ -1031,7 +1126,7 @@ halve_planar_kernel(ResizePlanarArgs a)
                                                (lower[2 * i] >> (16 * k)) & 0xffffu, (lower[2 * i + 1] >> (16 * k)) & 0xffffu };
                     float v[4];
                     if constexpr (LINEAR) transfer_halves(staged, 0, -1, bits, v);
-                    else                  transfer_halves(staged, a.slot(space), transfer_pair(space, 0), bits, v);
+                    else                  transfer_halves(staged, a.transfers.slot(space), a.transfers.pair(space), bits, v);
                     packed[i] |= encoded_half(space, blend_taps<true>(i ? t1 : t0, v[0], v[1], v[2], v[3])) << (16 * k);
                 }
             }
@@ -1064,10 +1159,9 @@ hipError_t launch_resize_planar(uint16_t const* src, int srcWidth, int srcHeight
     bool const stage = !linear && a.tiles * tileWidth >= 128 * units;            // as in plan_groups: each copy serves two pixels a thread or more
     for (int space = 1; space <= 2; ++space) {
         bool used = false;
-        for (int i = 0; i < setChannels; ++i) used = used || ((a.spaces >> (2 * i)) & 3u) == uint32_t(space);
-        if (!stage || !used) continue;
-        a.transfers.staged[a.transfers.count] = int8_t(transfer_pair(space, 0));
-        a.slots |= uint32_t(++a.transfers.count) << (2 * space);
+        for (int i = 0; i < setChannels; ++i) used = used || a.space(i) == space;
+        int const pair = transfer_pair(space, 0);
+        a.transfers.set(space, pair, stage && used ? a.transfers.stage(pair) : 0);
     }
     dim3 grid(1);
     a.pairsPerLane = pairs;
@@ -1082,7 +1176,7 @@ hipError_t launch_resize_planar(uint16_t const* src, int srcWidth, int srcHeight
         a.pairsPerLane = (pairs + ranges - 1) / ranges;
         grid = dim3(unsigned(a.tiles), unsigned((pairs + a.pairsPerLane - 1) / a.pairsPerLane));
     }
-    size_t const lds = size_t(a.transfers.count) * kStageStride * sizeof(float);
+    size_t const lds = size_t(a.transfers.count()) * kStageStride * sizeof(float);
     a.step = int(grid.x);
     a.threads = threads;
     if (half) return linear ? launch_kernel<halve_planar_kernel<true>>(grid, dim3(threads), lds, stream, a)
@@ -1123,13 +1217,9 @@ static hipError_t launch_write_groups_of(GroupsArgs const& args, int srcChannels
 
 static hipError_t launch_write_groups(WriteChannelsArgs const& a, hipStream_t stream)
 {
-    GroupLaunch plan = plan_groups(a.width, a.height, a.srcColorSpaces, a.dstColorSpaces, a.numChannels, a.format == NTC_HIP_DEV_FORMAT_FLOAT16);
-    if (a.format == NTC_HIP_DEV_FORMAT_UNORM8) {             // a workgroup fills its table once for all of its tiles
-        int const resident = 8 * compute_units_of_current_device();
-        if (plan.grid.step > resident) plan.grid.step = resident;
-    }
+    GroupLaunch const plan = plan_groups(a.width, a.height, a.srcColorSpaces, a.dstColorSpaces, a.numChannels, a.format == NTC_HIP_DEV_FORMAT_FLOAT16);
     GroupsArgs const args{ a.planarPairs, const_cast<uint8_t*>(a.src), a.rowPitch, a.width, a.height, plan.grid, plan.transfers,
-                           uint8_t(a.setChannels), uint8_t(a.firstChannel), uint8_t(a.numChannels), 0, uint8_t(a.verticalFlip != 0) };
+                           uint8_t(a.setChannels), uint8_t(a.firstChannel), uint8_t(a.numChannels), 0, a.verticalFlip != 0 };
     int const channels = int(a.pixelStride) / bytes_per_channel(a.format);
     switch (a.format) {
     case NTC_HIP_DEV_FORMAT_UNORM8:  return launch_write_groups_of<NTC_HIP_DEV_FORMAT_UNORM8>(args, channels, plan, stream);

@@ -72,6 +72,17 @@ template <int TOP> struct DivideByTop {
     }
 };
 
+// put_unorm8(): every float, at a byte of its own choice.
+struct PutUnorm8 {
+    static constexpr uint64_t cases = uint64_t(1) << 32;
+    static __device__ int check(uint64_t i)
+    {
+        float const v = __uint_as_float(uint32_t(i));
+        uint32_t const at = uint32_t(i ^ (i >> 13)) & 3u, others = ~(0xffu << (8u * at));
+        return verdict(put_unorm8(v, at, 0x93a5c7e1u & others) == ((0x93a5c7e1u & others) | unorm_code(v, 255.f) << (8u * at)));
+    }
+};
+
 #elif defined(SUBJECT_BC)
 
 // code_quotient(): five and six bits.
@@ -187,6 +198,7 @@ extern "C" {
 #if defined(SUBJECT_COPY)
 int exact_encoded_half_srgb(Report* r) { return sweep<EncodedHalf<1>>(r); }
 int exact_encoded_half_hlg(Report* r) { return sweep<EncodedHalf<2>>(r); }
+int exact_put_unorm8(Report* r) { return sweep<PutUnorm8>(r); }
 int exact_divide_by_255(Report* r) { return sweep<DivideByTop<255>>(r); }
 int exact_divide_by_65535(Report* r) { return sweep<DivideByTop<65535>>(r); }
 #elif defined(SUBJECT_BC)

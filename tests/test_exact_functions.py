@@ -18,7 +18,7 @@ class Report(C.Structure):
 
 @pytest.mark.parametrize("subject,function,cases", [
     ("copy", "encoded_half_srgb", 1 << 32), ("copy", "encoded_half_hlg", 1 << 32),
-    ("copy", "divide_by_255", (1 << 23) + 256), ("copy", "divide_by_65535", (1 << 23) + 65536),
+    ("copy", "put_unorm8", 1 << 32), ("copy", "divide_by_255", (1 << 23) + 256), ("copy", "divide_by_65535", (1 << 23) + 65536),
     ("bc", "code_quotient", 96), ("bc", "bc4_palette", 65536),
     ("bc6", "quotient_of_integers", (1 << 17) * ((1 << 17) - 1)), ("bc6", "quotient_of_log2", None),
     ("bc6", "quotient_of_msle", 0x7c00 * (0x7c00 + 256 + 65536 + 65505)), ("bc6", "quotient_of_codes", 3 * 65536 + 64),
