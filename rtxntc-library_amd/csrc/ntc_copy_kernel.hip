@@ -1259,14 +1259,12 @@ hipError_t launch_write_channels(WriteChannelsArgs const& args, hipStream_t stre
 
 // Per-channel sum of squared differences between a decoded mip and its reference image, both in the
 // internal layout: the loss branch of InferenceKernel (src/Inference.cu:77-118) as a pass of its own.
-// MASKED (maskChannel >= 0): the decoded mask channel is first clamped to [0, 1] and stored back
+// With a mask channel (maskChannel >= 0) the decoded mask channel is first clamped to [0, 1] and stored back
 // clamped (Inference.cu:96-97,112; a negative zero becomes +0 as the device max() of the reference
 // returns), and with discardMaskedOut a texel whose REFERENCE mask value is zero counts on the mask
 // channel only (Inference.cu:80-84,107-108).
-// A lane takes PX adjacent texels (2 when the width is even: 8-byte loads) of rowsPerWave rows; all
-// loads of a row are issued before its arithmetic.  Squares are fp32 as in the reference; their sum over the
-// lane's texels of a row goes into a double accumulator, and the workgroup writes 16 double partial sums;
-// ReduceLoss likewise finishes in double (src/Optimizer.cu:382-387).
+// Squares are fp32 as in the reference; the sum of two texels' goes into a double accumulator, and the
+// workgroup writes 16 double partial sums; ReduceLoss likewise finishes in double (src/Optimizer.cu:382-387).
 //
 // The same launch finishes the sum and hands it to the host (a second kernel, a copy and a stream synchronisation made
 // most of the 28 us a call on 64 x 64 texels took).  Workgroups form at most kLossRows groups; the last one of a group
@@ -1327,15 +1325,151 @@ __device__ __forceinline__ double add_from_row(double v)
     return v + __builtin_bit_cast(double, uint64_t(high) << 32 | low);
 }
 
-template <int PX, bool MASKED>
-__global__ void __launch_bounds__(256)
-image_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int width, int height, int setChannels, int rowsPerWave,
-                  uint32_t validChannelMask, int maskChannel, int discardMaskedOut, uint32_t gridX, uint32_t blocks, uint32_t groupSize, LossWorkspace work)
+// A workgroup's sums, channel threadIdx.x's in `mine` of the threads 0 ... 15, on their way to the host.
+__device__ __forceinline__ void hand_over_sums(double mine, uint32_t validChannelMask, uint32_t block, uint32_t blocks, uint32_t groupSize, LossWorkspace const& work)
 {
-    constexpr int PAIRS = NTC_HIP_DEV_MAX_CHANNELS / 2;
+    if (!((validChannelMask >> (threadIdx.x & 31u)) & 1u)) mine = 0.0;
+    uint32_t const group = block / groupSize, first = group * groupSize, members = min(groupSize, blocks - first);
+    double total = mine;                                     // threads 0 ... 15: a channel's each
+    if (members > 1) {
+        __shared__ double scratch[16][NTC_HIP_DEV_MAX_CHANNELS];
+        __shared__ int last;
+        if (threadIdx.x < NTC_HIP_DEV_MAX_CHANNELS) publish(work.partials + size_t(block) * NTC_HIP_DEV_MAX_CHANNELS + threadIdx.x, mine);
+        if (!arrived_last(work.counters + group * kLossCounterStride, members, last)) return;
+        total = sum_entries(work.partials + size_t(first) * NTC_HIP_DEV_MAX_CHANNELS, int(members), scratch);
+    }
+    // To the host in one trip: each half of a double is stored together with the serial number, so that every word
+    // says for itself whether it has arrived.  Stores of system scope go past the caches.  (Plain stores and a release
+    // behind them write back the die's whole L2.)
+    if (threadIdx.x >= 64) return;
+    int const lane = int(threadIdx.x);
+    uint64_t const sum = __builtin_bit_cast(uint64_t, __shfl(total, lane >> 1, 64));
+    uint64_t const word = uint64_t(work.serial) << 32 | ((lane & 1) ? sum >> 32 : sum & 0xffffffffu);
+    if (lane < 2 * NTC_HIP_DEV_MAX_CHANNELS)
+        __hip_atomic_store(&work.rows[group].words[lane], word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Squared differences of two texels' first or second halves (SHIFT = 0, 16), added up.
+template <int SHIFT> __device__ __forceinline__ float two_squares(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1)
+{
+    auto const half = [](uint32_t w) { return float(__builtin_bit_cast(_Float16, uint16_t(w >> SHIFT))); };
+    float const d0 = half(a0) - half(b0), d1 = half(a1) - half(b1);
+    float s = 0.f;
+    s += d0 * d0;
+    s += d1 * d1;
+    return s;
+}
+
+// The sums of 256 lanes' 16 accumulators, channel threadIdx.x's in the threads 0 ... 15: 16 threads per channel add 16 of its
+// 256 values each, then each other's.  (With exchanges between lanes, 17 of a double and 1500 instructions when every lane
+// hands over half of what it holds at a step, this took 1 us longer.)
+__device__ __forceinline__ double sum_of_lanes(double const (&acc)[NTC_HIP_DEV_MAX_CHANNELS], int setChannels)
+{
     constexpr int STRIDE = 256 + 16;                         // (channels half the banks apart)
     __shared__ double lanes[NTC_HIP_DEV_MAX_CHANNELS * STRIDE];
     __shared__ double sums[NTC_HIP_DEV_MAX_CHANNELS];
+#pragma unroll
+    for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) lanes[c * STRIDE + int(threadIdx.x)] = acc[c];
+    __syncthreads();
+    int const channel = int(threadIdx.x) >> 4, part = int(threadIdx.x) & 15;
+    double mine = 0.0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) mine += lanes[channel * STRIDE + part + 16 * k];
+    mine = add_from_row<0xB1>(mine);                         // quad_perm: the neighbour,
+    mine = add_from_row<0x4E>(mine);                         // the other pair,
+    mine = add_from_row<0x141>(mine);                        // row_half_mirror: the other quad,
+    mine = add_from_row<0x140>(mine);                        // row_mirror: the other eight
+    if (part == 0) sums[channel] = channel < setChannels ? mine : 0.0;
+    __syncthreads();
+    return sums[threadIdx.x & (NTC_HIP_DEV_MAX_CHANNELS - 1)];
+}
+
+// Without a mask channel.  The internal layout is row after row of channel pairs, so that whole rows are one piece of memory,
+// which the workgroup goes through in order, 4 KB of each image a load; STEPS of a pair's row and PAIRS pairs are under way
+// together, eight loads a lane (sixteen do not leave the registers for four waves per SIMD).  Bound by memory for large
+// mips, by the launch and the way to the host for small ones.  Whole calls of 16 channels, 4096 x 4096, 2048 x 2048, 1024 x
+// 1024 and 512 x 512: 189, 51, 23 and 16.5 us; 197, 56, 29 and 18.5 with 8-byte loads of all pairs by lanes of two texels,
+// and the groups' counters on one line (6 channels: 80, 28, 16.5 and 15.5; 111, 37, 25 and 18); 209, 51, 30 and 26 with a
+// wave for each pair, whose rows lie a power of two apart.  A kernel that does nothing but read the two images of 16
+// channels takes 172, 38 and 10 for the first three, a call of nothing 11.
+template <int STEPS, int PAIRS>
+__global__ void __launch_bounds__(256, 4)
+image_loss_kernel(uint16_t const* __restrict__ a, uint16_t const* __restrict__ b, int width, int height, int setChannels, int rowsPerWorkgroup, int log2Lanes,
+                  uint32_t validChannelMask, uint32_t blocks, uint32_t groupSize, LossWorkspace work)
+{
+    constexpr int MAX_PAIRS = NTC_HIP_DEV_MAX_CHANNELS / 2;
+    int const pairs = setChannels >> 1, stride = 4 << log2Lanes, first = (int(threadIdx.x) & ((1 << log2Lanes) - 1)) * 4;
+    double acc[NTC_HIP_DEV_MAX_CHANNELS];
+#pragma unroll
+    for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) acc[c] = 0.0;
+    auto const add = [&](int p, u32x4_a4 const& va, u32x4_a4 const& vb) {
+        acc[2 * p] += double(two_squares<0>(va[0], va[1], vb[0], vb[1]));
+        acc[2 * p + 1] += double(two_squares<16>(va[0], va[1], vb[0], vb[1]));
+        acc[2 * p] += double(two_squares<0>(va[2], va[3], vb[2], vb[3]));
+        acc[2 * p + 1] += double(two_squares<16>(va[2], va[3], vb[2], vb[3]));
+    };
+    int const begin = int(blockIdx.x) * rowsPerWorkgroup, end = min(height, begin + rowsPerWorkgroup);
+    // (addresses: the workgroup's rows, the pair and the step in scalar registers, the lane's place in 32 bits)
+    size_t const rows = size_t(begin) * size_t(setChannels) * size_t(width);
+    char const* const ra = reinterpret_cast<char const*>(a + rows);
+    char const* const rb = reinterpret_cast<char const*>(b + rows);
+    for (int y = begin + (int(threadIdx.x) >> log2Lanes); y < end; y += 256 >> log2Lanes) {
+        uint32_t const row = uint32_t(y - begin) * uint32_t(pairs) * uint32_t(width) * 4u;
+#pragma unroll
+        for (int p0 = 0; p0 < MAX_PAIRS; p0 += PAIRS) {
+            if (p0 >= pairs) break;                          // uniform
+            size_t offset[PAIRS];                            // (no branch around a load: pairs that the set does not have read its last one again, and their sums are dropped)
+#pragma unroll
+            for (int p = 0; p < PAIRS; ++p) offset[p] = size_t(min(p0 + p, pairs - 1)) * size_t(width) * 4u;
+            int x = first;
+            for (; x + (STEPS - 1) * stride + 4 <= width; x += STEPS * stride) {
+                uint32_t const lane = row + uint32_t(x) * 4u;
+                u32x4_a4 va[PAIRS][STEPS], vb[PAIRS][STEPS];
+#pragma unroll
+                for (int p = 0; p < PAIRS; ++p)
+#pragma unroll
+                    for (int k = 0; k < STEPS; ++k) {
+                        va[p][k] = *reinterpret_cast<u32x4_a4 const*>(ra + offset[p] + size_t(k) * size_t(stride) * 4u + lane);
+                        vb[p][k] = *reinterpret_cast<u32x4_a4 const*>(rb + offset[p] + size_t(k) * size_t(stride) * 4u + lane);
+                    }
+                __builtin_amdgcn_sched_barrier(0);           // keep the loads ahead of the arithmetic
+#pragma unroll
+                for (int p = 0; p < PAIRS; ++p)
+#pragma unroll
+                    for (int k = 0; k < STEPS; ++k) add(p0 + p, va[p][k], vb[p][k]);
+            }
+#pragma unroll 1
+            for (; x < width; x += stride) {                 // what is left of the row, its last one to three texels alone
+                uint32_t const lane = row + uint32_t(x) * 4u;
+#pragma unroll
+                for (int p = 0; p < PAIRS; ++p) {
+                    char const* const la = ra + offset[p] + lane;
+                    char const* const lb = rb + offset[p] + lane;
+                    u32x4_a4 va{}, vb{};
+                    if (x + 4 <= width) {
+                        va = *reinterpret_cast<u32x4_a4 const*>(la);
+                        vb = *reinterpret_cast<u32x4_a4 const*>(lb);
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) if (x + k < width) { va[k] = reinterpret_cast<uint32_t const*>(la)[k]; vb[k] = reinterpret_cast<uint32_t const*>(lb)[k]; }
+                    }
+                    add(p0 + p, va, vb);
+                }
+            }
+        }
+    }
+    hand_over_sums(sum_of_lanes(acc, setChannels), validChannelMask, blockIdx.x, blocks, groupSize, work);
+}
+
+// With a mask channel, or (maskChannel < 0) for images that the other kernel does not take.  A lane takes PX adjacent texels
+// (2 when the width is even: 8-byte loads) of rowsPerWave rows, all pairs of them together, because every channel counts by the mask's, and all
+// loads of a row are issued before its arithmetic.
+template <int PX>
+__global__ void __launch_bounds__(256)
+masked_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int width, int height, int setChannels, int rowsPerWave,
+                   uint32_t validChannelMask, int maskChannel, int discardMaskedOut, uint32_t gridX, uint32_t blocks, uint32_t groupSize, LossWorkspace work)
+{
+    constexpr int PAIRS = NTC_HIP_DEV_MAX_CHANNELS / 2;
     int const lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int const x = (blockIdx.x * 64 + lane) * PX;
     int const pairs = setChannels >> 1;
@@ -1361,16 +1495,14 @@ image_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int 
             }
         }
         __builtin_amdgcn_sched_barrier(0);                   // keep the loads ahead of the arithmetic
-        [[maybe_unused]] bool maskedOut[PX];
-        if constexpr (MASKED) {
+        bool maskedOut[PX];
 #pragma unroll
-            for (int k = 0; k < PX; ++k) maskedOut[k] = false;
+        for (int k = 0; k < PX; ++k) maskedOut[k] = false;
 #pragma unroll
-            for (int p = 0; p < PAIRS; ++p) {
-                if ((maskChannel >> 1) != p || !discardMaskedOut) continue;          // uniform
+        for (int p = 0; p < PAIRS; ++p) {
+            if ((maskChannel >> 1) != p || !discardMaskedOut) continue;              // uniform
 #pragma unroll
-                for (int k = 0; k < PX; ++k) maskedOut[k] = (((maskChannel & 1) ? vb[p][k] >> 16 : vb[p][k]) & 0x7FFFu) == 0;
-            }
+            for (int k = 0; k < PX; ++k) maskedOut[k] = (((maskChannel & 1) ? vb[p][k] >> 16 : vb[p][k]) & 0x7FFFu) == 0;
         }
 #pragma unroll
         for (int p = 0; p < PAIRS; ++p) {
@@ -1379,21 +1511,17 @@ image_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int 
             for (int k = 0; k < PX; ++k) {
                 float a0 = float(__builtin_bit_cast(_Float16, uint16_t(va[p][k])));
                 float a1 = float(__builtin_bit_cast(_Float16, uint16_t(va[p][k] >> 16)));
-                if constexpr (MASKED) {
-                    if ((maskChannel >> 1) == p) {              // uniform; the mask channel is below setChannels
-                        if (maskChannel & 1) a1 = a1 > 0.f ? fminf(a1, 1.f) : 0.f;
-                        else                 a0 = a0 > 0.f ? fminf(a0, 1.f) : 0.f;
-                        uint32_t const clamped = uint32_t(__builtin_bit_cast(uint16_t, _Float16(a0)))
-                                               | uint32_t(__builtin_bit_cast(uint16_t, _Float16(a1))) << 16;
-                        if (clamped != va[p][k]) *reinterpret_cast<uint32_t*>(a + base + size_t(2 * p) * size_t(width) + size_t(2 * k)) = clamped;
-                    }
+                if ((maskChannel >> 1) == p) {                  // uniform; the mask channel is below setChannels
+                    if (maskChannel & 1) a1 = a1 > 0.f ? fminf(a1, 1.f) : 0.f;
+                    else                 a0 = a0 > 0.f ? fminf(a0, 1.f) : 0.f;
+                    uint32_t const clamped = uint32_t(__builtin_bit_cast(uint16_t, _Float16(a0)))
+                                           | uint32_t(__builtin_bit_cast(uint16_t, _Float16(a1))) << 16;
+                    if (clamped != va[p][k]) *reinterpret_cast<uint32_t*>(a + base + size_t(2 * p) * size_t(width) + size_t(2 * k)) = clamped;
                 }
                 float d0 = a0 - float(__builtin_bit_cast(_Float16, uint16_t(vb[p][k])));
                 float d1 = a1 - float(__builtin_bit_cast(_Float16, uint16_t(vb[p][k] >> 16)));
-                if constexpr (MASKED) {
-                    if (maskedOut[k] && maskChannel != 2 * p) d0 = 0.f;
-                    if (maskedOut[k] && maskChannel != 2 * p + 1) d1 = 0.f;
-                }
+                if (maskedOut[k] && maskChannel != 2 * p) d0 = 0.f;
+                if (maskedOut[k] && maskChannel != 2 * p + 1) d1 = 0.f;
                 s0 += d0 * d0;
                 s1 += d1 * d1;
             }
@@ -1401,57 +1529,40 @@ image_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int 
             acc[2 * p + 1] += double(s1);
         }
     }
-    // Across the workgroup: 16 threads per channel add 16 of its 256 values each, then each other's.  (With exchanges
-    // between lanes, 17 of a double and 1500 instructions when every lane hands over half of what it holds at a step,
-    // this took 1 us longer.)
-#pragma unroll
-    for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) lanes[c * STRIDE + int(threadIdx.x)] = acc[c];
-    __syncthreads();
-    int const channel = int(threadIdx.x) >> 4, part = int(threadIdx.x) & 15;
-    double mine = 0.0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) mine += lanes[channel * STRIDE + part + 16 * k];
-    mine = add_from_row<0xB1>(mine);                         // quad_perm: the neighbour,
-    mine = add_from_row<0x4E>(mine);                         // the other pair,
-    mine = add_from_row<0x141>(mine);                        // row_half_mirror: the other quad,
-    mine = add_from_row<0x140>(mine);                        // row_mirror: the other eight
-    if (channel >= setChannels || !((validChannelMask >> channel) & 1u)) mine = 0.0;
-    uint32_t const block = blockIdx.y * gridX + blockIdx.x;
-    uint32_t const group = block / groupSize, first = group * groupSize, members = min(groupSize, blocks - first);
-    double total;                                            // threads 0 ... 15: a channel's each
-    if (members > 1) {
-        __shared__ double scratch[16][NTC_HIP_DEV_MAX_CHANNELS];
-        __shared__ int last;
-        if (part == 0) publish(work.partials + size_t(block) * NTC_HIP_DEV_MAX_CHANNELS + channel, mine);
-        if (!arrived_last(work.counters + group, members, last)) return;
-        total = sum_entries(work.partials + size_t(first) * NTC_HIP_DEV_MAX_CHANNELS, int(members), scratch);
-    } else {
-        if (part == 0) sums[channel] = mine;
-        __syncthreads();
-        total = sums[threadIdx.x & (NTC_HIP_DEV_MAX_CHANNELS - 1)];
-    }
-    // To the host in one trip: each half of a double is stored together with the serial number, so that every word
-    // says for itself whether it has arrived.  Stores of system scope go past the caches.  (Plain stores and a release
-    // behind them write back the die's whole L2.)
-    if (threadIdx.x >= 64) return;
-    uint64_t const sum = __builtin_bit_cast(uint64_t, __shfl(total, lane >> 1, 64));
-    uint64_t const word = uint64_t(work.serial) << 32 | ((lane & 1) ? sum >> 32 : sum & 0xffffffffu);
-    if (lane < 2 * NTC_HIP_DEV_MAX_CHANNELS)
-        __hip_atomic_store(&work.rows[group].words[lane], word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    hand_over_sums(sum_of_lanes(acc, setChannels), validChannelMask, blockIdx.y * gridX + blockIdx.x, blocks, groupSize, work);
 }
 
 hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int height, int setChannels, uint32_t validChannelMask,
                              int maskChannel, int discardMaskedOut, LossWorkspace const& work, hipStream_t stream, hipEvent_t done)
 {
     LossGrid const grid = image_loss_grid(width, height, compute_units_of_current_device());
-    bool const two = (width & 1) == 0, masked = maskChannel >= 0;
-    auto launch = [&](auto perLane, auto masks) {
-        constexpr auto kernel = image_loss_kernel<decltype(perLane)::value, decltype(masks)::value>;
-        return launch_kernel_with_event<kernel>(dim3(grid.x, grid.y), dim3(256), 0, stream, done, a, b, width, height, setChannels, grid.rowsPerWave,
-                                     validChannelMask, maskChannel, discardMaskedOut, grid.x, grid.x * grid.y, grid.groupSize, work);
+    uint32_t const blocks = grid.x * grid.y;
+    // Without a mask: 2^log2Lanes lanes to a row, as few as cover a narrow one with four texels each, all 256 at most, and a
+    // multiple of the rows that a workgroup's lanes take together.  (Workgroups that this leaves no row hand over zeros.)
+    int log2Lanes = 0;
+    while (log2Lanes < 8 && (4 << log2Lanes) < width) ++log2Lanes;
+    uint32_t const together = 256u >> log2Lanes, rows = ((uint32_t(height) + blocks - 1u) / blocks + together - 1u) / together * together;
+    // The masked kernel's too are rows of less than four texels, each loaded alone (1 x 1 13.2 us, 11.5 the other way), rows
+    // beyond 31 bits of offsets, and wide images of few rows, which leave most workgroups none (16
+    // channels, 16384 x 1 30 us, 15.6 the other way; 8192 x 8 22 and 16.5; 4096 x 64 19.5 and 17.1; 2048 x 128, twice the even
+    // share, 17.5 and 17.7)
+    uint64_t const share = uint64_t(rows) * uint64_t(width), even = uint64_t(width) * uint64_t(height) / blocks;
+    bool const shared = share <= 2u * (even < 1024u ? 1024u : even);
+    if (maskChannel < 0 && width >= 4 && shared && share * uint64_t(setChannels) * 2u < 0x80000000u) {
+        auto launch = [&](auto steps, auto pairs) {
+            return launch_kernel_with_event<image_loss_kernel<decltype(steps)::value, decltype(pairs)::value>>(dim3(blocks), dim3(256), 0, stream, done,
+                                         a, b, width, height, setChannels, int(rows), log2Lanes, validChannelMask, blocks, grid.groupSize, work);
+        };
+        // a row is one, two or more steps of 1024 texels
+        if (width >= 4096) return launch(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{});
+        if (width >= 2048) return launch(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});
+        return launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 4>{});
+    }
+    auto launch = [&](auto perLane) {
+        return launch_kernel_with_event<masked_loss_kernel<decltype(perLane)::value>>(dim3(grid.x, grid.y), dim3(256), 0, stream, done,
+                                     a, b, width, height, setChannels, grid.rowsPerWave, validChannelMask, maskChannel, discardMaskedOut, grid.x, blocks, grid.groupSize, work);
     };
-    auto of_width = [&](auto perLane) { return masked ? launch(perLane, std::true_type{}) : launch(perLane, std::false_type{}); };
-    return two ? of_width(std::integral_constant<int, 2>{}) : of_width(std::integral_constant<int, 1>{});
+    return (width & 1) == 0 ? launch(std::integral_constant<int, 2>{}) : launch(std::integral_constant<int, 1>{});
 }
 
 // ---- image difference (src/shaders/ImageDifference.hlsl) -------------------------------------------

@@ -117,11 +117,13 @@ struct WriteChannelsArgs {
 };
 hipError_t launch_write_channels(WriteChannelsArgs const& args, hipStream_t stream);
 
-// Grid of the loss kernel: a workgroup (= one row of 16 double partial sums) covers 64 lanes x 1 or 2
-// texels (2 when the width is even) by 4 waves x rowsPerWave rows.  Four workgroups are resident on a compute unit; as
+// Grid of the loss kernels.  With a mask channel a workgroup (= one row of 16 double partial sums) covers 64 lanes x 1 or 2
+// texels (2 when the width is even) by 4 waves x rowsPerWave rows; without one as many workgroups divide the image by whole rows.  Four workgroups are resident on a compute unit; as
 // many rows per wave as make the grid about that large (every workgroup ends in 16 reductions across its lanes, and a
 // row is a memory round trip), from one, for images that would not fill the GPU, to 32.
 constexpr uint32_t kLossRows = 32;                          // groups of workgroups, each of which hands its sums to the host
+// Counters of the groups' workgroups lie 256 bytes apart: on one line a thousand arrivals wait for each other.
+constexpr uint32_t kLossCounterStride = 64;
 struct LossGrid { uint32_t x, y, groupSize; int32_t rowsPerWave; };
 inline LossGrid image_loss_grid(int width, int height, int computeUnits)
 {
@@ -136,7 +138,7 @@ inline LossGrid image_loss_grid(int width, int height, int computeUnits)
 struct LossRow { uint64_t words[32]; };
 struct LossWorkspace {
     double* partials;              // 16 per workgroup
-    uint32_t* counters;            // kLossRows: zero before and after every launch
+    uint32_t* counters;            // kLossRows, kLossCounterStride apart: zero before and after every launch
     LossRow* rows;                 // kLossRows, device address
     uint32_t serial;
 };

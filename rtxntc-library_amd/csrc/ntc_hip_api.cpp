@@ -507,8 +507,8 @@ int prepare_loss_workspace(Library& L, size_t blocks)
     if (L.lossDev) { HIP_TRY(hipFree(L.lossDev)); L.lossDev = nullptr; }
     HIP_TRY(hipMalloc(reinterpret_cast<void**>(&L.lossDev), blocks * NTC_HIP_DEV_MAX_CHANNELS * sizeof(double)));
     if (L.lossBlocks == 0) {
-        HIP_TRY(hipMalloc(reinterpret_cast<void**>(&L.lossCounters), kLossRows * sizeof(uint32_t)));
-        HIP_TRY(launch_fill(reinterpret_cast<uint8_t*>(L.lossCounters), 0, kLossRows * sizeof(uint32_t), L.stream));
+        HIP_TRY(hipMalloc(reinterpret_cast<void**>(&L.lossCounters), kLossRows * kLossCounterStride * sizeof(uint32_t)));
+        HIP_TRY(launch_fill(reinterpret_cast<uint8_t*>(L.lossCounters), 0, kLossRows * kLossCounterStride * sizeof(uint32_t), L.stream));
         HIP_TRY(hipEventCreateWithFlags(&L.lossDone, hipEventDisableTiming));
         HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&L.lossHost), kLossRows * sizeof(LossRow), hipHostMallocMapped | hipHostMallocCoherent));
         std::memset(L.lossHost, 0, kLossRows * sizeof(LossRow));

@@ -137,6 +137,21 @@ def test_loss_sums_of_one_group_and_of_many(ntc, device, oracle, w, h):
     assert np.allclose(results[0], want, rtol=2e-7, atol=0) and np.array_equal(results[0], results[1])
 
 
+@pytest.mark.parametrize("w,h,channels", [(3, 9, 2), (4, 1001, 16), (7, 777, 2), (255, 130, 14), (1023, 37, 10), (1029, 1030, 6), (2050, 601, 4),
+                                          (3071, 2, 16), (4099, 1100, 2), (8192, 3, 6)])
+def test_loss_sums_of_whole_rows(ntc, device, oracle, w, h, channels):
+    """Rows of one, two and more steps of the workgroup's lanes with what is left of them, several rows a workgroup's lanes
+    take together, fewer pairs than are loaded together, and images that fall to the masked kernel."""
+    rng = np.random.default_rng(w * h)
+    a, b = halves(rng, w * h * channels), halves(rng, w * h * channels)
+    d_a, d_b = device.upload(a), device.upload(b)
+    want, got = np.zeros(16, dtype=np.float64), (ntc.abi.C.c_float * 16)()
+    mask = 0x5FF7 & ((1 << channels) - 1)
+    oracle.ntc_oracle_image_loss(a.ctypes.data, b.ctypes.data, w, h, channels, mask, want.ctypes.data)
+    device.call("image_loss", d_a.ptr, d_b.ptr, d_a.nbytes, w, h, channels, mask, -1, 0, got)
+    assert np.allclose(got[:], want, rtol=2e-7, atol=0)      # (double sums, rounded to float once)
+
+
 @pytest.mark.parametrize("mask_channel", [-1, 5])
 def test_loss_behind_queued_work(ntc, device, mask_channel):
     """Work of several milliseconds in front of the call, the last of which writes the image: the host's look for early sums
