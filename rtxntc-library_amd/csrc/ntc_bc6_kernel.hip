@@ -137,6 +137,18 @@ template <bool WIDE> struct Msle {
         V3 const sq = d * d * V3{ 0.299f, 0.587f, 0.114f };
         return sq.x + sq.y + sq.z;
     }
+    // With the hardware's logarithm: within 2^-19 of its value, 0 where that is 0, infinite or no number where that is not
+    // a number of normal size.
+    BC6_INLINE float estimate(V3 b) const
+    {
+        V3 const n = b + V3{ 1.f, 1.f, 1.f };
+        V3 q;
+        if constexpr (WIDE) q = V3{ n.x / a.x, n.y / a.y, n.z / a.z };
+        else                q = V3{ corrected(n.x, a.x, r.x), corrected(n.y, a.y, r.y), corrected(n.z, a.z, r.z) };
+        V3 const d{ __builtin_amdgcn_logf(q.x), __builtin_amdgcn_logf(q.y), __builtin_amdgcn_logf(q.z) };
+        V3 const sq = d * d;
+        return __builtin_fmaf(sq.z, 0.114f, __builtin_fmaf(sq.y, 0.587f, sq.x * 0.299f));
+    }
 };
 
 // (the quotients by constants here and below are those of integers, times a power of two)
@@ -154,6 +166,14 @@ BC6_INLINE V3 interpolate(V3 e0, V3 e1, float weight)
     V3 const c = (e0 * (64.f - weight) + e1 * weight + V3{ 32.f, 32.f, 32.f }) * (31.f / 4096.f);
     return { from_half_bits(c.x), from_half_bits(c.y), from_half_bits(c.z) };
 }
+// The same of the two-subset endpoints, integers whose products are exact.
+BC6_INLINE V3 interpolate_integers(V3 e0, V3 e1, float weight)
+{
+    float const w0 = 64.f - weight;
+    V3 const c = V3{ __builtin_fmaf(e0.x, w0, __builtin_fmaf(e1.x, weight, 32.f)), __builtin_fmaf(e0.y, w0, __builtin_fmaf(e1.y, weight, 32.f)),
+                     __builtin_fmaf(e0.z, w0, __builtin_fmaf(e1.z, weight, 32.f)) } * (31.f / 4096.f);
+    return { from_half_bits(c.x), from_half_bits(c.y), from_half_bits(c.z) };
+}
 BC6_INLINE uint32_t index_of(float pos, float e0, float e1, float scale, float bias, float top)
 {
     float const a = pos - e0, b = e1 - e0;                   // half codes: integers
@@ -162,6 +182,16 @@ BC6_INLINE uint32_t index_of(float pos, float e0, float e1, float scale, float b
 }
 BC6_INLINE uint32_t index3(float pos, float e0, float e1) { return index_of(pos, e0, e1, 6.98182f, 0.00909f, 7.f); }
 BC6_INLINE uint32_t index4(float pos, float e0, float e1) { return index_of(pos, e0, e1, 14.93333f, 0.03333f, 15.f); }
+// The format's weights of those indices, floor(64 index / 7 + 1/2) and floor(64 index / 15 + 1/2).
+constexpr uint32_t weight3(uint32_t index) { return 9u * index + (index >> 2); }
+constexpr uint32_t weight4(uint32_t index) { return (273u * index + 32u) >> 6; }
+constexpr bool weights_agree()
+{
+    for (uint32_t i = 0; i < 16; ++i)
+        if ((i < 8 && weight3(i) != (128u * i + 7u) / 14u) || weight4(i) != (128u * i + 15u) / 30u) return false;
+    return true;
+}
+static_assert(weights_agree());
 template <bool WIDE> BC6_INLINE V3 divided(V3 v, float s)
 {
     if constexpr (WIDE) return { v.x / s, v.y / s, v.z / s };
@@ -179,28 +209,34 @@ BC6_INLINE float exp1(float c) { return exp2_of_log(c) - 1.f; }
 //   1. one wave: the one-subset endpoints; then all: bounds of the patterns' scores, patterns taken in turn, and the
 //      scores of those that the bounds leave;
 //   2. a wave per subset of each block's pattern: its endpoints;
-//   3. each wave four of the sixteen texels: indices and errors of all three candidates;
-//   4. one wave: the errors added up in texel order, the choice, the block.
-// Bound by the issue of vector instructions: 72 % of the slots at 2048 x 2048, the rest goes where one wave works and the
-// others wait for it, or for texels from LDS.  Each part is a function with registers of its own, so that four waves fit
-// a SIMD and nothing is spilled in a loop; the search is one call because a call saves registers to scratch (a call per
-// two patterns: 257 us at 2048 x 2048 instead of 204).  One lane per block, all parts in one body with 168 registers,
-// took 121 us at 64 x 64, 151 at 1024 x 1024 and 287 at 2048 x 2048: small images waited for the chain of one lane's
-// scores, large ones for its spills and longer divisions.  Shared by the waves: 30, 61 and 204 (195 beside other
-// kernels), of which the 32 scores, 625 instructions each, were more than half; with their bounds first: 165 at 2048 x
-// 2048.
+//   3. each wave four of the sixteen texels: indices and estimates of the errors of all three candidates, and the errors
+//      as they are defined where the estimates are too close to tell;
+//   4. one wave: the block.
+// Bound by the issue of vector instructions and by waves that wait for the one that works alone: 68 % of the slots with four
+// workgroups on a compute unit.  31.5 KB of LDS (what one part leaves, the next one overwrites) and 96 registers let five be
+// there: 141 us at 2048 x 2048 with four, 133 with five, 137 with six, which takes texels in three planes and registers kept
+// in scratch.  Each part is a function with registers of its own, so that nothing is spilled in a loop; the search is one
+// call because a call saves registers to scratch (a call per two patterns: 257 us at 2048 x 2048 instead of 204).  One lane
+// per block, all parts in one body with 168 registers, took 121 us at 64 x 64, 151 at 1024 x 1024 and 287 at 2048 x 2048:
+// small images waited for the chain of one lane's scores, large ones for its spills and longer divisions.  Shared by the
+// waves: 30, 61 and 204 (195 beside other kernels), of which the 32 scores, 625 instructions each, were more than half;
+// with their bounds first 165 beside others, 29, 47 and 147 alone; with estimated errors (the logarithms were 13 % of the
+// instructions) and five workgroups 27, 42 and 126, 4096 x 4096 520 -> 417.
 struct Bc6Lds {
     float4 texels[16][64];
     float one[11][64];                                       // one subset: lo, hi, direction, codes of the ends along it
-    float two[2][11][64];                                    // each of two subsets
     union {
-        float errors[3][16][64];                             // per texel: one subset, 7 + 6 bits, 9 + 5 bits
         float least[32][64];                                 // until the pattern is picked: lower bounds of the scores
+        struct {
+            float two[2][11][64];                            // each of two subsets
+            float errors[3][4][64];                          // of four texels, estimated: one subset, 7 + 6 bits, 9 + 5 bits
+        };
     };
     uint32_t indices[2][4][64];                              // of four texels: 4 bits each, 3 bits each
     int next;
     uint64_t pick[64];                                       // score bits << 32 | pattern
     uint32_t bound[64], candidates[64], unbounded[64];       // smallest upper bound of a score; patterns that it leaves; some have no bounds
+                                                             // (at the end: choices by the errors as they are defined; the blocks that need them)
     uint32_t unscored[64];                                   // pattern 0's score is a NaN: the search stays there
 };
 using Bc6Ptr = __attribute__((address_space(3))) Bc6Lds*;
@@ -475,58 +511,100 @@ BC6_INLINE void base_and_deltas(Bc6Ptr lds, int b, float levels, float limit, V3
     for (int i = 1; i < 4; ++i) q[i] = clamp3(q[i] - q[0], limit);
 }
 
-// Indices and errors of four texels under the three candidates.
+// Indices of four texels under the three candidates and, as estimates, what they add to the candidates' errors.
 template <bool WIDE>
-BC6_TASK void texel_errors(Bc6Ptr lds, int b, int quarter)
+BC6_TASK void estimate_errors(Bc6Ptr lds, int b, int quarter)
 {
     quarter = __builtin_amdgcn_readfirstlane(quarter);
-    uint32_t indices = 0;
+    SubsetEnds const one = load_ends(lds->one, b);
+    V3 const u0 = unquantize(quantize(one.lo, 1024.f), 1024.f), u1 = unquantize(quantize(one.hi, 1024.f), 1024.f);
+    V3 u7[4], u9[4];
+    {
+        V3 q[4];
+        base_and_deltas(lds, b, 128.f, 31.f, q);
+        u7[0] = unquantize(q[0], 128.f);
+#pragma unroll
+        for (int i = 1; i < 4; ++i) u7[i] = unquantize(q[0] + q[i], 128.f);
+        base_and_deltas(lds, b, 512.f, 15.f, q);
+        u9[0] = unquantize(q[0], 512.f);
+#pragma unroll
+        for (int i = 1; i < 4; ++i) u9[i] = unquantize(q[0] + q[i], 512.f);
+    }
+    uint32_t const second = kSecondSubset[picked_pattern(lds, b)] >> (4 * quarter);
+    uint32_t indices4 = 0, indices3 = 0;
+    float error1 = 0.f, error7 = 0.f, error9 = 0.f;
+#pragma unroll 2
+    for (int i = 0; i < 4; ++i) {
+        V3 const p = texel(lds, b, 4 * quarter + i);
+        Msle<WIDE> const error(p);
+        uint32_t const index = index4(to_half_bits(dot(p, one.dir)), one.e0, one.e1);
+        indices4 |= index << (4 * i);
+        error1 += error.estimate(interpolate(u0, u1, float(weight4(index))));
+        bool const s = (second >> i) & 1u;
+        V3 const dir{ lds->two[s][6][b], lds->two[s][7][b], lds->two[s][8][b] };
+        uint32_t const inSubset = index3(to_half_bits(dot(p, dir)), lds->two[s][9][b], lds->two[s][10][b]);
+        indices3 |= inSubset << (3 * i);
+        float const weight = float(weight3(inSubset));
+        error7 += error.estimate(interpolate_integers(s ? u7[2] : u7[0], s ? u7[3] : u7[1], weight));
+        error9 += error.estimate(interpolate_integers(s ? u9[2] : u9[0], s ? u9[3] : u9[1], weight));
+    }
+    lds->indices[0][quarter][b] = indices4; lds->indices[1][quarter][b] = indices3;
+    lds->errors[0][quarter][b] = error1; lds->errors[1][quarter][b] = error7; lds->errors[2][quarter][b] = error9;
+}
+
+// What the estimates say of the choice between the candidates; 3: nothing.  An estimate and the error as it is defined
+// are sums of 48 terms that differ by 2^-19, in different orders: within 2^-18.5 of each other.
+BC6_INLINE int estimated_choice(Bc6Ptr lds, int b)
+{
+    float e[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) e[c] = (lds->errors[c][0][b] + lds->errors[c][1][b]) + (lds->errors[c][2][b] + lds->errors[c][3][b]);
+    constexpr float kSure = 1.f - 0x1p-17f;
+    auto const less = [&](int x, int y) { return e[x] < e[y] * kSure; };
+    if (less(0, 1) && less(0, 2)) return 0;
+    if (less(1, 2) && less(1, 0)) return 1;
+    if (less(2, 1) && less(2, 0)) return 2;
+    return 3;
+}
+
+// The choice between the candidates of one block (by its lanes, sixteen to a block, a texel each) by their errors as they
+// are defined, added up in texel order.
+template <bool WIDE>
+BC6_TASK int defined_choice(Bc6Ptr lds, int b, int t)
+{
+    V3 const p = texel(lds, b, t);
+    Msle<WIDE> const error(p);
+    float of[3], sum[3] = { 0.f, 0.f, 0.f };
     {
         SubsetEnds const s = load_ends(lds->one, b);
         V3 const u0 = unquantize(quantize(s.lo, 1024.f), 1024.f), u1 = unquantize(quantize(s.hi, 1024.f), 1024.f);
-#pragma unroll 2
-        for (int i = 0; i < 4; ++i) {
-            V3 const p = texel(lds, b, 4 * quarter + i);
-            uint32_t const index = index4(to_half_bits(dot(p, s.dir)), s.e0, s.e1);
-            lds->errors[0][4 * quarter + i][b] = Msle<WIDE>(p)(interpolate(u0, u1, floorf(corrected(float(index) * 64.f, 15.f, 1.f / 15.f) + 0.5f)));
-            indices |= index << (4 * i);
-        }
-        lds->indices[0][quarter][b] = indices;
+        of[0] = error(interpolate(u0, u1, float(weight4((lds->indices[0][t >> 2][b] >> (4 * (t & 3))) & 15u))));
     }
-    V3 q7[4], q9[4];
-    base_and_deltas(lds, b, 128.f, 31.f, q7);
-    base_and_deltas(lds, b, 512.f, 15.f, q9);
-    V3 u7[4], u9[4];
-    u7[0] = unquantize(q7[0], 128.f); u9[0] = unquantize(q9[0], 512.f);
-#pragma unroll
-    for (int i = 1; i < 4; ++i) { u7[i] = unquantize(q7[0] + q7[i], 128.f); u9[i] = unquantize(q9[0] + q9[i], 512.f); }
-    uint32_t const second = kSecondSubset[picked_pattern(lds, b)];
-    indices = 0;
+    int const s = (kSecondSubset[picked_pattern(lds, b)] >> t) & 1;
+    float const weight = float(weight3((lds->indices[1][t >> 2][b] >> (3 * (t & 3))) & 7u));
 #pragma unroll 1
-    for (int i = 0; i < 4; ++i) {
-        int const t = 4 * quarter + i;
-        V3 const p = texel(lds, b, t);
-        bool const s = (second >> t) & 1u;
-        V3 const dir{ lds->two[s][6][b], lds->two[s][7][b], lds->two[s][8][b] };
-        uint32_t const index = index3(to_half_bits(dot(p, dir)), lds->two[s][9][b], lds->two[s][10][b]);
-        float const weight = floorf(corrected(float(index) * 64.f, 7.f, 1.f / 7.f) + 0.5f);
-        Msle<WIDE> const error(p);
-        lds->errors[1][t][b] = error(interpolate(s ? u7[2] : u7[0], s ? u7[3] : u7[1], weight));
-        lds->errors[2][t][b] = error(interpolate(s ? u9[2] : u9[0], s ? u9[3] : u9[1], weight));
-        indices |= index << (3 * i);
+    for (int c = 1; c < 3; ++c) {
+        float const levels = c == 1 ? 128.f : 512.f;
+        V3 q[4];
+        base_and_deltas(lds, b, levels, c == 1 ? 31.f : 15.f, q);
+        V3 const u0 = unquantize(s ? q[0] + q[2] : q[0], levels), u1 = unquantize(q[0] + (s ? q[3] : q[1]), levels);
+        float const e = error(interpolate_integers(u0, u1, weight));
+        of[1] = c == 1 ? e : of[1]; of[2] = e;
     }
-    lds->indices[1][quarter][b] = indices;
+    int const lane = int(threadIdx.x) & 63;
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) sum[c] += __shfl(of[c], (lane & 48) + k, 64);
+    float const least = fminf(sum[1], sum[2]);
+    return !(least < sum[0]) ? 0 : least == sum[1] ? 1 : 2;
 }
 
-// The choice between the candidates and the block.
-BC6_INLINE void final_block(Bc6Ptr lds, int b, uint64_t& outLo, uint64_t& outHi)
+// The block of the candidate: 0 one subset, 1 two with 7 + 6 bits, 2 two with 9 + 5 bits.
+BC6_INLINE void final_block(Bc6Ptr lds, int b, int choice, uint64_t& outLo, uint64_t& outHi)
 {
-    float error1 = 0.f, error7 = 0.f, error9 = 0.f;
-#pragma unroll
-    for (int t = 0; t < 16; ++t) { error1 += lds->errors[0][t][b]; error7 += lds->errors[1][t][b]; error9 += lds->errors[2][t][b]; }
-    float const error = fminf(error7, error9);
     Bits bits;
-    if (!(error < error1)) {
+    if (choice == 0) {
         V3 const q0 = quantize(V3{ lds->one[0][b], lds->one[1][b], lds->one[2][b] }, 1024.f), q1 = quantize(V3{ lds->one[3][b], lds->one[4][b], lds->one[5][b] }, 1024.f);
         bits.put(0, 0x03, 5);
         bits.put(5, uint32_t(q0.x), 10); bits.put(15, uint32_t(q0.y), 10); bits.put(25, uint32_t(q0.z), 10);
@@ -538,7 +616,7 @@ BC6_INLINE void final_block(Bc6Ptr lds, int b, uint64_t& outLo, uint64_t& outHi)
         return;
     }
     int const pattern = picked_pattern(lds, b), anchor1 = kSecondAnchor[pattern];
-    bool const sevenSix = error == error7;
+    bool const sevenSix = choice == 1;
     V3 q[4];
     base_and_deltas(lds, b, sevenSix ? 128.f : 512.f, sevenSix ? 31.f : 15.f, q);
     int const baseBits = sevenSix ? 7 : 9, deltaBits = sevenSix ? 6 : 5;
@@ -574,7 +652,7 @@ BC6_INLINE void final_block(Bc6Ptr lds, int b, uint64_t& outLo, uint64_t& outHi)
 } // namespace
 
 template <bool WIDE>
-__global__ void __launch_bounds__(256, 4)
+__global__ void __launch_bounds__(256, 5)
 bc6_compress_kernel(BlockCompressArgs a)
 {
     __shared__ Bc6Lds shared;
@@ -609,11 +687,24 @@ bc6_compress_kernel(BlockCompressArgs a)
     __syncthreads();
     if (wave < 2) subset_ends<WIDE>(lds, lane, wave);
     __syncthreads();
-    texel_errors<WIDE>(lds, lane, wave);
+    estimate_errors<WIDE>(lds, lane, wave);
     __syncthreads();
+    int choice = estimated_choice(lds, lane);
+    uint64_t const open = __ballot(choice == 3);             // the same in all waves, few
+    if (open) {
+        if (choice == 3) shared.candidates[__popcll(open & ((uint64_t(1) << lane) - 1u))] = uint32_t(lane);
+        __syncthreads();
+        int const last = __popcll(open) - 1;
+        for (int first = 4 * wave; first <= last; first += 16) {
+            int const b = int(shared.candidates[min(first + (lane >> 4), last)]);
+            shared.bound[b] = uint32_t(defined_choice<WIDE>(lds, b, lane & 15));
+        }
+        __syncthreads();
+        if (choice == 3) choice = int(shared.bound[lane]);
+    }
     if (wave != 0 || !inside) return;
     uint64_t lo, hi;
-    final_block(lds, lane, lo, hi);
+    final_block(lds, lane, choice, lo, hi);
     uint64_t* const dst = reinterpret_cast<uint64_t*>(a.dst + size_t(by + a.dstOffsetY) * a.dstRowPitch) + size_t(bx + a.dstOffsetX) * 2;
     dst[0] = lo; dst[1] = hi;
 }

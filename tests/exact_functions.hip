@@ -150,6 +150,16 @@ struct QuotientOfMsle {
         return verdict(same(corrected(a, b, reciprocal<1>(b)), a / b));
     }
 };
+// Msle::estimate(): the hardware's logarithm of every quotient that can occur is within 2^-21 of normal_log2(), and 0 where that is 0.
+struct LogEstimate {
+    static constexpr uint64_t cases = uint64_t(34) << 23;
+    static __device__ int check(uint64_t i)
+    {
+        uint32_t const bits = ((127u - 17u) << 23) + uint32_t(i);
+        float const log = normal_log2(bits, 0);
+        return verdict(fabsf(__builtin_amdgcn_logf(__uint_as_float(bits)) - log) <= fabsf(log) * 0x1p-21f);
+    }
+};
 // quantize() and the indices' places.
 struct QuotientOfCodes {
     static constexpr uint64_t cases = 3 * 65536 + 64;
@@ -208,6 +218,7 @@ int exact_bc4_palette(Report* r) { return sweep<Bc4Palette>(r); }
 int exact_quotient_of_integers(Report* r) { return sweep<QuotientOfIntegers>(r); }
 int exact_quotient_of_log2(Report* r) { return sweep<QuotientOfLog2>(r); }
 int exact_quotient_of_msle(Report* r) { return sweep<QuotientOfMsle>(r); }
+int exact_log_estimate(Report* r) { return sweep<LogEstimate>(r); }
 int exact_quotient_of_codes(Report* r) { return sweep<QuotientOfCodes>(r); }
 int exact_quotient_of_diagonals(Report* r) { return sweep<QuotientOfDiagonals>(r); }
 #else

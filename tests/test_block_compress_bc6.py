@@ -265,3 +265,22 @@ def test_gpu_bc6_equal_and_short_patterns(ntc, device, oracle, fmt, diagonal):
     got = compress(ntc, None, device, image, fmt, 3, 6, blocks_x, blocks_y)
     bad = np.argwhere(got != want)
     assert bad.size == 0, (fmt, diagonal, len(bad), bad[:3])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", [3, 4])
+@pytest.mark.parametrize("open_blocks", [0, 1, 4, 5, 17, 64])
+def test_gpu_bc6_choice_by_errors_as_defined(ntc, device, oracle, fmt, open_blocks):
+    """Workgroups of 64 blocks of which none, some and all need the errors as they are defined: endpoints that decode to
+    infinity leave the estimates without a number."""
+    rng = np.random.default_rng(662 + open_blocks)
+    image = rng.integers(0x2000, 0x5000, (32, 64, 3)).astype(np.uint16).view(np.float16)
+    for group in range(2):
+        for b in rng.permutation(64)[:open_blocks]:
+            x, y = 32 * group + 4 * (b % 8), 4 * (b // 8)
+            image[y: y + 4, x: x + 4] = rng.integers(0x7BF0, 0x7C00, (4, 4, 3)).astype(np.uint16).view(np.float16)
+    image = image.astype({3: np.float16, 4: np.float32}[fmt])
+    want = compress(ntc, oracle, None, image, fmt, 3, 6, 16, 8)
+    got = compress(ntc, None, device, image, fmt, 3, 6, 16, 8)
+    bad = np.argwhere(got != want)
+    assert bad.size == 0, (fmt, open_blocks, len(bad), bad[:3])

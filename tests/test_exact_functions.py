@@ -21,7 +21,7 @@ class Report(C.Structure):
     ("copy", "put_unorm8", 1 << 32), ("copy", "divide_by_255", (1 << 23) + 256), ("copy", "divide_by_65535", (1 << 23) + 65536),
     ("bc", "code_quotient", 96), ("bc", "bc4_palette", 65536),
     ("bc6", "quotient_of_integers", (1 << 17) * ((1 << 17) - 1)), ("bc6", "quotient_of_log2", None),
-    ("bc6", "quotient_of_msle", 0x7c00 * (0x7c00 + 256 + 65536 + 65505)), ("bc6", "quotient_of_codes", 3 * 65536 + 64),
+    ("bc6", "quotient_of_msle", 0x7c00 * (0x7c00 + 256 + 65536 + 65505)), ("bc6", "log_estimate", 34 << 23), ("bc6", "quotient_of_codes", 3 * 65536 + 64),
     ("bc6", "quotient_of_diagonals", 1 << 30), ("decode", "texel_centre", (1 << 15) * 65537)])
 def test_gpu_shortcut_equals_the_operation(device, subject, function, cases):
     path = os.path.join(HERE, f"libexact_{subject}.so")
