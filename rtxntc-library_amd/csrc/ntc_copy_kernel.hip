@@ -1618,6 +1618,17 @@ __device__ __forceinline__ float pixel_channel(uint32_t const (&words)[bytes_per
     else                                                     return __builtin_bit_cast(float, w);
 }
 
+// A tile's sum as it is added to the accumulators.
+__device__ __forceinline__ unsigned long long fixed_share(float total, int width, int height)
+{
+    total = __fdiv_rn(total, float(width * height));
+    total = __fmul_rn(total, 65536.f);
+    float const whole = floorf(total);
+    // float -> uint32 conversions saturate; a NaN (from NaN pixels) adds nothing
+    unsigned long long const high = uint32_t(whole), low = uint32_t(floorf(__fmul_rn(__fsub_rn(total, whole), 4294967296.f)));
+    return (high << 32) | low;
+}
+
 // FORMAT: of both images, four channels each; 0: any two images.
 template <int FORMAT, bool MSLE>
 __global__ void __launch_bounds__(256)
@@ -1683,16 +1694,134 @@ image_difference_kernel(ImageDifferenceArgs a, int tilesX, int tiles, int step)
         if (threadIdx.x < 4) {
             int const c = threadIdx.x;
             float total = __fadd_rn(__fadd_rn(__fadd_rn(sums[0][c], sums[1][c]), sums[2][c]), sums[3][c]);
-            total = __fdiv_rn(total, float(a.width * a.height));
-            total = __fmul_rn(total, 65536.f);
-            float const whole = floorf(total);
-            // float -> uint32 conversions saturate; a NaN (from NaN pixels) adds nothing
-            unsigned long long const high = uint32_t(whole), low = uint32_t(floorf(__fmul_rn(__fsub_rn(total, whole), 4294967296.f)));
-            fixed += (high << 32) | low;
+            fixed += fixed_share(total, a.width, a.height);
         }
         __syncthreads();
     }
     if (threadIdx.x < 4 && fixed) atomicAdd(a.output + threadIdx.x, fixed);
+}
+
+// MSE of pixels of at most eight bytes without padding, in images of many tiles: four waves take four tiles side by side, a
+// wave sixteen rows of all four, a lane four columns, 16 bytes a load.  A column's sum is made by one lane in row order as
+// above; the butterfly's offsets 32 ... 4 are rotations of a tile's sixteen lanes (what is below the rotation's bit is equal
+// by then), 2 and 1 are between a lane's own columns.  TEAMS of four waves share a workgroup's four atomics: a thousand
+// workgroups that end together wait for each other's.  Bound by memory.  RGBA8, 2048 x 2048, 3072 x 3072, 4096 x 4096 and
+// 8192 x 4096: 11.3, 19.8, 23.7 and 49 us (17.6, 24, 30 and 51 with four-byte loads; one team 26.3 and four 31.4 of the
+// third, 48 and 45.5 of the last; a wave to a tile, whose loads are four row pieces a power of two apart, 22 and 27 of the
+// second and third); halves, the first three: 14, 27.8 and 39.4 (19.6, 30.3 and 43.5).  MSLE, bound by logarithms, gains
+// from more waves, not from wider loads (3072 x 3072 39 us, 47 here), and pixels of four floats are 16-byte loads anyway.
+template <int CONTROL> __device__ __forceinline__ float add_rotated(float v)
+{
+    return __fadd_rn(v, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CONTROL, 0xF, 0xF, true)));
+}
+template <int FORMAT, int TEAMS>
+__global__ void __launch_bounds__(256 * TEAMS, 4)
+image_difference_wide_kernel(ImageDifferenceArgs a, int groupsX, int groups)
+{
+    constexpr int BPC = bytes_per_channel(FORMAT), ROWS = 4 / BPC;
+    __shared__ float sums[2][TEAMS][4][16];                  // [turn][team][part][4 * tile + channel]
+    __shared__ unsigned long long shares[TEAMS][4];
+    int const lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6) & 3, team = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 8);
+    float const threshold = a.useAlphaThreshold ? a.alphaThreshold : -__builtin_inff();
+    unsigned long long fixed = 0;                            // threads 0 ... 15: the workgroup's share of a channel's sum, of the nth tiles
+    int turn = 0;
+    for (int base = blockIdx.x * TEAMS; base < groups; base += gridDim.x * TEAMS, turn ^= 1) {
+        int const group = base + team;                       // (beyond the last one: below the extent, nothing is read)
+        int const groupY = group / groupsX, groupX = group - groupY * groupsX;
+        int const x = groupX * 256 + lane * 4, y = groupY * 64 + wave * 16;
+        float mse[4][4];                                     // [column][channel]
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) mse[i][c] = 0.f;
+        u32x4_any wordsA[ROWS][BPC], wordsB[ROWS][BPC];      // rows of four pixels: a row gone through is loaded over
+        auto const add_row = [&](int r, int columns) {
+            __builtin_amdgcn_sched_barrier(0);               // (a row at a time, or the channels of more pixels than there are registers for)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (i >= columns) break;
+                uint32_t wa[BPC], wb[BPC];
+#pragma unroll
+                for (int d = 0; d < BPC; ++d) { int const at = i * BPC + d; wa[d] = wordsA[r][at >> 2][at & 3]; wb[d] = wordsB[r][at >> 2][at & 3]; }
+                float t1[4], t2[4], diff[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    t1[c] = pixel_channel<FORMAT>(wa, c); t2[c] = pixel_channel<FORMAT>(wb, c);
+                    diff[c] = __fsub_rn(t1[c], t2[c]);
+                }
+                if (t1[3] < threshold && t2[3] < threshold) { diff[0] = 0.f; diff[1] = 0.f; diff[2] = 0.f; }
+#pragma unroll
+                for (int c = 0; c < 4; ++c) mse[i][c] = __fadd_rn(mse[i][c], __fmul_rn(diff[c], diff[c]));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        if (groupX * 256 + 256 <= a.width && groupY * 64 + 64 <= a.height) {
+            uint8_t const* pa = a.a.data + size_t(y + a.top) * a.a.rowPitch + size_t(x + a.left) * (4 * BPC);
+            uint8_t const* pb = a.b.data + size_t(y + a.top) * a.b.rowPitch + size_t(x + a.left) * (4 * BPC);
+            auto const load = [&](int r) {
+#pragma unroll
+                for (int v = 0; v < BPC; ++v) {
+                    wordsA[r][v] = reinterpret_cast<u32x4_any const*>(pa)[v];
+                    wordsB[r][v] = reinterpret_cast<u32x4_any const*>(pb)[v];
+                }
+                pa += a.a.rowPitch; pb += a.b.rowPitch;
+            };
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) load(r);
+#pragma unroll 1
+            for (int first = 0; first < 16; first += ROWS) {
+#pragma unroll
+                for (int r = 0; r < ROWS; ++r) {
+                    add_row(r, 4);
+                    if (first + ROWS < 16) load(r);
+                }
+            }
+        } else {
+            int const columns = a.width - x;                 // (pixels outside the extent are read inside it and dropped)
+#pragma unroll 1
+            for (int first = 0; first < 16 && y + first < a.height; first += ROWS) {
+#pragma unroll
+                for (int r = 0; r < ROWS; ++r) {
+                    size_t const row = size_t(min(y + first + r, a.height - 1) + a.top);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        size_t const column = size_t(min(x + i, a.width - 1) + a.left) * (4 * BPC);
+                        uint32_t wa[BPC], wb[BPC];
+                        load_pixel<FORMAT>(a.a.data + row * a.a.rowPitch + column, wa);
+                        load_pixel<FORMAT>(a.b.data + row * a.b.rowPitch + column, wb);
+#pragma unroll
+                        for (int d = 0; d < BPC; ++d) { int const at = i * BPC + d; wordsA[r][at >> 2][at & 3] = wa[d]; wordsB[r][at >> 2][at & 3] = wb[d]; }
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < ROWS; ++r) add_row(r, y + first + r < a.height ? columns : 0);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = add_rotated<0x121>(add_rotated<0x122>(add_rotated<0x124>(add_rotated<0x128>(mse[i][c]))));
+            float const sum = __fadd_rn(__fadd_rn(v[0], v[2]), __fadd_rn(v[1], v[3]));
+            if ((lane & 15) == c) sums[turn][team][wave][4 * (lane >> 4) + c] = sum;
+        }
+        __syncthreads();                                     // (the next turn's sums lie elsewhere, and the one after it is behind the next barrier)
+        if (wave == 0 && lane < 16) {
+            float const (&of)[4][16] = sums[turn][team];
+            fixed += fixed_share(__fadd_rn(__fadd_rn(__fadd_rn(of[0][lane], of[1][lane]), of[2][lane]), of[3][lane]), a.width, a.height);
+        }
+    }
+    if (wave == 0 && lane < 16) {
+        fixed += __shfl_down(fixed, 8, 16);
+        fixed += __shfl_down(fixed, 4, 16);
+        if (lane < 4) shares[team][lane] = fixed;
+    }
+    if constexpr (TEAMS > 1) __syncthreads();
+    if (threadIdx.x < 4) {
+#pragma unroll
+        for (int t = 1; t < TEAMS; ++t) fixed += shares[t][lane];
+        if (fixed) atomicAdd(a.output + threadIdx.x, fixed);
+    }
 }
 
 hipError_t launch_image_difference(ImageDifferenceArgs const& a, hipStream_t stream)
@@ -1702,6 +1831,14 @@ hipError_t launch_image_difference(ImageDifferenceArgs const& a, hipStream_t str
     int const workgroups = tiles < resident ? tiles : resident;
     auto of_format = [&](auto format) {
         constexpr int FORMAT = decltype(format)::value;
+        if constexpr (FORMAT != 0 && bytes_per_channel(FORMAT) <= 2) {
+            constexpr uint64_t PIXEL = 4 * bytes_per_channel(FORMAT);
+            int const groupsX = (a.width + 255) / 256, groups = groupsX * ((a.height + 63) / 64);
+            // (with fewer groups of tiles than compute units the other kernel's are more waves: 2048 x 1024 11.2 us)
+            if (!a.useMSLE && groups >= compute_units_of_current_device() && a.a.pixelStride == PIXEL && a.b.pixelStride == PIXEL)
+                return groups < resident ? launch_kernel<image_difference_wide_kernel<FORMAT, 1>>(dim3(groups), dim3(256), 0, stream, a, groupsX, groups)
+                                         : launch_kernel<image_difference_wide_kernel<FORMAT, 2>>(dim3(resident / 2), dim3(512), 0, stream, a, groupsX, groups);
+        }
         return a.useMSLE ? launch_kernel<image_difference_kernel<FORMAT, true>>(dim3(workgroups), dim3(256), 0, stream, a, tilesX, tiles, workgroups)
                          : launch_kernel<image_difference_kernel<FORMAT, false>>(dim3(workgroups), dim3(256), 0, stream, a, tilesX, tiles, workgroups);
     };

@@ -160,6 +160,25 @@ def test_gpu_image_difference_matches_checker(ntc, device, oracle, fmt, channels
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("fmt", [1, 2, 3])
+@pytest.mark.parametrize("w,h,extent,thr", [(3, 16500, None, None), (1030, 3300, (5, 3, 1024, 3264), 0.5), (2051, 2050, None, None),
+                                            (259, 66000, (1, 1, 257, 65537), 0.5)])
+def test_gpu_image_difference_of_many_tiles(ntc, device, oracle, fmt, w, h, extent, thr):
+    """Pixels without padding: whole groups of four tiles, groups that the extent cuts off on either side, one and two
+    groups a workgroup and more groups than are resident."""
+    rng = np.random.default_rng(w + fmt)
+    dtype = {1: np.uint8, 2: np.uint16, 3: np.float16}[fmt]
+    a = rng.random((h, w, 4), dtype=np.float32)
+    b = np.clip(a + (rng.random((h, w, 4), dtype=np.float32) - 0.5) * 0.1, 0, 1)
+    raw_a, raw_b = [(x if fmt == 3 else np.rint(x * np.iinfo(dtype).max)).astype(dtype).reshape(-1).view(np.uint8) for x in (a, b)]
+    desc = (4 * BPC[fmt], 4 * BPC[fmt] * w, w, h, fmt, 4)
+    d_a, d_b = device.upload(raw_a), device.upload(raw_b)
+    extent = extent or (0, 0, w, h)
+    want = oracle_difference(ntc, oracle, raw_a, raw_b, desc, desc, extent, alpha_threshold=thr)
+    assert gpu_difference(ntc, device, d_a, d_b, desc, desc, extent, alpha_threshold=thr) == want
+
+
+@pytest.mark.gpu
 def test_gpu_image_difference_large_and_arguments(ntc, device, oracle):
     """4096 x 4096 RGBA8 against itself plus one changed pixel (exact result), and the argument checks."""
     w, h = 4096, 4096
