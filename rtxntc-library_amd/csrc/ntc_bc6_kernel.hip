@@ -661,10 +661,11 @@ bc6_compress_kernel(BlockCompressArgs a)
     int const bx = blockIdx.x * 8 + (lane & 7), by = blockIdx.y * 8 + (lane >> 3);
     bool const inside = bx < a.widthInBlocks && by < a.heightInBlocks;
     // a row of the block per wave; lanes outside encode black
+    float texels[1][4][3] = {};
+    if (inside) source_rows<3, 1>(a, a.srcLeft + bx * 4, a.srcTop + by * 4 + wave, 0, texels);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        float c[4] = { 0.f, 0.f, 0.f, 0.f };
-        if (inside) source_pixel(a, a.srcLeft + bx * 4 + i, a.srcTop + by * 4 + wave, c);
+        float const (&c)[3] = texels[0][i];
         shared.texels[4 * wave + i][lane] = make_float4(clampf(c[0], 0.f, kHalfMax), clampf(c[1], 0.f, kHalfMax), clampf(c[2], 0.f, kHalfMax), 0.f);
     }
     if (wave == 0) {

@@ -507,11 +507,12 @@ BC7_INLINE void bc7_encode_fixed(Color<4> const (&px)[16], int list, int mode, i
 
 BC7_INLINE void load_block(BlockCompressArgs const& a, int bx, int by, Color<4> (&px)[16])
 {
+    float values[4][4][4];
+    source_rows<4, 4>(a, a.srcLeft + bx * 4, a.srcTop + by * 4, 0, values);
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-        int const x = a.srcLeft + bx * 4 + (t & 3), y = a.srcTop + by * 4 + (t >> 2);
-        source_pixel(a, x, y, px[t].c);
-    }
+    for (int t = 0; t < 16; ++t)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) px[t].c[k] = values[t >> 2][t & 3][k];
 }
 BC7_INLINE void store_block(BlockCompressArgs const& a, int bx, int by, uint64_t lo, uint64_t hi)
 {
@@ -1442,10 +1443,11 @@ bc7_compress_kernel(BlockCompressArgs a)
         int const bx = block_x(b), by = block_y(b);
         bool const inside = bx < a.widthInBlocks && by < a.heightInBlocks;
         uint32_t alphas = 0;
+        float texels[1][4][4] = {};
+        if (inside) source_rows<4, 1>(a, a.srcLeft + bx * 4, a.srcTop + by * 4 + row, 0, texels);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            float c[4] = { 0.f, 0.f, 0.f, 0.f };
-            if (inside) source_pixel(a, a.srcLeft + bx * 4 + i, a.srcTop + by * 4 + row, c);
+            float const (&c)[4] = texels[0][i];
             alphas |= (c[3] < 1.f ? kBelowOne : 0u) | (c[3] != 1.f ? kNotOne : 0u);
             shared.texels[4 * row + i][b] = make_float4(c[0], c[1], c[2], c[3]);
         }
@@ -1590,9 +1592,11 @@ bc7_compress_kernel(BlockCompressArgs a)
 // into lists in LDS (the reference's ReorderThreadsByMode, CompressBC7.hlsl:1445-1509), then its waves take pieces of 64
 // blocks of one list each, the longest modes first, so that a wave runs one mode only (modes 4 and 5 are one piece of
 // code).  Sorting 256 blocks among as many threads left each wave with three or four modes: 2048 x 2048 blocks, modes 4 and
-// 5 on five blocks of six, took 86 us, with every block in one mode 27 to 50; now 51 us, from lists of 1024 blocks.  Images
-// of no more than 256 blocks per compute unit sort 256 (1024 x 1024: 31 us, 71 before).  Which lane encodes which block
-// depends on the order the LDS counters are hit in; what is written for a block does not.
+// 5 on five blocks of six, took 86 us, with every block in one mode 27 to 50; 50 us from lists of 1024 blocks, with a wave's
+// pixels loaded one after the other for a third of the time; 38.5 with all of them under way and the map's words loaded and
+// counted at once.  Images of no more than 256 blocks per compute unit sort 256 (1024 x 1024: 71 us before, 31, and 23.5).
+// What is left is 19 pieces for 12 waves, unequal ones.  Which lane encodes which block depends on the order the LDS counters
+// are hit in; what is written for a block does not.
 // Three waves per SIMD (168 registers) serve this kernel best.
 template <int SIDE, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES, 3)
@@ -1607,21 +1611,30 @@ bc7_compress_modes_kernel(BlockCompressArgs a)
     if (tid < LISTS) counts[tid] = 0;
     if (tid == LISTS) next = 0;
     __syncthreads();
-    for (int b = tid; b < (BLOCKS + THREADS - 1) / THREADS * THREADS; b += THREADS) {
-        int const bx = int(blockIdx.x) * SIDE + b % SIDE, by = int(blockIdx.y) * SIDE + b / SIDE;
+    // 9 bits per block of the mode map, which lie in one word or two; all loads before the first entry is looked at
+    constexpr int TURNS = (BLOCKS + THREADS - 1) / THREADS;
+    uint32_t words[TURNS][2];
+    uint32_t shifts[TURNS];
+    bool mapped[TURNS];
+    int64_t const lastWord = ((int64_t(a.modeMapWidthInBlocks) * a.modeMapHeightInBlocks * 9 + 31) >> 5) - 1;
+#pragma unroll
+    for (int turn = 0; turn < TURNS; ++turn) {
+        int const b = tid + turn * THREADS;
+        int64_t const mx = int64_t(blockIdx.x) * SIDE + b % SIDE + a.modeMapOffsetX, my = int64_t(blockIdx.y) * SIDE + b / SIDE + a.modeMapOffsetY;
+        mapped[turn] = mx >= 0 && my >= 0 && mx < a.modeMapWidthInBlocks && my < a.modeMapHeightInBlocks;
+        int64_t const bit = mapped[turn] ? (my * a.modeMapWidthInBlocks + mx) * 9 : 0;
+        words[turn][0] = a.modeBuffer[bit >> 5];
+        words[turn][1] = a.modeBuffer[min((bit >> 5) + 1, lastWord)];
+        shifts[turn] = uint32_t(bit & 31);
+    }
+#pragma unroll
+    for (int turn = 0; turn < TURNS; ++turn) {
+        int const b = tid + turn * THREADS, bx = int(blockIdx.x) * SIDE + b % SIDE, by = int(blockIdx.y) * SIDE + b / SIDE;
         int list = -1;
         uint32_t entry = 0;
         if (b < BLOCKS && bx < a.widthInBlocks && by < a.heightInBlocks) {
-            // 9 bits per block of the mode map; 0 = no entry, 0x1BF stands for mode 0 partition 0
-            int64_t const mx = int64_t(bx) + a.modeMapOffsetX, my = int64_t(by) + a.modeMapOffsetY;
-            if (mx >= 0 && my >= 0 && mx < a.modeMapWidthInBlocks && my < a.modeMapHeightInBlocks) {
-                uint64_t const bit = (uint64_t(my) * uint64_t(a.modeMapWidthInBlocks) + uint64_t(mx)) * 9u;
-                uint32_t const* words = a.modeBuffer + (bit >> 5);
-                uint32_t const shift = uint32_t(bit & 31u);
-                entry = words[0] >> shift;
-                if (shift > 23u) entry |= words[1] << (32u - shift);
-                entry &= 0x1FFu;
-            }
+            // 0 = no entry, 0x1BF stands for mode 0 partition 0
+            if (mapped[turn]) entry = uint32_t((uint64_t(words[turn][1]) << 32 | words[turn][0]) >> shifts[turn]) & 0x1FFu;
             if (entry == 0u) {
                 store_block(a, bx, by, 0x0001f00000f80004ull, 0x1f9e00003ff0001full);     // the reference's marker: black, red, green and blue squares
             } else {
@@ -1629,13 +1642,19 @@ bc7_compress_modes_kernel(BlockCompressArgs a)
                 list = int((0x46553120u >> (4u * (entry >> 6))) & 15u);
             }
         }
-        for (int l = 0; l < LISTS; ++l) {                    // one atomic per wave and list
-            uint64_t const mine = __ballot(list == l);
-            if (mine == 0) continue;
-            int at = 0;
-            if (lane == 0) at = atomicAdd(&counts[l], int(__popcll(mine)));
-            at = __builtin_amdgcn_readfirstlane(at);
-            if (list == l) tasks[l][at + int(__builtin_amdgcn_mbcnt_hi(uint32_t(mine >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(mine), 0u)))] = entry << 10 | uint32_t(b);
+        // one atomic per wave, a lane for each list
+        uint64_t ofList[LISTS];
+        int count = 0, at = 0;
+#pragma unroll
+        for (int l = 0; l < LISTS; ++l) {
+            ofList[l] = __ballot(list == l);
+            if (lane == l) count = int(__popcll(ofList[l]));
+        }
+        if (lane < LISTS && count) at = atomicAdd(&counts[lane], count);
+#pragma unroll
+        for (int l = 0; l < LISTS; ++l) {
+            int const start = __builtin_amdgcn_readlane(at, l);
+            if (list == l) tasks[l][start + int(__builtin_amdgcn_mbcnt_hi(uint32_t(ofList[l] >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(ofList[l]), 0u)))] = entry << 10 | uint32_t(b);
         }
     }
     __syncthreads();

@@ -484,3 +484,31 @@ def test_gpu_bc7_arguments(ntc, device, oracle):
     assert device.lib.ntc_hip_block_compress(p) == ntc.abi.ERR_INVALID_ARG
     p.modeMapWidthInBlocks = 8
     device.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt,stored,channels", [(1, 4, 4), (1, 8, 4), (1, 5, 4), (1, 3, 3), (1, 1, 1), (2, 4, 4), (3, 3, 3), (3, 4, 4), (4, 4, 4), (5, 2, 2)])
+@pytest.mark.parametrize("w,h,left,top", [(1, 1, 0, 0), (3, 9, 0, 0), (4, 4, 0, 0), (7, 6, 2, 1), (22, 13, 3, 2)])
+def test_gpu_blocks_at_the_image_edges(ntc, device, oracle, fmt, stored, channels, w, h, left, top):
+    """Blocks that the image cuts off or does not reach, in images narrower than a block, from pixels of every format with and
+    without padding: what the kernels' row loads read and replace."""
+    rng = np.random.default_rng(700 + fmt + stored + w)
+    dtype = {1: np.uint8, 2: np.uint16, 3: np.float16, 4: np.float32, 5: np.uint32}[fmt]
+    image = rng.random((h, w, stored)) if fmt in (3, 4) else rng.integers(0, {1: 256, 2: 65536, 5: 2}[fmt], (h, w, stored))
+    image = image.astype(dtype)
+    bx, by = (w + 3) // 4 + 1, (h + 3) // 4 + 1
+    for dst in (1, 2, 3, 4, 5, 6, 7):
+        want = compress(ntc, oracle, None, image, fmt, channels, dst, bx, by, left, top)
+        got = compress(ntc, None, device, image, fmt, channels, dst, bx, by, left, top)
+        assert np.array_equal(got, want), (dst, np.argwhere(got != want)[:3])
+    modes = rng.integers(0, 8, bx * by)
+    entries = [entry_of(m, {4: 6, 5: 2, 6: 0}.get(int(m), 5)) for m in modes]
+    kw = dict(mode_buffer=pack_mode_buffer(entries), left=left, top=top)
+    want = compress_bc7(ntc, oracle, None, image, fmt, channels, bx, by, **kw)
+    assert np.array_equal(compress_bc7(ntc, None, device, image, fmt, channels, bx, by, **kw), want)
+    if w == 22:
+        # so many blocks that each is one lane's
+        for dst in (1, 2, 3):
+            want = compress(ntc, oracle, None, image, fmt, channels, dst, 16 * 41, 4 * 32, left, top)
+            got = compress(ntc, None, device, image, fmt, channels, dst, 16 * 41, 4 * 32, left, top)
+            assert np.array_equal(got, want), (dst, np.argwhere(got != want)[:3])
