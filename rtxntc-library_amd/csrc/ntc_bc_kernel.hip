@@ -64,7 +64,8 @@ __device__ __forceinline__ void bc4_palette8(uint32_t e0, uint32_t e1, uint32_t 
 
 // Nearest palette entry for every texel (the first of equally near ones); returns the summed squared error.
 // values8: the texels times eight, so that |value - entry| * 8 + k is one instruction per entry: the smallest of these
-// keys is the nearest entry, the first among equally near ones.  keys: the chosen ones.
+// keys is the nearest entry, the first among equally near ones.  keys: the chosen ones.  (Sums of 16-bit differences: of a
+// 32-bit one with k = 0 the compiler makes a maximum, a minimum and a difference.)
 __device__ __forceinline__ uint32_t bc4_assign(uint32_t const (&values8)[16], Bc4& block, uint32_t (&keys)[16])
 {
     uint32_t p[8];
@@ -75,7 +76,7 @@ __device__ __forceinline__ uint32_t bc4_assign(uint32_t const (&values8)[16], Bc
     for (int t = 15; t >= 0; --t) {
         uint32_t key[8];
 #pragma unroll
-        for (uint32_t k = 0; k < 8; ++k) key[k] = __usad(values8[t], p[k], k);
+        for (uint32_t k = 0; k < 8; ++k) key[k] = __builtin_amdgcn_sad_u16(values8[t], p[k], k);
         uint32_t const best = min3_u32(min3_u32(key[0], key[1], key[2]), min3_u32(key[3], key[4], key[5]), min(key[6], key[7]));
         uint32_t const distance = best >> 3;
         total += __umul24(distance, distance);               // at most 16 * 255^2: exact as the float sum it stands for
@@ -99,7 +100,7 @@ __device__ __forceinline__ void bc4_refit(uint32_t const (&values8)[16], uint32_
     float aa = 0.f, bb = 0.f, ab = 0.f, ax = 0.f, bx = 0.f;
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
-        uint32_t const select = (keys[t] & 7u) | 0x0c0c0c00u;                    // upper bytes: zero
+        uint32_t const select = keys[t] & 7u;                                    // (only the lowest byte of the permute is looked at)
         float alpha, beta;
         if constexpr (EIGHT) {
             float const w = float(__builtin_amdgcn_perm(0x01020304u, 0x05060007u, select) & 0xffu);
@@ -108,7 +109,7 @@ __device__ __forceinline__ void bc4_refit(uint32_t const (&values8)[16], uint32_
         } else {
             float const w = float(__builtin_amdgcn_perm(0x00000102u, 0x03040005u, select) & 0xffu);
             alpha = w * (1.f / 5.f);
-            beta = (keys[t] & 7u) >= 6u ? 0.f : 1.f - alpha;                     // adding zeros is leaving the texel out
+            beta = select >= 6u ? 0.f : 1.f - alpha;                     // adding zeros is leaving the texel out
         }
         float const x = float(values8[t] >> 3);
         aa += alpha * alpha; bb += beta * beta; ab += alpha * beta;
@@ -188,18 +189,28 @@ __device__ __forceinline__ void bc4_load(BlockCompressArgs const& a, int bx, int
         // UNORM8 pixels without padding, the whole block inside the image: a row of four is four dwords at most, and
         // a code is its own value (rint(code / 255 * 255) = code)
         uint8_t const* px = a.src + size_t(y0) * a.rowPitch + size_t(x0) * a.pixelStride + size_t(c);
+        auto const rows = [&](auto load) {                   // all of them under way before the first is looked at
+            uint32_t words[4][4];
 #pragma unroll
-        for (int y = 0; y < 4; ++y, px += a.rowPitch) {
-            uint32_t words[4];
-            if (a.pixelStride == 1) {                        // uniform; the image has no channel 1
-                uint32_t const v = c == 0 ? *reinterpret_cast<u32_unaligned const*>(px) : 0u;
+            for (int y = 0; y < 4; ++y) load(px + size_t(y) * a.rowPitch, words[y]);
+#pragma unroll
+            for (int t = 0; t < 16; ++t) values8[t] = (words[t >> 2][t & 3] & 0xffu) << 3;
+        };
+        if (a.pixelStride == 1) {                            // uniform; the image has no channel 1
+            rows([&](uint8_t const* row, uint32_t (&words)[4]) {
+                uint32_t const v = c == 0 ? *reinterpret_cast<u32_unaligned const*>(row) : 0u;
                 words[0] = v; words[1] = v >> 8; words[2] = v >> 16; words[3] = v >> 24;
-            } else {
+            });
+        } else if (a.pixelStride == 2) {
+            rows([&](uint8_t const* row, uint32_t (&words)[4]) {
+                u32x2_unaligned const v = *reinterpret_cast<u32x2_unaligned const*>(row - c);
+                words[0] = v[0] >> (8 * c); words[1] = v[0] >> (8 * c + 16); words[2] = v[1] >> (8 * c); words[3] = v[1] >> (8 * c + 16);
+            });
+        } else {
+            rows([&](uint8_t const* row, uint32_t (&words)[4]) {
 #pragma unroll
-                for (int x = 0; x < 4; ++x) words[x] = px[size_t(x) * a.pixelStride];
-            }
-#pragma unroll
-            for (int x = 0; x < 4; ++x) values8[4 * y + x] = (words[x] & 0xffu) << 3;
+                for (int x = 0; x < 4; ++x) words[x] = row[size_t(x) * a.pixelStride];
+            });
         }
     } else {
         float texels[4][4][1];
@@ -520,10 +531,11 @@ __device__ __forceinline__ uint64_t bc2_alpha(float const (&alpha)[16])
 // A wave encodes one channel of 64 blocks (16 x 4) with one palette, so that the palettes' refinements, each a chain of
 // up to nine passes over the texels, run side by side and not one after the other: a workgroup is the two palettes of
 // both channels of 64 blocks (BC5) or of one channel of 128 (BC4).  The waves of the six-value palette leave their
-// candidates in LDS for those of the eight-value one to choose from.  2048 x 2048: BC5 66 us, BC4 36 (136 and 67 with one
-// lane per block and all of its channels and palettes, two to three instructions per palette entry and the weights from
-// memory);
-// 64 x 64: 10 and 9 us, 54 and 29 before.
+// candidates in LDS for those of the eight-value one to choose from.  Bound by vector issue.  2048 x 2048: BC5 58 us, BC4 34
+// (136 and 67 with one lane per block and all of its channels and palettes, two to three instructions per palette entry and
+// the weights from memory; 64 and 36.8 with three instructions for an entry's distance where its number is 0);
+// 64 x 64: 8.7 and 8.5 us (54 and 29).  Three waves per SIMD more at the price of spills, or the indices without registers
+// of their own, are slower (61 to 69 and 35 to 40).
 template <int CHANNELS>
 __global__ void __launch_bounds__(256)
 bc4_compress_kernel(BlockCompressArgs a)

@@ -8,6 +8,7 @@
 namespace ntc_hip_dev {
 
 typedef uint32_t __attribute__((aligned(1))) u32_unaligned;
+typedef uint32_t u32x2_unaligned __attribute__((ext_vector_type(2), aligned(1)));
 
 // fminf / fmaxf as single instructions.  The compiler brackets the library functions with two
 // canonicalising instructions (it cannot know that its operands are already quiet); v_min_f32 /
