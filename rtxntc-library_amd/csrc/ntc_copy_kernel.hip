@@ -1716,7 +1716,7 @@ template <int CONTROL> __device__ __forceinline__ float add_rotated(float v)
 }
 template <int FORMAT, int TEAMS>
 __global__ void __launch_bounds__(256 * TEAMS, 4)
-image_difference_wide_kernel(ImageDifferenceArgs a, int groupsX, int groups)
+image_difference_wide_kernel(ImageDifferenceArgs a, int groupsX, int groups, int step)
 {
     constexpr int BPC = bytes_per_channel(FORMAT), ROWS = 4 / BPC;
     __shared__ float sums[2][TEAMS][4][16];                  // [turn][team][part][4 * tile + channel]
@@ -1725,7 +1725,7 @@ image_difference_wide_kernel(ImageDifferenceArgs a, int groupsX, int groups)
     float const threshold = a.useAlphaThreshold ? a.alphaThreshold : -__builtin_inff();
     unsigned long long fixed = 0;                            // threads 0 ... 15: the workgroup's share of a channel's sum, of the nth tiles
     int turn = 0;
-    for (int base = blockIdx.x * TEAMS; base < groups; base += gridDim.x * TEAMS, turn ^= 1) {
+    for (int base = blockIdx.x * TEAMS; base < groups; base += step, turn ^= 1) {
         int const group = base + team;                       // (beyond the last one: below the extent, nothing is read)
         int const groupY = group / groupsX, groupX = group - groupY * groupsX;
         int const x = groupX * 256 + lane * 4, y = groupY * 64 + wave * 16;
@@ -1836,8 +1836,8 @@ hipError_t launch_image_difference(ImageDifferenceArgs const& a, hipStream_t str
             int const groupsX = (a.width + 255) / 256, groups = groupsX * ((a.height + 63) / 64);
             // (with fewer groups of tiles than compute units the other kernel's are more waves: 2048 x 1024 11.2 us)
             if (!a.useMSLE && groups >= compute_units_of_current_device() && a.a.pixelStride == PIXEL && a.b.pixelStride == PIXEL)
-                return groups < resident ? launch_kernel<image_difference_wide_kernel<FORMAT, 1>>(dim3(groups), dim3(256), 0, stream, a, groupsX, groups)
-                                         : launch_kernel<image_difference_wide_kernel<FORMAT, 2>>(dim3(resident / 2), dim3(512), 0, stream, a, groupsX, groups);
+                return groups < resident ? launch_kernel<image_difference_wide_kernel<FORMAT, 1>>(dim3(groups), dim3(256), 0, stream, a, groupsX, groups, groups)
+                                         : launch_kernel<image_difference_wide_kernel<FORMAT, 2>>(dim3(resident / 2), dim3(512), 0, stream, a, groupsX, groups, resident);
         }
         return a.useMSLE ? launch_kernel<image_difference_kernel<FORMAT, true>>(dim3(workgroups), dim3(256), 0, stream, a, tilesX, tiles, workgroups)
                          : launch_kernel<image_difference_kernel<FORMAT, false>>(dim3(workgroups), dim3(256), 0, stream, a, tilesX, tiles, workgroups);
