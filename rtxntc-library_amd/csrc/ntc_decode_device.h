@@ -152,12 +152,16 @@ __device__ __forceinline__ void load_cells(uint16_t const* grid, int gridWidth, 
 
 // Four 4-bit features of the four taps, filtered.  A cell c = f0 | f1<<4 | f2<<8 | f3<<12: its bytes masked with 0x0f are
 // features 0 and 2, masked with 0xf0 sixteen times features 1 and 3, so t[1] and t[3] come out sixteen times as large,
-// with the same roundings.
+// with the same roundings.  (The compiler takes that apart again, five instructions a cell for two: 1920 x 1080 decoded in
+// 101 us instead of 97.6, 1800 x 1100 by the FP8 network in 103 instead of 98.)
 __device__ __forceinline__ void filter4(FloatTaps const& tp, uint32_t const (&cells)[4], float (&t)[4])
 {
     uint32_t even[4], odd[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) { even[k] = cells[k] & 0x0f0fu; odd[k] = cells[k] & 0xf0f0u; }
+    for (int k = 0; k < 4; ++k) {
+        even[k] = cells[k] & 0x0f0fu; odd[k] = cells[k] & 0xf0f0u;
+        asm volatile("" : "+v"(even[k]), "+v"(odd[k]));
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         uint32_t const (&q)[4] = (i & 1) ? odd : even;
