@@ -1325,24 +1325,45 @@ __device__ __forceinline__ double add_from_row(double v)
     return v + __builtin_bit_cast(double, uint64_t(high) << 32 | low);
 }
 
-// A workgroup's sums, channel threadIdx.x's in `mine` of the threads 0 ... 15, on their way to the host.
-__device__ __forceinline__ void hand_over_sums(double mine, uint32_t validChannelMask, uint32_t block, uint32_t blocks, uint32_t groupSize, LossWorkspace const& work)
+// The sums of 256 lanes' 16 accumulators and their way to the host.  Across the workgroup: 16 threads per channel add 16 of
+// its 256 values each, then each other's.  (With exchanges between lanes, 17 of a double and 1500 instructions when every
+// lane hands over half of what it holds at a step, this took 1 us longer.)
+__device__ __forceinline__ void hand_over_sums(double const (&acc)[NTC_HIP_DEV_MAX_CHANNELS], int setChannels, uint32_t validChannelMask,
+                                               uint32_t block, uint32_t blocks, uint32_t groupSize, LossWorkspace const& work)
 {
-    if (!((validChannelMask >> (threadIdx.x & 31u)) & 1u)) mine = 0.0;
+    constexpr int STRIDE = 256 + 16;                         // (channels half the banks apart)
+    __shared__ double lanes[NTC_HIP_DEV_MAX_CHANNELS * STRIDE];
+    __shared__ double sums[NTC_HIP_DEV_MAX_CHANNELS];
+    int const lane = threadIdx.x & 63;
+#pragma unroll
+    for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) lanes[c * STRIDE + int(threadIdx.x)] = acc[c];
+    __syncthreads();
+    int const channel = int(threadIdx.x) >> 4, part = int(threadIdx.x) & 15;
+    double mine = 0.0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) mine += lanes[channel * STRIDE + part + 16 * k];
+    mine = add_from_row<0xB1>(mine);                         // quad_perm: the neighbour,
+    mine = add_from_row<0x4E>(mine);                         // the other pair,
+    mine = add_from_row<0x141>(mine);                        // row_half_mirror: the other quad,
+    mine = add_from_row<0x140>(mine);                        // row_mirror: the other eight
+    if (channel >= setChannels || !((validChannelMask >> channel) & 1u)) mine = 0.0;
     uint32_t const group = block / groupSize, first = group * groupSize, members = min(groupSize, blocks - first);
-    double total = mine;                                     // threads 0 ... 15: a channel's each
+    double total;                                            // threads 0 ... 15: a channel's each
     if (members > 1) {
         __shared__ double scratch[16][NTC_HIP_DEV_MAX_CHANNELS];
         __shared__ int last;
-        if (threadIdx.x < NTC_HIP_DEV_MAX_CHANNELS) publish(work.partials + size_t(block) * NTC_HIP_DEV_MAX_CHANNELS + threadIdx.x, mine);
+        if (part == 0) publish(work.partials + size_t(block) * NTC_HIP_DEV_MAX_CHANNELS + channel, mine);
         if (!arrived_last(work.counters + group * kLossCounterStride, members, last)) return;
         total = sum_entries(work.partials + size_t(first) * NTC_HIP_DEV_MAX_CHANNELS, int(members), scratch);
+    } else {
+        if (part == 0) sums[channel] = mine;
+        __syncthreads();
+        total = sums[threadIdx.x & (NTC_HIP_DEV_MAX_CHANNELS - 1)];
     }
     // To the host in one trip: each half of a double is stored together with the serial number, so that every word
     // says for itself whether it has arrived.  Stores of system scope go past the caches.  (Plain stores and a release
     // behind them write back the die's whole L2.)
     if (threadIdx.x >= 64) return;
-    int const lane = int(threadIdx.x);
     uint64_t const sum = __builtin_bit_cast(uint64_t, __shfl(total, lane >> 1, 64));
     uint64_t const word = uint64_t(work.serial) << 32 | ((lane & 1) ? sum >> 32 : sum & 0xffffffffu);
     if (lane < 2 * NTC_HIP_DEV_MAX_CHANNELS)
@@ -1358,30 +1379,6 @@ template <int SHIFT> __device__ __forceinline__ float two_squares(uint32_t a0, u
     s += d0 * d0;
     s += d1 * d1;
     return s;
-}
-
-// The sums of 256 lanes' 16 accumulators, channel threadIdx.x's in the threads 0 ... 15: 16 threads per channel add 16 of its
-// 256 values each, then each other's.  (With exchanges between lanes, 17 of a double and 1500 instructions when every lane
-// hands over half of what it holds at a step, this took 1 us longer.)
-__device__ __forceinline__ double sum_of_lanes(double const (&acc)[NTC_HIP_DEV_MAX_CHANNELS], int setChannels)
-{
-    constexpr int STRIDE = 256 + 16;                         // (channels half the banks apart)
-    __shared__ double lanes[NTC_HIP_DEV_MAX_CHANNELS * STRIDE];
-    __shared__ double sums[NTC_HIP_DEV_MAX_CHANNELS];
-#pragma unroll
-    for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) lanes[c * STRIDE + int(threadIdx.x)] = acc[c];
-    __syncthreads();
-    int const channel = int(threadIdx.x) >> 4, part = int(threadIdx.x) & 15;
-    double mine = 0.0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) mine += lanes[channel * STRIDE + part + 16 * k];
-    mine = add_from_row<0xB1>(mine);                         // quad_perm: the neighbour,
-    mine = add_from_row<0x4E>(mine);                         // the other pair,
-    mine = add_from_row<0x141>(mine);                        // row_half_mirror: the other quad,
-    mine = add_from_row<0x140>(mine);                        // row_mirror: the other eight
-    if (part == 0) sums[channel] = channel < setChannels ? mine : 0.0;
-    __syncthreads();
-    return sums[threadIdx.x & (NTC_HIP_DEV_MAX_CHANNELS - 1)];
 }
 
 // Without a mask channel.  The internal layout is row after row of channel pairs, so that whole rows are one piece of memory,
@@ -1458,15 +1455,15 @@ image_loss_kernel(uint16_t const* __restrict__ a, uint16_t const* __restrict__ b
             }
         }
     }
-    hand_over_sums(sum_of_lanes(acc, setChannels), validChannelMask, blockIdx.x, blocks, groupSize, work);
+    hand_over_sums(acc, setChannels, validChannelMask, blockIdx.x, blocks, groupSize, work);
 }
 
-// With a mask channel, or (maskChannel < 0) for images that the other kernel does not take.  A lane takes PX adjacent texels
+// With a mask channel, or without one for images that the other kernel does not take.  A lane takes PX adjacent texels
 // (2 when the width is even: 8-byte loads) of rowsPerWave rows, all pairs of them together, because every channel counts by the mask's, and all
 // loads of a row are issued before its arithmetic.
-template <int PX>
+template <int PX, bool MASKED>
 __global__ void __launch_bounds__(256)
-masked_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int width, int height, int setChannels, int rowsPerWave,
+texel_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int width, int height, int setChannels, int rowsPerWave,
                    uint32_t validChannelMask, int maskChannel, int discardMaskedOut, uint32_t gridX, uint32_t blocks, uint32_t groupSize, LossWorkspace work)
 {
     constexpr int PAIRS = NTC_HIP_DEV_MAX_CHANNELS / 2;
@@ -1495,14 +1492,16 @@ masked_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int
             }
         }
         __builtin_amdgcn_sched_barrier(0);                   // keep the loads ahead of the arithmetic
-        bool maskedOut[PX];
+        [[maybe_unused]] bool maskedOut[PX];
+        if constexpr (MASKED) {
 #pragma unroll
-        for (int k = 0; k < PX; ++k) maskedOut[k] = false;
+            for (int k = 0; k < PX; ++k) maskedOut[k] = false;
 #pragma unroll
-        for (int p = 0; p < PAIRS; ++p) {
-            if ((maskChannel >> 1) != p || !discardMaskedOut) continue;              // uniform
+            for (int p = 0; p < PAIRS; ++p) {
+                if ((maskChannel >> 1) != p || !discardMaskedOut) continue;          // uniform
 #pragma unroll
-            for (int k = 0; k < PX; ++k) maskedOut[k] = (((maskChannel & 1) ? vb[p][k] >> 16 : vb[p][k]) & 0x7FFFu) == 0;
+                for (int k = 0; k < PX; ++k) maskedOut[k] = (((maskChannel & 1) ? vb[p][k] >> 16 : vb[p][k]) & 0x7FFFu) == 0;
+            }
         }
 #pragma unroll
         for (int p = 0; p < PAIRS; ++p) {
@@ -1511,17 +1510,21 @@ masked_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int
             for (int k = 0; k < PX; ++k) {
                 float a0 = float(__builtin_bit_cast(_Float16, uint16_t(va[p][k])));
                 float a1 = float(__builtin_bit_cast(_Float16, uint16_t(va[p][k] >> 16)));
-                if ((maskChannel >> 1) == p) {                  // uniform; the mask channel is below setChannels
-                    if (maskChannel & 1) a1 = a1 > 0.f ? fminf(a1, 1.f) : 0.f;
-                    else                 a0 = a0 > 0.f ? fminf(a0, 1.f) : 0.f;
-                    uint32_t const clamped = uint32_t(__builtin_bit_cast(uint16_t, _Float16(a0)))
-                                           | uint32_t(__builtin_bit_cast(uint16_t, _Float16(a1))) << 16;
-                    if (clamped != va[p][k]) *reinterpret_cast<uint32_t*>(a + base + size_t(2 * p) * size_t(width) + size_t(2 * k)) = clamped;
+                if constexpr (MASKED) {
+                    if ((maskChannel >> 1) == p) {              // uniform; the mask channel is below setChannels
+                        if (maskChannel & 1) a1 = a1 > 0.f ? fminf(a1, 1.f) : 0.f;
+                        else                 a0 = a0 > 0.f ? fminf(a0, 1.f) : 0.f;
+                        uint32_t const clamped = uint32_t(__builtin_bit_cast(uint16_t, _Float16(a0)))
+                                               | uint32_t(__builtin_bit_cast(uint16_t, _Float16(a1))) << 16;
+                        if (clamped != va[p][k]) *reinterpret_cast<uint32_t*>(a + base + size_t(2 * p) * size_t(width) + size_t(2 * k)) = clamped;
+                    }
                 }
                 float d0 = a0 - float(__builtin_bit_cast(_Float16, uint16_t(vb[p][k])));
                 float d1 = a1 - float(__builtin_bit_cast(_Float16, uint16_t(vb[p][k] >> 16)));
-                if (maskedOut[k] && maskChannel != 2 * p) d0 = 0.f;
-                if (maskedOut[k] && maskChannel != 2 * p + 1) d1 = 0.f;
+                if constexpr (MASKED) {
+                    if (maskedOut[k] && maskChannel != 2 * p) d0 = 0.f;
+                    if (maskedOut[k] && maskChannel != 2 * p + 1) d1 = 0.f;
+                }
                 s0 += d0 * d0;
                 s1 += d1 * d1;
             }
@@ -1529,7 +1532,7 @@ masked_loss_kernel(uint16_t* __restrict__ a, uint16_t const* __restrict__ b, int
             acc[2 * p + 1] += double(s1);
         }
     }
-    hand_over_sums(sum_of_lanes(acc, setChannels), validChannelMask, blockIdx.y * gridX + blockIdx.x, blocks, groupSize, work);
+    hand_over_sums(acc, setChannels, validChannelMask, blockIdx.y * gridX + blockIdx.x, blocks, groupSize, work);
 }
 
 hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int height, int setChannels, uint32_t validChannelMask,
@@ -1542,13 +1545,14 @@ hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int heig
     int log2Lanes = 0;
     while (log2Lanes < 8 && (4 << log2Lanes) < width) ++log2Lanes;
     uint32_t const together = 256u >> log2Lanes, rows = ((uint32_t(height) + blocks - 1u) / blocks + together - 1u) / together * together;
-    // The masked kernel's too are rows of less than four texels, each loaded alone (1 x 1 13.2 us, 11.5 the other way), rows
-    // beyond 31 bits of offsets, and wide images of few rows, which leave most workgroups none (16
-    // channels, 16384 x 1 30 us, 15.6 the other way; 8192 x 8 22 and 16.5; 4096 x 64 19.5 and 17.1; 2048 x 128, twice the even
-    // share, 17.5 and 17.7)
+    // The other kernel's are images of less than 131072 texels, a trip to memory or two for a workgroup, which it makes with
+    // all pairs' loads at once and without a tail of a row (300 x 200 and 150 x 100 of 16 channels 15.5 and 15.2 us, 17.1 and
+    // 20.4 by whole rows; 400 x 300 16.3 and 17.7, 512 x 512 18.5 and 16.5); rows of less than four texels; rows beyond 31 bits
+    // of offsets; and wide images of few rows, which leave most workgroups none (16384 x 1 30 us, 15.6 the other way;
+    // 8192 x 8 22 and 16.5; 4096 x 64 19.5 and 17.1; 2048 x 128, twice the even share, 17.5 and 17.7).
     uint64_t const share = uint64_t(rows) * uint64_t(width), even = uint64_t(width) * uint64_t(height) / blocks;
     bool const shared = share <= 2u * (even < 1024u ? 1024u : even);
-    if (maskChannel < 0 && width >= 4 && shared && share * uint64_t(setChannels) * 2u < 0x80000000u) {
+    if (maskChannel < 0 && width >= 4 && uint64_t(width) * uint64_t(height) >= 131072u && shared && share * uint64_t(setChannels) * 2u < 0x80000000u) {
         auto launch = [&](auto steps, auto pairs) {
             return launch_kernel_with_event<image_loss_kernel<decltype(steps)::value, decltype(pairs)::value>>(dim3(blocks), dim3(256), 0, stream, done,
                                          a, b, width, height, setChannels, int(rows), log2Lanes, validChannelMask, blocks, grid.groupSize, work);
@@ -1558,11 +1562,12 @@ hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int heig
         if (width >= 2048) return launch(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});
         return launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 4>{});
     }
-    auto launch = [&](auto perLane) {
-        return launch_kernel_with_event<masked_loss_kernel<decltype(perLane)::value>>(dim3(grid.x, grid.y), dim3(256), 0, stream, done,
+    auto launch = [&](auto perLane, auto masked) {
+        return launch_kernel_with_event<texel_loss_kernel<decltype(perLane)::value, decltype(masked)::value>>(dim3(grid.x, grid.y), dim3(256), 0, stream, done,
                                      a, b, width, height, setChannels, grid.rowsPerWave, validChannelMask, maskChannel, discardMaskedOut, grid.x, blocks, grid.groupSize, work);
     };
-    return (width & 1) == 0 ? launch(std::integral_constant<int, 2>{}) : launch(std::integral_constant<int, 1>{});
+    auto of_width = [&](auto perLane) { return maskChannel >= 0 ? launch(perLane, std::true_type{}) : launch(perLane, std::false_type{}); };
+    return (width & 1) == 0 ? of_width(std::integral_constant<int, 2>{}) : of_width(std::integral_constant<int, 1>{});
 }
 
 // ---- image difference (src/shaders/ImageDifference.hlsl) -------------------------------------------

@@ -137,11 +137,11 @@ def test_loss_sums_of_one_group_and_of_many(ntc, device, oracle, w, h):
     assert np.allclose(results[0], want, rtol=2e-7, atol=0) and np.array_equal(results[0], results[1])
 
 
-@pytest.mark.parametrize("w,h,channels", [(3, 9, 2), (4, 1001, 16), (7, 777, 2), (255, 130, 14), (1023, 37, 10), (1029, 1030, 6), (2050, 601, 4),
-                                          (3071, 2, 16), (4099, 1100, 2), (8192, 3, 6)])
+@pytest.mark.parametrize("w,h,channels", [(3, 50000, 2), (4, 40001, 16), (7, 20777, 2), (255, 530, 14), (1023, 137, 10), (1029, 1030, 6), (2050, 601, 4),
+                                          (361, 363, 8), (4099, 1100, 2), (65536, 3, 2)])
 def test_loss_sums_of_whole_rows(ntc, device, oracle, w, h, channels):
     """Rows of one, two and more steps of the workgroup's lanes with what is left of them, several rows a workgroup's lanes
-    take together, fewer pairs than are loaded together, and images that fall to the masked kernel."""
+    take together, fewer pairs than are loaded together, and images that fall to the other kernel."""
     rng = np.random.default_rng(w * h)
     a, b = halves(rng, w * h * channels), halves(rng, w * h * channels)
     d_a, d_b = device.upload(a), device.upload(b)
