@@ -1381,10 +1381,10 @@ template <int SHIFT> __device__ __forceinline__ float two_squares(uint32_t a0, u
     return s;
 }
 
-// Without a mask channel.  The internal layout is row after row of channel pairs, so that whole rows are one piece of memory,
+// Large images without a mask channel.  The internal layout is row after row of channel pairs, so that whole rows are one piece of memory,
 // which the workgroup goes through in order, 4 KB of each image a load; STEPS of a pair's row and PAIRS pairs are under way
 // together, eight loads a lane (sixteen do not leave the registers for four waves per SIMD).  Bound by memory for large
-// mips, by the launch and the way to the host for small ones.  Whole calls of 16 channels, 4096 x 4096, 2048 x 2048, 1024 x
+// mips, by the launch and the way to the host below 512 x 512.  Whole calls of 16 channels, 4096 x 4096, 2048 x 2048, 1024 x
 // 1024 and 512 x 512: 189, 51, 23 and 16.5 us; 197, 56, 29 and 18.5 with 8-byte loads of all pairs by lanes of two texels,
 // and the groups' counters on one line (6 channels: 80, 28, 16.5 and 15.5; 111, 37, 25 and 18); 209, 51, 30 and 26 with a
 // wave for each pair, whose rows lie a power of two apart.  A kernel that does nothing but read the two images of 16

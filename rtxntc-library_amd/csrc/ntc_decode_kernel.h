@@ -117,10 +117,11 @@ struct WriteChannelsArgs {
 };
 hipError_t launch_write_channels(WriteChannelsArgs const& args, hipStream_t stream);
 
-// Grid of the loss kernels.  With a mask channel a workgroup (= one row of 16 double partial sums) covers 64 lanes x 1 or 2
-// texels (2 when the width is even) by 4 waves x rowsPerWave rows; without one as many workgroups divide the image by whole rows.  Four workgroups are resident on a compute unit; as
-// many rows per wave as make the grid about that large (every workgroup ends in 16 reductions across its lanes, and a
-// row is a memory round trip), from one, for images that would not fill the GPU, to 32.
+// Grid of the loss kernels: a workgroup (= one row of 16 double partial sums) covers 64 lanes x 1 or 2 texels (2 when the
+// width is even) by 4 waves x rowsPerWave rows; large images without a mask channel are divided among as many workgroups by
+// whole rows.  Four workgroups are resident on a compute unit; as many rows per wave as make the grid about that large (every
+// workgroup ends in 16 reductions across its lanes, and a row is a memory round trip), from one, for images that would not
+// fill the GPU, to 32.
 constexpr uint32_t kLossRows = 32;                          // groups of workgroups, each of which hands its sums to the host
 // Counters of the groups' workgroups lie 256 bytes apart: on one line a thousand arrivals wait for each other.
 constexpr uint32_t kLossCounterStride = 64;
