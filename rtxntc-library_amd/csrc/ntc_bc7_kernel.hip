@@ -625,7 +625,13 @@ template <int C> BC7_INLINE float inverse_square(Color<C> const& axis) { float c
 // add up to less than 42 T, T the sum of the block's squared offsets (|h|^2 and the squared mean are at most the subset's
 // share of T, and a subset has at most 13 texels), and none passes through more than 34 roundings: together less than
 // 1100 units of roundoff of T.  kBoundError, of 2048 units, is taken off each bound.
-constexpr float kBoundError = 0x1p-13f;
+// The other 948 units, more than 2^-63 because T is at least kLeastOffsets, are for what does not shrink with T:
+//  * products that round among subnormal numbers, by up to 2^-150.  Those that end a M a, five of a subset at most, are
+//    multiplied by 1 / (|a|^2 + kLeastLength), at most 2^72: together less than 2^-74.  All others are multiplied by a
+//    component of a as well, which leaves 2^36 of an offset at most, or by no more than offsets.
+//  * kLeastLength itself, which makes (a M a) / |a|^2 too small by up to kLeastLength / |a|^2 of it: by 13 / 4 of
+//    kLeastLength in a subset, because no texel is further from h than |a| / 2; together less than 2^-68.
+constexpr float kBoundError = 0x1p-13f, kLeastLength = 0x1p-72f;
 // Which components' ends trade places depends on the covariances' signs as orient_by() finds them.  Where one could be
 // 0 within the errors of either evaluation (texel by texel about a rounded mean, which is off by 16 units of roundoff of
 // the texels' size; by sums here, off by 100 units of T), the nearest of the four diagonals counts.
@@ -633,7 +639,8 @@ constexpr float kUnsureOfOffsets = 0x1p-16f, kUnsureOfTexels = 0x1p-35f;
 // Bounds are kept as codes of eight bits: errors over T, four bits of the exponent (2^-16 ... 1) and four of the mantissa,
 // rounded down.  Blocks whose T is no number between these have no bounds, and all of their partitions are estimated.
 constexpr float kNearLine = 1.f / 64.f;                      // squared distances over the squared diagonal; eight points leave 16 / 588 of it
-constexpr float kLeastOffsets = 0x1p-60f, kMostOffsets = 0x1p60f;
+// (The least T of halves that are not all equal is 2^-48.)
+constexpr float kLeastOffsets = 0x1p-48f, kMostOffsets = 0x1p60f;
 BC7_INLINE uint32_t error_code(float error, float scale)
 {
     constexpr uint32_t first = (127u - 16u) << 4;
@@ -732,7 +739,7 @@ BC7_INLINE void add_distances(float n, Sums<C> const& sums, Color<C> const& lo, 
 {
     Color<C> const a = sub(hi, lo);
     Color<C> middle2, w;
-    float length = 0x1p-100f;
+    float length = kLeastLength;
 #pragma unroll
     for (int k = 0; k < C; ++k) {
         middle2.c[k] = lo.c[k] + hi.c[k];

@@ -426,8 +426,9 @@ def test_gpu_bc7_opaque_blocks_whose_alpha_is_not_one_match_checker(ntc, device,
 def image_for_bounds(rng, content, w, h):
     """RGBA float32, a quarter of the blocks with alpha.  Which of the search's ways the partitions' errors take: "noise" a
     few estimates beyond the first; "edges" more than the queues hold; "grey" no bounds, because channels are proportional;
-    "level" subsets that are level in channels; "faint" covariances whose signs are within their errors; "tiny" and "huge"
-    texels' offsets outside the range that has bounds."""
+    "level" subsets that are level in channels; "faint" covariances whose signs are within their errors; "specks" every eighth
+    block a first texel of 2^-24 ... 2^-27 among others of 2^-47 ... 2^-51, whose products are near the least of floats; "tiny"
+    and "huge" texels' offsets outside the range that has bounds."""
     ys, xs = np.mgrid[0:h, 0:w].astype(np.float32)
     ramps = 0.3 + 0.4 * np.stack([xs / w, ys / h, (xs + 2 * ys) / (w + 2 * h)], axis=-1)
     noise = rng.normal(0, 0.02, (h, w, 3))
@@ -442,15 +443,21 @@ def image_for_bounds(rng, content, w, h):
         rgb[..., 0] = np.where(rng.random((h, w)) < 0.03, 0.75, 0.5)
     elif content == "faint":
         rgb = 0.5 + noise * np.float32(2.0 ** -14)
-    else:
+    elif content in ("tiny", "huge"):
         rgb = noise * (1e-12 if content == "tiny" else 1e12) * np.where(rng.random((h, w, 1)) < 0.5, 1, 30)
     alpha = np.ones((h, w, 1))
     alpha[: h // 2, : w // 2] = np.where(rng.random((h // 2, w // 2, 1)) < 0.2, rng.random((h // 2, w // 2, 1)), 1)
+    if content == "specks":
+        rgb = ramps + noise
+        for y, x in ((y, x) for y in range(0, h, 4) for x in range(y % 32, w, 32)):
+            block = rng.random((4, 4, 3)) * 2.0 ** rng.uniform(-51, -47)
+            block[0, 0] = rng.random(3) * 2.0 ** rng.uniform(-27, -24)
+            rgb[y:y + 4, x:x + 4], alpha[y:y + 4, x:x + 4] = block, 0 if x < w // 2 else 1
     return np.concatenate([rgb, alpha], axis=-1).astype(np.float32)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("content", ["noise", "edges", "grey", "level", "faint", "tiny", "huge"])
+@pytest.mark.parametrize("content", ["noise", "edges", "grey", "level", "faint", "specks", "tiny", "huge"])
 @pytest.mark.parametrize("size", [(68, 60), (520, 524)])    # workgroups of one group of 64 blocks, and of two
 def test_gpu_bc7_search_with_bounds_matches_checker(ntc, device, oracle, size, content):
     image = image_for_bounds(np.random.default_rng(80), content, *size)
