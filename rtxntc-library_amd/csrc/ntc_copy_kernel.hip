@@ -1263,8 +1263,9 @@ hipError_t launch_write_channels(WriteChannelsArgs const& args, hipStream_t stre
 // clamped (Inference.cu:96-97,112; a negative zero becomes +0 as the device max() of the reference
 // returns), and with discardMaskedOut a texel whose REFERENCE mask value is zero counts on the mask
 // channel only (Inference.cu:80-84,107-108).
-// Squares are fp32 as in the reference; the sum of two texels' goes into a double accumulator, and the
-// workgroup writes 16 double partial sums; ReduceLoss likewise finishes in double (src/Optimizer.cu:382-387).
+// Squares are fp32 as in the reference; the sum of two texels' (where the width is odd, each texel's) goes into a double
+// accumulator, and the workgroup writes 16 double partial sums; ReduceLoss likewise finishes in double
+// (src/Optimizer.cu:382-387).
 //
 // The same launch finishes the sum and hands it to the host (a second kernel, a copy and a stream synchronisation made
 // most of the 28 us a call on 64 x 64 texels took).  Workgroups form at most kLossRows groups; the last one of a group
@@ -1370,15 +1371,12 @@ __device__ __forceinline__ void hand_over_sums(double const (&acc)[NTC_HIP_DEV_M
         __hip_atomic_store(&work.rows[group].words[lane], word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Squared differences of two texels' first or second halves (SHIFT = 0, 16), added up.
-template <int SHIFT> __device__ __forceinline__ float two_squares(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1)
+// Squared difference of two texels' first or second halves (SHIFT = 0, 16).
+template <int SHIFT> __device__ __forceinline__ float square(uint32_t a, uint32_t b)
 {
     auto const half = [](uint32_t w) { return float(__builtin_bit_cast(_Float16, uint16_t(w >> SHIFT))); };
-    float const d0 = half(a0) - half(b0), d1 = half(a1) - half(b1);
-    float s = 0.f;
-    s += d0 * d0;
-    s += d1 * d1;
-    return s;
+    float const d = half(a) - half(b);
+    return d * d;
 }
 
 // Large images without a mask channel.  The internal layout is row after row of channel pairs, so that whole rows are one piece of memory,
@@ -1389,7 +1387,7 @@ template <int SHIFT> __device__ __forceinline__ float two_squares(uint32_t a0, u
 // and the groups' counters on one line (6 channels: 80, 28, 16.5 and 15.5; 111, 37, 25 and 18); 209, 51, 30 and 26 with a
 // wave for each pair, whose rows lie a power of two apart.  A kernel that does nothing but read the two images of 16
 // channels takes 172, 38 and 10 for the first three, a call of nothing 11.
-template <int STEPS, int PAIRS>
+template <int STEPS, int PAIRS, bool ODD>
 __global__ void __launch_bounds__(256, 4)
 image_loss_kernel(uint16_t const* __restrict__ a, uint16_t const* __restrict__ b, int width, int height, int setChannels, int rowsPerWorkgroup, int log2Lanes,
                   uint32_t validChannelMask, uint32_t blocks, uint32_t groupSize, LossWorkspace work)
@@ -1400,10 +1398,18 @@ image_loss_kernel(uint16_t const* __restrict__ a, uint16_t const* __restrict__ b
 #pragma unroll
     for (int c = 0; c < NTC_HIP_DEV_MAX_CHANNELS; ++c) acc[c] = 0.0;
     auto const add = [&](int p, u32x4_a4 const& va, u32x4_a4 const& vb) {
-        acc[2 * p] += double(two_squares<0>(va[0], va[1], vb[0], vb[1]));
-        acc[2 * p + 1] += double(two_squares<16>(va[0], va[1], vb[0], vb[1]));
-        acc[2 * p] += double(two_squares<0>(va[2], va[3], vb[2], vb[3]));
-        acc[2 * p + 1] += double(two_squares<16>(va[2], va[3], vb[2], vb[3]));
+#pragma unroll
+        for (int k = 0; k < 4; k += 2) {
+            float const s0 = square<0>(va[k], vb[k]), t0 = square<0>(va[k + 1], vb[k + 1]);
+            float const s1 = square<16>(va[k], vb[k]), t1 = square<16>(va[k + 1], vb[k + 1]);
+            if constexpr (ODD) {
+                acc[2 * p] += double(s0); acc[2 * p] += double(t0);
+                acc[2 * p + 1] += double(s1); acc[2 * p + 1] += double(t1);
+            } else {
+                acc[2 * p] += double(s0 + t0);
+                acc[2 * p + 1] += double(s1 + t1);
+            }
+        }
     };
     int const begin = int(blockIdx.x) * rowsPerWorkgroup, end = min(height, begin + rowsPerWorkgroup);
     // (addresses: the workgroup's rows, the pair and the step in scalar registers, the lane's place in 32 bits)
@@ -1553,14 +1559,16 @@ hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int heig
     uint64_t const share = uint64_t(rows) * uint64_t(width), even = uint64_t(width) * uint64_t(height) / blocks;
     bool const shared = share <= 2u * (even < 1024u ? 1024u : even);
     if (maskChannel < 0 && width >= 4 && uint64_t(width) * uint64_t(height) >= 131072u && shared && share * uint64_t(setChannels) * 2u < 0x80000000u) {
-        auto launch = [&](auto steps, auto pairs) {
-            return launch_kernel_with_event<image_loss_kernel<decltype(steps)::value, decltype(pairs)::value>>(dim3(blocks), dim3(256), 0, stream, done,
+        auto launch = [&](auto steps, auto pairs, auto odd) {
+            return launch_kernel_with_event<image_loss_kernel<decltype(steps)::value, decltype(pairs)::value, decltype(odd)::value>>(dim3(blocks), dim3(256), 0, stream, done,
                                          a, b, width, height, setChannels, int(rows), log2Lanes, validChannelMask, blocks, grid.groupSize, work);
         };
-        // a row is one, two or more steps of 1024 texels
-        if (width >= 4096) return launch(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{});
-        if (width >= 2048) return launch(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});
-        return launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 4>{});
+        auto of_steps = [&](auto odd) {                      // a row is one, two or more steps of 1024 texels
+            if (width >= 4096) return launch(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{}, odd);
+            if (width >= 2048) return launch(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{}, odd);
+            return launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 4>{}, odd);
+        };
+        return (width & 1) == 0 ? of_steps(std::false_type{}) : of_steps(std::true_type{});
     }
     auto launch = [&](auto perLane, auto masked) {
         return launch_kernel_with_event<texel_loss_kernel<decltype(perLane)::value, decltype(masked)::value>>(dim3(grid.x, grid.y), dim3(256), 0, stream, done,

@@ -149,7 +149,25 @@ def test_loss_sums_of_whole_rows(ntc, device, oracle, w, h, channels):
     mask = 0x5FF7 & ((1 << channels) - 1)
     oracle.ntc_oracle_image_loss(a.ctypes.data, b.ctypes.data, w, h, channels, mask, want.ctypes.data)
     device.call("image_loss", d_a.ptr, d_b.ptr, d_a.nbytes, w, h, channels, mask, -1, 0, got)
-    assert np.allclose(got[:], want, rtol=2e-7, atol=0)      # (double sums, rounded to float once)
+    # (two texels' squares are added in float, the rest in double; rounded to float once)
+    assert np.allclose(got[:], want, rtol=2e-7, atol=0)
+
+
+@pytest.mark.parametrize("w,h", [(75, 64), (255, 530), (1023, 137), (1029, 1030), (2051, 601), (4099, 1100)])
+def test_loss_of_odd_widths_adds_every_square_in_double(ntc, device, w, h):
+    """Every other square is less than half a unit in the last place of the one before it: a sum of the two in float would
+    drop it, and the mean comes out a unit lower."""
+    faint = np.float16(0.995 * 2.0 ** -12)
+    image = np.zeros((h, 2, w, 2), dtype=np.float16)
+    image[:, :, 0:w - 1:2] = 1
+    image[:, :, 1:w - 1:2] = faint
+    flat, ones = image.reshape(-1).view(np.uint16), (w - 1) // 2 * h
+    d_a, d_b = device.upload(flat), device.upload(np.zeros_like(flat))
+    want = np.float32(ones * (1 + float(faint) ** 2) / (w * h))
+    assert want != np.float32(ones / (w * h))
+    got = (ntc.abi.C.c_float * 16)()
+    device.call("image_loss", d_a.ptr, d_b.ptr, d_a.nbytes, w, h, 4, 0xF, -1, 0, got)
+    assert list(got[:4]) == [want] * 4
 
 
 @pytest.mark.parametrize("mask_channel", [-1, 5])
