@@ -1381,7 +1381,9 @@ template <int SHIFT> __device__ __forceinline__ float square(uint32_t a, uint32_
 
 // Large images without a mask channel.  The internal layout is row after row of channel pairs, so that whole rows are one piece of memory,
 // which the workgroup goes through in order, 4 KB of each image a load; STEPS of a pair's row and PAIRS pairs are under way
-// together, eight loads a lane (sixteen do not leave the registers for four waves per SIMD).  Bound by memory for large
+// together, eight loads a lane (sixteen do not leave the registers for four waves per SIMD).  The workgroups' shares differ
+// by PAIRS pairs of a row at most: with whole rows, as many in each, 2500 x 2500 took 92 us and 1920 x 1080 41, now 84 and 39
+// (86.5 and 39 with 8-byte loads by lanes of two texels, see below).  Bound by memory for large
 // mips, by the launch and the way to the host below 512 x 512.  Whole calls of 16 channels, 4096 x 4096, 2048 x 2048, 1024 x
 // 1024 and 512 x 512: 189, 51, 23 and 16.5 us; 197, 56, 29 and 18.5 with 8-byte loads of all pairs by lanes of two texels,
 // and the groups' counters on one line (6 channels: 80, 28, 16.5 and 15.5; 111, 37, 25 and 18); 209, 51, 30 and 26 with a
@@ -1389,7 +1391,7 @@ template <int SHIFT> __device__ __forceinline__ float square(uint32_t a, uint32_
 // channels takes 172, 38 and 10 for the first three, a call of nothing 11.
 template <int STEPS, int PAIRS, bool ODD>
 __global__ void __launch_bounds__(256, 4)
-image_loss_kernel(uint16_t const* __restrict__ a, uint16_t const* __restrict__ b, int width, int height, int setChannels, int rowsPerWorkgroup, int log2Lanes,
+image_loss_kernel(uint16_t const* __restrict__ a, uint16_t const* __restrict__ b, int width, int height, int setChannels, int share, int more, int log2Lanes,
                   uint32_t validChannelMask, uint32_t blocks, uint32_t groupSize, LossWorkspace work)
 {
     constexpr int MAX_PAIRS = NTC_HIP_DEV_MAX_CHANNELS / 2;
@@ -1411,16 +1413,22 @@ image_loss_kernel(uint16_t const* __restrict__ a, uint16_t const* __restrict__ b
             }
         }
     };
-    int const begin = int(blockIdx.x) * rowsPerWorkgroup, end = min(height, begin + rowsPerWorkgroup);
+    // Units of PAIRS pairs of the rows that the lanes take together: `share` to a workgroup, and one more to the first `more`.
+    int const block = int(blockIdx.x), together = 256 >> log2Lanes, groups = (pairs + PAIRS - 1) / PAIRS;
+    int const firstUnit = block * share + min(block, more), endUnit = firstUnit + share + (block < more ? 1 : 0);
+    int const begin = firstUnit / groups * together;
     // (addresses: the workgroup's rows, the pair and the step in scalar registers, the lane's place in 32 bits)
     size_t const rows = size_t(begin) * size_t(setChannels) * size_t(width);
     char const* const ra = reinterpret_cast<char const*>(a + rows);
     char const* const rb = reinterpret_cast<char const*>(b + rows);
-    for (int y = begin + (int(threadIdx.x) >> log2Lanes); y < end; y += 256 >> log2Lanes) {
+    int y = begin + (int(threadIdx.x) >> log2Lanes);
+    for (int unit = firstUnit - firstUnit % groups; unit < endUnit; unit += groups, y += together) {
+        if (y >= height) continue;
         uint32_t const row = uint32_t(y - begin) * uint32_t(pairs) * uint32_t(width) * 4u;
 #pragma unroll
         for (int p0 = 0; p0 < MAX_PAIRS; p0 += PAIRS) {
-            if (p0 >= pairs) break;                          // uniform
+            if (unit + p0 / PAIRS < firstUnit) continue;     // uniform, as the next
+            if (p0 >= pairs || unit + p0 / PAIRS >= endUnit) break;
             size_t offset[PAIRS];                            // (no branch around a load: pairs that the set does not have read its last one again, and their sums are dropped)
 #pragma unroll
             for (int p = 0; p < PAIRS; ++p) offset[p] = size_t(min(p0 + p, pairs - 1)) * size_t(width) * 4u;
@@ -1546,26 +1554,36 @@ hipError_t launch_image_loss(uint16_t* a, uint16_t const* b, int width, int heig
 {
     LossGrid const grid = image_loss_grid(width, height, compute_units_of_current_device());
     uint32_t const blocks = grid.x * grid.y;
-    // Without a mask: 2^log2Lanes lanes to a row, as few as cover a narrow one with four texels each, all 256 at most, and a
-    // multiple of the rows that a workgroup's lanes take together.  (Workgroups that this leaves no row hand over zeros.)
+    // Without a mask: 2^log2Lanes lanes to a row, as few as cover a narrow one with four texels each, all 256 at most.  Rows are
+    // divided among the workgroups that are resident together; the others, and those that this leaves no row, hand over zeros.
     int log2Lanes = 0;
     while (log2Lanes < 8 && (4 << log2Lanes) < width) ++log2Lanes;
-    uint32_t const together = 256u >> log2Lanes, rows = ((uint32_t(height) + blocks - 1u) / blocks + together - 1u) / together * together;
+    uint32_t const together = 256u >> log2Lanes, turns = (uint32_t(height) + together - 1u) / together;
+    uint32_t const busy = min(blocks, 4u * uint32_t(compute_units_of_current_device())), rows = (turns + busy - 1u) / busy * together;
     // The other kernel's are images of less than 131072 texels, a trip to memory or two for a workgroup, which it makes with
     // all pairs' loads at once and without a tail of a row (300 x 200 and 150 x 100 of 16 channels 15.5 and 15.2 us, 17.1 and
     // 20.4 by whole rows; 400 x 300 16.3 and 17.7, 512 x 512 18.5 and 16.5); rows of less than four texels; rows beyond 31 bits
     // of offsets; and wide images of few rows, which leave most workgroups none (16384 x 1 30 us, 15.6 the other way;
     // 8192 x 8 22 and 16.5; 4096 x 64 19.5 and 17.1; 2048 x 128, twice the even share, 17.5 and 17.7).
-    uint64_t const share = uint64_t(rows) * uint64_t(width), even = uint64_t(width) * uint64_t(height) / blocks;
+    uint64_t const share = uint64_t(rows) * uint64_t(width), even = uint64_t(width) * uint64_t(height) / busy;
     bool const shared = share <= 2u * (even < 1024u ? 1024u : even);
     if (maskChannel < 0 && width >= 4 && uint64_t(width) * uint64_t(height) >= 131072u && shared && share * uint64_t(setChannels) * 2u < 0x80000000u) {
         auto launch = [&](auto steps, auto pairs, auto odd) {
+            uint32_t const units = turns * ((uint32_t(setChannels) / 2u + decltype(pairs)::value - 1u) / decltype(pairs)::value);
             return launch_kernel_with_event<image_loss_kernel<decltype(steps)::value, decltype(pairs)::value, decltype(odd)::value>>(dim3(blocks), dim3(256), 0, stream, done,
-                                         a, b, width, height, setChannels, int(rows), log2Lanes, validChannelMask, blocks, grid.groupSize, work);
+                                         a, b, width, height, setChannels, int(units / busy), int(units % busy), log2Lanes, validChannelMask, blocks, grid.groupSize, work);
         };
-        auto of_steps = [&](auto odd) {                      // a row is one, two or more steps of 1024 texels
-            if (width >= 4096) return launch(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{}, odd);
-            if (width >= 2048) return launch(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{}, odd);
+        // Of the three shapes the one with the fewest trips to memory for a row: whole ones of its steps, then what is left a
+        // step at a time.  16 channels of images not read before, by the first, the second and the third shape of
+        // 2100 x 2100: -, 68 and 65.5 us; 3500 x 2000 -, 96 and 92.5; 5000 x 3000 180, - and 178; with even shares of rows.
+        uint32_t const pairs = uint32_t(setChannels) / 2u, w = uint32_t(width);
+        auto const trips = [&](uint32_t steps, uint32_t pairsTogether) {
+            return (pairs + pairsTogether - 1u) / pairsTogether * (w / (1024u * steps) + (w % (1024u * steps) + 1023u) / 1024u);
+        };
+        uint32_t const four = trips(4, 1), two = trips(2, 2), one = trips(1, 4);
+        auto of_steps = [&](auto odd) {
+            if (four <= two && four <= one) return launch(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{}, odd);
+            if (two <= one) return launch(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{}, odd);
             return launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 4>{}, odd);
         };
         return (width & 1) == 0 ? of_steps(std::false_type{}) : of_steps(std::true_type{});

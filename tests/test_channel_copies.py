@@ -138,10 +138,11 @@ def test_loss_sums_of_one_group_and_of_many(ntc, device, oracle, w, h):
 
 
 @pytest.mark.parametrize("w,h,channels", [(3, 50000, 2), (4, 40001, 16), (7, 20777, 2), (255, 530, 14), (1023, 137, 10), (1029, 1030, 6), (2050, 601, 4),
-                                          (361, 363, 8), (4099, 1100, 2), (65536, 3, 2)])
+                                          (361, 363, 8), (4099, 1100, 2), (65536, 3, 2), (2100, 403, 16), (3841, 402, 12), (5000, 301, 16), (7170, 3000, 2)])
 def test_loss_sums_of_whole_rows(ntc, device, oracle, w, h, channels):
     """Rows of one, two and more steps of the workgroup's lanes with what is left of them, several rows a workgroup's lanes
-    take together, fewer pairs than are loaded together, and images that fall to the other kernel."""
+    take together, fewer pairs than are loaded together, shares that begin and end inside a row, more workgroups than have a
+    share, and images that fall to the other kernel."""
     rng = np.random.default_rng(w * h)
     a, b = halves(rng, w * h * channels), halves(rng, w * h * channels)
     d_a, d_b = device.upload(a), device.upload(b)
