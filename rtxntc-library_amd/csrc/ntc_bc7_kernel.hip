@@ -1483,6 +1483,8 @@ bc7_compress_kernel(BlockCompressArgs a)
     auto const wait_for = [&](int& counter, int count) {
         while (__hip_atomic_load(&counter, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < count) __builtin_amdgcn_s_sleep(1);
     };
+    // (Lane 0's release is for what all lanes of the wave wrote: it waits until the wave's LDS operations are done, which are
+    // counted for the wave and complete in order.)
     auto const add_one = [&](int& counter) { if (lane == 0) __hip_atomic_fetch_add(&counter, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP); };
     // Mode 7's partition comes with the two subsets where every alpha is 1, whose terms are zeros.  Opaque blocks of float
     // images can hold alphas above 1 and NaNs: their groups bound it over four channels, as blocks with alpha.
