@@ -542,10 +542,12 @@ BC7_INLINE void store_block(BlockCompressArgs const& a, int bx, int by, uint64_t
 // search divided and every partition estimated, 64 x 64 took 98 us, 512 x 512 102, 1024 x 1024 274 and 2048 x 2048 927 (half
 // of it opaque; 183 M vector instructions at 1024 x 1024, seven of ten of them estimates); with bounds first 79, 88, 191
 // and 721 (140 M).  Bounds cost a third of an estimate and leave few to make where texels have noise or detail in three
-// channels; where channels are proportional, every partition's bound is nothing, and searches whose blocks are mostly like
-// that are estimated as a whole without bounds (kNearLine: 1024 x 1024 grey 277 -> 254 us, 700 with queues for them).
-// Hard edges in every block leave a fifth and more of the partitions, more than a queue takes: there the bounds are
-// in vain (284 -> 311 us).
+// channels; where a block's colours lie near a line, because channels are proportional or an edge between two colours runs
+// through it, most partitions' bounds are below the smallest error.  Searches with many such blocks are estimated as a whole
+// without bounds (kMostExpected): 1024 x 1024 opaque, by estimates of every partition / by bounds first, whole where a queue
+// overflows or 48 of 64 blocks are near a line / now: grey 272 / 239 / 239 us, noise of 1.5 codes on proportional channels
+// 273 / 275 / 240 and of 4 codes 274 / 307 / 240, hard edges in every block 276 / 299 / 243 and with noise 275 / 306 / 245,
+// antialiased boxes and strokes 278 / 317 / 244 and with noise 275 / 317 / 241; not antialiased 272 / 174 / 187.
 //
 // Wave priorities fall from phase to phase.  With equal ones the older of the two workgroups of a compute unit runs ahead
 // through the first phase and leaves the younger one alone with half the waves at the end (347 and 485 thousand cycles at
@@ -638,7 +640,16 @@ constexpr float kBoundError = 0x1p-13f, kLeastLength = 0x1p-72f;
 constexpr float kUnsureOfOffsets = 0x1p-16f, kUnsureOfTexels = 0x1p-35f;
 // Bounds are kept as codes of eight bits: errors over T, four bits of the exponent (2^-16 ... 1) and four of the mantissa,
 // rounded down.  Blocks whose T is no number between these have no bounds, and all of their partitions are estimated.
-constexpr float kNearLine = 1.f / 64.f;                      // squared distances over the squared diagonal; eight points leave 16 / 588 of it
+// Blocks near a line: what the partitions leave of their distances is less than the steps along the diagonals, and the
+// bounds tell little.  How many partitions they leave in the searches for modes 0 to 3 goes by the block's squared distances
+// over its squared diagonal (eight points leave 16 / 588 of it), much the same for noise, edges and gradients: 2 above 1 / 8, 5 to 18
+// down to 1 / 16, 9 to 33, 14 to 47 and 16 to 57 down to 1 / 24, 1 / 37 and 1 / 64, 25 to 63 below.  The weights in bound_task()
+// add up to the smaller ones.  Where more than kMostExpected of a group's 4096 are expected the search goes without bounds: 14 a
+// block overflow its queue, 9 are as slow as estimating all, and 5 because the slowest group is what counts (hard edges with
+// noise 283, 272, 257, 245 and 241 us with 10, 8, 6, 5 and 4, smooth images 241, 241, 232, 234 and 235, boxes that are not
+// antialiased 185, 185, 185, 187 and 195).  Blocks of two colours are left out for two subsets, where one partition has no error.
+constexpr float kNearLine = 1.f / 64.f;
+constexpr int kMostExpected = 5 * 64;
 // (The least T of halves that are not all equal is 2^-48.)
 constexpr float kLeastOffsets = 0x1p-48f, kMostOffsets = 0x1p60f;
 BC7_INLINE uint32_t error_code(float error, float scale)
@@ -782,15 +793,31 @@ BC7_TASK void bound_task(SearchPtr<S> lds, int b, int first, int last)
     float const unsure = __builtin_fmaf(offsets, kUnsureOfOffsets, dot(origin, origin) * kUnsureOfTexels);
     if constexpr (ORIENTED) lds->scale[kind][b] = scale;
     if constexpr (PLAIN) lds->scale[kPickTwoAlpha][b] = scale;
-    // Blocks near a line: what the partitions leave of their distances is less than the steps along the diagonals, and the
-    // bounds tell nothing.  Where three of four blocks are such, every partition is estimated (lowest stays as it is).
+    // Whether bounds are in vain (see kNearLine): then every partition is estimated (lowest stays as it is).
     {
         Color<C> lo, hi;
         subset_box<C, 16, false, S>(lds, b, kAllTexels, origin, lo, hi, total);
         float oriented = 0.f, plain = 0.f;
         add_distances<C, ORIENTED, !ORIENTED>(16.f, total, lo, hi, unsure, oriented, plain);
         Color<C> const a = sub(hi, lo);
-        if (__popcll(__ballot(bounded && (ORIENTED ? oriented : plain) < dot(a, a) * kNearLine)) >= 48) return;
+        float const square = dot(a, a), distances = ORIENTED ? oriented : plain;
+        bool counts = bounded;
+        if constexpr (ORIENTED && SUBSETS == 2) {            // two colours lie at the ends of the diagonal
+            float about = offsets;
+#pragma unroll
+            for (int k = 0; k < C; ++k) {
+                float const middle2 = lo.c[k] + hi.c[k];
+                about = __builtin_fmaf(-middle2, __builtin_fmaf(-4.f, middle2, total.s[k]), about);
+            }
+            counts = counts && about < square * 3.996f;
+        }
+        auto const near = [&](float limit) { return __popcll(__ballot(counts && distances < square * limit)); };
+        if constexpr (ORIENTED) {
+            if (2 * __popcll(__ballot(bounded)) + 5 * near(1.f / 8.f) + 5 * near(1.f / 16.f) + 6 * near(1.f / 24.f) + 7 * near(1.f / 37.f)
+                + 15 * near(kNearLine) > kMostExpected) return;
+        } else {
+            if (near(kNearLine) >= 48) return;
+        }
     }
     uint32_t lowestOriented = ~0u, lowestPlain = ~0u, codesOriented = 0, codesPlain = 0;
 #pragma unroll 1

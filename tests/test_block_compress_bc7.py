@@ -426,7 +426,8 @@ def test_gpu_bc7_opaque_blocks_whose_alpha_is_not_one_match_checker(ntc, device,
 def image_for_bounds(rng, content, w, h):
     """RGBA float32, a quarter of the blocks with alpha.  Which of the search's ways the partitions' errors take: "noise" a
     few estimates beyond the first; "edges" more than the queues hold; "grey" no bounds, because channels are proportional;
-    "level" subsets that are level in channels; "faint" covariances whose signs are within their errors; "specks" every eighth
+    "level" subsets that are level in channels; "colours" two in a block or one; "mixed" a part of the blocks grey, from none of
+    a group's to all, so that some searches go without bounds; "faint" covariances whose signs are within their errors; "specks" every eighth
     block a first texel of 2^-24 ... 2^-27 among others of 2^-47 ... 2^-51, whose products are near the least of floats; "tiny"
     and "huge" texels' offsets outside the range that has bounds."""
     ys, xs = np.mgrid[0:h, 0:w].astype(np.float32)
@@ -441,6 +442,12 @@ def image_for_bounds(rng, content, w, h):
     elif content == "level":
         rgb = np.round((ramps + noise) * 16) / 16
         rgb[..., 0] = np.where(rng.random((h, w)) < 0.03, 0.75, 0.5)
+    elif content == "colours":
+        pair = np.repeat(np.repeat(rng.random((2, h // 4, w // 4, 3)), 4, axis=1), 4, axis=2)
+        rgb = np.where(rng.random((h, w, 1)) < np.repeat(np.repeat(rng.choice([0, 0.5], (h // 4, w // 4, 1)), 4, axis=0), 4, axis=1), pair[0], pair[1])
+    elif content == "mixed":
+        grey = rng.random((h // 4, w // 4, 1)) * w < np.arange(w // 4)[None, :, None] * 4
+        rgb = np.where(np.repeat(np.repeat(grey, 4, axis=0), 4, axis=1), (ramps + noise)[..., :1] * [1.0, 0.9, 0.8] + noise * 0.05, ramps + noise)
     elif content == "faint":
         rgb = 0.5 + noise * np.float32(2.0 ** -14)
     elif content in ("tiny", "huge"):
@@ -457,12 +464,12 @@ def image_for_bounds(rng, content, w, h):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("content", ["noise", "edges", "grey", "level", "faint", "specks", "tiny", "huge"])
+@pytest.mark.parametrize("content", ["noise", "edges", "grey", "level", "colours", "mixed", "faint", "specks", "tiny", "huge"])
 @pytest.mark.parametrize("size", [(68, 60), (520, 524)])    # workgroups of one group of 64 blocks, and of two
 def test_gpu_bc7_search_with_bounds_matches_checker(ntc, device, oracle, size, content):
     image = image_for_bounds(np.random.default_rng(80), content, *size)
     formats = [(4, image)]
-    if content in ("noise", "edges", "grey", "level"):
+    if content in ("noise", "edges", "grey", "level", "colours", "mixed"):
         formats.append((1, np.clip(np.rint(image * 255), 0, 255).astype(np.uint8)))
     for fmt, texels in formats:
         args = (np.ascontiguousarray(texels), fmt, 4, size[0] // 4, size[1] // 4)
