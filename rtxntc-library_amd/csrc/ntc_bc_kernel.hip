@@ -36,14 +36,30 @@ namespace ntc_hip_dev {
 
 namespace {
 
-// A block's endpoints, and its sixteen 3-bit indices in two words of eight.
-struct Bc4 {
-    uint32_t e0, e1, low, high;
-    __device__ __forceinline__ uint64_t bits() const
-    {
-        return uint64_t(e0) | (uint64_t(e1) << 8) | (uint64_t(low) << 16) | (uint64_t(high) << 40);
-    }
+// A block of one channel: four texels of a row a word, and in 16-bit lanes, of each row the texels 0 and 2, 1 and 3.
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+struct Bc4Texels {
+    uint32_t rows[4];
+    u16x2 even[4], odd[4];
+    uint32_t lo, hi, squares;                                // extremes, sum of squares
 };
+
+// A block's endpoints, and where its texels lie between them: a position a byte, four texels a word.  Position 0 is
+// endpoint 0, the last one (7, or 5 in the six-value palette) endpoint 1; 6 and 7 of the six-value palette are 0 and 255.
+struct Bc4 { uint32_t e0, e1, positions[4]; };
+
+// The block: endpoints and, of sixteen texels, the 3-bit indices that their positions stand for.
+template <bool EIGHT>
+__device__ __forceinline__ uint64_t bc4_bits(Bc4 const& block)
+{
+    uint64_t bits = uint64_t(block.e0) | (uint64_t(block.e1) << 8);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        uint32_t const k = __builtin_amdgcn_perm(EIGHT ? 0x01070605u : 0x07060105u, 0x04030200u, block.positions[r]);
+        bits |= uint64_t(__builtin_amdgcn_udot4(k, 0x00400801u, (k >> 24) << 9, false)) << (16 + 12 * r);
+    }
+    return bits;
+}
 
 // The eight values that two endpoints stand for, times eight.  With e0 > e1 entry k + 1 is ((7 - k) e0 + k e1 + 3) / 7,
 // else ((5 - k) e0 + k e1 + 2) / 5 and the last two are 0 and 255 (the reference's rounding biases); a product and a
@@ -62,88 +78,245 @@ __device__ __forceinline__ void bc4_palette8(uint32_t e0, uint32_t e1, uint32_t 
     if (!eight) { p[6] = 0u; p[7] = 255u << 3; }
 }
 
-// Nearest palette entry for every texel (the first of equally near ones); returns the summed squared error.
-// values8: the texels times eight, so that |value - entry| * 8 + k is one instruction per entry: the smallest of these
-// keys is the nearest entry, the first among equally near ones.  keys: the chosen ones.  (Sums of 16-bit differences: of a
-// 32-bit one with k = 0 the compiler makes a maximum, a minimum and a difference.)
-__device__ __forceinline__ uint32_t bc4_assign(uint32_t const (&values8)[16], Bc4& block, uint32_t (&keys)[16])
+// The entries between two endpoints R apart, and where a texel lies among them.  The entry at position j is
+// q(j) = (j R + LAST / 2) / LAST away from endpoint 0 (that is what the biased quotients come to).  A texel d away from it
+// takes the nearest entry, of equally near ones the first in the order of the indices: the earlier position, but the last
+// one before those between the ends.  In sixteen bits and for 0 <= d <= R that position is
+//     (scale * d + start + kink * max(d - before, 0)) >> 13:
+// the steps of a line while all ties fall to one side, lifted at its end (kink) where the last two entries tie.  Scale and
+// start are found by trial, as the compiler runs, for every d that there is.
+struct alignas(16) Bc4Range { uint32_t near, far, line, bend; };         // q(0) ... q(3), q(4) ... q(7), scale | start << 16, kink | before << 16
+template <uint32_t LAST> struct Bc4Ranges { Bc4Range of[256]; };
+template <uint32_t LAST>
+constexpr Bc4Ranges<LAST> bc4_ranges()
 {
-    uint32_t p[8];
+    Bc4Ranges<LAST> table{};
+    for (uint32_t range = 0; range < 256; ++range) {
+        uint32_t q[8] = {}, position[256] = {};
+        for (uint32_t j = 0; j <= LAST; ++j) q[j] = (j * range + LAST / 2) / LAST;
+        Bc4Range& entry = table.of[range];
+        entry.near = q[0] | q[1] << 8 | q[2] << 16 | q[3] << 24;
+        entry.far = q[4] | q[5] << 8 | q[6] << 16 | q[7] << 24;
+        if (range == 0) continue;                            // position 0
+        uint32_t const first = (q[LAST - 1] + range + 1) / 2;                    // the last position's first texel
+        for (uint32_t d = 0, j = 0; d < first; ++d) {
+            while (2 * d > q[j] + q[j + 1]) ++j;
+            uint32_t same = j;
+            while (same > 0 && q[same - 1] == q[same]) --same;
+            position[d] = same;
+        }
+        bool found = false;
+        // (from the line through the ends outwards; two entries of range 2 lie four positions apart)
+        uint32_t const middle = LAST == 7 && range == 2 ? 2 * 8192 : LAST * 8192 / range;
+        for (uint32_t trial = 0; trial < 8 && !found; ++trial) {
+            uint32_t const scale = trial & 1 ? middle - trial / 2 - 1 : middle + trial / 2;
+            int32_t from = 0, to = 8191;
+            for (uint32_t d = 0; d < first; ++d) {
+                int32_t const least = int32_t(position[d] * 8192) - int32_t(d * scale);
+                if (least > from) from = least;
+                if (least + 8191 < to) to = least + 8191;
+                if (from > to) break;
+            }
+            if (from > to) continue;
+            uint32_t const start = uint32_t(to), reached = first * scale + start, kink = reached < LAST * 8192 ? LAST * 8192 - reached : 0;
+            found = range * scale + start + (range - first + 1) * kink < (LAST + 1) * 8192;
+            entry.line = scale | start << 16;
+            entry.bend = kink | (first - 1) << 16;
+        }
+        if (!found) __builtin_unreachable();                 // (does not compile)
+    }
+    return table;
+}
+struct Bc4Tables { Bc4Ranges<7> eight; Bc4Ranges<5> six; };
+__device__ constexpr Bc4Tables kBc4Tables{ bc4_ranges<7>(), bc4_ranges<5>() };
+
+// Copies them to the workgroup's memory: every thread takes part, they are there after the next barrier.
+__device__ __forceinline__ void bc4_stage(Bc4Tables& tables, uint32_t threads)
+{
+    for (uint32_t i = threadIdx.x; i < 256; i += threads) {
+        tables.eight.of[i] = kBc4Tables.eight.of[i];
+        tables.six.of[i] = kBc4Tables.six.of[i];
+    }
+}
+
+// Nearest palette entry for every texel, from the definition: the palette that the endpoints' order stands for, whatever
+// palette is searched for.
+template <bool EIGHT>
+__device__ __forceinline__ uint32_t bc4_assign_defined(Bc4Texels const& texels, Bc4& block)
+{
+    uint32_t p[8], total = 0;
     bc4_palette8(block.e0, block.e1, p);
-    uint32_t total = 0;
-    block.low = block.high = 0;
 #pragma unroll
-    for (int t = 15; t >= 0; --t) {
-        uint32_t key[8];
+    for (int r = 0; r < 4; ++r) {
+        uint32_t indices = 0;
+#pragma unroll 1
+        for (int i = 0; i < 32; i += 8) {
+            uint32_t const value8 = ((texels.rows[r] >> i) & 0xffu) << 3;
+            uint32_t best = ~0u;
 #pragma unroll
-        for (uint32_t k = 0; k < 8; ++k) key[k] = __builtin_amdgcn_sad_u16(values8[t], p[k], k);
-        uint32_t const best = min3_u32(min3_u32(key[0], key[1], key[2]), min3_u32(key[3], key[4], key[5]), min(key[6], key[7]));
-        uint32_t const distance = best >> 3;
-        total += __umul24(distance, distance);               // at most 16 * 255^2: exact as the float sum it stands for
-        uint32_t& word = t < 8 ? block.low : block.high;
-        word = (word << 3) | (best & 7u);
-        keys[t] = best;
+            for (uint32_t k = 0; k < 8; ++k) best = min(best, uint32_t(abs(int(value8) - int(p[k]))) | k);
+            total += (best >> 3) * (best >> 3);
+            indices |= (best & 7u) << i;
+        }
+        block.positions[r] = __builtin_amdgcn_perm(EIGHT ? 0x06050403u : 0x07060403u, EIGHT ? 0x02010700u : 0x02010500u, indices);
     }
     return total;
 }
 
-__device__ __forceinline__ uint32_t bc4_endpoint(float v) { return uint32_t(rintf(fminf(fmaxf(v, 0.f), 255.f))); }   // a NaN becomes 0
-
-// Least-squares endpoints for the block's current assignment.  EIGHT: every texel takes part and the weights of
-// endpoint 0 are 1, 0, 6/7 ... 1/7; otherwise indices 6 and 7 (the fixed 0 and 255) are left out and the weights are
-// 1, 0, 4/5 ... 1/5, and a singular system leaves the endpoints alone.  The numerators are bytes of a permute, and
-// w / 7 as w * hi + w * lo with hi + lo = 1/7, w / 5 as w * (1/5), are the correctly rounded quotients for all of them.
-// (Weights from a table in constant memory were a gather per texel and round.)
+// Nearest palette entry for every texel (the first of equally near ones); returns the summed squared error.
+// Positions by a line in packed 16-bit arithmetic, entries by byte permutes, the error from byte dot products as
+// sum v^2 - 2 sum v p + sum p^2: 14 instructions for four texels.  (The distances to all eight entries and their minima took 70.)
 template <bool EIGHT>
-__device__ __forceinline__ void bc4_refit(uint32_t const (&values8)[16], uint32_t const (&keys)[16], Bc4& block, bool keep255, bool keep0)
+__device__ __forceinline__ uint32_t bc4_assign(Bc4Texels const& texels, Bc4Tables const& tables, Bc4& block)
+{
+    if (EIGHT ? block.e0 <= block.e1 : block.e0 > block.e1) return bc4_assign_defined<EIGHT>(texels, block);   // the other palette: rare
+    uint32_t const range = EIGHT ? block.e0 - block.e1 : block.e1 - block.e0, base = block.e0 * 0x01010101u;
+    Bc4Range const entry = EIGHT ? tables.eight.of[range] : tables.six.of[range];
+    uint32_t const near = EIGHT ? base - entry.near : base + entry.near;         // (no byte borrows or carries)
+    uint32_t const far = EIGHT ? base - entry.far : ((base + entry.far) & 0xffffu) | 0xff000000u;
+    uint16_t const e0 = uint16_t(block.e0), r16 = uint16_t(range), scale = uint16_t(entry.line), start = uint16_t(entry.line >> 16);
+    uint16_t const kink = uint16_t(entry.bend), before = uint16_t(entry.bend >> 16);
+    auto const place = [&](u16x2 v) {
+        u16x2 d = EIGHT ? __builtin_elementwise_sub_sat(u16x2(e0), v) : __builtin_elementwise_sub_sat(v, u16x2(e0));
+        d = __builtin_elementwise_min(d, u16x2(r16));
+        return __builtin_elementwise_sub_sat(d, u16x2(before)) * kink + (d * scale + start);
+    };
+    u16x2 even[4], odd[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) { even[r] = place(texels.even[r]); odd[r] = place(texels.odd[r]); }
+    if constexpr (!EIGHT) {
+        // texels nearer to 0 than to endpoint 0, or to 255 than to endpoint 1: positions 0 and 5 (0 if the endpoints are
+        // one) become 6 and 7
+        if (__any(2u * texels.lo < block.e0 || 2u * texels.hi > 255u + block.e1)) {
+            uint16_t const top = uint16_t(255u + block.e1), from5 = uint16_t((range ? 2u : 7u) << 13);
+            auto const ends = [&](u16x2& s, u16x2 v) {
+                u16x2 const twice = v + v, one = u16x2(uint16_t(1));
+                s += __builtin_elementwise_min(__builtin_elementwise_sub_sat(u16x2(e0), twice), one) * uint16_t(6 << 13);
+                s += __builtin_elementwise_min(__builtin_elementwise_sub_sat(twice, u16x2(top)), one) * from5;
+            };
+#pragma unroll
+            for (int r = 0; r < 4; ++r) { ends(even[r], texels.even[r]); ends(odd[r], texels.odd[r]); }
+        }
+    }
+    uint32_t square = texels.squares, product = 0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        uint32_t const high = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, odd[r]), __builtin_bit_cast(uint32_t, even[r]), 0x07030501u);
+        block.positions[r] = (high >> 5) & 0x07070707u;
+        uint32_t const p = __builtin_amdgcn_perm(far, near, block.positions[r]);
+        square = __builtin_amdgcn_udot4(p, p, square, false);
+        product = __builtin_amdgcn_udot4(p, texels.rows[r], product, false);
+    }
+    return square - 2u * product;                            // at most 16 * 255^2: exact as the float sum it stands for
+}
+
+__device__ __forceinline__ float bc4_endpoint(float v) { return rintf(__builtin_amdgcn_fmed3f(v, 0.f, 255.f)); }   // a NaN becomes 0
+
+// Least-squares endpoints for the block's current positions, as they are defined: float sums in the texels' order.  EIGHT:
+// every texel takes part and the weights of endpoint 0 are 1, 0, 6/7 ... 1/7; otherwise positions 6 and 7 (the fixed 0 and
+// 255) are left out and the weights are 1, 0, 4/5 ... 1/5, and a singular system leaves the endpoints alone.  w / 7 as
+// w * hi + w * lo with hi + lo = 1/7, w / 5 as w * (1/5), are the correctly rounded quotients for all of them.
+template <bool EIGHT>
+__device__ __forceinline__ void bc4_solve_defined(Bc4Texels const& texels, Bc4 const& block, float& e0, float& e1)
 {
     float aa = 0.f, bb = 0.f, ab = 0.f, ax = 0.f, bx = 0.f;
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-        uint32_t const select = keys[t] & 7u;                                    // (only the lowest byte of the permute is looked at)
-        float alpha, beta;
-        if constexpr (EIGHT) {
-            float const w = float(__builtin_amdgcn_perm(0x01020304u, 0x05060007u, select) & 0xffu);
-            alpha = __builtin_fmaf(w, 1.f / 7.f, w * float(1.0 / 7.0 - double(1.f / 7.f)));
-            beta = 1.f - alpha;
-        } else {
-            float const w = float(__builtin_amdgcn_perm(0x00000102u, 0x03040005u, select) & 0xffu);
-            alpha = w * (1.f / 5.f);
-            beta = select >= 6u ? 0.f : 1.f - alpha;                     // adding zeros is leaving the texel out
+    for (int r = 0; r < 4; ++r) {
+        uint32_t const weights = EIGHT ? 0x07070707u - block.positions[r] : __builtin_amdgcn_perm(0x00000001u, 0x02030405u, block.positions[r]);
+#pragma unroll
+        for (int i = 0; i < 32; i += 8) {
+            float const w = float((weights >> i) & 0xffu), x = float((texels.rows[r] >> i) & 0xffu);
+            float alpha, beta;
+            if constexpr (EIGHT) {
+                alpha = __builtin_fmaf(w, 1.f / 7.f, w * float(1.0 / 7.0 - double(1.f / 7.f)));
+                beta = 1.f - alpha;
+            } else {
+                alpha = w * (1.f / 5.f);
+                beta = ((block.positions[r] >> i) & 0xffu) >= 6u ? 0.f : 1.f - alpha;        // adding zeros is leaving the texel out
+            }
+            aa += alpha * alpha; bb += beta * beta; ab += alpha * beta;
+            ax += alpha * x; bx += beta * x;
         }
-        float const x = float(values8[t] >> 3);
-        aa += alpha * alpha; bb += beta * beta; ab += alpha * beta;
-        ax += alpha * x; bx += beta * x;
     }
     if constexpr (EIGHT) {
         float const factor = 1.f / (aa * bb - ab * ab);
-        uint32_t const e0 = keep255 ? 255u : bc4_endpoint((ax * bb - bx * ab) * factor);
-        uint32_t const e1 = keep0 ? 0u : bc4_endpoint((bx * aa - ax * ab) * factor);
-        block.e0 = max(e0, e1); block.e1 = min(e0, e1);
+        e0 = bc4_endpoint((ax * bb - bx * ab) * factor);
+        e1 = bc4_endpoint((bx * aa - ax * ab) * factor);
     } else {
         float const det = aa * bb - ab * ab;
-        if (det == 0.f) return;
-        block.e0 = bc4_endpoint((ax * bb - bx * ab) / det);
-        block.e1 = bc4_endpoint((bx * aa - ax * ab) / det);
+        if (det == 0.f) { e0 = float(block.e0); e1 = float(block.e1); return; }
+        e0 = bc4_endpoint((ax * bb - bx * ab) / det);
+        e1 = bc4_endpoint((bx * aa - ax * ab) / det);
     }
 }
 
-// Up to eight rounds of refit + re-assign from the endpoints (e0, e1); returns the best block and its error.
+// The endpoints that bc4_solve_defined() comes to.  Its sums are those of small integers over LAST or LAST^2, which byte
+// dot products give exactly; where no rounding boundary is nearer to the quotient of these than the floats can be off,
+// both round alike.  Relative errors in units of 2^-24: 15 of the additions and at most 2.6 of the terms in a sum, so 36.3 of
+// the products' magnitudes in a numerator and 36 in the determinant, the quotient's own two and four here: 44 with the
+// products of errors, 2 % while the determinant is within 1 % (if it is not, the 51 makes `off` greater than 1/2).  One
+// lane in a hundred cannot tell; most of those are at exact ties, which the floats' errors decide.
 template <bool EIGHT>
-__device__ __forceinline__ Bc4 bc4_refine(uint32_t const (&values8)[16], uint32_t e0, uint32_t e1, bool keep255, bool keep0, uint32_t& bestError)
+__device__ __forceinline__ void bc4_refit(Bc4Texels const& texels, Bc4& block, bool keep255, bool keep0)
 {
-    Bc4 block{ e0 & 0xffu, e1 & 0xffu, 0u, 0u };
-    uint32_t keys[16];
-    bestError = bc4_assign(values8, block, keys);
+    uint32_t aa = 0, bb = 0, ab = 0, ax = 0, bx = 0;
+    if constexpr (EIGHT) {
+        uint32_t sum = 0, x = 0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            uint32_t const j = block.positions[r];
+            sum = __builtin_amdgcn_udot4(j, 0x01010101u, sum, false);
+            x = __builtin_amdgcn_udot4(texels.rows[r], 0x07070707u, x, false);
+            bb = __builtin_amdgcn_udot4(j, j, bb, false);
+            bx = __builtin_amdgcn_udot4(j, texels.rows[r], bx, false);
+        }
+        aa = 16u * 49u - 14u * sum + bb; ab = 7u * sum - bb; ax = x - bx;        // weights 7 - j
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            uint32_t const w = __builtin_amdgcn_perm(0x00000001u, 0x02030405u, block.positions[r]);
+            uint32_t const j = __builtin_amdgcn_perm(0x00000504u, 0x03020100u, block.positions[r]);
+            aa = __builtin_amdgcn_udot4(w, w, aa, false); bb = __builtin_amdgcn_udot4(j, j, bb, false); ab = __builtin_amdgcn_udot4(w, j, ab, false);
+            ax = __builtin_amdgcn_udot4(w, texels.rows[r], ax, false); bx = __builtin_amdgcn_udot4(j, texels.rows[r], bx, false);
+        }
+    }
+    constexpr float kLast = EIGHT ? 7.f : 5.f, kUnits = 44.f * 0x1p-24f;
+    uint32_t const axbb = __umul24(ax, bb), bxab = __umul24(bx, ab), bxaa = __umul24(bx, aa), axab = __umul24(ax, ab), aabb = __umul24(aa, bb), abab = __umul24(ab, ab);
+    float const perDet = __builtin_amdgcn_rcpf(float(aabb - abab)), unit = kUnits * perDet, dets = float(aabb + abab) * unit;
+    float const q0 = float(int32_t(axbb - bxab)) * kLast * perDet, q1 = float(int32_t(bxaa - axab)) * kLast * perDet;
+    float const off0 = __builtin_fmaf(float(axbb + bxab) * kLast, unit, max_f32(fabsf(q0), 51.f) * dets);
+    float const off1 = __builtin_fmaf(float(bxaa + axab) * kLast, unit, max_f32(fabsf(q1), 51.f) * dets);
+    bool const sure0 = fabsf(__builtin_amdgcn_fractf(q0) - 0.5f) > off0, sure1 = fabsf(__builtin_amdgcn_fractf(q1) - 0.5f) > off1;      // (a NaN is not)
+    float e0 = bc4_endpoint(q0), e1 = bc4_endpoint(q1);
+    if (!((EIGHT && keep255) || sure0) || !((EIGHT && keep0) || sure1)) bc4_solve_defined<EIGHT>(texels, block, e0, e1);
+    block.e0 = uint32_t(e0); block.e1 = uint32_t(e1);
+    if constexpr (EIGHT) {
+        if (keep255) block.e0 = 255u;
+        if (keep0) block.e1 = 0u;
+        uint32_t const top = max(block.e0, block.e1);
+        block.e1 = min(block.e0, block.e1); block.e0 = top;
+    }
+}
+
+// Up to eight rounds of refit + re-assign from the endpoints (e0, e1); returns the best block and its error.  (No round
+// betters an error of 0.)
+template <bool EIGHT>
+__device__ __forceinline__ Bc4 bc4_refine(Bc4Texels const& texels, Bc4Tables const& tables, uint32_t e0, uint32_t e1, bool keep255, bool keep0, uint32_t& bestError)
+{
+    Bc4 block{ e0 & 0xffu, e1 & 0xffu, {} };
+    bestError = bc4_assign<EIGHT>(texels, tables, block);
     Bc4 best = block;
+    if (bestError == 0) return best;
 #pragma unroll 1
     for (int round = 0; round < 8; ++round) {
-        bc4_refit<EIGHT>(values8, keys, block, keep255, keep0);
-        uint32_t const error = bc4_assign(values8, block, keys);
+        bc4_refit<EIGHT>(texels, block, keep255, keep0);
+        uint32_t const error = bc4_assign<EIGHT>(texels, tables, block);
         if (error >= bestError) break;
-        bool const repeated = block.low == best.low && block.high == best.high;
+        uint32_t moved = 0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) moved |= block.positions[r] ^ best.positions[r];
         best = block;
-        if (repeated) break;
+        if (moved == 0) break;
         bestError = error;
     }
     return best;
@@ -151,73 +324,92 @@ __device__ __forceinline__ Bc4 bc4_refine(uint32_t const (&values8)[16], uint32_
 
 // The candidate of one palette.
 template <bool EIGHT>
-__device__ __forceinline__ Bc4 bc4_candidate(uint32_t const (&values8)[16], uint32_t& error)
+__device__ __forceinline__ Bc4 bc4_candidate(Bc4Texels const& texels, Bc4Tables const& tables, uint32_t& error)
 {
-    uint32_t lo = 255u << 3, hi = 0;
+    uint32_t const lo = texels.lo, hi = texels.hi;
     if constexpr (EIGHT) {
-#pragma unroll
-        for (int t = 0; t < 16; ++t) { lo = min(lo, values8[t]); hi = max(hi, values8[t]); }
-        lo >>= 3; hi >>= 3;
         bool const keep0 = lo == 0, keep255 = hi == 255u;
         uint32_t const inset = (hi - lo) / 34u;
-        return bc4_refine<true>(values8, keep255 ? 255u : hi - inset, keep0 ? 0u : lo + inset, keep255, keep0, error);
+        error = 0;
+        if (lo == hi) return Bc4{ hi, lo, {} };              // (a palette of six that has the value)
+        return bc4_refine<true>(texels, tables, keep255 ? 255u : hi - inset, keep0 ? 0u : lo + inset, keep255, keep0, error);
     } else {
         // extremes among the values that are not 0 / not 255
+        uint32_t inner = 255u, outer = 0;
+        if (lo != 0 && hi != 255u) { inner = lo; outer = hi; }
+        else {
 #pragma unroll
-        for (int t = 0; t < 16; ++t) {
-            if (values8[t] != 0) lo = min(lo, values8[t]);
-            if (values8[t] != (255u << 3)) hi = max(hi, values8[t]);
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int i = 0; i < 32; i += 8) {
+                    uint32_t const v = (texels.rows[r] >> i) & 0xffu;
+                    if (v != 0) inner = min(inner, v);
+                    if (v != 255u) outer = max(outer, v);
+                }
         }
-        lo >>= 3; hi >>= 3;
-        // unsigned arithmetic on purpose: with no inner values (all texels 0 or 255) the difference wraps, as in the reference
-        uint32_t const inset = (hi - lo) / 34u;
-        return bc4_refine<false>(values8, lo + inset, hi - inset, false, false, error);
+        // eight values hold a range of seven, and 0 with 255, without error, and win then
+        error = ~0u;
+        if (hi - lo <= 7u || inner > outer) return Bc4{ 0u, 0u, {} };
+        uint32_t const inset = (outer - inner) / 34u;
+        return bc4_refine<false>(texels, tables, inner + inset, outer - inset, false, false, error);
     }
 }
 
-__device__ __forceinline__ uint32_t bc4_value8(float texel)
+__device__ __forceinline__ uint32_t bc4_value(float texel)
 {
     float const s = fminf(fmaxf(texel, 0.f), 1.f);           // saturate: a NaN becomes 0
-    return uint32_t(rintf(s * 255.f)) << 3;
+    return uint32_t(rintf(s * 255.f));
 }
 
-// Channel `c` of the sixteen texels of block (bx, by), as 8-bit values times eight.
-__device__ __forceinline__ void bc4_load(BlockCompressArgs const& a, int bx, int by, int c, uint32_t (&values8)[16])
+// What the searches ask of a block, from its rows.
+__device__ __forceinline__ void bc4_prepare(Bc4Texels& texels)
+{
+    texels.squares = 0;
+    u16x2 lo = u16x2(uint16_t(255)), hi = u16x2(uint16_t(0));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        texels.even[r] = __builtin_bit_cast(u16x2, texels.rows[r] & 0x00ff00ffu);
+        texels.odd[r] = __builtin_bit_cast(u16x2, (texels.rows[r] >> 8) & 0x00ff00ffu);
+        lo = __builtin_elementwise_min(lo, __builtin_elementwise_min(texels.even[r], texels.odd[r]));
+        hi = __builtin_elementwise_max(hi, __builtin_elementwise_max(texels.even[r], texels.odd[r]));
+        texels.squares = __builtin_amdgcn_udot4(texels.rows[r], texels.rows[r], texels.squares, false);
+    }
+    texels.lo = min(lo[0], lo[1]); texels.hi = max(hi[0], hi[1]);
+}
+
+// Channel `c` of the sixteen texels of block (bx, by), as 8-bit values.
+__device__ __forceinline__ void bc4_load(BlockCompressArgs const& a, int bx, int by, int c, Bc4Texels& texels)
 {
     int const x0 = a.srcLeft + bx * 4, y0 = a.srcTop + by * 4;
     if (a.packedRows && x0 + 4 <= a.srcWidth && y0 + 4 <= a.srcHeight) {
         // UNORM8 pixels without padding, the whole block inside the image: a row of four is four dwords at most, and
-        // a code is its own value (rint(code / 255 * 255) = code)
-        uint8_t const* px = a.src + size_t(y0) * a.rowPitch + size_t(x0) * a.pixelStride + size_t(c);
-        auto const rows = [&](auto load) {                   // all of them under way before the first is looked at
-            uint32_t words[4][4];
-#pragma unroll
-            for (int y = 0; y < 4; ++y) load(px + size_t(y) * a.rowPitch, words[y]);
-#pragma unroll
-            for (int t = 0; t < 16; ++t) values8[t] = (words[t >> 2][t & 3] & 0xffu) << 3;
-        };
+        // a code is its own value (rint(code / 255 * 255) = code).  All of them are under way before the first is looked at.
+        uint8_t const* px = a.src + size_t(y0) * a.rowPitch + size_t(x0) * a.pixelStride;
+        auto const row = [&](int y) { return px + size_t(y) * a.rowPitch; };
         if (a.pixelStride == 1) {                            // uniform; the image has no channel 1
-            rows([&](uint8_t const* row, uint32_t (&words)[4]) {
-                uint32_t const v = c == 0 ? *reinterpret_cast<u32_unaligned const*>(row) : 0u;
-                words[0] = v; words[1] = v >> 8; words[2] = v >> 16; words[3] = v >> 24;
-            });
-        } else if (a.pixelStride == 2) {
-            rows([&](uint8_t const* row, uint32_t (&words)[4]) {
-                u32x2_unaligned const v = *reinterpret_cast<u32x2_unaligned const*>(row - c);
-                words[0] = v[0] >> (8 * c); words[1] = v[0] >> (8 * c + 16); words[2] = v[1] >> (8 * c); words[3] = v[1] >> (8 * c + 16);
-            });
-        } else {
-            rows([&](uint8_t const* row, uint32_t (&words)[4]) {
 #pragma unroll
-                for (int x = 0; x < 4; ++x) words[x] = row[size_t(x) * a.pixelStride];
-            });
+            for (int y = 0; y < 4; ++y) texels.rows[y] = c == 0 ? *reinterpret_cast<u32_unaligned const*>(row(y)) : 0u;
+        } else if (a.pixelStride == 2) {
+            u32x2_unaligned words[4];
+#pragma unroll
+            for (int y = 0; y < 4; ++y) words[y] = *reinterpret_cast<u32x2_unaligned const*>(row(y));
+#pragma unroll
+            for (int y = 0; y < 4; ++y) texels.rows[y] = __builtin_amdgcn_perm(words[y][1], words[y][0], c == 0 ? 0x06040200u : 0x07050301u);
+        } else {
+            uint32_t bytes[4][4];
+#pragma unroll
+            for (int t = 0; t < 16; ++t) bytes[t >> 2][t & 3] = row(t >> 2)[size_t(t & 3) * a.pixelStride + size_t(c)];
+#pragma unroll
+            for (int y = 0; y < 4; ++y) texels.rows[y] = bytes[y][0] | bytes[y][1] << 8 | bytes[y][2] << 16 | bytes[y][3] << 24;
         }
     } else {
-        float texels[4][4][1];
-        source_rows<1, 4>(a, x0, y0, c, texels);
+        float values[4][4][1];
+        source_rows<1, 4>(a, x0, y0, c, values);
 #pragma unroll
-        for (int t = 0; t < 16; ++t) values8[t] = bc4_value8(texels[t >> 2][t & 3][0]);
+        for (int y = 0; y < 4; ++y)
+            texels.rows[y] = bc4_value(values[y][0][0]) | bc4_value(values[y][1][0]) << 8 | bc4_value(values[y][2][0]) << 16 | bc4_value(values[y][3][0]) << 24;
     }
+    bc4_prepare(texels);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -531,36 +723,40 @@ __device__ __forceinline__ uint64_t bc2_alpha(float const (&alpha)[16])
 // A wave encodes one channel of 64 blocks (16 x 4) with one palette, so that the palettes' refinements, each a chain of
 // up to nine passes over the texels, run side by side and not one after the other: a workgroup is the two palettes of
 // both channels of 64 blocks (BC5) or of one channel of 128 (BC4).  The waves of the six-value palette leave their
-// candidates in LDS for those of the eight-value one to choose from.  Bound by vector issue.  2048 x 2048: BC5 58 us, BC4 34
-// (136 and 67 with one lane per block and all of its channels and palettes, two to three instructions per palette entry and
-// the weights from memory; 64 and 36.8 with three instructions for an entry's distance where its number is 0);
-// 64 x 64: 8.7 and 8.5 us (54 and 29).  Three waves per SIMD more at the price of spills, or the indices without registers
-// of their own, are slower (61 to 69 and 35 to 40).
+// candidates in LDS for those of the eight-value one to choose from.  Bound by vector issue: 870 instructions a wave, two
+// thirds of them the refits and passes of the few lanes that go on longest.  2048 x 2048: BC5 29.4 us, BC4 17.9 (57.7 and 34 with
+// the distances to all eight entries and float sums for every refit, 2 200 instructions a wave); 64 x 64: 6.5 us each (8.6).
+// Six, seven or eight waves per SIMD instead of five, with fewer registers, measure the same or 1 us more.
 template <int CHANNELS>
 __global__ void __launch_bounds__(256)
 bc4_compress_kernel(BlockCompressArgs a)
 {
-    __shared__ uint32_t candidates[2][5][64];
+    __shared__ Bc4Tables tables;
+    __shared__ uint64_t candidates[2][64];
+    __shared__ uint32_t errors[2][64];
     int const wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63, pair = wave >> 1;
     int const bx = blockIdx.x * 16 + (lane & 15), by = (CHANNELS == 1 ? blockIdx.y * 8 + pair * 4 : blockIdx.y * 4) + (lane >> 4);
     bool const inside = bx < a.widthInBlocks && by < a.heightInBlocks;
     int const channel = CHANNELS == 1 ? 0 : pair;
     bool const eight = (wave & 1) == 0;
-    uint32_t values8[16], error = 0;
-    Bc4 mine{ 0u, 0u, 0u, 0u };
+    Bc4Texels texels;
+    bc4_stage(tables, 256);
+    if (inside) bc4_load(a, bx, by, channel, texels);
+    __syncthreads();
+    uint64_t mine = 0;
+    uint32_t error = 0;
     if (inside) {
-        bc4_load(a, bx, by, channel, values8);
-        mine = eight ? bc4_candidate<true>(values8, error) : bc4_candidate<false>(values8, error);
-        if (!eight) {
-            candidates[pair][0][lane] = mine.e0; candidates[pair][1][lane] = mine.e1;
-            candidates[pair][2][lane] = mine.low; candidates[pair][3][lane] = mine.high; candidates[pair][4][lane] = error;
+        if (eight) {
+            mine = bc4_bits<true>(bc4_candidate<true>(texels, tables, error));
+        } else {
+            candidates[pair][lane] = bc4_bits<false>(bc4_candidate<false>(texels, tables, error));
+            errors[pair][lane] = error;
         }
     }
     __syncthreads();
     if (!inside || !eight) return;
-    if (candidates[pair][4][lane] < error)
-        mine = Bc4{ candidates[pair][0][lane], candidates[pair][1][lane], candidates[pair][2][lane], candidates[pair][3][lane] };
-    reinterpret_cast<uint64_t*>(a.dst + size_t(by + a.dstOffsetY) * a.dstRowPitch)[size_t(bx + a.dstOffsetX) * CHANNELS + channel] = mine.bits();
+    if (errors[pair][lane] < error) mine = candidates[pair][lane];
+    reinterpret_cast<uint64_t*>(a.dst + size_t(by + a.dstOffsetY) * a.dstRowPitch)[size_t(bx + a.dstOffsetX) * CHANNELS + channel] = mine;
 }
 
 // BC1 (8 bytes per block), BC2 and BC3 (alpha block, then colour block), bound by vector instructions: a block's
@@ -575,8 +771,10 @@ bc4_compress_kernel(BlockCompressArgs a)
 //
 // 64 x 64 and 1024 x 1024: BC1 27 and 29 us in one lane before, 15 and 16 split; BC2 19 and 20, 15 and 15; BC3 25 and 33,
 // 15 and 19.  2048 x 2048: BC1 58 before, 51 (two waves per SIMD with everything in registers; 82 with three that spill; 55
-// split), 46.5 with all pixels loaded at once; BC2 38, 34 (47 split), 31.6; BC3 61, 52 (72 split).  Thirds are selected and not divided, and k / 31 is a product.
+// split), 46.5 with all pixels loaded at once; BC2 38, 34 (47 split), 31.6; BC3 61, 52 (72 split), 40.5 with the alpha search in integers.  Thirds are selected and not divided, and k / 31 is a product.
 struct Bc1Exchange { float4 texels[16][64]; uint32_t words[6][64]; uint64_t alpha[64]; uint32_t sixError[64]; };
+struct NoTables {};
+template <int FORMAT> using Bc1Tables = std::conditional_t<FORMAT == 3, Bc4Tables, NoTables>;          // of the alpha search
 template <int FORMAT> constexpr int kBc1Waves = FORMAT == 3 ? 3 : 2;
 
 template <int FORMAT>
@@ -602,6 +800,8 @@ __global__ void __launch_bounds__(64 * kBc1Waves<FORMAT>) __attribute__((amdgpu_
 bc1_compress_split_kernel(BlockCompressArgs a)
 {
     __shared__ Bc1Exchange exchange;
+    __shared__ Bc1Tables<FORMAT> tables;
+    if constexpr (FORMAT == 3) bc4_stage(tables, 64 * kBc1Waves<FORMAT>);
     int const wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63;
     int const bx = blockIdx.x * 16 + (lane & 15), by = blockIdx.y * 4 + (lane >> 4);
     bool const inside = bx < a.widthInBlocks && by < a.heightInBlocks;
@@ -623,18 +823,23 @@ bc1_compress_split_kernel(BlockCompressArgs a)
         }
     }
     __syncthreads();
-    auto const alpha_candidate = [&](auto eight, uint32_t& error) {
-        uint32_t values8[16];
+    auto const alpha_candidate = [&](auto eight, auto const& tables, uint32_t& error) {
+        Bc4Texels texels;
 #pragma unroll
-        for (int t = 0; t < 16; ++t) values8[t] = bc4_value8(exchange.texels[t][lane].w);
-        return bc4_candidate<decltype(eight)::value>(values8, error);
+        for (int y = 0; y < 4; ++y) {
+            texels.rows[y] = 0;
+#pragma unroll
+            for (int x = 0; x < 4; ++x) texels.rows[y] |= bc4_value(exchange.texels[4 * y + x][lane].w) << (8 * x);
+        }
+        bc4_prepare(texels);
+        return bc4_bits<decltype(eight)::value>(bc4_candidate<decltype(eight)::value>(texels, tables, error));
     };
     ColorBlock best{ 0u, 0u, 0.f };
-    Bc4 alphaBlock{ 0u, 0u, 0u, 0u };
+    uint64_t alphaBlock = 0;
     uint32_t alphaError = 0;
     if (inside) {
         if (wave == 2) {
-            alphaBlock = alpha_candidate(std::true_type{}, alphaError);
+            if constexpr (FORMAT == 3) alphaBlock = alpha_candidate(std::true_type{}, tables, alphaError);
         } else {
             Rgba px[16];
 #pragma unroll
@@ -656,8 +861,7 @@ bc1_compress_split_kernel(BlockCompressArgs a)
                     for (int t = 0; t < 16; ++t) alpha[t] = exchange.texels[t][lane].w;
                     exchange.alpha[lane] = bc2_alpha(alpha);
                 } else {
-                    alphaBlock = alpha_candidate(std::false_type{}, alphaError);
-                    exchange.alpha[lane] = alphaBlock.bits();
+                    exchange.alpha[lane] = alpha_candidate(std::false_type{}, tables, alphaError);
                     exchange.sixError[lane] = alphaError;
                 }
             }
@@ -667,7 +871,7 @@ bc1_compress_split_kernel(BlockCompressArgs a)
     if (!inside || wave == 1) return;
     uint64_t* const dst = bc1_place<FORMAT>(a, bx, by);
     if (wave == 2) {
-        dst[0] = exchange.sixError[lane] < alphaError ? exchange.alpha[lane] : alphaBlock.bits();
+        dst[0] = exchange.sixError[lane] < alphaError ? exchange.alpha[lane] : alphaBlock;
         return;
     }
     ColorBlock chosen{ exchange.words[0][lane], exchange.words[1][lane], __uint_as_float(exchange.words[2][lane]) };
@@ -690,6 +894,11 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(FORMAT
 bc1_compress_kernel(BlockCompressArgs a)
 {
     int const bx = blockIdx.x * 16 + (threadIdx.x & 15), by = blockIdx.y * 8 + (threadIdx.x >> 4);
+    __shared__ Bc1Tables<FORMAT> tables;
+    if constexpr (FORMAT == 3) {
+        bc4_stage(tables, 128);
+        __syncthreads();
+    }
     if (bx >= a.widthInBlocks || by >= a.heightInBlocks) return;
     Rgba px[16];
     float alpha[16];
@@ -706,11 +915,14 @@ bc1_compress_kernel(BlockCompressArgs a)
     uint64_t* const dst = bc1_place<FORMAT>(a, bx, by);
     if constexpr (FORMAT == 2) dst[0] = bc2_alpha(alpha);
     if constexpr (FORMAT == 3) {
-        uint32_t values8[16], error8, error6;
+        Bc4Texels texels;
+        uint32_t error8, error6;
 #pragma unroll
-        for (int t = 0; t < 16; ++t) values8[t] = bc4_value8(alpha[t]);
-        Bc4 const block8 = bc4_candidate<true>(values8, error8), block6 = bc4_candidate<false>(values8, error6);
-        dst[0] = error6 < error8 ? block6.bits() : block8.bits();
+        for (int y = 0; y < 4; ++y)
+            texels.rows[y] = bc4_value(alpha[4 * y]) | bc4_value(alpha[4 * y + 1]) << 8 | bc4_value(alpha[4 * y + 2]) << 16 | bc4_value(alpha[4 * y + 3]) << 24;
+        bc4_prepare(texels);
+        Bc4 const block8 = bc4_candidate<true>(texels, tables, error8), block6 = bc4_candidate<false>(texels, tables, error6);
+        dst[0] = error6 < error8 ? bc4_bits<false>(block6) : bc4_bits<true>(block8);
     }
     ColorBlock best = bc1_simple_candidates<FORMAT == 1>(px, a.alphaThreshold);
     ColorBlock const four = bc1_four_colors<FORMAT != 1>(px);

@@ -114,6 +114,58 @@ struct Bc4Palette {
     }
 };
 
+// bc4_assign(): every pair of endpoints and every value, sixteen values a block, in the search that the pair belongs to.
+struct Bc4Positions {
+    static constexpr uint64_t cases = 65536 * 16;
+    static __device__ int check(uint64_t i)
+    {
+        uint32_t const e0 = uint32_t(i >> 12), e1 = uint32_t(i >> 4) & 255u, first = (uint32_t(i) & 15u) * 16u;
+        Bc4Texels texels;
+        for (uint32_t r = 0; r < 4; ++r) texels.rows[r] = (first + 4u * r) * 0x01010101u + 0x03020100u;
+        bc4_prepare(texels);
+        Bc4 got{ e0, e1, {} }, want{ e0, e1, {} };
+        uint32_t const gotError = e0 > e1 ? bc4_assign<true>(texels, kBc4Tables, got) : bc4_assign<false>(texels, kBc4Tables, got);
+        uint32_t const wantError = e0 > e1 ? bc4_assign_defined<true>(texels, want) : bc4_assign_defined<false>(texels, want);
+        bool right = gotError == wantError;
+        for (int r = 0; r < 4; ++r) right = right && got.positions[r] == want.positions[r];
+        return verdict(right);
+    }
+};
+// bc4_refit(): 2^24 blocks, smooth ones, noise and blocks of few values, whose ties the float sums decide.
+struct Bc4Refit {
+    static constexpr uint64_t cases = uint64_t(1) << 24;
+    template <bool EIGHT> static __device__ bool same_endpoints(Bc4Texels const& texels, Bc4 block)
+    {
+        Bc4 got = block;
+        bc4_refit<EIGHT>(texels, got, false, false);
+        float e0, e1;
+        bc4_solve_defined<EIGHT>(texels, block, e0, e1);
+        return EIGHT ? got.e0 == uint32_t(fmaxf(e0, e1)) && got.e1 == uint32_t(fminf(e0, e1)) : got.e0 == uint32_t(e0) && got.e1 == uint32_t(e1);
+    }
+    static __device__ int check(uint64_t i)
+    {
+        uint64_t h = (i + 1) * 0x9e3779b97f4a7c15ull;
+        auto const next = [&] { h ^= h >> 29; h *= 0xbf58476d1ce4e5b9ull; h ^= h >> 32; return uint32_t(h); };
+        uint32_t const kind = uint32_t(i) & 3u, base = next() & 127u, pool = next();
+        Bc4Texels texels;
+        for (int r = 0; r < 4; ++r) {
+            uint32_t const bits = next();
+            texels.rows[r] = 0;
+            for (int x = 0; x < 4; ++x) {
+                uint32_t const b = (bits >> (8 * x)) & 255u;
+                uint32_t const v = kind == 0 ? b : kind == 1 ? base + (b & 15u) + 8u * uint32_t(r + x) : kind == 2 ? (pool >> (8u * (b & 3u))) & 255u : base + (b & 31u);
+                texels.rows[r] |= v << (8 * x);
+            }
+        }
+        bc4_prepare(texels);
+        uint32_t const hi = texels.hi, lo = texels.lo;
+        Bc4 eight{ hi, lo, {} }, six{ lo + (hi - lo) / 8u, hi - (hi - lo) / 8u, {} };
+        bc4_assign_defined<true>(texels, eight);
+        bc4_assign_defined<false>(texels, six);
+        return verdict(same_endpoints<true>(texels, eight) && same_endpoints<false>(texels, six));
+    }
+};
+
 #elif defined(SUBJECT_BC6)
 
 // quotient<0>(): integers below 2^17.
@@ -214,6 +266,8 @@ int exact_divide_by_65535(Report* r) { return sweep<DivideByTop<65535>>(r); }
 #elif defined(SUBJECT_BC)
 int exact_code_quotient(Report* r) { return sweep<CodeQuotient>(r); }
 int exact_bc4_palette(Report* r) { return sweep<Bc4Palette>(r); }
+int exact_bc4_positions(Report* r) { return sweep<Bc4Positions>(r); }
+int exact_bc4_refit(Report* r) { return sweep<Bc4Refit>(r); }
 #elif defined(SUBJECT_BC6)
 int exact_quotient_of_integers(Report* r) { return sweep<QuotientOfIntegers>(r); }
 int exact_quotient_of_log2(Report* r) { return sweep<QuotientOfLog2>(r); }

@@ -19,7 +19,7 @@ class Report(C.Structure):
 @pytest.mark.parametrize("subject,function,cases", [
     ("copy", "encoded_half_srgb", 1 << 32), ("copy", "encoded_half_hlg", 1 << 32),
     ("copy", "put_unorm8", 1 << 32), ("copy", "divide_by_255", (1 << 23) + 256), ("copy", "divide_by_65535", (1 << 23) + 65536),
-    ("bc", "code_quotient", 96), ("bc", "bc4_palette", 65536),
+    ("bc", "code_quotient", 96), ("bc", "bc4_palette", 65536), ("bc", "bc4_positions", 1 << 20), ("bc", "bc4_refit", 1 << 24),
     ("bc6", "quotient_of_integers", (1 << 17) * ((1 << 17) - 1)), ("bc6", "quotient_of_log2", None),
     ("bc6", "quotient_of_msle", 0x7c00 * (0x7c00 + 256 + 65536 + 65505)), ("bc6", "log_estimate", 34 << 23), ("bc6", "quotient_of_codes", 3 * 65536 + 64),
     ("bc6", "quotient_of_diagonals", 1 << 30), ("decode", "texel_centre", (1 << 15) * 65537)])
