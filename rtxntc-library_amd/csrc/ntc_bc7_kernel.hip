@@ -530,9 +530,11 @@ BC7_INLINE void store_block(BlockCompressArgs const& a, int bx, int by, uint64_t
 //      opaque blocks, of two subsets for mode 7.  Tasks of a range of its partitions bound the errors from below, all
 //      lanes with the same partition; when a search's are done, one more task estimates the error of the partition with
 //      the smallest bound and queues those whose bounds do not exceed it: one to seven of 64 on textures with detail.
-//   2. Tasks of 64 queued estimates, from any blocks of a search; tasks of one candidate, or of the three forms of modes 4
-//      and 5 of one channel rotation, from its endpoints to the encoded block, where every lane has a partition of its
-//      own and walks its own list of texels.
+//      Beside them a task for each group: lower bounds of the errors of the four channel rotations of modes 4 and 5 and of
+//      mode 6, then the three forms of the rotation with the smallest one, whose error leaves out what is bounded above it.
+//   2. Tasks of 64 queued estimates, from any blocks of a search; tasks of 64 rotations or of 64 blocks of mode 6 that were
+//      not left out; tasks of one candidate, from its endpoints to the encoded block, where every lane has a partition of
+//      its own and walks its own list of texels.
 //   3. A thread per block goes through the candidates in the order given at the top with "not larger replaces".
 // Blocks with and without alpha are gathered in groups of their own for the tasks that only one kind has.  Waves take the
 // tasks of a phase in turn; one that builds upon others waits for their count.
@@ -548,11 +550,17 @@ BC7_INLINE void store_block(BlockCompressArgs const& a, int bx, int by, uint64_t
 // overflows or 48 of 64 blocks are near a line / now: grey 272 / 239 / 239 us, noise of 1.5 codes on proportional channels
 // 273 / 275 / 240 and of 4 codes 274 / 307 / 240, hard edges in every block 276 / 299 / 243 and with noise 275 / 306 / 245,
 // antialiased boxes and strokes 278 / 317 / 244 and with noise 275 / 317 / 241; not antialiased 272 / 174 / 187.
+// Rotations and mode 6 by their bounds: of the half opaque image all blocks' mode 6 but 12 to 14 %, 2 of 5 (opaque) or of 2
+// (others) rotations; where alphas are 1 their planes have two channels: 1024 x 1024 opaque noise 187 -> 162 us, a smooth
+// image 234 -> 226, grey 240 -> 234, hard edges 243 -> 237, ramps 191 -> 183, one colour 151 -> 149.
 //
 // Wave priorities fall from phase to phase.  With equal ones the older of the two workgroups of a compute unit runs ahead
 // through the first phase and leaves the younger one alone with half the waves at the end (347 and 485 thousand cycles at
 // 1024 x 1024); a workgroup that is behind now comes first (365 and 422 thousand; 209 -> 188 us).
-enum { kSlots = 10, kPickThree = 0, kPickTwo, kPickTwoAlpha, kPicks };
+// Slots of candidates: modes 0, 2, 1, 3, the rotations after the first in their order, modes 6 and 7.
+enum { kSlotRotations = 4, kSlotSix = 7, kSlotSeven, kSlots };
+enum : uint32_t { kKeepRotation = 4, kKeepSix = 64 };
+enum { kPickThree = 0, kPickTwo, kPickTwoAlpha, kPicks };
 enum : uint32_t { kBelowOne = 1, kNotOne = 2 };              // what some alpha of a block is (one above 1 or a NaN is only the second)
 
 // The searches of a workgroup: its opaque groups' partitions of two subsets, then of three, then the partitions for mode 7
@@ -567,16 +575,19 @@ struct SearchLds {
     uint32_t lowest[kPicks][BLOCKS];                         // the smallest bound's bits, the low six replaced by its partition
     union {
         uint32_t bounds[kPicks][16][BLOCKS];                 // codes of four partitions each; until the picks are made
-        struct { uint4 words[kSlots - 1][BLOCKS]; float errors[kSlots - 1][BLOCKS]; } late;
+        struct { uint4 words[kSlots][BLOCKS]; float errors[kSlots][BLOCKS]; } late;
     };
-    struct { uint4 words[BLOCKS]; float errors[BLOCKS]; } early;                   // mode 6
+    struct { uint4 words[BLOCKS]; float errors[BLOCKS]; } early;                   // the first rotation's candidate (before: least errors of all four)
+    uint32_t plans[BLOCKS];                                  // the first rotation; kKeepRotation << r and kKeepSix
+    uint16_t flatRotations[2 * BLOCKS], rotations[3 * BLOCKS];                     // those kept, rotation << 7 | block: with planes of two channels, of three
+    uint8_t sixes[BLOCKS];                                   // blocks that mode 6 is kept for
     uint16_t queues[kSearches][kQueued];                     // partition << 7 | block
     int queued[kSearches];
     uint8_t whole[kSearches];                                // searches that estimate every partition
     uint32_t alphas[BLOCKS];                                 // kBelowOne | kNotOne
     uint8_t blocks[2][BLOCKS];                               // numbers of the opaque blocks, of those with alpha
-    int counts[2], next[2], wholes;
-    int bounded[kSearches], estimated;                       // tasks done: those of a search's bounds, those of estimates
+    int counts[2], next[2], wholes, kept[3];                 // kept: rotations of both kinds, mode 6
+    int bounded[kSearches], selected, rotated, estimated;    // tasks done: those of a search's bounds, of selections, first rotations and estimates
 };
 template <class S> using SearchPtr = __attribute__((address_space(3))) S*;
 
@@ -1225,15 +1236,10 @@ BC7_INLINE uint64_t without_bit(uint64_t v, int at)
     return (v & below) | ((v >> 1) & ~below);
 }
 
-// Slot 8, mode 6, has a place of its own: it is there before the picks are made.
-template <class S> BC7_INLINE void put_candidate(SearchPtr<S> lds, int slot, int b, float error, uint64_t lo, uint64_t hi)
+template <class W, class E> BC7_INLINE void put_candidate(W words, E errors, float error, uint64_t lo, uint64_t hi)
 {
-    auto const put = [&](auto words, auto errors) {
-        *errors = error;
-        words->x = uint32_t(lo); words->y = uint32_t(lo >> 32); words->z = uint32_t(hi); words->w = uint32_t(hi >> 32);
-    };
-    if (slot == 8) put(&lds->early.words[b], &lds->early.errors[b]);             // uniform
-    else           put(&lds->late.words[min(slot, 8)][b], &lds->late.errors[min(slot, 8)][b]);
+    *errors = error;
+    words->x = uint32_t(lo); words->y = uint32_t(lo >> 32); words->z = uint32_t(hi); words->w = uint32_t(hi >> 32);
 }
 
 template <class S, class M, int C, bool ORIENT>
@@ -1316,17 +1322,25 @@ BC7_TASK void finish_task(SearchPtr<S> lds, int b, int pick, int slot)
     }
     indices = without_bit(indices, top);
     put_indices(bits.lo, bits.hi, bits.at, indices);
-    put_candidate<S>(lds, slot, b, error, bits.lo, bits.hi);
+    put_candidate(&lds->late.words[slot][b], &lds->late.errors[slot][b], error, bits.lo, bits.hi);
 }
 
-// The colour plane and the scalar plane of a texel under a channel rotation (uniform).
-template <class S> BC7_INLINE void planes_of(SearchPtr<S> lds, int b, int t, int rotation, Color<3>& rgb, Color<1>& a)
+// The colour plane and the scalar plane of a texel under the lane's channel rotation.  C = 2: every alpha of the lane's
+// block is 1 and the rotation takes a colour channel out, so that the plane is the other two and that 1 in its place: its
+// differences are zeros, which sums do not see, and its ends stay 1, which decodes to 1.
+template <int C, class S> BC7_INLINE void planes_of(SearchPtr<S> lds, int b, int t, int rotation, Color<C>& plane, Color<1>& a)
 {
     Color<4> const p = texel<4, S>(lds, b, t);
-    rgb.c[0] = rotation == 1 ? p.c[3] : p.c[0];
-    rgb.c[1] = rotation == 2 ? p.c[3] : p.c[1];
-    rgb.c[2] = rotation == 3 ? p.c[3] : p.c[2];
-    a.c[0] = rotation == 0 ? p.c[3] : rotation == 1 ? p.c[0] : rotation == 2 ? p.c[1] : p.c[2];
+    if constexpr (C == 2) {
+        plane.c[0] = rotation == 1 ? p.c[1] : p.c[0];
+        plane.c[1] = rotation == 3 ? p.c[1] : p.c[2];
+        a.c[0] = rotation == 1 ? p.c[0] : rotation == 2 ? p.c[1] : p.c[2];
+    } else {
+        plane.c[0] = rotation == 1 ? p.c[3] : p.c[0];
+        plane.c[1] = rotation == 2 ? p.c[3] : p.c[1];
+        plane.c[2] = rotation == 3 ? p.c[3] : p.c[2];
+        a.c[0] = rotation == 0 ? p.c[3] : rotation == 1 ? p.c[0] : rotation == 2 ? p.c[1] : p.c[2];
+    }
 }
 
 template <int FORM> struct DualForm {                        // mode 4 with 2-bit colour indices, with 3-bit ones, mode 5
@@ -1334,39 +1348,48 @@ template <int FORM> struct DualForm {                        // mode 4 with 2-bi
     static constexpr int colorBits = FORM == 2 ? 7 : 5, alphaBits = FORM == 2 ? 8 : 6;
 };
 
-template <class S, int FORM>
-BC7_TASK void dual_plane_form(SearchPtr<S> lds, int b, int rotation, Ends<3> color, Ends<1> alpha, Best& best)
+template <class S, int FORM, int C>
+BC7_TASK void dual_plane_form(SearchPtr<S> lds, int b, int rotation, Ends<C> color, Ends<1> alpha, Best& best)
 {
     using F = DualForm<FORM>;
-    rotation = __builtin_amdgcn_readfirstlane(rotation);
-    Quantized<3> q0, q1;
+    Quantized<C> q0, q1;
     Quantized<1> qa0, qa1;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) { q0.c[k] = quantize(color.e0.c[k], F::colorBits); q1.c[k] = quantize(color.e1.c[k], F::colorBits); }
+    for (int k = 0; k < C; ++k) { q0.c[k] = quantize(color.e0.c[k], F::colorBits); q1.c[k] = quantize(color.e1.c[k], F::colorBits); }
     qa0.c[0] = quantize(alpha.e0.c[0], F::alphaBits); qa1.c[0] = quantize(alpha.e1.c[0], F::alphaBits);
-    Decoded<3, F::colorIndexBits> const colorEnds(q0, q1, F::colorBits);
+    Decoded<C, F::colorIndexBits> const colorEnds(q0, q1, F::colorBits);
     Decoded<1, F::alphaIndexBits> const alphaEnds(qa0, qa1, F::alphaBits);
     uint64_t colorIndices = 0, alphaIndices = 0;
     float colorError = 0.f, alphaError = 0.f;
 #pragma unroll 4
     for (int t = 0; t < 16; ++t) {
-        Color<3> rgb;
+        Color<C> rgb;
         Color<1> a;
-        planes_of<S>(lds, b, t, rotation, rgb, a);
+        planes_of<C, S>(lds, b, t, rotation, rgb, a);
         colorIndices |= uint64_t(colorEnds.index(rgb, colorError)) << (t * F::colorIndexBits);
         alphaIndices |= uint64_t(alphaEnds.index(a, alphaError)) << (t * F::alphaIndexBits);
     }
     float const error = colorError + alphaError;
     if (error > best.error) return;
     auto const complemented = [](uint64_t v, int bits) { return bits == 2 ? v ^ 0xffffffffull : v ^ 0xffffffffffffull; };
-    if (colorIndices & (1u << (F::colorIndexBits - 1))) { colorIndices = complemented(colorIndices, F::colorIndexBits); Quantized<3> const x = q0; q0 = q1; q1 = x; }
+    if (colorIndices & (1u << (F::colorIndexBits - 1))) { colorIndices = complemented(colorIndices, F::colorIndexBits); Quantized<C> const x = q0; q0 = q1; q1 = x; }
     if (alphaIndices & (1u << (F::alphaIndexBits - 1))) { alphaIndices = complemented(alphaIndices, F::alphaIndexBits); Quantized<1> const x = qa0; qa0 = qa1; qa1 = x; }
     Bits bits;
     bits.put(F::mode + 1, 1u << F::mode);
     bits.put(2, uint32_t(rotation));
     if constexpr (F::mode == 4) bits.put(1, FORM == 1 ? 1u : 0u);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) { bits.put(F::colorBits, uint32_t(q0.c[k])); bits.put(F::colorBits, uint32_t(q1.c[k])); }
+    for (int k = 0; k < 3; ++k) {
+        uint32_t v0, v1;
+        if constexpr (C == 2) {                              // the alpha's place is that of the rotation
+            constexpr uint32_t one = (1u << F::colorBits) - 1u;
+            v0 = rotation == k + 1 ? one : uint32_t(k == 0 ? q0.c[0] : k == 2 ? q0.c[1] : rotation == 1 ? q0.c[0] : q0.c[1]);
+            v1 = rotation == k + 1 ? one : uint32_t(k == 0 ? q1.c[0] : k == 2 ? q1.c[1] : rotation == 1 ? q1.c[0] : q1.c[1]);
+        } else {
+            v0 = uint32_t(q0.c[k]); v1 = uint32_t(q1.c[k]);
+        }
+        bits.put(F::colorBits, v0); bits.put(F::colorBits, v1);
+    }
     bits.put(F::alphaBits, uint32_t(qa0.c[0])); bits.put(F::alphaBits, uint32_t(qa1.c[0]));
     colorIndices = without_bit(colorIndices, F::colorIndexBits - 1);
     alphaIndices = without_bit(alphaIndices, F::alphaIndexBits - 1);
@@ -1379,33 +1402,32 @@ BC7_TASK void dual_plane_form(SearchPtr<S> lds, int b, int rotation, Ends<3> col
 
 // The refined ends of one rotation's planes, for 2-bit and for 3-bit indices: mode 5 shares its colour ends with mode
 // 4's narrow form and its scalar ends with the wide form.
-template <class S>
-BC7_TASK void dual_plane_ends(SearchPtr<S> lds, int b, int rotation, Ends<3> (&color)[2], Ends<1> (&alpha)[2])
+template <class S, int C>
+BC7_TASK void dual_plane_ends(SearchPtr<S> lds, int b, int rotation, Ends<C> (&color)[2], Ends<1> (&alpha)[2])
 {
-    rotation = __builtin_amdgcn_readfirstlane(rotation);
-    Ends<3> c;
+    Ends<C> c;
     Ends<1> s;
     {
-        Color<3> center;
-        for (int k = 0; k < 3; ++k) { c.e0.c[k] = FLT_MAX; c.e1.c[k] = -FLT_MAX; center.c[k] = 0.f; }
+        Color<C> center;
+        for (int k = 0; k < C; ++k) { c.e0.c[k] = FLT_MAX; c.e1.c[k] = -FLT_MAX; center.c[k] = 0.f; }
         s.e0.c[0] = FLT_MAX; s.e1.c[0] = -FLT_MAX;
 #pragma unroll 4
         for (int t = 0; t < 16; ++t) {
-            Color<3> rgb;
+            Color<C> rgb;
             Color<1> a;
-            planes_of<S>(lds, b, t, rotation, rgb, a);
+            planes_of<C, S>(lds, b, t, rotation, rgb, a);
 #pragma unroll
-            for (int k = 0; k < 3; ++k) { c.e0.c[k] = min_f32(c.e0.c[k], rgb.c[k]); c.e1.c[k] = max_f32(c.e1.c[k], rgb.c[k]); center.c[k] += rgb.c[k]; }
+            for (int k = 0; k < C; ++k) { c.e0.c[k] = min_f32(c.e0.c[k], rgb.c[k]); c.e1.c[k] = max_f32(c.e1.c[k], rgb.c[k]); center.c[k] += rgb.c[k]; }
             s.e0.c[0] = min_f32(s.e0.c[0], a.c[0]); s.e1.c[0] = max_f32(s.e1.c[0], a.c[0]);
         }
 #pragma unroll
-        for (int k = 0; k < 3; ++k) center.c[k] /= 16.f;
-        float cov[3][3] = {};
+        for (int k = 0; k < C; ++k) center.c[k] /= 16.f;
+        float cov[C][C] = {};
 #pragma unroll 4
         for (int t = 0; t < 16; ++t) {
-            Color<3> rgb;
+            Color<C> rgb;
             Color<1> a;
-            planes_of<S>(lds, b, t, rotation, rgb, a);
+            planes_of<C, S>(lds, b, t, rotation, rgb, a);
             add_covariance(cov, sub(rgb, center));
         }
         orient_by(cov, c.e0, c.e1);
@@ -1415,9 +1437,9 @@ BC7_TASK void dual_plane_ends(SearchPtr<S> lds, int b, int rotation, Ends<3> (&c
     bool colorGoesOn[2] = { true, true }, alphaGoesOn[2] = { true, true };
 #pragma unroll 1
     for (int iter = 0; iter < 2; ++iter) {
-        Refinement<3> colorSums[2];
+        Refinement<C> colorSums[2];
         Refinement<1> alphaSums[2];
-        Color<3> axis[2];
+        Color<C> axis[2];
         Color<1> range[2];
         float mul[2], scale[2];
 #pragma unroll
@@ -1427,9 +1449,9 @@ BC7_TASK void dual_plane_ends(SearchPtr<S> lds, int b, int rotation, Ends<3> (&c
         }
 #pragma unroll 2
         for (int t = 0; t < 16; ++t) {
-            Color<3> rgb;
+            Color<C> rgb;
             Color<1> a;
-            planes_of<S>(lds, b, t, rotation, rgb, a);
+            planes_of<C, S>(lds, b, t, rotation, rgb, a);
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 colorSums[i].add(saturate(dot(sub(rgb, color[i].e0), axis[i]) * mul[i]), rgb, 2 + i);
@@ -1442,6 +1464,96 @@ BC7_TASK void dual_plane_ends(SearchPtr<S> lds, int b, int rotation, Ends<3> (&c
             if (alphaGoesOn[i]) alphaGoesOn[i] = alphaSums[i].solve(alpha[i].e0, alpha[i].e1);
         }
     }
+}
+
+// ---- what rotations cannot win
+//
+// A decoder shows a plane of three channels as points of a line, each component rounded to eight bits, so that the plane's
+// error is at least the squared distances from the best line, trace less largest eigenvalue of the centred moments, with the
+// roundings taken off: sqrt(error) >= sqrt(distances) - 4 sqrt(3) / 510, sixteen texels of three components that round by 1/510
+// (two where the third is an alpha of 1, which is shown exactly).  That holds for modes 4 and 5 of the rotation and for
+// mode 6, whose line lies in four channels, with any three of them.
+// Moments are of offsets from texel 0, T the sum of their squares, within 40 units of roundoff of T each, so that distances are
+// within 240: kBoundError covers them.  The eigenvalue is bounded by m + 2 p, m the mean eigenvalue and 6 p^2 the squared
+// deviations from it, and brought down by Newton's steps, which stay above the largest root of the characteristic
+// polynomial; in units of the trace that and its derivative are within 2^-17 of themselves, which the steps leave out.
+// Blocks whose T is no number between kLeastOffsets and kMostOffsets have no bounds.
+template <class S> BC7_TASK void bound_rotations(SearchPtr<S> lds, int b)
+{
+    Color<4> const origin = texel<4, S>(lds, b, 0);
+    Sums<4> sums;
+#pragma unroll 5
+    for (int t = 1; t < 16; ++t) sums.add(sub(texel<4, S>(lds, b, t), origin));
+    float const offsets = sums.trace();
+    bool const bounded = offsets >= kLeastOffsets && offsets <= kMostOffsets, ones = !(lds->alphas[b] & kNotOne);
+    float m[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = i; j < 4; ++j) m[i][j] = m[j][i] = __builtin_fmaf(sums.s[i] * (-1.f / 16.f), sums.s[j], sums.q[i][j]);
+    float least[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        int const x = r == 1 ? 3 : 0, y = r == 2 ? 3 : 1, z = r == 3 ? 3 : 2;
+        float const trace = m[x][x] + m[y][y] + m[z][z], unit = __builtin_amdgcn_rcpf(trace);
+        float const xx = m[x][x] * unit, yy = m[y][y] * unit, zz = m[z][z] * unit, xy = m[x][y] * unit, xz = m[x][z] * unit, yz = m[y][z] * unit;
+        float const mixed = __builtin_fmaf(xy, xy, __builtin_fmaf(xz, xz, yz * yz));
+        float const squares = __builtin_fmaf(xx, xx, __builtin_fmaf(yy, yy, __builtin_fmaf(zz, zz, mixed + mixed)));
+        float const c1 = __builtin_fmaf(xx, yy, __builtin_fmaf(xx, zz, __builtin_fmaf(yy, zz, -mixed)));
+        float const c0 = __builtin_fmaf(xx, __builtin_fmaf(yy, zz, -yz * yz), __builtin_fmaf(2.f * xy, xz * yz, -__builtin_fmaf(xz * xz, yy, xy * xy * zz)));
+        float root = __builtin_fmaf(2.f, __builtin_amdgcn_sqrtf((fmaxf(squares - 1.f / 3.f, 0.f) + 0x1p-20f) * (1.f / 6.f)), 1.f / 3.f);
+#pragma unroll
+        for (int step = 0; step < 3; ++step) {
+            float const value = __builtin_fmaf(root, __builtin_fmaf(root, root - 1.f, c1), -c0), slope = __builtin_fmaf(root, __builtin_fmaf(3.f, root, -2.f), c1);
+            root = __builtin_fmaf(-fmaxf(value - 0x1p-17f, 0.f), __builtin_amdgcn_rcpf(fmaxf(slope, 0.f) + 0x1p-16f), root);
+        }
+        float const distances = __builtin_fmaf(trace, 1.f - 0x1p-16f - root, -kBoundError * offsets);
+        float const rounding = (r != 0 && ones ? 1.4142f : 1.7321f) * (4.f * 1.001f / 510.f);
+        float const rest = fmaxf(__builtin_amdgcn_sqrtf(fmaxf(distances, 0.f)) - rounding, 0.f);           // (a NaN: 0)
+        least[r] = bounded ? rest * rest * (1.f - 0x1p-10f) : 0.f;
+    }
+    lds->early.words[b].x = __float_as_uint(least[0]); lds->early.words[b].y = __float_as_uint(least[1]);
+    lds->early.words[b].z = __float_as_uint(least[2]); lds->early.words[b].w = __float_as_uint(least[3]);
+}
+// The rotation of the smallest bound; where alphas are 1 not 0, whose plane has all that leaves the other ones' lines.
+template <class S> BC7_INLINE int first_rotation(SearchPtr<S> lds, int b)
+{
+    bool const ones = !(lds->alphas[b] & kNotOne);
+    float const least[4] = { __uint_as_float(lds->early.words[b].x), __uint_as_float(lds->early.words[b].y), __uint_as_float(lds->early.words[b].z), __uint_as_float(lds->early.words[b].w) };
+    int const low = ones || least[1] < least[0] ? 1 : 0, high = least[3] < least[2] ? 3 : 2;
+    return fminf(least[2], least[3]) < (low ? least[1] : least[0]) ? high : low;
+}
+// With the first rotation's error: the other rotations and mode 6 into their lists where their bounds do not exceed it.
+template <class S> BC7_INLINE void keep_candidates(SearchPtr<S> lds, int b, int first, float error, bool mine)
+{
+    float const least[4] = { __uint_as_float(lds->early.words[b].x), __uint_as_float(lds->early.words[b].y), __uint_as_float(lds->early.words[b].z), __uint_as_float(lds->early.words[b].w) };
+    bool const ones = !(lds->alphas[b] & kNotOne);
+    uint32_t plan = uint32_t(first);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) if (r != first && !(least[r] > error)) plan |= kKeepRotation << r;
+    if (!(fmaxf(fmaxf(least[0], least[1]), fmaxf(least[2], least[3])) > error)) plan |= kKeepSix;
+    if (!mine) return;
+    lds->plans[b] = plan;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        if (plan & (kKeepRotation << r)) {
+            if (r > 0 && ones) lds->flatRotations[atomicAdd((int*)&lds->kept[0], 1)] = uint16_t(r << 7 | b);
+            else               lds->rotations[atomicAdd((int*)&lds->kept[1], 1)] = uint16_t(r << 7 | b);
+        }
+    if (plan & kKeepSix) lds->sixes[atomicAdd((int*)&lds->kept[2], 1)] = uint8_t(b);
+}
+
+// Modes 4 and 5 of the lane's rotation: the best of their three forms.
+template <class S, int C> BC7_INLINE Best dual_planes(SearchPtr<S> lds, int b, int rotation)
+{
+    Ends<C> color[2];                                        // refined for 2-bit and 3-bit indices
+    Ends<1> alpha[2];
+    dual_plane_ends<S, C>(lds, b, rotation, color, alpha);
+    Best best{ FLT_MAX, 0, 0 };
+    dual_plane_form<S, 0, C>(lds, b, rotation, color[0], alpha[1], best);
+    dual_plane_form<S, 1, C>(lds, b, rotation, color[1], alpha[0], best);
+    dual_plane_form<S, 2, C>(lds, b, rotation, color[0], alpha[0], best);
+    return best;
 }
 
 template <int GROUPS, int WAVES>
@@ -1471,7 +1583,7 @@ bc7_compress_kernel(BlockCompressArgs a)
     }
     if (tid < kSearches) shared.queued[tid] = shared.bounded[tid] = 0;
     if (tid < 2) shared.next[tid] = 0;
-    if (tid == 0) shared.wholes = shared.estimated = 0;
+    if (tid == 0) shared.wholes = shared.selected = shared.rotated = shared.estimated = shared.kept[0] = shared.kept[1] = shared.kept[2] = 0;
     __syncthreads();
     if (int const b = tid % BLOCKS, row = tid / BLOCKS; row < 4) {
         int const bx = block_x(b), by = block_y(b);
@@ -1505,6 +1617,7 @@ bc7_compress_kernel(BlockCompressArgs a)
     // the lane's block of a group of one kind (lanes beyond the last block repeat it)
     auto const block_of = [&](int kind, int group) { return int(shared.blocks[kind][min(64 * group + lane, (kind ? withAlpha : opaque) - 1)]); };
     auto const block_of_group = [&](int group) { return group < opaqueGroups ? block_of(0, group) : block_of(1, group - opaqueGroups); };
+    auto const own_lane = [&](int group) { return 64 * (group < opaqueGroups ? group : group - opaqueGroups) + lane < (group < opaqueGroups ? opaque : withAlpha); };
 
     // Waits for the earlier tasks that a task builds upon: each was taken before it, by a wave that comes to its end.
     auto const wait_for = [&](int& counter, int count) {
@@ -1523,11 +1636,20 @@ bc7_compress_kernel(BlockCompressArgs a)
     auto const what_of = [&](int search, int b) { return kind_of(search) != kPickTwoAlpha ? kind_of(search) : group_of(search) < opaqueGroups && all_ones(b) ? int(kCorners3) : int(kCorners4); };
     auto const bounds_of = [&](int search) { return kind_of(search) == kPickTwoAlpha && group_of(search) < opaqueGroups ? group_of(search) : search; };
 
-    // ---- 1. bounds of the partitions' errors; mode 6, which has no partitions; the errors of the first partitions
+    // ---- 1. bounds of the partitions' errors; one rotation of modes 4 and 5 for each block; the errors of the first partitions
     __builtin_amdgcn_s_setprio(3);
     int const searches = 2 * opaqueGroups + groups, boundTasks = (2 * opaqueGroups + alphaGroups) * CHUNKS;
-    for (int task = next_task(0); task < boundTasks + groups + searches; task = next_task(0)) {
-        if (task < boundTasks) {
+    for (int taken = next_task(0); taken < groups + boundTasks + searches; taken = next_task(0)) {
+        int const task = taken < boundTasks ? taken : taken < boundTasks + groups ? taken - boundTasks - groups : taken - groups;
+        if (task < 0) {
+            int const group = task + groups, b = block_of_group(group);
+            bound_rotations<S>(lds, b);
+            int const first = first_rotation<S>(lds, b);
+            Best const best = all_ones(b) ? dual_planes<S, 2>(lds, b, first) : dual_planes<S, 3>(lds, b, first);
+            keep_candidates<S>(lds, b, first, best.error, own_lane(group));
+            put_candidate(&lds->early.words[b], &lds->early.errors[b], best.error, best.lo, best.hi);
+            add_one(shared.rotated);
+        } else if (task < boundTasks) {
             int const first = (task % CHUNKS) * CHUNK, nth = task / CHUNKS, search = nth < 2 * opaqueGroups ? nth : nth + opaqueGroups;
             int const b = block_of_group(group_of(search));
             if (kind_of(search) == kPickThree) {
@@ -1539,23 +1661,22 @@ bc7_compress_kernel(BlockCompressArgs a)
                 bound_task<S, 2, 4, false, true>(lds, b, first, first + CHUNK);
             }
             add_one(shared.bounded[search]);
-        } else if (task < boundTasks + groups) {
-            finish_task<S, Mode6, 4, true>(lds, block_of_group(task - boundTasks), 0, 8);
         } else {
-            int const search = task - boundTasks - groups, group = group_of(search);
-            int const b = block_of_group(group), mine = 64 * (group < opaqueGroups ? group : group - opaqueGroups) + lane < (group < opaqueGroups ? opaque : withAlpha);
+            int const search = task - boundTasks, group = group_of(search);
+            int const b = block_of_group(group);
             wait_for(shared.bounded[bounds_of(search)], CHUNKS);
-            select_task<S>(lds, b, what_of(search, b), search, mine);
+            select_task<S>(lds, b, what_of(search, b), search, own_lane(group));
+            add_one(shared.selected);
         }
     }
     __builtin_amdgcn_s_setprio(1);
-    __syncthreads();
+    wait_for(shared.selected, searches);
 
     // ---- 2. the errors of the partitions that are left, then candidates: first those that need no partition
     int const wholeTasks = __builtin_amdgcn_readfirstlane(shared.wholes) * (64 / kWholeChunk);
     int estimates = wholeTasks;
     for (int search = 0; search < searches; ++search) estimates += (__builtin_amdgcn_readfirstlane(shared.queued[search]) + 63) / 64;
-    for (int task = next_task(1); task < estimates + 4 * opaqueGroups + 5 * groups; task = next_task(1)) {
+    for (int task = next_task(1);; task = next_task(1)) {
         if (task < wholeTasks) {
             int const search = __builtin_amdgcn_readfirstlane(int(shared.whole[task / (64 / kWholeChunk)])), first = task % (64 / kWholeChunk) * kWholeChunk;
             int const b = block_of_group(group_of(search)), what = what_of(search, b);
@@ -1582,21 +1703,26 @@ bc7_compress_kernel(BlockCompressArgs a)
             continue;
         }
         __builtin_amdgcn_s_setprio(0);
-        int const candidate = task - estimates;
-        if (candidate < 4 * groups) {
-            int const which = candidate & 3, b = block_of_group(candidate >> 2);
-            Ends<3> color[2];                                // refined for 2-bit and 3-bit indices
-            Ends<1> alpha[2];
-            dual_plane_ends<S>(lds, b, which, color, alpha);
-            Best best{ FLT_MAX, 0, 0 };
-            dual_plane_form<S, 0>(lds, b, which, color[0], alpha[1], best);
-            dual_plane_form<S, 1>(lds, b, which, color[1], alpha[0], best);
-            dual_plane_form<S, 2>(lds, b, which, color[0], alpha[0], best);
-            put_candidate<S>(lds, 4 + which, b, best.error, best.lo, best.hi);
+        wait_for(shared.rotated, groups);
+        int const keptFlat = __builtin_amdgcn_readfirstlane(shared.kept[0]), keptRotations = __builtin_amdgcn_readfirstlane(shared.kept[1]);
+        int const keptSixes = __builtin_amdgcn_readfirstlane(shared.kept[2]);
+        int const flatTasks = (keptFlat + 63) / 64, rotationTasks = flatTasks + (keptRotations + 63) / 64, sixTasks = (keptSixes + 63) / 64, candidate = task - estimates;
+        if (candidate >= rotationTasks + sixTasks + 4 * opaqueGroups + groups) break;        // uniform: every wave gets here
+        if (candidate < rotationTasks) {
+            bool const flat = candidate < flatTasks;
+            int const item = flat ? shared.flatRotations[min(candidate * 64 + lane, keptFlat - 1)] : shared.rotations[min((candidate - flatTasks) * 64 + lane, keptRotations - 1)];
+            int const b = item & 127, rotation = item >> 7;
+            Best const best = flat ? dual_planes<S, 2>(lds, b, rotation) : dual_planes<S, 3>(lds, b, rotation);
+            int const slot = kSlotRotations + rotation - (rotation > int(shared.plans[b] & 3u) ? 1 : 0);
+            put_candidate(&lds->late.words[slot][b], &lds->late.errors[slot][b], best.error, best.lo, best.hi);
+            continue;
+        }
+        if (candidate < rotationTasks + sixTasks) {
+            finish_task<S, Mode6, 4, true>(lds, shared.sixes[min((candidate - rotationTasks) * 64 + lane, keptSixes - 1)], 0, kSlotSix);
             continue;
         }
         wait_for(shared.estimated, estimates);
-        int const picked = candidate - 4 * groups;
+        int const picked = candidate - rotationTasks - sixTasks;
         if (picked < 4 * opaqueGroups) {
             int const which = picked & 3, b = block_of(0, picked >> 2);
             if (which == 0)      finish_task<S, Mode0, 3, true>(lds, b, kPickThree, 0);
@@ -1604,7 +1730,7 @@ bc7_compress_kernel(BlockCompressArgs a)
             else if (which == 2) finish_task<S, Mode1, 3, true>(lds, b, kPickTwo, 2);
             else                 finish_task<S, Mode3, 3, true>(lds, b, kPickTwo, 3);
         } else {
-            finish_task<S, Mode7, 4, false>(lds, block_of_group(picked - 4 * opaqueGroups), kPickTwoAlpha, 9);
+            finish_task<S, Mode7, 4, false>(lds, block_of_group(picked - 4 * opaqueGroups), kPickTwoAlpha, kSlotSeven);
         }
     }
     __syncthreads();
@@ -1615,10 +1741,17 @@ bc7_compress_kernel(BlockCompressArgs a)
         if (bx < a.widthInBlocks && by < a.heightInBlocks) {
             float bestError = FLT_MAX;
             uint4 best = make_uint4(0u, 0u, 0u, 0u);
-            for (int slot = (shared.alphas[b] & kBelowOne) ? 4 : 0; slot < kSlots; ++slot) {
-                float const error = slot == 8 ? shared.early.errors[b] : shared.late.errors[min(slot, 8)][b];
-                if (!(error > bestError)) { bestError = error; best = slot == 8 ? shared.early.words[b] : shared.late.words[min(slot, 8)][b]; }
+            uint32_t const plan = shared.plans[b];
+            auto const consider = [&](float error, uint4 const& words) { if (!(error > bestError)) { bestError = error; best = words; } };
+            auto const consider_late = [&](int slot) { consider(shared.late.errors[slot][b], shared.late.words[slot][b]); };
+            if (!(shared.alphas[b] & kBelowOne))
+                for (int slot = 0; slot < kSlotRotations; ++slot) consider_late(slot);
+            for (int r = 0; r < 4; ++r) {
+                if (r == int(plan & 3u))             consider(shared.early.errors[b], shared.early.words[b]);
+                else if (plan & (kKeepRotation << r)) consider_late(kSlotRotations + r - (r > int(plan & 3u) ? 1 : 0));
             }
+            if (plan & kKeepSix) consider_late(kSlotSix);
+            consider_late(kSlotSeven);
             store_block(a, bx, by, uint64_t(best.x) | uint64_t(best.y) << 32, uint64_t(best.z) | uint64_t(best.w) << 32);
         }
     }

@@ -477,6 +477,47 @@ def test_gpu_bc7_search_with_bounds_matches_checker(ntc, device, oracle, size, c
         assert np.array_equal(got, want), (fmt, np.argwhere(got != want)[:4])
 
 
+def image_for_rotations(rng, content, w, h):
+    """RGBA float32, blocks with and without alpha, for the bounds of modes 4, 5 and 6: "line" two channels on a line that the
+    third is no part of, so that one rotation has no error but roundings; "plane" all four on one line, which leaves mode 6; "codes"
+    steps of one 8-bit code, less than the roundings taken off; "level" constant alphas that are not 1, and constant blocks;
+    "steep" a channel with far more contrast than the others; "beyond" texels outside 0 ... 1."""
+    ys, xs = np.mgrid[0:h, 0:w].astype(np.float32)
+    ramp = 0.25 + 0.5 * (xs + 2 * ys)[..., None] / (w + 2 * h)
+    noise = rng.normal(0, 0.03, (h, w, 4))
+    swing = ramp + noise[..., :1]
+    rgba = np.concatenate([swing, 0.9 * swing, 0.2 + 0.5 * swing, 1.1 * swing - 0.1], axis=-1)
+    each_block = lambda v: np.repeat(np.repeat(v, 4, axis=0), 4, axis=1)                       # noqa: E731
+    if content == "line":
+        rgba = np.where(np.arange(4) == each_block(rng.integers(0, 4, (h // 4, w // 4)))[..., None], 0.5 + noise[..., 1:2], rgba)
+    elif content == "codes":
+        rgba = (np.rint(ramp * 255) + rng.integers(0, 2, (h, w, 4))) / 255
+    elif content == "level":
+        rgba = ramp + noise * each_block(rng.random((h // 4, w // 4, 1)) < 0.5)
+        rgba[..., 3] = each_block(rng.choice([0.0, 0.5, 0.999, 1.0], (h // 4, w // 4)))
+    elif content == "steep":
+        rgba = ramp + noise * [0.05, 8.0, 0.05, 0.3]
+    elif content == "beyond":
+        rgba = ramp + noise * 20
+    if content != "level":
+        rgba[..., 3] = np.where(each_block(rng.random((h // 4, w // 4)) < 0.6), 1, rgba[..., 3])
+    return (rgba if content == "beyond" else np.clip(rgba, 0, 1)).astype(np.float32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("content", ["line", "plane", "codes", "level", "steep", "beyond"])
+@pytest.mark.parametrize("size", [(68, 60), (520, 524)])    # workgroups of one group of 64 blocks, and of two
+def test_gpu_bc7_rotations_with_bounds_match_checker(ntc, device, oracle, size, content):
+    image = image_for_rotations(np.random.default_rng(81), content, *size)
+    formats = [(4, image)]
+    if content != "beyond":
+        formats.append((1, np.rint(image * 255).astype(np.uint8)))
+    for fmt, texels in formats:
+        args = (np.ascontiguousarray(texels), fmt, 4, size[0] // 4, size[1] // 4)
+        got, want = compress_bc7(ntc, None, device, *args), compress_bc7(ntc, oracle, None, *args)
+        assert np.array_equal(got, want), (fmt, np.argwhere(got != want)[:4])
+
+
 @pytest.mark.gpu
 def test_gpu_bc7_arguments(ntc, device, oracle):
     from test_image_difference import fill_image
