@@ -445,6 +445,21 @@ def test_tables_in_and_beyond_the_kernel_arguments(ntc, device, sets, entry):
         assert_equal_bytes(host.output, case.d_output.download(), f"{entry}, set {s} of {sets}")
 
 
+# Launches of few tiles find a tile's entry by whole waves, 64 entries at a time: from the arguments and from the table in
+# memory, on both sides of a wave's width, with mips of several tiles among those of one.
+@pytest.mark.parametrize("sets,mips", [(1, 1), (1, 7), (9, 7), (32, 2), (65, 1), (13, 5), (128, 1)])
+def test_entries_of_launches_of_few_tiles(ntc, device, sets, mips):
+    cases = [cfg_case(ntc, ntc.presets.spec_cfg01(), 64 if mips > 1 else 4 + s % 60, 64 if sets == 1 else 16 if mips == 7 else 4, mips, 8,
+                      ntc.abi.OUT_FP16_PLANAR_PAIRS, seed=900 + s, scale_log2_range=ACTIVE) for s in range(sets)]
+    dsets = [c.device_set(device) for c in cases]
+    device.decode(dsets)
+    device.synchronize()
+    for s, case in enumerate(cases):
+        host = case.host_set()
+        host.decode(threads=2)
+        assert_equal_bytes(host.output, case.d_output.download(), f"set {s} of {sets}")
+
+
 def test_timer_spans_the_calls_between_its_two_ends(ntc, device):
     """ntc_hip_timer_begin / _end: device time of whatever was queued between them.  A span around five decodes is
     at least as long as five decodes timed back to back by ntc_hip_decode_timed (it also holds the table uploads
