@@ -348,7 +348,7 @@ __device__ __forceinline__ void prepare_inputs_fp8(DevMip const& m, Fp8Lds<V> co
             float t[4], value[4];
             filter4(tp, cells[grid][L], t);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) value[i] = (4 * L + i < V::F) ? __builtin_fmaf(t[i], (i & 1) ? 0.13333334f / 16.f : 0.13333334f, -1.f) : 0.f;
+            for (int i = 0; i < 4; ++i) value[i] = (4 * L + i < V::F) ? __builtin_fmaf(t[i], 0.13333334f, -1.f) : 0.f;
             in[8 * grid + 2 * L]     = round_e4m3_pk(halves_rne(value[0], value[1]));
             in[8 * grid + 2 * L + 1] = round_e4m3_pk(halves_rne(value[2], value[3]));
         }

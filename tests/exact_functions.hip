@@ -252,6 +252,56 @@ struct TexelCentre {
     }
 };
 
+// floors_of(): every float of [0, 256), in every place beside numbers of its neighbourhood.
+struct FloorsOf {
+    static constexpr uint64_t cases = 0x43800000u;
+    static __device__ int check(uint64_t i)
+    {
+        uint32_t const bits = uint32_t(i), top = 0x437fffffu;
+        float const v[4] = { __uint_as_float(bits), __uint_as_float(min(bits + 1u, top)), __uint_as_float(bits ^ (bits >= 0x80u ? 0x55u : 0u)), __uint_as_float(top - bits) };
+        uint32_t expected = 0;
+        for (int k = 0; k < 4; ++k) expected |= uint32_t(floorf(v[k])) << (8 * k);
+        return verdict(floors_of(v[0] * 0x1p-24f, v[1] * 0x1p-24f, v[2] * 0x1p-24f, v[3] * 0x1p-24f) == expected);
+    }
+};
+
+// filter4() and bilinear4() against the definition, for scattered cells and fractions: zeros, the largest below 1, few and
+// many bits, products of two that are subnormal.
+struct FilteredFeatures {
+    static constexpr uint64_t cases = uint64_t(1) << 26;
+    static __device__ uint32_t hash(uint32_t h) { h ^= h >> 16; h *= 0x7feb352du; h ^= h >> 15; h *= 0x846ca68bu; return h ^ h >> 16; }
+    static __device__ float fraction(uint32_t h)
+    {
+        switch (h & 7u) {
+        case 0: return 0.f;
+        case 1: return 0x1.fffffep-1f;
+        case 2: return float(h >> 28) * 0x1p-4f;
+        case 3: return float(h >> 8) * 0x1p-24f * __builtin_ldexpf(1.f, -int(h >> 3 & 31u) * 4);
+        default: return float(h >> 8) * 0x1p-24f;
+        }
+    }
+    static __device__ int check(uint64_t i)
+    {
+        uint32_t const h = hash(uint32_t(i)), c = hash(h + 1u), e = hash(h + 2u);
+        FloatAxis const x{ 0, 0, fraction(hash(h + 3u)) }, y{ 0, 0, fraction(hash(h + 4u)) };
+        uint32_t const cells[4] = { c & 0xffffu, c >> 16, e & 0xffffu, e >> 16 };
+        FloatTaps const taps(x, y);
+        float t[4];
+        filter4(taps, cells, t);
+        float const dxn = 1.f - x.d, dyn = 1.f - y.d, w00 = dxn * dyn, w10 = x.d * dyn, w01 = dxn * y.d, w11 = x.d * y.d;
+        uint32_t bytes = 0;
+        bool right = true;
+        for (int f = 0; f < 4; ++f) {
+            float q[4];
+            for (int k = 0; k < 4; ++k) q[k] = float((cells[k] >> (4 * f)) & 15u);
+            float const s = __builtin_fmaf(w11, q[3], __builtin_fmaf(w01, q[2], __builtin_fmaf(w10, q[1], w00 * q[0])));
+            right = right && (same(t[f], s) || (fabsf(s) < 0x1p-100f && fabsf(t[f] - s) < 0x1p-120f));       // (the definition's weights are subnormal there)
+            bytes |= ((uint32_t(floorf(17.f * s)) + 128u) & 0xffu) << (8 * f);
+        }
+        return verdict(right && bilinear4(taps, cells) == bytes);
+    }
+};
+
 #endif
 
 } // namespace
@@ -277,5 +327,7 @@ int exact_quotient_of_codes(Report* r) { return sweep<QuotientOfCodes>(r); }
 int exact_quotient_of_diagonals(Report* r) { return sweep<QuotientOfDiagonals>(r); }
 #else
 int exact_texel_centre(Report* r) { return sweep<TexelCentre>(r); }
+int exact_floors_of(Report* r) { return sweep<FloorsOf>(r); }
+int exact_filtered_features(Report* r) { return sweep<FilteredFeatures>(r); }
 #endif
 }

@@ -22,7 +22,8 @@ class Report(C.Structure):
     ("bc", "code_quotient", 96), ("bc", "bc4_palette", 65536), ("bc", "bc4_positions", 1 << 20), ("bc", "bc4_refit", 1 << 24),
     ("bc6", "quotient_of_integers", (1 << 17) * ((1 << 17) - 1)), ("bc6", "quotient_of_log2", None),
     ("bc6", "quotient_of_msle", 0x7c00 * (0x7c00 + 256 + 65536 + 65505)), ("bc6", "log_estimate", 34 << 23), ("bc6", "quotient_of_codes", 3 * 65536 + 64),
-    ("bc6", "quotient_of_diagonals", 1 << 30), ("decode", "texel_centre", (1 << 15) * 65537)])
+    ("bc6", "quotient_of_diagonals", 1 << 30), ("decode", "texel_centre", (1 << 15) * 65537),
+    ("decode", "floors_of", 0x43800000), ("decode", "filtered_features", 1 << 26)])
 def test_gpu_shortcut_equals_the_operation(device, subject, function, cases):
     path = os.path.join(HERE, f"libexact_{subject}.so")
     assert os.path.exists(path), f"{path} is not built; run __graft_entry__.build() (make -C tests)"
