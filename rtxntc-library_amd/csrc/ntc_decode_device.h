@@ -248,7 +248,7 @@ __device__ __forceinline__ uint32_t to_half2_bits(float a, float b)
 // The result drops into byte `slot` of `packed`.
 __device__ __forceinline__ uint32_t pack_unorm8(_Float16 h, uint32_t slot, uint32_t packed)
 {
-    return __builtin_amdgcn_cvt_pk_u8_f32(float(h) * 255.f, slot, packed);
+    return __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(float(h), 255.f, 0.f), slot, packed);
 }
 
 typedef __attribute__((address_space(1))) uint8_t* GlobalOutPtr;
