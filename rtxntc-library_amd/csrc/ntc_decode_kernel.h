@@ -63,9 +63,10 @@ struct DevMip {
 // would have to hand on to each other.  (A table copied from pinned memory took a copy and an event record per call:
 // one 128 x 128 mip, another set each call: 16.3 us, 9.1 us with the table in the arguments.)  Longer tables
 // - batches of sets - lie in device memory at `entries`, which is null otherwise.
-constexpr int kInlineMips = 16;                            // one set with a full mip chain; 1 920 bytes of arguments
+constexpr int kInlineMips = 16;                            // one set with a full mip chain; 2 176 bytes of arguments
 struct MipTable {
     DevMip inlined[kInlineMips];
+    int32_t starts[kInlineMips];   // of the inlined ones: their tileStart, side by side; 0x7fffffff where there is none
     DevMip const* entries;
 };
 

@@ -463,6 +463,7 @@ int place_table(Library& L, TableSink const& sink, MipTable& table)
     table.entries = nullptr;
     if (sink.count <= size_t(kInlineMips)) {
         std::memcpy(table.inlined, sink.entries(), sink.count * sizeof(DevMip));
+        for (int k = 0; k < kInlineMips; ++k) table.starts[k] = size_t(k) < sink.count ? table.inlined[k].tileStart : 0x7fffffff;
         return 0;
     }
     if (int r = upload_table(L, sink.entries(), sink.count)) return r;

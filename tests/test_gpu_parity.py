@@ -445,18 +445,21 @@ def test_tables_in_and_beyond_the_kernel_arguments(ntc, device, sets, entry):
         assert_equal_bytes(host.output, case.d_output.download(), f"{entry}, set {s} of {sets}")
 
 
-# Launches of few tiles find a tile's entry by whole waves, 64 entries at a time: from the arguments and from the table in
-# memory, on both sides of a wave's width, with mips of several tiles among those of one.
-@pytest.mark.parametrize("sets,mips", [(1, 1), (1, 7), (9, 7), (32, 2), (65, 1), (13, 5), (128, 1)])
-def test_entries_of_launches_of_few_tiles(ntc, device, sets, mips):
-    cases = [cfg_case(ntc, ntc.presets.spec_cfg01(), 64 if mips > 1 else 4 + s % 60, 64 if sets == 1 else 16 if mips == 7 else 4, mips, 8,
-                      ntc.abi.OUT_FP16_PLANAR_PAIRS, seed=900 + s, scale_log2_range=ACTIVE) for s in range(sets)]
+# A tile's entry is found by whole waves, 64 entries at a time, in launches of up to 128 tiles, from numbers in the arguments
+# in larger ones, and by a loop where the table lies in memory: both sides of 16 and 64 entries, mips of several tiles
+# among those of one.
+@pytest.mark.parametrize("sets,mips,width,height", [
+    (1, 1, 64, 64), (1, 7, 64, 64), (9, 7, 64, 16), (32, 2, 64, 4), (65, 1, 52, 4), (13, 5, 64, 4), (128, 1, 33, 4),
+    (1, 9, 256, 200), (2, 8, 128, 128), (5, 3, 100, 120), (16, 1, 64, 40), (17, 1, 64, 40), (3, 6, 130, 90)])
+def test_entries_of_tiles(ntc, device, sets, mips, width, height):
+    cases = [cfg_case(ntc, ntc.presets.spec_cfg01(), width, height, mips, 8, ntc.abi.OUT_FP16_PLANAR_PAIRS, seed=900 + s, scale_log2_range=ACTIVE)
+             for s in range(sets)]
     dsets = [c.device_set(device) for c in cases]
     device.decode(dsets)
     device.synchronize()
     for s, case in enumerate(cases):
         host = case.host_set()
-        host.decode(threads=2)
+        host.decode(threads=8)
         assert_equal_bytes(host.output, case.d_output.download(), f"set {s} of {sets}")
 
 
