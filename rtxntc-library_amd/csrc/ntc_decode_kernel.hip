@@ -1369,6 +1369,7 @@ decode_few_kernel(MipTable table, int numMips, int log2Parts)
     // at once (a loop over the entries, each a trip to memory, and the fields as they were used: 64 x 64 with its 7 mips 7.3
     // us, 6.3 now; 128 x 128 with its 8 7.8 and 6.9).
     DevMip const mip = mips[__builtin_amdgcn_readfirstlane(numMips > 1 ? table_entry_of(mips, numMips, 0, tile) : 0)];
+    asm volatile("" :: "s"(mip.width), "s"(mip.tilesX), "s"(mip.posMask));     // (every line of it: 128 x 128 5.92 us, 5.80)
     RunMip const m(mip);
     int const staged = __builtin_amdgcn_readfirstlane(stage_weights<V>(lds, m.full.weights, wave * 64 + lane_id(), 1));
     __syncthreads();
