@@ -197,76 +197,51 @@ template <int C> BC7_INLINE void refine(Color<C> const (&px)[16], uint32_t mask,
     }
 }
 
-// Squared error of the subset if every texel took the nearest of the 2^indexBits points between the
-// (unquantised) endpoints.
-template <int C> BC7_INLINE float estimate(Color<C> const (&px)[16], uint32_t mask, Color<C> const& e0, Color<C> const& e1, int indexBits)
-{
-    Color<C> const axis = sub(e1, e0);
-    float mul = dot(axis, axis);
-    if (mul > 0.f) mul = 1.f / mul;
-    float const maxIndex = float((1u << indexBits) - 1u), indexScale = 1.f / maxIndex;
-    float error = 0.f;
-#pragma unroll
-    for (int t = 0; t < 16; ++t)
-        if (has_texel(mask, t)) {
-            Color<C> const p = sub(px[t], e0);
-            float f = dot(p, axis) * mul;
-            f = rintf(f * maxIndex) * indexScale;
-            Color<C> diff;
-#pragma unroll
-            for (int k = 0; k < C; ++k) diff.c[k] = f * axis.c[k] - p.c[k];
-            error += dot(diff, diff);
-        }
-    return error;
-}
-
 BC7_INLINE int quantize(float v, int bits) { return int(rintf(saturate(v) * float((1u << bits) - 1u))); }
 BC7_INLINE int expand8(int q, int bits) { return (q << (8 - bits)) | (q >> (2 * bits - 8)); }
 
-// Squared error of the subset as a decoder reconstructs it (integer interpolation with 6-bit weights).
-template <int C> BC7_INLINE float decoded_error(Color<C> const (&px)[16], int const (&index)[16], uint32_t mask, Quantized<C> q0, Quantized<C> q1,
-                                                int indexBits, int endpointBits)
-{
-#pragma unroll
-    for (int k = 0; k < C; ++k) { q0.c[k] = expand8(q0.c[k], endpointBits); q1.c[k] = expand8(q1.c[k], endpointBits); }
-    float const indexScale = 64.f / float((1u << indexBits) - 1u);
-    float error = 0.f;
-#pragma unroll
-    for (int t = 0; t < 16; ++t)
-        if (has_texel(mask, t)) {
-            int const w = int(rintf(float(index[t]) * indexScale));
-            Color<C> diff;
-#pragma unroll
-            for (int k = 0; k < C; ++k) diff.c[k] = float((q0.c[k] * (64 - w) + q1.c[k] * w + 32) >> 6) / 255.f - px[t].c[k];
-            error += dot(diff, diff);
-        }
-    return error;
-}
-
-// Indices of the subset's texels along the dequantised endpoints.  A decoder assumes the top index bit
-// of the anchor texel to be 0: if it is 1 all indices of the subset are complemented and true is
-// returned (the caller swaps the endpoints).
-template <int C> BC7_INLINE bool assign(Color<C> const (&px)[16], uint32_t mask, int anchor, int indexBits, int endpointBits,
-                                        Quantized<C> const& q0, Quantized<C> const& q1, int (&index)[16])
+// Indices of the subset's texels along the dequantised endpoints, each in its place in the block: `two` for 2-bit ones,
+// `three` for 3-bit ones, whichever BITS says, both for 0 (then indexBits tells).
+template <int C, int BITS> BC7_INLINE void assign(Color<C> const (&px)[16], uint32_t mask, int indexBits, int endpointBits,
+                                                  Quantized<C> const& q0, Quantized<C> const& q1, uint32_t& two, uint64_t& more)
 {
     Color<C> e0, e1;
 #pragma unroll
-    for (int k = 0; k < C; ++k) { e0.c[k] = float(expand8(q0.c[k], endpointBits)) / 255.f; e1.c[k] = float(expand8(q1.c[k], endpointBits)) / 255.f; }
+    for (int k = 0; k < C; ++k) {
+        e0.c[k] = unorm_quotient(float(expand8(q0.c[k], endpointBits)), 255.f, 1.f / 255.f);
+        e1.c[k] = unorm_quotient(float(expand8(q1.c[k], endpointBits)), 255.f, 1.f / 255.f);
+    }
     Color<C> const axis = sub(e1, e0);
     float mul = dot(axis, axis);
     if (mul > 0.f) mul = 1.f / mul;
-    bool flip = false;
 #pragma unroll
     for (int t = 0; t < 16; ++t)
         if (has_texel(mask, t)) {
-            index[t] = quantize(dot(sub(px[t], e0), axis) * mul, indexBits);
-            if (t == anchor) flip = (index[t] >> (indexBits - 1)) & 1;
+            uint32_t const index = uint32_t(quantize(dot(sub(px[t], e0), axis) * mul, indexBits));
+            if constexpr (BITS == 0 || BITS == 2) two |= index << (2 * t);
+            if constexpr (BITS == 0)              more |= uint64_t(index) << (3 * t);
+            else if constexpr (BITS > 2)          more |= uint64_t(index) << (BITS * t);
         }
-    int const all = (1 << indexBits) - 1;
+}
+
+// A field of a block from bit `at` on, and the removal of the anchors' top index bits, which are zero.
+BC7_INLINE void put_indices(uint64_t& lo, uint64_t& hi, int at, uint64_t v)
+{
+    if (at < 64) { lo |= v << at; hi |= at ? v >> (64 - at) : 0; }
+    else hi |= v << (at - 64);
+}
+// The three bits of each index of a subset.
+BC7_INLINE uint64_t three_bits_of(uint32_t spreadMask)
+{
+    uint64_t x = 0;
 #pragma unroll
-    for (int t = 0; t < 16; ++t)
-        if (flip && has_texel(mask, t)) index[t] ^= all;
-    return flip;
+    for (int t = 0; t < 16; ++t) x |= uint64_t((spreadMask >> (2 * t)) & 1u) << (3 * t);
+    return x * 7u;
+}
+BC7_INLINE uint64_t without_bit(uint64_t v, int at)
+{
+    uint64_t const below = (uint64_t(1) << at) - 1u;
+    return (v & below) | ((v >> 1) & ~below);
 }
 
 struct Bits {
@@ -282,6 +257,7 @@ struct Bits {
 };
 
 struct Best { float error; uint64_t lo, hi; };
+struct Block { uint64_t lo, hi; };
 
 enum { kNoPBit = 0, kPBitPerEndpoint = 1, kPBitPerSubset = 2 };
 template <int ID, int SUBSETS_, int PARTITION_BITS, int ENDPOINT_BITS /* with the p-bit */, int INDEX_BITS, int PBIT>
@@ -329,11 +305,10 @@ template <class M, int C> BC7_INLINE void quantize_endpoints(Color<C> const (&e)
     }
 }
 
-// Refines the start endpoints of every subset, quantises, assigns indices and, if the result is not
-// worse than the best so far (always, with a fixed mode), encodes the block.
-template <class M, int C> BC7_INLINE void finish(Color<C> const (&px)[16], int partition, Color<C> const (&start)[2 * M::subsets], bool fixedMode, Best& best)
+// Refines the start endpoints of every subset, quantises, assigns indices and encodes the block.
+template <class M, int C> BC7_INLINE Block finish(Color<C> const (&px)[16], int partition, Color<C> const (&start)[2 * M::subsets])
 {
-    constexpr int N = 2 * M::subsets;
+    constexpr int N = 2 * M::subsets, top = M::indexBits - 1;
     uint32_t const word = partition_word<M::subsets>(partition);
     Color<C> e[N];
     Quantized<C> q[N];
@@ -342,24 +317,24 @@ template <class M, int C> BC7_INLINE void finish(Color<C> const (&px)[16], int p
 #pragma unroll
     for (int s = 0; s < M::subsets; ++s) refine(px, spread_mask(word, s), e[2 * s], e[2 * s + 1], M::indexBits);
     quantize_endpoints<M, C>(e, q);
-    int index[16];
-#pragma unroll
-    for (int t = 0; t < 16; ++t) index[t] = 0;
+    uint64_t indices = 0;
     int anchors[M::subsets];
-    float error = 0.f;
 #pragma unroll
     for (int s = 0; s < M::subsets; ++s) {
         uint32_t const mask = spread_mask(word, s);
+        uint32_t two = 0;
+        uint64_t more = 0;
+        assign<C, M::indexBits>(px, mask, M::indexBits, M::endpointBits, q[2 * s], q[2 * s + 1], two, more);
+        uint64_t const own = M::indexBits == 2 ? uint64_t(two) : more;
+        indices |= own;
+        // a decoder assumes the anchor's top index bit to be 0: if it is 1 the subset's indices are complemented and its
+        // endpoints trade places
         anchors[s] = subset_anchor<M::subsets>(partition, s);
-        if (assign(px, mask, anchors[s], M::indexBits, M::endpointBits, q[2 * s], q[2 * s + 1], index)) {
+        if ((own >> (anchors[s] * M::indexBits + top)) & 1u) {
+            indices ^= M::indexBits == 2 ? uint64_t(mask * 3u) : M::indexBits == 4 ? ~uint64_t(0) : three_bits_of(mask);
             Quantized<C> const t = q[2 * s]; q[2 * s] = q[2 * s + 1]; q[2 * s + 1] = t;
         }
-        if (!fixedMode) {
-            float const e2 = decoded_error(px, index, mask, q[2 * s], q[2 * s + 1], M::indexBits, M::endpointBits);
-            error = s == 0 ? e2 : error + e2;
-        }
     }
-    if (error > best.error) return;
     Bits b;
     b.put(M::id + 1, 1u << M::id);
     b.put(M::partitionBits, uint32_t(partition));
@@ -376,14 +351,15 @@ template <class M, int C> BC7_INLINE void finish(Color<C> const (&px)[16], int p
 #pragma unroll
         for (int s = 0; s < M::subsets; ++s) b.put(1, uint32_t(q[2 * s].c[0]));
     }
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-        bool anchor = t == 0;
-#pragma unroll
-        for (int s = 1; s < M::subsets; ++s) anchor = anchor || t == anchors[s];
-        b.put(anchor ? M::indexBits - 1 : M::indexBits, uint32_t(index[t]));
+    if constexpr (M::subsets == 3) {
+        indices = without_bit(indices, max(anchors[1], anchors[2]) * M::indexBits + top);
+        indices = without_bit(indices, min(anchors[1], anchors[2]) * M::indexBits + top);
+    } else if constexpr (M::subsets == 2) {
+        indices = without_bit(indices, anchors[1] * M::indexBits + top);
     }
-    best.error = error; best.lo = b.lo; best.hi = b.hi;
+    indices = without_bit(indices, top);
+    put_indices(b.lo, b.hi, b.at, indices);
+    return { b.lo, b.hi };
 }
 
 // Start endpoints of every subset of a partition: the subset's bounding box, oriented if asked.
@@ -413,9 +389,10 @@ BC7_INLINE void split_planes(Color<4> const (&rgba)[16], uint32_t rotation, Colo
 }
 template <int C> struct Ends { Color<C> e0, e1; };
 
-// One candidate of the two modes from the refined endpoints of both planes.
-BC7_INLINE void finish_dual_plane(int mode, bool wideColorIndex, Color<3> const (&rgb)[16], Color<1> const (&a)[16], Ends<3> const& color, Ends<1> const& alpha,
-                                  uint32_t rotation, bool fixedMode, Best& best)
+// The block of the two modes from the refined endpoints of both planes.  Mode 4's fields are 8 bits of mode, rotation and
+// choice, 42 of endpoints, its 2-bit indices and its 3-bit ones; mode 5's 8 bits, 58, the colours' indices, the scalars'.
+BC7_INLINE Block finish_dual_plane(int mode, bool wideColorIndex, Color<3> const (&rgb)[16], Color<1> const (&a)[16], Ends<3> const& color, Ends<1> const& alpha,
+                                   uint32_t rotation)
 {
     int const colorIndexBits = mode == 5 ? 2 : (wideColorIndex ? 3 : 2), alphaIndexBits = mode == 5 ? 2 : (wideColorIndex ? 2 : 3);
     int const colorBits = mode == 5 ? 7 : 5, alphaBits = mode == 5 ? 8 : 6;
@@ -424,28 +401,32 @@ BC7_INLINE void finish_dual_plane(int mode, bool wideColorIndex, Color<3> const 
     for (int k = 0; k < 3; ++k) { q0.c[k] = quantize(color.e0.c[k], colorBits); q1.c[k] = quantize(color.e1.c[k], colorBits); }
     Quantized<1> qa0, qa1;
     qa0.c[0] = quantize(alpha.e0.c[0], alphaBits); qa1.c[0] = quantize(alpha.e1.c[0], alphaBits);
-    int colorIndex[16], alphaIndex[16];
-    float error = 0.f;
-    if (assign(rgb, kAllTexels, 0, colorIndexBits, colorBits, q0, q1, colorIndex)) { Quantized<3> const t = q0; q0 = q1; q1 = t; }
-    if (!fixedMode) error = decoded_error(rgb, colorIndex, kAllTexels, q0, q1, colorIndexBits, colorBits);
-    if (assign(a, kAllTexels, 0, alphaIndexBits, alphaBits, qa0, qa1, alphaIndex)) { Quantized<1> const t = qa0; qa0 = qa1; qa1 = t; }
-    if (!fixedMode) error += decoded_error(a, alphaIndex, kAllTexels, qa0, qa1, alphaIndexBits, alphaBits);
-    if (error > best.error) return;
-    Bits b;
-    b.put(mode + 1, 1u << mode);
-    b.put(2, rotation);
-    if (mode == 4) b.put(1, wideColorIndex ? 1u : 0u);
+    // indices of one plane with the first one's top bit taken out; true: they are complemented and the endpoints trade places
+    auto const packed = [](int bits, uint32_t two, uint64_t three, uint64_t& indices) {
+        indices = bits == 2 ? uint64_t(two) : three;
+        bool const flip = (uint32_t(indices) >> (bits - 1)) & 1u;
+        if (flip) indices ^= bits == 2 ? 0xffffffffull : 0xffffffffffffull;
+        uint64_t const below = bits == 2 ? 1u : 3u;
+        indices = (indices & below) | ((indices >> 1) & ~below);
+        return flip;
+    };
+    uint64_t colorIndices, alphaIndices, three = 0;
+    uint32_t two = 0;
+    assign<3, 0>(rgb, kAllTexels, colorIndexBits, colorBits, q0, q1, two, three);
+    if (packed(colorIndexBits, two, three, colorIndices)) { Quantized<3> const t = q0; q0 = q1; q1 = t; }
+    two = 0; three = 0;
+    assign<1, 0>(a, kAllTexels, alphaIndexBits, alphaBits, qa0, qa1, two, three);
+    if (packed(alphaIndexBits, two, three, alphaIndices)) { Quantized<1> const t = qa0; qa0 = qa1; qa1 = t; }
+    uint64_t ends = uint32_t(qa1.c[0]) << alphaBits | uint32_t(qa0.c[0]);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) { b.put(colorBits, uint32_t(q0.c[k])); b.put(colorBits, uint32_t(q1.c[k])); }
-    b.put(alphaBits, uint32_t(qa0.c[0])); b.put(alphaBits, uint32_t(qa1.c[0]));
-    // mode 4 stores its 2-bit indices first, then the 3-bit ones; mode 5 colour first, then the scalar
+    for (int k = 2; k >= 0; --k) ends = ends << (2 * colorBits) | (uint32_t(q1.c[k]) << colorBits | uint32_t(q0.c[k]));
+    uint32_t const head = mode == 5 ? 0x20u | rotation << 6 : 0x10u | rotation << 5 | (wideColorIndex ? 0x80u : 0u);
+    Block block{ uint64_t(head) | ends << 8, ends >> 56 };
     bool const alphaFirst = mode == 4 && wideColorIndex;
-    int const firstBits = alphaFirst ? alphaIndexBits : colorIndexBits, secondBits = alphaFirst ? colorIndexBits : alphaIndexBits;
-#pragma unroll
-    for (int t = 0; t < 16; ++t) b.put(t == 0 ? firstBits - 1 : firstBits, uint32_t(alphaFirst ? alphaIndex[t] : colorIndex[t]));
-#pragma unroll
-    for (int t = 0; t < 16; ++t) b.put(t == 0 ? secondBits - 1 : secondBits, uint32_t(alphaFirst ? colorIndex[t] : alphaIndex[t]));
-    best.error = error; best.lo = b.lo; best.hi = b.hi;
+    int const at = mode == 5 ? 66 : 50;                      // then 31 bits of 2-bit indices
+    put_indices(block.lo, block.hi, at, alphaFirst ? alphaIndices : colorIndices);
+    put_indices(block.lo, block.hi, at + 31, alphaFirst ? colorIndices : alphaIndices);
+    return block;
 }
 
 template <int C> BC7_INLINE Ends<C> box_of(Color<C> const (&px)[16])
@@ -461,21 +442,19 @@ template <int C> BC7_INLINE Ends<C> refined(Color<C> const (&px)[16], Ends<C> e,
     return e;
 }
 
-// One candidate, with a given mode.
-BC7_INLINE void fixed_dual_plane(int mode, bool wideColorIndex, Color<4> const (&rgba)[16], uint32_t rotation, Best& best)
+BC7_INLINE Block fixed_dual_plane(int mode, bool wideColorIndex, Color<4> const (&rgba)[16], uint32_t rotation)
 {
     Color<3> rgb[16];
     Color<1> a[16];
     split_planes(rgba, rotation, rgb, a);
     int const colorIndexBits = mode == 5 ? 2 : (wideColorIndex ? 3 : 2), alphaIndexBits = mode == 5 ? 2 : (wideColorIndex ? 2 : 3);
-    finish_dual_plane(mode, wideColorIndex, rgb, a, refined(rgb, box_of(rgb), colorIndexBits), refined(a, box_of(a), alphaIndexBits), rotation, true, best);
+    return finish_dual_plane(mode, wideColorIndex, rgb, a, refined(rgb, box_of(rgb), colorIndexBits), refined(a, box_of(a), alphaIndexBits), rotation);
 }
 
 // One block with a given mode and partition (for modes 4 / 5: rotation in bits 0-1 of the partition, "wide colour
 // index" in bit 2).  `list` says the mode but for 4 and 5, and is uniform.
-BC7_INLINE void bc7_encode_fixed(Color<4> const (&px)[16], int list, int mode, int partition, uint64_t& lo, uint64_t& hi)
+BC7_INLINE Block bc7_encode_fixed(Color<4> const (&px)[16], int list, int mode, int partition)
 {
-    Best best{ FLT_MAX, 0, 0 };
     if (list <= 3) {
         Color<3> rgb[16];
 #pragma unroll
@@ -483,26 +462,21 @@ BC7_INLINE void bc7_encode_fixed(Color<4> const (&px)[16], int list, int mode, i
         if (list <= 1) {
             Color<3> ends[6];
             partition_ends<3, 3, true>(rgb, partition, ends);
-            if (list == 0) finish<Mode0>(rgb, partition, ends, true, best);
-            else           finish<Mode2>(rgb, partition, ends, true, best);
-        } else {
-            Color<3> ends[4];
-            partition_ends<2, 3, true>(rgb, partition, ends);
-            if (list == 2) finish<Mode1>(rgb, partition, ends, true, best);
-            else           finish<Mode3>(rgb, partition, ends, true, best);
+            return list == 0 ? finish<Mode0>(rgb, partition, ends) : finish<Mode2>(rgb, partition, ends);
         }
-    } else if (list == 5) {
-        fixed_dual_plane(mode, mode == 4 && (partition & 4), px, uint32_t(partition) & 3u, best);
-    } else if (list == 6) {
+        Color<3> ends[4];
+        partition_ends<2, 3, true>(rgb, partition, ends);
+        return list == 2 ? finish<Mode1>(rgb, partition, ends) : finish<Mode3>(rgb, partition, ends);
+    }
+    if (list == 5) return fixed_dual_plane(mode, mode == 4 && (partition & 4), px, uint32_t(partition) & 3u);
+    if (list == 6) {
         Color<4> ends[2];
         partition_ends<1, 4, true>(px, 0, ends);
-        finish<Mode6>(px, 0, ends, true, best);
-    } else {
-        Color<4> ends[4];
-        partition_ends<2, 4, false>(px, partition, ends);
-        finish<Mode7>(px, partition, ends, true, best);
+        return finish<Mode6>(px, 0, ends);
     }
-    lo = best.lo; hi = best.hi;
+    Color<4> ends[4];
+    partition_ends<2, 4, false>(px, partition, ends);
+    return finish<Mode7>(px, partition, ends);
 }
 
 BC7_INLINE void load_block(BlockCompressArgs const& a, int bx, int by, Color<4> (&px)[16])
@@ -1224,18 +1198,6 @@ template <int C, int INDEX_BITS> struct Decoded {
     }
 };
 
-// A field of a block from bit `at` on, and the removal of the anchors' top index bits, which are zero.
-BC7_INLINE void put_indices(uint64_t& lo, uint64_t& hi, int at, uint64_t v)
-{
-    if (at < 64) { lo |= v << at; hi |= at ? v >> (64 - at) : 0; }
-    else hi |= v << (at - 64);
-}
-BC7_INLINE uint64_t without_bit(uint64_t v, int at)
-{
-    uint64_t const below = (uint64_t(1) << at) - 1u;
-    return (v & below) | ((v >> 1) & ~below);
-}
-
 template <class W, class E> BC7_INLINE void put_candidate(W words, E errors, float error, uint64_t lo, uint64_t hi)
 {
     *errors = error;
@@ -1846,9 +1808,8 @@ bc7_compress_modes_kernel(BlockCompressArgs a)
         int const b = int(task & 1023u), bx = int(blockIdx.x) * SIDE + b % SIDE, by = int(blockIdx.y) * SIDE + b / SIDE;
         Color<4> px[16];
         load_block(a, bx, by, px);
-        uint64_t lo, hi;
-        bc7_encode_fixed(px, list, int(task >> 16), int(task >> 10) & 63, lo, hi);
-        store_block(a, bx, by, lo, hi);
+        Block const block = bc7_encode_fixed(px, list, int(task >> 16), int(task >> 10) & 63);
+        store_block(a, bx, by, block.lo, block.hi);
     }
 }
 
