@@ -511,13 +511,31 @@ BC6_INLINE void base_and_deltas(Bc6Ptr lds, int b, float levels, float limit, V3
     for (int i = 1; i < 4; ++i) q[i] = clamp3(q[i] - q[0], limit);
 }
 
-// Indices of four texels under the three candidates and, as estimates, what they add to the candidates' errors.
+// Indices of four texels under the one-subset candidate and, as an estimate, what they add to its error.
 template <bool WIDE>
-BC6_TASK void estimate_errors(Bc6Ptr lds, int b, int quarter)
+BC6_TASK void estimate_one_subset(Bc6Ptr lds, int b, int quarter)
 {
     quarter = __builtin_amdgcn_readfirstlane(quarter);
     SubsetEnds const one = load_ends(lds->one, b);
     V3 const u0 = unquantize(quantize(one.lo, 1024.f), 1024.f), u1 = unquantize(quantize(one.hi, 1024.f), 1024.f);
+    uint32_t indices4 = 0;
+    float error1 = 0.f;
+#pragma unroll 2
+    for (int i = 0; i < 4; ++i) {
+        V3 const p = texel(lds, b, 4 * quarter + i);
+        uint32_t const index = index4(to_half_bits(dot(p, one.dir)), one.e0, one.e1);
+        indices4 |= index << (4 * i);
+        error1 += Msle<WIDE>(p).estimate(interpolate(u0, u1, float(weight4(index))));
+    }
+    lds->indices[0][quarter][b] = indices4;
+    lds->errors[0][quarter][b] = error1;
+}
+
+// The same under the two candidates with two subsets.
+template <bool WIDE>
+BC6_TASK void estimate_two_subsets(Bc6Ptr lds, int b, int quarter)
+{
+    quarter = __builtin_amdgcn_readfirstlane(quarter);
     V3 u7[4], u9[4];
     {
         V3 q[4];
@@ -531,15 +549,12 @@ BC6_TASK void estimate_errors(Bc6Ptr lds, int b, int quarter)
         for (int i = 1; i < 4; ++i) u9[i] = unquantize(q[0] + q[i], 512.f);
     }
     uint32_t const second = kSecondSubset[picked_pattern(lds, b)] >> (4 * quarter);
-    uint32_t indices4 = 0, indices3 = 0;
-    float error1 = 0.f, error7 = 0.f, error9 = 0.f;
+    uint32_t indices3 = 0;
+    float error7 = 0.f, error9 = 0.f;
 #pragma unroll 2
     for (int i = 0; i < 4; ++i) {
         V3 const p = texel(lds, b, 4 * quarter + i);
         Msle<WIDE> const error(p);
-        uint32_t const index = index4(to_half_bits(dot(p, one.dir)), one.e0, one.e1);
-        indices4 |= index << (4 * i);
-        error1 += error.estimate(interpolate(u0, u1, float(weight4(index))));
         bool const s = (second >> i) & 1u;
         V3 const dir{ lds->two[s][6][b], lds->two[s][7][b], lds->two[s][8][b] };
         uint32_t const inSubset = index3(to_half_bits(dot(p, dir)), lds->two[s][9][b], lds->two[s][10][b]);
@@ -548,8 +563,8 @@ BC6_TASK void estimate_errors(Bc6Ptr lds, int b, int quarter)
         error7 += error.estimate(interpolate_integers(s ? u7[2] : u7[0], s ? u7[3] : u7[1], weight));
         error9 += error.estimate(interpolate_integers(s ? u9[2] : u9[0], s ? u9[3] : u9[1], weight));
     }
-    lds->indices[0][quarter][b] = indices4; lds->indices[1][quarter][b] = indices3;
-    lds->errors[0][quarter][b] = error1; lds->errors[1][quarter][b] = error7; lds->errors[2][quarter][b] = error9;
+    lds->indices[1][quarter][b] = indices3;
+    lds->errors[1][quarter][b] = error7; lds->errors[2][quarter][b] = error9;
 }
 
 // What the estimates say of the choice between the candidates; 3: nothing.  An estimate and the error as it is defined
@@ -686,9 +701,15 @@ bc6_compress_kernel(BlockCompressArgs a)
     }
     if (__any(mask != 0u)) score_candidates<WIDE>(lds, lane, wave, mask);
     __syncthreads();
-    if (wave < 2) subset_ends<WIDE>(lds, lane, wave);
+    // (two waves for the subsets, the others for the candidate that has none: as much work)
+    if (wave < 2) {
+        subset_ends<WIDE>(lds, lane, wave);
+    } else {
+        estimate_one_subset<WIDE>(lds, lane, 2 * wave - 4);
+        estimate_one_subset<WIDE>(lds, lane, 2 * wave - 3);
+    }
     __syncthreads();
-    estimate_errors<WIDE>(lds, lane, wave);
+    estimate_two_subsets<WIDE>(lds, lane, wave);
     __syncthreads();
     int choice = estimated_choice(lds, lane);
     uint64_t const open = __ballot(choice == 3);             // the same in all waves, few
