@@ -520,14 +520,33 @@ typedef __attribute__((address_space(1))) u32_align2 const* GlobalU32A2Ptr;
 // 6 or 8 bytes and a 2 x 2 footprint usually lies in one or two cache lines.
 typedef __attribute__((address_space(1))) u32x2 const* GlobalU32x2Ptr;
 
+// Byte offset of a cell in the brick order: the sum of what its column and its row say, each taken once for two taps.
+// (Below 2^32: a grid holds less than 2^31 bytes.)
 template <int LAYERS>
-__device__ __forceinline__ uint32_t brick_offset(uint32_t cx, uint32_t cy, uint32_t log2GridWidth)
+__device__ __forceinline__ uint32_t brick_column(uint32_t cx)
+{
+    constexpr uint32_t T = brick_side_log2(LAYERS), MASK = (1u << T) - 1u;
+    return (cx >> T) * uint32_t(brick_bytes(LAYERS)) + (cx & MASK) * uint32_t(2 * LAYERS);
+}
+template <int LAYERS>
+__device__ __forceinline__ uint32_t brick_row(uint32_t cy, uint32_t log2GridWidth)
 {
     constexpr uint32_t T = brick_side_log2(LAYERS), MASK = (1u << T) - 1u;
     uint32_t const lgBricksX = log2GridWidth > T ? log2GridWidth - T : 0u;
-    uint32_t const brick = ((cy >> T) << lgBricksX) + (cx >> T);
-    uint32_t const cell = ((cy & MASK) << T) + (cx & MASK);
-    return brick * uint32_t(brick_bytes(LAYERS)) + cell * uint32_t(2 * LAYERS);     // below 2^32: a grid holds less than 2^31 bytes
+    return ((cy >> T) << lgBricksX) * uint32_t(brick_bytes(LAYERS)) + (cy & MASK) * uint32_t(2 * LAYERS << T);
+}
+
+template <int LAYERS> __device__ __forceinline__ void load_brick_cell(GlobalU8Ptr base, uint32_t off, uint32_t (&out)[2]);
+// The cells of the four taps: (x0, y0), (x1, y0), (x0, y1), (x1, y1).
+template <int LAYERS>
+__device__ __forceinline__ void load_brick_cells(GlobalU8Ptr base, uint32_t x0, uint32_t x1, uint32_t y0, uint32_t y1, uint32_t log2GridWidth, uint32_t (&out)[4][2])
+{
+    uint32_t const c0 = brick_column<LAYERS>(x0), c1 = brick_column<LAYERS>(x1);
+    uint32_t const r0 = brick_row<LAYERS>(y0, log2GridWidth), r1 = brick_row<LAYERS>(y1, log2GridWidth);
+    load_brick_cell<LAYERS>(base, r0 + c0, out[0]);
+    load_brick_cell<LAYERS>(base, r0 + c1, out[1]);
+    load_brick_cell<LAYERS>(base, r1 + c0, out[2]);
+    load_brick_cell<LAYERS>(base, r1 + c1, out[3]);
 }
 
 // All layers of one cell: layer L in the low or high half of out[L / 2].
@@ -551,6 +570,34 @@ __device__ __forceinline__ void load_brick_cell(GlobalU8Ptr base, uint32_t off, 
 // What a query needs of its mip, kept in LDS: every lane of a wave may address another mip, and
 // fetching these fields per lane from the table in global memory put a long dependent load in
 // front of the latent gathers.
+// The lane's query of the 64 of a wave, the call's last one again beyond it.  Whole waves, all but one of a call, read and
+// write at lane offsets from scalar addresses: a store takes half the instructions.  (With the
+// taps' offsets by column and row, 2^24 queries of the headline network 588.8 -> 575.7 us, 2^22 of the 0.9.2 one 163 -> 158.)
+__device__ __forceinline__ DevQuery load_query(DevQuery const* queries, uint64_t q0, uint64_t numQueries, int lane)
+{
+    if (q0 + 64u <= numQueries) {                            // uniform
+        GlobalU8Ptr const first = (GlobalU8Ptr)uniform_pointer(reinterpret_cast<uint64_t>(queries + q0));
+        __attribute__((address_space(1))) DevQuery const* const own = reinterpret_cast<__attribute__((address_space(1))) DevQuery const*>(first + uint32_t(lane) * uint32_t(sizeof(DevQuery)));
+        return DevQuery{ own->u, own->v, own->mip };
+    }
+    return queries[min(q0 + uint64_t(lane), numQueries - 1)];
+}
+
+// The outputs of a whole wave of valid queries, none of which can overflow a half: lane (j, g) holds channels 4g..4g+3 of query
+// q0 + 16b + j.
+template <class ACC>
+__device__ __forceinline__ void store_whole_queries(uint16_t* out, uint64_t q0, int j, int g, ACC const (&D)[4], v4f S)
+{
+    GlobalOutPtr const first = uniform_pointer(reinterpret_cast<uint64_t>(out + q0 * 16u));
+    uint32_t const own = uint32_t(j) * 32u + uint32_t(g) * 8u;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        uint32_t const h01 = to_half2_bits<false>(float(D[b][0]) * S[0], float(D[b][1]) * S[1]);
+        uint32_t const h23 = to_half2_bits<false>(float(D[b][2]) * S[2], float(D[b][3]) * S[3]);
+        *reinterpret_cast<__attribute__((address_space(1))) u32x2*>(first + (own + 512u * uint32_t(b))) = u32x2{ h01, h23 };
+    }
+}
+
 struct QueryMip {
     uint16_t const* hr;
     uint16_t const* lr;

@@ -429,10 +429,7 @@ __device__ __forceinline__ void fetch_latents_bricked(Mip const& m, int x, int y
         uint32_t const lg = (axisX >> 24) & 0xffu;                // log2(grid width)
         f.fx[grid] = ax.f; f.fy[grid] = ay.f;
         uint32_t cell[4][2];                                      // taps 00, 10, 01, 11
-        load_brick_cell<LAYERS>(g, brick_offset<LAYERS>(ax.c0, ay.c0, lg), cell[0]);
-        load_brick_cell<LAYERS>(g, brick_offset<LAYERS>(ax.c1, ay.c0, lg), cell[1]);
-        load_brick_cell<LAYERS>(g, brick_offset<LAYERS>(ax.c0, ay.c1, lg), cell[2]);
-        load_brick_cell<LAYERS>(g, brick_offset<LAYERS>(ax.c1, ay.c1, lg), cell[3]);
+        load_brick_cells<LAYERS>(g, ax.c0, ax.c1, ay.c0, ay.c1, lg, cell);
 #pragma unroll
         for (int L = 0; L < LAYERS; ++L)
 #pragma unroll
@@ -866,8 +863,7 @@ query_fp8_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queri
     for (uint64_t block = blockIdx.x; block < numBlocks; block += uint32_t(workgroups)) {
         uint64_t const q0 = block * perBlock + uint64_t(wave) * 64;
         if (q0 >= numQueries || wave >= waves) continue;
-        uint64_t const qi = min(q0 + uint64_t(lane), numQueries - 1);
-        DevQuery const query = queries[qi];
+        DevQuery const query = load_query(queries, q0, numQueries, lane);
         bool const validMip = query.mip >= 0 && query.mip < numMips;
         QueryMip const& m = qmips[validMip ? query.mip : 0];
         int x = int(floorf(query.u * float(m.width)));
@@ -888,21 +884,21 @@ query_fp8_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queri
         mlp_forward_fp8<V>(lds, wave, lane, modes, in, D, S);
 
         // lane (j, g) holds channels 4g..4g+3 of query q0 + 16b + j; validity travels by shuffle
-        auto store_outputs = [&](auto checked) __attribute__((always_inline)) {
-            constexpr bool CHECKED = decltype(checked)::value;
+        auto store_outputs = [&]() __attribute__((always_inline)) {
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
                 uint64_t const q = q0 + uint64_t(16 * b + j);
                 int const ok = __shfl(validMip ? 1 : 0, 16 * b + j, 64);
                 if (q >= numQueries) continue;
-                uint32_t h01 = to_half2_bits<CHECKED>(float(D[b][0]) * S[0], float(D[b][1]) * S[1]);
-                uint32_t h23 = to_half2_bits<CHECKED>(float(D[b][2]) * S[2], float(D[b][3]) * S[3]);
+                uint32_t h01 = to_half2_bits(float(D[b][0]) * S[0], float(D[b][1]) * S[1]);
+                uint32_t h23 = to_half2_bits(float(D[b][2]) * S[2], float(D[b][3]) * S[3]);
                 if (!ok) { h01 = 0; h23 = 0; }
                 *reinterpret_cast<u32x2*>(out + q * 16 + 4 * g) = u32x2{ h01, h23 };
             }
         };
-        if (V::ONE && (modes & kFp8OutputsBounded)) store_outputs(std::false_type{});      // see decode_fp8_kernel
-        else                                        store_outputs(std::true_type{});
+        // (see decode_fp8_kernel)
+        if (V::ONE && (modes & kFp8OutputsBounded) && __all(validMip) && q0 + 64u <= numQueries) store_whole_queries(out, q0, j, g, D, S);
+        else                                                                                     store_outputs();
     }
 }
 

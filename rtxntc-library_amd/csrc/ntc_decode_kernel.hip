@@ -713,14 +713,8 @@ __device__ __forceinline__ void prepare_inputs_bricked(Mip const& m, LdsT<V> con
 
     // taps in the order a00 (x0, y0), a10 (x1, y0), a01 (x0, y1), a11 (x1, y1)
     uint32_t hc[4][2], lc[4][2];
-    load_brick_cell<HL>(gh, brick_offset<HL>(hx.c0, hy.c0, hlg), hc[0]);
-    load_brick_cell<HL>(gh, brick_offset<HL>(hx.c1, hy.c0, hlg), hc[1]);
-    load_brick_cell<HL>(gh, brick_offset<HL>(hx.c0, hy.c1, hlg), hc[2]);
-    load_brick_cell<HL>(gh, brick_offset<HL>(hx.c1, hy.c1, hlg), hc[3]);
-    load_brick_cell<LL>(gl, brick_offset<LL>(lx.c0, ly.c0, llg), lc[0]);
-    load_brick_cell<LL>(gl, brick_offset<LL>(lx.c1, ly.c0, llg), lc[1]);
-    load_brick_cell<LL>(gl, brick_offset<LL>(lx.c0, ly.c1, llg), lc[2]);
-    load_brick_cell<LL>(gl, brick_offset<LL>(lx.c1, ly.c1, llg), lc[3]);
+    load_brick_cells<HL>(gh, hx.c0, hx.c1, hy.c0, hy.c1, hlg, hc);
+    load_brick_cells<LL>(gl, lx.c0, lx.c1, ly.c0, ly.c1, llg, lc);
     __builtin_amdgcn_sched_barrier(0);                       // all loads before any arithmetic
 
     auto layer_of = [](uint32_t const (&cell)[2], int L) -> uint32_t { return (L & 1) ? cell[L >> 1] >> 16 : cell[L >> 1] & 0xffffu; };
@@ -1429,11 +1423,10 @@ __device__ __forceinline__ bool prepare_query_inputs(DevMip const* mips, QueryMi
     return validMip;
 }
 
-template <bool CHECKED>
 __device__ __forceinline__ void store_query_outputs(uint16_t* out, v4f F, v4f S, bool valid)
 {
-    uint32_t h01 = to_half2_bits<CHECKED>(F[0] * S[0], F[1] * S[1]);
-    uint32_t h23 = to_half2_bits<CHECKED>(F[2] * S[2], F[3] * S[3]);
+    uint32_t h01 = to_half2_bits(F[0] * S[0], F[1] * S[1]);
+    uint32_t h23 = to_half2_bits(F[2] * S[2], F[3] * S[3]);
     if (!valid) { h01 = 0; h23 = 0; }
     *reinterpret_cast<u32x2*>(out) = u32x2{ h01, h23 };
 }
@@ -1467,26 +1460,25 @@ query_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queries, 
         uint64_t const q0 = block * perBlock + uint64_t(wave) * 64;
         if (q0 >= numQueries || wave >= waves) continue;
         uint32_t in[16];
-        bool const validMip = prepare_query_inputs<V>(mips, qmips, numMips, bricked, lds, queries[min(q0 + uint64_t(lane), numQueries - 1)], in);
+        bool const validMip = prepare_query_inputs<V>(mips, qmips, numMips, bricked, lds, load_query(queries, q0, numQueries, lane), in);
+        bool const whole = __all(validMip) && q0 + 64u <= numQueries;
 
         // lane (j, g) holds channels 4g..4g+3 of query q0 + 16b + j; validity travels by shuffle
-        auto store_outputs = [&](auto checked, int b, v4f Fb, v4f S) __attribute__((always_inline)) {
-            constexpr bool CHECKED = decltype(checked)::value;
+        auto store_outputs = [&](int b, v4f Fb, v4f S) __attribute__((always_inline)) {
             uint64_t const q = q0 + uint64_t(16 * b + j);
             int const ok = __shfl(validMip ? 1 : 0, 16 * b + j, 64);
-            if (q < numQueries) store_query_outputs<CHECKED>(out + q * 16 + 4 * g, Fb, S, ok != 0);
+            if (q < numQueries) store_query_outputs(out + q * 16 + 4 * g, Fb, S, ok != 0);
         };
         if (V::F16_LAYERS && useF16) {
             // output-layer accumulators as floats: exact integers below 2^24
             v4f F[4];
             v4f S;
             mlp_forward_f16<V>(lds, wave, lane, (staged & kL0Magic) != 0, in, F, S);
-            if (staged & kOutputsBounded) {                                                  // as in decode_kernel
-#pragma unroll
-                for (int b = 0; b < 4; ++b) store_outputs(std::false_type{}, b, F[b], S);
+            if ((staged & kOutputsBounded) && whole) {                                       // as in decode_kernel
+                store_whole_queries(out, q0, j, g, F, S);
             } else {
 #pragma unroll
-                for (int b = 0; b < 4; ++b) store_outputs(std::true_type{}, b, F[b], S);
+                for (int b = 0; b < 4; ++b) store_outputs(b, F[b], S);
             }
         } else {
             // every layer on the int8 matrix instruction, one 16-query block at a time; the int32 -> float
@@ -1499,7 +1491,7 @@ query_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queries, 
                 int laneB = lane;
                 asm volatile("" : "+v"(laneB));                  // keeps the weight reads inside the loop
                 mlp_forward_block<V>(lds, laneB, read_input_block<V>(lds, wave, lane, b), D, S);
-                store_outputs(std::true_type{}, b, v4f{ float(D[0]), float(D[1]), float(D[2]), float(D[3]) }, S);
+                store_outputs(b, v4f{ float(D[0]), float(D[1]), float(D[2]), float(D[3]) }, S);
             }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
@@ -1535,7 +1527,7 @@ query_few_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queri
         mlp_forward_block<V>(lds, lane, X, D, S);
         F = v4f{ float(D[0]), float(D[1]), float(D[2]), float(D[3]) };
     }
-    if (q < numQueries) store_query_outputs<true>(out + q * 16 + 4 * g, F, S, valid);
+    if (q < numQueries) store_query_outputs(out + q * 16 + 4 * g, F, S, valid);
 }
 
 // 16x64 by 64x16 int8 product with the operand layout the decode kernel assumes.
