@@ -415,7 +415,7 @@ __device__ __forceinline__ void fetch_latents_fast(Mip const& m, int x, int y, F
 }
 
 // The same cells from the query-ordered copy of the grids (bricks with all layers of a cell together): four
-// loads per grid instead of four per layer.
+// loads per grid instead of four per layer.  Odd layers' cells are the upper halves of the words.
 template <class V, class Mip>
 __device__ __forceinline__ void fetch_latents_bricked(Mip const& m, int x, int y, Fp8Fetch<V>& f)
 {
@@ -433,13 +433,13 @@ __device__ __forceinline__ void fetch_latents_bricked(Mip const& m, int x, int y
 #pragma unroll
         for (int L = 0; L < LAYERS; ++L)
 #pragma unroll
-            for (int tap = 0; tap < 4; ++tap)
-                f.cell[grid][L][tap] = (L & 1) ? cell[tap][L >> 1] >> 16 : cell[tap][L >> 1] & 0xffffu;
+            for (int tap = 0; tap < 4; ++tap) f.cell[grid][L][tap] = cell[tap][L >> 1];
     }
 }
 
+// (bricked, uniform: the cells are fetch_latents_bricked's)
 template <class V, class Mip>
-__device__ __forceinline__ void finish_inputs_fast(Mip const& m, Fp8Lds<V> const& lds, int x, int y, Fp8Fetch<V> const& f, uint32_t (&in)[24])
+__device__ __forceinline__ void finish_inputs_fast(Mip const& m, Fp8Lds<V> const& lds, int x, int y, Fp8Fetch<V> const& f, bool bricked, uint32_t (&in)[24])
 {
 #pragma unroll
     for (int i = 0; i < 24; ++i) in[i] = 0;
@@ -448,7 +448,8 @@ __device__ __forceinline__ void finish_inputs_fast(Mip const& m, Fp8Lds<V> const
         uint32_t const axisX = grid == 0 ? m.hrAxisX : m.lrAxisX, axisY = grid == 0 ? m.hrAxisY : m.lrAxisY;
         uint32_t const nx = (axisX >> 8) & 0xffu, ny = (axisY >> 8) & 0xffu;
         uint32_t const wx1 = f.fx[grid], wx0 = (1u << nx) - wx1, wy1 = f.fy[grid], wy0 = (1u << ny) - wy1;
-        uint32_t const msk = 0x000f000fu, sel = 0x0c010c00u;     // v_perm_b32: bytes [0, zero, 1, zero] of the cell
+        uint32_t const msk = 0x000f000fu;
+        uint32_t const sels[2] = { 0x0c010c00u, bricked ? 0x0c030c02u : 0x0c010c00u };       // v_perm_b32: bytes [0, zero, 1, zero] of the cell
         uint32_t const n = nx + ny;
         if (V::F % 4 == 0 && n <= 6u && !(n & 1u)) {             // (uniform in the raster kernel, per lane for queries)
             // Table form: with doubled weights and start values 2*base resp. 17 * 2*base the 16-bit lanes of T and
@@ -459,6 +460,7 @@ __device__ __forceinline__ void finish_inputs_fast(Mip const& m, Fp8Lds<V> const
             uint8_t const* const lut = reinterpret_cast<uint8_t const*>(lds.featureLut);
 #pragma unroll
             for (int L = 0; L < Fp8Fetch<V>::LAYERS; ++L) {
+                uint32_t const sel = sels[L & 1];
                 uint32_t const p00 = __builtin_amdgcn_perm(0u, f.cell[grid][L][0], sel), p10 = __builtin_amdgcn_perm(0u, f.cell[grid][L][1], sel);
                 uint32_t const p01 = __builtin_amdgcn_perm(0u, f.cell[grid][L][2], sel), p11 = __builtin_amdgcn_perm(0u, f.cell[grid][L][3], sel);
                 uint32_t const S = mad24(w11, p11, mad24(w01, p01, mad24(w10, p10, mad24(w00, p00, s0))));
@@ -475,6 +477,7 @@ __device__ __forceinline__ void finish_inputs_fast(Mip const& m, Fp8Lds<V> const
         float const k = __builtin_ldexpf(0.13333334f, -int(nx + ny));
 #pragma unroll
         for (int L = 0; L < Fp8Fetch<V>::LAYERS; ++L) {
+            uint32_t const sel = sels[L & 1];
             uint32_t const p00 = __builtin_amdgcn_perm(0u, f.cell[grid][L][0], sel), p10 = __builtin_amdgcn_perm(0u, f.cell[grid][L][1], sel);
             uint32_t const p01 = __builtin_amdgcn_perm(0u, f.cell[grid][L][2], sel), p11 = __builtin_amdgcn_perm(0u, f.cell[grid][L][3], sel);
             uint32_t const S = mad24(w11, p11, mad24(w01, p01, mad24(w10, p10, mul24(w00, p00))));
@@ -766,7 +769,7 @@ decode_fp8_kernel(MipTable table, int numMips, int totalTiles, int workgroups, F
             if (m.fast) {
                 Fp8Fetch<V> fetch;
                 fetch_latents_fast<V>(m.full, x, y, fetch);
-                finish_inputs_fast<V>(m.full, lds, x, y, fetch, in);
+                finish_inputs_fast<V>(m.full, lds, x, y, fetch, false, in);
             } else {
                 prepare_inputs_fp8<V>(m.full, lds, x, y, in);
             }
@@ -875,7 +878,7 @@ query_fp8_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queri
             Fp8Fetch<V> fetch;
             if (bricked) fetch_latents_bricked<V>(m, x, y, fetch);
             else         fetch_latents_fast<V>(m, x, y, fetch);
-            finish_inputs_fast<V>(m, lds, x, y, fetch, in);
+            finish_inputs_fast<V>(m, lds, x, y, fetch, bricked, in);
         } else {
             prepare_inputs_fp8<V>(mips[validMip ? query.mip : 0], lds, x, y, in);
         }

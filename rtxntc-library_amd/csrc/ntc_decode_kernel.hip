@@ -66,11 +66,13 @@ __device__ __forceinline__ uint32_t activate4(v4i acc, v4f scale)
 // f0 + 16 f1 and f2 + 16 f3); E = P & 0x000f000f holds the even features alone.  S = sum w*P and T = sum w*E stay
 // below 2^16 per lane (255 * 2^n), so lanes never mix, and (S - T) / 16 is sum w*f for the odd features, exactly.
 // Times 17 (T + 16 T, and D/16 + D for the odd ones) is at most 17 * 15 * 2^8 < 2^16: still inside the lane.
+// UPPER: the cells are the upper halves of what is given.
+template <bool UPPER = false>
 __device__ __forceinline__ uint32_t bilinear4_int(uint32_t c00, uint32_t c10, uint32_t c01, uint32_t c11,
                                                   uint32_t w00, uint32_t w10, uint32_t w01, uint32_t w11, uint32_t n)
 {
     uint32_t const m = 0x000f000fu;
-    uint32_t const sel = 0x0c010c00u;                        // v_perm_b32: bytes [0, zero, 1, zero] of the cell
+    uint32_t const sel = UPPER ? 0x0c030c02u : 0x0c010c00u;  // v_perm_b32: bytes [0, zero, 1, zero] of the cell
     uint32_t const p00 = __builtin_amdgcn_perm(0u, c00, sel), p10 = __builtin_amdgcn_perm(0u, c10, sel);
     uint32_t const p01 = __builtin_amdgcn_perm(0u, c01, sel), p11 = __builtin_amdgcn_perm(0u, c11, sel);
     uint32_t const S = mad24(w11, p11, mad24(w01, p01, mad24(w10, p10, mul24(w00, p00))));
@@ -717,7 +719,11 @@ __device__ __forceinline__ void prepare_inputs_bricked(Mip const& m, LdsT<V> con
     load_brick_cells<LL>(gl, lx.c0, lx.c1, ly.c0, ly.c1, llg, lc);
     __builtin_amdgcn_sched_barrier(0);                       // all loads before any arithmetic
 
-    auto layer_of = [](uint32_t const (&cell)[2], int L) -> uint32_t { return (L & 1) ? cell[L >> 1] >> 16 : cell[L >> 1] & 0xffffu; };
+    // layer L lies in the lower or the upper half of a word
+    auto const filtered = [](uint32_t const (&c)[4][2], auto layer, uint32_t w00, uint32_t w10, uint32_t w01, uint32_t w11, uint32_t n) {
+        constexpr int at = decltype(layer)::value >> 1;
+        return bilinear4_int<(decltype(layer)::value & 1) != 0>(c[0][at], c[1][at], c[2][at], c[3][at], w00, w10, w01, w11, n);
+    };
     if constexpr (V::HR_MODE == 1) {
         static_assert(V::HR_MODE != 1 || (V::HR_BITS == 2 && V::HR_F == 8 && V::HR_SLOTS == 8), "concat grids: 8 x 2-bit");
 #pragma unroll
@@ -729,23 +735,31 @@ __device__ __forceinline__ void prepare_inputs_bricked(Mip const& m, LdsT<V> con
         uint32_t const nx = (m.hrAxisX >> 8) & 0xffu, ny = (m.hrAxisY >> 8) & 0xffu;
         uint32_t const wx1 = hx.f, wx0 = (1u << nx) - hx.f, wy1 = hy.f, wy0 = (1u << ny) - hy.f;
         uint32_t const w00 = mul24(wx0, wy0), w10 = mul24(wx1, wy0), w01 = mul24(wx0, wy1), w11 = mul24(wx1, wy1);
-#pragma unroll
-        for (int L = 0; L < HL; ++L) {
-            uint32_t b = bilinear4_int(layer_of(hc[0], L), layer_of(hc[1], L), layer_of(hc[2], L), layer_of(hc[3], L), w00, w10, w01, w11, nx + ny);
-            if (4 * L + 4 > V::HR_F) b &= (1u << (8 * (V::HR_F - 4 * L))) - 1u;
-            in[L] = b;
-        }
+        auto const layer = [&](auto number) {
+            constexpr int L = decltype(number)::value;
+            if constexpr (L < HL) {
+                uint32_t b = filtered(hc, number, w00, w10, w01, w11, nx + ny);
+                if (4 * L + 4 > V::HR_F) b &= (1u << (8 * (V::HR_F - 4 * L))) - 1u;
+                in[L] = b;
+            }
+        };
+        layer(std::integral_constant<int, 0>{}); layer(std::integral_constant<int, 1>{});
+        layer(std::integral_constant<int, 2>{}); layer(std::integral_constant<int, 3>{});
     }
     {
         uint32_t const nx = (m.lrAxisX >> 8) & 0xffu, ny = (m.lrAxisY >> 8) & 0xffu;
         uint32_t const wx1 = lx.f, wx0 = (1u << nx) - lx.f, wy1 = ly.f, wy0 = (1u << ny) - ly.f;
         uint32_t const w00 = mul24(wx0, wy0), w10 = mul24(wx1, wy0), w01 = mul24(wx0, wy1), w11 = mul24(wx1, wy1);
-#pragma unroll
-        for (int L = 0; L < LL; ++L) {
-            uint32_t b = bilinear4_int(layer_of(lc[0], L), layer_of(lc[1], L), layer_of(lc[2], L), layer_of(lc[3], L), w00, w10, w01, w11, nx + ny);
-            if (4 * L + 4 > V::LR_F) b &= (1u << (8 * (V::LR_F - 4 * L))) - 1u;
-            in[V::HR_INPUTS / 4 + L] = b;
-        }
+        auto const layer = [&](auto number) {
+            constexpr int L = decltype(number)::value;
+            if constexpr (L < LL) {
+                uint32_t b = filtered(lc, number, w00, w10, w01, w11, nx + ny);
+                if (4 * L + 4 > V::LR_F) b &= (1u << (8 * (V::LR_F - 4 * L))) - 1u;
+                in[V::HR_INPUTS / 4 + L] = b;
+            }
+        };
+        layer(std::integral_constant<int, 0>{}); layer(std::integral_constant<int, 1>{});
+        layer(std::integral_constant<int, 2>{}); layer(std::integral_constant<int, 3>{});
     }
     {
         position_from_tables<V>(m.posMask, lds, x, y, in);
