@@ -182,9 +182,13 @@ __device__ __forceinline__ float divide_by_top(float a, float top, float recipro
     return __builtin_fmaf(a, reciprocal, a * float(1.0 / double(top) - double(reciprocal)));
 }
 
-// HashBasedRNG, src/CudaUtils.h:117-184: Jenkins hash of the pixel index seeds a Murmur3 round per draw.
+// HashBasedRNG, src/CudaUtils.h:117-184: Jenkins hash of the pixel index seeds a Murmur3 round per draw.  The round turns
+// the exclusive or of the seed and the draw's word by 13 bits; here each is turned by itself, the seed once for all draws.
+// And an instruction of three operands takes the place of one with a shifted one, which shares no issue slot (2048 x 2048
+// RGBA of 8 bits, dithered, 18.7 -> 18.3 us).
+__device__ __forceinline__ constexpr uint32_t turned_left(uint32_t v, int bits) { return v << bits | v >> (32 - bits); }
 struct DitherRng {
-    uint32_t seed, index;
+    uint32_t seed, index;                                    // the seed turned by 13 bits
     __device__ DitherRng() {}
     __device__ explicit DitherRng(uint32_t linearIndex) : index(0)
     {
@@ -195,7 +199,7 @@ struct DitherRng {
         a = (a + 0xd3a2646cu) ^ (a << 9);
         a = (a + 0xfd7046c5u) + (a << 3);
         a = (a ^ 0xb55a4f09u) ^ (a >> 16);
-        seed = a;
+        seed = turned_left(a, 13);
     }
     __device__ float next_offset()                           // a draw of [0, 1) less one half (both differences are exact)
     {
@@ -203,13 +207,10 @@ struct DitherRng {
     }
     __device__ float offset(uint32_t draw) const             // that of one draw, counted from 0
     {
-        uint32_t k = (draw + 1u) * 0xcc9e2d51u;
-        k = (k << 15) | (k >> 17);
-        k *= 0x1b873593u;
-        uint32_t h = seed ^ k;
-        h = ((h << 13) | (h >> 19)) * 5u + 0xe6546b64u;
-        h ^= 4u;
-        h ^= h >> 16; h *= 0x85ebca6bu;
+        uint32_t const k = turned_left(turned_left((draw + 1u) * 0xcc9e2d51u, 15) * 0x1b873593u, 13);
+        uint32_t h = (seed ^ k) * 5u + 0xe6546b64u;
+        h = __builtin_amdgcn_bitop3_b32(h, h >> 16, 4u, 0x96);               // h ^= 4, h ^= h >> 16
+        h *= 0x85ebca6bu;
         h ^= h >> 13; h *= 0xc2b2ae35u;
         h ^= h >> 16;
         return __builtin_bit_cast(float, (h & 0x7fffffu) | 0x3f800000u) - 1.5f;
