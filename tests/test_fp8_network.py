@@ -370,6 +370,31 @@ def test_gpu_fp8_outputs_near_and_beyond_the_fp16_range(ntc, device, scale):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("bias", [0, 1, (1 << 24) - 520193, (1 << 24) - 520192, (1 << 24) - 520191, (1 << 24) + 1, 0x7fffffff])
+@pytest.mark.parametrize("form", ["random", "zero", "extreme"])
+def test_gpu_fp8_output_sums_from_the_bias(ntc, device, bias, form):
+    """The output layer's sums start at the bias where every bias of the layer is at most 2^24 - 32 * 127 * 128, either
+    sign: both sides of that line, with drawn weights, with none (a sum of nothing keeps the sign of its zero) and with
+    weights of -128 throughout.  The sums are integers below 2^24 on the float path, so the outputs are the checker's
+    bytes; halves of sums near 2^24 step by 2^13, so a sum off by one shows in 1 of 8192 outputs, of 131072 here."""
+    layout = ntc.synth.weight_layout(ntc.presets.spec_ref092_fp8(16))
+    last = ntc.abi.MLP_LAYERS - 1
+    case = fp8_case(ntc, 16, 128, 64, 4, 2, 16, ntc.abi.OUT_FP16_PLANAR_PAIRS, seed=402, bias_sigma=0.5)
+    channels = np.arange(16)
+    case.weights[layout.scaleOffset[last]:layout.scaleOffset[last] + 64] = np.full(16, 0.0021, dtype=np.float32).view(np.uint8)
+    biases = np.where(channels % 2 == 0, bias, -bias).astype(np.int32)
+    if bias > 1 << 20:
+        biases[channels >= 12] = [3, -3, 0, 77]
+    case.weights[layout.biasOffset[last]:layout.biasOffset[last] + 64] = biases.view(np.uint8)
+    if form != "random":
+        w = case.weights[layout.weightOffset[last]:layout.weightOffset[last] + 16 * 32]
+        w[:] = 0 if form == "zero" else 128
+    expected, got = run_both(device, case)
+    assert first_mismatch(expected, got) is None, (bias, form)
+    assert np.count_nonzero(got) > 0 or bias < 2
+
+
+@pytest.mark.gpu
 def test_gpu_fp8_level_of_detail_input_up_to_three(ntc, device):
     """The exactness of the layer sums is proven for inputs of at most 3 in magnitude.  Features and positional
     encoding lie in [-1, 1]; the level-of-detail input comes from the caller's descriptor: +-3 decodes to the
