@@ -751,7 +751,7 @@ __device__ __forceinline__ void mlp_forward_fp8(Fp8Lds<V>& lds, int wave, int la
 // of a common sequence drift apart in time, and the latent reads from memory doubled.)
 template <class V>
 __global__ void __launch_bounds__(V::THREADS, 1)
-decode_fp8_kernel(MipTable table, int numMips, int totalTiles, int workgroups, Fp8Handoff handoff)
+decode_fp8_kernel(MipTable table, int numMips, TileShares shares, Fp8Handoff handoff)
 {
     DevMip const* const mips = table_entries(table.entries);
     bool const every = !V::ONE && !handoff.word;
@@ -762,9 +762,8 @@ decode_fp8_kernel(MipTable table, int numMips, int totalTiles, int workgroups, F
     int const member = wave >> 2;                            // which quartet of the workgroup
     int const j = lane & 15, g = lane >> 4;
 
-    int const per = (totalTiles + workgroups - 1) / workgroups;
-    int const tileBegin = blockIdx.x * per;
-    int const tileEnd = min(totalTiles, tileBegin + per);
+    TileRange const tiles = tiles_of_workgroup<false>(shares, blockIdx.x);
+    int const tileBegin = tiles.begin, tileEnd = tiles.end;
     if (tileBegin >= tileEnd) return;                        // uniform across the workgroup
 
     int modes = 7;                                           // uniform: the hidden layers' modes (stage_fp8_weights)
@@ -943,10 +942,10 @@ static hipError_t launch_fp8_variant(MipTable const& mips, int numMips, int tota
     // 11.0 and 25.1 us in two launches, 9.6 and 24.6 in one; 2048 x 1024: 74.7 and 76.7.  With two planes: 15.3 and 34.0,
     // 11.2 and 29.8.)
     if (totalTiles <= 8 * compute_units_of_current_device())
-        return launch_kernel<decode_fp8_kernel<Any>>(dim3(gridSize), dim3(Any::THREADS), 0, stream, mips, numMips, totalTiles, gridSize, Fp8Handoff{ nullptr, 0u });
-    hipError_t const e = launch_kernel<decode_fp8_kernel<One>>(dim3(gridSize), dim3(One::THREADS), 0, stream, mips, numMips, totalTiles, gridSize, handoff);
+        return launch_kernel<decode_fp8_kernel<Any>>(dim3(gridSize), dim3(Any::THREADS), 0, stream, mips, numMips, tile_shares(totalTiles, gridSize), Fp8Handoff{ nullptr, 0u });
+    hipError_t const e = launch_kernel<decode_fp8_kernel<One>>(dim3(gridSize), dim3(One::THREADS), 0, stream, mips, numMips, tile_shares(totalTiles, gridSize), handoff);
     if (e != hipSuccess) return e;
-    return launch_kernel<decode_fp8_kernel<Any>>(dim3(gridSize), dim3(Any::THREADS), 0, stream, mips, numMips, totalTiles, gridSize, handoff);
+    return launch_kernel<decode_fp8_kernel<Any>>(dim3(gridSize), dim3(Any::THREADS), 0, stream, mips, numMips, tile_shares(totalTiles, gridSize), handoff);
 }
 
 hipError_t launch_decode_fp8(int variant, MipTable const& mips, int numMips, int totalTiles, int gridSize, Fp8Handoff handoff, hipStream_t stream)

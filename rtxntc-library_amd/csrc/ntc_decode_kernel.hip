@@ -1172,7 +1172,7 @@ __device__ __forceinline__ int inlined_entry_of(int tile)
 
 template <class V>
 __global__ void __launch_bounds__(V::THREADS, V::WAVES_PER_SIMD)
-decode_kernel(MipTable table, int numMips, int totalTiles, int workgroups)
+decode_kernel(MipTable table, int numMips, TileShares shares)
 {
     DevMip const* const mips = table_entries(table.entries);
     __shared__ LdsT<V> lds;
@@ -1182,15 +1182,8 @@ decode_kernel(MipTable table, int numMips, int totalTiles, int workgroups)
     int const member = wave >> 2;                            // which quartet this wave belongs to
     int const j = lane & 15, g = lane >> 4;
 
-    // Contiguous share of the tile list for this workgroup.  Workgroups are dealt to the eight dies (XCDs) of the
-    // device in turn, and each die has a cache of its own: the shares are numbered so that a die's workgroups hold
-    // neighbouring shares - one eighth of the list per die - and the grid rows that vertically adjacent shares both
-    // read come from memory once per die, not once per share.
-    int const per = (totalTiles + workgroups - 1) / workgroups;
-    constexpr int kDies = 8;
-    int const share = (workgroups % kDies == 0) ? int(blockIdx.x % kDies) * (workgroups / kDies) + int(blockIdx.x / kDies) : int(blockIdx.x);
-    int const tileBegin = share * per;
-    int const tileEnd = min(totalTiles, tileBegin + per);
+    TileRange const tiles = tiles_of_workgroup<true>(shares, blockIdx.x);
+    int const tileBegin = tiles.begin, tileEnd = tiles.end;
 
     uint8_t const* stagedBlob = nullptr;
     int staged = 0;                                          // uniform: how layers 1..3 of the staged set run (kStagedF16, ...)
@@ -1612,7 +1605,7 @@ static hipError_t launch_variant(MipTable const& mips, int numMips, int totalTil
     // against 7.9 with whole tiles.
     int const units = compute_units_of_current_device(), log2Parts = 4 * totalTiles <= units ? 2 : (2 * totalTiles <= units ? 1 : 0);
     if (log2Parts) return launch_kernel<decode_few_kernel<V>>(dim3(unsigned(totalTiles) << log2Parts), dim3(V::THREADS), 0, stream, mips, numMips, log2Parts);
-    return launch_kernel<decode_kernel<V>>(dim3(gridSize), dim3(V::THREADS), 0, stream, mips, numMips, totalTiles, gridSize);
+    return launch_kernel<decode_kernel<V>>(dim3(gridSize), dim3(V::THREADS), 0, stream, mips, numMips, tile_shares(totalTiles, gridSize));
 }
 
 hipError_t launch_decode(int variant, MipTable const& mips, int numMips, int totalTiles, int gridSize, hipStream_t stream)

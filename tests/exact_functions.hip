@@ -329,5 +329,12 @@ int exact_quotient_of_diagonals(Report* r) { return sweep<QuotientOfDiagonals>(r
 int exact_texel_centre(Report* r) { return sweep<TexelCentre>(r); }
 int exact_floors_of(Report* r) { return sweep<FloorsOf>(r); }
 int exact_filtered_features(Report* r) { return sweep<FilteredFeatures>(r); }
+// (on the host: the same code as on the device)
+void tiles_of_workgroup(int byDie, int totalTiles, int workgroups, int workgroup, int* range)
+{
+    ntc_hip_dev::TileShares const shares = ntc_hip_dev::tile_shares(totalTiles, workgroups);
+    ntc_hip_dev::TileRange const t = byDie ? ntc_hip_dev::tiles_of_workgroup<true>(shares, uint32_t(workgroup)) : ntc_hip_dev::tiles_of_workgroup<false>(shares, uint32_t(workgroup));
+    range[0] = t.begin; range[1] = t.end;
+}
 #endif
 }
