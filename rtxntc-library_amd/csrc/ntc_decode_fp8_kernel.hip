@@ -175,6 +175,15 @@ constexpr int kFp8OutputsBounded = 1 << 8;
 // bias, kept as a float, and stay integers that are exact in every order, with no conversion to an integer and back.
 // (2048 x 2048 of 12 mips: 183.6 -> 178.8 us for the 48 instructions of a tile's 64 x 16 outputs, of about 1700.)
 constexpr int kFp8SmallBias = 1 << 9, kFp8MostBias = (1 << 24) - 32 * 127 * 128;
+// Bit 10 + tile: the sums of this tile of 16 channels (of the nine of the hidden layers), on one plane, start at the bias:
+// with the bias, too, every partial sum is a multiple of one unit and below 2^24 of them, so that adding the bias first
+// gives the one rounding that adding it last gives.  The unit is 2^-18 or, where the channel's weights leave room, a finer
+// one: small biases have bits below 2^-18.  (144 additions less a texel, in the one-plane instantiation: 2048 x 2048 of 12
+// mips 184 -> 175.6 us with biases around 0.3, nine tenths of whose tiles start so, 184 -> 180 around 0.03, and the same as
+// before around 0.002, where none does.  With zeros to start at and the bias added behind a branch, read from LDS there,
+// tiles that do not start so were 2 - 5 % slower; the general instantiation, which also serves small launches, took 0.4 us
+// longer for 128 x 128 with the longer code.)
+constexpr int kFp8StartShift = 10, kFp8StartTiles = 0x1ff << kFp8StartShift;
 
 // Fills the positional table: one entry per thread, threads 0..62.
 template <class Lds>
@@ -276,7 +285,13 @@ __device__ __attribute__((noinline)) int stage_fp8_weights(Fp8Lds<V>& lds, uint8
         sum += __shfl_xor(sum, 16, 64);
         sum += __shfl_xor(sum, 32, 64);
         bool const wild = top != 0 || (bias & 0x7fffu) > 0x7b00u;       // or a bias that is not a finite half of at most 57344
-        found = (__any(wild) ? 1u << layer : 0u) | (__any(sum > kOnePlaneLimit) ? 16u << layer : 0u);
+        // the channel's sums in units of 2^-18, the bias included, and the finest unit in which they stay below 2^24
+        float const b = fabsf(float(__builtin_bit_cast(_Float16, uint16_t(bias))));
+        bool starts = V::ONE && sum <= kOnePlaneLimit && b < 64.f;
+        uint32_t const units = starts ? uint32_t(sum) * 1536u + uint32_t(__builtin_ceilf(b * 0x1p18f)) + 1u : 0u;
+        float const inUnits = __builtin_ldexpf(starts ? b : 0.f, 18 + __builtin_clz(units | 1u) - 8);
+        starts = starts && units < (1u << 24) && inUnits == floorf(inUnits);
+        found = (__any(wild) ? 1u << layer : 0u) | (__any(sum > kOnePlaneLimit) ? 16u << layer : 0u) | (__any(!starts) ? 1u << (kFp8StartShift + tile) : 0u);
     } else if (mine) {
         float const b = fabsf(float(int32_t(bias))), s = fabsf(__builtin_bit_cast(float, scale));
         found = (__any(!((b + 520192.f) * s < 60000.f) || !(b < 2.0e9f)) ? 1u << 8 : 0u)
@@ -291,7 +306,7 @@ __device__ __attribute__((noinline)) int stage_fp8_weights(Fp8Lds<V>& lds, uint8
     flags = __builtin_amdgcn_readfirstlane(flags);
     int const oneMask = int(~(flags >> 4) & ~flags & 7u);
     int const modes = int(flags & 7u) | (oneMask << kOnePlaneShift) | ((flags & (1u << 8)) ? 0 : kFp8OutputsBounded)
-                    | ((flags & (1u << 9)) ? 0 : kFp8SmallBias);
+                    | ((flags & (1u << 9)) ? 0 : kFp8SmallBias) | (int(~flags) & kFp8StartTiles);
     if (!own_fp8_set<V>(modes, every != 0) || !mine) return modes;
 
     if (layer == 3) {                                        // int8 weights as halves, 32 inputs = one block
@@ -299,7 +314,7 @@ __device__ __attribute__((noinline)) int stage_fp8_weights(Fp8Lds<V>& lds, uint8
         if (kg == 0) { (&lds.outScale[0][0])[i] = __builtin_bit_cast(float, scale); (&lds.outBias[0][0])[i] = (modes & kFp8SmallBias) ? __builtin_bit_cast(int32_t, float(int32_t(bias))) : int32_t(bias); }
         return modes;
     }
-    if (kg == 0) (&lds.bias[0][0][0])[16 * tile + i] = float(__builtin_bit_cast(_Float16, uint16_t(bias)));
+    if (kg == 0) (&lds.bias[0][0][0])[16 * tile + i] = float(__builtin_bit_cast(_Float16, uint16_t(bias))) + 0.f;      // (never -0)
     int32_t w[4][4];
 #pragma unroll
     for (int d = 0; d < 4; ++d) e4m3_times_512(v[d], w[d]);
@@ -506,7 +521,8 @@ __device__ __forceinline__ void finish_inputs_fast(Mip const& m, Fp8Lds<V> const
 // s2 = +0 and (s2 + s1) = s1 exactly (a plane's sum is never -0: its accumulator starts at +0), so the first
 // addition is left out; and its outputs are finite, so the activation's lower clamp is left out too.  With
 // PLANES == 1, s0 is the sum over the whole weights, which is what ((s2 + s1) + s0) comes to there without rounding.
-template <bool LAST_HIDDEN, int PLANES>
+// BIASED: the bias is in it.
+template <bool LAST_HIDDEN, int PLANES, bool BIASED>
 __device__ __forceinline__ void fp8_epilogue(v4f s2, v4f s1, v4f s0, v4f bias, uint32_t (&out)[2])
 {
     float r[4];
@@ -515,7 +531,7 @@ __device__ __forceinline__ void fp8_epilogue(v4f s2, v4f s1, v4f s0, v4f bias, u
         float a = s0[i];
         if (PLANES == 3)      a = (s2[i] + s1[i]) + s0[i];
         else if (PLANES == 2) a = s1[i] + s0[i];
-        r[i] = a + bias[i];
+        r[i] = BIASED ? a : a + bias[i];
     }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -570,8 +586,8 @@ struct TileOperands { uint4 a32[3][NK32]; uint2 a16[3]; v4f bias; };     // one 
 // One hidden layer: TILES output tiles of 16 channels; its inputs as NK32 blocks of 32 (B32[kb][b]) and, with
 // HAS16, one block of 16 (B16[b]); load(t, operands) reads tile t's weight operands and bias.  A layer with a
 // block of 16 runs on 16-deep instructions only (see mfma16).
-template <int PLANES, int TILES, int NK32, bool HAS16, bool LAST_HIDDEN, class Load>
-__device__ __forceinline__ void fp8_hidden_layer(Load&& load, uint4 const (&B32)[NK32][4], uint2 const (&B16)[4], uint32_t (&H)[4][4][2])
+template <int PLANES, bool MAY_START, int TILES, int NK32, bool HAS16, bool LAST_HIDDEN, class Load>
+__device__ __forceinline__ void fp8_hidden_layer(Load&& load, int started, uint4 const (&B32)[NK32][4], uint2 const (&B16)[4], uint32_t (&H)[4][4][2])
 {
     v4f const zero = { 0.f, 0.f, 0.f, 0.f };
     // The operands of output tile t + 1 are loaded before the work on tile t (two sets of registers, alternating);
@@ -591,45 +607,50 @@ __device__ __forceinline__ void fp8_hidden_layer(Load&& load, uint4 const (&B32)
             __builtin_amdgcn_sched_barrier(0x67f);           // everything but LDS instructions may cross
         }
         TileOperands<NK32, HAS16> const& o = ops[t & 1];
-        __builtin_amdgcn_s_setprio(kPrioMatrix);
-        v4f acc[3][4];
+        auto const tile = [&](auto starts) __attribute__((always_inline)) {
+            constexpr bool STARTS = decltype(starts)::value;
+            __builtin_amdgcn_s_setprio(kPrioMatrix);
+            v4f acc[3][4];
 #pragma unroll
-        for (int p = 0; p < 3; ++p) {
+            for (int p = 0; p < 3; ++p) {
 #pragma unroll
-            for (int b = 0; b < 4; ++b) acc[p][b] = zero;
-            if (p >= PLANES) continue;
+                for (int b = 0; b < 4; ++b) acc[p][b] = STARTS ? o.bias : zero;
+                if (p >= PLANES) continue;
 #pragma unroll
-            for (int kb = 0; kb < NK32; ++kb) {
-                if (HAS16) mfma32_as_two_16(o.a32[p][kb], B32[kb], acc[p]);
-                else       mfma32(o.a32[p][kb], B32[kb], acc[p]);
+                for (int kb = 0; kb < NK32; ++kb) {
+                    if (HAS16) mfma32_as_two_16(o.a32[p][kb], B32[kb], acc[p]);
+                    else       mfma32(o.a32[p][kb], B32[kb], acc[p]);
+                }
+                if (HAS16) mfma16(o.a16[p], B16, acc[p]);
             }
-            if (HAS16) mfma16(o.a16[p], B16, acc[p]);
-        }
-        __builtin_amdgcn_s_setprio(kPrioEpilogue);
+            __builtin_amdgcn_s_setprio(kPrioEpilogue);
 #pragma unroll
-        for (int b = 0; b < 4; ++b) fp8_epilogue<LAST_HIDDEN, PLANES>(acc[2][b], acc[1][b], acc[0][b], o.bias, H[b][t]);
+            for (int b = 0; b < 4; ++b) fp8_epilogue<LAST_HIDDEN, PLANES, STARTS>(acc[2][b], acc[1][b], acc[0][b], o.bias, H[b][t]);
+        };
+        if (MAY_START && (started & (1 << t))) tile(std::true_type{});       // uniform
+        else                                   tile(std::false_type{});
     }
 }
 
 template <class V, int PLANES>
-__device__ __forceinline__ void fp8_layer0(Fp8Lds<V> const& lds, int lane, uint4 const (&X32)[4], uint2 const (&X16)[4], uint32_t (&H)[4][4][2])
+__device__ __forceinline__ void fp8_layer0(Fp8Lds<V> const& lds, int lane, int started, uint4 const (&X32)[4], uint2 const (&X16)[4], uint32_t (&H)[4][4][2])
 {
     int const g = lane >> 4;
     uint4 B32[1][4];
 #pragma unroll
     for (int b = 0; b < 4; ++b) B32[0][b] = X32[b];
-    fp8_hidden_layer<PLANES, V::T0, 1, true, false>([&](int t, TileOperands<1, true>& o) {
+    fp8_hidden_layer<PLANES, V::ONE, V::T0, 1, true, false>([&](int t, TileOperands<1, true>& o) {
 #pragma unroll
         for (int p = 0; p < PLANES; ++p) {
             o.a32[p][0] = lds.w0[p][t][lane];
             o.a16[p] = reinterpret_cast<uint2 const*>(&lds.w0[p][t][64])[lane];
         }
         o.bias = *reinterpret_cast<v4f const*>(&lds.bias[t][g][0]);
-    }, B32, X16, H);
+    }, started, B32, X16, H);
 }
 
 template <class V, int PLANES>
-__device__ __forceinline__ void fp8_layer1(Fp8Lds<V> const& lds, int lane, uint32_t const (&Hin)[4][4][2], uint32_t (&H)[4][4][2])
+__device__ __forceinline__ void fp8_layer1(Fp8Lds<V> const& lds, int lane, int started, uint32_t const (&Hin)[4][4][2], uint32_t (&H)[4][4][2])
 {
     int const g = lane >> 4;
     uint4 B32[2][4];
@@ -640,19 +661,19 @@ __device__ __forceinline__ void fp8_layer1(Fp8Lds<V> const& lds, int lane, uint3
         B32[1][b] = make_uint4(Hin[b][2][0], Hin[b][2][1], Hin[b][3][0], Hin[b][3][1]);
         B16[b] = make_uint2(0u, 0u);
     }
-    fp8_hidden_layer<PLANES, V::T1, 2, false, false>([&](int t, TileOperands<2, false>& o) {
+    fp8_hidden_layer<PLANES, V::ONE, V::T1, 2, false, false>([&](int t, TileOperands<2, false>& o) {
 #pragma unroll
         for (int p = 0; p < PLANES; ++p) {
             o.a32[p][0] = lds.w1[p][t][lane];
             o.a32[p][1] = lds.w1[p][t][64 + lane];
         }
         o.bias = *reinterpret_cast<v4f const*>(&lds.bias[V::T0 + t][g][0]);
-    }, B32, B16, H);
+    }, started >> V::T0, B32, B16, H);
 }
 
 // layer 2: its activations are quantised to the int8 inputs of the output layer
 template <class V, int PLANES>
-__device__ __forceinline__ void fp8_layer2(Fp8Lds<V> const& lds, int lane, uint32_t const (&Hin)[4][4][2], uint32_t (&H)[4][4][2])
+__device__ __forceinline__ void fp8_layer2(Fp8Lds<V> const& lds, int lane, int started, uint32_t const (&Hin)[4][4][2], uint32_t (&H)[4][4][2])
 {
     int const g = lane >> 4;
     uint4 B32[1][4];
@@ -662,14 +683,14 @@ __device__ __forceinline__ void fp8_layer2(Fp8Lds<V> const& lds, int lane, uint3
         B32[0][b] = make_uint4(Hin[b][0][0], Hin[b][0][1], Hin[b][1][0], Hin[b][1][1]);
         B16[b] = make_uint2(Hin[b][2][0], Hin[b][2][1]);
     }
-    fp8_hidden_layer<PLANES, V::T2, 1, true, true>([&](int t, TileOperands<1, true>& o) {
+    fp8_hidden_layer<PLANES, V::ONE, V::T2, 1, true, true>([&](int t, TileOperands<1, true>& o) {
 #pragma unroll
         for (int p = 0; p < PLANES; ++p) {
             o.a32[p][0] = lds.w2[p][t][lane];
             o.a16[p] = reinterpret_cast<uint2 const*>(&lds.w2[p][t][64])[lane];
         }
         o.bias = *reinterpret_cast<v4f const*>(&lds.bias[V::T0 + V::T1 + t][g][0]);
-    }, B32, B16, H);
+    }, started >> (V::T0 + V::T1), B32, B16, H);
 }
 
 // The FP8 network for the 64 texels of one wave.  `in` is the lane's own texel; `modes` (uniform) holds the hidden
@@ -698,22 +719,23 @@ __device__ __forceinline__ void mlp_forward_fp8(Fp8Lds<V>& lds, int wave, int la
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
 
+    int const started = modes >> kFp8StartShift;             // uniform: tiles whose sums start at the bias
     uint32_t Ha[4][4][2], Hb[4][4][2];                       // [texel block][tile of 16 channels][2 dwords = 4 halves]
     if constexpr (V::ONE) {
-        fp8_layer0<V, 1>(lds, lane, X32, X16, Ha);                                                                 // 48 -> 64
-        fp8_layer1<V, 1>(lds, lane, Ha, Hb);                                                                       // 64 -> 48
-        fp8_layer2<V, 1>(lds, lane, Hb, Ha);                                                                       // 48 -> 32
+        fp8_layer0<V, 1>(lds, lane, started, X32, X16, Ha);                                                                 // 48 -> 64
+        fp8_layer1<V, 1>(lds, lane, started, Ha, Hb);                                                                       // 64 -> 48
+        fp8_layer2<V, 1>(lds, lane, started, Hb, Ha);                                                                       // 48 -> 32
     } else {
         int const one = modes >> kOnePlaneShift;
-        if (one & 1)        fp8_layer0<V, 1>(lds, lane, X32, X16, Ha);
-        else if (modes & 1) fp8_layer0<V, 3>(lds, lane, X32, X16, Ha);
-        else                fp8_layer0<V, 2>(lds, lane, X32, X16, Ha);
-        if (one & 2)        fp8_layer1<V, 1>(lds, lane, Ha, Hb);
-        else if (modes & 2) fp8_layer1<V, 3>(lds, lane, Ha, Hb);
-        else                fp8_layer1<V, 2>(lds, lane, Ha, Hb);
-        if (one & 4)        fp8_layer2<V, 1>(lds, lane, Hb, Ha);
-        else if (modes & 4) fp8_layer2<V, 3>(lds, lane, Hb, Ha);
-        else                fp8_layer2<V, 2>(lds, lane, Hb, Ha);
+        if (one & 1)        fp8_layer0<V, 1>(lds, lane, started, X32, X16, Ha);
+        else if (modes & 1) fp8_layer0<V, 3>(lds, lane, started, X32, X16, Ha);
+        else                fp8_layer0<V, 2>(lds, lane, started, X32, X16, Ha);
+        if (one & 2)        fp8_layer1<V, 1>(lds, lane, started, Ha, Hb);
+        else if (modes & 2) fp8_layer1<V, 3>(lds, lane, started, Ha, Hb);
+        else                fp8_layer1<V, 2>(lds, lane, started, Ha, Hb);
+        if (one & 4)        fp8_layer2<V, 1>(lds, lane, started, Hb, Ha);
+        else if (modes & 4) fp8_layer2<V, 3>(lds, lane, started, Hb, Ha);
+        else                fp8_layer2<V, 2>(lds, lane, started, Hb, Ha);
     }
     // output layer: 32 -> 16, exact: |sum W q| <= 32 * 127 * 128 < 2^24
     {

@@ -395,6 +395,47 @@ def test_gpu_fp8_output_sums_from_the_bias(ntc, device, bias, form):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("layer", [0, 1, 2])
+@pytest.mark.parametrize("form", ["unit", "fine", "below", "limit", "beyond", "zeros", "mixed"])
+def test_gpu_fp8_hidden_sums_from_the_bias(ntc, device, layer, form):
+    """Tiles of 16 channels whose sums start at the bias, and those that add it last.  A channel's sums, bias included, are
+    less than 2^24 units of 2^-18 or of the finest unit that leaves room; the bias is a multiple of it, or one step of a half
+    below it; the sums of the weights alone are at the one-plane limit, where the smallest bias is too much; only one
+    channel of the layer is such.  The launch is large enough for the one-plane instantiation."""
+    spec = ntc.presets.spec_ref092_fp8(16)
+    layout = ntc.synth.weight_layout(spec)
+    n_in, n_out = spec.layer_inputs(layer), spec.layer_outputs(layer)
+    case = fp8_case(ntc, 16, 1024, 520, 1, 2, 16, ntc.abi.OUT_FP16_PLANAR_PAIRS, seed=410 + layer, bias_sigma=0.5)
+    at = layout.weightOffset[layer]
+    w = case.weights[at:at + n_in * n_out].reshape(n_out, n_in)
+    bias = case.weights[layout.biasOffset[layer]:layout.biasOffset[layer] + 2 * n_out].view(np.uint16).view(np.float16)
+    signs = np.where(np.arange(n_out) % 2 == 0, 1.0, -1.0)
+    if form == "unit":                                       # 5462 to 10922 times 1536 units: no finer unit
+        w[:, 0] = np.where(signs > 0, 0x50, 0xd0)            # 8 = 4096 / 512
+        bias[:] = signs * 2.0 ** -18 * (1 + np.arange(n_out) * 37 % 1024)
+    elif form == "fine":                                     # sums of 2^-9 alone: biases down to the last bit of a half
+        w[:] = np.where(np.arange(n_in) % 3 == 0, 0x01, 0x81)
+        bias[:] = signs * 2.0 ** -24 * (1 + np.arange(n_out) * 61 % 1024)
+    elif form == "below":
+        w[:, 0] = np.where(signs > 0, 0x50, 0xd0)
+        bias[:] = signs * (2.0 ** -9 + 2.0 ** -19 + 2.0 ** -18 * (np.arange(n_out) * 5 % 16))
+    elif form in ("limit", "beyond"):                        # 10922 = 8192 + 2048 + 512 + 128 + 32 + 8 + 2 units of 2^-9: 256 units of 2^-18 are left
+        w[:] = 0
+        for k, byte in enumerate((0x58, 0x48, 0x38, 0x28, 0x18, 0x08, 0x02)):
+            w[:, k] = byte
+        bias[:] = signs * (255.0 if form == "limit" else 256.0) * 2.0 ** -18
+        if form == "beyond":
+            bias[:] = signs * 60.0
+    elif form == "zeros":                                    # weights and biases of either zero
+        w[:] = np.where(np.arange(n_in) % 2 == 0, 0x00, 0x80)
+        bias[:] = signs * 0.0
+    else:
+        bias[:] = np.where(np.arange(n_out) == n_out - 3, 2.0 ** -24, signs * 0.25)
+    expected, got = run_both(device, case)
+    assert first_mismatch(expected, got) is None, (layer, form)
+
+
+@pytest.mark.gpu
 def test_gpu_fp8_level_of_detail_input_up_to_three(ntc, device):
     """The exactness of the layer sums is proven for inputs of at most 3 in magnitude.  Features and positional
     encoding lie in [-1, 1]; the level-of-detail input comes from the caller's descriptor: +-3 decodes to the
