@@ -208,9 +208,10 @@ BC6_INLINE float exp1(float c) { return exp2_of_log(c) - 1.f; }
 // Four waves encode 64 blocks, whose texels lie in LDS; the lanes of a wave are blocks.
 //   1. one wave: the one-subset endpoints; then all: bounds of the patterns' scores, patterns taken in turn, and the
 //      scores of those that the bounds leave;
-//   2. a wave per subset of each block's pattern: its endpoints;
-//   3. each wave four of the sixteen texels: indices and estimates of the errors of all three candidates, and the errors
-//      as they are defined where the estimates are too close to tell;
+//   2. a wave per subset of each block's pattern: its endpoints; beside them the other two waves, eight texels each: the
+//      one-subset candidate's indices and the estimate of its error;
+//   3. each wave four of the sixteen texels: the same for the two-subset candidates, and the errors as they are defined
+//      where the estimates are too close to tell;
 //   4. one wave: the block.
 // Bound by the issue of vector instructions and by waves that wait for the one that works alone: 68 % of the slots with four
 // workgroups on a compute unit.  31.5 KB of LDS (what one part leaves, the next one overwrites) and 96 registers let five be
@@ -221,7 +222,9 @@ BC6_INLINE float exp1(float c) { return exp2_of_log(c) - 1.f; }
 // small images waited for the chain of one lane's scores, large ones for its spills and longer divisions.  Shared by the
 // waves: 30, 61 and 204 (195 beside other kernels), of which the 32 scores, 625 instructions each, were more than half;
 // with their bounds first 165 beside others, 29, 47 and 147 alone; with estimated errors (the logarithms were 13 % of the
-// instructions) and five workgroups 27, 42 and 126, 4096 x 4096 520 -> 417.
+// instructions) and five workgroups 26.6, 42 and 124, 4096 x 4096 520 -> 417; with the one-subset errors beside the subsets'
+// endpoints 25.7, 41 and 123.  (Bounds from offsets to the block's corner, with the smaller subset's sums only: 8 % fewer
+// instructions and no time, because what goes issues two at a time and the minima and maxima that stay do not.)
 struct Bc6Lds {
     float4 texels[16][64];
     float one[11][64];                                       // one subset: lo, hi, direction, codes of the ends along it

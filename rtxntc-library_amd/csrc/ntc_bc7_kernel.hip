@@ -1728,7 +1728,8 @@ bc7_compress_kernel(BlockCompressArgs a)
 // code).  Sorting 256 blocks among as many threads left each wave with three or four modes: 2048 x 2048 blocks, modes 4 and
 // 5 on five blocks of six, took 86 us, with every block in one mode 27 to 50; 50 us from lists of 1024 blocks, with a wave's
 // pixels loaded one after the other for a third of the time; 38.5 with all of them under way and the map's words loaded and
-// counted at once.  Images of no more than 256 blocks per compute unit sort 256 (1024 x 1024: 71 us before, 31, and 23.5).
+// counted at once; 34.0 with indices packed two and three bits at a time as they are made.  Images of no more than 256 blocks
+// per compute unit sort 256 (1024 x 1024: 71 us before, 31, 23.5, and 21.3; 128 x 128 22.3 -> 20.4 by the packing).
 // What is left is 19 pieces for 12 waves, unequal ones.  Which lane encodes which block depends on the order the LDS counters
 // are hit in; what is written for a block does not.
 // Three waves per SIMD (168 registers) serve this kernel best.
