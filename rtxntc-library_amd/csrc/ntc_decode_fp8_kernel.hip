@@ -540,12 +540,13 @@ __device__ __forceinline__ void fp8_epilogue(v4f s2, v4f s1, v4f s0, v4f bias, u
     }
 }
 
-// acc[b] += A(block of 32 inputs) * X for the four 16-texel blocks of the wave.
-__device__ __forceinline__ void mfma32(uint4 const& a, uint4 const (&x)[4], v4f (&acc)[4])
+// acc[b] += A(block of 32 inputs) * X for the 16-texel blocks of the wave: four, or one where a launch has few tiles.
+template <int B>
+__device__ __forceinline__ void mfma32(uint4 const& a, uint4 const (&x)[B], v4f (&acc)[B])
 {
     v8h const A = __builtin_bit_cast(v8h, a);
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, __builtin_bit_cast(v8h, x[b]), acc[b], 0, 0, 0);
+    for (int b = 0; b < B; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, __builtin_bit_cast(v8h, x[b]), acc[b], 0, 0, 0);
 }
 // The same for a block of 16 inputs.  32-deep and 16-deep instructions are never mixed in one accumulator's
 // chain: in either order that gave wrong sums here with some instruction schedules (the wait between the two
@@ -555,17 +556,19 @@ __device__ __forceinline__ void mfma32(uint4 const& a, uint4 const (&x)[4], v4f 
 // last four halves are two valid 16-deep operands.  (The other way round - the block of 16 padded with zero
 // weights to a 32-deep instruction, 148 instead of 196 matrix instructions per wave tile - measured 1.5 % slower:
 // two 16-deep instructions cost this kernel no more than one 32-deep one.)
-__device__ __forceinline__ void mfma16(uint2 const& a, uint2 const (&x)[4], v4f (&acc)[4])
+template <int B>
+__device__ __forceinline__ void mfma16(uint2 const& a, uint2 const (&x)[B], v4f (&acc)[B])
 {
     v4h const A = __builtin_bit_cast(v4h, a);
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x16f16(A, __builtin_bit_cast(v4h, x[b]), acc[b], 0, 0, 0);
+    for (int b = 0; b < B; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x16f16(A, __builtin_bit_cast(v4h, x[b]), acc[b], 0, 0, 0);
 }
-__device__ __forceinline__ void mfma32_as_two_16(uint4 const& a, uint4 const (&x)[4], v4f (&acc)[4])
+template <int B>
+__device__ __forceinline__ void mfma32_as_two_16(uint4 const& a, uint4 const (&x)[B], v4f (&acc)[B])
 {
-    uint2 lo[4], hi[4];
+    uint2 lo[B], hi[B];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) { lo[b] = make_uint2(x[b].x, x[b].y); hi[b] = make_uint2(x[b].z, x[b].w); }
+    for (int b = 0; b < B; ++b) { lo[b] = make_uint2(x[b].x, x[b].y); hi[b] = make_uint2(x[b].z, x[b].w); }
     mfma16(make_uint2(a.x, a.y), lo, acc);
     mfma16(make_uint2(a.z, a.w), hi, acc);
 }
@@ -586,8 +589,8 @@ struct TileOperands { uint4 a32[3][NK32]; uint2 a16[3]; v4f bias; };     // one 
 // One hidden layer: TILES output tiles of 16 channels; its inputs as NK32 blocks of 32 (B32[kb][b]) and, with
 // HAS16, one block of 16 (B16[b]); load(t, operands) reads tile t's weight operands and bias.  A layer with a
 // block of 16 runs on 16-deep instructions only (see mfma16).
-template <int PLANES, bool MAY_START, int TILES, int NK32, bool HAS16, bool LAST_HIDDEN, class Load>
-__device__ __forceinline__ void fp8_hidden_layer(Load&& load, int started, uint4 const (&B32)[NK32][4], uint2 const (&B16)[4], uint32_t (&H)[4][4][2])
+template <int PLANES, bool MAY_START, int TILES, int NK32, bool HAS16, bool LAST_HIDDEN, int B, class Load>
+__device__ __forceinline__ void fp8_hidden_layer(Load&& load, int started, uint4 const (&B32)[NK32][B], uint2 const (&B16)[B], uint32_t (&H)[B][4][2])
 {
     v4f const zero = { 0.f, 0.f, 0.f, 0.f };
     // The operands of output tile t + 1 are loaded before the work on tile t (two sets of registers, alternating);
@@ -610,11 +613,11 @@ __device__ __forceinline__ void fp8_hidden_layer(Load&& load, int started, uint4
         auto const tile = [&](auto starts) __attribute__((always_inline)) {
             constexpr bool STARTS = decltype(starts)::value;
             __builtin_amdgcn_s_setprio(kPrioMatrix);
-            v4f acc[3][4];
+            v4f acc[3][B];
 #pragma unroll
             for (int p = 0; p < 3; ++p) {
 #pragma unroll
-                for (int b = 0; b < 4; ++b) acc[p][b] = STARTS ? o.bias : zero;
+                for (int b = 0; b < B; ++b) acc[p][b] = STARTS ? o.bias : zero;
                 if (p >= PLANES) continue;
 #pragma unroll
                 for (int kb = 0; kb < NK32; ++kb) {
@@ -625,20 +628,20 @@ __device__ __forceinline__ void fp8_hidden_layer(Load&& load, int started, uint4
             }
             __builtin_amdgcn_s_setprio(kPrioEpilogue);
 #pragma unroll
-            for (int b = 0; b < 4; ++b) fp8_epilogue<LAST_HIDDEN, PLANES, STARTS>(acc[2][b], acc[1][b], acc[0][b], o.bias, H[b][t]);
+            for (int b = 0; b < B; ++b) fp8_epilogue<LAST_HIDDEN, PLANES, STARTS>(acc[2][b], acc[1][b], acc[0][b], o.bias, H[b][t]);
         };
         if (MAY_START && (started & (1 << t))) tile(std::true_type{});       // uniform
         else                                   tile(std::false_type{});
     }
 }
 
-template <class V, int PLANES>
-__device__ __forceinline__ void fp8_layer0(Fp8Lds<V> const& lds, int lane, int started, uint4 const (&X32)[4], uint2 const (&X16)[4], uint32_t (&H)[4][4][2])
+template <class V, int PLANES, int B>
+__device__ __forceinline__ void fp8_layer0(Fp8Lds<V> const& lds, int lane, int started, uint4 const (&X32)[B], uint2 const (&X16)[B], uint32_t (&H)[B][4][2])
 {
     int const g = lane >> 4;
-    uint4 B32[1][4];
+    uint4 B32[1][B];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) B32[0][b] = X32[b];
+    for (int b = 0; b < B; ++b) B32[0][b] = X32[b];
     fp8_hidden_layer<PLANES, V::ONE, V::T0, 1, true, false>([&](int t, TileOperands<1, true>& o) {
 #pragma unroll
         for (int p = 0; p < PLANES; ++p) {
@@ -649,14 +652,14 @@ __device__ __forceinline__ void fp8_layer0(Fp8Lds<V> const& lds, int lane, int s
     }, started, B32, X16, H);
 }
 
-template <class V, int PLANES>
-__device__ __forceinline__ void fp8_layer1(Fp8Lds<V> const& lds, int lane, int started, uint32_t const (&Hin)[4][4][2], uint32_t (&H)[4][4][2])
+template <class V, int PLANES, int B>
+__device__ __forceinline__ void fp8_layer1(Fp8Lds<V> const& lds, int lane, int started, uint32_t const (&Hin)[B][4][2], uint32_t (&H)[B][4][2])
 {
     int const g = lane >> 4;
-    uint4 B32[2][4];
-    uint2 B16[4];
+    uint4 B32[2][B];
+    uint2 B16[B];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
+    for (int b = 0; b < B; ++b) {
         B32[0][b] = make_uint4(Hin[b][0][0], Hin[b][0][1], Hin[b][1][0], Hin[b][1][1]);
         B32[1][b] = make_uint4(Hin[b][2][0], Hin[b][2][1], Hin[b][3][0], Hin[b][3][1]);
         B16[b] = make_uint2(0u, 0u);
@@ -672,14 +675,14 @@ __device__ __forceinline__ void fp8_layer1(Fp8Lds<V> const& lds, int lane, int s
 }
 
 // layer 2: its activations are quantised to the int8 inputs of the output layer
-template <class V, int PLANES>
-__device__ __forceinline__ void fp8_layer2(Fp8Lds<V> const& lds, int lane, int started, uint32_t const (&Hin)[4][4][2], uint32_t (&H)[4][4][2])
+template <class V, int PLANES, int B>
+__device__ __forceinline__ void fp8_layer2(Fp8Lds<V> const& lds, int lane, int started, uint32_t const (&Hin)[B][4][2], uint32_t (&H)[B][4][2])
 {
     int const g = lane >> 4;
-    uint4 B32[1][4];
-    uint2 B16[4];
+    uint4 B32[1][B];
+    uint2 B16[B];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
+    for (int b = 0; b < B; ++b) {
         B32[0][b] = make_uint4(Hin[b][0][0], Hin[b][0][1], Hin[b][1][0], Hin[b][1][1]);
         B16[b] = make_uint2(Hin[b][2][0], Hin[b][2][1]);
     }
@@ -693,26 +696,26 @@ __device__ __forceinline__ void fp8_layer2(Fp8Lds<V> const& lds, int lane, int s
     }, started >> (V::T0 + V::T1), B32, B16, H);
 }
 
-// The FP8 network for the 64 texels of one wave.  `in` is the lane's own texel; `modes` (uniform) holds the hidden
+// The FP8 network for B blocks of 16 texels of one wave.  `in` is the lane's own texel (B = 1: texel lane % 16); `modes` (uniform) holds the hidden
 // layers' modes as stage_fp8_weights returns them.  On return D[b] holds, for lane (j, g), the int32 accumulators, as floats,
 // of output channels 4g..4g+3 of texel 16b + j, and S their scales.
-template <class V>
-__device__ __forceinline__ void mlp_forward_fp8(Fp8Lds<V>& lds, int wave, int lane, int modes, uint32_t const (&in)[24], v4f (&D)[4], v4f& S)
+template <class V, int B>
+__device__ __forceinline__ void mlp_forward_fp8(Fp8Lds<V>& lds, int wave, int lane, int modes, uint32_t const (&in)[24], v4f (&D)[B], v4f& S)
 {
     int const j = lane & 15, g = lane >> 4;
     // transpose: lane = texel -> lane (j, kg) holds inputs 8kg..8kg+7 (block of 32) and 32+4kg..+3 (block of 16)
     {
-        uint4* dst = reinterpret_cast<uint4*>(&lds.in[wave][lane][0]);
+        uint4* dst = reinterpret_cast<uint4*>(&lds.in[wave][B == 1 ? j : lane][0]);
 #pragma unroll
         for (int q = 0; q < 6; ++q) dst[q] = make_uint4(in[4 * q], in[4 * q + 1], in[4 * q + 2], in[4 * q + 3]);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    uint4 X32[4];
-    uint2 X16[4];
+    uint4 X32[B];
+    uint2 X16[B];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
+    for (int b = 0; b < B; ++b) {
         X32[b] = *reinterpret_cast<uint4 const*>(&lds.in[wave][16 * b + j][4 * g]);
         X16[b] = *reinterpret_cast<uint2 const*>(&lds.in[wave][16 * b + j][16 + 2 * g]);
     }
@@ -720,7 +723,7 @@ __device__ __forceinline__ void mlp_forward_fp8(Fp8Lds<V>& lds, int wave, int la
     __builtin_amdgcn_wave_barrier();
 
     int const started = modes >> kFp8StartShift;             // uniform: tiles whose sums start at the bias
-    uint32_t Ha[4][4][2], Hb[4][4][2];                       // [texel block][tile of 16 channels][2 dwords = 4 halves]
+    uint32_t Ha[B][4][2], Hb[B][4][2];                       // [texel block][tile of 16 channels][2 dwords = 4 halves]
     if constexpr (V::ONE) {
         fp8_layer0<V, 1>(lds, lane, started, X32, X16, Ha);                                                                 // 48 -> 64
         fp8_layer1<V, 1>(lds, lane, started, Ha, Hb);                                                                       // 64 -> 48
@@ -742,9 +745,9 @@ __device__ __forceinline__ void mlp_forward_fp8(Fp8Lds<V>& lds, int wave, int la
         v4f const zero = { 0.f, 0.f, 0.f, 0.f };
         v4i const bias = *reinterpret_cast<v4i const*>(&lds.outBias[g][0]);
         bool const small = (modes & kFp8SmallBias) != 0;     // uniform
-        uint4 x[4];
+        uint4 x[B];
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
+        for (int b = 0; b < B; ++b) {
             x[b] = make_uint4(Ha[b][0][0], Ha[b][0][1], Ha[b][1][0], Ha[b][1][1]);
             D[b] = small ? __builtin_bit_cast(v4f, bias) : zero;
         }
@@ -754,7 +757,7 @@ __device__ __forceinline__ void mlp_forward_fp8(Fp8Lds<V>& lds, int wave, int la
         S = *reinterpret_cast<v4f const*>(&lds.outScale[g][0]);
         if (!small) {
 #pragma unroll
-            for (int b = 0; b < 4; ++b)
+            for (int b = 0; b < B; ++b)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) D[b][r] = float(int(uint32_t(int(D[b][r])) + uint32_t(bias[r])));      // wraps like int32
         }
@@ -855,6 +858,41 @@ decode_fp8_kernel(MipTable table, int numMips, TileShares shares, Fp8Handoff han
         }
         segBegin = segEnd;
     }
+}
+
+// Few tiles: a tile in 2^log2Parts workgroups, 16 / 2^log2Parts of the first waves of each take a block of 16 x 1 texels.  Such
+// a launch takes as long as one wave's tile behind the weights, here with a quarter of the arithmetic, and hardly two waves
+// share a SIMD (128 x 128 9.85 -> 7.8 us, 64 x 64 with its 7 mips 10.4 -> 8.1, 256 x 128 9.95 -> 8.6).
+template <class V>
+__global__ void __launch_bounds__(V::THREADS, 1)
+decode_few_fp8_kernel(MipTable table, int numMips, int log2Parts)
+{
+    DevMip const* const mips = table_entries(table.entries);
+    __shared__ Fp8Lds<V> lds;
+    int const lane = threadIdx.x & 63;
+    int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int const j = lane & 15, g = lane >> 4;
+    int const tile = int(blockIdx.x >> log2Parts), part = int(blockIdx.x) - (tile << log2Parts);
+    DevMip const mip = mips[__builtin_amdgcn_readfirstlane(numMips > 1 ? table_entry_of(mips, numMips, 0, tile) : 0)];
+    RunMip const m(mip);
+    int const modes = __builtin_amdgcn_readfirstlane(stage_fp8_weights<V>(lds, m.full.weights, wave * 64 + lane_id(), 1, 1));
+    __syncthreads();
+    if (wave >= 16 >> log2Parts) return;
+    int const block = (part << (4 - log2Parts)) + wave;
+    int const local = tile - m.full.tileStart, tileY = local / m.full.tilesX, tileX = local - tileY * m.full.tilesX;
+    int const x = tileX * 64 + (block & 3) * 16 + j, y = tileY * 4 + (block >> 2);
+    if (x - j >= m.width || y >= m.height) return;           // uniform
+    uint32_t in[24];                                         // four lanes alike per texel
+    if (m.fast) {
+        Fp8Fetch<V> fetch;
+        fetch_latents_fast<V>(m.full, min(x, m.width - 1), y, fetch);
+        finish_inputs_fast<V>(m.full, lds, min(x, m.width - 1), y, fetch, false, in);
+    } else {
+        prepare_inputs_fp8<V>(m.full, lds, min(x, m.width - 1), y, in);
+    }
+    v4f D[1], S;
+    mlp_forward_fp8<V>(lds, wave, lane, modes, in, D, S);
+    store_row_any_format(m, D[0], S, x, y, 4 * g);
 }
 
 // Random-access decode with the FP8 network (NtcSampleTextureSet_CoopVec_FP8, InferenceCoopVec.hlsli:400-440,
@@ -959,11 +997,15 @@ static hipError_t launch_fp8_variant(MipTable const& mips, int numMips, int tota
 {
     using One = Fp8Variant<FEATURES, true>;
     using Any = Fp8Variant<FEATURES, false>;
-    // Up to eight tiles per compute unit one launch of the general instantiation decodes every set: the second launch and
+    // Up to half as many tiles as compute units: quarter or half tiles.  (Beyond, two workgroups would take turns on a
+    // compute unit: the weight planes leave no room for two.)
+    int const units = compute_units_of_current_device(), log2Parts = 4 * totalTiles <= units ? 2 : (2 * totalTiles <= units ? 1 : 0);
+    if (log2Parts) return launch_kernel<decode_few_fp8_kernel<Any>>(dim3(unsigned(totalTiles) << log2Parts), dim3(Any::THREADS), 0, stream, mips, numMips, log2Parts);
+    // Up to eight tiles per compute unit, too, one launch of the general instantiation decodes every set: the second launch and
     // a pass over weights cost more than three waves per SIMD instead of four.  (64 x 64 ... 1024 x 512 with one plane:
-    // 11.0 and 25.1 us in two launches, 9.6 and 24.6 in one; 2048 x 1024: 74.7 and 76.7.  With two planes: 15.3 and 34.0,
+    // 11.0 and 25.1 us in two launches, 9.6 (in whole tiles) and 24.6 in one; 2048 x 1024: 74.7 and 76.7.  With two planes: 15.3 and 34.0,
     // 11.2 and 29.8.)
-    if (totalTiles <= 8 * compute_units_of_current_device())
+    if (totalTiles <= 8 * units)
         return launch_kernel<decode_fp8_kernel<Any>>(dim3(gridSize), dim3(Any::THREADS), 0, stream, mips, numMips, tile_shares(totalTiles, gridSize), Fp8Handoff{ nullptr, 0u });
     hipError_t const e = launch_kernel<decode_fp8_kernel<One>>(dim3(gridSize), dim3(One::THREADS), 0, stream, mips, numMips, tile_shares(totalTiles, gridSize), handoff);
     if (e != hipSuccess) return e;

@@ -436,6 +436,18 @@ def test_gpu_fp8_hidden_sums_from_the_bias(ntc, device, layer, form):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("w,h,mips,fmt", [(1, 1, 1, 0), (17, 5, 3, 1), (64, 4, 1, 2), (1024, 16, 1, 0), (1025, 16, 1, 1), (512, 64, 1, 2), (513, 64, 1, 0), (250, 60, 8, 1), (256, 128, 1, 2)])
+@pytest.mark.parametrize("sigma", [0.1, 1.5, 300.0])
+def test_gpu_fp8_decode_of_few_tiles(ntc, device, w, h, mips, fmt, sigma):
+    """Launches of at most a quarter and half as many tiles as compute units (64 and 128 of 64 x 4 texels here), which deal
+    a tile to four and two workgroups, and of a few more, ragged ones among them; on one, two and three weight planes."""
+    formats = (ntc.abi.OUT_FP16_PLANAR_PAIRS, ntc.abi.OUT_FP16_PIXELS, ntc.abi.OUT_UNORM8_PIXELS)
+    case = fp8_case(ntc, 16, w, h, mips, 2, 13, formats[fmt], seed=w + h, weight_sigma=sigma, bias_sigma=0.3)
+    expected, got = run_both(device, case)
+    assert first_mismatch(expected, got) is None, (w, h, mips, fmt, sigma)
+
+
+@pytest.mark.gpu
 def test_gpu_fp8_level_of_detail_input_up_to_three(ntc, device):
     """The exactness of the layer sums is proven for inputs of at most 3 in magnitude.  Features and positional
     encoding lie in [-1, 1]; the level-of-detail input comes from the caller's descriptor: +-3 decodes to the
