@@ -436,7 +436,7 @@ def test_gpu_fp8_hidden_sums_from_the_bias(ntc, device, layer, form):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("w,h,mips,fmt", [(1, 1, 1, 0), (17, 5, 3, 1), (64, 4, 1, 2), (1024, 16, 1, 0), (1025, 16, 1, 1), (512, 64, 1, 2), (513, 64, 1, 0), (250, 60, 8, 1), (256, 128, 1, 2)])
+@pytest.mark.parametrize("w,h,mips,fmt", [(2, 2, 1, 0), (17, 5, 3, 1), (64, 4, 1, 2), (1024, 16, 1, 0), (1025, 16, 1, 1), (512, 64, 1, 2), (513, 64, 1, 0), (250, 60, 8, 1), (256, 128, 1, 2)])
 @pytest.mark.parametrize("sigma", [0.1, 1.5, 300.0])
 def test_gpu_fp8_decode_of_few_tiles(ntc, device, w, h, mips, fmt, sigma):
     """Launches of at most a quarter and half as many tiles as compute units (64 and 128 of 64 x 4 texels here), which deal
