@@ -583,6 +583,15 @@ __device__ __forceinline__ DevQuery load_query(DevQuery const* queries, uint64_t
     return queries[min(q0 + uint64_t(lane), numQueries - 1)];
 }
 
+// Four outputs of a query, zeros where its mip does not exist.
+__device__ __forceinline__ void store_query_outputs(uint16_t* out, v4f F, v4f S, bool valid)
+{
+    uint32_t h01 = to_half2_bits(F[0] * S[0], F[1] * S[1]);
+    uint32_t h23 = to_half2_bits(F[2] * S[2], F[3] * S[3]);
+    if (!valid) { h01 = 0; h23 = 0; }
+    *reinterpret_cast<u32x2*>(out) = u32x2{ h01, h23 };
+}
+
 // The outputs of a whole wave of valid queries, none of which can overflow a half: lane (j, g) holds channels 4g..4g+3 of query
 // q0 + 16b + j.
 template <class ACC>

@@ -895,6 +895,43 @@ decode_few_fp8_kernel(MipTable table, int numMips, int log2Parts)
     store_row_any_format(m, D[0], S, x, y, 4 * g);
 }
 
+// The fields of the mips that queries need, into LDS (threads 0 ... 15).
+__device__ __forceinline__ void load_fp8_query_mips(QueryMip (&qmips)[16], DevMip const* mips, int numMips)
+{
+    if (threadIdx.x < 16) {
+        DevMip const& d = mips[min(int(threadIdx.x), numMips - 1)];
+        QueryMip& q = qmips[threadIdx.x];
+        q.hr = d.hr; q.lr = d.lr;
+        q.hrAxisX = d.hrAxisX; q.hrAxisY = d.hrAxisY; q.lrAxisX = d.lrAxisX; q.lrAxisY = d.lrAxisY;
+        q.hrWidth = d.hrWidth; q.hrHeight = d.hrHeight; q.lrWidth = d.lrWidth; q.lrHeight = d.lrHeight;
+        q.width = d.width; q.height = d.height;
+        q.posMask = d.posMask; q.fast = d.fast; q.positionLod = d.positionLod;
+        q.hrBricks = d.hrBricks; q.lrBricks = d.lrBricks;
+    }
+}
+
+// The input vector of a lane's query.  Returns whether its mip exists (mip 0's inputs otherwise).
+template <class V>
+__device__ __forceinline__ bool prepare_query_inputs_fp8(DevMip const* mips, QueryMip const (&qmips)[16], int numMips, bool bricked, Fp8Lds<V> const& lds,
+                                                         DevQuery const& query, uint32_t (&in)[24])
+{
+    bool const validMip = query.mip >= 0 && query.mip < numMips;
+    QueryMip const& m = qmips[validMip ? query.mip : 0];
+    int x = int(floorf(query.u * float(m.width)));
+    int y = int(floorf(query.v * float(m.height)));
+    x = max(0, min(x, m.width - 1));
+    y = max(0, min(y, m.height - 1));
+    if (__all(m.fast != 0)) {                                // every lane's mip is power-of-two sized
+        Fp8Fetch<V> fetch;
+        if (bricked) fetch_latents_bricked<V>(m, x, y, fetch);
+        else         fetch_latents_fast<V>(m, x, y, fetch);
+        finish_inputs_fast<V>(m, lds, x, y, fetch, bricked, in);
+    } else {
+        prepare_inputs_fp8<V>(mips[validMip ? query.mip : 0], lds, x, y, in);
+    }
+    return validMip;
+}
+
 // Random-access decode with the FP8 network (NtcSampleTextureSet_CoopVec_FP8, InferenceCoopVec.hlsli:400-440,
 // for a list of sample points): query_kernel of ntc_decode_kernel.hip with this file's input stage and network.  Lane = query in the input stage (each lane with its own mip, kept in LDS); one set, hence one
 // weight blob, per launch.  A query whose mip is out of range writes zeros.
@@ -908,16 +945,7 @@ query_fp8_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queri
     if (!V::ONE && !every && *handoff.word != handoff.serial) return;        // the set went to the one-plane launch before this one
     __shared__ Fp8Lds<V> lds;
     __shared__ QueryMip qmips[16];
-    if (threadIdx.x < 16) {
-        DevMip const& d = mips[min(int(threadIdx.x), numMips - 1)];
-        QueryMip& q = qmips[threadIdx.x];
-        q.hr = d.hr; q.lr = d.lr;
-        q.hrAxisX = d.hrAxisX; q.hrAxisY = d.hrAxisY; q.lrAxisX = d.lrAxisX; q.lrAxisY = d.lrAxisY;
-        q.hrWidth = d.hrWidth; q.hrHeight = d.hrHeight; q.lrWidth = d.lrWidth; q.lrHeight = d.lrHeight;
-        q.width = d.width; q.height = d.height;
-        q.posMask = d.posMask; q.fast = d.fast; q.positionLod = d.positionLod;
-        q.hrBricks = d.hrBricks; q.lrBricks = d.lrBricks;
-    }
+    load_fp8_query_mips(qmips, mips, numMips);
     bool const bricked = mips[0].hrBricks != nullptr;          // a set has the query-ordered copy for all of its mips or for none
     int const lane = threadIdx.x & 63;
     int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -936,21 +964,8 @@ query_fp8_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queri
         uint64_t const q0 = block * perBlock + uint64_t(wave) * 64;
         if (q0 >= numQueries || wave >= waves) continue;
         DevQuery const query = load_query(queries, q0, numQueries, lane);
-        bool const validMip = query.mip >= 0 && query.mip < numMips;
-        QueryMip const& m = qmips[validMip ? query.mip : 0];
-        int x = int(floorf(query.u * float(m.width)));
-        int y = int(floorf(query.v * float(m.height)));
-        x = max(0, min(x, m.width - 1));
-        y = max(0, min(y, m.height - 1));
         uint32_t in[24];
-        if (__all(m.fast != 0)) {                                // every lane's mip is power-of-two sized
-            Fp8Fetch<V> fetch;
-            if (bricked) fetch_latents_bricked<V>(m, x, y, fetch);
-            else         fetch_latents_fast<V>(m, x, y, fetch);
-            finish_inputs_fast<V>(m, lds, x, y, fetch, bricked, in);
-        } else {
-            prepare_inputs_fp8<V>(mips[validMip ? query.mip : 0], lds, x, y, in);
-        }
+        bool const validMip = prepare_query_inputs_fp8<V>(mips, qmips, numMips, bricked, lds, query, in);
         v4f D[4], S;
         mlp_forward_fp8<V>(lds, wave, lane, modes, in, D, S);
 
@@ -960,17 +975,36 @@ query_fp8_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queri
             for (int b = 0; b < 4; ++b) {
                 uint64_t const q = q0 + uint64_t(16 * b + j);
                 int const ok = __shfl(validMip ? 1 : 0, 16 * b + j, 64);
-                if (q >= numQueries) continue;
-                uint32_t h01 = to_half2_bits(float(D[b][0]) * S[0], float(D[b][1]) * S[1]);
-                uint32_t h23 = to_half2_bits(float(D[b][2]) * S[2], float(D[b][3]) * S[3]);
-                if (!ok) { h01 = 0; h23 = 0; }
-                *reinterpret_cast<u32x2*>(out + q * 16 + 4 * g) = u32x2{ h01, h23 };
+                if (q < numQueries) store_query_outputs(out + q * 16 + 4 * g, D[b], S, ok != 0);
             }
         };
         // (see decode_fp8_kernel)
         if (V::ONE && (modes & kFp8OutputsBounded) && __all(validMip) && q0 + 64u <= numQueries) store_whole_queries(out, q0, j, g, D, S);
         else                                                                                     store_outputs();
     }
+}
+
+// Few queries: 16 to a wave, as decode_few_fp8_kernel takes texels.
+template <class V>
+__global__ void __launch_bounds__(V::THREADS, 1)
+query_few_fp8_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queries, uint64_t numQueries, uint16_t* __restrict__ out, int waves)
+{
+    DevMip const* const mips = table_entries(table.entries);
+    __shared__ Fp8Lds<V> lds;
+    __shared__ QueryMip qmips[16];
+    load_fp8_query_mips(qmips, mips, numMips);
+    int const lane = threadIdx.x & 63;
+    int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int const j = lane & 15, g = lane >> 4;
+    int const modes = __builtin_amdgcn_readfirstlane(stage_fp8_weights<V>(lds, mips[0].weights, wave * 64 + lane_id(), 1, 1));
+    __syncthreads();
+    uint64_t const q0 = (uint64_t(blockIdx.x) * uint32_t(waves) + uint64_t(wave)) * 16, q = q0 + uint64_t(j);
+    if (wave >= waves || q0 >= numQueries) return;           // uniform
+    uint32_t in[24];                                         // four lanes alike per query
+    bool const valid = prepare_query_inputs_fp8<V>(mips, qmips, numMips, mips[0].hrBricks != nullptr, lds, queries[min(q, numQueries - 1)], in);
+    v4f D[1], S;
+    mlp_forward_fp8<V>(lds, wave, lane, modes, in, D, S);
+    if (q < numQueries) store_query_outputs(out + q * 16 + 4 * g, D[0], S, valid);
 }
 
 // The two fp16 primitives of the activation stage applied to a list of halves (for the tests): out[0..n) the
@@ -1028,16 +1062,23 @@ static hipError_t launch_fp8_query_variant(MipTable const& mips, int numMips, De
 {
     using One = Fp8Variant<FEATURES, true>;
     using Any = Fp8Variant<FEATURES, false>;
+    // Up to 128 queries per compute unit 16 to a wave, four waves or eight of a workgroup at work (4096 queries 10.0 -> 8.2 us,
+    // 16000 10.1 -> 8.4, 32768 10.3 -> 9.5; 40000 with twelve waves 10.4 and 10.4: the inputs are made four times over).
+    uint64_t const units = uint64_t(compute_units_of_current_device());
+    if (numQueries <= 128 * units) {
+        int const waves = numQueries <= 64 * units ? 4 : 8;
+        return launch_kernel<query_few_fp8_kernel<Any>>(dim3(unsigned((numQueries + 16 * waves - 1) / (16 * waves))), dim3(Any::THREADS), 0, stream, mips, numMips, queries, numQueries, out, waves);
+    }
     // As few of a workgroup's waves at work as keep the workgroups within the compute units, four at least: then hardly
-    // two share a SIMD (16000 queries: 16.2 us with all sixteen, 11.3; 100000: 17.4, 13.8).
+    // two share a SIMD (100000 queries: 17.4 us with all sixteen, 13.8).
     int waves = One::WAVES;
     uint64_t grid = uint64_t(gridSize);
-    for (uint64_t const units = uint64_t(compute_units_of_current_device()); waves > 4 && (numQueries + 32 * waves - 1) / (32 * waves) <= units; ) {
+    for (; waves > 4 && (numQueries + 32 * waves - 1) / (32 * waves) <= units; ) {
         waves /= 2;
         grid = (numQueries + 64 * waves - 1) / (64 * waves);
     }
     // one launch, as in launch_fp8_variant (131072 queries: 14.0 us in two launches, 13.1 in one; 262144: 18.9 and 23.2)
-    if (numQueries <= 512 * uint64_t(compute_units_of_current_device()))
+    if (numQueries <= 512 * units)
         return launch_kernel<query_fp8_kernel<Any>>(dim3(unsigned(grid)), dim3(Any::THREADS), 0, stream, mips, numMips, queries, numQueries, out, int(grid),
                                                     waves < Any::WAVES ? waves : Any::WAVES, Fp8Handoff{ nullptr, 0u });
     hipError_t const e = launch_kernel<query_fp8_kernel<One>>(dim3(unsigned(grid)), dim3(One::THREADS), 0, stream, mips, numMips, queries, numQueries, out, int(grid), waves, handoff);

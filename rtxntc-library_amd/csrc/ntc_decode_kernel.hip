@@ -1430,14 +1430,6 @@ __device__ __forceinline__ bool prepare_query_inputs(DevMip const* mips, QueryMi
     return validMip;
 }
 
-__device__ __forceinline__ void store_query_outputs(uint16_t* out, v4f F, v4f S, bool valid)
-{
-    uint32_t h01 = to_half2_bits(F[0] * S[0], F[1] * S[1]);
-    uint32_t h23 = to_half2_bits(F[2] * S[2], F[3] * S[3]);
-    if (!valid) { h01 = 0; h23 = 0; }
-    *reinterpret_cast<u32x2*>(out) = u32x2{ h01, h23 };
-}
-
 // Random-access decode ("inference on sample", NtcSampleTextureSet of Inference.hlsli:282-357):
 // one query = (u, v, mip) -> the 16 outputs of texel (floor(u*W), floor(v*H)) of that mip, clamped to
 // the image, as 16 fp16.  Lane = query in the input stage (each lane carries its own mip, so the

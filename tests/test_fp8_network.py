@@ -603,6 +603,28 @@ def test_checker_fp8_queries_are_its_raster_decode_at_the_texels_hit(ntc, oracle
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [15, 16, 17, 16384, 16385, 32768, 32769, 65537, 131073])
+@pytest.mark.parametrize("sigma", [0.1, 1.5])
+def test_gpu_fp8_queries_by_number(ntc, device, oracle, n, sigma):
+    """The numbers of queries at which a launch takes another form (16 queries a wave up to 64 and 128 per compute unit, 256
+    of them here, then 64 with more and more waves of a workgroup, two launches), one below, at and one beyond."""
+    A = ntc.abi
+    case = fp8_case(ntc, 16, 200 if n % 2 else 256, 256, 8, 2, 16, A.OUT_FP16_PLANAR_PAIRS, seed=n, weight_sigma=sigma)
+    host = case.host_set()
+    q = fp8_queries(np.random.default_rng(n), n, len(case.mips))
+    want = np.zeros((n, 16), dtype=np.uint16)
+    assert oracle.ntc_oracle_decode_queries(host.desc, q.ctypes.data, n, want.ctypes.data, 8) == 0
+    dset = case.device_set(device)
+    d_q = device.upload(q.view(np.uint8))
+    d_out = device.alloc((n + 4) * 32)
+    d_out.fill(0xCD)
+    A.check(device.lib.ntc_hip_decode_queries(dset, d_q.ptr, n, d_out.ptr, d_out.nbytes))
+    device.synchronize()
+    got = d_out.download(np.uint16).reshape(n + 4, 16)
+    assert np.array_equal(got[:n], want) and np.all(got[n:] == 0xCDCD)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("features,size,grid_scale,n,sigma", [(16, 512, 2, 6000, 0.35), (12, 256, 4, 3001, 0.35), (8, 512, 1, 777, 0.35), (4, 256, 2, 1, 0.35),
                                                          (16, 320, 3, 4000, 0.35), (8, 200, 2, 2049, 0.35), (16, 256, 2, 5000, (0.35, 40.0, 300.0))])
 def test_gpu_fp8_queries_match_checker(ntc, device, oracle, features, size, grid_scale, n, sigma):
