@@ -1529,11 +1529,11 @@ bc7_compress_kernel(BlockCompressArgs a)
     __shared__ S shared;
     SearchPtr<S> const lds = (SearchPtr<S>)&shared;
     int const tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // Blocks: 8 x 8 per group, the groups side by side.  The two workgroups of a compute unit come from rows half a grid apart
-    // where all of them are resident; the lower half's are shifted by half a row, so that their blocks are far from each
-    // other in both directions and seldom both of the costlier kind (1024 x 1024, alpha in the right half: 180 -> 171 us).
-    int const column = blockIdx.y >= gridDim.y / 2 ? int((blockIdx.x + gridDim.x / 2) % gridDim.x) : int(blockIdx.x);
-    auto const block_x = [&](int b) { return column * 8 * GROUPS + (b >> 6) * 8 + (b & 7); };
+    // Blocks: 8 x 8 per group, the groups side by side.  (Which blocks share a compute unit where all workgroups are
+    // resident is no rule's to choose: with the lower half's columns turned by half a row 1024 x 1024 with alpha, or texture
+    // beside grey, in the right half took 173 and 207 us for 181 and 235, in two opposite quadrants 183 and 235 for 175 and
+    // 205.  A workgroup's groups half an image apart: 196 and 213, 198 and 215, for kinds then meet in one workgroup.)
+    auto const block_x = [&](int b) { return int(blockIdx.x) * 8 * GROUPS + (b >> 6) * 8 + (b & 7); };
     auto const block_y = [&](int b) { return int(blockIdx.y) * 8 + ((b >> 3) & 7); };
     // the next of the tasks that the waves take in turn
     auto const next_task = [&](int counter) {
