@@ -592,19 +592,26 @@ __device__ __forceinline__ void store_query_outputs(uint16_t* out, v4f F, v4f S,
     *reinterpret_cast<u32x2*>(out) = u32x2{ h01, h23 };
 }
 
-// The outputs of a whole wave of valid queries, none of which can overflow a half: lane (j, g) holds channels 4g..4g+3 of query
-// q0 + 16b + j.
+// The outputs of a whole wave of queries, none of which can overflow a half: lane (j, g) holds channels 4g..4g+3 of query
+// q0 + 16b + j.  valid: the bit of each query whose mip exists; the others' outputs are zeros.  (With one in twenty that does not,
+// so that hardly a wave is without, 65 536 queries of the 0.9.2 network take 7.8 us and 2^22 151; where such waves stored as
+// the last, partial one does, lane by lane and checked, 8.0 and 155.)
 template <class ACC>
-__device__ __forceinline__ void store_whole_queries(uint16_t* out, uint64_t q0, int j, int g, ACC const (&D)[4], v4f S)
+__device__ __forceinline__ void store_whole_queries(uint16_t* out, uint64_t q0, int j, int g, ACC const (&D)[4], v4f S, uint64_t valid)
 {
     GlobalOutPtr const first = uniform_pointer(reinterpret_cast<uint64_t>(out + q0 * 16u));
     uint32_t const own = uint32_t(j) * 32u + uint32_t(g) * 8u;
+    auto const store = [&](auto every) __attribute__((always_inline)) {
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        uint32_t const h01 = to_half2_bits<false>(float(D[b][0]) * S[0], float(D[b][1]) * S[1]);
-        uint32_t const h23 = to_half2_bits<false>(float(D[b][2]) * S[2], float(D[b][3]) * S[3]);
-        *reinterpret_cast<__attribute__((address_space(1))) u32x2*>(first + (own + 512u * uint32_t(b))) = u32x2{ h01, h23 };
-    }
+        for (int b = 0; b < 4; ++b) {
+            uint32_t h01 = to_half2_bits<false>(float(D[b][0]) * S[0], float(D[b][1]) * S[1]);
+            uint32_t h23 = to_half2_bits<false>(float(D[b][2]) * S[2], float(D[b][3]) * S[3]);
+            if (!decltype(every)::value && !((uint32_t(valid >> (16 * b)) >> j) & 1u)) { h01 = 0; h23 = 0; }
+            *reinterpret_cast<__attribute__((address_space(1))) u32x2*>(first + (own + 512u * uint32_t(b))) = u32x2{ h01, h23 };
+        }
+    };
+    if (valid == ~uint64_t(0)) store(std::true_type{});      // uniform
+    else                       store(std::false_type{});
 }
 
 struct QueryMip {

@@ -979,8 +979,8 @@ query_fp8_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queri
             }
         };
         // (see decode_fp8_kernel)
-        if (V::ONE && (modes & kFp8OutputsBounded) && __all(validMip) && q0 + 64u <= numQueries) store_whole_queries(out, q0, j, g, D, S);
-        else                                                                                     store_outputs();
+        if (V::ONE && (modes & kFp8OutputsBounded) && q0 + 64u <= numQueries) store_whole_queries(out, q0, j, g, D, S, __ballot(validMip));
+        else                                                                  store_outputs();
     }
 }
 

@@ -1460,7 +1460,6 @@ query_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queries, 
         if (q0 >= numQueries || wave >= waves) continue;
         uint32_t in[16];
         bool const validMip = prepare_query_inputs<V>(mips, qmips, numMips, bricked, lds, load_query(queries, q0, numQueries, lane), in);
-        bool const whole = __all(validMip) && q0 + 64u <= numQueries;
 
         // lane (j, g) holds channels 4g..4g+3 of query q0 + 16b + j; validity travels by shuffle
         auto store_outputs = [&](int b, v4f Fb, v4f S) __attribute__((always_inline)) {
@@ -1473,8 +1472,8 @@ query_kernel(MipTable table, int numMips, DevQuery const* __restrict__ queries, 
             v4f F[4];
             v4f S;
             mlp_forward_f16<V>(lds, wave, lane, (staged & kL0Magic) != 0, in, F, S);
-            if ((staged & kOutputsBounded) && whole) {                                       // as in decode_kernel
-                store_whole_queries(out, q0, j, g, F, S);
+            if ((staged & kOutputsBounded) && q0 + 64u <= numQueries) {                      // as in decode_kernel
+                store_whole_queries(out, q0, j, g, F, S, __ballot(validMip));
             } else {
 #pragma unroll
                 for (int b = 0; b < 4; ++b) store_outputs(b, F[b], S);

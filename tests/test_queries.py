@@ -165,3 +165,38 @@ def test_gpu_query_counts_around_the_compute_units(ntc, device, oracle, kind):
             device.synchronize()
             got = d_out.download(np.uint16).reshape(most, 16)
             assert np.array_equal(got[:n], want[:n]) and (got[n:] == 0xCDCD).all(), (kind, n, use_bricks)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bounded", [True, False])
+@pytest.mark.parametrize("kind", ["cfg01", "fp8_8"])
+def test_gpu_queries_of_mips_that_do_not_exist_in_every_wave(ntc, device, oracle, kind, bounded):
+    """Whole waves without such a query, with one at each place of a wave, with many and with nothing else, and a partial
+    wave; with outputs that cannot overflow a half and with outputs that may (and with these scales do)."""
+    A, P = ntc.abi, ntc.presets
+    if kind == "cfg01":
+        case = cfg_case(ntc, P.spec_cfg01(), 256, 128, 9, 16, A.OUT_FP16_PLANAR_PAIRS, 71, scale_log2_range=ACTIVE)
+    else:
+        spec = P.spec_ref092_fp8(8)
+        case = ref_case(ntc, spec, 128, 128, 8, 2, 16, A.OUT_FP16_PLANAR_PAIRS, 72, weights=ntc.synth.make_fp8_weights(spec, 73))
+    if not bounded:
+        layout = ntc.synth.weight_layout(case.spec)
+        last = A.MLP_LAYERS - 1
+        case.weights[layout.scaleOffset[last]:layout.scaleOffset[last] + 64].view(np.float32)[:] *= 2.0 ** 14
+    host = case.host_set()
+    n = 520 * device.compute_units + 37                      # beyond the counts that go sixteen to a wave, or to the general network
+    q = make_queries(np.random.default_rng(74), n, len(case.mips), with_edges=False)
+    wave = np.arange(n) // 64
+    lane = np.arange(n) % 64
+    missing = (wave % 4 == 1) & (lane == (wave // 4) % 64) | (wave % 4 == 2) & (np.random.default_rng(75).random(n) < 0.3) | (wave % 16 == 7)
+    q["mip"][missing] = np.where(lane[missing] % 2 == 0, -1 - lane[missing], len(case.mips) + lane[missing])
+    want = oracle_queries(oracle, host, q)
+    assert not want[missing].any() and (np.abs(want.view(np.float16)[~missing].astype(np.float32)).max() > 60000) == (not bounded)
+    dset = case.device_set(device)
+    d_q, d_out = device.upload(q.view(np.uint8)), device.alloc(n * 32 + 64)
+    d_out.fill(0xCD)
+    A.check(device.lib.ntc_hip_decode_queries(dset, d_q.ptr, n, d_out.ptr, d_out.nbytes))
+    device.synchronize()
+    got = d_out.download(np.uint16).reshape(-1, 16)
+    bad = np.nonzero((got[:n] != want).any(axis=1))[0]
+    assert bad.size == 0 and (got[n:] == 0xCDCD).all(), (bad.size, bad[:3])
