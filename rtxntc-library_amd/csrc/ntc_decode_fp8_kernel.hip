@@ -1062,10 +1062,17 @@ static hipError_t launch_fp8_query_variant(MipTable const& mips, int numMips, De
 {
     using One = Fp8Variant<FEATURES, true>;
     using Any = Fp8Variant<FEATURES, false>;
-    // Up to 128 queries per compute unit 16 to a wave, four waves or eight of a workgroup at work (4096 queries 10.0 -> 8.2 us,
-    // 16000 10.1 -> 8.4, 32768 10.3 -> 9.5; 40000 with twelve waves 10.4 and 10.4: the inputs are made four times over).
+    // 16 to a wave, four waves of a workgroup at work up to 64 queries per compute unit, eight up to 128: a wave's network takes
+    // a quarter of the time, but the inputs are made four times over, by as many gathers, and with eight waves they weigh more
+    // than that where features are many and each is gathered by itself (16000 and 32768 queries in us, before / so: from the
+    // query-ordered copy, 16 features 9.7 / 7.8 and 9.8 / 8.9; from the grids, 12 features 10.3 / 8.5 and 10.3 / 10.1, 16 features
+    // 10.7 / 9.1 and 10.7 / 11.3; sizes that are no powers of two, 8 features 9.8 / 8.0 and 9.8 / 9.6, 12 features 10.4 / 8.6 and
+    // 10.5 / 10.7, 16 features 11.0 / 9.4 and 11.1 / 12.0; 40000 with twelve waves 10.4 / 10.4).
     uint64_t const units = uint64_t(compute_units_of_current_device());
-    if (numQueries <= 128 * units) {
+    bool powers = true, ordered = true;                      // (a set's mips all lie in the arguments)
+    for (int k = 0; k < numMips; ++k) { powers = powers && mips.inlined[k].fast; ordered = ordered && mips.inlined[k].hrBricks; }
+    int const mostFeatures = !powers ? 8 : ordered ? 16 : 12;
+    if (numQueries <= (FEATURES <= mostFeatures ? 128 : 64) * units) {
         int const waves = numQueries <= 64 * units ? 4 : 8;
         return launch_kernel<query_few_fp8_kernel<Any>>(dim3(unsigned((numQueries + 16 * waves - 1) / (16 * waves))), dim3(Any::THREADS), 0, stream, mips, numMips, queries, numQueries, out, waves);
     }

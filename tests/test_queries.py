@@ -200,3 +200,31 @@ def test_gpu_queries_of_mips_that_do_not_exist_in_every_wave(ntc, device, oracle
     got = d_out.download(np.uint16).reshape(-1, 16)
     bad = np.nonzero((got[:n] != want).any(axis=1))[0]
     assert bad.size == 0 and (got[n:] == 0xCDCD).all(), (bad.size, bad[:3])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("size", [256, 320])
+@pytest.mark.parametrize("features", [8, 12, 16])
+def test_gpu_fp8_query_counts_where_sixteen_to_a_wave_end(ntc, device, oracle, features, size):
+    """The last counts that go 16 to a wave with four and with eight waves and the first ones beyond, from the query-ordered
+    copy and from the grids, for sizes that are and are no powers of two: where the line lies depends on all of them."""
+    A, P = ntc.abi, ntc.presets
+    spec = P.spec_ref092_fp8(features)
+    case = ref_case(ntc, spec, size, size, 9, 2, 16, A.OUT_FP16_PLANAR_PAIRS, 81, weights=ntc.synth.make_fp8_weights(spec, 82))
+    units = device.compute_units
+    most = 128 * units + 1
+    host = case.host_set()
+    q = make_queries(np.random.default_rng(83), most, len(case.mips))
+    want = oracle_queries(oracle, host, q)
+    dset = case.device_set(device)
+    d_bricks = device.alloc(device.lib.ntc_hip_query_latents_bytes(dset))
+    A.check(device.lib.ntc_hip_build_query_latents(dset, d_bricks.ptr, d_bricks.nbytes))
+    d_q, d_out = device.upload(q.view(np.uint8)), device.alloc(most * 32)
+    for n in (64 * units, 64 * units + 1, 128 * units, most):
+        for use_bricks in (False, True):
+            dset.queryLatents, dset.queryLatentsBytes = (d_bricks.ptr, d_bricks.nbytes) if use_bricks else (None, 0)
+            d_out.fill(0xCD)
+            A.check(device.lib.ntc_hip_decode_queries(dset, d_q.ptr, n, d_out.ptr, d_out.nbytes))
+            device.synchronize()
+            got = d_out.download(np.uint16).reshape(most, 16)
+            assert np.array_equal(got[:n], want[:n]) and (got[n:] == 0xCDCD).all(), (n, use_bricks)
