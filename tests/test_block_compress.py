@@ -252,6 +252,33 @@ def test_gpu_extreme_blocks_of_packed_rows_match_checker(ntc, device, oracle, ch
     assert np.array_equal(d_dst.download().view(np.uint64).reshape(by, pitch // 8), want)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dst_format", [3, 4, 5])
+@pytest.mark.parametrize("w,h", [(256, 64), (2080, 1028)])
+def test_gpu_blocks_that_no_refit_moves_match_checker(ntc, device, oracle, dst_format, w, h):
+    """Blocks with both 0 and 255 and other values near them only, near one of them, or anywhere: the endpoints of the
+    eight-value palette stay, those of the six-value one have no texel between them, one, or many.  (The larger image is
+    beyond those whose colour blocks and alpha blocks are dealt to several waves.)"""
+    rng = np.random.default_rng(w + dst_format)
+    channels = {3: 4, 4: 1, 5: 2}[dst_format]
+    spread = rng.choice([0, 1, 2, 3, 7, 20, 127], size=(h // 4, w // 4, 1, 1, 1))
+    values = rng.integers(0, 128, (h // 4, w // 4, 4, 4, channels)) % (spread + 1)
+    high = rng.random(values.shape) < rng.choice([0.1, 0.5, 0.9], size=(h // 4, w // 4, 1, 1, 1))
+    values = np.where(high, 255 - values, values)
+    values[:, :, 0, 0], values[:, :, 3, 2] = 0, 255
+    image = np.ascontiguousarray(values.transpose(0, 2, 1, 3, 4).reshape(h, w, channels).astype(np.uint8))
+    bx, by, per = w // 4, h // 4, 8 if dst_format == 4 else 16
+    pitch = bx * per
+    want = oracle_bc(ntc, oracle, image, 1, channels, dst_format, bx, by, 0, 0, 0, 0, pitch)
+    d_src, d_dst = device.upload(image.reshape(-1)), device.upload(np.full(by * pitch, 0xEE, dtype=np.uint8))
+    p = ntc.abi.BlockCompress()
+    fill_image(p.src, d_src.ptr, d_src.nbytes, channels, channels * w, w, h, 1, channels)
+    p.widthInBlocks, p.heightInBlocks, p.dstFormat, p.dst, p.dstBytes, p.dstRowPitch = bx, by, dst_format, d_dst.ptr, d_dst.nbytes, pitch
+    device.call("block_compress", p)
+    device.synchronize()
+    assert np.array_equal(d_dst.download().view(np.uint64).reshape(by, pitch // 8), want)
+
+
 def test_unorm_quotient_shortcut_is_exact():
     """The kernels turn UNORM8 / UNORM16 texels into floats with q = k * r, q + fma(-q, d, k) * r (r = 1 / d
     rounded) instead of a division; that is the correctly rounded k / d for every k (exact rationals here)."""
