@@ -774,7 +774,9 @@ bc4_compress_kernel(BlockCompressArgs a)
 //
 // 64 x 64 and 1024 x 1024: BC1 27 and 29 us in one lane before, 15 and 16 split; BC2 19 and 20, 15 and 15; BC3 25 and 33,
 // 15 and 19.  2048 x 2048: BC1 58 before, 51 (two waves per SIMD with everything in registers; 82 with three that spill; 55
-// split), 46.5 with all pixels loaded at once; BC2 38, 34 (47 split), 31.6; BC3 61, 52 (72 split), 40.5 with the alpha search in integers.  Thirds are selected and not divided, and k / 31 is a product.
+// split), 46.5 with all pixels loaded at once; BC2 38, 34 (47 split), 31.6; BC3 61, 52 (72 split), 40.5 with the alpha search in
+// integers, 33 with it behind the colours and nothing spilled (with hard edges in alpha 50 before, 53 and 36).  Thirds are selected
+// and not divided, and k / 31 is a product.
 struct Bc1Exchange { float4 texels[16][64]; uint32_t words[6][64]; uint64_t alpha[64]; uint32_t sixError[64]; };
 struct NoTables {};
 template <int FORMAT> using Bc1Tables = std::conditional_t<FORMAT == 3, Bc4Tables, NoTables>;          // of the alpha search
@@ -906,26 +908,20 @@ bc1_compress_kernel(BlockCompressArgs a)
     Rgba px[16];
     float alpha[16];
     float texels[4][4][4];
-    if constexpr (FORMAT != 3) source_rows<4, 4>(a, a.srcLeft + bx * 4, a.srcTop + by * 4, 0, texels);
+    source_rows<4, 4>(a, a.srcLeft + bx * 4, a.srcTop + by * 4, 0, texels);
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
         float (&c)[4] = texels[t >> 2][t & 3];
-        // (BC3 spills as it is: with all pixels under way 52.8 us instead of 52)
-        if constexpr (FORMAT == 3) source_pixel(a, a.srcLeft + bx * 4 + (t & 3), a.srcTop + by * 4 + (t >> 2), c);
         px[t] = Rgba{ c[0], c[1], c[2], FORMAT == 1 ? c[3] : 1.f };
         alpha[t] = c[3];
     }
     uint64_t* const dst = bc1_place<FORMAT>(a, bx, by);
     if constexpr (FORMAT == 2) dst[0] = bc2_alpha(alpha);
+    uint32_t rows[4];                                        // BC3: alpha is encoded when the colours are done with
     if constexpr (FORMAT == 3) {
-        Bc4Texels texels;
-        uint32_t error8, error6;
 #pragma unroll
         for (int y = 0; y < 4; ++y)
-            texels.rows[y] = bc4_value(alpha[4 * y]) | bc4_value(alpha[4 * y + 1]) << 8 | bc4_value(alpha[4 * y + 2]) << 16 | bc4_value(alpha[4 * y + 3]) << 24;
-        bc4_prepare(texels);
-        Bc4 const block8 = bc4_candidate<true>(texels, tables, error8), block6 = bc4_candidate<false>(texels, tables, error6);
-        dst[0] = error6 < error8 ? bc4_bits<false>(block6) : bc4_bits<true>(block8);
+            rows[y] = bc4_value(alpha[4 * y]) | bc4_value(alpha[4 * y + 1]) << 8 | bc4_value(alpha[4 * y + 2]) << 16 | bc4_value(alpha[4 * y + 3]) << 24;
     }
     ColorBlock best = bc1_simple_candidates<FORMAT == 1>(px, a.alphaThreshold);
     ColorBlock const four = bc1_four_colors<FORMAT != 1>(px);
@@ -935,6 +931,15 @@ bc1_compress_kernel(BlockCompressArgs a)
         if (three.error < best.error) best = three;
     }
     dst[FORMAT == 1 ? 0 : 1] = uint64_t(best.endpoints) | (uint64_t(best.indices) << 32);
+    if constexpr (FORMAT == 3) {
+        Bc4Texels texels;
+        uint32_t error8, error6;
+#pragma unroll
+        for (int y = 0; y < 4; ++y) texels.rows[y] = rows[y];
+        bc4_prepare(texels);
+        Bc4 const block8 = bc4_candidate<true>(texels, tables, error8), block6 = bc4_candidate<false>(texels, tables, error6);
+        dst[0] = error6 < error8 ? bc4_bits<false>(block6) : bc4_bits<true>(block8);
+    }
 }
 
 template <int FORMAT>
