@@ -506,6 +506,7 @@ BC7_INLINE void store_block(BlockCompressArgs const& a, int bx, int by, uint64_t
 //      the smallest bound and queues those whose bounds do not exceed it: one to seven of 64 on textures with detail.
 //      Beside them a task for each group: lower bounds of the errors of the four channel rotations of modes 4 and 5 and of
 //      mode 6, then the three forms of the rotation with the smallest one, whose error leaves out what is bounded above it.
+//      (Or, where it is the chain that counts, a task for each rotation and one for mode 6: see all_by_bounds.)
 //   2. Tasks of 64 queued estimates, from any blocks of a search; tasks of 64 rotations or of 64 blocks of mode 6 that were
 //      not left out; tasks of one candidate, from its endpoints to the encoded block, where every lane has a partition of
 //      its own and walks its own list of texels.
@@ -540,6 +541,13 @@ enum : uint32_t { kBelowOne = 1, kNotOne = 2 };              // what some alpha 
 // The searches of a workgroup: its opaque groups' partitions of two subsets, then of three, then the partitions for mode 7
 // of all groups, the opaque ones first.  (128 blocks are two groups of one kind, or three of both.)
 enum { kSearches = 7, kQueued = 14 * 64, kWholeChunk = 8 };
+// Of 128 blocks, candidates take the bounds' place when the picks are made; of 64, whose workgroup has a compute unit to itself,
+// they have one of their own and some are made beside the bounds.
+template <int BLOCKS> struct SearchBounds { uint32_t codes[kPicks][16][BLOCKS]; };         // of four partitions each
+template <int BLOCKS> struct SearchCandidates { uint4 words[kSlots][BLOCKS]; float errors[kSlots][BLOCKS]; };
+template <int BLOCKS> struct SearchScratch { union { SearchBounds<BLOCKS> bounds; SearchCandidates<BLOCKS> late; }; };
+template <> struct SearchScratch<64> { SearchBounds<64> bounds; SearchCandidates<64> late; };
+
 template <int BLOCKS_>
 struct SearchLds {
     static constexpr int BLOCKS = BLOCKS_;
@@ -547,10 +555,7 @@ struct SearchLds {
     uint64_t picks[kPicks][BLOCKS];                          // error bits << 32 | partition
     float scale[kPicks][BLOCKS];                             // of errors before they become codes; 0: the block has no bounds
     uint32_t lowest[kPicks][BLOCKS];                         // the smallest bound's bits, the low six replaced by its partition
-    union {
-        uint32_t bounds[kPicks][16][BLOCKS];                 // codes of four partitions each; until the picks are made
-        struct { uint4 words[kSlots][BLOCKS]; float errors[kSlots][BLOCKS]; } late;
-    };
+    SearchScratch<BLOCKS> scratch;
     struct { uint4 words[BLOCKS]; float errors[BLOCKS]; } early;                   // the first rotation's candidate (before: least errors of all four)
     uint32_t plans[BLOCKS];                                  // the first rotation; kKeepRotation << r and kKeepSix
     uint16_t flatRotations[2 * BLOCKS], rotations[3 * BLOCKS];                     // those kept, rotation << 7 | block: with planes of two channels, of three
@@ -855,8 +860,8 @@ BC7_TASK void bound_task(SearchPtr<S> lds, int b, int first, int last)
         if constexpr (ORIENTED) consider(oriented, lowestOriented, codesOriented);
         if constexpr (PLAIN) consider(plain, lowestPlain, codesPlain);
         if ((p & 3) == 3) {
-            if constexpr (ORIENTED) lds->bounds[kind][p >> 2][b] = codesOriented;
-            if constexpr (PLAIN) lds->bounds[kPickTwoAlpha][p >> 2][b] = codesPlain;
+            if constexpr (ORIENTED) lds->scratch.bounds.codes[kind][p >> 2][b] = codesOriented;
+            if constexpr (PLAIN) lds->scratch.bounds.codes[kPickTwoAlpha][p >> 2][b] = codesPlain;
         }
     }
     if constexpr (ORIENTED) __hip_atomic_fetch_min(&lds->lowest[kind][b], lowestOriented, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -1024,7 +1029,7 @@ BC7_TASK void select_task(SearchPtr<S> lds, int b, int what, int search, int min
         uint32_t const bits = uint32_t(pick >> 32), code = error_code(__uint_as_float(bits), lds->scale[kind][b]);
 #pragma unroll 4
         for (int j = 0; j < 16; ++j) {
-            uint32_t const codes = lds->bounds[kind][j][b];
+            uint32_t const codes = lds->scratch.bounds.codes[kind][j][b];
             uint32_t four = 0;
 #pragma unroll
             for (int i = 0; i < 4; ++i) four |= ((codes >> (8 * i)) & 0xffu) <= code ? 1u << i : 0u;
@@ -1220,7 +1225,7 @@ BC7_TASK void finish_task(SearchPtr<S> lds, int b, int pick, int slot)
         partition = none ? 0 : int(uint32_t(key));
     }
     if (partition >= (1 << M::partitionBits)) {              // mode 0 has sixteen partitions only
-        lds->late.errors[slot][b] = __uint_as_float(0x7f800000u);    // never taken
+        lds->scratch.late.errors[slot][b] = __uint_as_float(0x7f800000u);    // never taken
         return;
     }
     uint32_t const word = partition_word<M::subsets>(partition);
@@ -1284,7 +1289,7 @@ BC7_TASK void finish_task(SearchPtr<S> lds, int b, int pick, int slot)
     }
     indices = without_bit(indices, top);
     put_indices(bits.lo, bits.hi, bits.at, indices);
-    put_candidate(&lds->late.words[slot][b], &lds->late.errors[slot][b], error, bits.lo, bits.hi);
+    put_candidate(&lds->scratch.late.words[slot][b], &lds->scratch.late.errors[slot][b], error, bits.lo, bits.hi);
 }
 
 // The colour plane and the scalar plane of a texel under the lane's channel rotation.  C = 2: every alpha of the lane's
@@ -1524,6 +1529,7 @@ bc7_compress_kernel(BlockCompressArgs a)
 {
     // (a task of bounds sums the block first: as many partitions in one as leave a task for each wave)
     constexpr int BLOCKS = 64 * GROUPS, THREADS = 64 * WAVES, CHUNK = GROUPS == 1 ? 8 : 16, CHUNKS = 64 / CHUNK;
+    constexpr bool ALONE = GROUPS == 1;                      // on its compute unit
     static_assert(THREADS >= 4 * BLOCKS && BLOCKS <= 128, "a thread per row of a block at least; seven bits number a block");
     using S = SearchLds<BLOCKS>;
     __shared__ S shared;
@@ -1604,16 +1610,49 @@ bc7_compress_kernel(BlockCompressArgs a)
     // ---- 1. bounds of the partitions' errors; one rotation of modes 4 and 5 for each block; the errors of the first partitions
     __builtin_amdgcn_s_setprio(3);
     int const searches = 2 * opaqueGroups + groups, boundTasks = (2 * opaqueGroups + alphaGroups) * CHUNKS;
-    for (int taken = next_task(0); taken < groups + boundTasks + searches; taken = next_task(0)) {
-        int const task = taken < boundTasks ? taken : taken < boundTasks + groups ? taken - boundTasks - groups : taken - groups;
-        if (task < 0) {
-            int const group = task + groups, b = block_of_group(group);
-            bound_rotations<S>(lds, b);
-            int const first = first_rotation<S>(lds, b);
-            Best const best = all_ones(b) ? dual_planes<S, 2>(lds, b, first) : dual_planes<S, 3>(lds, b, first);
-            keep_candidates<S>(lds, b, first, best.error, own_lane(group));
-            put_candidate(&lds->early.words[b], &lds->early.errors[b], best.error, best.lo, best.hi);
-            add_one(shared.rotated);
+    auto const rotate_first = [&](int group) {
+        int const b = block_of_group(group);
+        bound_rotations<S>(lds, b);
+        int const first = first_rotation<S>(lds, b);
+        Best const best = all_ones(b) ? dual_planes<S, 2>(lds, b, first) : dual_planes<S, 3>(lds, b, first);
+        keep_candidates<S>(lds, b, first, best.error, own_lane(group));
+        put_candidate(&lds->early.words[b], &lds->early.errors[b], best.error, best.lo, best.hi);
+        add_one(shared.rotated);
+    };
+    // Whether rotations and mode 6 are left out by their bounds for blocks with alpha, too.  A workgroup with a compute unit to
+    // itself takes as long as its chains; few blocks with alpha have more to do than mode 7's search, and one rotation after
+    // the other was the longer chain (256 x 256 of alpha, smooth 47.0 us with all at once behind the bounds, 61.3 by bounds, 43.0
+    // with all at once beside them, behind the selections in the list and in priority; flat 44.5, 54.6, 36.7; with an opaque
+    // background 83.5, 86.0, 81.3).  But where it has opaque blocks near lines, too, all of whose partitions it estimates, it is
+    // the work that counts: grey 95, 92.6, and 98.  (Opaque blocks, bounds / all at once: flat 65 / 61, detail 74 / 76, grey 75 / 77.)
+    auto const all_by_bounds = [&] {
+        if (!ALONE) return true;
+        if (opaqueGroups == 0) return false;
+        int const b = block_of(0, 0);
+        wait_for(shared.bounded[0], CHUNKS);
+        return __any(lds->scale[kPickTwo][b] != 0.f) && !__any(lds->lowest[kPickTwo][b] != ~0u);
+    };
+    int const early = ALONE ? opaqueGroups : groups, late = ALONE ? 5 * alphaGroups : 0;       // tasks before the selections and after them
+    for (int taken = next_task(0); taken < boundTasks + early + searches + late; taken = next_task(0)) {
+        int const task = taken < boundTasks ? taken : taken < boundTasks + early ? taken - boundTasks - early : taken - early;
+        if (ALONE && task >= boundTasks + searches) {
+            int const nth = task - boundTasks - searches, rotation = nth / alphaGroups, group = nth % alphaGroups, b = block_of(1, group);
+            if (all_by_bounds()) {
+                if (rotation == 0) rotate_first(opaqueGroups + group);
+                continue;
+            }
+            __builtin_amdgcn_s_setprio(0);
+            if (rotation == 4) { finish_task<S, Mode6, 4, true>(lds, b, 0, kSlotSix); continue; }
+            Best const best = dual_planes<S, 3>(lds, b, rotation);
+            if (rotation == 0) {
+                lds->plans[b] = 7u * (kKeepRotation << 1) | kKeepSix;
+                put_candidate(&lds->early.words[b], &lds->early.errors[b], best.error, best.lo, best.hi);
+            } else {
+                int const slot = kSlotRotations + rotation - 1;
+                put_candidate(&lds->scratch.late.words[slot][b], &lds->scratch.late.errors[slot][b], best.error, best.lo, best.hi);
+            }
+        } else if (task < 0) {
+            rotate_first(task + early);
         } else if (task < boundTasks) {
             int const first = (task % CHUNKS) * CHUNK, nth = task / CHUNKS, search = nth < 2 * opaqueGroups ? nth : nth + opaqueGroups;
             int const b = block_of_group(group_of(search));
@@ -1636,6 +1675,7 @@ bc7_compress_kernel(BlockCompressArgs a)
     }
     __builtin_amdgcn_s_setprio(1);
     wait_for(shared.selected, searches);
+    bool const byBounds = all_by_bounds();
 
     // ---- 2. the errors of the partitions that are left, then candidates: first those that need no partition
     int const wholeTasks = __builtin_amdgcn_readfirstlane(shared.wholes) * (64 / kWholeChunk);
@@ -1668,7 +1708,7 @@ bc7_compress_kernel(BlockCompressArgs a)
             continue;
         }
         __builtin_amdgcn_s_setprio(0);
-        wait_for(shared.rotated, groups);
+        wait_for(shared.rotated, byBounds ? groups : opaqueGroups);
         int const keptFlat = __builtin_amdgcn_readfirstlane(shared.kept[0]), keptRotations = __builtin_amdgcn_readfirstlane(shared.kept[1]);
         int const keptSixes = __builtin_amdgcn_readfirstlane(shared.kept[2]);
         int const flatTasks = (keptFlat + 63) / 64, rotationTasks = flatTasks + (keptRotations + 63) / 64, sixTasks = (keptSixes + 63) / 64, candidate = task - estimates;
@@ -1679,7 +1719,7 @@ bc7_compress_kernel(BlockCompressArgs a)
             int const b = item & 127, rotation = item >> 7;
             Best const best = flat ? dual_planes<S, 2>(lds, b, rotation) : dual_planes<S, 3>(lds, b, rotation);
             int const slot = kSlotRotations + rotation - (rotation > int(shared.plans[b] & 3u) ? 1 : 0);
-            put_candidate(&lds->late.words[slot][b], &lds->late.errors[slot][b], best.error, best.lo, best.hi);
+            put_candidate(&lds->scratch.late.words[slot][b], &lds->scratch.late.errors[slot][b], best.error, best.lo, best.hi);
             continue;
         }
         if (candidate < rotationTasks + sixTasks) {
@@ -1708,7 +1748,7 @@ bc7_compress_kernel(BlockCompressArgs a)
             uint4 best = make_uint4(0u, 0u, 0u, 0u);
             uint32_t const plan = shared.plans[b];
             auto const consider = [&](float error, uint4 const& words) { if (!(error > bestError)) { bestError = error; best = words; } };
-            auto const consider_late = [&](int slot) { consider(shared.late.errors[slot][b], shared.late.words[slot][b]); };
+            auto const consider_late = [&](int slot) { consider(shared.scratch.late.errors[slot][b], shared.scratch.late.words[slot][b]); };
             if (!(shared.alphas[b] & kBelowOne))
                 for (int slot = 0; slot < kSlotRotations; ++slot) consider_late(slot);
             for (int r = 0; r < 4; ++r) {

@@ -519,6 +519,24 @@ def test_gpu_bc7_rotations_with_bounds_match_checker(ntc, device, oracle, size, 
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("content", ["plane", "level", "steep"])      # opaque blocks near a line, constant or not, and not
+@pytest.mark.parametrize("alpha", ["none", "one", "half", "all but one", "all"])
+def test_gpu_bc7_rotations_of_small_images_match_checker(ntc, device, oracle, alpha, content):
+    """Images of one group of 64 blocks to a workgroup with no, one, some or nothing but blocks with alpha in it: which of them
+    are by their bounds and which at once depends on both kinds."""
+    w, h = 132, 100
+    image = image_for_rotations(np.random.default_rng(82), content, w, h)
+    numbers = np.add.outer(np.arange(h // 4) * 3, np.arange(w // 4))
+    share = {"none": 0 * numbers, "one": numbers % 32 == 5, "half": numbers % 2, "all but one": numbers % 32 != 5, "all": 0 * numbers + 1}[alpha]
+    share = np.repeat(np.repeat(share, 4, axis=0), 4, axis=1) != 0
+    image[..., 3] = np.where(share, np.minimum(image[..., 0], 0.99) if content != "level" else 0.25, 1)
+    for fmt, texels in ((4, image), (1, np.rint(image * 255).astype(np.uint8))):
+        args = (np.ascontiguousarray(texels), fmt, 4, w // 4, h // 4)
+        got, want = compress_bc7(ntc, None, device, *args), compress_bc7(ntc, oracle, None, *args)
+        assert np.array_equal(got, want), (fmt, np.argwhere(got != want)[:4])
+
+
+@pytest.mark.gpu
 def test_gpu_bc7_arguments(ntc, device, oracle):
     from test_image_difference import fill_image
     rng = np.random.default_rng(9)
