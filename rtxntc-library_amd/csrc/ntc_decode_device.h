@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "ntc_decode_kernel.h"
+#include "ntc_launch.h"
+#include <type_traits>
 
 namespace ntc_hip_dev {
 
@@ -69,6 +71,17 @@ __device__ __forceinline__ DevMip const* table_entries(DevMip const* entries)
     ConstantMips const inlined = (ConstantMips)__builtin_amdgcn_kernarg_segment_ptr();
     ConstantMips const stored = (ConstantMips)(uintptr_t)entries;
     return (DevMip const*)(entries ? stored : inlined);
+}
+
+// Launches a kernel whose first argument is the table, and no other kind: that is what table_entries() relies on.
+template <class Kernel> struct TableFirst { static constexpr bool value = false; };
+template <class... Others> struct TableFirst<void (*)(MipTable, Others...)> { static constexpr bool value = true; };
+static_assert(std::is_standard_layout_v<MipTable> && std::is_trivially_copyable_v<MipTable>, "offsets in a kernel's arguments are those of the struct");
+template <auto KERNEL, class... ARGS>
+inline hipError_t launch_with_table(dim3 grid, dim3 block, size_t ldsBytes, hipStream_t stream, MipTable const& table, ARGS const&... args)
+{
+    static_assert(TableFirst<decltype(KERNEL)>::value, "the table lies where the arguments begin");
+    return launch_kernel<KERNEL>(grid, block, ldsBytes, stream, table, args...);
 }
 
 // ---- small device helpers -----------------------------------------------------------

@@ -1034,16 +1034,16 @@ static hipError_t launch_fp8_variant(MipTable const& mips, int numMips, int tota
     // Up to half as many tiles as compute units: quarter or half tiles.  (Beyond, two workgroups would take turns on a
     // compute unit: the weight planes leave no room for two.)
     int const units = compute_units_of_current_device(), log2Parts = 4 * totalTiles <= units ? 2 : (2 * totalTiles <= units ? 1 : 0);
-    if (log2Parts) return launch_kernel<decode_few_fp8_kernel<Any>>(dim3(unsigned(totalTiles) << log2Parts), dim3(Any::THREADS), 0, stream, mips, numMips, log2Parts);
+    if (log2Parts) return launch_with_table<decode_few_fp8_kernel<Any>>(dim3(unsigned(totalTiles) << log2Parts), dim3(Any::THREADS), 0, stream, mips, numMips, log2Parts);
     // Up to eight tiles per compute unit, too, one launch of the general instantiation decodes every set: the second launch and
     // a pass over weights cost more than three waves per SIMD instead of four.  (64 x 64 ... 1024 x 512 with one plane:
     // 11.0 and 25.1 us in two launches, 9.6 (in whole tiles) and 24.6 in one; 2048 x 1024: 74.7 and 76.7.  With two planes: 15.3 and 34.0,
     // 11.2 and 29.8.)
     if (totalTiles <= 8 * units)
-        return launch_kernel<decode_fp8_kernel<Any>>(dim3(gridSize), dim3(Any::THREADS), 0, stream, mips, numMips, tile_shares(totalTiles, gridSize), Fp8Handoff{ nullptr, 0u });
-    hipError_t const e = launch_kernel<decode_fp8_kernel<One>>(dim3(gridSize), dim3(One::THREADS), 0, stream, mips, numMips, tile_shares(totalTiles, gridSize), handoff);
+        return launch_with_table<decode_fp8_kernel<Any>>(dim3(gridSize), dim3(Any::THREADS), 0, stream, mips, numMips, tile_shares(totalTiles, gridSize), Fp8Handoff{ nullptr, 0u });
+    hipError_t const e = launch_with_table<decode_fp8_kernel<One>>(dim3(gridSize), dim3(One::THREADS), 0, stream, mips, numMips, tile_shares(totalTiles, gridSize), handoff);
     if (e != hipSuccess) return e;
-    return launch_kernel<decode_fp8_kernel<Any>>(dim3(gridSize), dim3(Any::THREADS), 0, stream, mips, numMips, tile_shares(totalTiles, gridSize), handoff);
+    return launch_with_table<decode_fp8_kernel<Any>>(dim3(gridSize), dim3(Any::THREADS), 0, stream, mips, numMips, tile_shares(totalTiles, gridSize), handoff);
 }
 
 hipError_t launch_decode_fp8(int variant, MipTable const& mips, int numMips, int totalTiles, int gridSize, Fp8Handoff handoff, hipStream_t stream)
@@ -1074,7 +1074,7 @@ static hipError_t launch_fp8_query_variant(MipTable const& mips, int numMips, De
     int const mostFeatures = !powers ? 8 : ordered ? 16 : 12;
     if (numQueries <= (FEATURES <= mostFeatures ? 128 : 64) * units) {
         int const waves = numQueries <= 64 * units ? 4 : 8;
-        return launch_kernel<query_few_fp8_kernel<Any>>(dim3(unsigned((numQueries + 16 * waves - 1) / (16 * waves))), dim3(Any::THREADS), 0, stream, mips, numMips, queries, numQueries, out, waves);
+        return launch_with_table<query_few_fp8_kernel<Any>>(dim3(unsigned((numQueries + 16 * waves - 1) / (16 * waves))), dim3(Any::THREADS), 0, stream, mips, numMips, queries, numQueries, out, waves);
     }
     // As few of a workgroup's waves at work as keep the workgroups within the compute units, four at least: then hardly
     // two share a SIMD (100000 queries: 17.4 us with all sixteen, 13.8).
@@ -1086,11 +1086,11 @@ static hipError_t launch_fp8_query_variant(MipTable const& mips, int numMips, De
     }
     // one launch, as in launch_fp8_variant (131072 queries: 14.0 us in two launches, 13.1 in one; 262144: 18.9 and 23.2)
     if (numQueries <= 512 * units)
-        return launch_kernel<query_fp8_kernel<Any>>(dim3(unsigned(grid)), dim3(Any::THREADS), 0, stream, mips, numMips, queries, numQueries, out, int(grid),
+        return launch_with_table<query_fp8_kernel<Any>>(dim3(unsigned(grid)), dim3(Any::THREADS), 0, stream, mips, numMips, queries, numQueries, out, int(grid),
                                                     waves < Any::WAVES ? waves : Any::WAVES, Fp8Handoff{ nullptr, 0u });
-    hipError_t const e = launch_kernel<query_fp8_kernel<One>>(dim3(unsigned(grid)), dim3(One::THREADS), 0, stream, mips, numMips, queries, numQueries, out, int(grid), waves, handoff);
+    hipError_t const e = launch_with_table<query_fp8_kernel<One>>(dim3(unsigned(grid)), dim3(One::THREADS), 0, stream, mips, numMips, queries, numQueries, out, int(grid), waves, handoff);
     if (e != hipSuccess) return e;
-    return launch_kernel<query_fp8_kernel<Any>>(dim3(unsigned(grid)), dim3(Any::THREADS), 0, stream, mips, numMips, queries, numQueries, out, int(grid),
+    return launch_with_table<query_fp8_kernel<Any>>(dim3(unsigned(grid)), dim3(Any::THREADS), 0, stream, mips, numMips, queries, numQueries, out, int(grid),
                                                 waves < Any::WAVES ? waves : Any::WAVES, handoff);
 }
 

@@ -63,12 +63,13 @@ struct DevMip {
 // would have to hand on to each other.  (A table copied from pinned memory took a copy and an event record per call:
 // one 128 x 128 mip, another set each call: 16.3 us, 9.1 us with the table in the arguments.)  Longer tables
 // - batches of sets - lie in device memory at `entries`, which is null otherwise.
-constexpr int kInlineMips = 16;                            // one set with a full mip chain; 2 176 bytes of arguments
+constexpr int kInlineMips = 16;                            // one set with a full mip chain
 struct MipTable {
     DevMip inlined[kInlineMips];
     int32_t starts[kInlineMips];   // of the inlined ones: their tileStart, side by side; 0x7fffffff where there is none
     DevMip const* entries;
 };
+static_assert(sizeof(DevMip) == 136 && sizeof(MipTable) == 2248, "arguments and tables are measured and documented with these sizes");
 
 // Brick geometry of a grid with `layers` u16 layers: log2 of the brick's side in cells.
 constexpr int brick_side_log2(int layers) { return layers == 1 ? 3 : 2; }

@@ -1153,12 +1153,12 @@ __device__ __forceinline__ void mlp_forward_f16(LdsT<V>& lds, int wave, int lane
     wave_priority<kPrioOther>();
 }
 
-// Two workgroups of eight waves per CU: sixteen waves, 128 VGPRs each, four to a SIMD.
 // The last entry whose tiles begin at or before `tile`, of a table in the kernel's arguments: one scalar load and no trip to
 // memory for each entry, a dozen in front of a workgroup's weights where a launch of few tiles has a mip chain (256 x 256
 // with its 9 mips 11.6 us, 10.4 now; 300 x 200 of sixteen features 12.3 and 11.3).  Not for a single mip: the line of the
 // arguments that the numbers lie in is a trip by itself (256 x 256 8.4 and 8.7; the empty assembly keeps the load from being
-// made ahead of the question).
+// made ahead of the question).  For a table whose `entries` is null, the kernel's
+// first argument as for table_entries(): no other has starts.
 __device__ __forceinline__ int inlined_entry_of(int tile)
 {
     typedef __attribute__((address_space(4))) int32_t const* ConstantInts;
@@ -1170,6 +1170,7 @@ __device__ __forceinline__ int inlined_entry_of(int tile)
     return entry;
 }
 
+// Two workgroups of eight waves per CU: sixteen waves, 128 VGPRs each, four to a SIMD.
 template <class V>
 __global__ void __launch_bounds__(V::THREADS, V::WAVES_PER_SIMD)
 decode_kernel(MipTable table, int numMips, TileShares shares)
@@ -1595,8 +1596,8 @@ static hipError_t launch_variant(MipTable const& mips, int numMips, int totalTil
     // waves would share one, and each would read every weight from LDS for a quarter of the texels: 256 x 256 8.5 us
     // against 7.9 with whole tiles.
     int const units = compute_units_of_current_device(), log2Parts = 4 * totalTiles <= units ? 2 : (2 * totalTiles <= units ? 1 : 0);
-    if (log2Parts) return launch_kernel<decode_few_kernel<V>>(dim3(unsigned(totalTiles) << log2Parts), dim3(V::THREADS), 0, stream, mips, numMips, log2Parts);
-    return launch_kernel<decode_kernel<V>>(dim3(gridSize), dim3(V::THREADS), 0, stream, mips, numMips, tile_shares(totalTiles, gridSize));
+    if (log2Parts) return launch_with_table<decode_few_kernel<V>>(dim3(unsigned(totalTiles) << log2Parts), dim3(V::THREADS), 0, stream, mips, numMips, log2Parts);
+    return launch_with_table<decode_kernel<V>>(dim3(gridSize), dim3(V::THREADS), 0, stream, mips, numMips, tile_shares(totalTiles, gridSize));
 }
 
 hipError_t launch_decode(int variant, MipTable const& mips, int numMips, int totalTiles, int gridSize, hipStream_t stream)
@@ -1622,9 +1623,9 @@ static hipError_t launch_query_variant(MipTable const& mips, int numMips, DevQue
     // 65536: 15.6, 8.4).
     int const units = compute_units_of_current_device();
     uint64_t const few = (numQueries + 16 * V::WAVES - 1) / (16 * V::WAVES);
-    if (few <= uint64_t(units)) return launch_kernel<query_few_kernel<V>>(dim3(unsigned(few)), dim3(V::THREADS), 0, stream, mips, numMips, queries, numQueries, out);
-    if (2 * gridSize <= units) return launch_kernel<query_kernel<V>>(dim3(2 * gridSize), dim3(V::THREADS), 0, stream, mips, numMips, queries, numQueries, out, 2 * gridSize, V::WAVES / 2);
-    return launch_kernel<query_kernel<V>>(dim3(gridSize), dim3(V::THREADS), 0, stream, mips, numMips, queries, numQueries, out, gridSize, V::WAVES);
+    if (few <= uint64_t(units)) return launch_with_table<query_few_kernel<V>>(dim3(unsigned(few)), dim3(V::THREADS), 0, stream, mips, numMips, queries, numQueries, out);
+    if (2 * gridSize <= units) return launch_with_table<query_kernel<V>>(dim3(2 * gridSize), dim3(V::THREADS), 0, stream, mips, numMips, queries, numQueries, out, 2 * gridSize, V::WAVES / 2);
+    return launch_with_table<query_kernel<V>>(dim3(gridSize), dim3(V::THREADS), 0, stream, mips, numMips, queries, numQueries, out, gridSize, V::WAVES);
 }
 
 // Plain grid ([layer][row][column] u16) -> bricks; one thread per stored u16, reads coalesced.
