@@ -200,8 +200,8 @@ template <int C> BC7_INLINE void refine(Color<C> const (&px)[16], uint32_t mask,
 BC7_INLINE int quantize(float v, int bits) { return int(rintf(saturate(v) * float((1u << bits) - 1u))); }
 BC7_INLINE int expand8(int q, int bits) { return (q << (8 - bits)) | (q >> (2 * bits - 8)); }
 
-// Indices of the subset's texels along the dequantised endpoints, each in its place in the block: `two` for 2-bit ones,
-// `three` for 3-bit ones, whichever BITS says, both for 0 (then indexBits tells).
+// Indices of the subset's texels along the dequantised endpoints, each in its place in the block: `two` for 2-bit ones, `more`
+// for those of three bits and four, whichever BITS says; for 0 both, and `indexBits` tells which of them is meant.
 template <int C, int BITS> BC7_INLINE void assign(Color<C> const (&px)[16], uint32_t mask, int indexBits, int endpointBits,
                                                   Quantized<C> const& q0, Quantized<C> const& q1, uint32_t& two, uint64_t& more)
 {

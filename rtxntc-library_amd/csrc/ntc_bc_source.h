@@ -18,8 +18,6 @@ __device__ __forceinline__ float max_f32(float a, float b) { float r; asm("v_max
 
 __device__ __forceinline__ float min3_f32(float a, float b, float c) { float r; asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c)); return r; }
 __device__ __forceinline__ float max3_f32(float a, float b, float c) { float r; asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c)); return r; }
-// (The compiler makes two-operand minima of a nest of min().)
-__device__ __forceinline__ uint32_t min3_u32(uint32_t a, uint32_t b, uint32_t c) { uint32_t r; asm("v_min3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c)); return r; }
 
 // k / d for an integer k in [0, d], d = 255 or 65535, r = 1 / d rounded: one Newton step on k * r gives the
 // correctly rounded quotient for every such k (all 256 + 65536 cases are checked in the tests with exact

@@ -343,9 +343,10 @@ struct RunMip {
 // Look-ups in the table of a decode call (one entry per mip of every set, sorted by tileStart).  Both go through
 // the table a wave at a time - one load per lane and a ballot - where a loop over the entries pays a memory round
 // trip for each: a workgroup does this once per segment of its share, twelve entries further for a full mip chain.
-// Every wave computes the same, uniform, result.  Used by decode_fp8_kernel (-0.6 % on a 4096 x 4096 decode);
-// decode_kernel keeps the plain loops: there the same change took 1.3 % off a batch of eight sets and added
-// 0.3 - 3 % to single sets, through the tile loop's register allocation.
+// Every wave computes the same, uniform, result.  Used by decode_fp8_kernel (-0.6 % on a 4096 x 4096 decode) and by the
+// kernels for few tiles.  decode_kernel finds the first entry of a table in its arguments by inlined_entry_of(), and keeps
+// the plain loops for longer tables and for a segment's end: there this took 1.3 % off a batch of eight sets and added 0.3 - 3 %
+// to single sets, through the tile loop's register allocation.
 
 // The last entry at or after `entry` whose tiles begin at or before `tile`.
 __device__ __forceinline__ int table_entry_of(DevMip const* __restrict__ mips, int numMips, int entry, int tile)
@@ -580,9 +581,6 @@ __device__ __forceinline__ void load_brick_cell(GlobalU8Ptr base, uint32_t off, 
     }
 }
 
-// What a query needs of its mip, kept in LDS: every lane of a wave may address another mip, and
-// fetching these fields per lane from the table in global memory put a long dependent load in
-// front of the latent gathers.
 // The lane's query of the 64 of a wave, the call's last one again beyond it.  Whole waves, all but one of a call, read and
 // write at lane offsets from scalar addresses: a store takes half the instructions.  (With the
 // taps' offsets by column and row, 2^24 queries of the headline network 588.8 -> 575.7 us, 2^22 of the 0.9.2 one 163 -> 158.)
@@ -627,6 +625,9 @@ __device__ __forceinline__ void store_whole_queries(uint16_t* out, uint64_t q0, 
     else                       store(std::false_type{});
 }
 
+// What a query needs of its mip, kept in LDS: every lane of a wave may address another mip, and
+// fetching these fields per lane from the table in global memory put a long dependent load in
+// front of the latent gathers.
 struct QueryMip {
     uint16_t const* hr;
     uint16_t const* lr;

@@ -268,7 +268,9 @@ __device__ __attribute__((noinline)) int stage_fp8_weights(Fp8Lds<V>& lds, uint8
         build_fp8_feature_lut<V::THREADS>(lds, tid);
     }
 
-    uint32_t found = 0;                                      // bit l: not tame; bit 4 + l: not one plane; bit 8: outputs not bounded
+    // bit l: layer l is not tame; 4 + l: not one plane; 8: outputs not bounded; 9: a large output bias; 10 + tile (kFp8StartShift):
+    // the tile's sums do not start at the bias
+    uint32_t found = 0;
     if (mine && layer < 3) {
         int32_t sum = 0, top = 0;
 #pragma unroll
