@@ -568,6 +568,7 @@ struct SearchLds {
     int counts[2], next[2], wholes, kept[3];                 // kept: rotations of both kinds, mode 6
     int bounded[kSearches], selected, rotated, estimated;    // tasks done: those of a search's bounds, of selections, first rotations and estimates
 };
+static_assert(2 * sizeof(SearchLds<128>) <= 160 * 1024, "two workgroups share a compute unit's memory: one works while the other waits for its last task");
 template <class S> using SearchPtr = __attribute__((address_space(3))) S*;
 
 // The tasks are functions of their own (arguments reach them per lane: what is uniform is made so again): in one body
